@@ -1,88 +1,279 @@
 // True fp32 matrix product for the 32-bit path: C[M,N] = A[M,K] * W[N,K]^T, everything
-// row-major fp32, plain FMA (no matrix-core reduced-precision mode).
+// row-major fp32, on the matrix cores' 32-bit instruction (no reduced-precision mode).
 //
 // It stands where the reference calls cublasGemmEx with the OP_T/OP_N trick for a row-major
-// [out,in] weight (base/src/engine.cu:652-671).  Each output element is one accumulator that
-// takes k = 0..K-1 in ascending order, so a row of C does not depend on M, on the tile it falls
-// in or on the other rows: the fp32 path is bit-identical under any batching.
+// [out,in] weight (base/src/engine.cu:652-671).  The order of an output's sum depends on K alone:
+// K is cut into parts (gf_part), a part's products go 16 columns at a time through four
+// v_mfma_f32_16x16x4_f32 into one accumulator (instruction j takes columns j, j + 4, j + 8, j + 12 of the 16:
+// what the four lane groups hold at place j of the 16 bytes each of them loads), the parts of the front half are
+// added in order, those of the back half are, and the two sums are added.  Both kernels below do just that, so a row
+// of C does not depend on M, on the tile it falls in, on which kernel ran or on the other rows: the fp32 path is
+// bit-identical under any batching.
+//
+// us a call, weights from memory, against one kernel of 64 x 64 tiles and plain FMAs for every M (before -> now;
+// relative error against 64 bits at K = 2,048 / 8,192: 8e-7 / 1.6e-6 -> 2.1e-7 / 4.1e-7):
+//   rows x outputs x K    3 x 128,256 x 2,048: 480 -> 260 (4.0 TB/s)     3 x 16,384 x 2,048: 147 -> 33 (4.1 TB/s)
+//                         3 x 2,048 x 8,192: 544 -> 19 (3.5 TB/s)        3 x 3,072 x 2,048: 141 -> 11
+//                         32 x 2,048 x 8,192: 545 -> 58                  64 x 2,048 x 8,192: 559 -> 59 (the tiles: 167)
+//                         402 x 16,384 x 2,048: 449 -> 329 (82 TFLOP/s)  402 x 2,048 x 8,192: 556 -> 167 (81)
+//                         2,048 x 16,384 x 2,048: 1,748 -> 1,319 (104)
+// The few-rows kernel stays below the 6 TB/s of a plain read stream: a load takes 64 bytes from each of 16 rows.
 #include "common.h"
 
-#define GF_BM 64
-#define GF_BN 64
-#define GF_BK 16
+typedef float gf_f32x4 __attribute__((ext_vector_type(4)));
 
-__global__ void __launch_bounds__(256)
-gemm_nt_f32_kernel(float *__restrict__ C, const float *__restrict__ A, const float *__restrict__ W,
-                   int M, int N, int K, int lda, int ldw, int ldc) {
-    __shared__ float As[GF_BK][GF_BM + 4];
-    __shared__ float Ws[GF_BK][GF_BN + 4];
-    const int tid = threadIdx.x;
-    const int tx = tid % 16, ty = tid / 16;
-    const int m0 = blockIdx.y * GF_BM, n0 = blockIdx.x * GF_BN;
-    const int lrow = tid / 4, lk = (tid % 4) * 4;
-    const bool vec_ok = (K % 4 == 0) && (lda % 4 == 0) && (ldw % 4 == 0);
+#define GF_STEP 16                  // columns of K that one 16-byte load a lane covers
+#define GF_MAX_PARTS 16
+#define GF_ROWS_UP_TO 64            // rows up to which the few-rows kernel runs: one row of tiles does not fill the chip
+#define GF_BM 64                    // the tile kernel: rows a workgroup, columns of K a round, padding of a row in LDS
+#define GF_BK 32
+#define GF_PAD 4
 
-    float acc[4][4];
-#pragma unroll
-    for (int i = 0; i < 4; ++i)
-#pragma unroll
-        for (int j = 0; j < 4; ++j) acc[i][j] = 0.f;
+// Columns of K a part takes: a sixteenth of K in whole rounds of the tile kernel, at least 64 - so at most 16 parts.
+static inline int gf_part(int K) {
+    const int rounds = (K + GF_BK - 1) / GF_BK;
+    const int part = (rounds + GF_MAX_PARTS - 1) / GF_MAX_PARTS * GF_BK;
+    return part < 64 ? 64 : part;
+}
 
-    for (int k0 = 0; k0 < K; k0 += GF_BK) {
-        float a[4] = {0.f, 0.f, 0.f, 0.f}, w[4] = {0.f, 0.f, 0.f, 0.f};
-        const int am = m0 + lrow, wn = n0 + lrow, kk = k0 + lk;
-        if (am < M) {
-            const float *p = A + (size_t)am * lda + kk;
-            if (vec_ok && kk + 3 < K) {
-                const float4 v = *reinterpret_cast<const float4 *>(p);
-                a[0] = v.x; a[1] = v.y; a[2] = v.z; a[3] = v.w;
-            } else {
+// Parts of the front half: an output is (sum of the front parts, in order) + (sum of the others, in order).
+__host__ __device__ inline int gf_half(int parts) { return (parts + 1) / 2; }
+
+// four neighbouring elements of a row, zeros past the row's end or for a row that is not there
+template <bool VEC, bool STREAMED>
+__device__ inline gf_f32x4 gf_load(const float *__restrict__ p, int row, int rows, int k, int K, int ld) {
+    gf_f32x4 v = {0.f, 0.f, 0.f, 0.f};
+    if (row < rows) {
+        const float *a = p + (size_t)row * ld + k;
+        if (VEC) {
+            if (k < K) v = STREAMED ? __builtin_nontemporal_load(reinterpret_cast<const gf_f32x4 *>(a))
+                                    : *reinterpret_cast<const gf_f32x4 *>(a);      // (K is a multiple of 4)
+        } else {
 #pragma unroll
-                for (int e = 0; e < 4; ++e)
-                    if (kk + e < K) a[e] = p[e];
-            }
-        }
-        if (wn < N) {
-            const float *p = W + (size_t)wn * ldw + kk;
-            if (vec_ok && kk + 3 < K) {
-                const float4 v = *reinterpret_cast<const float4 *>(p);
-                w[0] = v.x; w[1] = v.y; w[2] = v.z; w[3] = v.w;
-            } else {
-#pragma unroll
-                for (int e = 0; e < 4; ++e)
-                    if (kk + e < K) w[e] = p[e];
-            }
-        }
-        __syncthreads();
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-            As[lk + e][lrow] = a[e];
-            Ws[lk + e][lrow] = w[e];
-        }
-        __syncthreads();
-#pragma unroll
-        for (int k = 0; k < GF_BK; ++k) {
-            float av[4], wv[4];
-#pragma unroll
-            for (int i = 0; i < 4; ++i) av[i] = As[k][ty * 4 + i];
-#pragma unroll
-            for (int j = 0; j < 4; ++j) wv[j] = Ws[k][tx * 4 + j];
-#pragma unroll
-            for (int i = 0; i < 4; ++i)
-#pragma unroll
-                for (int j = 0; j < 4; ++j) acc[i][j] = fmaf(av[i], wv[j], acc[i][j]);
+            for (int e = 0; e < 4; ++e)
+                if (k + e < K) v[e] = a[e];
         }
     }
+    return v;
+}
+
+// Few rows: what bounds it is the stream of W.  A workgroup takes 16 outputs and 16 MT rows, a wavefront one part of
+// K (all parts of a tile of W are on their way at once, `DEPTH` steps of each in registers before the first
+// product); the parts are added in order through LDS.  PAIR: up to 8 rows and 8 outputs a workgroup, a wavefront
+// takes two parts - operand rows 0-7 the first, 8-15 the second, on both sides, so that the products wanted are
+// the two blocks on the diagonal.  That puts twice the workgroups on a narrow matrix (128 of them would leave
+// half the chip without a share of the stream).
+template <int MT, int DEPTH, bool PAIR, bool VEC>
+__global__ void __launch_bounds__(KVA_WAVE * GF_MAX_PARTS)
+gemm_f32_rows_kernel(float *__restrict__ C, const float *__restrict__ A, const float *__restrict__ W, int M, int N,
+                     int K, int lda, int ldw, int ldc, int part) {
+    constexpr int OUT = PAIR ? 8 : 16;
+    __shared__ float sums[GF_MAX_PARTS][MT][OUT][OUT + 1];
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / KVA_WAVE);     // (scalar: so are the branches around the products)
+    const int lane = threadIdx.x % KVA_WAVE, r = lane % 16, g = lane / 16;
+    const int n0 = blockIdx.x * OUT, m0 = blockIdx.y * 16 * MT;
+    const int first = PAIR ? 2 * wave : wave;                       // the wavefront's (first) part
+    const int steps = (min(K, (first + 1) * part) - first * part + GF_STEP - 1) / GF_STEP;
+    const int mine = PAIR ? first + r / 8 : first, lo = mine * part, hi = min(K, lo + part);     // (lo may lie past K: zeros)
+    const int wr = n0 + (PAIR ? r % 8 : r), ar = m0 + (PAIR ? r % 8 : r);
+    gf_f32x4 acc[MT];
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-        const int m = m0 + ty * 4 + i;
+    for (int t = 0; t < MT; ++t) acc[t] = gf_f32x4{0.f, 0.f, 0.f, 0.f};
+    gf_f32x4 w[2][DEPTH], x[2][DEPTH][MT];
+    auto fetch = [&](int buf, int s0) {
+#pragma unroll
+        for (int d = 0; d < DEPTH; ++d) {
+            const int k = lo + (s0 + d) * GF_STEP + 4 * g;          // (past the part's end: zeros)
+            w[buf][d] = gf_load<VEC, true>(W, wr, N, k, hi, ldw);
+#pragma unroll
+            for (int t = 0; t < MT; ++t) x[buf][d][t] = gf_load<VEC, false>(A, ar + 16 * t, M, k, hi, lda);
+        }
+    };
+    auto products = [&](int buf, int s0) {
+#pragma unroll
+        for (int d = 0; d < DEPTH; ++d)
+            if (s0 + d < steps)
+#pragma unroll
+                for (int j = 0; j < 4; ++j)
+#pragma unroll
+                    for (int t = 0; t < MT; ++t)
+                        acc[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(w[buf][d][j], x[buf][d][t][j], acc[t], 0, 0, 0);
+    };
+    fetch(0, 0);
+    for (int s0 = 0; s0 < steps; s0 += 2 * DEPTH) {
+        fetch(1, s0 + DEPTH);
+        products(0, s0);
+        fetch(0, s0 + 2 * DEPTH);
+        products(1, s0 + DEPTH);
+    }
+#pragma unroll
+    for (int t = 0; t < MT; ++t)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {                               // [row][output]
+            if (!PAIR) sums[wave][t][r][4 * g + i] = acc[t][i];
+            else if (r / 8 == g / 2) sums[mine][t][r % 8][(4 * g + i) % 8] = acc[t][i];
+        }
+    __syncthreads();
+    const int parts = (K + part - 1) / part, half = gf_half(parts);
+    for (int e = threadIdx.x; e < MT * OUT * OUT; e += blockDim.x) {
+        const int t = e / (OUT * OUT), m = e % (OUT * OUT) / OUT, n = e % OUT;
+        float front = 0.f, back = 0.f;
+        for (int p = 0; p < half; ++p) front += sums[p][t][m][n];
+        for (int p = half; p < parts; ++p) back += sums[p][t][m][n];
+        if (m0 + 16 * t + m < M && n0 + n < N) C[(size_t)(m0 + 16 * t + m) * ldc + n0 + n] = front + back;
+    }
+}
+
+// Many rows: bound by the matrix cores (a 32-bit product takes 16 times the cycles of a 16-bit one).  A workgroup
+// takes 64 rows x 32 NT outputs: four wavefronts (32 x 16 NT each) the front half of the parts, four the back half -
+// two wavefronts a SIMD where the tiles are about as many as the compute units.  32 columns of both operands of
+// each half go through LDS at a time (rows 36 elements apart: the 16 rows of an operand read start in different
+// banks), the next ones' loads in flight over the products.  Workgroups of one stripe of outputs are neighbours on
+// one die, whose L2 then holds that stripe of W for all of their rows.
+template <int NT>
+struct GfTile {
+    float a[2][GF_BM][GF_BK + GF_PAD], w[2][32 * NT][GF_BK + GF_PAD];
+};
+
+template <int NT, bool VEC>
+__global__ void __launch_bounds__(512)
+gemm_f32_tile_kernel(float *__restrict__ C, const float *__restrict__ A, const float *__restrict__ W, int M, int N,
+                     int K, int lda, int ldw, int ldc, int part, int mtiles, int tiles) {
+    constexpr int BN = 32 * NT, AL = GF_BM * GF_BK / 4 / 256, WL = BN * GF_BK / 4 / 256;
+    __shared__ GfTile<NT> lds[2];
+    const int per = (tiles + 7) / 8, tile = (int)(blockIdx.x % 8) * per + (int)(blockIdx.x / 8);
+    if (tile >= tiles) return;                                       // (the whole workgroup)
+    const int m0 = tile % mtiles * GF_BM, n0 = tile / mtiles * BN;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / KVA_WAVE), back = wave / 4;
+    const int tid = threadIdx.x % 256, lane = tid % KVA_WAVE, r = lane % 16, g = lane / 16;
+    const int wm = wave % 2 * 32, wn = wave / 2 % 2 * 16 * NT;
+    const int split = min(K, gf_half((K + part - 1) / part) * part); // the back half's first column
+    const int lo = back ? split : 0, hi = back ? K : split;
+    GfTile<NT> &L = lds[back];
+    gf_f32x4 acc[NT][2], tot[NT][2], la[2][AL], lw[2][WL];
+#pragma unroll
+    for (int i = 0; i < NT; ++i)
+#pragma unroll
+        for (int j = 0; j < 2; ++j) acc[i][j] = tot[i][j] = gf_f32x4{0.f, 0.f, 0.f, 0.f};
+    const int lrow = tid / 8, lk = tid % 8 * 4;                      // 32 rows a pass, 8 lanes a row
+    auto fetch = [&](int set, int k0) {                              // (past the half's end: zeros)
+#pragma unroll
+        for (int i = 0; i < AL; ++i) la[set][i] = gf_load<VEC, false>(A, m0 + lrow + 32 * i, M, k0 + lk, hi, lda);
+#pragma unroll
+        for (int i = 0; i < WL; ++i) lw[set][i] = gf_load<VEC, false>(W, n0 + lrow + 32 * i, N, k0 + lk, hi, ldw);
+    };
+    auto put = [&](int set) {
+#pragma unroll
+        for (int i = 0; i < AL; ++i) *reinterpret_cast<gf_f32x4 *>(&L.a[set][lrow + 32 * i][lk]) = la[set][i];
+#pragma unroll
+        for (int i = 0; i < WL; ++i) *reinterpret_cast<gf_f32x4 *>(&L.w[set][lrow + 32 * i][lk]) = lw[set][i];
+    };
+    int left = part;                                                 // columns of the current part still to come
+    auto round = [&](int set) {
+#pragma unroll
+        for (int s = 0; s < GF_BK / GF_STEP; ++s) {
+            gf_f32x4 a[2], w[NT];
+#pragma unroll
+            for (int j = 0; j < 2; ++j)
+                a[j] = *reinterpret_cast<const gf_f32x4 *>(&L.a[set][wm + 16 * j + r][s * GF_STEP + 4 * g]);
+#pragma unroll
+            for (int i = 0; i < NT; ++i)
+                w[i] = *reinterpret_cast<const gf_f32x4 *>(&L.w[set][wn + 16 * i + r][s * GF_STEP + 4 * g]);
+#pragma unroll
+            for (int e = 0; e < 4; ++e)
+#pragma unroll
+                for (int i = 0; i < NT; ++i)
+#pragma unroll
+                    for (int j = 0; j < 2; ++j)
+                        acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(w[i][e], a[j][e], acc[i][j], 0, 0, 0);
+        }
+        left -= GF_BK;
+        if (left == 0) {
+            left = part;
+#pragma unroll
+            for (int i = 0; i < NT; ++i)
+#pragma unroll
+                for (int j = 0; j < 2; ++j) {
+#pragma unroll
+                    for (int c = 0; c < 4; ++c) tot[i][j][c] += acc[i][j][c];
+                    acc[i][j] = gf_f32x4{0.f, 0.f, 0.f, 0.f};
+                }
+        }
+    };
+    // Two rounds at a time: while one is multiplied from its LDS buffer the next one waits in registers and the one
+    // after that is asked for.  The front half is never the shorter one: its rounds are both halves' (the back half's
+    // last ones may be zeros).
+    fetch(0, lo);
+    fetch(1, lo + GF_BK);
+    for (int d = 0; d < split; d += 2 * GF_BK) {
+        put(0);
+        __syncthreads();
+        fetch(0, lo + d + 2 * GF_BK);
+        round(0);
+        put(1);
+        __syncthreads();
+        fetch(1, lo + d + 3 * GF_BK);
+        round(1);
+    }
+    __syncthreads();
+    if (left != part)                                                // a last, shorter part
+#pragma unroll
+        for (int i = 0; i < NT; ++i)
+#pragma unroll
+            for (int j = 0; j < 2; ++j)
+#pragma unroll
+                for (int c = 0; c < 4; ++c) tot[i][j][c] += acc[i][j][c];
+    // the back half's sums to the front half, through LDS (the operands there have been read)
+    gf_f32x4 *over = reinterpret_cast<gf_f32x4 *>(&lds[0]);
+    static_assert(sizeof(lds) >= sizeof(gf_f32x4) * 256 * NT * 2, "the back half's sums fit where the operands were");
+    if (back)
+#pragma unroll
+        for (int i = 0; i < NT; ++i)
+#pragma unroll
+            for (int j = 0; j < 2; ++j) over[(i * 2 + j) * 256 + tid] = tot[i][j];
+    __syncthreads();
+    if (back) return;
+#pragma unroll
+    for (int j = 0; j < 2; ++j) {
+        const int m = m0 + wm + 16 * j + r;
         if (m >= M) continue;
 #pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            const int n = n0 + tx * 4 + j;
-            if (n < N) C[(size_t)m * ldc + n] = acc[i][j];
+        for (int i = 0; i < NT; ++i) {
+            const int n = n0 + wn + 16 * i + 4 * g;
+            float *c = C + (size_t)m * ldc + n;
+            const gf_f32x4 o = over[(i * 2 + j) * 256 + tid];
+            gf_f32x4 v;
+#pragma unroll
+            for (int e = 0; e < 4; ++e) v[e] = tot[i][j][e] + o[e];
+            if (VEC && n + 3 < N) *reinterpret_cast<gf_f32x4 *>(c) = v;
+            else
+#pragma unroll
+                for (int e = 0; e < 4; ++e)
+                    if (n + e < N) c[e] = v[e];
         }
     }
+}
+
+template <bool VEC>
+static void gf_launch(float *C, const float *A, const float *W, int M, int N, int K, int lda, int ldw, int ldc,
+                      hipStream_t stream) {
+    const int part = gf_part(K), parts = (K + part - 1) / part;
+    if (M <= GF_ROWS_UP_TO) {
+        const int out = M <= 8 ? 8 : 16;
+        const dim3 grid((N + out - 1) / out, (M + 31) / 32), block(KVA_WAVE * (M <= 8 ? (parts + 1) / 2 : parts));
+        if (M <= 8)
+            hipLaunchKernelGGL((gemm_f32_rows_kernel<1, 2, true, VEC>), grid, block, 0, stream, C, A, W, M, N, K, lda, ldw, ldc, part);
+        else if (M <= 16)
+            hipLaunchKernelGGL((gemm_f32_rows_kernel<1, 2, false, VEC>), grid, block, 0, stream, C, A, W, M, N, K, lda, ldw, ldc, part);
+        else
+            hipLaunchKernelGGL((gemm_f32_rows_kernel<2, 2, false, VEC>), grid, block, 0, stream, C, A, W, M, N, K, lda, ldw, ldc, part);
+        return;
+    }
+    const int mtiles = (M + GF_BM - 1) / GF_BM, wide = mtiles * ((N + 127) / 128), narrow = mtiles * ((N + 63) / 64);
+    if (wide >= 256)
+        hipLaunchKernelGGL((gemm_f32_tile_kernel<4, VEC>), dim3((wide + 7) / 8 * 8), dim3(512), 0, stream, C, A, W, M, N, K, lda, ldw, ldc, part, mtiles, wide);
+    else
+        hipLaunchKernelGGL((gemm_f32_tile_kernel<2, VEC>), dim3((narrow + 7) / 8 * 8), dim3(512), 0, stream, C, A, W, M, N, K, lda, ldw, ldc, part, mtiles, narrow);
 }
 
 extern "C" int kva_gemm_nt_f32(float *C, const float *A, const float *W, int M, int N, int K,
@@ -90,9 +281,12 @@ extern "C" int kva_gemm_nt_f32(float *C, const float *A, const float *W, int M, 
     KVA_REQUIRE(M >= 0 && N > 0 && K > 0, "gemm_f32: bad sizes M=%d N=%d K=%d", M, N, K);
     KVA_REQUIRE(lda >= K && ldw >= K && ldc >= N, "gemm_f32: leading dimensions too small");
     if (M == 0) return KVA_OK;
-    dim3 grid((N + GF_BN - 1) / GF_BN, (M + GF_BM - 1) / GF_BM), block(256);
-    KVA_REQUIRE(grid.y <= 65535, "gemm_f32: M=%d is too large for one launch", M);
-    hipLaunchKernelGGL(gemm_nt_f32_kernel, grid, block, 0, stream, C, A, W, M, N, K, lda, ldw, ldc);
+    KVA_REQUIRE((M + GF_BM - 1) / GF_BM <= 65535, "gemm_f32: M=%d is too large for one launch", M);
+    // 16-byte loads and stores where every row of all three starts at a multiple of 16 bytes
+    const bool vec = K % 4 == 0 && lda % 4 == 0 && ldw % 4 == 0 && ldc % 4 == 0 &&
+                     ((uintptr_t)A | (uintptr_t)W | (uintptr_t)C) % 16 == 0;
+    if (vec) gf_launch<true>(C, A, W, M, N, K, lda, ldw, ldc, stream);
+    else gf_launch<false>(C, A, W, M, N, K, lda, ldw, ldc, stream);
     KVA_CHECK_LAUNCH("gemm_nt_f32");
     return KVA_OK;
 }

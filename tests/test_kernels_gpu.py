@@ -178,6 +178,28 @@ def test_gemm_f32_is_true_fp32_and_row_independent(m, n, k, gpu):
     assert torch.equal(one[0], out[m - 1])
 
 
+@pytest.mark.parametrize("k", [1, 15, 64, 100, 1040, 2048, 2050, 5000])
+@pytest.mark.parametrize("n", [16, 130, 4161])
+def test_gemm_f32_rows_are_the_same_bits_in_every_kernel(n, k, gpu):
+    """One row alone, 16, 17, 32 rows (the few-rows kernel), 33, 64, 65 and 600 rows (both tiles): the same bits."""
+    a, w = rnd(600, k).to(gpu), rnd(n, k, seed=1).to(gpu)
+    rows = {}
+    for m in (1, 16, 17, 32, 33, 64, 65, 600):
+        rows[m] = K.gemm_nt_f32(a[:m], w, torch.full((m, n), float("nan"), device=gpu))
+    for m, got in rows.items():
+        assert torch.equal(got, rows[600][:m]), m
+    last = K.gemm_nt_f32(a[599:], w, torch.empty(1, n, device=gpu))
+    assert torch.equal(last[0], rows[600][599])
+    want = a.double() @ w.double().t()
+    # K products and additions of relative error 2^-24 each, by their root: rms errors add up in squares
+    assert (rows[600] - want).double().pow(2).mean().sqrt() <= 2.0 ** -24 * max(4.0, (2.0 * k) ** 0.5) * (a.double().pow(2) @ w.double().pow(2).t()).sqrt().mean()
+    # a view whose rows do not start at multiples of 16 bytes
+    flat = torch.zeros(65 * k + 1, device=gpu)
+    flat[1:] = a[:65].reshape(-1)
+    odd = K.gemm_nt_f32(flat[1:].view(65, k), w, torch.empty(65, n, device=gpu))
+    assert torch.equal(odd, rows[65])
+
+
 def rope_reference(x, pos, inv, heads, d, rot):
     cos, sin = plain.rope_cos_sin(pos, inv)
     x = x.view(len(pos), heads, d).clone()
