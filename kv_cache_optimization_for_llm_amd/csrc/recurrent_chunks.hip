@@ -1,0 +1,639 @@
+// The gated delta rule and gated linear attention over prompts, 64 tokens at a time on the matrix cores.
+//
+// recurrent.hip walks a request's tokens one after the other, about 0.3 us a token whatever the chip could do beside
+// it.  Written out over a chunk of tokens 1..C that starts from the state S, with D_ij the product of the decays
+// (per key channel) of the tokens j + 1..i:
+//
+//   u_i = beta_i (v_i - S^T (D_i0 k_i) - sum_{j<i} (k_i . D_ij k_j) u_j)        (linear attention: u_i = v_i)
+//   o_i = S^T (D_i0 q_i) + sum_{j<=i} (q_i . D_ij k_j) u_j
+//   S  <- D_C0 S + sum_j (D_Cj k_j) u_j^T
+//
+// The u_i are the solution of a unit lower triangular system with right-hand sides beta v and beta D_0 k, so
+//   U = Uv - W S,    O = Qd S + P U,    S <- diag(G) S + Kd^T U
+// with Uv, W, Qd, P, Kd, G of a chunk known without S.  Three kernels: `prepare` makes those, all chunks side by side;
+// `states` hands S on from chunk to chunk, a head's value columns 16 to a workgroup, and leaves the S each chunk
+// starts from and its U; `outputs` makes O, all chunks side by side again.
+//
+// Everything is 32-bit, on v_mfma_f32_16x16x4_f32.  Decays only ever enter as products of decays between two
+// tokens (at most 1, no logarithms, no quotients): a decay of zero or of anything else is as exact as in the walk.
+// Order of sums: chunks are counted from the step's first token of the request, so here - unlike in the walk - the
+// last bits of a token's result depend on how the request was cut into steps.  The 32-bit path therefore walks.
+//
+// us a call, the walk -> these three kernels (prepare + states + outputs), one prompt of 2,048 tokens:
+//   delta rule, 8 heads of 128 x 128 over 4 key heads:  724 -> 102 (27 + 54 + 20; 8,192 tokens: 2,870 -> 373)
+//   linear attention, 16 heads of 64 x 128:             547 -> 75 (37 + 21 + 16; 8,192 tokens: 2,174 -> 333)
+// `states` is a chain: 64 matrix-core instructions of 32 cycles a wavefront and chunk (0.85 us) and two trips through
+// LDS, 1.7 us in all; with operands row by row instead of in operand order and a head's workgroups spread over the
+// dies it took 3.3.  `prepare` and `outputs` are short of workgroups (256) more than of anything else.
+#include "recurrent.h"
+
+#define CK 64                       // tokens a chunk
+#define CK_PAD 4                    // a row in LDS is that much longer: rows start in different banks
+
+typedef float ck_f32x4 __attribute__((ext_vector_type(4)));
+
+struct ChunkArgs {
+    float *out;                     // [T, heads * vdim]
+    float *state;                   // seat rows; S [heads, dim, vdim] at state_off
+    size_t seat_stride;
+    int state_off;
+    const int *entry_q_start, *entry_seat;
+    int heads, kv_heads, vdim;
+    int shortest;                   // entries of fewer tokens are left to the walk
+    float *work;                    // per (chunk, head) a block of ck_block() floats
+};
+
+// A (chunk, head)'s block: W [CK][D], Qd [CK][D], Kd^T [D][CK], P [CK][CK], U^T [vdim][CK], S^T [vdim][D], each in
+// operand order, and G [D].
+__host__ __device__ inline size_t ck_block(int dim, int vdim) {
+    return (size_t)3 * CK * dim + CK * CK + (size_t)vdim * (CK + dim) + dim;
+}
+
+// Operand order: 16 rows x 16 columns at a time as the 64 lanes hold them, lane (row r, group g) the columns 4 g .. 4 g +
+// 3 - so that a wavefront loads and stores 1 KiB of neighbouring bytes (row by row it is 64 bytes of each of 16
+// rows).  A product's result has, in lane (r, g), rows 4 g .. 4 g + 3 of column r: the operand order of its transpose.
+__device__ inline size_t ck_frag(int rowtile, int coltile, int coltiles, int lane) {
+    return ((size_t)(rowtile * coltiles + coltile) * KVA_WAVE + lane) * 4;
+}
+
+template <int D>
+struct ChunkBlock {
+    float *w, *q, *kt, *p, *ut, *st, *g;
+    __device__ inline ChunkBlock(const ChunkArgs &a, int q0, int e, int chunk, int head) {
+        // entry e's chunks begin at q0 / CK + e: sums of ceil(n / CK) never exceed that
+        w = a.work + ((size_t)(q0 / CK + e + chunk) * a.heads + head) * ck_block(D, a.vdim);
+        q = w + CK * D;
+        kt = q + CK * D;
+        p = kt + CK * D;
+        ut = p + CK * CK;
+        st = ut + (size_t)a.vdim * CK;
+        g = st + (size_t)a.vdim * D;
+    }
+};
+
+__device__ inline ck_f32x4 ck_ld(const float *p) { return *reinterpret_cast<const ck_f32x4 *>(p); }
+__device__ inline void ck_st(float *p, ck_f32x4 v) { *reinterpret_cast<ck_f32x4 *>(p) = v; }
+__device__ inline ck_f32x4 ck_mul(ck_f32x4 a, ck_f32x4 b) {
+    return ck_f32x4{a[0] * b[0], a[1] * b[1], a[2] * b[2], a[3] * b[3]};
+}
+__device__ inline ck_f32x4 ck_mul(ck_f32x4 a, float b) { return ck_f32x4{a[0] * b, a[1] * b, a[2] * b, a[3] * b}; }
+// 16 terms of the sums
+__device__ inline ck_f32x4 ck_mfma(ck_f32x4 a, ck_f32x4 b, ck_f32x4 c) {
+#pragma unroll
+    for (int e = 0; e < 4; ++e) c = __builtin_amdgcn_mfma_f32_16x16x4f32(a[e], b[e], c, 0, 0, 0);
+    return c;
+}
+
+// Where q, k, v and the decays come from.
+struct ChunkInput {
+    const float *qkv;               // delta rule: q, k, v after the convolution [T, qkv_stride]
+    const void *y;                  // the projection [T, y_stride]: beta and decay columns; linear attention: q, k, v
+    int qkv_stride, y_dtype, y_stride, q_off, k_off, v_off, beta_off, decay_off, act;
+    const float *a_log, *dt_bias;   // one decay a head and token, from a column of y; or
+    const float *channel_decay;     // one per head, token and key channel [T, decay_stride]; or
+    const float *head_decay;        // one a head
+    int decay_stride;
+    float unit_eps, q_mul;
+};
+
+// One workgroup a (chunk, head), four wavefronts, wavefront b its tokens 16 b .. 16 b + 15.  CD: a decay per key channel.
+// Without, decays are numbers that multiply products of q and k formed without them; with, a lane takes its share of
+// D_ij k_j from token to token inside a block of 16 and blocks meet through their products of decays.
+template <int D, bool DELTA, bool CD>
+__global__ void __launch_bounds__(256)
+chunk_prepare_kernel(ChunkArgs a, ChunkInput in) {
+    constexpr int DS = D + CK_PAD, STEPS = D / 16, TS = CK + CK_PAD;
+    __shared__ __attribute__((aligned(16))) float Q[CK][DS];        // q (CD: then D_i(block start) q)
+    __shared__ __attribute__((aligned(16))) float Kx[CK][DS];       // k (CD: then D_i(block start) k)
+    __shared__ __attribute__((aligned(16))) float Al[CD ? CK : 1][DS];      // decays, then D_(block end)j k
+    __shared__ __attribute__((aligned(16))) float Bt[CD ? 4 : 1][D];        // a block's product of decays
+    __shared__ __attribute__((aligned(16))) float A[DELTA ? CK * CK : 4];   // beta k . D k, operand order
+    __shared__ __attribute__((aligned(16))) float T[DELTA ? CK : 1][TS];    // (1 + A)^-1
+    __shared__ __attribute__((aligned(16))) float Ti[DELTA ? 4 : 1][16][16 + CK_PAD];   // its diagonal blocks
+    __shared__ __attribute__((aligned(16))) float beta[CK], gs[CK], nq[CK], nk[CK];
+    __shared__ float Dd[CD ? 1 : 4][16][17];                        // decays between two tokens of a block
+    __shared__ __attribute__((aligned(16))) float from0[CK];        // D_i0
+    __shared__ float to_end[CK], whole[4];                         // D_Cj; a block's own product
+    const int e = blockIdx.z, head = blockIdx.y, chunk = blockIdx.x;
+    const int q0 = a.entry_q_start[e], n = a.entry_q_start[e + 1] - q0;
+    if (n < a.shortest || chunk * CK >= n) return;
+    const int m = min(CK, n - chunk * CK), row0 = q0 + chunk * CK, kvh = head / (a.heads / a.kv_heads);
+    const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid / KVA_WAVE), lane = tid % KVA_WAVE;
+    const int r = lane % 16, g = lane / 16, b0 = wave * 16;
+    ChunkBlock<D> out(a, q0, e, chunk, head);
+
+    // ---- the chunk's tokens; rows behind the last one are zero (decay 1): they change nothing
+    if (DELTA) {
+        constexpr int PER = CK * D / 4 / 256;
+        ck_f32x4 lq[PER], lk[PER];
+#pragma unroll
+        for (int j = 0; j < PER; ++j) {
+            const int x = tid + 256 * j, t = x / (D / 4), i = x % (D / 4) * 4;
+            const float *row = in.qkv + (size_t)(row0 + min(t, m - 1)) * in.qkv_stride + kvh * D + i;
+            lq[j] = ck_ld(row + in.q_off);
+            lk[j] = ck_ld(row + in.k_off);
+        }
+#pragma unroll
+        for (int j = 0; j < PER; ++j) {
+            const int x = tid + 256 * j, t = x / (D / 4), i = x % (D / 4) * 4;
+            ck_st(&Q[t][i], t < m ? lq[j] : ck_f32x4{0.f, 0.f, 0.f, 0.f});
+            ck_st(&Kx[t][i], t < m ? lk[j] : ck_f32x4{0.f, 0.f, 0.f, 0.f});
+        }
+    } else {
+        constexpr int PER = CK * D / 256, AT = 16;
+        for (int j0 = 0; j0 < PER; j0 += AT) {
+            float lq[AT], lk[AT];
+#pragma unroll
+            for (int j = 0; j < AT; ++j) {
+                const int x = tid + 256 * (j0 + j), t = x / D, i = x % D;
+                const size_t row = (size_t)(row0 + min(t, m - 1)) * in.y_stride + head * D + i;
+                lq[j] = rec_ld(in.y, in.y_dtype, row + in.q_off);
+                lk[j] = rec_ld(in.y, in.y_dtype, row + in.k_off);
+            }
+#pragma unroll
+            for (int j = 0; j < AT; ++j) {
+                const int x = tid + 256 * (j0 + j), t = x / D, i = x % D;
+                Q[t][i] = t < m ? rec_act(lq[j], in.act) * in.q_mul : 0.f;
+                Kx[t][i] = t < m ? rec_act(lk[j], in.act) : 0.f;
+            }
+        }
+    }
+    if (CD) {
+        constexpr int PER = CK * D / 256, AT = 16;
+        for (int j0 = 0; j0 < PER; j0 += AT) {
+            float la[AT];
+#pragma unroll
+            for (int j = 0; j < AT; ++j) {
+                const int x = tid + 256 * (j0 + j), t = x / D, i = x % D;
+                la[j] = in.channel_decay[(size_t)(row0 + min(t, m - 1)) * in.decay_stride + head * D + i];
+            }
+#pragma unroll
+            for (int j = 0; j < AT; ++j) {
+                const int x = tid + 256 * (j0 + j), t = x / D, i = x % D;
+                Al[CD ? t : 0][i] = t < m ? la[j] : 1.f;
+            }
+        }
+    }
+    if (tid < CK) {
+        float b = 0.f, d = 1.f;
+        if (tid < m) {
+            const size_t yrow = (size_t)(row0 + tid) * in.y_stride;
+            if (DELTA) b = rec_sigmoid(rec_ld(in.y, in.y_dtype, yrow + in.beta_off + head));
+            if (in.head_decay) d = in.head_decay[head];
+            else if (!CD)
+                d = expf(-expf(in.a_log[head]) * rec_softplus(rec_ld(in.y, in.y_dtype, yrow + in.decay_off + head) + in.dt_bias[head]));
+        }
+        beta[tid] = b;
+        gs[tid] = d;
+        nq[tid] = nk[tid] = 1.f;
+    }
+    __syncthreads();
+    if (DELTA) {                    // what makes q and k unit vectors (q also times dim^-1/2): four lanes a token
+        const int t = tid / 4, part = tid % 4;
+        ck_f32x4 sq = {0.f, 0.f, 0.f, 0.f}, sk = sq;
+#pragma unroll
+        for (int i = 4 * part; i < D; i += 16) {
+            const ck_f32x4 q = ck_ld(&Q[t][i]), k = ck_ld(&Kx[t][i]);
+#pragma unroll
+            for (int c = 0; c < 4; ++c) {
+                sq[c] += q[c] * q[c];
+                sk[c] += k[c] * k[c];
+            }
+        }
+        float uq = (sq[0] + sq[1]) + (sq[2] + sq[3]), uk = (sk[0] + sk[1]) + (sk[2] + sk[3]);
+        uq += __shfl_xor(uq, 1, KVA_WAVE); uq += __shfl_xor(uq, 2, KVA_WAVE);
+        uk += __shfl_xor(uk, 1, KVA_WAVE); uk += __shfl_xor(uk, 2, KVA_WAVE);
+        uq = in.q_mul / sqrtf(uq + in.unit_eps);
+        uk = 1.0f / sqrtf(uk + in.unit_eps);
+        if (CD) {
+#pragma unroll
+            for (int i = 4 * part; i < D; i += 16) {
+                ck_st(&Q[t][i], ck_mul(ck_ld(&Q[t][i]), uq));
+                ck_st(&Kx[t][i], ck_mul(ck_ld(&Kx[t][i]), uk));
+            }
+        } else if (part == 0) {
+            nq[t] = uq;
+            nk[t] = uk;
+        }
+    }
+    if (!CD && wave == 0) {         // lane (block g, j = r): the decays from token j on, then those before it
+        float d = 0.f, pre = 1.f;
+        for (int i = 0; i < 16; ++i) {
+            const float x = gs[16 * g + i];
+            d = r < i ? d * x : r == i ? 1.f : 0.f;
+            pre = i <= r ? pre * x : pre;
+            Dd[CD ? 0 : g][i][r] = d;
+        }
+        const float b1 = __shfl(pre, 15, KVA_WAVE), b2 = __shfl(pre, 31, KVA_WAVE), b3 = __shfl(pre, 47, KVA_WAVE), b4 = __shfl(pre, 63, KVA_WAVE);
+        const float lead = g == 0 ? 1.f : g == 1 ? b1 : g == 2 ? b1 * b2 : b1 * b2 * b3;
+        const float rest = g == 3 ? 1.f : g == 2 ? b4 : g == 1 ? b3 * b4 : b2 * b3 * b4;
+        from0[lane] = pre * lead;   // (token 16 g + r is `lane`)
+        to_end[lane] = d * rest;
+        if (r == 15) whole[g] = pre;
+    }
+    __syncthreads();
+
+    // ---- P and A
+    if (CD) {
+        // inside a block: lane (j = r, g) takes its share of D_ij k_j from token to token; the sums over the channels that
+        // token i needs with every j are formed side by side
+        ck_f32x4 kd[STEPS], pre[STEPS], mine_q[STEPS], mine_k[STEPS];
+#pragma unroll
+        for (int s = 0; s < STEPS; ++s) {
+            kd[s] = ck_f32x4{0.f, 0.f, 0.f, 0.f};
+            pre[s] = ck_f32x4{1.f, 1.f, 1.f, 1.f};
+            mine_q[s] = ck_ld(&Q[b0 + r][16 * s + 4 * g]);
+            mine_k[s] = ck_ld(&Kx[b0 + r][16 * s + 4 * g]);
+        }
+        for (int i = 0; i < 16; ++i) {
+            float sp[4] = {0.f, 0.f, 0.f, 0.f}, sa[4] = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+            for (int s = 0; s < STEPS; ++s) {
+                const ck_f32x4 al = ck_ld(&Al[CD ? b0 + i : 0][16 * s + 4 * g]), q = ck_ld(&Q[b0 + i][16 * s + 4 * g]), k = ck_ld(&Kx[b0 + i][16 * s + 4 * g]);
+#pragma unroll
+                for (int c = 0; c < 4; ++c) {
+                    pre[s][c] = i <= r ? pre[s][c] * al[c] : pre[s][c];
+                    kd[s][c] = r < i ? kd[s][c] * al[c] : r == i ? k[c] : 0.f;
+                    sp[c] += q[c] * kd[s][c];
+                    if (DELTA) sa[c] += k[c] * kd[s][c];
+                }
+            }
+            const float p = quad_rows_sum((sp[0] + sp[1]) + (sp[2] + sp[3]));       // zero for r > i
+            const size_t at = ck_frag(wave, wave, 4, i + 16 * (r / 4)) + r % 4;
+            if (g == 0) out.p[at] = p;
+            if (DELTA) {
+                const float x = quad_rows_sum((sa[0] + sa[1]) + (sa[2] + sa[3]));
+                if (g == 0) A[DELTA ? at : 0] = r < i ? beta[b0 + i] * x : 0.f;
+            }
+        }
+#pragma unroll
+        for (int s = 0; s < STEPS; ++s) {           // (so far a wavefront has read only its own 16 rows)
+            ck_st(&Q[b0 + r][16 * s + 4 * g], ck_mul(mine_q[s], pre[s]));
+            ck_st(&Kx[b0 + r][16 * s + 4 * g], ck_mul(mine_k[s], pre[s]));
+            ck_st(&Al[CD ? b0 + r : 0][16 * s + 4 * g], kd[s]);
+            if (r == 15) ck_st(&Bt[CD ? wave : 0][16 * s + 4 * g], pre[s]);
+        }
+        __syncthreads();
+    }
+    // tiles (I, J): with CD the six with I > J, without it the diagonal ones too; P's first, then A's.  The result is
+    // formed transposed, [j][i]: lane (i = r, j = 4 g ..), operand order.
+    constexpr int PAIRS = CD ? 6 : 10;
+    for (int task = wave; task < (DELTA ? 2 : 1) * PAIRS; task += 4) {
+        const int pair = task % PAIRS;
+        const bool keys = task >= PAIRS;
+        const int I = pair < 6 ? (pair == 0 ? 1 : pair <= 2 ? 2 : 3) : pair - 6, J = pair < 6 ? (pair == 0 ? 0 : pair <= 2 ? pair - 1 : pair - 3) : pair - 6;
+        ck_f32x4 acc[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
+#pragma unroll
+        for (int s = 0; s < STEPS; ++s) {
+            const ck_f32x4 x = ck_ld(keys ? &Kx[16 * I + r][16 * s + 4 * g] : &Q[16 * I + r][16 * s + 4 * g]);
+            ck_f32x4 k = ck_ld(CD ? &Al[CD ? 16 * J + r : 0][16 * s + 4 * g] : &Kx[16 * J + r][16 * s + 4 * g]);
+            if (CD)
+                for (int b = J + 1; b < I; ++b) k = ck_mul(k, ck_ld(&Bt[CD ? b : 0][16 * s + 4 * g]));
+            acc[s % 2] = ck_mfma(k, x, acc[s % 2]);
+        }
+        const int i = 16 * I + r;
+        float mid = 1.f;                            // the product of the blocks between
+        if (!CD)
+            for (int b = J + 1; b < I; ++b) mid *= whole[b];
+        ck_f32x4 v;
+#pragma unroll
+        for (int c = 0; c < 4; ++c) {
+            const int jj = 4 * g + c;
+            v[c] = acc[0][c] + acc[1][c];
+            if (!CD) {
+                // D_ij: to the end of j's block, the blocks between, from the start of i's
+                const float d = I == J ? Dd[CD ? 0 : I][r][jj] : Dd[CD ? 0 : J][15][jj] * mid * (Dd[CD ? 0 : I][r][0] * gs[16 * I]);
+                v[c] *= d * nk[16 * J + jj] * (keys ? nk[i] : nq[i]);
+            }
+            if (keys) v[c] = I == J && jj >= r ? 0.f : v[c] * beta[i];
+        }
+        if (keys) { if (DELTA) ck_st(&A[DELTA ? ck_frag(I, J, 4, lane) : 0], v); }
+        else ck_st(out.p + ck_frag(I, J, 4, lane), v);
+    }
+    __syncthreads();
+
+    // ---- Qd, Kd^T, G
+    for (int x = wave; x < 4 * STEPS; x += 4) {
+        const int I = x / STEPS, s = x % STEPS;
+        ck_f32x4 q = ck_ld(&Q[16 * I + r][16 * s + 4 * g]);
+        if (CD) for (int b = 0; b < I; ++b) q = ck_mul(q, ck_ld(&Bt[CD ? b : 0][16 * s + 4 * g]));
+        else q = ck_mul(q, nq[16 * I + r] * from0[16 * I + r]);
+        ck_st(out.q + ck_frag(I, s, STEPS, lane), q);
+    }
+    for (int x = wave; x < 4 * STEPS; x += 4) {
+        const int J = x % 4, c0 = x / 4 * 16;
+        ck_f32x4 k;
+        float rest = 1.f;
+        if (CD) for (int b = J + 1; b < 4; ++b) rest *= Bt[CD ? b : 0][c0 + r];
+#pragma unroll
+        for (int c = 0; c < 4; ++c) {
+            const int j = 16 * J + 4 * g + c;
+            k[c] = CD ? Al[CD ? j : 0][c0 + r] * rest : Kx[j][c0 + r] * (nk[j] * to_end[j]);
+        }
+        ck_st(out.kt + ck_frag(x / 4, J, 4, lane), k);
+    }
+    if (tid < D) out.g[tid] = CD ? Bt[0][tid] * Bt[CD ? 1 : 0][tid] * Bt[CD ? 2 : 0][tid] * Bt[CD ? 3 : 0][tid] : from0[CK - 1];
+
+    const size_t vrow = DELTA ? (size_t)in.qkv_stride : (size_t)in.y_stride;
+    auto values = [&](int col, ck_f32x4(&v)[4]) {           // tokens 16 s + 4 g .. of a value column
+#pragma unroll
+        for (int s = 0; s < 4; ++s)
+#pragma unroll
+            for (int c = 0; c < 4; ++c) {
+                const int t = 16 * s + 4 * g + c;
+                const size_t at = (size_t)(row0 + min(t, m - 1)) * vrow + in.v_off + head * a.vdim + col;
+                v[s][c] = DELTA ? in.qkv[at] : rec_ld(in.y, in.y_dtype, at);
+            }
+#pragma unroll
+        for (int s = 0; s < 4; ++s)
+#pragma unroll
+            for (int c = 0; c < 4; ++c) {
+                if (!DELTA) v[s][c] = rec_act(v[s][c], in.act);
+                if (16 * s + 4 * g + c >= m) v[s][c] = 0.f;
+            }
+    };
+    if (!DELTA) {                   // U is V
+        for (int tile = wave; tile < a.vdim / 16; tile += 4) {
+            ck_f32x4 v[4];
+            values(16 * tile + r, v);
+#pragma unroll
+            for (int s = 0; s < 4; ++s) ck_st(out.ut + ck_frag(tile, s, 4, lane), v[s]);
+        }
+        return;
+    }
+
+    // ---- T = (1 + A)^-1: its diagonal blocks, column r by forward substitution ...
+    if (g == 0) {
+        float x[16];
+#pragma unroll
+        for (int i = 0; i < 16; ++i) {
+            float s = i == r ? 1.f : 0.f;
+#pragma unroll
+            for (int j = 0; j < i; ++j) s -= A[DELTA ? ck_frag(wave, wave, 4, i + 16 * (j / 4)) + j % 4 : 0] * x[j];
+            x[i] = s;
+            Ti[DELTA ? wave : 0][i][r] = s;
+        }
+    }
+    __syncthreads();
+    // ... then T_IJ = -T_II sum_{J<=K<I} A_IK T_KJ, wavefront J its block column, results being the next products' operands
+    {
+        const int J = wave;
+        ck_f32x4 col[4];            // T_IJ for I = J .. 3: lane (column r, rows 4 g ..)
+#pragma unroll
+        for (int I = 0; I < 4; ++I) {
+            ck_f32x4 t = {0.f, 0.f, 0.f, 0.f};
+            if (I == J) {
+#pragma unroll
+                for (int c = 0; c < 4; ++c) t[c] = Ti[DELTA ? J : 0][4 * g + c][r];
+            } else if (I > J) {
+                ck_f32x4 sum = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+                for (int K = 0; K < I; ++K)
+                    if (K >= J) sum = ck_mfma(ck_ld(&A[DELTA ? ck_frag(I, K, 4, lane) : 0]), col[K], sum);
+                t = ck_mfma(ck_ld(&Ti[DELTA ? I : 0][r][4 * g]), sum, t);
+#pragma unroll
+                for (int c = 0; c < 4; ++c) t[c] = -t[c];
+            }
+            col[I] = t;
+#pragma unroll
+            for (int c = 0; c < 4; ++c) T[DELTA ? 16 * I + 4 * g + c : 0][16 * J + r] = t[c];
+        }
+    }
+    __syncthreads();
+    // ---- W = T (beta D_0 k), transposed: lane (i = r, channels 4 g ..); Uv = T (beta v): lane (column r, tokens 4 g ..)
+    ck_f32x4 bj[4], wj[4];          // what token j's row is multiplied by
+#pragma unroll
+    for (int J = 0; J < 4; ++J) {
+        bj[J] = ck_ld(&beta[16 * J + 4 * g]);
+        wj[J] = CD ? bj[J] : ck_mul(ck_mul(bj[J], ck_ld(&nk[16 * J + 4 * g])), ck_ld(&from0[16 * J + 4 * g]));
+    }
+    for (int tile = wave; tile < STEPS; tile += 4) {
+        ck_f32x4 k[4];
+        float lead = 1.f;
+#pragma unroll
+        for (int J = 0; J < 4; ++J) {
+#pragma unroll
+            for (int c = 0; c < 4; ++c) k[J][c] = Kx[16 * J + 4 * g + c][16 * tile + r] * lead * wj[J][c];
+            if (CD) lead *= Bt[CD ? J : 0][16 * tile + r];
+        }
+#pragma unroll
+        for (int I = 0; I < 4; ++I) {
+            ck_f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+            for (int J = 0; J <= I; ++J) acc = ck_mfma(k[J], ck_ld(&T[DELTA ? 16 * I + r : 0][16 * J + 4 * g]), acc);
+            ck_st(out.w + ck_frag(I, tile, STEPS, lane), acc);
+        }
+    }
+    for (int tile = wave; tile < a.vdim / 16; tile += 4) {
+        ck_f32x4 v[4];
+        values(16 * tile + r, v);
+#pragma unroll
+        for (int J = 0; J < 4; ++J) v[J] = ck_mul(v[J], bj[J]);
+#pragma unroll
+        for (int I = 0; I < 4; ++I) {
+            ck_f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+            for (int J = 0; J <= I; ++J) acc = ck_mfma(ck_ld(&T[DELTA ? 16 * I + r : 0][16 * J + 4 * g]), v[J], acc);
+            ck_st(out.ut + ck_frag(tile, I, 4, lane), acc);
+        }
+    }
+}
+
+// One workgroup a (request, head, 16 value columns), chunk after chunk.  A wavefront keeps D / 64 tiles of 16 rows of
+// S's columns in registers, all of S^T [16][D] stands in LDS for U = Uv - W S, of which a wavefront makes 16
+// tokens; U^T goes through LDS to S <- G S + Kd^T U.  The next chunk's operands are on their way over a chunk.  A
+// head's workgroups are `heads` apart in the launch: on one die where the heads are a multiple of eight, so that W
+// and Kd come from memory once.
+template <int D, bool DELTA>
+__global__ void __launch_bounds__(256)
+chunk_states_kernel(ChunkArgs a) {
+    constexpr int STEPS = D / 16, MT = D / 64;
+    __shared__ __attribute__((aligned(16))) float St[16 * D];       // operand order
+    __shared__ __attribute__((aligned(16))) float Ut[16 * CK];
+    const int e = blockIdx.y, head = blockIdx.x % a.heads, tile = blockIdx.x / a.heads;
+    const int q0 = a.entry_q_start[e], n = a.entry_q_start[e + 1] - q0;
+    if (n < a.shortest) return;
+    const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid / KVA_WAVE), lane = tid % KVA_WAVE;
+    const int r = lane % 16, g = lane / 16, chunks = (n + CK - 1) / CK, col = 16 * tile + r;
+    float *Sg = a.state + (size_t)a.entry_seat[e] * a.seat_stride + a.state_off + (size_t)head * D * a.vdim;
+    ck_f32x4 S[MT];                 // rows 16 (wave MT + t) + 4 g .. + 3 of the column
+#pragma unroll
+    for (int t = 0; t < MT; ++t)
+#pragma unroll
+        for (int c = 0; c < 4; ++c) S[t][c] = Sg[(size_t)(16 * (wave * MT + t) + 4 * g + c) * a.vdim + col];
+    struct Operands {
+        ck_f32x4 w[DELTA ? STEPS : 1], kt[MT][CK / 16], uv, dec[MT];
+    } o[2];
+    auto fetch = [&](Operands &x, int chunk) {
+        const ChunkBlock<D> b(a, q0, e, min(chunk, chunks - 1), head);
+        x.uv = ck_ld(b.ut + ck_frag(tile, wave, 4, lane));
+        if (DELTA)
+#pragma unroll
+            for (int s = 0; s < STEPS; ++s) x.w[DELTA ? s : 0] = ck_ld(b.w + ck_frag(wave, s, STEPS, lane));
+#pragma unroll
+        for (int t = 0; t < MT; ++t) {
+#pragma unroll
+            for (int s = 0; s < CK / 16; ++s) x.kt[t][s] = ck_ld(b.kt + ck_frag(wave * MT + t, s, 4, lane));
+            x.dec[t] = ck_ld(b.g + 16 * (wave * MT + t) + 4 * g);
+        }
+    };
+    auto step = [&](const Operands &x, Operands &next, int chunk) {
+        const ChunkBlock<D> b(a, q0, e, chunk, head);
+#pragma unroll
+        for (int t = 0; t < MT; ++t) {
+            if (DELTA) ck_st(&St[ck_frag(0, wave * MT + t, STEPS, lane)], S[t]);
+            ck_st(b.st + ck_frag(tile, wave * MT + t, STEPS, lane), S[t]);
+        }
+        __syncthreads();
+        fetch(next, chunk + 1);
+        ck_f32x4 u = x.uv;
+        if (DELTA) {
+            // two chains of products: one alone waits for its own results
+            ck_f32x4 y[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
+#pragma unroll
+            for (int s = 0; s < STEPS; ++s) y[s % 2] = ck_mfma(x.w[DELTA ? s : 0], ck_ld(&St[ck_frag(0, s, STEPS, lane)]), y[s % 2]);
+#pragma unroll
+            for (int c = 0; c < 4; ++c) u[c] -= y[0][c] + y[1][c];
+            ck_st(b.ut + ck_frag(tile, wave, 4, lane), u);
+        }
+        ck_st(&Ut[ck_frag(0, wave, 4, lane)], u);
+        __syncthreads();
+#pragma unroll
+        for (int t = 0; t < MT; ++t) S[t] = ck_mul(S[t], x.dec[t]);
+#pragma unroll
+        for (int s = 0; s < CK / 16; ++s) {
+            const ck_f32x4 y = ck_ld(&Ut[ck_frag(0, s, 4, lane)]);
+#pragma unroll
+            for (int t = 0; t < MT; ++t) S[t] = ck_mfma(x.kt[t][s], y, S[t]);
+        }
+    };
+    fetch(o[0], 0);
+    for (int chunk = 0; chunk < chunks; chunk += 2) {
+        step(o[0], o[1], chunk);
+        if (chunk + 1 < chunks) step(o[1], o[0], chunk + 1);
+    }
+#pragma unroll
+    for (int t = 0; t < MT; ++t)
+#pragma unroll
+        for (int c = 0; c < 4; ++c) Sg[(size_t)(16 * (wave * MT + t) + 4 * g + c) * a.vdim + col] = S[t][c];
+}
+
+// One workgroup a (chunk, head), a wavefront every fourth 32 value columns, for all 64 tokens: O = Qd S + P U, every
+// operand from where the other two kernels left it, in operand order.
+template <int D>
+__global__ void __launch_bounds__(256)
+chunk_outputs_kernel(ChunkArgs a) {
+    constexpr int STEPS = D / 16;
+    const int e = blockIdx.z, head = blockIdx.y, chunk = blockIdx.x;
+    const int q0 = a.entry_q_start[e], n = a.entry_q_start[e + 1] - q0;
+    if (n < a.shortest || chunk * CK >= n) return;
+    const int m = min(CK, n - chunk * CK), row0 = q0 + chunk * CK, tiles = a.vdim / 16;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / KVA_WAVE), lane = threadIdx.x % KVA_WAVE, r = lane % 16, g = lane / 16;
+    const ChunkBlock<D> b(a, q0, e, chunk, head);
+    for (int tile = 2 * wave; tile < tiles; tile += 8) {
+        const int second = min(tile + 1, tiles - 1);        // (an odd last tile twice: the second result is dropped)
+        ck_f32x4 acc[CK / 16][2];
+#pragma unroll
+        for (int t = 0; t < CK / 16; ++t) acc[t][0] = acc[t][1] = ck_f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll 4
+        for (int s = 0; s < STEPS; ++s) {
+            const ck_f32x4 x = ck_ld(b.st + ck_frag(tile, s, STEPS, lane)), y = ck_ld(b.st + ck_frag(second, s, STEPS, lane));
+#pragma unroll
+            for (int t = 0; t < CK / 16; ++t) {
+                const ck_f32x4 q = ck_ld(b.q + ck_frag(t, s, STEPS, lane));
+                acc[t][0] = ck_mfma(q, x, acc[t][0]);
+                acc[t][1] = ck_mfma(q, y, acc[t][1]);
+            }
+        }
+#pragma unroll
+        for (int s = 0; s < CK / 16; ++s) {
+            const ck_f32x4 x = ck_ld(b.ut + ck_frag(tile, s, 4, lane)), y = ck_ld(b.ut + ck_frag(second, s, 4, lane));
+#pragma unroll
+            for (int t = s; t < CK / 16; ++t) {             // (P has no blocks above its diagonal)
+                const ck_f32x4 p = ck_ld(b.p + ck_frag(t, s, 4, lane));
+                acc[t][0] = ck_mfma(p, x, acc[t][0]);
+                acc[t][1] = ck_mfma(p, y, acc[t][1]);
+            }
+        }
+#pragma unroll
+        for (int t = 0; t < CK / 16; ++t)
+#pragma unroll
+            for (int c = 0; c < 4; ++c) {
+                const int i = 16 * t + 4 * g + c;
+                float *o = a.out + (size_t)(row0 + i) * a.heads * a.vdim + head * a.vdim + r;
+                if (i < m) {
+                    o[16 * tile] = acc[t][0][c];
+                    if (tile + 1 < tiles) o[16 * (tile + 1)] = acc[t][1][c];
+                }
+            }
+    }
+}
+
+// Sizes these kernels are built for; other ones walk.
+static bool ck_fits(int dim, int vdim) { return (dim == 64 || dim == 128) && vdim > 0 && vdim % 16 == 0; }
+
+// floats of workspace for a step of `tokens` tokens in `entries` entries; 0: not for these sizes
+extern "C" long long kva_recurrent_chunks_workspace(int tokens, int entries, int heads, int dim, int vdim) {
+    if (!ck_fits(dim, vdim) || tokens < 0 || entries < 0 || heads <= 0) return 0;
+    return (long long)(tokens / CK + entries) * heads * (long long)ck_block(dim, vdim);
+}
+
+template <int D, bool DELTA>
+static void ck_launch(const ChunkArgs &a, const ChunkInput &in, int longest, int entries, hipStream_t stream) {
+    const dim3 grid((longest + CK - 1) / CK, a.heads, entries);
+    if (in.channel_decay) hipLaunchKernelGGL((chunk_prepare_kernel<D, DELTA, true>), grid, dim3(256), 0, stream, a, in);
+    else hipLaunchKernelGGL((chunk_prepare_kernel<D, DELTA, false>), grid, dim3(256), 0, stream, a, in);
+    hipLaunchKernelGGL((chunk_states_kernel<D, DELTA>), dim3(a.heads * (a.vdim / 16), entries), dim3(256), 0, stream, a);
+    hipLaunchKernelGGL(chunk_outputs_kernel<D>, grid, dim3(256), 0, stream, a);
+}
+
+static int ck_check(const char *what, const ChunkArgs &a, int dim, int longest, int entries, int tokens, long long work_floats) {
+    KVA_REQUIRE(a.out && a.state && a.entry_q_start && a.entry_seat && a.work, "%s: missing operand", what);
+    KVA_REQUIRE(ck_fits(dim, a.vdim), "%s: chunks are built for key sizes 64 and 128 and value sizes that are multiples of 16, not %d x %d", what, dim, a.vdim);
+    KVA_REQUIRE(a.heads > 0 && a.heads <= 65535 && a.kv_heads > 0 && a.heads % a.kv_heads == 0, "%s: %d heads over %d key heads", what, a.heads, a.kv_heads);
+    KVA_REQUIRE(entries > 0 && entries <= 65535 && longest > 0 && longest <= tokens && a.shortest >= 1, "%s: %d entries of up to %d tokens", what, entries, longest);
+    KVA_REQUIRE((uintptr_t)a.work % 16 == 0, "%s: the workspace must start at a multiple of 16 bytes", what);
+    KVA_REQUIRE(a.heads * (long long)(a.vdim / 16) < (1LL << 31), "%s: %d heads of %d values", what, a.heads, a.vdim);
+    KVA_REQUIRE(work_floats >= kva_recurrent_chunks_workspace(tokens, entries, a.heads, dim, a.vdim), "%s: the workspace is too small", what);
+    return KVA_OK;
+}
+
+// The same operands as kva_gated_delta_rule; entries of fewer than `shortest` tokens are left alone, no entry has more
+// than `longest` of the step's `tokens`.
+extern "C" int kva_gated_delta_rule_chunks(float *out, float *state, long long seat_stride, int state_off, const float *qkv,
+                                           int conv_stride, const void *y, int y_dtype, int y_stride, int beta_off,
+                                           int decay_off, const float *a_log, const float *dt_bias, float unit_eps,
+                                           const float *channel_decay, int decay_stride, const int *entry_q_start,
+                                           const int *entry_seat, int entries, int heads, int kv_heads, int dim, int vdim,
+                                           int tokens, int shortest, int longest, float *work, long long work_floats,
+                                           hipStream_t stream) {
+    const ChunkArgs a{out, state, (size_t)seat_stride, state_off, entry_q_start, entry_seat, heads, kv_heads, vdim, shortest, work};
+    if (int rc = ck_check("gated_delta_rule", a, dim, longest, entries, tokens, work_floats)) return rc;
+    KVA_REQUIRE(qkv && y && ((a_log && dt_bias) || (channel_decay && decay_stride >= heads * dim)), "gated_delta_rule: missing operand");
+    KVA_REQUIRE((uintptr_t)qkv % 16 == 0 && conv_stride % 4 == 0, "gated_delta_rule: rows of q, k and v must start at multiples of 16 bytes");
+    const ChunkInput in{qkv, y, conv_stride, y_dtype, y_stride, 0, kv_heads * dim, 2 * kv_heads * dim, beta_off, decay_off, 0,
+                        a_log, dt_bias, channel_decay, nullptr, decay_stride, unit_eps, 1.0f / sqrtf((float)dim)};
+    if (dim == 64) ck_launch<64, true>(a, in, longest, entries, stream);
+    else ck_launch<128, true>(a, in, longest, entries, stream);
+    KVA_CHECK_LAUNCH("gated_delta_rule_chunks");
+    return KVA_OK;
+}
+
+// The same operands as kva_gated_linear_attention.
+extern "C" int kva_gated_linear_attention_chunks(float *out, float *state, long long seat_stride, int state_off,
+                                                 const void *y, int y_dtype, int y_stride, int q_off, int k_off, int v_off,
+                                                 const float *alpha, int alpha_stride, float q_mul, const float *head_decay,
+                                                 int act, const int *entry_q_start, const int *entry_seat, int entries,
+                                                 int heads, int dim, int vdim, int tokens, int shortest, int longest,
+                                                 float *work, long long work_floats, hipStream_t stream) {
+    const ChunkArgs a{out, state, (size_t)seat_stride, state_off, entry_q_start, entry_seat, heads, heads, vdim, shortest, work};
+    if (int rc = ck_check("gated_linear_attention", a, dim, longest, entries, tokens, work_floats)) return rc;
+    KVA_REQUIRE(y && ((alpha && alpha_stride >= heads * dim) || (!alpha && head_decay)), "gated_linear_attention: missing operand");
+    KVA_REQUIRE(act == 0 || act == 1, "gated_linear_attention: activation %d is neither none (0) nor silu (1)", act);
+    const ChunkInput in{nullptr, y, 0, y_dtype, y_stride, q_off, k_off, v_off, 0, 0, act, nullptr, nullptr, alpha, head_decay,
+                        alpha_stride, 0.f, q_mul};
+    if (dim == 64) ck_launch<64, false>(a, in, longest, entries, stream);
+    else ck_launch<128, false>(a, in, longest, entries, stream);
+    KVA_CHECK_LAUNCH("gated_linear_attention_chunks");
+    return KVA_OK;
+}

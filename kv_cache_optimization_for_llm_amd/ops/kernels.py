@@ -1722,10 +1722,43 @@ def causal_conv_act(y: torch.Tensor, col_off: int, weight: torch.Tensor, out: to
     return out
 
 
+# Under bf16 projections an entry of so many tokens and more goes through the recurrence in chunks of 64.  The walk takes
+# about 0.35 us a token with the delta rule (8 heads of 128 x 128) and 0.2 with linear attention (16 of 64 x 128), the
+# chunks' three launches 37 and 30 us for a first chunk: 64 / 128 / 2,048 tokens 27 / 49 / 724 against 37 / 42 / 102 us,
+# and 16 / 27 / 547 against 31 / 32 / 75.
+DELTA_RULE_CHUNKS_FROM = 96
+LINEAR_ATTENTION_CHUNKS_FROM = 160
+
+
+def recurrent_chunk_floats(dim: int, vdim: int) -> int:
+    """Floats of workspace a chunk of 64 tokens takes per head (csrc/recurrent_chunks.hip: ``ck_block``)."""
+    return 3 * 64 * dim + 64 * 64 + vdim * (64 + dim) + dim
+
+
+def _recurrent_plan(lengths, chunks_from: int, entries: int, tokens: int, heads: int, dim: int, vdim: int,
+                    dtype: torch.dtype, what: str):
+    """(entries from this many tokens on go in chunks, the longest entry, floats of workspace, whether any entry walks) for
+    entries of ``lengths`` tokens (host numbers; ``None``: not known, all walk)."""
+    if lengths is None:
+        return 1 << 30, 0, 0, True
+    lengths = [int(n) for n in lengths]
+    if len(lengths) != entries or sum(lengths) != tokens:
+        raise KernelError(f"{what}: one length per entry, of all the rows together")
+    longest, shortest = max(lengths, default=0), min(lengths, default=0)
+    work = 0
+    # (32-bit projections: a token's bits do not depend on how its request was cut, so they walk)
+    if dtype == torch.bfloat16 and longest >= chunks_from:
+        work = int(hip_lib().kva_recurrent_chunks_workspace(tokens, entries, heads, dim, vdim))
+    if work == 0:
+        return 1 << 30, 0, 0, True
+    return int(chunks_from), longest, work, shortest < chunks_from
+
+
 def gated_delta_rule(qkv: torch.Tensor, y: torch.Tensor, beta_off: int, decay_off: int, a_log: Optional[torch.Tensor],
                      dt_bias: Optional[torch.Tensor], out: torch.Tensor, state: torch.Tensor, state_off: int,
                      entry_q_start: torch.Tensor, entry_seat: torch.Tensor, heads: int, kv_heads: int, dim: int,
-                     vdim: int, unit_eps: float = 1e-6, channel_decay: Optional[torch.Tensor] = None) -> torch.Tensor:
+                     vdim: int, unit_eps: float = 1e-6, channel_decay: Optional[torch.Tensor] = None,
+                     lengths=None) -> torch.Tensor:
     """Per head and token, in order: ``S <- g S; u = beta (v - S^T k); S <- S + k u^T; o = S^T q`` with
     q and k made unit vectors (``x / sqrt(sum x^2 + unit_eps)``, q also times ``dim^-1/2``),
     ``beta = sigmoid(y[t, beta_off + h])`` and ``g = exp(-exp(a_log[h]) softplus(y[t, decay_off + h] +
@@ -1735,7 +1768,9 @@ def gated_delta_rule(qkv: torch.Tensor, y: torch.Tensor, beta_off: int, decay_of
 
     ``channel_decay`` (fp32 ``[T, heads * dim]``, e.g. from :func:`small_product_f32` with ``rate_log``):
     the decay has one value per head and key channel and multiplies the rows of ``S`` one by one,
-    ``S <- diag(g) S``; ``decay_off``, ``a_log`` and ``dt_bias`` are then not used."""
+    ``S <- diag(g) S``; ``decay_off``, ``a_log`` and ``dt_bias`` are then not used.
+
+    ``lengths``: the entries' numbers of tokens on the host; with bf16 ``y`` long entries then go in chunks."""
     tokens = out.shape[0]
     if qkv.shape != (tokens, 2 * kv_heads * dim + heads * vdim) or qkv.dtype != torch.float32 \
             or out.shape != (tokens, heads * vdim) or out.dtype != torch.float32 or y.dim() != 2 or y.shape[0] != tokens:
@@ -1751,19 +1786,27 @@ def gated_delta_rule(qkv: torch.Tensor, y: torch.Tensor, beta_off: int, decay_of
         raise KernelError("gated_delta_rule: decay columns inside y, one rate and one bias per head")
     seat_stride = _state_row(state, state_off, heads * dim * vdim, "gated_delta_rule")
     qs, seat, entries = _entries((entry_q_start, entry_seat), "gated_delta_rule")
-    check(hip_lib().kva_gated_delta_rule(
-        _dev(out, "out"), _dev(state, "state"), seat_stride, int(state_off), _dev(qkv, "qkv"), qkv.shape[1],
-        _dev(y, "y"), dtype_code(y.dtype), y.shape[1], int(beta_off), int(decay_off),
-        _opt(a_log, "a_log", torch.float32), _opt(dt_bias, "dt_bias", torch.float32), float(unit_eps),
-        _opt(channel_decay, "channel_decay"), channel_decay.shape[1] if channel_decay is not None else 0, qs, seat,
-        entries, heads, kv_heads, dim, vdim, _stream()), "gated_delta_rule")
+    below, longest, floats, walks = _recurrent_plan(lengths, DELTA_RULE_CHUNKS_FROM, entries, tokens, heads, dim, vdim, y.dtype,
+                                                    "gated_delta_rule")
+    operands = (_dev(out, "out"), _dev(state, "state"), seat_stride, int(state_off), _dev(qkv, "qkv"), qkv.shape[1],
+                _dev(y, "y"), dtype_code(y.dtype), y.shape[1], int(beta_off), int(decay_off),
+                _opt(a_log, "a_log", torch.float32), _opt(dt_bias, "dt_bias", torch.float32), float(unit_eps),
+                _opt(channel_decay, "channel_decay"), channel_decay.shape[1] if channel_decay is not None else 0, qs, seat,
+                entries, heads, kv_heads, dim, vdim)
+    if floats:
+        work = torch.empty(floats, dtype=torch.float32, device=out.device)
+        check(hip_lib().kva_gated_delta_rule_chunks(*operands, tokens, below, longest, _dev(work, "work"), floats, _stream()),
+              "gated_delta_rule")
+    if walks:
+        check(hip_lib().kva_gated_delta_rule(*operands, below, _stream()), "gated_delta_rule")
     return out
 
 
 def gated_linear_attention(y: torch.Tensor, q_off: int, k_off: int, v_off: int, alpha: Optional[torch.Tensor], q_mul: float,
                            out: torch.Tensor, state: torch.Tensor, state_off: int, entry_q_start: torch.Tensor,
                            entry_seat: torch.Tensor, heads: int, dim: int, vdim: int,
-                           head_decay: Optional[torch.Tensor] = None, activation: Optional[str] = None) -> torch.Tensor:
+                           head_decay: Optional[torch.Tensor] = None, activation: Optional[str] = None,
+                           lengths=None) -> torch.Tensor:
     """Per head and token, in order: ``S <- diag(alpha) S + k v^T; o = S^T (q_mul q)`` with a decay per
     key channel ``alpha`` (fp32 ``[T, heads * dim]``; :func:`small_product_f32` makes it from a low-rank
     projection).  q, k (``heads x dim``) and v (``heads x vdim``) are columns of ``y`` from ``q_off``,
@@ -1771,7 +1814,8 @@ def gated_linear_attention(y: torch.Tensor, q_off: int, k_off: int, v_off: int, 
 
     ``alpha=None`` with ``head_decay`` (fp32 ``[heads]``): one fixed decay a head for all its channels
     and every token, ``S <- decay_h S + k v^T``.  ``activation="silu"``: q, k and v pass a silu (in
-    fp32) on their way in."""
+    fp32) on their way in.  ``lengths``: the entries' numbers of tokens on the host; with bf16 ``y`` long entries then go
+    in chunks."""
     tokens = out.shape[0]
     if y.dim() != 2 or y.shape[0] != tokens or out.shape != (tokens, heads * vdim) or out.dtype != torch.float32:
         raise KernelError(f"gated_linear_attention: y {tuple(y.shape)}, out {tuple(out.shape)} do not fit")
@@ -1787,11 +1831,18 @@ def gated_linear_attention(y: torch.Tensor, q_off: int, k_off: int, v_off: int, 
             raise KernelError("gated_linear_attention: q, k or v columns lie outside y")
     seat_stride = _state_row(state, state_off, heads * dim * vdim, "gated_linear_attention")
     qs, seat, entries = _entries((entry_q_start, entry_seat), "gated_linear_attention")
-    check(hip_lib().kva_gated_linear_attention(
-        _dev(out, "out"), _dev(state, "state"), seat_stride, int(state_off), _dev(y, "y"), dtype_code(y.dtype),
-        y.shape[1], int(q_off), int(k_off), int(v_off), _opt(alpha, "alpha"), alpha.shape[1] if alpha is not None else 0,
-        float(q_mul), _opt(head_decay, "head_decay"), 1 if activation == "silu" else 0, qs, seat,
-        entries, heads, dim, vdim, _stream()), "gated_linear_attention")
+    below, longest, floats, walks = _recurrent_plan(lengths, LINEAR_ATTENTION_CHUNKS_FROM, entries, tokens, heads, dim, vdim,
+                                                    y.dtype, "gated_linear_attention")
+    operands = (_dev(out, "out"), _dev(state, "state"), seat_stride, int(state_off), _dev(y, "y"), dtype_code(y.dtype),
+                y.shape[1], int(q_off), int(k_off), int(v_off), _opt(alpha, "alpha"), alpha.shape[1] if alpha is not None else 0,
+                float(q_mul), _opt(head_decay, "head_decay"), 1 if activation == "silu" else 0, qs, seat,
+                entries, heads, dim, vdim)
+    if floats:
+        work = torch.empty(floats, dtype=torch.float32, device=out.device)
+        check(hip_lib().kva_gated_linear_attention_chunks(*operands, tokens, below, longest, _dev(work, "work"), floats, _stream()),
+              "gated_linear_attention")
+    if walks:
+        check(hip_lib().kva_gated_linear_attention(*operands, below, _stream()), "gated_linear_attention")
     return out
 
 

@@ -47,6 +47,11 @@ def _names(defaults: Dict[str, str], given: Optional[Dict[str, str]], prefix: st
     return {key: prefix + name for key, name in names.items()}
 
 
+def _chunk_elements(mixer) -> int:
+    """Elements a token that the recurrence's kernels for long entries keep per chunk of 64 tokens."""
+    return mixer.num_heads * -(-K.recurrent_chunk_floats(mixer.head_dim, mixer.value_dim) // 64)
+
+
 @MIXERS.register("gated_linear_attention")
 class GatedLinearAttention(ProjectedMixer):
     graph_safe = True
@@ -104,7 +109,7 @@ class GatedLinearAttention(ProjectedMixer):
         return self.num_heads * self.head_dim * self.value_dim
 
     def activation_elements(self) -> int:
-        return 3 * self.num_heads * self.head_dim + 5 * self.inner_width + self.hidden_size
+        return 3 * self.num_heads * self.head_dim + 5 * self.inner_width + self.hidden_size + _chunk_elements(self)
 
     def forward_inner(self, y, col0, ctx: MixerContext, state_off, out, out_col0, mul) -> None:
         batch, T = ctx.batch, y.shape[0]
@@ -115,7 +120,7 @@ class GatedLinearAttention(ProjectedMixer):
         o = torch.empty((T, self.inner_width), dtype=torch.float32, device=y.device)
         K.gated_linear_attention(y, col0 + self.q_off, col0 + self.k_off, col0 + self.v_off, alpha, self.query_scale, o,
                                  ctx.state, state_off, batch.entry_q_start, batch.entry_seat, self.num_heads,
-                                 self.head_dim, self.value_dim)
+                                 self.head_dim, self.value_dim, lengths=np.diff(batch.h_entry_q_start))
         K.head_norm_gate(o, self.norm_weight, self.norm_eps, y, col0 + self.g_off, out, out_col0, self.num_heads,
                          self.value_dim, "silu", mul)
 
@@ -227,10 +232,11 @@ class GatedDeltaRule(ProjectedMixer):
         return self.num_heads * self.head_dim * self.value_dim + self.conv_channels * (self.conv_taps - 1)
 
     def activation_elements(self) -> int:
-        return 3 * self.conv_channels + 4 * self.inner_width + self.hidden_size
+        return 3 * self.conv_channels + 4 * self.inner_width + self.hidden_size + _chunk_elements(self)
 
     def forward_inner(self, y, col0, ctx: MixerContext, state_off, out, out_col0, mul) -> None:
         batch, T = ctx.batch, y.shape[0]
+        lengths = np.diff(batch.h_entry_q_start)
         s_elems = self.num_heads * self.head_dim * self.value_dim
         qkv = torch.empty((T, self.conv_channels), dtype=torch.float32, device=y.device)
         K.causal_conv_act(y, col0, self.conv_weight, qkv, ctx.state, state_off + s_elems, batch.entry_q_start,
@@ -244,11 +250,11 @@ class GatedDeltaRule(ProjectedMixer):
                                     bias=self.dt_bias, rate_log=self.a_log)
             K.gated_delta_rule(qkv, y, col0 + self.beta_off, 0, None, None, o, ctx.state, state_off,
                                batch.entry_q_start, batch.entry_seat, self.num_heads, self.num_kv_heads,
-                               self.head_dim, self.value_dim, self.unit_eps, channel_decay=g)
+                               self.head_dim, self.value_dim, self.unit_eps, channel_decay=g, lengths=lengths)
         else:
             K.gated_delta_rule(qkv, y, col0 + self.beta_off, col0 + self.decay_off, self.a_log, self.dt_bias, o,
                                ctx.state, state_off, batch.entry_q_start, batch.entry_seat, self.num_heads,
-                               self.num_kv_heads, self.head_dim, self.value_dim, self.unit_eps)
+                               self.num_kv_heads, self.head_dim, self.value_dim, self.unit_eps, lengths=lengths)
         if self.low_rank_gate:
             g0 = col0 + self.g_off
             gate, gate_off = self.g2(y[:, g0:g0 + self.gate_cols].contiguous()), 0
@@ -309,14 +315,15 @@ class LightningAttention(ProjectedMixer):
         return self.num_heads * self.head_dim * self.value_dim
 
     def activation_elements(self) -> int:
-        return 2 * self.num_heads * self.head_dim + 5 * self.inner_width + self.hidden_size
+        return 2 * self.num_heads * self.head_dim + 5 * self.inner_width + self.hidden_size + _chunk_elements(self)
 
     def forward_inner(self, y, col0, ctx: MixerContext, state_off, out, out_col0, mul) -> None:
         batch, T = ctx.batch, y.shape[0]
         o = torch.empty((T, self.inner_width), dtype=torch.float32, device=y.device)
         K.gated_linear_attention(y, col0 + self.q_off, col0 + self.k_off, col0 + self.v_off, None, self.query_scale, o,
                                  ctx.state, state_off, batch.entry_q_start, batch.entry_seat, self.num_heads,
-                                 self.head_dim, self.value_dim, head_decay=self.head_decay, activation=self.activation)
+                                 self.head_dim, self.value_dim, head_decay=self.head_decay, activation=self.activation,
+                                 lengths=np.diff(batch.h_entry_q_start))
         # one norm over all the heads' read-outs: a single "head" as wide as the row
         K.head_norm_gate(o, self.norm_weight, self.norm_eps, y, col0 + self.g_off, out, out_col0, 1, self.inner_width,
                          self.gate, mul)

@@ -209,6 +209,103 @@ def test_gated_linear_attention_over_steps(heads, dim, vdim, portions, gpu):
             torch.testing.assert_close(got[s][:, h * vdim:(h + 1) * vdim].to(F), want, rtol=2e-4, atol=2e-4)
 
 
+def rms(x):
+    return x.to(F).pow(2).mean().sqrt().item()
+
+
+CHUNK_LENGTHS = {2: 131, 0: 9, 1: 64, 3: 65, 4: 200, 5: 63}
+
+
+@pytest.mark.parametrize("portions", [(1000,), (64, 1, 70, 65)])
+@pytest.mark.parametrize("decays", ["usual", "strong", "none", "channel", "channel with zeros"])
+@pytest.mark.parametrize("heads, kv_heads, dim, vdim", [(2, 1, 128, 128), (4, 2, 64, 16), (1, 1, 64, 144), (2, 2, 128, 272)])
+def test_gated_delta_rule_in_chunks(heads, kv_heads, dim, vdim, decays, portions, gpu, monkeypatch):
+    """Entries of 64 tokens and more in chunks, shorter ones (and a chunk's odd end) beside them: read-outs and states
+    are as close to 64 bits as those of the walk over the tokens, within a factor that two orders of one sum differ by."""
+    monkeypatch.setattr(K, "DELTA_RULE_CHUNKS_FROM", 64)
+    g = torch.Generator().manual_seed(heads * dim + vdim)
+    C = 2 * kv_heads * dim + heads * vdim
+    qkv = {s: torch.randn(n, C, generator=g) for s, n in CHUNK_LENGTHS.items()}
+    y = {s: (torch.randn(n, 2 * heads + 3, generator=g) * 2).to(torch.bfloat16) for s, n in CHUNK_LENGTHS.items()}
+    a_log = torch.randn(heads, generator=g) * 0.5 + {"usual": -1.0, "strong": 4.0, "none": -60.0}.get(decays, 0.0)
+    dt_bias, boff, doff, alpha = torch.randn(heads, generator=g) * 0.5, 1, heads + 2, None
+    if decays.startswith("channel"):
+        alpha = {s: torch.rand(n, heads * dim, generator=g) ** 0.3 for s, n in CHUNK_LENGTHS.items()}
+        if "zeros" in decays:
+            for a in alpha.values():
+                a[torch.rand(a.shape, generator=g) < 0.02] = 0.0
+    got, states = {}, {}
+    for chunked in (True, False):
+        state = torch.zeros((len(CHUNK_LENGTHS), 4 + heads * dim * vdim), dtype=torch.float32, device="cuda")
+
+        def launch(seats, lens, starts):
+            rows, ys = (torch.cat([x[s][a:a + n] for s, n, a in zip(seats, lens, starts)]) for x in (qkv, y))
+            al = None if alpha is None else dev(torch.cat([alpha[s][a:a + n] for s, n, a in zip(seats, lens, starts)]))
+            out = torch.full((rows.shape[0], heads * vdim), float("nan"), dtype=torch.float32, device="cuda")
+            return K.gated_delta_rule(dev(rows), ys.to("cuda"), boff, doff, dev(a_log), dev(dt_bias), out, state, 4,
+                                      ints(np.cumsum([0] + lens)), ints(seats), heads, kv_heads, dim, vdim, channel_decay=al,
+                                      lengths=lens if chunked else None)
+        got[chunked] = run_in_steps(CHUNK_LENGTHS, portions, launch)
+        states[chunked] = state.cpu()
+    for s, n in CHUNK_LENGTHS.items():
+        r, ys = qkv[s].to(F), y[s].to(F)
+        q = plain.unit_vectors(r[:, :kv_heads * dim].view(n, kv_heads, dim)) * dim ** -0.5
+        k = plain.unit_vectors(r[:, kv_heads * dim:2 * kv_heads * dim].view(n, kv_heads, dim))
+        v = r[:, 2 * kv_heads * dim:].view(n, heads, vdim)
+        beta = torch.sigmoid(ys[:, boff:boff + heads])
+        one = torch.exp(-torch.exp(a_log.to(F)) * torch.nn.functional.softplus(ys[:, doff:doff + heads] + dt_bias.to(F)))
+        for h in range(heads):
+            kv = h // (heads // kv_heads)
+            S, want = torch.zeros(dim, vdim, dtype=F), torch.empty(n, vdim, dtype=F)
+            for t in range(n):
+                S = (one[t, h] if alpha is None else alpha[s][t, h * dim:(h + 1) * dim, None].to(F)) * S
+                S = S + torch.outer(k[t, kv], beta[t, h] * (v[t, h] - S.T @ k[t, kv]))
+                want[t] = S.T @ q[t, kv]
+            cols, at = slice(h * vdim, (h + 1) * vdim), slice(4 + h * dim * vdim, 4 + (h + 1) * dim * vdim)
+            for what, true, pair in (("out", want, [got[c][s][:, cols] for c in (True, False)]),
+                                     ("state", S, [states[c][s, at].view(dim, vdim) for c in (True, False)])):
+                assert rms(pair[0].to(F) - true) <= max(2.5 * rms(pair[1].to(F) - true), 2e-7 * rms(true)), (what, s, h)
+    assert (states[True][:, :4] == 0).all()
+
+
+@pytest.mark.parametrize("portions", [(1000,), (64, 1, 70, 65)])
+@pytest.mark.parametrize("decays", ["usual", "zeros", "fixed", "fixed at zero", "none"])
+@pytest.mark.parametrize("heads, dim, vdim, act", [(3, 64, 128, None), (2, 128, 16, "silu"), (1, 64, 48, "silu")])
+def test_gated_linear_attention_in_chunks(heads, dim, vdim, act, decays, portions, gpu, monkeypatch):
+    monkeypatch.setattr(K, "LINEAR_ATTENTION_CHUNKS_FROM", 64)
+    g = torch.Generator().manual_seed(heads * dim + vdim + 1)
+    offs = (3, 3 + heads * dim, 3 + 2 * heads * dim)
+    y = {s: torch.randn(n, offs[2] + heads * vdim + 2, generator=g).to(torch.bfloat16) for s, n in CHUNK_LENGTHS.items()}
+    alpha, fixed = {s: torch.rand(n, heads * dim, generator=g) ** 0.2 for s, n in CHUNK_LENGTHS.items()}, None
+    if decays == "zeros":
+        for a in alpha.values():
+            a[torch.rand(a.shape, generator=g) < 0.02] = 0.0
+    if decays in ("fixed", "fixed at zero", "none"):
+        fixed = torch.rand(heads, generator=g) * 0.5 + 0.5 if decays == "fixed" else torch.full((heads,), 0.0 if "zero" in decays else 1.0)
+        alpha = {s: fixed.repeat_interleave(dim)[None].expand(n, -1) for s, n in CHUNK_LENGTHS.items()}
+    got, states = {}, {}
+    for chunked in (True, False):
+        state = torch.zeros((len(CHUNK_LENGTHS), heads * dim * vdim), dtype=torch.float32, device="cuda")
+
+        def launch(seats, lens, starts):
+            ys, al = (torch.cat([x[s][a:a + n] for s, n, a in zip(seats, lens, starts)]) for x in (y, alpha))
+            out = torch.full((ys.shape[0], heads * vdim), float("nan"), dtype=torch.float32, device="cuda")
+            return K.gated_linear_attention(ys.to("cuda"), *offs, dev(al) if fixed is None else None, dim ** -0.5, out, state, 0,
+                                            ints(np.cumsum([0] + lens)), ints(seats), heads, dim, vdim, activation=act,
+                                            head_decay=None if fixed is None else dev(fixed), lengths=lens if chunked else None)
+        got[chunked] = run_in_steps(CHUNK_LENGTHS, portions, launch)
+        states[chunked] = state.cpu()
+    for s, n in CHUNK_LENGTHS.items():
+        q, k, v = (plain.silu(y[s][:, o:o + heads * w].to(F)) if act else y[s][:, o:o + heads * w].to(F) for o, w in zip(offs, (dim, dim, vdim)))
+        for h in range(heads):
+            a, b = slice(h * dim, (h + 1) * dim), slice(h * vdim, (h + 1) * vdim)
+            want, S = plain.decayed_outer_recurrence(q[:, a] * dim ** -0.5, k[:, a], v[:, b], alpha[s][:, a].to(F))
+            at = slice(h * dim * vdim, (h + 1) * dim * vdim)
+            for what, true, pair in (("out", want, [got[c][s][:, b] for c in (True, False)]),
+                                     ("state", S, [states[c][s, at].view(dim, vdim) for c in (True, False)])):
+                assert rms(pair[0].to(F) - true) <= max(2.5 * rms(pair[1].to(F) - true), 2e-7 * rms(true)), (what, s, h)
+
+
 def test_a_seat_used_again_after_zeroing_forgets_and_a_far_token_is_remembered(gpu):
     """A value written at the first position with a key of its own comes back 700 tokens later when
     nothing decays (both recurrences); the same seat zeroed gives a fresh request's numbers."""
