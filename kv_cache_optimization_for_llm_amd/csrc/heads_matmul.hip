@@ -259,8 +259,12 @@ template <int RT>
 __global__ void __launch_bounds__(256)
 heads_matmul_lds_kernel(bf16_t *__restrict__ out, int o_row, int o_head, const bf16_t *__restrict__ x, int x_row, int x_head,
                         const bf16_t *__restrict__ w, int M, int N, int K, int n_blocks, int m_blocks, HeadsGate gate, HeadsRotate ro) {
-    __shared__ __align__(16) typename LdsProduct<RT>::Shared shared;
-    constexpr int ROWS = LdsProduct<RT>::ROWS;
+    typedef LdsProduct<RT, 4, 4> Product;
+    __shared__ __align__(16) union {
+        typename Product::Shared operands;
+        bf16_t results[Product::ROWS * (Product::OUTS + 8)];
+    } shared;
+    constexpr int ROWS = Product::ROWS;
     const int cols = n_blocks + (ro.rot > 0 ? 1 : 0);           // the last column of workgroups rotates
     const int id = die_order(blockIdx.x, gridDim.x);
     const int h = id / (cols * m_blocks), m0 = (id / cols) % m_blocks * ROWS, col = id % cols;
@@ -268,22 +272,20 @@ heads_matmul_lds_kernel(bf16_t *__restrict__ out, int o_row, int o_head, const b
         heads_rotate<bf16_t>(ro, h, m0, min(M, m0 + ROWS));
         return;
     }
-    const int n0 = col * LDSP_N;
+    const int n0 = col * Product::OUTS;
     const int lane = threadIdx.x % KVA_WAVE, wave = threadIdx.x / KVA_WAVE, r = lane & 15, g = lane >> 4;
-    LdsProduct<RT> p;
+    Product p;
 #pragma unroll
-    for (int i = 0; i < LdsProduct<RT>::XI; ++i)
-        p.xp[i] = x + (size_t)min(m0 + p.row() + 32 * i, M - 1) * x_row + (size_t)h * x_head + p.element();
+    for (int i = 0; i < Product::XI; ++i)
+        p.xp[i] = x + (size_t)min(m0 + p.row(i), M - 1) * x_row + (size_t)h * x_head + p.element();
     p.plain_w(w + (size_t)h * N * K, N, K, n0);
     f32x4 acc[4][RT];
-    p.run(shared, K, acc);
+    p.run(shared.operands, K, acc);
     // Results go out 16 bytes a lane, 256 neighbouring bytes a row: through LDS, where the operands were (a lane
     // holds 4 outputs of a row).  Rows that are not aligned for that are written as they are.
-    constexpr int OUT_STRIDE = LDSP_N + 8;
-    static_assert(sizeof(shared) >= ROWS * OUT_STRIDE * sizeof(bf16_t), "the results fit where the operands were");
+    constexpr int OUT_STRIDE = Product::OUTS + 8;
     const bool through = (o_row | o_head | N) % 8 == 0 && (reinterpret_cast<uintptr_t>(out) & 15) == 0;
-    bf16_t *tile = shared.x[0];
-    if (through) __syncthreads();                               // nobody reads the operands any more
+    bf16_t *tile = shared.results;
 #pragma unroll
     for (int rt = 0; rt < RT; ++rt) {
         const int row = (wave & 1) * 16 * RT + 16 * rt + r, t = m0 + row;
@@ -328,7 +330,7 @@ extern "C" int kva_heads_matmul_mfma(void *out, int o_row, int o_head, const voi
     HEADS_OPTIONS(gate, ro);
     if (rows == 0) return KVA_OK;
     if (rows > HM_LDS_ROWS && N >= 64) {
-        const int n_blocks = (N + LDSP_N - 1) / LDSP_N, cols = n_blocks + (rot > 0 ? 1 : 0);
+        const int n_blocks = (N + 127) / 128, cols = n_blocks + (rot > 0 ? 1 : 0);
         // the smaller tile where the larger would leave compute units without work
         const bool small = (long long)n_blocks * heads * ((rows + 127) / 128) < 512;
         const int tile = small ? 64 : 128, m_blocks = (rows + tile - 1) / tile;

@@ -1,102 +1,118 @@
 // A bf16 product of many rows on the matrix cores, operands through LDS: the middle of kernels that differ in
 // where their operands' rows lie and in what they do with the result (experts' products, products per head).
 //
-// A workgroup of four wavefronts takes 32 RT rows of x and 128 outputs (rows of w), a wavefront half of
-// either.  64 elements of K of both operands go through LDS at a time, two deep (the next ones' loads are in
-// flight while these are multiplied), in rows padded so that a fragment's 16 lanes lie on banks of their own.
-// K (a multiple of 8) is added in ascending order into one accumulator an output.
+// A workgroup of four wavefronts takes 32 RT rows of x and 32 NT outputs (rows of w), a wavefront half of
+// either.  32 elements of K of both operands are a stage; STAGES of them stand in LDS in a ring.  They get there
+// without a stop in registers (global_load_lds, 16 bytes a lane), STAGES - 1 of them on their way while one is
+// multiplied: a stage is 512 cycles of matrix products with RT = 4 and NT = 8, a trip to L2 two to four
+// times that.  K (a multiple of 32) is added in ascending order into one accumulator an output.
+//
+// Before, operands went through registers, one stage of 64 elements ahead, 128 x 128 at a time, and results to memory
+// one by one: experts' products of 8,192 slots of 16 experts, 1,536 x 2,048 / 2,048 x 768: 122 / 61 -> 78 / 60 us; of 4
+// experts, 1,024 x 2,048 / 2,048 x 1,024: 132 / 70 -> 56 / 43; 2,048 slots of 16: 67 / 29 -> 36 / 22.  The middle alone
+// (4,096 x 4,096 x 2,048, w in operand order): 1.23 PFLOP/s; without its loads 1.61, without its reads 1.41.
+//
+// What bounds it: a wavefront reads (RT + NT) KiB of operands from LDS for RT NT products of 16 cycles; four of them
+// at RT = 4, NT = 8 ask for 96 of the 128 bytes a cycle that LDS gives, at 4 x 4 for all 128.
 #pragma once
 #include "common.h"
 #include "attention_frag.h"
 
-#define LDSP_K 64
-#define LDSP_STRIDE 72
-#define LDSP_N 128
+#define LDSP_K 32
 
-template <int RT>
+// 16 bytes a lane from memory to LDS, the wavefront's 1 KiB in the order of the lanes from `to` (the same in all) on
+__device__ __forceinline__ void load_to_lds(const void *from, void *to) {
+    __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) unsigned int *)from,
+                                     (__attribute__((address_space(3))) unsigned int *)to, 16, 0, 0);
+}
+// The wavefront's loads but the last N have arrived; then all wavefronts' have.  Nothing that reads or writes memory
+// moves across.
+template <int N>
+__device__ __forceinline__ void wait_and_meet() {
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_sched_barrier(0);
+    __builtin_amdgcn_s_waitcnt((N & 15) | (N >> 4 << 14) | 0x70 | 0xf00);       // vmcnt(N), the other counters as they are
+    __builtin_amdgcn_s_barrier();
+    __builtin_amdgcn_sched_barrier(0);
+    asm volatile("" ::: "memory");
+}
+
+template <int RT, int NT, int STAGES>
 struct LdsProduct {
-    static constexpr int ROWS = 32 * RT;
-    static constexpr int XI = ROWS * LDSP_K / 8 / 256, WI = LDSP_N * LDSP_K / 8 / 256;      // 16-byte pieces a thread loads
+    static constexpr int ROWS = 32 * RT, OUTS = 32 * NT;
+    static constexpr int XI = ROWS * LDSP_K / 8 / 256, WI = OUTS * LDSP_K / 8 / 256;      // 16-byte pieces a thread loads
+    // Blocks of 16 rows x 32 elements, 1 KiB each.  x (and w kept row by row): row by row, the four 16-byte pieces of
+    // row r in the order piece ^ (r / 4 % 4), so that the 16 rows of an operand lie in different banks.  w kept in operand
+    // order stands as it is kept.
     struct Shared {
-        bf16_t x[2][ROWS * LDSP_STRIDE], w[2][LDSP_N * LDSP_STRIDE];
+        bf16_t x[STAGES][ROWS * LDSP_K], w[STAGES][OUTS * LDSP_K];
     };
-    // Thread t loads elements 8 (t % 8) .. of rows t / 8 + 32 i of x: `xp` points at its first element of the row.
-    // Its pieces of w are the caller's choice: `wp` their first elements, `wkc` their place in the 64 elements,
-    // `wat` where they go in LDS; `wmul` elements of w's storage go by per element of K.
+    // Piece i of thread t: row row(i) of x, elements element() .. + 7: `xp` points at its first one of the row.
     const bf16_t *xp[XI], *wp[WI];
-    int wat[WI], wkc[WI], wmul;
+    int wmul;                       // elements of w's storage that go by per element of K
+    bool w_swizzled;
 
-    __device__ __forceinline__ static int row() { return threadIdx.x / 8; }
-    __device__ __forceinline__ static int element() { return 8 * (threadIdx.x % 8); }
+    __device__ __forceinline__ static int row(int i) { return threadIdx.x / 4 + 64 * i; }
+    __device__ __forceinline__ static int element() { return 8 * ((threadIdx.x % 4) ^ (threadIdx.x / 16 % 4)); }
 
-    // w row by row, rows n0 .. n0 + 127 (past the last one the last one again)
+    // w row by row, rows n0 .. n0 + OUTS - 1 (past the last one the last one again)
     __device__ __forceinline__ void plain_w(const bf16_t *w, int N, int K, int n0) {
         wmul = 1;
+        w_swizzled = true;
 #pragma unroll
-        for (int i = 0; i < WI; ++i) {
-            wkc[i] = element();
-            wat[i] = (row() + 32 * i) * LDSP_STRIDE + wkc[i];
-            wp[i] = w + (size_t)min(n0 + row() + 32 * i, N - 1) * K + wkc[i];
-        }
+        for (int i = 0; i < WI; ++i) wp[i] = w + (size_t)min(n0 + row(i), N - 1) * K + element();
     }
     // w in operand order [N / 16][K / 32][lane][8]: a wavefront's pieces are neighbouring bytes
     __device__ __forceinline__ void tiled_w(const bf16_t *w, int N, int K, int n0) {
-        const int lane = threadIdx.x % KVA_WAVE, wave = threadIdx.x / KVA_WAVE, r = lane & 15, g = lane >> 4;
         wmul = 16;
+        w_swizzled = false;
 #pragma unroll
-        for (int i = 0; i < WI; ++i) {
-            const int f = wave + 4 * i, nt = f >> 1;
-            wkc[i] = 32 * (f & 1) + 8 * g;
-            wat[i] = (16 * nt + r) * LDSP_STRIDE + wkc[i];
-            wp[i] = w + (size_t)min(n0 + 16 * nt, N - 16) * K + (f & 1) * 16 * 32 + 8 * lane;
-        }
+        for (int i = 0; i < WI; ++i)
+            wp[i] = w + (size_t)min(n0 + 16 * (int)(threadIdx.x / KVA_WAVE + 4 * i), N - 16) * K + 8 * (threadIdx.x % KVA_WAVE);
     }
 
     // acc[nt][rt]: lane (r = lane % 16, g = lane / 16) of wavefront (half of the rows wave % 2, of the outputs
-    // wave / 2) gets outputs 64 (wave / 2) + 16 nt + 4 g .. + 3 of row (wave % 2) 16 RT + 16 rt + r
-    __device__ __forceinline__ void run(Shared &s, int K, f32x4 (&acc)[4][RT]) const {
-        const int lane = threadIdx.x % KVA_WAVE, wave = threadIdx.x / KVA_WAVE, r = lane & 15, g = lane >> 4;
-        const int wr = wave & 1, wn = wave >> 1, kc = element();
-        uint4 xv[XI], wv[WI];
-#define LDSP_LOAD(K0)                                                                                                    \
-    {                                                                                                                    \
-        _Pragma("unroll") for (int i = 0; i < XI; ++i)                                                                   \
-            xv[i] = (K0) + kc < K ? *reinterpret_cast<const uint4 *>(xp[i] + (K0)) : make_uint4(0u, 0u, 0u, 0u);          \
-        _Pragma("unroll") for (int i = 0; i < WI; ++i)                                                                   \
-            wv[i] = (K0) + wkc[i] < K ? *reinterpret_cast<const uint4 *>(wp[i] + (K0) * wmul) : make_uint4(0u, 0u, 0u, 0u); \
-    }
+    // wave / 2) gets outputs 16 NT (wave / 2) + 16 nt + 4 g .. + 3 of row (wave % 2) 16 RT + 16 rt + r
+    __device__ __forceinline__ void run(Shared &s, int K, f32x4 (&acc)[NT][RT]) const {
+        const int lane = threadIdx.x % KVA_WAVE, wave = __builtin_amdgcn_readfirstlane(threadIdx.x / KVA_WAVE), r = lane & 15, g = lane >> 4;
+        const int wr = wave & 1, wn = wave >> 1;
+        const int swizzled = r * LDSP_K + 8 * (g ^ (r / 4)), xat = swizzled, wat = w_swizzled ? swizzled : 8 * lane;
+        auto load = [&](int slot, int k0) {
 #pragma unroll
-        for (int nt = 0; nt < 4; ++nt)
+            for (int i = 0; i < XI; ++i) load_to_lds(xp[i] + k0, &s.x[slot][(wave + 4 * i) * 512]);
+#pragma unroll
+            for (int i = 0; i < WI; ++i) load_to_lds(wp[i] + k0 * wmul, &s.w[slot][(wave + 4 * i) * 512]);
+        };
+#pragma unroll
+        for (int nt = 0; nt < NT; ++nt)
 #pragma unroll
             for (int rt = 0; rt < RT; ++rt) acc[nt][rt] = f32x4{0.f, 0.f, 0.f, 0.f};
-        LDSP_LOAD(0)
-        int buf = 0;
-        for (int k0 = 0; k0 < K; k0 += LDSP_K, buf ^= 1) {
+        const int last = K - LDSP_K;        // (past the end the last stage again: as many loads are on their way in every turn)
 #pragma unroll
-            for (int i = 0; i < XI; ++i) *reinterpret_cast<uint4 *>(&s.x[buf][(row() + 32 * i) * LDSP_STRIDE + kc]) = xv[i];
+        for (int i = 0; i < STAGES - 1; ++i) load(i, min(i * LDSP_K, last));
+        int slot = 0;
+        for (int k0 = 0; k0 < K; k0 += LDSP_K) {
+            wait_and_meet<(STAGES - 2) * (XI + WI)>();
+            const bf16_t *xr = &s.x[slot][wr * RT * 512 + xat], *wrow = &s.w[slot][wn * NT * 512 + wat];
+            Frag8 xf[RT], wf[NT];
 #pragma unroll
-            for (int i = 0; i < WI; ++i) *reinterpret_cast<uint4 *>(&s.w[buf][wat[i]]) = wv[i];
-            __syncthreads();            // (a buffer was read last two turns ago: every wavefront has passed the barrier between)
-            if (k0 + LDSP_K < K) LDSP_LOAD(k0 + LDSP_K)
-            const bf16_t *xr = &s.x[buf][(wr * 16 * RT + r) * LDSP_STRIDE + 8 * g], *wrow = &s.w[buf][(wn * 64 + r) * LDSP_STRIDE + 8 * g];
-            Frag8 xf[2][RT], wf[2][4];
+            for (int rt = 0; rt < RT; ++rt) xf[rt].v = *reinterpret_cast<const b16x8 *>(xr + rt * 512);
 #pragma unroll
-            for (int ks = 0; ks < 2; ++ks) {
-#pragma unroll
-                for (int nt = 0; nt < 4; ++nt) wf[ks][nt].u4 = *reinterpret_cast<const uint4 *>(wrow + nt * 16 * LDSP_STRIDE + 32 * ks);
-#pragma unroll
-                for (int rt = 0; rt < RT; ++rt) xf[ks][rt].u4 = *reinterpret_cast<const uint4 *>(xr + rt * 16 * LDSP_STRIDE + 32 * ks);
-            }
+            for (int nt = 0; nt < NT; ++nt) wf[nt].v = *reinterpret_cast<const b16x8 *>(wrow + nt * 512);
+            // (read as vectors of bf16, in front of the next loads: the compiler then knows that no load on its way writes what
+            // is read here - of which wait_and_meet makes sure - and does not wait for all of them)
             __builtin_amdgcn_sched_barrier(0);
+            // the slot read in the turn before: every wavefront has passed the barrier since
+            const int into = slot == 0 ? STAGES - 1 : slot - 1;
+            load(into, min(k0 + (STAGES - 1) * LDSP_K, last));
 #pragma unroll
-            for (int ks = 0; ks < 2; ++ks)
+            for (int nt = 0; nt < NT; ++nt)
 #pragma unroll
-                for (int nt = 0; nt < 4; ++nt)
-#pragma unroll
-                    for (int rt = 0; rt < RT; ++rt)
-                        acc[nt][rt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf[ks][nt].v, xf[ks][rt].v, acc[nt][rt], 0, 0, 0);
+                for (int rt = 0; rt < RT; ++rt)
+                    acc[nt][rt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf[nt].v, xf[rt].v, acc[nt][rt], 0, 0, 0);
+            slot = slot + 1 == STAGES ? 0 : slot + 1;
         }
-#undef LDSP_LOAD
+        wait_and_meet<0>();                 // nothing is on its way any more, nobody reads: the caller may use the LDS
     }
 };
 

@@ -646,53 +646,107 @@ moe_expert_rows_mfma_kernel(MoeRows a, void *__restrict__ out, int out_dtype, co
     }
 }
 
-// matrix cores, many rows an expert: a workgroup takes a group of 2 RT tiles of one expert (32 RT rows) and 128
-// outputs, operands through LDS (lds_product.h).  A die reads few experts.
-template <int RT>
-__global__ void __launch_bounds__(256)
+// Eight neighbouring results of a place from n on (n a multiple of 8), the slot's weight (or 1) at hand: as moe_store
+// and moe_store_gated do one by one.
+__device__ inline void moe_store8(const MoeRows &a, void *__restrict__ out, int out_dtype, int place, int slot, float weight, int n, const float *v) {
+    float f[8];
+#pragma unroll
+    for (int i = 0; i < 8; ++i) f[i] = v[i] * weight;
+    if (a.gated) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+            f[i] = a.act == 4 ? kva_gated_activate(f[2 * i], f[2 * i + 1], KVA_ACT_SWISH_CLAMPED, a.limit) : moe_activate(f[2 * i], a.act) * f[2 * i + 1];
+    } else if (a.mode == 0) {
+#pragma unroll
+        for (int i = 0; i < 8; ++i) f[i] = moe_activate(f[i], a.act);
+    }
+    const int width = a.gated ? a.N / 2 : a.N, at = a.gated ? n / 2 : n, count = a.gated ? 4 : 8;
+    const size_t first = (size_t)(a.mode == 0 ? place : slot) * width + at;
+    if (n + 8 <= a.N && width % 8 == 0 && (reinterpret_cast<uintptr_t>(out) & 15) == 0) {
+        if (out_dtype == KVA_BF16) {
+            uint16_t *o = reinterpret_cast<uint16_t *>(out) + first;
+            const Frag8 h = {.p2 = {pack_bf16(f[0], f[1]), pack_bf16(f[2], f[3]), pack_bf16(f[4], f[5]), pack_bf16(f[6], f[7])}};
+            if (a.gated) *reinterpret_cast<uint2 *>(o) = h.u2[0];
+            else *reinterpret_cast<uint4 *>(o) = h.u4;
+        } else {
+            float4 *o = reinterpret_cast<float4 *>(reinterpret_cast<float *>(out) + first);
+            o[0] = make_float4(f[0], f[1], f[2], f[3]);
+            if (!a.gated) o[1] = make_float4(f[4], f[5], f[6], f[7]);
+        }
+        return;
+    }
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+        if (i >= count || at + i >= width) continue;
+        if (out_dtype == KVA_BF16) reinterpret_cast<uint16_t *>(out)[first + i] = float_to_bf16_bits(f[i]);
+        else reinterpret_cast<float *>(out)[first + i] = f[i];
+    }
+}
+
+template <int RT, int NT, int STAGES>
+union MoeLds {
+    static constexpr int STRIDE = 128 + 4;          // a row of results in LDS
+    typename LdsProduct<RT, NT, STAGES>::Shared operands;
+    float results[LdsProduct<RT, NT, STAGES>::ROWS * STRIDE];
+};
+
+// matrix cores, many rows an expert: a workgroup takes a group of 2 RT tiles of one expert (32 RT rows) and 32 NT
+// outputs, operands through LDS (lds_product.h).  The list was laid out for any split among the experts; the groups
+// that hold something come first, and only they are dealt out, neighbours to one die: a die reads few experts.
+template <int RT, int NT, int STAGES>
+__global__ void __launch_bounds__(256, 2)
 moe_expert_rows_lds_kernel(MoeRows a, void *__restrict__ out, int out_dtype, const bf16_t *__restrict__ x,
-                           const bf16_t *__restrict__ w, int n_blocks) {
-    __shared__ __align__(16) typename LdsProduct<RT>::Shared shared;
-    const int id = die_order(blockIdx.x, gridDim.x);
-    const int first = (id / n_blocks) * 2 * RT, n0 = (id % n_blocks) * LDSP_N;
+                           const bf16_t *__restrict__ w, int n_blocks, int groups) {
+    typedef LdsProduct<RT, NT, STAGES> Product;
+    __shared__ __align__(16) MoeLds<RT, NT, STAGES> shared;
+    __shared__ int slot_of[Product::ROWS];
+    __shared__ float weight_of[Product::ROWS];
+    const int lane = threadIdx.x % KVA_WAVE, wave = threadIdx.x / KVA_WAVE, r = lane & 15, g = lane >> 4;
+    int used = 0;
+    for (int g0 = 0; g0 < groups; g0 += KVA_WAVE)
+        used += __popcll(__ballot(g0 + lane < groups && a.tile_expert[(size_t)min(g0 + lane, groups - 1) * 2 * RT] >= 0));
+    const int total = used * n_blocks;
+    if ((int)blockIdx.x >= total) return;
+    const int id = die_order(blockIdx.x, total);
+    const int first = (id / n_blocks) * 2 * RT, n0 = (id % n_blocks) * Product::OUTS;
     const int e = a.tile_expert[first];
     if (e < 0) return;
-    const int lane = threadIdx.x % KVA_WAVE, wave = threadIdx.x / KVA_WAVE, r = lane & 15, g = lane >> 4;
     const int wr = wave & 1, wn = wave >> 1;
-    LdsProduct<RT> p;
+    Product p;
 #pragma unroll
-    for (int i = 0; i < LdsProduct<RT>::XI; ++i) {
-        const int place = first * MOE_TILE + p.row() + 32 * i, slot = a.sorted_slot[place];
+    for (int i = 0; i < Product::XI; ++i) {
+        const int place = first * MOE_TILE + p.row(i), slot = a.sorted_slot[place];
         p.xp[i] = x + (a.mode == 0 ? (size_t)(slot < 0 ? 0 : slot / a.top) : (size_t)place) * a.K + p.element();
+    }
+    if (threadIdx.x < Product::ROWS) {
+        const int slot = a.sorted_slot[first * MOE_TILE + threadIdx.x];
+        slot_of[threadIdx.x] = slot;
+        weight_of[threadIdx.x] = a.slot_weight && slot >= 0 ? a.slot_weight[slot] : 1.f;
     }
     const bf16_t *we = w + (size_t)e * a.N * a.K;
     if (a.tiled) p.tiled_w(we, a.N, a.K, n0);
     else p.plain_w(we, a.N, a.K, n0);
-    f32x4 acc[4][RT];
-    p.run(shared, a.K, acc);
-    // lane (row r, group g) holds outputs 4 g .. 4 g + 3 of tile nt, of its row of tile rt
+    f32x4 acc[NT][RT];
+    p.run(shared.operands, a.K, acc);
+    // The results go out by rows, through LDS in 32 bits (where the operands were): four tiles of either half of the
+    // outputs at a time, then 8 neighbouring outputs a thread.
 #pragma unroll
-    for (int rt = 0; rt < RT; ++rt) {
-        const int place = first * MOE_TILE + (wr * RT + rt) * 16 + r, slot = a.sorted_slot[place];
-        if (slot < 0) continue;
-        const float weight = a.mode == 1 && a.slot_weight ? a.slot_weight[slot] : 1.f;
+    for (int part = 0; part < NT / 4; ++part) {
+        if (part > 0) __syncthreads();
 #pragma unroll
-        for (int nt = 0; nt < 4; ++nt) {
-            const int n = n0 + wn * 64 + nt * 16 + 4 * g;
-            const f32x4 v = acc[nt][rt];
-            if (a.mode == 1 && a.N % 4 == 0) {
-                if (n < a.N)
-                    *reinterpret_cast<float4 *>(reinterpret_cast<float *>(out) + (size_t)slot * a.N + n) =
-                        make_float4(v[0] * weight, v[1] * weight, v[2] * weight, v[3] * weight);
-            } else if (a.gated) {
-                if (n + 1 < a.N) moe_store_gated(a, out, out_dtype, place, slot, n, v[0], v[1]);
-                if (n + 3 < a.N) moe_store_gated(a, out, out_dtype, place, slot, n + 2, v[2], v[3]);
-            } else {
+        for (int nt = 0; nt < 4; ++nt)
 #pragma unroll
-                for (int i = 0; i < 4; ++i)
-                    if (n + i < a.N) moe_store(a, out, out_dtype, place, slot, n + i, v[i]);
+            for (int rt = 0; rt < RT; ++rt)
+                *reinterpret_cast<f32x4 *>(&shared.results[((wr * RT + rt) * 16 + r) * MoeLds<RT, NT, STAGES>::STRIDE + wn * 64 + nt * 16 + 4 * g]) =
+                    acc[4 * part + nt][rt];
+        __syncthreads();
+        const int c = 8 * (threadIdx.x % 16), n = n0 + c / 64 * 16 * NT + part * 64 + c % 64;
+        if (n < a.N)
+            for (int row = threadIdx.x / 16; row < Product::ROWS; row += 16) {
+                const int slot = slot_of[row];
+                if (slot >= 0)
+                    moe_store8(a, out, out_dtype, first * MOE_TILE + row, slot, weight_of[row], n, &shared.results[row * MoeLds<RT, NT, STAGES>::STRIDE + c]);
             }
-        }
     }
 }
 
@@ -717,15 +771,20 @@ extern "C" int kva_moe_expert_rows(void *out, int out_dtype, const void *x, cons
     if (max_tiles == 0) return KVA_OK;
     MoeRows a{sorted_slot, tile_expert, slot_weight, top, N, K, mode, act, tiled, gated, limit};
     if (group > 1) {
-        const int n_blocks = (N + LDSP_N - 1) / LDSP_N;
-        const long long blocks = (long long)n_blocks * (max_tiles / group);
-        KVA_REQUIRE(blocks <= 0x7fffffff, "moe_expert_rows: too many workgroups");
-        if (group == 8)
-            hipLaunchKernelGGL((moe_expert_rows_lds_kernel<4>), dim3((unsigned)blocks), dim3(256), 0, stream, a, out, out_dtype,
-                               (const bf16_t *)x, (const bf16_t *)w, n_blocks);
+        // 256 outputs a workgroup (two workgroups a compute unit) where that leaves no unit idle; 128 where it would:
+        // 8,192 slots of 4 experts, 1,024 x 2,048 (256 workgroups of the wide kind) 75 against 56 us, 2,048 x 1,024 (512)
+        // 43 against 53; 3,356 slots of 16 experts, 1,536 x 2,048 (258) 59 against 44
+        const int groups = max_tiles / group, wide = (N + 255) / 256, narrow = (N + 127) / 128;
+        KVA_REQUIRE((long long)narrow * groups <= 0x7fffffff, "moe_expert_rows: too many workgroups");
+        if (group == 8 && (long long)wide * groups >= 400)
+            hipLaunchKernelGGL((moe_expert_rows_lds_kernel<4, 8, 3>), dim3(wide * groups), dim3(256), 0, stream, a, out, out_dtype,
+                               (const bf16_t *)x, (const bf16_t *)w, wide, groups);
+        else if (group == 8)
+            hipLaunchKernelGGL((moe_expert_rows_lds_kernel<4, 4, 4>), dim3(narrow * groups), dim3(256), 0, stream, a, out, out_dtype,
+                               (const bf16_t *)x, (const bf16_t *)w, narrow, groups);
         else
-            hipLaunchKernelGGL((moe_expert_rows_lds_kernel<2>), dim3((unsigned)blocks), dim3(256), 0, stream, a, out, out_dtype,
-                               (const bf16_t *)x, (const bf16_t *)w, n_blocks);
+            hipLaunchKernelGGL((moe_expert_rows_lds_kernel<2, 4, 4>), dim3(narrow * groups), dim3(256), 0, stream, a, out, out_dtype,
+                               (const bf16_t *)x, (const bf16_t *)w, narrow, groups);
     } else if (dtype == KVA_BF16 && K % 32 == 0) {
         // few tiles: 16 outputs a workgroup, so that enough of them stream the matrices; many: 64 outputs and
         // four row tiles, which share what they load
