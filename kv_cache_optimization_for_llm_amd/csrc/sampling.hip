@@ -9,21 +9,23 @@
 // mask row are penalised first (l > 0 ? l / p : l * p).
 //
 // How: two launches, and the logits are read once.
-//   1. sample_scan_kernel, one workgroup per (chunk of a row, row): every thread keeps an online
-//      (maximum, sum of exp((l - maximum) / T)) pair and its best (value, id) over the tokens it
-//      reads; the workgroup joins them and leaves one record per chunk.
-//   2. sample_pick_kernel, one wavefront per row: joins the chunk records (row maximum, argmax),
+//   1. sample_scan_kernel, one workgroup per (chunk of a row, row): the tokens, up to 4,096 at a time, are loaded
+//      into registers (16 bytes a lane where rows are aligned for it), the workgroup's best (value, id) is found,
+//      then the sum of exp((l - maximum) / T); one record per chunk.
+//   2. sample_pick_kernel, one workgroup per row: joins the chunk records (row maximum, argmax),
 //      rescales the chunk sums to the row maximum, finds the chunk that holds the target by a
-//      wavefront prefix scan, reads that one chunk again (a thousand tokens), scans the lanes'
-//      spans the same way, and the lane that holds the target walks its few tokens.  The chosen
+//      wavefront prefix scan and reads that one chunk again, 64 neighbouring tokens a load: the 64 that
+//      hold the target are found by their sums, the token by a prefix scan over the lanes.  The chosen
 //      token is also marked in the request's mask row when there is one.
+//
+// 64 rows of 128,256 logits (33 MB), half of them at a temperature: both kernels 14 us in a graph.  With 128 workgroups
+// a row whose threads took four tokens each, one by one, and a single wavefront that walked its spans of the chunk: 30.
 #include "common.h"
 #include <math.h>
 
 #define SAMPLE_THREADS 256
-#define SCAN_IN_FLIGHT 8
+#define SCAN_TOKENS 4096         // tokens a workgroup holds in registers at a time
 #define SAMPLE_MAX_CHUNKS 1024
-#define PICK_CHUNKS_PER_LANE (SAMPLE_MAX_CHUNKS / KVA_WAVE)
 #define KVA_NO_TOKEN (-1)       // what a row gets whose logits name no token
 
 namespace {
@@ -78,7 +80,7 @@ __device__ inline const unsigned char *mask_row(const unsigned char *penalty_mas
     return seat < 0 ? nullptr : penalty_mask + (size_t)seat * vocab;
 }
 
-// exp((l - top) / T); a logit that is -inf or NaN weighs nothing (as in Online::add)
+// exp((l - top) / T); a logit that is -inf or NaN weighs nothing
 __device__ inline float token_weight(float l, float top, float inv_t) {
     return l > -INFINITY ? expf((l - top) * inv_t) : 0.f;
 }
@@ -86,15 +88,6 @@ __device__ inline float token_weight(float l, float top, float inv_t) {
 // Running softmax denominator: sum of exp((l - m) * inv_t) over what has been added, m their maximum.
 struct Online {
     float m, s;
-    __device__ inline void add(float l, float inv_t) {
-        if (!(l > -INFINITY)) return;        // -inf and NaN weigh nothing
-        if (l > m) {
-            s = s * expf((m - l) * inv_t) + 1.f;
-            m = l;
-        } else {
-            s += expf((l - m) * inv_t);
-        }
-    }
     __device__ inline void join(Online o, float inv_t) {
         if (o.m == -INFINITY) return;
         if (m == -INFINITY) {
@@ -128,15 +121,18 @@ struct ChunkRecord {
     float sum;
 };
 
-// grid (chunks, rows)
+// grid (chunks, rows).  VEC: rows and chunks start at multiples of 16 bytes.
+template <bool VEC>
 __global__ void __launch_bounds__(SAMPLE_THREADS)
 sample_scan_kernel(const float *__restrict__ logits, int vocab, int chunk_tokens,
                    const unsigned char *__restrict__ penalty_mask, const int *__restrict__ row_seat,
                    float penalty, const float *__restrict__ inv_temperature,
                    ChunkRecord *__restrict__ records) {
-    __shared__ Best wave_b[SAMPLE_THREADS / KVA_WAVE];
-    __shared__ Online wave_o[SAMPLE_THREADS / KVA_WAVE];
+    constexpr int WAVES = SAMPLE_THREADS / KVA_WAVE;
+    __shared__ Best wave_b[2][WAVES];
+    __shared__ float wave_s[2][WAVES];
     const int row = blockIdx.y, chunk = blockIdx.x, chunks = gridDim.x;
+    const int lane = threadIdx.x % KVA_WAVE, wave = threadIdx.x / KVA_WAVE;
     const int begin = chunk * chunk_tokens;
     const int end = min(begin + chunk_tokens, vocab);
     const float *rl = logits + (size_t)row * vocab;
@@ -145,54 +141,51 @@ sample_scan_kernel(const float *__restrict__ logits, int vocab, int chunk_tokens
     const bool sampled = inv_t > 0.f;
     Best b{-INFINITY, vocab};
     Online o{-INFINITY, 0.f};
-    // A thread's tokens in turns of SCAN_IN_FLIGHT, every load of a turn asked for before the first
-    // is used (a plain loop over a thread's four or eight tokens is a trip to memory each).
-    for (int base = begin + threadIdx.x; base < end; base += SCAN_IN_FLIGHT * SAMPLE_THREADS) {
-        float l[SCAN_IN_FLIGHT];
-        unsigned char marked[SCAN_IN_FLIGHT];
+    for (int base = begin, turn = 0; base < end; base += SCAN_TOKENS, turn ^= 1) {
+        // thread t's tokens: 4 t .. 4 t + 3 of every 1,024 (their loads side by side); past the end: -inf, no weight
+        float l[SCAN_TOKENS / SAMPLE_THREADS];
 #pragma unroll
-        for (int j = 0; j < SCAN_IN_FLIGHT; ++j) {
-            const int t = base + j * SAMPLE_THREADS;
-            l[j] = rl[t < end ? t : end - 1];
-            marked[j] = mk != nullptr ? mk[t < end ? t : end - 1] : (unsigned char)0;
-        }
+        for (int j = 0; j < SCAN_TOKENS / SAMPLE_THREADS; j += 4) {
+            const int t = base + j * SAMPLE_THREADS + 4 * threadIdx.x;
+            if (VEC) {
+                const float4 v = t < end ? *reinterpret_cast<const float4 *>(rl + t) : make_float4(-INFINITY, -INFINITY, -INFINITY, -INFINITY);
+                l[j] = v.x; l[j + 1] = v.y; l[j + 2] = v.z; l[j + 3] = v.w;
+            } else {
 #pragma unroll
-        for (int j = 0; j < SCAN_IN_FLIGHT; ++j) {
-            const int t = base + j * SAMPLE_THREADS;
-            if (t >= end) break;
-            const float v = marked[j] != 0 ? (l[j] > 0.f ? l[j] / penalty : l[j] * penalty) : l[j];
-            b = better(b, Best{v, t});
-            if (sampled) o.add(v, inv_t);
+                for (int i = 0; i < 4; ++i) l[j + i] = t + i < end ? rl[t + i] : -INFINITY;
+            }
         }
-    }
-    b = wave_best(b);
-    if (sampled) {
+        Best mine{-INFINITY, vocab};
 #pragma unroll
-        for (int off = KVA_WAVE / 2; off > 0; off >>= 1) {
-            Online other;
-            other.m = __shfl_xor(o.m, off, KVA_WAVE);
-            other.s = __shfl_xor(o.s, off, KVA_WAVE);
-            o.join(other, inv_t);
+        for (int j = 0; j < SCAN_TOKENS / SAMPLE_THREADS; ++j) {
+            const int t = base + j / 4 * 4 * SAMPLE_THREADS + 4 * threadIdx.x + j % 4;
+            if (mk != nullptr && t < end) l[j] = penalised(l[j], mk, t, penalty);
+            if (l[j] > mine.value) mine = Best{l[j], t};        // (a thread's tokens come in ascending order: the first of equal ones)
         }
-    }
-    const int lane = threadIdx.x % KVA_WAVE, wave = threadIdx.x / KVA_WAVE;
-    if (lane == 0) {
-        wave_b[wave] = b;
-        wave_o[wave] = o;
-    }
-    __syncthreads();
-    if (threadIdx.x == 0) {
+        mine = wave_best(mine);
+        if (lane == 0) wave_b[turn][wave] = mine;
+        __syncthreads();
 #pragma unroll
-        for (int w = 1; w < SAMPLE_THREADS / KVA_WAVE; ++w) {
-            b = better(b, wave_b[w]);
-            if (sampled) o.join(wave_o[w], inv_t);
-        }
-        records[(size_t)row * chunks + chunk] = ChunkRecord{b.value, b.index, o.m, o.s};
+        for (int w = 0; w < WAVES; ++w) mine = better(mine, wave_b[turn][w]);
+        b = better(b, mine);
+        if (!sampled) continue;                                 // (the row's: the whole workgroup)
+        float s = 0.f;
+        if (mine.value > -INFINITY)
+#pragma unroll
+            for (int j = 0; j < SCAN_TOKENS / SAMPLE_THREADS; ++j) s += token_weight(l[j], mine.value, inv_t);
+        s = wave_sum_valu(s);
+        if (lane == 0) wave_s[turn][wave] = s;
+        __syncthreads();
+        s = 0.f;
+#pragma unroll
+        for (int w = 0; w < WAVES; ++w) s += wave_s[turn][w];
+        o.join(Online{mine.value, s}, inv_t);
     }
+    if (threadIdx.x == 0) records[(size_t)row * chunks + chunk] = ChunkRecord{b.value, b.index, o.m, o.s};
 }
 
-// grid (rows), one wavefront
-__global__ void __launch_bounds__(KVA_WAVE)
+// grid (rows).  Every wavefront joins the records by itself (they agree); the chunk's tokens are shared out.
+__global__ void __launch_bounds__(SAMPLE_THREADS)
 sample_pick_kernel(const float *__restrict__ logits, int vocab, int chunk_tokens, int chunks,
                    const unsigned char *penalty_mask, const int *__restrict__ row_seat,
                    float penalty, const float *__restrict__ inv_temperature,
@@ -200,7 +193,10 @@ sample_pick_kernel(const float *__restrict__ logits, int vocab, int chunk_tokens
                    const unsigned int *__restrict__ rng_key, const unsigned int *__restrict__ rng_step,
                    unsigned char *mark_mask /* may be penalty_mask */, const int *__restrict__ mark_seat,
                    int *__restrict__ out_tokens, int *__restrict__ host_tokens) {
-    const int row = blockIdx.x, lane = threadIdx.x;
+    constexpr int WAVES = SAMPLE_THREADS / KVA_WAVE, GROUPS = SCAN_TOKENS / SAMPLE_THREADS;
+    __shared__ float wave_s[2][WAVES];
+    __shared__ int found_by[2][WAVES];
+    const int row = blockIdx.x, lane = threadIdx.x % KVA_WAVE, wave = __builtin_amdgcn_readfirstlane(threadIdx.x / KVA_WAVE);
     const ChunkRecord *rec = records + (size_t)row * chunks;
     // this lane's chunks: a contiguous run, so that lane order is chunk order
     const int per_lane = (chunks + KVA_WAVE - 1) / KVA_WAVE;
@@ -214,36 +210,29 @@ sample_pick_kernel(const float *__restrict__ logits, int vocab, int chunk_tokens
     if (inv_t > 0.f && !bad_row) {
         const float top = b.value;
         // chunk sums brought to the row maximum, summed per lane, scanned over the lanes
-        float weight[PICK_CHUNKS_PER_LANE];
+        auto weight = [&](int c) { return rec[c].sum > 0.f ? rec[c].sum * expf((rec[c].top - top) * inv_t) : 0.f; };
         float mine = 0.f;
-#pragma unroll
-        for (int i = 0; i < PICK_CHUNKS_PER_LANE; ++i) {
-            const int c = c0 + i;
-            weight[i] = (i < per_lane && c < c1 && rec[c].sum > 0.f) ? rec[c].sum * expf((rec[c].top - top) * inv_t) : 0.f;
-            mine += weight[i];
-        }
+        for (int c = c0; c < c1; ++c) mine += weight(c);
         const float upto = wave_prefix_sum(mine);
         const float total = __shfl(upto, KVA_WAVE - 1, KVA_WAVE);
         bad_row = !(total > 0.f) || total == INFINITY;
         const float target = counter_uniform(seed, rng_key[row], rng_step[row]) * total;
         // the first lane whose chunks reach past the target holds the chunk
-        int owner = first_lane(target < upto);
+        const int owner = first_lane(target < upto);
         int chunk = -1;
         float before = 0.f;
         if (lane == owner) {
             float run = upto - mine, last_before = run;
             int last_chunk = c0;
-#pragma unroll
-            for (int i = 0; i < PICK_CHUNKS_PER_LANE; ++i) {
-                if (chunk < 0 && i < per_lane && c0 + i < c1) {
-                    if (target < run + weight[i]) {
-                        chunk = c0 + i;
-                        before = run;
-                    } else {
-                        last_before = run;
-                        last_chunk = c0 + i;
-                        run += weight[i];
-                    }
+            for (int c = c0; c < c1 && chunk < 0; ++c) {
+                const float w = weight(c);
+                if (target < run + w) {
+                    chunk = c;
+                    before = run;
+                } else {
+                    last_before = run;
+                    last_chunk = c;
+                    run += w;
                 }
             }
             if (chunk < 0) {                 // rounding between the lane's own sum and the scan's
@@ -255,9 +244,8 @@ sample_pick_kernel(const float *__restrict__ logits, int vocab, int chunk_tokens
             // the target landed on the total through rounding: the last token of the last chunk
             // that weighs anything (before = -inf puts the target past every span below)
             int last = -1;
-#pragma unroll
-            for (int i = 0; i < PICK_CHUNKS_PER_LANE; ++i)
-                if (i < per_lane && c0 + i < c1 && weight[i] > 0.f) last = c0 + i;
+            for (int c = c0; c < c1; ++c)
+                if (weight(c) > 0.f) last = c;
 #pragma unroll
             for (int off = KVA_WAVE / 2; off > 0; off >>= 1) last = max(last, __shfl_xor(last, off, KVA_WAVE));
             chunk = last < 0 ? chunks - 1 : last;
@@ -266,31 +254,65 @@ sample_pick_kernel(const float *__restrict__ logits, int vocab, int chunk_tokens
             chunk = __shfl(chunk, owner, KVA_WAVE);
             before = __shfl(before, owner, KVA_WAVE);
         }
-        // inside the chunk: lanes own contiguous spans; the same scan finds the lane, which walks
+        // inside the chunk, 4,096 tokens at a time, a quarter a wavefront, lane = token: of 64 neighbouring tokens the
+        // sum first, the place inside only where the target is
         const int begin = chunk * chunk_tokens, end = min(begin + chunk_tokens, vocab);
-        const int span = (end - begin + KVA_WAVE - 1) / KVA_WAVE;
-        const int t0 = min(begin + lane * span, end), t1 = min(t0 + span, end);
         const float *rl = logits + (size_t)row * vocab;
         const unsigned char *mk = mask_row(penalty_mask, row_seat, row, vocab);
-        const float inner = target - before;
-        float local = 0.f;
-        for (int t = t0; t < t1; ++t) local += token_weight(penalised(rl[t], mk, t, penalty), top, inv_t);
-        const float reach = wave_prefix_sum(local);
-        owner = first_lane(t0 < t1 && inner < reach);
-        int found = end - 1;                 // past every span's reach (rounding): the chunk's last token
-        if (lane == owner) {
-            float acc = reach - local;
-            found = t1 - 1;
-            for (int t = t0; t < t1; ++t) {
-                acc += token_weight(penalised(rl[t], mk, t, penalty), top, inv_t);
-                if (inner < acc) {
-                    found = t;
-                    break;
+        float inner = target - before;
+        token = end - 1;                     // past every reach (rounding): the chunk's last token
+        for (int base = begin, turn = 0; base < end; base += SCAN_TOKENS, turn ^= 1) {
+            float w[GROUPS];
+            const int first = base + wave * (SCAN_TOKENS / WAVES) + lane;
+#pragma unroll
+            for (int i = 0; i < GROUPS; ++i) w[i] = first + KVA_WAVE * i < end ? rl[first + KVA_WAVE * i] : -INFINITY;
+            float all = 0.f;
+#pragma unroll
+            for (int i = 0; i < GROUPS; ++i) {
+                if (mk != nullptr && first + KVA_WAVE * i < end) w[i] = penalised(w[i], mk, first + KVA_WAVE * i, penalty);
+                w[i] = token_weight(w[i], top, inv_t);
+            }
+            float sums[GROUPS];
+#pragma unroll
+            for (int i = 0; i < GROUPS; ++i) {
+                sums[i] = wave_sum_valu(w[i]);
+                all += sums[i];
+            }
+            if (lane == 0) wave_s[turn][wave] = all;
+            __syncthreads();
+            float here = inner;
+            for (int v = 0; v < wave; ++v) here -= wave_s[turn][v];
+            int found = -1;
+            if (here < all && (wave == 0 || here >= 0.f)) {       // (an earlier wavefront's share holds it: negative)
+                float run = 0.f;
+                bool done = false;
+#pragma unroll
+                for (int i = 0; i < GROUPS; ++i) {
+                    if (!done && here < run + sums[i]) {
+                        const float reach = run + wave_prefix_sum(w[i]);
+                        const int at = first_lane(here < reach);
+                        // (rounding between the sum and the scan: the last of the 64 that weighs anything)
+                        const unsigned long long weighs = __ballot(w[i] > 0.f);
+                        found = first - lane + KVA_WAVE * i + (at >= 0 ? at : weighs ? 63 - __clzll((long long)weighs) : 0);
+                        done = true;
+                    }
+                    run += sums[i];
                 }
             }
+            if (lane == 0) found_by[turn][wave] = found;
+            __syncthreads();
+            int hit = -1;
+#pragma unroll
+            for (int v = WAVES - 1; v >= 0; --v) hit = found_by[turn][v] >= 0 ? found_by[turn][v] : hit;
+            if (hit >= 0) {
+                token = hit;
+                break;
+            }
+#pragma unroll
+            for (int v = 0; v < WAVES; ++v) inner -= wave_s[turn][v];
         }
-        token = __shfl(found, owner < 0 ? 0 : owner, KVA_WAVE);
     }
+    if (wave != 0) return;
     // A row without a finite best logit (all NaN, all -inf) has no token to name, greedy or sampled,
     // and neither has a temperature row whose weights do not add up to a positive finite total.
     // Such a row gets KVA_NO_TOKEN (-1): the host sees it and ends the request with an error, and
@@ -325,6 +347,14 @@ extern "C" int kva_host_memory_is_mapped(void *host) {
     return dev != nullptr ? 1 : 0;
 }
 
+// Queues a copy from pinned host memory.
+extern "C" int kva_upload(void *device, const void *host, long long bytes, hipStream_t stream) {
+    KVA_REQUIRE(device && host && bytes >= 0, "upload: missing operand");
+    const hipError_t e = hipMemcpyAsync(device, host, (size_t)bytes, hipMemcpyHostToDevice, stream);
+    KVA_REQUIRE(e == hipSuccess, "upload: %s", hipGetErrorString(e));
+    return KVA_OK;
+}
+
 // host_tokens (optional): pinned host memory (hipHostMalloc, torch's pin_memory) with room for a token
 // per row; the kernel that chooses the tokens writes them there as well, which saves the copy
 // that would otherwise follow it on the stream.  Refused unless the runtime says the memory is
@@ -352,12 +382,14 @@ extern "C" int kva_sample(int *out_tokens, const float *logits, int rows, int vo
                 "sample: temperature rows need inv_temperature, rng_key and rng_step");
     KVA_REQUIRE(workspace != nullptr || rows == 0, "sample: a workspace of kva_sample_workspace_bytes is needed");
     if (rows == 0) return KVA_OK;
-    const int chunk_tokens = (vocab + chunks - 1) / chunks;
+    // chunks start at multiples of four tokens (the last ones may be empty)
+    const int chunk_tokens = ((vocab + chunks - 1) / chunks + 3) / 4 * 4;
+    const bool vec = vocab % 4 == 0 && (uintptr_t)logits % 16 == 0;
     ChunkRecord *records = (ChunkRecord *)workspace;
     const float *inv_t = any_sampled ? inv_temperature : nullptr;
-    hipLaunchKernelGGL(sample_scan_kernel, dim3(chunks, rows), dim3(SAMPLE_THREADS), 0, stream, logits,
+    hipLaunchKernelGGL(vec ? sample_scan_kernel<true> : sample_scan_kernel<false>, dim3(chunks, rows), dim3(SAMPLE_THREADS), 0, stream, logits,
                        vocab, chunk_tokens, penalty_mask, row_seat, penalty, inv_t, records);
-    hipLaunchKernelGGL(sample_pick_kernel, dim3(rows), dim3(KVA_WAVE), 0, stream, logits, vocab,
+    hipLaunchKernelGGL(sample_pick_kernel, dim3(rows), dim3(SAMPLE_THREADS), 0, stream, logits, vocab,
                        chunk_tokens, chunks, penalty_mask, row_seat, penalty, inv_t, records, seed, rng_key,
                        rng_step, mark_mask, mark_seat, out_tokens, host_mapped);
     KVA_CHECK_LAUNCH("sample");

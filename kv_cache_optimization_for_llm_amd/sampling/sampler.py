@@ -46,8 +46,14 @@ class SampleRow:
     apply_penalty: bool = False
 
 
-def _as_i32(values: Sequence[int]) -> np.ndarray:
-    return (np.asarray(values, dtype=np.int64) & 0xFFFFFFFF).astype(np.uint32).view(np.int32)
+class _Staging:
+    """Per-row arguments on their way up: pinned memory, seen as int32, uint32 and float32 ``[5, rows]``."""
+
+    def __init__(self, rows: int):
+        self.pinned = torch.zeros((5, rows), dtype=torch.int32, pin_memory=True)
+        self.i32 = self.pinned.numpy()
+        self.u32, self.f32 = self.i32.view(np.uint32), self.i32.view(np.float32)
+        self.sent = None                    # an event behind the copy
 
 
 class PendingTokens:
@@ -86,26 +92,37 @@ class Sampler:
         self._landing_next = 0
         # per-row arguments of a sampling (temperatures, random-stream keys and steps, seats)
         self._args_dev: Optional[torch.Tensor] = None
-        self._args_host: List[tuple] = []
+        self._args_host: List[_Staging] = []
+        self._args_views: dict = {}
         self._args_next = 0
 
+    def chunks_for(self, rows: int) -> int:
+        """Workgroups a row of the first kernel: about eight a compute unit over all rows, never more tokens each than
+        it holds in registers (both kernels over 64 rows of 128,256: 14.2 us with 32 workgroups a row, 17 with 16 or 64, 24
+        with 128)."""
+        return min(self.chunks, max(-(-self.vocab_size // 4096), 2048 // max(rows, 1)))
+
     def _row_arguments(self, n: int):
-        """A pinned staging array [5, capacity] int32 to fill (float rows as their bits) and the
-        device array it is copied to by :meth:`_send_row_arguments`."""
+        """(a staging array [5, n] of int32 in pinned memory to fill, the same as uint32 and as float, the device arrays
+        its rows go to by :func:`ops.kernels.upload`, what to tell when it has been sent) for the next sampling of n
+        rows.  Slices and views are made once per number of rows: they cost more than what is done with them."""
         if self._args_dev is None or self._args_dev.shape[1] < n:
             cap = max(64, n)
             self._args_dev = torch.zeros((5, cap), dtype=torch.int32, device=self.device)
-            self._args_host = [(torch.zeros((5, cap), dtype=torch.int32, pin_memory=True), torch.cuda.Event())
-                               for _ in range(3)]
+            self._args_host = [_Staging(cap) for _ in range(3)]
+            self._args_views.clear()
+        views = self._args_views.get(n)
+        if views is None:
+            rows = [self._args_dev[i, :n] for i in range(5)]
+            rows[0] = rows[0].view(torch.float32)
+            if len(self._args_views) >= 256:
+                self._args_views.clear()
+            views = self._args_views[n] = rows
         self._args_next = (self._args_next + 1) % len(self._args_host)
-        staging, copied = self._args_host[self._args_next]
-        copied.synchronize()             # its last copy has left it (three steps ago)
-        return staging.numpy(), self._args_dev
-
-    def _send_row_arguments(self) -> None:
-        staging, copied = self._args_host[self._args_next]
-        self._args_dev.copy_(staging, non_blocking=True)
-        copied.record()
+        staging = self._args_host[self._args_next]
+        if staging.sent is not None:
+            staging.sent.synchronize()      # its last copy has left it (three steps ago)
+        return staging, views
 
     def reset_seat(self, seat: int, emitted: Sequence[int] = ()) -> None:
         """A request takes the seat: clear its mask and mark what it has emitted before (a
@@ -157,26 +174,28 @@ class Sampler:
         if any_sampled or self.mask is not None:
             # the per-row arguments go up in one copy from pinned memory (five small pageable
             # tensors, each copied by itself, were 0.4 ms of host time apiece in a serving loop)
-            host_args, dev_args = self._row_arguments(n)
+            staging, (dev_t, dev_key, dev_step, dev_seat, dev_mark) = self._row_arguments(n)
             if any_sampled:
-                host_args[0, :n] = np.asarray([1.0 / r.temperature if r.temperature > 0 else 0.0 for r in rows],
-                                              dtype=np.float32).view(np.int32)
-                host_args[1, :n] = _as_i32([r.rng_key for r in rows])
-                host_args[2, :n] = _as_i32([r.rng_step for r in rows])
-                inv_t, key, step = dev_args[0, :n].view(torch.float32), dev_args[1, :n], dev_args[2, :n]
+                staging.f32[0, :n] = [1.0 / r.temperature if r.temperature > 0 else 0.0 for r in rows]
+                staging.u32[1, :n] = [r.rng_key & 0xFFFFFFFF for r in rows]
+                staging.u32[2, :n] = [r.rng_step & 0xFFFFFFFF for r in rows]
+                inv_t, key, step = dev_t, dev_key, dev_step
             if use_mask:
-                host_args[3, :n] = [r.seat if r.apply_penalty else -1 for r in rows]
-                seat_t = dev_args[3, :n]
+                staging.i32[3, :n] = [r.seat if r.apply_penalty else -1 for r in rows]
+                seat_t = dev_seat
             if self.mask is not None:
                 # every token a request emits is marked in its mask row, by the launch that chooses it
-                host_args[4, :n] = [r.seat for r in rows]
-                mark_seat = dev_args[4, :n]
-            self._send_row_arguments()
-        K.sample(logits, out, chunks=self.chunks, inv_temperature=inv_t, seed=self.seed, rng_key=key,
-                 rng_step=step, penalty_mask=self.mask if use_mask else None, row_seat=seat_t,
-                 penalty=self.penalty, mark_mask=self.mask if mark_seat is not None else None,
-                 mark_seat=mark_seat, host_tokens=host if self._kernel_writes_host else None)
-        if not self._kernel_writes_host:
-            host[:n].copy_(out, non_blocking=True)
-        event.record()
+                staging.i32[4, :n] = [r.seat for r in rows]
+                mark_seat = dev_mark
+            staging.sent = event
+            K.upload(staging.pinned, self._args_dev)
+        try:
+            K.sample(logits, out, chunks=self.chunks_for(n), inv_temperature=inv_t, seed=self.seed, rng_key=key,
+                     rng_step=step, penalty_mask=self.mask if use_mask else None, row_seat=seat_t,
+                     penalty=self.penalty, mark_mask=self.mask if mark_seat is not None else None,
+                     mark_seat=mark_seat, host_tokens=host if self._kernel_writes_host else None)
+            if not self._kernel_writes_host:
+                host[:n].copy_(out, non_blocking=True)
+        finally:
+            event.record()
         return PendingTokens(host, event, n)

@@ -810,6 +810,40 @@ def test_sampler_against_flat_cdf(vocab, gpu):
     assert marked == [[1, 20], [2, 10], [3, 30]]
 
 
+@pytest.mark.parametrize("chunks", [1, 3, 64])
+@pytest.mark.parametrize("vocab", [1, 63, 4095, 4096, 4097, 10002, 32000])
+def test_sampler_at_the_edges_of_what_a_workgroup_holds(vocab, chunks, gpu):
+    """Chunks of more, as many and fewer tokens than a workgroup holds in registers, rows that do not start at multiples
+    of 16 bytes, empty last chunks, masked, infinite and NaN logits: the flat CDF's token, or (rounding) one whose
+    cumulative weight is within 1e-5 of the target."""
+    rows, g = 12, torch.Generator().manual_seed(vocab + chunks)
+    lg = torch.randn(rows, vocab, generator=g) * 3
+    lg[3] = float("-inf")
+    lg[3, vocab // 2] = 1.0
+    lg[4, ::2] = float("nan")
+    lg[5] = 0.25                                                    # all equal
+    mask = (torch.rand(rows, vocab, generator=g) < 0.3).to(torch.uint8)
+    inv_t = torch.tensor([0.0, 1.25, 0.5, 2.0, 1.0, 1.0, 0.0, 1.0, 4.0, 1.0, 0.0, 1.0])
+    seat = torch.tensor([r if r % 3 else -1 for r in range(rows)], dtype=torch.int32)
+    key, step = torch.arange(rows, dtype=torch.int32) * 8, torch.arange(rows, dtype=torch.int32) + 5
+    out = torch.empty(rows, dtype=torch.int32, device=gpu)
+    K.sample(lg.to(gpu), out, chunks=chunks, inv_temperature=inv_t.to(gpu), seed=77, rng_key=key.to(gpu), rng_step=step.to(gpu),
+             penalty_mask=mask.to(gpu), row_seat=seat.to(gpu), penalty=1.15)
+    for r in range(rows):
+        l, got = lg[r].double().numpy().copy(), int(out[r])
+        if seat[r] >= 0:
+            l = plain.penalised(l, np.nonzero(mask[r].numpy())[0], 1.15)
+        l[np.isnan(l)] = -np.inf
+        if not (l > -np.inf).any():
+            assert got == -1, r
+        elif inv_t[r] == 0:
+            assert got == int(np.argmax(l.astype(np.float32))), r
+        else:
+            w = np.exp((l - l.max()) * float(inv_t[r]))
+            cdf, u = np.cumsum(w) / w.sum(), plain.counter_uniform(77, int(key[r]), int(step[r]))
+            assert w[got] > 0 and (cdf[got - 1] if got else 0.0) - 1e-5 <= u <= cdf[got] + 1e-5, r
+
+
 def test_sampler_distribution_and_boundaries(gpu):
     """python/sampling_reference.py:110-134: top-8 frequencies within 5 % over 40 000 draws."""
     vocab = 5000
