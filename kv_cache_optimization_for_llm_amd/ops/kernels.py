@@ -960,6 +960,48 @@ def latent_encode_cache(y: torch.Tensor, kv_off: int, q_lat: Optional[torch.Tens
         1 if interleaved else 0, dtype_code(y.dtype), _stream()), "latent_encode_cache")
 
 
+def latent_prompt_supported(dim: int, rot: int, vdim: int, rank: int) -> bool:
+    """Whether :func:`latent_prompt` has an instance for these sizes."""
+    return bool(hip_lib().kva_latent_prompt_supported(int(dim), int(rot), int(vdim), int(rank)))
+
+
+def latent_prompt(q: torch.Tensor, cache: torch.Tensor, w: torch.Tensor, out: torch.Tensor, block_table: torch.Tensor,
+                  entry_seat: torch.Tensor, entry_q_start: torch.Tensor, entry_start_pos: torch.Tensor, cos: torch.Tensor,
+                  sin: torch.Tensor, interleaved: bool, scale: float, context: int, longest: int,
+                  sinks: Optional[torch.Tensor] = None, gates: Optional[torch.Tensor] = None) -> torch.Tensor:
+    """Causal attention of whole entries (no window) over the rows of ``cache`` ``[pages, page_size, rank + rot]`` with
+    keys and values expanded per head: ``q`` ``[T, heads, dim + rot]`` (its last ``rot`` elements are rotated here), ``w``
+    bf16 ``[heads (dim + vdim), rank]`` (all heads' key expansions, then all heads' value expansions) in operand order
+    (:func:`moe_tiled_weight`), ``out`` ``[T, heads * vdim]``.  ``gates`` as in :func:`heads_matmul`.  No entry has more than
+    ``longest`` tokens or ends past position ``context``."""
+    T, heads, key = q.shape
+    rot = 2 * cos.shape[1]
+    rank, dim = cache.shape[2] - rot, key - rot
+    vdim = out.shape[1] // heads
+    entries = entry_seat.shape[0]
+    if not latent_prompt_supported(dim, rot, vdim, rank) or cache.dim() != 3 or w.shape != (heads * (dim + vdim), rank) \
+            or out.shape != (T, heads * vdim) or q.stride(2) != 1 or not (q.dtype == cache.dtype == w.dtype == out.dtype == torch.bfloat16):
+        raise KernelError(f"latent_prompt: q {tuple(q.shape)}, cache {tuple(cache.shape)}, w {tuple(w.shape)}, out {tuple(out.shape)} do not fit")
+    if entry_q_start.shape != (entries + 1,) or entry_start_pos.shape != (entries,) or cos.shape != sin.shape:
+        raise KernelError("latent_prompt: entries' seats, first rows and first positions, tables [positions, rot / 2]")
+    gate = [None, 0, 0, 0]
+    if gates is not None:
+        element = gates.dim() == 3
+        if gates.shape != ((T, heads, vdim) if element else (T, heads)) or gates.dtype != q.dtype or gates.stride(-1) != 1:
+            raise KernelError(f"latent_prompt: gates {tuple(gates.shape)} do not fit {T} rows of {heads} heads")
+        gate = [_dev(gates, "gates", contiguous=False), gates.stride(0), gates.stride(1) if element else 1, 1 if element else 0]
+    kv = torch.empty((entries * int(context), heads * (dim + vdim)), dtype=q.dtype, device=q.device)
+    turned = torch.empty((entries * int(context), rot), dtype=q.dtype, device=q.device)
+    check(hip_lib().kva_latent_prompt(
+        _dev(out, "out"), _dev(q, "q", contiguous=False), q.stride(0), q.stride(1), _dev(cache, "cache"), _dev(w, "w"), _dev(kv, "kv"),
+        _dev(turned, "turned"), _dev(block_table, "block_table", torch.int32), block_table.shape[1],
+        _dev(entry_seat, "entry_seat", torch.int32), _dev(entry_q_start, "entry_q_start", torch.int32),
+        _dev(entry_start_pos, "entry_start_pos", torch.int32), entries, _dev(cos, "cos", torch.float32), _dev(sin, "sin", torch.float32),
+        1 if interleaved else 0, _opt(sinks, "sinks", torch.float32), *gate, cache.shape[1], heads, rank, int(context), int(longest),
+        float(scale), _stream()), "latent_prompt")
+    return out
+
+
 def heads_matmul(x: torch.Tensor, w: torch.Tensor, out: torch.Tensor, gates: Optional[torch.Tensor] = None,
                  rotate: Optional[tuple] = None) -> torch.Tensor:
     """``out[t, h, :] = w[h] @ x[t, h, :]`` for ``w`` ``[heads, N, K]``.  ``x`` ``[T, heads, K]`` and
@@ -2298,6 +2340,7 @@ KERNEL_CLASSES = {
     "qk_encode_cache": "rope + cache write", "latent_encode_cache": "rope + cache write",
     "heads_matmul": "per-head products",
     "attention_mfma_rope": "attention",
+    "latent_prompt": "attention (matrix cores)",
     "gemm_nt_f32": "gemm fp32", "gemm_vendor": "gemm (vendor library)",
     "gemm_skinny": "gemm (few rows)", "gemm_skinny_qkv_rope": "gemm (few rows)",
     "gemv": "gemm (few rows)", "gemv_qkv_rope": "gemm (few rows)", "gemv_merged": "gemm (few rows)",

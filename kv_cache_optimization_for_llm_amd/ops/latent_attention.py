@@ -41,6 +41,25 @@ def choose_ranges(items: int, max_context: int, visible: int = 0, workgroups: in
     return -(-max_context // per), per
 
 
+# Steps whose entries all have so many tokens, and contexts of at most so many times as many, expand keys and values
+# (ops.kernels.latent_prompt) while the expanded contexts stay below so many bytes.  Whole steps of 8 layers (16 heads of
+# 128 + 64 / 128, rank 512), over the cached rows -> expanded, ms: one prompt of 64 / 128 / 256 / 2,048 tokens 1.36 / 1.61 /
+# 1.67 / 4.77 -> 1.30 / 1.51 / 1.51 / 3.44; four of 128 / 256 behind 1,024: 2.41 / 3.16 -> 1.98 / 2.57; 128 / 192 / 256
+# behind 2,048: 1.87 / 2.36 / 2.21 -> 1.95 / 2.21 / 1.95; 256 behind 6,000: 2.82 -> 2.86; 512 behind 7,000: 4.17 -> 3.26.
+# Error of the logits against 64 bits: 0.0084 / 0.0082 and 0.0085 / 0.0081 (eight prompts of 512 / one of 2,048).
+EXPAND_FROM = 64
+EXPAND_CONTEXTS = 16
+EXPAND_BYTES = 512 << 20
+
+
+def expands(batch, heads: int, dim: int, rot: int, vdim: int, rank: int, window: int, dtype) -> bool:
+    """Whether a step's prompt portions attend over expanded keys and values."""
+    return (dtype == torch.bfloat16 and window <= 0 and batch.min_q_len >= EXPAND_FROM
+            and batch.max_context <= EXPAND_CONTEXTS * batch.min_q_len
+            and batch.num_entries * batch.max_context * (heads * (dim + vdim) + rot) * 2 <= EXPAND_BYTES
+            and K.latent_prompt_supported(dim, rot, vdim, rank))
+
+
 def latent_attention(q_lat: torch.Tensor, out: torch.Tensor, kv, batch, scale: float, window: int = 0,
                      keep_first: int = 0, sinks=None) -> torch.Tensor:
     """Causal attention of the step's tokens over the rows of ``kv.arrays["latent"]``

@@ -9,13 +9,15 @@ elements):
     score_h(i, j) = (q_p[h]_i . U_k[h] c_j + q_r[h]_i . k_r_j) * scale
     out_h(i)      = sum_j p_h(i, j) U_v[h] c_j
 
-Keys and values are never expanded.  The key expansion moves to the query side,
+For decoded tokens keys and values are not expanded.  The key expansion moves to the query side,
 ``q_p . U_k c = (U_k^T q_p) . c``, so a head's query becomes a row ``[U_k[h]^T q_p[h] ; q_r[h]]`` of
 the cache's own layout and every head attends over the same rows (one shared "kv head" of
 ``rank + rot_dim`` elements whose first ``rank`` are also the value); the value expansion moves
 behind the attention, ``sum_j p U_v c_j = U_v (sum_j p c_j)``.  What a step costs per cached token
 is then independent of the number of heads' key and value sizes, and a prompt cut anywhere
-continues from the rows alone.
+continues from the rows alone.  A prompt's tokens see every key many times: where the sizes have a kernel for it
+(``ops.latent_attention.expands``) a step of prompt portions expands the keys and values of its entries' contexts,
+rounded to bf16, and attends over those.
 
 Options: queries through a latent of their own (``c_q = RMSnorm(W_dq x)``, ``q = W_uq c_q``), a softmax sink
 per head (``exp(sink_h)`` added to the denominator; no key, no value, not scaled), a sigmoid output
@@ -115,6 +117,10 @@ class LatentAttention(Mixer):
         # U_k per head, transposed: the query-side product reads [heads, rank, dim]
         self.up_k_t = tensors[n["up_k"]].view(H, self.head_dim, self.rank).transpose(1, 2).contiguous()
         self.up_v = tensors[n["up_v"]].view(H, self.value_dim, self.rank).contiguous()
+        # both expansions joined, for prompts (ops.kernels.latent_prompt)
+        joined = torch.cat([tensors[n["up_k"]], tensors[n["up_v"]]], dim=0)
+        self.up_kv = K.moe_tiled_weight(joined[None])[0] if joined.dtype == torch.bfloat16 and joined.is_cuda \
+            and K.latent_prompt_supported(self.head_dim, self.rot_dim, self.value_dim, self.rank) else None
         self.norm_weight = tensors[n["down_norm"]].contiguous()
         self.sinks = tensors[n["sink"]].to(torch.float32).contiguous() if self.has_sink else None
 
@@ -125,6 +131,7 @@ class LatentAttention(Mixer):
     def activation_elements(self) -> int:
         H = self.num_heads
         return (self.proj.out_features if self.proj is not None else 0) + H * (self.key_dim + self.rank + self.value_dim) \
+            + H * (self.head_dim + self.value_dim) + self.rot_dim \
             + (self.q_rank + H * (self.head_dim + self.rot_dim) if self.q_rank else 0) + self.hidden_size
 
     def forward(self, x, ctx: MixerContext, tail=None):
@@ -145,16 +152,21 @@ class LatentAttention(Mixer):
                               kv.slot_mapping if write else None, H, self.head_dim, self.rank, interleaved=interleaved,
                               c_q=c_q, q_norm_weight=self.q_norm_weight)
         q = (self.q_up(c_q) if self.q_rank else y[:, :self.kv_off]).view(T, H, self.head_dim + self.rot_dim)
+        gates = y[:, self.gate_off:self.gate_off + self._gates()] if self.has_gate else None
+        if self.gate_elements:
+            gates = gates.unflatten(1, (H, self.value_dim))
+        out = torch.empty((T, H * self.value_dim), dtype=x.dtype, device=x.device)
+        if self.up_kv is not None and lat_ops.expands(batch, H, self.head_dim, self.rot_dim, self.value_dim, self.rank, self.window, x.dtype) \
+                and q.stride(0) % 8 == 0 and q.data_ptr() % 16 == 0:
+            K.latent_prompt(q, kv.arrays["latent"], self.up_kv, out, kv.block_table, batch.entry_seat, batch.entry_q_start,
+                            batch.entry_start_pos, cos, sin, interleaved, self.scale, batch.max_context, batch.max_q_len, self.sinks, gates)
+            return self.o(out)
         # queries from a latent exist only now: their rotated parts are turned in the expansion's launch
         rotate = (q[:, :, self.head_dim:], q_lat[:, :, self.rank:], cos, sin, batch.positions, interleaved) if self.q_rank else None
         # the key expansion on the query side: q_lat[:, h, :rank] = U_k[h]^T q_p[h]
         lat_ops.heads_product(q[:, :, :self.head_dim], self.up_k_t, q_lat[:, :, :self.rank], rotate=rotate)
         o_lat = torch.empty((T, H, self.rank), dtype=x.dtype, device=x.device)
         lat_ops.latent_attention(q_lat, o_lat, kv, batch, self.scale, self.window, self.keep_first, self.sinks)
-        out = torch.empty((T, H * self.value_dim), dtype=x.dtype, device=x.device)
         # the value expansion behind the attention, the output gate in the same pass
-        gates = y[:, self.gate_off:self.gate_off + self._gates()] if self.has_gate else None
-        if self.gate_elements:
-            gates = gates.unflatten(1, (H, self.value_dim))
         lat_ops.heads_product(o_lat, self.up_v, out.view(T, H, self.value_dim), gates=gates)
         return self.o(out)

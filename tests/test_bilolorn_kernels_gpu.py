@@ -329,6 +329,60 @@ def test_rows_of_several_entries_in_items_of_both_sizes(heads, rank, rot, page, 
 
 
 # ---------------------------------------------------------------- feed-forwards
+@pytest.mark.parametrize("interleaved, gate, sink", [(True, "element", True), (False, "head", False), (True, None, True)])
+@pytest.mark.parametrize("heads, rank, page, entries", [(1, 32, 16, [(0, 1)]), (3, 96, 16, [(0, 63), (5, 64), (200, 65)]), (16, 512, 16, [(0, 300), (700, 129)]),
+                                                        (4, 512, 48, [(31, 257), (0, 33), (96, 128), (1, 1)])])
+def test_prompts_over_expanded_keys_and_values(heads, rank, page, entries, interleaved, gate, sink, gpu):
+    """Entries (first position, tokens) whose tokens and contexts end inside, at and behind tiles of 64 tokens, blocks of 32 keys
+    and tiles of 128 positions, on pages in no order, a context bound larger than any of them."""
+    d, rot, dv, T = 128, 64, 128, sum(n for _, n in entries)
+    context = max(s + n for s, n in entries) + 37
+    blocks = -(-context // page)
+    g = torch.Generator().manual_seed(heads + rank)
+    table = torch.randperm(len(entries) * blocks, generator=g).view(len(entries), blocks).to(torch.int32)
+    seats = torch.randperm(len(entries), generator=g).to(torch.int32)
+    cache = torch.full((len(entries) * blocks, page, rank + rot), float("nan"), dtype=torch.bfloat16)      # what nobody wrote
+    rows = {}
+    for e, (start, n) in enumerate(entries):
+        rows[e] = rnd((start + n, rank + rot), 10 + e, torch.bfloat16)
+        for p in range(start + n):
+            cache[int(table[seats[e], p // page]), p % page] = rows[e][p]
+    q = rnd((T, heads, d + rot), 1, torch.bfloat16)
+    up_k, up_v = rnd((heads * d, rank), 2, torch.bfloat16, rank ** -0.5), rnd((heads * dv, rank), 3, torch.bfloat16, rank ** -0.5)
+    position = RotaryEncoding(head_dim=rot, max_positions=2048, theta=10000.0, frequencies="plain_f64", pairing="interleaved" if interleaved else "half")
+    cos, sin = position.tables(gpu)
+    sinks = rnd((heads,), 4, scale=2.0) if sink else None
+    gates = None if gate is None else rnd((T, heads, dv) if gate == "element" else (T, heads), 5, torch.bfloat16)
+    first = torch.tensor(np.cumsum([0] + [n for _, n in entries]), dtype=torch.int32)
+    out = torch.full((T, heads * dv), float("nan"), dtype=torch.bfloat16, device=gpu)
+    w = K.moe_tiled_weight(torch.cat([up_k, up_v])[None].to(gpu))[0]
+    K.latent_prompt(q.to(gpu), cache.to(gpu), w, out, table.to(gpu), seats.to(gpu), first.to(gpu),
+                    torch.tensor([s for s, _ in entries], dtype=torch.int32, device=gpu), cos, sin, interleaved, 192 ** -0.5, context,
+                    max(n for _, n in entries), None if sinks is None else sinks.to(gpu), None if gates is None else gates.to(gpu))
+    c64, s64 = cos.double().cpu(), sin.double().cpu()
+    for e, (start, n) in enumerate(entries):
+        at, lat = slice(int(first[e]), int(first[e]) + n), rows[e].double()
+        k = torch.cat([(lat[:, :rank] @ up_k.double().T).view(-1, heads, d), lat[:, None, rank:].expand(-1, heads, -1)], -1)
+        v = (lat[:, :rank] @ up_v.double().T).view(-1, heads, dv)
+        x, pos = q[at].double(), torch.arange(start, start + n)
+        c, s = c64[pos][:, None], s64[pos][:, None]
+        a, b = (x[..., d::2], x[..., d + 1::2]) if interleaved else (x[..., d:d + rot // 2], x[..., d + rot // 2:])
+        turned = torch.stack([a * c - b * s, b * c + a * s], -1).flatten(-2) if interleaved else torch.cat([a * c - b * s, b * c + a * s], -1)
+        x = torch.cat([x[..., :d], turned], -1)
+        score = torch.einsum("thd,khd->htk", x, k) * 192 ** -0.5
+        score = score.masked_fill(torch.arange(start + n)[None, None, :] > pos[None, :, None], float("-inf"))
+        if sinks is not None:
+            score = torch.cat([score, sinks.double()[:, None, None].expand(-1, n, 1)], -1)
+        p = torch.softmax(score, -1)[..., :start + n]
+        want = torch.einsum("htk,khd->thd", p, v)
+        if gates is not None:
+            z = torch.sigmoid(gates[at].double())
+            want = want * (z if gate == "element" else z[..., None])
+        got = out[at].double().cpu().view(n, heads, dv)
+        # keys, values, rotated queries, probabilities and results are rounded to bf16 (2^-9 each, relative): their squares add up
+        assert (got - want).norm() <= 2.0 ** -9 * 5 ** 0.5 * 1.5 * want.norm(), e
+
+
 @pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
 @pytest.mark.parametrize("rows, width, ff", [(1, 64, 96), (3, 30, 25), (40, 128, 200), (300, 64, 512)])
 def test_squared_relu_feed_forward(rows, width, ff, dtype, gpu):
