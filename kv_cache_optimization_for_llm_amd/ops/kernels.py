@@ -1839,6 +1839,8 @@ def gated_delta_rule(qkv: torch.Tensor, y: torch.Tensor, beta_off: int, decay_of
     qs, seat, entries = _entries((entry_q_start, entry_seat), "gated_delta_rule")
     below, longest, floats, walks = _recurrent_plan(lengths, DELTA_RULE_CHUNKS_FROM, entries, tokens, heads, dim, vdim, y.dtype,
                                                     "gated_delta_rule")
+    if qkv.data_ptr() % 16:         # (the chunks read 16 bytes at a time, the walk element by element)
+        below, floats, walks = 1 << 30, 0, True
     operands = (_dev(out, "out"), _dev(state, "state"), seat_stride, int(state_off), _dev(qkv, "qkv"), qkv.shape[1],
                 _dev(y, "y"), dtype_code(y.dtype), y.shape[1], int(beta_off), int(decay_off),
                 _opt(a_log, "a_log", torch.float32), _opt(dt_bias, "dt_bias", torch.float32), float(unit_eps),

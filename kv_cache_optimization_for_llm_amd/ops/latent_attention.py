@@ -54,7 +54,7 @@ EXPAND_BYTES = 512 << 20
 
 def expands(batch, heads: int, dim: int, rot: int, vdim: int, rank: int, window: int, dtype) -> bool:
     """Whether a step's prompt portions attend over expanded keys and values."""
-    return (dtype == torch.bfloat16 and window <= 0 and batch.min_q_len >= EXPAND_FROM
+    return (dtype == torch.bfloat16 and window <= 0 and heads <= 1024 and batch.min_q_len >= EXPAND_FROM
             and batch.max_context <= EXPAND_CONTEXTS * batch.min_q_len
             and batch.num_entries * batch.max_context * (heads * (dim + vdim) + rot) * 2 <= EXPAND_BYTES
             and K.latent_prompt_supported(dim, rot, vdim, rank))

@@ -2,6 +2,8 @@
 norms on both sides, the query latent beside the cache write, per-head products with a gate per element and a
 rotation in the same launch, experts by token id, the squared relu, the scaled embedding gather with its second
 copy, and the mixer as a whole with one key that stands out."""
+from types import SimpleNamespace
+
 import numpy as np
 import pytest
 import torch
@@ -514,3 +516,14 @@ def test_table_experts_with_and_without_the_expert_every_token_uses(rows, width,
     w = {k: (v.double() if v.is_floating_point() else v) for k, v in state.items()}
     mlp = {"router": {"top": top}, **({"shared": {"ff": shared}} if shared else {})}
     close(got, plain.table_experts(x.double(), ids, w, "p.", mlp), TOL[dtype])
+
+
+def test_which_steps_expand_keys_and_values(gpu):
+    def step(shortest, context, entries=1):
+        return SimpleNamespace(min_q_len=shortest, max_context=context, num_entries=entries)
+    rule = lambda batch, heads=16, rot=64, rank=512, window=0, dtype=torch.bfloat16: \
+        lat_ops.expands(batch, heads, 128, rot, 128, rank, window, dtype)
+    assert rule(step(64, 1024)) and rule(step(64, 64), heads=1024)
+    assert not rule(step(63, 63)) and not rule(step(64, 1025)) and not rule(step(64, 64), heads=1025)
+    assert not rule(step(2048, 2048, 64)) and not rule(step(64, 64), window=32) and not rule(step(64, 64), dtype=torch.float32)
+    assert not rule(step(64, 64), rot=32) and not rule(step(64, 64), rank=48)

@@ -268,6 +268,24 @@ def test_gated_delta_rule_in_chunks(heads, kv_heads, dim, vdim, decays, portions
     assert (states[True][:, :4] == 0).all()
 
 
+def test_gated_delta_rule_rows_at_any_address_walk(gpu):
+    """Rows that do not start at a multiple of 16 bytes are not read by the chunks."""
+    heads, dim, vdim, n = 2, 64, 16, 200
+    g = torch.Generator().manual_seed(5)
+    rows, y = torch.randn(n, heads * (2 * dim + vdim), generator=g), torch.randn(n, 2 * heads, generator=g).to(torch.bfloat16)
+    flat = torch.empty(rows.numel() + 1, dtype=torch.float32, device="cuda")
+    got = []
+    for at, lengths in ((1, [n]), (0, None)):
+        qkv = flat[at:at + rows.numel()].view(rows.shape)
+        qkv.copy_(rows)
+        state = torch.zeros((1, heads * dim * vdim), dtype=torch.float32, device="cuda")
+        out = torch.empty((n, heads * vdim), dtype=torch.float32, device="cuda")
+        K.gated_delta_rule(qkv, y.to("cuda"), 0, heads, dev(torch.zeros(heads)), dev(torch.zeros(heads)), out, state, 0,
+                           ints([0, n]), ints([0]), heads, heads, dim, vdim, lengths=lengths)
+        got.append((out.cpu(), state.cpu()))
+    assert torch.equal(got[0][0], got[1][0]) and torch.equal(got[0][1], got[1][1])
+
+
 @pytest.mark.parametrize("portions", [(1000,), (64, 1, 70, 65)])
 @pytest.mark.parametrize("decays", ["usual", "zeros", "fixed", "fixed at zero", "none"])
 @pytest.mark.parametrize("heads, dim, vdim, act", [(3, 64, 128, None), (2, 128, 16, "silu"), (1, 64, 48, "silu")])
