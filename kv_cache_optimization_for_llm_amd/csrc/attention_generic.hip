@@ -1,6 +1,6 @@
 // Causal grouped-query attention over the paged cache: the plain kernel.
 //
-// One wavefront per (token, query head).  The query at absolute position p of its request
+// One wavefront per token and query head, or several query heads of one key head.  The query at absolute position p of its request
 // attends to keys lo..p of the same request (lo = 0, or p - window + 1 with a window, or the start of
 // p's own chunk where positions see each other only inside chunks of a fixed size), all read
 // from the cache through the request's block-table row - the step has already written this
@@ -42,93 +42,160 @@ template <> struct Vec4<bf16_t> {
     }
 };
 
-template <typename T>
+// H query heads of one key head go together: a key's and a value's elements are loaded once for all of them, and their
+// sums, which are chains of dependent additions in a fixed order, run side by side.  With `fours` (pages of a multiple of
+// 4 keys) a lane reads its value element of 4 keys at once, a row of the transposed page, and 32 keys' loads are under way
+// together; a head's additions keep their order in every variant, so its bits do too.  One key's values a load, one head a
+// wavefront -> this, fp32, us: 603 tokens of 32 heads of 64 over 8 key heads at up to 201 / 2,000 keys 253 / 731 -> 35 / 78,
+// one token at 200 / 2,000 keys 34 / 307 -> 11 / 75 (bound by the chains: 64 dependent additions a block for the score,
+// 64 for the values), heads of 128 at 2,000 keys 659 -> 185.
+template <typename T, int H>
 __global__ void __launch_bounds__(KVA_WAVE)
 attention_rowwise_kernel(T *__restrict__ out, const T *__restrict__ q, int q_row_stride,
                          const T *__restrict__ k_cache, const T *__restrict__ v_cache,
                          const int *__restrict__ block_table, int max_blocks,
                          const int *__restrict__ tok_seat, const int *__restrict__ tok_pos,
-                         int num_q_heads, int num_kv_heads, int head_dim, int value_dim, int page_size,
+                         int num_q_heads, int num_kv_heads, int head_dim, int value_dim, int page_size, int fours,
                          float scale, int window, int keep_first, int chunk, const float *__restrict__ sinks) {
-    __shared__ float q_s[ATTN_MAX_HEAD_DIM];
-    __shared__ float p_s[KVA_WAVE];
+    __shared__ __attribute__((aligned(16))) float q_s[H][ATTN_MAX_HEAD_DIM];
+    __shared__ __attribute__((aligned(16))) float p_s[H][KVA_WAVE];
     __shared__ long long voff_s[KVA_WAVE];
 
     const int t = blockIdx.x;
-    const int qh = blockIdx.y;
+    const int qh = blockIdx.y * H;
     const int lane = threadIdx.x;
     const int kvh = qh / (num_q_heads / num_kv_heads);
     const int pos = tok_pos[t];
     const int *bt = block_table + (size_t)tok_seat[t] * max_blocks;
 
     const T *qrow = q + (size_t)t * q_row_stride + (size_t)qh * head_dim;
-    for (int j = lane; j < head_dim; j += KVA_WAVE) q_s[j] = to_float(qrow[j]);
+#pragma unroll
+    for (int h = 0; h < H; ++h)
+        for (int j = lane; j < head_dim; j += KVA_WAVE) q_s[h][j] = to_float(qrow[h * head_dim + j]);
     __syncthreads();
 
     const int lo = kva_first_visible(pos, window, chunk);
-    float m = -INFINITY, l = 0.f;
-    float acc[ATTN_MAX_HEAD_DIM / KVA_WAVE] = {0.f, 0.f, 0.f, 0.f};
+    float m[H], l[H], corr[H];
+    float acc[ATTN_MAX_HEAD_DIM / KVA_WAVE][H];
+#pragma unroll
+    for (int h = 0; h < H; ++h) {
+        m[h] = -INFINITY;
+        l[h] = 0.f;
+#pragma unroll
+        for (int c = 0; c < ATTN_MAX_HEAD_DIM / KVA_WAVE; ++c) acc[c][h] = 0.f;
+    }
 
     for (int kb = keep_first > 0 ? 0 : lo / KVA_WAVE; kb <= pos / KVA_WAVE; ++kb) {
         // a block with no visible key: behind the window and past the kept first positions
         if (kb * KVA_WAVE + KVA_WAVE <= lo && kb * KVA_WAVE >= keep_first) continue;
         const int key = kb * KVA_WAVE + lane;
         const bool valid = key <= pos && (key >= lo || key < keep_first);
-        float s = -INFINITY;
-        long long row_off = 0;
+        const unsigned long long seen = __ballot(valid);
+        float s[H];
+#pragma unroll
+        for (int h = 0; h < H; ++h) s[h] = -INFINITY;
         if (valid) {
             const int page = bt[key / page_size];
-            row_off = ((long long)page * num_kv_heads + kvh) * page_size * (long long)head_dim;
-            const T *kpage = k_cache + row_off;
+            const T *kpage = k_cache + ((long long)page * num_kv_heads + kvh) * page_size * (long long)head_dim;
             const int krow = key % page_size, kc = kva_k_chunk(head_dim);
-            float dot = 0.f;
+            float dot[H];
+#pragma unroll
+            for (int h = 0; h < H; ++h) dot[h] = 0.f;
+#pragma unroll 4
             for (int j = 0; j < head_dim; j += 4) {
                 float kv[4];
                 Vec4<T>::load(kpage + kva_k_at(krow, j, page_size, kc), kv);     // (4 elements never straddle a chunk)
-                dot += q_s[j] * kv[0];
-                dot += q_s[j + 1] * kv[1];
-                dot += q_s[j + 2] * kv[2];
-                dot += q_s[j + 3] * kv[3];
+#pragma unroll
+                for (int h = 0; h < H; ++h) {
+                    const float4 qv = *reinterpret_cast<const float4 *>(&q_s[h][j]);
+                    dot[h] += qv.x * kv[0];
+                    dot[h] += qv.y * kv[1];
+                    dot[h] += qv.z * kv[2];
+                    dot[h] += qv.w * kv[3];
+                }
             }
-            s = dot * scale;
+#pragma unroll
+            for (int h = 0; h < H; ++h) s[h] = dot[h] * scale;
         }
-        const float m_new = fmaxf(m, wave_max(s));
-        const float corr = (m == -INFINITY) ? 0.f : expf(m - m_new);
-        const float p = valid ? expf(s - m_new) : 0.f;
-        l = l * corr + wave_sum(p);
-        m = m_new;
         __syncthreads();  // the previous block's p_s / voff_s have been consumed
-        p_s[lane] = p;
-        // V is stored transposed inside a page: [page, kv_head, value_dim, page_size]
-        voff_s[lane] = valid ? ((long long)bt[key / page_size] * num_kv_heads + kvh) *
-                                       (long long)value_dim * page_size + key % page_size
-                             : -1;
+#pragma unroll
+        for (int h = 0; h < H; ++h) {
+            const float m_new = fmaxf(m[h], wave_max(s[h]));
+            corr[h] = (m[h] == -INFINITY) ? 0.f : expf(m[h] - m_new);
+            const float p = valid ? expf(s[h] - m_new) : 0.f;
+            l[h] = l[h] * corr[h] + wave_sum(p);
+            m[h] = m_new;
+            p_s[h][lane] = p;
+        }
+        // V is stored transposed inside a page: [page, kv_head, value_dim, page_size].  Four keys together are of one
+        // page; where none of the four is visible, the first visible key's place is read in their stead and not used.
+        const int first = __ffsll(seen) - 1;
+        const int group = fours ? ((seen >> (lane & ~3)) & 15 ? lane : first & ~3) : (valid ? lane : first);
+        const int vkey = kb * KVA_WAVE + group;
+        voff_s[lane] = ((long long)bt[vkey / page_size] * num_kv_heads + kvh) * (long long)value_dim * page_size +
+                       vkey % page_size;
         __syncthreads();
         const int last = (pos - kb * KVA_WAVE < KVA_WAVE - 1) ? pos - kb * KVA_WAVE : KVA_WAVE - 1;
 #pragma unroll
         for (int c = 0; c < ATTN_MAX_HEAD_DIM / KVA_WAVE; ++c) {
             const int j = lane + c * KVA_WAVE;
             if (j < value_dim) {
-                float a = acc[c] * corr;
-                for (int i = 0; i <= last; ++i)
-                    if (voff_s[i] >= 0) a += p_s[i] * to_float(v_cache[voff_s[i] + (long long)j * page_size]);
-                acc[c] = a;
+                const T *vcol = v_cache + (long long)j * page_size;
+                float a[H];
+#pragma unroll
+                for (int h = 0; h < H; ++h) a[h] = acc[c][h] * corr[h];
+                if (fours) {
+                    for (int i0 = 0; i0 <= last; i0 += 32) {
+                        float v[8][4];
+#pragma unroll
+                        for (int g = 0; g < 8; ++g) Vec4<T>::load(vcol + voff_s[i0 + 4 * g], v[g]);
+                        const uint32_t these = (uint32_t)(seen >> i0);
+                        if (these != 0xffffffffu) {
+#pragma unroll
+                            for (int g = 0; g < 8; ++g)
+#pragma unroll
+                                for (int u = 0; u < 4; ++u) v[g][u] = (these >> (4 * g + u)) & 1 ? v[g][u] : 0.f;
+                        }
+#pragma unroll
+                        for (int g = 0; g < 8; ++g)
+#pragma unroll
+                            for (int h = 0; h < H; ++h) {
+                                const float4 p = *reinterpret_cast<const float4 *>(&p_s[h][i0 + 4 * g]);
+                                a[h] += p.x * v[g][0];
+                                a[h] += p.y * v[g][1];
+                                a[h] += p.z * v[g][2];
+                                a[h] += p.w * v[g][3];
+                            }
+                    }
+                } else {
+                    for (int i = 0; i <= last; ++i)
+                        if ((seen >> i) & 1) {
+                            const float v = to_float(vcol[voff_s[i]]);
+#pragma unroll
+                            for (int h = 0; h < H; ++h) a[h] += p_s[h][i] * v;
+                        }
+                }
+#pragma unroll
+                for (int h = 0; h < H; ++h) acc[c][h] = a[h];
             }
         }
     }
-    if (sinks) {
-        // one more term of the denominator, exp(sink), with no key and no value
-        const float s = sinks[qh], m_new = fmaxf(m, s);
-        const float corr = (m == -INFINITY) ? 0.f : expf(m - m_new);
-        l = l * corr + expf(s - m_new);
 #pragma unroll
-        for (int c = 0; c < ATTN_MAX_HEAD_DIM / KVA_WAVE; ++c) acc[c] *= corr;
-    }
-    T *orow = out + (size_t)t * num_q_heads * value_dim + (size_t)qh * value_dim;
+    for (int h = 0; h < H; ++h) {
+        if (sinks) {
+            // one more term of the denominator, exp(sink), with no key and no value
+            const float s = sinks[qh + h], m_new = fmaxf(m[h], s);
+            const float more = (m[h] == -INFINITY) ? 0.f : expf(m[h] - m_new);
+            l[h] = l[h] * more + expf(s - m_new);
 #pragma unroll
-    for (int c = 0; c < ATTN_MAX_HEAD_DIM / KVA_WAVE; ++c) {
-        const int j = lane + c * KVA_WAVE;
-        if (j < value_dim) orow[j] = from_float<T>(acc[c] / l);
+            for (int c = 0; c < ATTN_MAX_HEAD_DIM / KVA_WAVE; ++c) acc[c][h] *= more;
+        }
+        T *orow = out + (size_t)t * num_q_heads * value_dim + (size_t)(qh + h) * value_dim;
+#pragma unroll
+        for (int c = 0; c < ATTN_MAX_HEAD_DIM / KVA_WAVE; ++c) {
+            const int j = lane + c * KVA_WAVE;
+            if (j < value_dim) orow[j] = from_float<T>(acc[c][h] / l[h]);
+        }
     }
 }
 
@@ -153,18 +220,34 @@ extern "C" int kva_attention_rowwise(void *out, const void *q, int q_row_stride,
                 value_dim, ATTN_MAX_HEAD_DIM);
     if (window == 0) keep_first = 0;
     if (tokens == 0) return KVA_OK;
-    dim3 grid(tokens, num_q_heads), block(KVA_WAVE);
-    if (dtype == KVA_F32)
-        hipLaunchKernelGGL(attention_rowwise_kernel<float>, grid, block, 0, stream, (float *)out,
-                           (const float *)q, q_row_stride, (const float *)k_cache,
-                           (const float *)v_cache, block_table, max_blocks, tok_seat, tok_pos,
-                           num_q_heads, num_kv_heads, head_dim, value_dim, page_size, scale, window, keep_first, chunk, sinks);
-    else if (dtype == KVA_BF16)
-        hipLaunchKernelGGL(attention_rowwise_kernel<bf16_t>, grid, block, 0, stream, (bf16_t *)out,
-                           (const bf16_t *)q, q_row_stride, (const bf16_t *)k_cache,
-                           (const bf16_t *)v_cache, block_table, max_blocks, tok_seat, tok_pos,
-                           num_q_heads, num_kv_heads, head_dim, value_dim, page_size, scale, window, keep_first, chunk, sinks);
+    const size_t element = dtype == KVA_F32 ? 4 : 2;
+    const int fours = page_size % 4 == 0 && (uintptr_t)v_cache % (4 * element) == 0;
+    const int group = num_q_heads / num_kv_heads;
+    // Heads together: wavefronts are few at first and then the heads' own chains of additions bound them (1 / 2 / 4 heads
+    // of 64, fp32, us: 1 token at 200 keys 11 / 14 / 18, 32 at 500 25 / 27 / 35, 64 at 1,000 63 / 61 / 77), from some
+    // 3,000 rows of a head on the reads do: 128 tokens of 32 heads 16 / 12 / 13, 201 26 / 21 / 22, 603 63 / 40 / 35;
+    // three: 603 tokens of 24 heads of 128 over 8 key heads 93 -> 48.
+    const long long rows = (long long)tokens * num_q_heads;
+    const int together = rows >= 12288 && group % 4 == 0 ? 4
+                         : rows >= 6144 && group % 3 == 0 ? 3
+                         : rows >= 3072 && group % 2 == 0 ? 2 : 1;
+#define KVA_ROWWISE(T, H)                                                                                              \
+    hipLaunchKernelGGL((attention_rowwise_kernel<T, H>), dim3(tokens, num_q_heads / H), dim3(KVA_WAVE), 0, stream, (T *)out, \
+                       (const T *)q, q_row_stride, (const T *)k_cache, (const T *)v_cache, block_table, max_blocks,    \
+                       tok_seat, tok_pos, num_q_heads, num_kv_heads, head_dim, value_dim, page_size, fours, scale,     \
+                       window, keep_first, chunk, sinks)
+#define KVA_ROWWISE_HEADS(T)                                                                                           \
+    do {                                                                                                               \
+        if (together == 4) KVA_ROWWISE(T, 4);                                                                          \
+        else if (together == 3) KVA_ROWWISE(T, 3);                                                                     \
+        else if (together == 2) KVA_ROWWISE(T, 2);                                                                     \
+        else KVA_ROWWISE(T, 1);                                                                                        \
+    } while (0)
+    if (dtype == KVA_F32) KVA_ROWWISE_HEADS(float);
+    else if (dtype == KVA_BF16) KVA_ROWWISE_HEADS(bf16_t);
     else KVA_REQUIRE(false, "attention: unsupported dtype %d", dtype);
+#undef KVA_ROWWISE_HEADS
+#undef KVA_ROWWISE
     KVA_CHECK_LAUNCH("attention_rowwise");
     return KVA_OK;
 }

@@ -314,6 +314,26 @@ def test_attention_rowwise(dtype, nq, nkv, d, page, window, gpu):
     close(out, want, DT[dtype], "attention_rowwise", tol32=3e-6, tol16=8e-3)
 
 
+@pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
+@pytest.mark.parametrize("page", [16, 6])               # (pages of 6: keys of a page are not read by fours)
+@pytest.mark.parametrize("nq, nkv, d", [(32, 4, 32), (36, 12, 16), (20, 10, 20), (28, 4, 64)])
+def test_attention_rowwise_is_the_same_bits_however_many_heads_go_together(dtype, page, nq, nkv, d, gpu):
+    """The launches lie on every side of the rule's lines (3,072 / 6,144 / 12,288 rows of a head)."""
+    dev, want, T, stride, scale, _ = attention_case(dtype, nq, nkv, d, page, 0, ENTRIES, 7, gpu)
+    outs = []
+    for rows in (0, 3072, 6144, 12288):
+        times = max(1, -(-rows // (T * nq)))
+        out = torch.full((T * times, nq * d), float("nan"), dtype=DT[dtype], device=gpu)
+        q, seat, pos = dev["qkv"].repeat(times, 1), dev["tok_seat"].repeat(times), dev["tok_pos"].repeat(times)
+        for a in range(0, T * times, T * times if rows else 16):
+            some = slice(a, a + (T * times if rows else 16))
+            K.attention_rowwise(q[some], stride, out[some], dev["kc"], dev["vc"], dev["table"], seat[some], pos[some], nq, nkv, d,
+                                scale, 0)
+        outs += [o.cpu() for o in out.split(T)]
+    close(outs[0], want, DT[dtype], "attention_rowwise", tol32=3e-6, tol16=8e-3)
+    assert all(torch.equal(o, outs[0]) for o in outs[1:])
+
+
 def items_for(lens, group, gpu, row_tiles=1):
     ent, row0 = [], []
     for e, n in enumerate(lens):
