@@ -53,10 +53,12 @@ EXPAND_BYTES = 512 << 20
 
 
 def expands(batch, heads: int, dim: int, rot: int, vdim: int, rank: int, window: int, dtype) -> bool:
-    """Whether a step's prompt portions attend over expanded keys and values."""
+    """Whether a step's prompt portions attend over expanded keys and values.  A captured step knows its contexts to the power
+    of two above them (at least 256): every step goes by that, so that it asks for the same work items with and without."""
+    context = 1 << max(8, (batch.max_context - 1).bit_length())
     return (dtype == torch.bfloat16 and window <= 0 and heads <= 1024 and batch.min_q_len >= EXPAND_FROM
-            and batch.max_context <= EXPAND_CONTEXTS * batch.min_q_len
-            and batch.num_entries * batch.max_context * (heads * (dim + vdim) + rot) * 2 <= EXPAND_BYTES
+            and context <= EXPAND_CONTEXTS * batch.min_q_len
+            and batch.num_entries * context * (heads * (dim + vdim) + rot) * 2 <= EXPAND_BYTES
             and K.latent_prompt_supported(dim, rot, vdim, rank))
 
 

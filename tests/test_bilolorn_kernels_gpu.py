@@ -9,6 +9,7 @@ import pytest
 import torch
 
 import plain_bilolorn as plain
+from kv_cache_optimization_for_llm_amd.engine.graphs import context_bucket
 from kv_cache_optimization_for_llm_amd.ops import kernels as K
 from kv_cache_optimization_for_llm_amd.ops import latent_attention as lat_ops
 from kv_cache_optimization_for_llm_amd.parts.base import MixerContext, PendingNorm
@@ -527,3 +528,6 @@ def test_which_steps_expand_keys_and_values(gpu):
     assert not rule(step(63, 63)) and not rule(step(64, 1025)) and not rule(step(64, 64), heads=1025)
     assert not rule(step(2048, 2048, 64)) and not rule(step(64, 64), window=32) and not rule(step(64, 64), dtype=torch.float32)
     assert not rule(step(64, 64), rot=32) and not rule(step(64, 64), rank=48)
+    # a captured step's contexts are rounded up: what it was captured for and every step it stands for take the same path
+    for shortest, context in ((100, 1500), (100, 1601), (64, 1), (256, 4096), (300, 4097), (1024, 8191), (4096, 40000)):
+        assert rule(step(shortest, context)) == rule(step(shortest, context_bucket(context)))
