@@ -433,6 +433,8 @@ attention_item(bf16_t *__restrict__ out, float *__restrict__ part_o, float *__re
             const int n0 = item_hi + 1 - (kstart + 4 * g);
             keep[0] = keep_first_keys(make_uint2(~0u, ~0u), n0);
             keep[1] = keep_first_keys(make_uint2(~0u, ~0u), n0 - 16);
+            // (a first tile in front of the item's keys was redirected to their first page, which may be their last)
+            if (FAST && kstart < lo_tile) keep[0] = make_uint2(0u, 0u);
         }
 #pragma unroll
         for (int rt = 0; rt < RT; ++rt)

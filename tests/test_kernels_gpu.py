@@ -343,6 +343,28 @@ def items_for(lens, group, gpu, row_tiles=1):
     return (torch.tensor(ent, dtype=torch.int32, device=gpu), torch.tensor(row0, dtype=torch.int32, device=gpu))
 
 
+def chunked_oracle(chunk, entries, *case):
+    """Chunks of so many positions: the window oracle row by row."""
+    whole = [attention_case("bfloat16", *case, w, entries, 11, "cpu")[1] for w in range(1, chunk + 1)]
+    pos = np.concatenate([np.arange(s, s + n) for s, n in entries])
+    return torch.stack([whole[p % chunk][t] for t, p in enumerate(pos)])
+
+
+@pytest.mark.parametrize("tiles", [1, 2])
+@pytest.mark.parametrize("window", [9, -40])
+def test_keys_that_begin_in_the_second_tile_of_a_block(window, tiles, gpu):
+    """The tile in front of them is read from their first page: stale places behind the last key there stay out."""
+    entries = [(17, 270), (255, 33), (1000, 17), (276, 5), (283, 1)]
+    dev, want, T, stride, scale, lens = attention_case("bfloat16", 8, 2, 64, 16, max(window, 0), entries, 11, gpu, stale=float("nan"))
+    if window < 0:
+        want = chunked_oracle(-window, entries, 8, 2, 64, 16)
+    ent, row0 = items_for(lens, 4, gpu, tiles)
+    out = torch.full((T, 8 * 64), float("nan"), dtype=torch.bfloat16, device=gpu)
+    K.attention_mfma(dev["qkv"], stride, out, dev["kc"], dev["vc"], dev["table"], ent, row0, dev["entry_seat"], dev["q_start"],
+                     dev["start_pos"], 8, 2, 64, scale, window, 1, 0, tiles)
+    close(out, want, torch.bfloat16, f"attention_mfma tiles={tiles}", tol16=8e-3)
+
+
 @pytest.mark.parametrize("nq, nkv, d, page, window", [
     (4, 2, 16, 16, 0), (6, 2, 48, 8, 0), (3, 3, 32, 4, 0), (8, 2, 64, 16, 45), (32, 8, 64, 16, 0),
     (5, 1, 80, 16, 0), (24, 8, 128, 16, 0), (4, 4, 96, 32, 33), (2, 1, 256, 16, 0), (14, 2, 112, 16, 0)])
