@@ -144,7 +144,9 @@ attention_item(bf16_t *__restrict__ out, float *__restrict__ part_o, float *__re
     int k_begin = item_lo & ~31;
     int k_end = item_hi + 1;                                            // exclusive
     if (splits > 1) {
-        const int s_lo = split * keys_per_split, s_hi = s_lo + keys_per_split;
+        // ranges at fixed positions, or (keys_per_split = 0) equal shares of what this item sees
+        const int per = keys_per_split > 0 ? keys_per_split : ((k_end - k_begin + splits - 1) / splits + 31) & ~31;
+        const int s_lo = (keys_per_split > 0 ? 0 : k_begin) + split * per, s_hi = s_lo + per;
         if (s_lo > k_begin) k_begin = s_lo;
         if (s_hi < k_end) k_end = s_hi;
     }
@@ -604,8 +606,10 @@ attention_item(bf16_t *__restrict__ out, float *__restrict__ part_o, float *__re
 // same heads' keys and values.  With `pair`, a wavefront takes item w and then item n-1-w of the
 // list: the caller orders the list by the number of keys an item visits (most first), so every
 // wavefront gets about the same work - rows late in a prompt visit many keys, early rows few.
+// Two row tiles of heads up to 64: 168 registers instead of 172, so that three wavefronts fit a SIMD (4 to a workgroup
+// on an item, 2,048 tokens of 32 heads of 64: 45 -> 39 us); with heads of 128 (289) a second one would cost scratch memory.
 template <int D, int RT, bool FAST, bool STREAM>
-__global__ void __launch_bounds__(KVA_WAVE * KVA_ATTN_MAX_WAVES)
+__global__ void __launch_bounds__(KVA_WAVE * KVA_ATTN_MAX_WAVES, RT == 2 && FAST && D <= 64 ? 3 : 1)
 attention_mfma_kernel(bf16_t *__restrict__ out, float *__restrict__ part_o, float *__restrict__ part_ml,
                       const bf16_t *__restrict__ q, int q_row_stride,
                       const bf16_t *__restrict__ k_cache, const bf16_t *__restrict__ v_cache,
@@ -763,17 +767,17 @@ extern "C" int kva_attention_mfma_row_tiles(int head_dim, int wide) {
 }
 
 // Wavefronts of one workgroup that share an item (each a key range of its own, added up in LDS):
-// 1, 2 or 4; more than one for items of one row tile, not in pairs, head sizes up to 128, and a
-// number of key ranges they divide.
+// 1, 2 or 4; more than one not in pairs, for head sizes up to 128, and with a
+// number of key ranges they divide (items of two row tiles: exactly theirs).
 static bool kva_attention_mfma_waves_ok(int waves, int splits, int head_dim, int row_tiles, int pair) {
     if (waves == 1) return true;
-    return (waves == 2 || waves == KVA_ATTN_MAX_WAVES) && row_tiles == 1 && !pair && head_dim <= 128 &&
-           splits >= waves && splits % waves == 0;
+    return (waves == 2 || waves == KVA_ATTN_MAX_WAVES) && !pair && head_dim <= 128 &&
+           (row_tiles == 1 ? splits >= waves && splits % waves == 0 : splits == waves);
 }
 
-// LDS in which all but the first of them leave their (o, m, l): head_dim + 2 floats per lane each.
-static size_t kva_attention_mfma_exchange_bytes(int waves, int head_dim) {
-    return waves > 1 ? (size_t)(waves - 1) * (head_dim / 16 * 4 + 2) * KVA_WAVE * sizeof(float) : 0;
+// LDS in which all but the first of them leave their (o, m, l): per row tile head_dim / 4 + 2 floats per lane each.
+static size_t kva_attention_mfma_exchange_bytes(int waves, int head_dim, int row_tiles) {
+    return waves > 1 ? (size_t)(waves - 1) * row_tiles * (head_dim / 16 * 4 + 2) * KVA_WAVE * sizeof(float) : 0;
 }
 
 // `out` null (more than one partial result a row left, splits / waves > 1): no merge launch; the
@@ -790,8 +794,8 @@ extern "C" int kva_attention_mfma(void *out, float *part_o, float *part_ml, cons
     KVA_REQUIRE(num_items >= 0 && num_q_heads > 0 && num_kv_heads > 0 && max_blocks > 0,
                 "attention_mfma: bad sizes");
     KVA_REQUIRE(kva_attention_mfma_waves_ok(waves, splits, head_dim, row_tiles, pair),
-                "attention_mfma: %d wavefronts per item need one row tile, no pairs, a head size up to 128 and a "
-                "number of key ranges (%d) they divide", waves, splits);
+                "attention_mfma: %d wavefronts per item need no pairs, a head size up to 128 and a "
+                "number of key ranges (%d) they divide (two row tiles: theirs alone)", waves, splits);
     KVA_REQUIRE(num_q_heads % num_kv_heads == 0, "attention_mfma: %d query heads is not a multiple of %d kv heads",
                 num_q_heads, num_kv_heads);
     KVA_REQUIRE(kva_attention_mfma_supported(head_dim, page_size),
@@ -800,7 +804,7 @@ extern "C" int kva_attention_mfma(void *out, float *part_o, float *part_ml, cons
     KVA_REQUIRE(q_row_stride % 8 == 0, "attention_mfma: query row stride %d must be a multiple of 8", q_row_stride);
     KVA_REQUIRE(splits >= 1 && splits <= MERGE_MAX_SPLITS && num_kv_heads <= 65535,
                 "attention_mfma: at most %d splits and 65535 kv heads", MERGE_MAX_SPLITS);
-    KVA_REQUIRE(splits == 1 || (keys_per_split > 0 && keys_per_split % 32 == 0),
+    KVA_REQUIRE(splits == 1 || (keys_per_split > 0 && keys_per_split % 32 == 0) || (keys_per_split == 0 && splits == waves),
                 "attention_mfma: splits need a key count that is a multiple of 32");
     KVA_REQUIRE(splits == waves || (part_o && part_ml), "attention_mfma: key ranges of several workgroups need a workspace");
     // without `out` the partial results (splits / waves a row) are left to the caller: no merge launch
@@ -813,7 +817,7 @@ extern "C" int kva_attention_mfma(void *out, float *part_o, float *part_ml, cons
     KVA_REQUIRE((long)num_items * num_kv_heads < (1L << 31), "attention_mfma: too many work items");
     const int waves_x = pair ? (num_items + 1) / 2 : num_items;
     dim3 grid(waves_x * num_kv_heads, 1, splits / waves), block(KVA_WAVE * waves);
-    const size_t lds = kva_attention_mfma_exchange_bytes(waves, head_dim);
+    const size_t lds = kva_attention_mfma_exchange_bytes(waves, head_dim, row_tiles);
     const bool fast = page_size == 16;
 #define LAUNCH(DD, RR, FF, SS)                                                                  \
     hipLaunchKernelGGL((attention_mfma_kernel<DD, RR, FF, SS>), grid, block, lds, stream, (bf16_t *)out, \
@@ -885,7 +889,7 @@ extern "C" int kva_attention_mfma_rope(void *out, float *part_o, float *part_ml,
     if (num_items == 0) return KVA_OK;
     KVA_REQUIRE((long)num_items * num_kv_heads < (1L << 31), "attention_mfma_rope: too many work items");
     dim3 grid(num_items * num_kv_heads, 1, splits / waves), block(KVA_WAVE * waves);
-    const size_t lds = kva_attention_mfma_exchange_bytes(waves, head_dim);
+    const size_t lds = kva_attention_mfma_exchange_bytes(waves, head_dim, 1);
     const RopeArgs rope{cos_t, sin_t, slots};
 #define LAUNCH(DD, SS)                                                                               \
     hipLaunchKernelGGL((attention_mfma_rope_kernel<DD, SS>), grid, block, lds, stream, (bf16_t *)out, part_o, \

@@ -220,8 +220,8 @@ class _PortionSlot:
 class PortionGraphs:
     """Graphs for steps that hold prompt portions (alone or beside decoded tokens).
 
-    A shape is (tokens per entry, wanted places, context bucket, whether the portions' rows visit
-    enough keys for the workgroup attention kernel): everything the forward pass decides on the
+    A shape is (tokens per entry, wanted places, context bucket, the power of two below the mean number of
+    keys the portions' rows visit, by which the attention kernel is chosen): everything the forward pass decides on the
     host.  Its first step runs eagerly and tells which sets of attention work items the pass asks
     for; the step at which it has come ``CAPTURE_AT`` times is captured over static buffers; later
     ones upload their indices and replay.  Logits come back in the shape's static buffer: they hold
@@ -248,7 +248,7 @@ class PortionGraphs:
 
     @staticmethod
     def shape_key(lens: Sequence[int], starts: Sequence[int], rows: Sequence[int]) -> Optional[tuple]:
-        from ..ops.attention import LDS_MEAN_KEYS_STEPS
+        from ..ops.attention import MEAN_KEYS_STEPS
         T = int(sum(lens))
         if T > PortionGraphs.MAX_TOKENS or len(rows) > PortionGraphs.MAX_LOGIT_ROWS:
             return None
@@ -257,7 +257,7 @@ class PortionGraphs:
         mean_keys = float(((st[long] + (ln[long] + 1) / 2) * ln[long]).sum() / ln[long].sum())
         bucket = context_bucket(int(max(s + n for s, n in zip(starts, lens))))
         return (tuple(int(n) for n in lens), tuple(int(r) for r in rows), bucket,
-                tuple(mean_keys >= t for t in LDS_MEAN_KEYS_STEPS))
+                tuple(mean_keys >= t for t in MEAN_KEYS_STEPS))
 
     def note(self, key: tuple, batch: StepBatch) -> None:
         """After the eager run of a shape: the sets of attention items its forward pass used."""

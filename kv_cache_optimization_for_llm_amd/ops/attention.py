@@ -6,6 +6,7 @@ contexts over several wavefronts when the batch alone would leave most of the GP
 """
 from __future__ import annotations
 
+import numpy as np
 import torch
 
 from . import kernels as K
@@ -63,7 +64,9 @@ _LDS_MIN_GROUPS_WIDE_HEADS = 16
 _LDS_TARGET_GROUPS_WIDE_HEADS = 512
 _LDS_MIN_KEYS_PER_SPLIT_WIDE_HEADS = 256
 # where the choice can change (a step shape that has a graph is told apart by these too)
-LDS_MEAN_KEYS_STEPS = tuple(sorted({_LDS_MIN_MEAN_KEYS_WIDE_HEADS, _LDS_SOME_GROUPS_MEAN_KEYS, _LDS_MIN_MEAN_KEYS}))
+# (choose_portion_waves knows the mean to the power of two below it; the lines above are among them)
+MEAN_KEYS_STEPS = tuple(1 << k for k in range(6, 20))
+assert {_LDS_MIN_MEAN_KEYS_WIDE_HEADS, _LDS_SOME_GROUPS_MEAN_KEYS, _LDS_MIN_MEAN_KEYS} <= set(MEAN_KEYS_STEPS)
 # few workgroups that each walk thousands of keys: the keys are cut into ranges, one workgroup each
 _LDS_TARGET_GROUPS = 1024
 _LDS_MIN_KEYS_PER_SPLIT = 1024
@@ -72,6 +75,39 @@ _LDS_MIN_KEYS_PER_SPLIT = 1024
 # chunked masks go to the tuned kernels where those take the head size (False: to the general rows kernel)
 CHUNKS_IN_TUNED_KERNELS = True
 _ROWS_TWO_TILES = 32 * 1024          # (token, head) rows of a step from which the general rows kernel takes two tiles an item
+
+
+def choose_portion_waves(waves: int, mean_keys: float, head_dim: int) -> int:
+    """Wavefronts of a workgroup (1: none of this, 2 or 4) that share an item of two row tiles of prompt portions, each an
+    equal share of what the item sees, for ``waves`` (item, kv head) pairs whose rows visit ``mean_keys`` keys on average.
+
+    One wavefront on two row tiles is a chain of products, softmax and products, 0.9 us a block of 32 keys with its SIMD to
+    itself, and fixed key ranges with a merge kernel cost that kernel and leave early rows' ranges empty.  us a call without
+    -> with, 32 heads of 64 over 8: one prompt of 256 / 512 / 1,024 / 1,536 / 2,048 / 2,304 / 2,560 tokens 14 / 26 / 22 / 34 / 44 /
+    51 / 56 -> 7 / 10 / 17 / 26 / 39 / 45 / 52 (3,072 the same, 4,096 94 -> 112 and from there the workgroup kernel); three of
+    509 20 -> 15; 256 tokens behind 1,024 / 4,096 / 8,000 24 / 35 / 49 -> 12 / 26 / 42, 512 behind 2,000 / 4,096 / 7,000 41 / 52 /
+    70 -> 23 / 36 / 53, 1,024 behind 2,000 / 6,000 65 / 107 -> 41 / 92, 2,048 behind 2,000 / 6,000 112 / 201 -> 89 / 188.  Not so: 64
+    behind 4,096 21 -> 24, 128 behind 8,000 32 -> 41, 512 behind 30,000 194 -> 199, eight of 200 10.4 -> 12.2 (a tie at four of 512).
+    Heads of 32 and 96 alike.  Heads of 128 hold a SIMD's registers with one wavefront, so what there is to win ends
+    earlier: 32 heads, 256 / 512 / 768 tokens 26 / 35 / 40 -> 10 / 14 / 19, 256 behind 1,024 / 4,096 34 / 41 -> 17 / 36, 512 behind 2,000
+    49 -> 36; 24 heads, 1,024 tokens 42 -> 22, four of 256 behind 1,000 57 -> 38; but four of 256 (32 heads) 13 -> 16, behind 1,000
+    38 -> 43, eight of 100 9.6 -> 11.9, 512 behind 7,000 90 -> 104."""
+    if head_dim > 128:
+        return 1
+    keys = max((step for step in MEAN_KEYS_STEPS if step <= mean_keys), default=0)
+    if head_dim > 96:
+        if waves <= 256 and keys >= 512:
+            return 4 if keys <= 12 * waves else 1
+        if waves <= 256:
+            return 2 if waves >= 128 else 1
+        return 2 if waves < 1024 and waves <= 12 * keys and keys <= 4 * waves else 1
+    if waves <= 512:
+        if keys >= 512:
+            return 4 if keys <= 16 * waves else 1
+        return 2 if waves >= 128 else 1
+    if waves > 2560 or (waves > 1024 and waves > 12 * keys):
+        return 1
+    return 4 if waves * keys >= 3 << 20 else 2
 
 
 def use_lds_kernel(groups: int, mean_keys: float, head_dim: int) -> bool:
@@ -476,6 +512,17 @@ def _plan(batch, group: int, num_kv_heads: int, head_dim: int, page_size: int, m
         return plan
     mixed = batch.min_q_len * group <= 16
     which = "long" if mixed else "all"
+    # two row tiles per wave, so each key and value loaded serves 32 query rows
+    tiles = K.attention_mfma_row_tiles(head_dim, True)
+    rows = np.diff(batch.h_entry_q_start).astype(np.int64) * group
+    count = int((-(-(rows[rows > 16] if mixed else rows) // (16 * tiles))).sum()) * num_kv_heads
+    sharing = choose_portion_waves(count, batch.mean_keys_of_long_entries(), head_dim)
+    if tiles == 2 and sharing > 1:
+        items = batch.attention_items(group, tiles, which)
+        plan.append(("wave", items, tiles, sharing, 0, False, which == "all", False, sharing))
+        if mixed:
+            decoded("short")
+        return plan
     done = False
     if K.attention_lds_supported(head_dim, page_size):
         items = batch.attention_items(group, 8, which)
@@ -485,9 +532,7 @@ def _plan(batch, group: int, num_kv_heads: int, head_dim: int, page_size: int, m
             plan.append(("lds", items[2], splits, per, which == "all"))
             done = True
     if not done:
-        # two row tiles per wave, so each key and value loaded serves 32 query rows; whole key
-        # ranges as long as that gives a wave per SIMD
-        tiles = K.attention_mfma_row_tiles(head_dim, True)
+        # whole key ranges as long as that gives a wave per SIMD
         items = batch.attention_items(group, tiles, which)
         waves = items[0].shape[0] * num_kv_heads
         if waves >= _WIDE_MIN_WAVES:

@@ -1174,9 +1174,11 @@ def attention_mfma(q: torch.Tensor, q_row_stride: int, out: torch.Tensor, k_cach
     another launch) and a split merge must leave those alone.  ``keep_cached`` (items of one row
     tile): keys and values are loaded through the caches instead of past them - for the few
     short contexts that are still in the memory-side cache when the next step reads them.
-    ``waves`` (1, 2 or 4; items of one row tile, head sizes up to 128): so many of the ``splits``
+    ``waves`` (1, 2 or 4; head sizes up to 128, no pairs): so many of the ``splits``
     key ranges go to the wavefronts of one workgroup, which adds their results up itself; only
-    ``splits // waves`` partial results per row are left for the merge (none: no merge launch).
+    ``splits // waves`` partial results per row are left for the merge (none: no merge launch; items of
+    two row tiles take no more than that).  ``keys_per_split`` 0 with ``splits == waves``: equal shares of
+    what each item sees.
     ``leave_partials`` (the items cover every row of the step): where more than one partial result
     a row is left they are not merged into ``out`` but returned as :class:`AttentionPartials`."""
     tokens = out.shape[0]

@@ -365,6 +365,26 @@ def test_keys_that_begin_in_the_second_tile_of_a_block(window, tiles, gpu):
     close(out, want, torch.bfloat16, f"attention_mfma tiles={tiles}", tol16=8e-3)
 
 
+@pytest.mark.parametrize("waves", [2, 4])
+@pytest.mark.parametrize("nq, nkv, d, page, window", [
+    (4, 2, 16, 16, 0), (3, 3, 32, 4, 0), (8, 2, 64, 16, 45), (32, 8, 64, 16, 0), (32, 8, 64, 16, -40), (5, 1, 80, 8, 0),
+    (24, 8, 128, 16, 0), (24, 8, 128, 16, 33), (6, 2, 96, 32, 0), (14, 2, 112, 16, 0)])
+def test_prompt_items_in_equal_shares(nq, nkv, d, page, window, waves, gpu):
+    """Entries from one key (three shares without a key) to several blocks a share; stale places hold NaN and infinities."""
+    entries = [(0, 1), (0, 37), (63, 1), (100, 29), (255, 33), (17, 270), (1000, 17)]
+    dev, want, T, stride, scale, lens = attention_case("bfloat16", nq, nkv, d, page, max(window, 0), entries, 11, gpu, stale=float("nan"))
+    if window < 0:
+        want = chunked_oracle(-window, entries, nq, nkv, d, page)
+    ent, row0 = items_for(lens, nq // nkv, gpu, 2)
+    out = torch.full((T, nq * d), float("nan"), dtype=torch.bfloat16, device=gpu)
+    K.attention_mfma(dev["qkv"], stride, out, dev["kc"], dev["vc"], dev["table"], ent, row0, dev["entry_seat"], dev["q_start"],
+                     dev["start_pos"], nq, nkv, d, scale, window, waves, 0, 2, False, waves=waves)
+    close(out, want, torch.bfloat16, f"attention_mfma waves={waves}", tol16=8e-3)
+    with pytest.raises(K.KernelError):          # (equal shares are for the wavefronts of one workgroup)
+        K.attention_mfma(dev["qkv"], stride, out, dev["kc"], dev["vc"], dev["table"], ent, row0, dev["entry_seat"], dev["q_start"],
+                         dev["start_pos"], nq, nkv, d, scale, window, 2 * waves, 0, 2, False, waves=waves)
+
+
 @pytest.mark.parametrize("nq, nkv, d, page, window", [
     (4, 2, 16, 16, 0), (6, 2, 48, 8, 0), (3, 3, 32, 4, 0), (8, 2, 64, 16, 45), (32, 8, 64, 16, 0),
     (5, 1, 80, 16, 0), (24, 8, 128, 16, 0), (4, 4, 96, 32, 33), (2, 1, 256, 16, 0), (14, 2, 112, 16, 0)])
