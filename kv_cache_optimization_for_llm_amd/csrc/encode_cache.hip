@@ -115,15 +115,33 @@ qk_encode_cache_kernel(T *__restrict__ qkv, int row_stride, int k_off, int v_off
     }
 }
 
-// bf16, interleaved pairs, heads of 8 * 2^k elements (up to 512): a lane takes 8 neighbouring
-// elements of a head (four whole pairs: 16 bytes in, 16 bytes out - one chunk of the K page), the
-// 2^k lanes of a head add their squares up between them.
+// bf16, heads of 8 * 2^k elements (up to 512), pairs of neighbours or of elements rot / 2 apart with rot / 2 a multiple of 8:
+// a lane takes 8 neighbouring elements of a head (16 bytes in, 16 bytes out - one chunk of the K page), the 2^k lanes of a
+// head add their squares up between them, and a lane whose elements pair with another lane's gets those from its registers.
+// (One element at a time, a wavefront a head after the other, 2,048 tokens of 32 + 8 heads of 64 with a bias and half of
+// a head rotated took 73 us; so it takes 29, most of it the values' 2-byte stores into the transposed pages.)
+__device__ inline void enc_unpack8(const uint4 in, float (&x)[8]) {
+    const uint32_t w[4] = {in.x, in.y, in.z, in.w};
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        x[2 * i] = bf16_bits_to_float((uint16_t)(w[i] & 0xffffu));
+        x[2 * i + 1] = bf16_bits_to_float((uint16_t)(w[i] >> 16));
+    }
+}
+
+__device__ inline void enc_load8(const float *p, float (&x)[8]) {
+    const float4 a = *reinterpret_cast<const float4 *>(p), b = *reinterpret_cast<const float4 *>(p + 4);
+    x[0] = a.x; x[1] = a.y; x[2] = a.z; x[3] = a.w; x[4] = b.x; x[5] = b.y; x[6] = b.z; x[7] = b.w;
+}
+
 __global__ void __launch_bounds__(256)
 qk_encode_cache_vec_kernel(bf16_t *__restrict__ qkv, int row_stride, int k_off, int v_off, bf16_t *__restrict__ k_cache,
                            bf16_t *__restrict__ v_cache, const float *__restrict__ cos_table,
                            const float *__restrict__ sin_table, const int *__restrict__ positions,
                            const int *__restrict__ slot_mapping, int num_q_heads, int num_kv_heads, int head_dim,
-                           int value_dim, int rot, float unit_eps, int page_size) {
+                           int value_dim, int rot, int interleaved, float unit_eps, int page_size,
+                           const bf16_t *__restrict__ bias, const float *__restrict__ q_weight,
+                           const float *__restrict__ k_weight, int norm_first) {
     const int t = blockIdx.x;
     bf16_t *row = qkv + (size_t)t * row_stride;
     const int pos = positions[t];
@@ -138,34 +156,55 @@ qk_encode_cache_vec_kernel(bf16_t *__restrict__ qkv, int row_stride, int k_off, 
         const int head = on ? w / vecs : 0, j = on ? w % vecs : 0;
         const bool is_q = head < num_q_heads;
         bf16_t *h = is_q ? row + (size_t)head * head_dim : row + k_off + (size_t)(head - num_q_heads) * head_dim;
-        float x[8], y[8];
-        const uint4 in = *reinterpret_cast<const uint4 *>(h + 8 * j);
-        const uint32_t iw[4] = {in.x, in.y, in.z, in.w};
-        float sq = 0.f;
+        const float *weight = is_q ? q_weight : k_weight;         // (optional) of an RMS norm over the head
+        float x[8], y[8], wt[8];
+        enc_unpack8(*reinterpret_cast<const uint4 *>(h + 8 * j), x);
+        if (bias) {                                               // (optional) laid out [q heads | k heads | v heads]
+            enc_unpack8(*reinterpret_cast<const uint4 *>(bias + (size_t)head * head_dim + 8 * j), y);
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            x[2 * i] = bf16_bits_to_float((uint16_t)(iw[i] & 0xffffu));
-            x[2 * i + 1] = bf16_bits_to_float((uint16_t)(iw[i] >> 16));
-            const int p = 4 * j + i;                              // pair (2p, 2p + 1) of the head
-            if (p < half) {
-                const float co = cs[p], si = sn[p];
-                y[2 * i] = x[2 * i] * co - x[2 * i + 1] * si;
-                y[2 * i + 1] = x[2 * i + 1] * co + x[2 * i] * si;
-            } else {
-                y[2 * i] = x[2 * i];
-                y[2 * i + 1] = x[2 * i + 1];
-            }
-            sq += y[2 * i] * y[2 * i] + y[2 * i + 1] * y[2 * i + 1];
+            for (int i = 0; i < 8; ++i) x[i] += y[i];
         }
-        float mul = 1.f;
-        if (unit_eps >= 0.f) {
+#pragma unroll
+        for (int i = 0; i < 8; ++i) wt[i] = 1.f;
+        if (weight) enc_load8(weight + 8 * j, wt);
+        auto unit = [&](float (&z)[8]) {                          // divides the head by its root mean square
+            float sq = 0.f;
+#pragma unroll
+            for (int i = 0; i < 4; ++i) sq += z[2 * i] * z[2 * i] + z[2 * i + 1] * z[2 * i + 1];
             for (int o = vecs / 2; o > 0; o >>= 1) sq += __shfl_xor(sq, o, KVA_WAVE);
-            mul = 1.0f / sqrtf(sq / (float)head_dim + unit_eps);
+            const float mul = 1.0f / sqrtf(sq / (float)head_dim + unit_eps);
+#pragma unroll
+            for (int i = 0; i < 8; ++i) z[i] = z[i] * mul * wt[i];
+        };
+        if (norm_first) unit(x);                                  // (the normed head is what is rotated)
+        if (interleaved) {
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                const int p = 4 * j + i;                          // pair (2p, 2p + 1) of the head
+                const float co = p < half ? cs[p] : 1.f, si = p < half ? sn[p] : 0.f;
+                y[2 * i] = p < half ? x[2 * i] * co - x[2 * i + 1] * si : x[2 * i];
+                y[2 * i + 1] = p < half ? x[2 * i + 1] * co + x[2 * i] * si : x[2 * i + 1];
+            }
+        } else {
+            const int apart = half / 8;                           // pair p: elements p and p + rot / 2
+            const bool first = 8 * j < half, turns = 8 * j < rot;
+            const int lane = threadIdx.x % KVA_WAVE, from = turns ? (first ? lane + apart : lane - apart) : lane;
+            float co[8], si[8];
+            if (turns) {
+                enc_load8(cs + (first ? 8 * j : 8 * j - half), co);
+                enc_load8(sn + (first ? 8 * j : 8 * j - half), si);
+            }
+#pragma unroll
+            for (int i = 0; i < 8; ++i) {
+                const float other = __shfl(x[i], from, KVA_WAVE);
+                y[i] = !turns ? x[i] : first ? x[i] * co[i] - other * si[i] : x[i] * co[i] + other * si[i];
+            }
         }
+        if (!norm_first && unit_eps >= 0.f) unit(y);
         uint32_t ow[4];
 #pragma unroll
         for (int i = 0; i < 4; ++i)
-            ow[i] = (uint32_t)float_to_bf16_bits(y[2 * i] * mul) | ((uint32_t)float_to_bf16_bits(y[2 * i + 1] * mul) << 16);
+            ow[i] = (uint32_t)float_to_bf16_bits(y[2 * i]) | ((uint32_t)float_to_bf16_bits(y[2 * i + 1]) << 16);
         const uint4 res = make_uint4(ow[0], ow[1], ow[2], ow[3]);
         if (!on) continue;
         if (is_q) {
@@ -177,9 +216,11 @@ qk_encode_cache_vec_kernel(bf16_t *__restrict__ qkv, int row_stride, int k_off, 
     }
     if (slot >= 0) {
         const bf16_t *v = row + v_off;
+        const bf16_t *vb = bias ? bias + (size_t)(num_q_heads + num_kv_heads) * head_dim : nullptr;
         for (int w = threadIdx.x; w < num_kv_heads * value_dim; w += blockDim.x) {
             const int kvh = w / value_dim, j = w % value_dim;
-            v_cache[(((size_t)page * num_kv_heads + kvh) * value_dim + j) * page_size + off] = v[w];
+            v_cache[(((size_t)page * num_kv_heads + kvh) * value_dim + j) * page_size + off] =
+                vb ? from_float<bf16_t>(to_float(v[w]) + to_float(vb[w])) : v[w];
         }
     }
 }
@@ -209,11 +250,14 @@ extern "C" int kva_qk_encode_cache(void *qkv, int row_stride, int k_off, int v_o
     if (tokens == 0) return KVA_OK;
     if (rot == 0) cos_table = sin_table = reinterpret_cast<const float *>(qkv);     // never read
     const int vecs = head_dim / 8;
-    if (!bias && !q_weight && !k_weight && !norm_first && dtype == KVA_BF16 && interleaved && head_dim % 8 == 0 && (vecs & (vecs - 1)) == 0 && vecs <= KVA_WAVE &&
-        row_stride % 8 == 0 && k_off % 8 == 0 && (reinterpret_cast<uintptr_t>(qkv) & 15) == 0) {
+    const uintptr_t wide = (uintptr_t)qkv | (uintptr_t)bias | (uintptr_t)q_weight | (uintptr_t)k_weight |
+                           (interleaved || rot == 0 ? 0 : (uintptr_t)cos_table | (uintptr_t)sin_table);
+    if (dtype == KVA_BF16 && head_dim % 8 == 0 && (vecs & (vecs - 1)) == 0 && vecs <= KVA_WAVE &&
+        (interleaved || rot % 16 == 0) && row_stride % 8 == 0 && k_off % 8 == 0 && (wide & 15) == 0) {
         hipLaunchKernelGGL(qk_encode_cache_vec_kernel, dim3(tokens), dim3(256), 0, stream, (bf16_t *)qkv, row_stride,
                            k_off, v_off, (bf16_t *)k_cache, (bf16_t *)v_cache, cos_table, sin_table, positions,
-                           slot_mapping, num_q_heads, num_kv_heads, head_dim, value_dim, rot, unit_eps, page_size);
+                           slot_mapping, num_q_heads, num_kv_heads, head_dim, value_dim, rot, interleaved, unit_eps,
+                           page_size, (const bf16_t *)bias, q_weight, k_weight, norm_first);
         KVA_CHECK_LAUNCH("qk_encode_cache");
         return KVA_OK;
     }

@@ -337,3 +337,69 @@ def test_windowed_attention_on_the_matrix_cores(heads, kv_heads, dim, vdim, wind
                               dim, scale, window, keep_first, sinks.to(gpu), vdim, ranges, per_range, row_tiles)
         assert torch.isfinite(out.float()).all(), f"entry {start}+{n}"
         close(out.view(n, heads, vdim), want_all[start:upto], 3e-2, f"entry {start}+{n}")
+
+
+@pytest.mark.parametrize("x_dtype, out_dtype", [("float32", "float32"), ("float32", "bfloat16"), ("bfloat16", "bfloat16")])
+@pytest.mark.parametrize("width, offset", [(8, 0), (2048, 0), (2056, 0), (4096, 0), (8192, 0), (8200, 0), (2048, 1)])
+def test_layer_norm_rows_in_registers(width, offset, x_dtype, out_dtype, gpu):
+    """Widths around what a thread holds once, twice and four times, and operands that do not start at 16 bytes."""
+    def put(t):
+        flat = torch.empty(t.numel() + offset, dtype=t.dtype, device=gpu)
+        return flat[offset:].view(t.shape).copy_(t)
+    x, d1 = (rnd((5, width), 1, scale=3.0) + 1.5).to(DT[x_dtype]), rnd((5, width), 2, DT[out_dtype])
+    d2, w1, w2 = rnd((5, width), 3), 1 + 0.1 * rnd((width,), 4), 1 + 0.1 * rnd((width,), 5)
+    for rms in (False, True):
+        for scale in (1.0, 0.7):
+            xs, o1, o2 = put(x), put(torch.zeros((5, width), dtype=DT[out_dtype])), put(torch.zeros((5, width), dtype=DT[out_dtype]))
+            K.layernorm(xs, put(w1), 1e-5, o1, deltas=(put(d1), put(d2)), weight2=put(w2), out2=o2, rms=rms, delta_scale=scale)
+            total = x.double() + scale * (d1.double() + d2.double())
+            close(xs, total, 1e-6 if x_dtype == "float32" else 5e-3, "the stream after the add")
+            held = xs.double().cpu()
+            centred = held if rms else held - held.mean(-1, keepdim=True)
+            n = centred / torch.sqrt((centred ** 2).mean(-1, keepdim=True) + 1e-5)
+            close(o1, n * w1.double(), TOL[out_dtype], "first copy")
+            close(o2, n * w2.double(), TOL[out_dtype], "second copy")
+
+
+@pytest.mark.parametrize("dim, rot", [(8, 0), (8, 8), (16, 16), (32, 16), (64, 32), (64, 64), (128, 96), (512, 512)])
+@pytest.mark.parametrize("interleaved", [True, False])
+@pytest.mark.parametrize("norm", [None, "unit", "weights", "weights first"])
+@pytest.mark.parametrize("with_bias, offset", [(False, 0), (True, 0), (True, 1)])
+def test_heads_of_a_power_of_two_in_registers(dim, rot, interleaved, norm, with_bias, offset, gpu):
+    """Every form together with and without the others; a bias at an odd address takes the general kernel."""
+    heads, kv_heads, vdim, T, page, eps = 5, 3, 24, 11, 8, 1e-2
+    width = (heads + kv_heads) * dim + kv_heads * vdim
+    qkv, bias = rnd((T, width), 7, torch.bfloat16), rnd((width,), 8, torch.bfloat16)
+    wq, wk = 1 + 0.2 * rnd((dim,), 9), 1 + 0.2 * rnd((dim,), 10)
+    table, slots, pages = cache_for(T, page, 3)
+    slots[4] = -1
+    angle = rnd((T, max(1, rot // 2)), 11, scale=2.0)
+    cos, sin = (torch.cos(angle), torch.sin(angle)) if rot else (None, None)
+    k_cache = torch.zeros((pages, *K.k_page_shape(kv_heads, dim)[:2], page, K.k_chunk(dim)), dtype=torch.bfloat16, device=gpu)
+    v_cache = torch.zeros((pages, kv_heads, vdim, page), dtype=torch.bfloat16, device=gpu)
+    buf = torch.zeros(width + offset, dtype=torch.bfloat16, device=gpu)
+    buf[offset:] = bias.to(gpu)
+    got, weighted = qkv.to(gpu), norm is not None and "weights" in norm
+    K.qk_encode_cache(got, torch.arange(T, dtype=torch.int32, device=gpu), heads, kv_heads, dim, vdim, None if cos is None else cos.to(gpu),
+                      None if sin is None else sin.to(gpu), interleaved, None if norm is None else eps, k_cache, v_cache, slots.to(gpu),
+                      bias=buf[offset:] if with_bias else None, q_weight=wq.to(gpu) if weighted else None,
+                      k_weight=wk.to(gpu) if weighted else None, norm_first=norm == "weights first")
+    full = qkv.double() + (bias.double() if with_bias else 0.0)
+    first = torch.arange(0, rot, 2) if interleaved else torch.arange(rot // 2)
+    second = first + 1 if interleaved else first + rot // 2
+
+    def encode(x, w):
+        def unit(z):
+            return z / torch.sqrt((z ** 2).mean(-1, keepdim=True) + eps) * (w.double() if weighted else 1.0)
+        x = unit(x) if norm == "weights first" else x.clone()
+        if rot:
+            c, s, u, v = cos.double()[:, None], sin.double()[:, None], x[..., first].clone(), x[..., second].clone()
+            x[..., first], x[..., second] = u * c - v * s, v * c + u * s
+        return unit(x) if norm in ("unit", "weights") else x
+    close(got[:, :heads * dim].view(T, heads, dim), encode(full[:, :heads * dim].view(T, heads, dim), wq), TOL["bfloat16"], "queries")
+    written = slots >= 0
+    sl = slots.long()[written]
+    keys = K.pages_to_keys(k_cache).reshape(pages, kv_heads, page, dim)
+    want = encode(full[:, heads * dim:(heads + kv_heads) * dim].view(T, kv_heads, dim), wk)[written]
+    close(keys[sl // page, :, sl % page], want, TOL["bfloat16"], "cached keys")
+    close(v_cache[sl // page, :, :, sl % page], full[:, (heads + kv_heads) * dim:].view(T, kv_heads, vdim)[written], 4e-3, "cached values")
