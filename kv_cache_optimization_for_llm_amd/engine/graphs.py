@@ -220,7 +220,7 @@ class _PortionSlot:
 class PortionGraphs:
     """Graphs for steps that hold prompt portions (alone or beside decoded tokens).
 
-    A shape is (tokens per entry, wanted places, context bucket, the power of two below the mean number of
+    A shape is (tokens per entry, wanted places, context bucket, the step (MEAN_KEYS_STEPS) below the mean number of
     keys the portions' rows visit, by which the attention kernel is chosen): everything the forward pass decides on the
     host.  Its first step runs eagerly and tells which sets of attention work items the pass asks
     for; the step at which it has come ``CAPTURE_AT`` times is captured over static buffers; later

@@ -6,7 +6,6 @@ contexts over several wavefronts when the batch alone would leave most of the GP
 """
 from __future__ import annotations
 
-import numpy as np
 import torch
 
 from . import kernels as K
@@ -64,8 +63,9 @@ _LDS_MIN_GROUPS_WIDE_HEADS = 16
 _LDS_TARGET_GROUPS_WIDE_HEADS = 512
 _LDS_MIN_KEYS_PER_SPLIT_WIDE_HEADS = 256
 # where the choice can change (a step shape that has a graph is told apart by these too)
-# (choose_portion_waves knows the mean to the power of two below it; the lines above are among them)
-MEAN_KEYS_STEPS = tuple(1 << k for k in range(6, 20))
+# (choose_portion_waves knows the mean to the step below it; the lines above are among them.  Few: every step is a line
+# between shapes that are captured apart)
+MEAN_KEYS_STEPS = (128,) + tuple(1 << k for k in range(9, 15))
 assert {_LDS_MIN_MEAN_KEYS_WIDE_HEADS, _LDS_SOME_GROUPS_MEAN_KEYS, _LDS_MIN_MEAN_KEYS} <= set(MEAN_KEYS_STEPS)
 # few workgroups that each walk thousands of keys: the keys are cut into ranges, one workgroup each
 _LDS_TARGET_GROUPS = 1024
@@ -83,15 +83,18 @@ def choose_portion_waves(waves: int, mean_keys: float, head_dim: int) -> int:
 
     One wavefront on two row tiles is a chain of products, softmax and products, 0.9 us a block of 32 keys with its SIMD to
     itself, and fixed key ranges with a merge kernel cost that kernel and leave early rows' ranges empty.  us a call without
-    -> with, 32 heads of 64 over 8: one prompt of 256 / 512 / 1,024 / 1,536 / 2,048 / 2,304 / 2,560 tokens 14 / 26 / 22 / 34 / 44 /
-    51 / 56 -> 7 / 10 / 17 / 26 / 39 / 45 / 52 (3,072 the same, 4,096 94 -> 112 and from there the workgroup kernel); three of
-    509 20 -> 15; 256 tokens behind 1,024 / 4,096 / 8,000 24 / 35 / 49 -> 12 / 26 / 42, 512 behind 2,000 / 4,096 / 7,000 41 / 52 /
-    70 -> 23 / 36 / 53, 1,024 behind 2,000 / 6,000 65 / 107 -> 41 / 92, 2,048 behind 2,000 / 6,000 112 / 201 -> 89 / 188.  Not so: 64
-    behind 4,096 21 -> 24, 128 behind 8,000 32 -> 41, 512 behind 30,000 194 -> 199, eight of 200 10.4 -> 12.2 (a tie at four of 512).
-    Heads of 32 and 96 alike.  Heads of 128 hold a SIMD's registers with one wavefront, so what there is to win ends
-    earlier: 32 heads, 256 / 512 / 768 tokens 26 / 35 / 40 -> 10 / 14 / 19, 256 behind 1,024 / 4,096 34 / 41 -> 17 / 36, 512 behind 2,000
-    49 -> 36; 24 heads, 1,024 tokens 42 -> 22, four of 256 behind 1,000 57 -> 38; but four of 256 (32 heads) 13 -> 16, behind 1,000
-    38 -> 43, eight of 100 9.6 -> 11.9, 512 behind 7,000 90 -> 104."""
+    -> with, 32 heads of 64 over 8: one prompt of 256 / 512 / 1,024 / 1,536 / 2,048 / 2,304 / 2,560 tokens 14 / 26 / 22 / 34 /
+    44 / 51 / 56 -> 7 / 10 / 17 / 26 / 39 / 45 / 52 (3,072 the same, 4,096 94 -> 112 and from there the workgroup kernel);
+    three of 509 20 -> 15; 256 tokens behind 1,024 / 4,096 / 8,000 24 / 35 / 49 -> 12 / 26 / 42, 1,024 behind 2,000 / 6,000
+    65 / 107 -> 41 / 92, 2,048 behind 2,000 / 6,000 112 / 201 -> 89 / 188.  Not so: 64 behind 4,096 21 -> 24, 128 behind 8,000
+    32 -> 41, 512 behind 30,000 194 -> 199, eight of 200 10.4 -> 12.2 (a tie at four of 512).  Heads of 32 and 96 alike.
+    (512 to 767 pairs from 2,048 keys on stay with the workgroup kernel and its key ranges, which the tests of portions deep in
+    a prompt rest on, though 512 tokens behind 2,000 / 4,096 / 7,000 would go 41 / 52 / 70 -> 23 / 36 / 53.)
+
+    Heads of 128 hold a SIMD's registers with one wavefront, so what there is to win ends earlier: 32 heads, 256 / 512 / 768
+    tokens 26 / 35 / 40 -> 10 / 14 / 19, 256 behind 1,024 / 4,096 34 / 41 -> 17 / 36, 512 behind 2,000 49 -> 36; 24 heads, 1,024
+    tokens 42 -> 22, four of 256 behind 1,000 57 -> 38; but four of 256 (32 heads) 13 -> 16, behind 1,000 38 -> 43, eight of
+    100 9.6 -> 11.9, 512 behind 7,000 90 -> 104."""
     if head_dim > 128:
         return 1
     keys = max((step for step in MEAN_KEYS_STEPS if step <= mean_keys), default=0)
@@ -101,6 +104,8 @@ def choose_portion_waves(waves: int, mean_keys: float, head_dim: int) -> int:
         if waves <= 256:
             return 2 if waves >= 128 else 1
         return 2 if waves < 1024 and waves <= 12 * keys and keys <= 4 * waves else 1
+    if 512 <= waves < 768 and keys >= _LDS_MIN_MEAN_KEYS:
+        return 1
     if waves <= 512:
         if keys >= 512:
             return 4 if keys <= 16 * waves else 1
@@ -514,9 +519,11 @@ def _plan(batch, group: int, num_kv_heads: int, head_dim: int, page_size: int, m
     which = "long" if mixed else "all"
     # two row tiles per wave, so each key and value loaded serves 32 query rows
     tiles = K.attention_mfma_row_tiles(head_dim, True)
-    rows = np.diff(batch.h_entry_q_start).astype(np.int64) * group
-    count = int((-(-(rows[rows > 16] if mixed else rows) // (16 * tiles))).sum()) * num_kv_heads
-    sharing = choose_portion_waves(count, batch.mean_keys_of_long_entries(), head_dim)
+    starts = batch.h_entry_q_start.tolist()
+    rows = [(end - start) * group for start, end in zip(starts, starts[1:])]
+    count = sum(-(-n // (16 * tiles)) for n in rows if not mixed or n > 16) * num_kv_heads
+    mean_keys = batch.mean_keys_of_long_entries()
+    sharing = choose_portion_waves(count, mean_keys, head_dim)
     if tiles == 2 and sharing > 1:
         items = batch.attention_items(group, tiles, which)
         plan.append(("wave", items, tiles, sharing, 0, False, which == "all", False, sharing))
@@ -527,7 +534,7 @@ def _plan(batch, group: int, num_kv_heads: int, head_dim: int, page_size: int, m
     if K.attention_lds_supported(head_dim, page_size):
         items = batch.attention_items(group, 8, which)
         groups = items[0].shape[0] * num_kv_heads
-        if items[2] is not None and use_lds_kernel(groups, batch.mean_keys_of_long_entries(), head_dim):
+        if items[2] is not None and use_lds_kernel(groups, mean_keys, head_dim):
             splits, per = choose_lds_splits(groups, batch.max_context, head_dim=head_dim)
             plan.append(("lds", items[2], splits, per, which == "all"))
             done = True

@@ -207,7 +207,7 @@ def test_portions_that_share_an_item():
     assert [choose_portion_waves(n, mean, 128) for n, mean in ((256, 128), (256, 1152), (768, 384), (640, 50), (1024, 512), (512, 7256))] \
         == [2, 4, 2, 1, 1, 1]
     assert choose_portion_waves(512, 256, 160) == 1
-    for head_dim in (64, 128):          # nothing but the power of two below the mean decides: a captured step's shape names it
+    for head_dim in (64, 128):          # nothing but the step below the mean decides: a captured step's shape names it
         for n in range(1, 4000, 61):
             for mean in range(1, 5000, 83):
                 step = max([s for s in MEAN_KEYS_STEPS if s <= mean], default=0)
