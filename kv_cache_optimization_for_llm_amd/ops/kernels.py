@@ -1785,7 +1785,7 @@ LINEAR_ATTENTION_CHUNKS_FROM = 160
 
 def recurrent_chunk_floats(dim: int, vdim: int) -> int:
     """Floats of workspace a chunk of 64 tokens takes per head (csrc/recurrent_chunks.hip: ``ck_block``)."""
-    return 3 * 64 * dim + 64 * 64 + vdim * (64 + dim) + dim
+    return 3 * 64 * dim + 64 * 64 + vdim * (2 * 64 + dim) + dim
 
 
 def _recurrent_plan(lengths, chunks_from: int, entries: int, tokens: int, heads: int, dim: int, vdim: int,

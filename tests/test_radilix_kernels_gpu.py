@@ -324,6 +324,47 @@ def test_gated_linear_attention_in_chunks(heads, dim, vdim, act, decays, portion
                 assert rms(pair[0].to(F) - true) <= max(2.5 * rms(pair[1].to(F) - true), 2e-7 * rms(true)), (what, s, h)
 
 
+@pytest.mark.parametrize("share", [0.0, 1.0, 3.0])
+@pytest.mark.parametrize("decays", ["none", "slow", "usual", "slow, channel"])
+@pytest.mark.parametrize("rule", ["delta", "linear"])
+def test_chunks_are_as_close_to_64_bits_as_the_walk(rule, decays, share, gpu):
+    """Also where keys and queries share a direction, so that u are differences of neighbouring tokens' values.  (Measured: 0.2
+    to 0.6 of the walk's error with the delta rule, 0.5 to 1.0 with linear attention.)"""
+    heads, dim, vdim, n = 2, 128, 128, 900
+    g = torch.Generator().manual_seed(7 + int(share))
+    q, k = (torch.randn(n, heads, dim, generator=g) + share * torch.randn(1, heads, dim, generator=g) for _ in range(2))
+    v = torch.randn(n, heads, vdim, generator=g)
+    span = {"none": 0.0, "slow": 0.01, "usual": 0.1}[decays.split(",")[0]]
+    alpha = torch.exp(-span * torch.rand(n, heads, dim if "channel" in decays else 1, generator=g)).expand(-1, -1, dim).contiguous()
+    y = torch.randn(n, heads, generator=g).to(torch.bfloat16)
+    rows = torch.cat([x.reshape(n, -1) for x in (q, k, v)], dim=1)
+    if rule == "linear":
+        y = rows = rows.to(torch.bfloat16)
+        q, k, v = (x.view(n, heads, -1) for x in rows.float().split([heads * dim, heads * dim, heads * vdim], dim=1))
+    S, want = torch.zeros(heads, dim, vdim, dtype=F), torch.empty(n, heads, vdim, dtype=F)
+    q, k, v, a = q.to(F), k.to(F), v.to(F), alpha.to(F)
+    if rule == "delta":
+        q, k, beta = plain.unit_vectors(q), plain.unit_vectors(k), torch.sigmoid(y.to(F))
+    for t in range(n):
+        S = a[t, :, :, None] * S
+        u = beta[t, :, None] * (v[t] - torch.einsum("hdv,hd->hv", S, k[t])) if rule == "delta" else v[t]
+        S = S + k[t, :, :, None] * u[:, None]
+        want[t] = torch.einsum("hdv,hd->hv", S, q[t]) * dim ** -0.5
+    error = {}
+    for lengths in ([n], None):
+        state = torch.zeros((1, heads * dim * vdim), dtype=torch.float32, device="cuda")
+        out = torch.empty((n, heads * vdim), dtype=torch.float32, device="cuda")
+        if rule == "delta":
+            K.gated_delta_rule(dev(rows), y.to("cuda"), 0, 0, None, None, out, state, 0, ints([0, n]), ints([0]), heads, heads, dim, vdim,
+                               channel_decay=dev(alpha.view(n, -1)), lengths=lengths)
+        else:
+            K.gated_linear_attention(y.to("cuda"), 0, heads * dim, 2 * heads * dim, dev(alpha.view(n, -1)), dim ** -0.5, out, state, 0,
+                                     ints([0, n]), ints([0]), heads, dim, vdim, lengths=lengths)
+        error[lengths is None] = (rms(out.cpu().view(n, heads, vdim) - want) / rms(want), rms(state.cpu().view(heads, dim, vdim) - S) / rms(S))
+    print(rule, decays, share, error)
+    assert all(c <= w for c, w in zip(error[False], error[True])), error
+
+
 def test_a_seat_used_again_after_zeroing_forgets_and_a_far_token_is_remembered(gpu):
     """A value written at the first position with a key of its own comes back 700 tokens later when
     nothing decays (both recurrences); the same seat zeroed gives a fresh request's numbers."""
