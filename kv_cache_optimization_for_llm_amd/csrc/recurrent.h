@@ -18,3 +18,17 @@ __device__ inline float rec_sigmoid(float z) { return 1.f / (1.f + expf(-z)); }
 __device__ inline float rec_silu(float z) { return z / (1.f + expf(-z)); }
 __device__ inline float rec_softplus(float z) { return fmaxf(z, 0.f) + log1pf(expf(-fabsf(z))); }
 __device__ inline float rec_act(float z, int act) { return act == 1 ? rec_silu(z) : z; }
+
+// Long entries' chunks of 64 tokens (recurrent_chunks.hip) are numbered through, entry e's from here on: sums of
+// ceil(n / 64) never exceed that.
+#define REC_CHUNK_TOKENS 64
+__device__ inline int rec_first_chunk(int q0, int e) { return q0 / REC_CHUNK_TOKENS + e; }
+
+// Whether an input of (an entry's n tokens, head) is infinite or not a number, as chunk_prepare_kernel leaves it per
+// chunk in `odd` [chunks][heads].  Asked by whole wavefronts.
+__device__ inline bool rec_odd_entry(const int *__restrict__ odd, int q0, int e, int n, int heads, int head) {
+    const int first = rec_first_chunk(q0, e), chunks = (n + REC_CHUNK_TOKENS - 1) / REC_CHUNK_TOKENS;
+    int seen = 0;
+    for (int c = threadIdx.x % KVA_WAVE; c < chunks; c += KVA_WAVE) seen |= odd[(size_t)(first + c) * heads + head];
+    return __ballot(seen != 0) != 0;
+}

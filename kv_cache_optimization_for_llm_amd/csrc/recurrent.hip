@@ -235,7 +235,8 @@ struct RecArgs {
     int state_off;
     const int *entry_q_start, *entry_seat;
     int heads, kv_heads, dim, vdim, chunk;
-    int below;                  // entries of that many tokens or more are left to the kernels that take chunks
+    int below;                  // entries of that many tokens or more are left to the kernels that take chunks ...
+    const int *odd;             // ... unless they hold something that is not a number (rec_odd_entry)
 };
 
 // Gated delta rule.  q, k, v are the convolution's fp32 output rows [T, conv_stride]: q at
@@ -252,7 +253,7 @@ gated_delta_rule_kernel(RecArgs a, const float *__restrict__ qkv, int conv_strid
     const int head = blockIdx.x / slices, col = (blockIdx.x % slices) * REC_COLS + c;
     const int e = blockIdx.y;
     const int q0 = a.entry_q_start[e], n = a.entry_q_start[e + 1] - q0;
-    if (n <= 0 || n >= a.below) return;
+    if (n <= 0 || (n >= a.below && !(a.odd && rec_odd_entry(a.odd, q0, e, n, a.heads, head)))) return;
     const int d = a.dim, dv = a.vdim, kvh = head / (a.heads / a.kv_heads);
     const bool on = col < dv;
     float *S = lds, *qs = S + d * REC_COLS, *ks = qs + a.chunk * d, *bs = ks + a.chunk * d, *gs = bs + a.chunk;
@@ -337,7 +338,7 @@ gated_linear_attention_kernel(RecArgs a, const void *__restrict__ y, int y_dtype
     const int head = blockIdx.x / slices, col = (blockIdx.x % slices) * REC_COLS + c;
     const int e = blockIdx.y;
     const int q0 = a.entry_q_start[e], n = a.entry_q_start[e + 1] - q0;
-    if (n <= 0 || n >= a.below) return;
+    if (n <= 0 || (n >= a.below && !(a.odd && rec_odd_entry(a.odd, q0, e, n, a.heads, head)))) return;
     const int d = a.dim, dv = a.vdim;
     const bool on = col < dv;
     float *S = lds, *qs = S + d * REC_COLS, *ks = qs + a.chunk * d, *as = ks + a.chunk * d;
@@ -432,7 +433,7 @@ gated_delta_rule_reg_kernel(RecArgs a, const float *__restrict__ qkv, int conv_s
     const int col = block_col0 + wave * REG_COLS + c;
     const int e = blockIdx.y;
     const int q0 = a.entry_q_start[e], n = a.entry_q_start[e + 1] - q0;
-    if (n <= 0 || n >= a.below) return;
+    if (n <= 0 || (n >= a.below && !(a.odd && rec_odd_entry(a.odd, q0, e, n, a.heads, head)))) return;
     const int d = a.dim, dv = a.vdim, kvh = head / (a.heads / a.kv_heads);
     const bool on = col < dv;
     float *Sg = a.state + (size_t)a.entry_seat[e] * a.seat_stride + a.state_off + (size_t)head * d * dv;
@@ -607,7 +608,7 @@ gated_linear_attention_reg_kernel(RecArgs a, const void *__restrict__ y, int y_d
     const int col = block_col0 + wave * REG_COLS + c;
     const int e = blockIdx.y;
     const int q0 = a.entry_q_start[e], n = a.entry_q_start[e + 1] - q0;
-    if (n <= 0 || n >= a.below) return;
+    if (n <= 0 || (n >= a.below && !(a.odd && rec_odd_entry(a.odd, q0, e, n, a.heads, head)))) return;
     const int d = a.dim, dv = a.vdim;
     const bool on = col < dv;
     float *Sg = a.state + (size_t)a.entry_seat[e] * a.seat_stride + a.state_off + (size_t)head * d * dv;
@@ -735,7 +736,7 @@ extern "C" int kva_gated_delta_rule(float *out, float *state, long long seat_str
                                     int decay_off, const float *a_log, const float *dt_bias, float unit_eps,
                                     const float *channel_decay, int decay_stride,
                                     const int *entry_q_start, const int *entry_seat, int entries, int heads,
-                                    int kv_heads, int dim, int vdim, int below, hipStream_t stream) {
+                                    int kv_heads, int dim, int vdim, int below, const int *odd, hipStream_t stream) {
     if (int rc = rec_check("gated_delta_rule", out, state, entry_q_start, entry_seat, entries, heads, kv_heads, dim, vdim)) return rc;
     // the decay: one per head, formed here from a column of y, a rate and a bias - or one per head and
     // key channel, handed in ready-made (fp32 [T, >= heads * dim])
@@ -743,7 +744,7 @@ extern "C" int kva_gated_delta_rule(float *out, float *state, long long seat_str
                 "gated_delta_rule: missing operand");
     if (entries == 0) return KVA_OK;
     if (dim <= 128) {
-        RecArgs a{out, state, (size_t)seat_stride, state_off, entry_q_start, entry_seat, heads, kv_heads, dim, vdim, REC_CHUNK, below};
+        RecArgs a{out, state, (size_t)seat_stride, state_off, entry_q_start, entry_seat, heads, kv_heads, dim, vdim, REC_CHUNK, below, odd};
         const dim3 grid(heads * ((vdim + REG_BLOCK_COLS - 1) / REG_BLOCK_COLS), entries);
 #define KVA_DELTA_REG(RP)                                                                                              \
     do {                                                                                                               \
@@ -765,7 +766,7 @@ extern "C" int kva_gated_delta_rule(float *out, float *state, long long seat_str
     const int arrays = channel_decay ? 3 : 2;
     const int chunk = rec_chunk(dim, arrays);
     KVA_REQUIRE(chunk > 0, "gated_delta_rule: key size %d does not fit the LDS", dim);
-    RecArgs a{out, state, (size_t)seat_stride, state_off, entry_q_start, entry_seat, heads, kv_heads, dim, vdim, chunk, below};
+    RecArgs a{out, state, (size_t)seat_stride, state_off, entry_q_start, entry_seat, heads, kv_heads, dim, vdim, chunk, below, odd};
     const size_t lds = ((size_t)dim * REC_COLS + (size_t)chunk * dim * arrays + 2 * chunk) * sizeof(float);
     const int slices = (vdim + REC_COLS - 1) / REC_COLS;
     hipLaunchKernelGGL(gated_delta_rule_kernel, dim3(heads * slices, entries), dim3(KVA_WAVE), lds, stream, a, qkv,
@@ -780,14 +781,15 @@ extern "C" int kva_gated_linear_attention(float *out, float *state, long long se
                                           const float *alpha, int alpha_stride, float q_mul,
                                           const float *head_decay, int act,
                                           const int *entry_q_start, const int *entry_seat,
-                                          int entries, int heads, int dim, int vdim, int below, hipStream_t stream) {
+                                          int entries, int heads, int dim, int vdim, int below, const int *odd,
+                                          hipStream_t stream) {
     if (int rc = rec_check("gated_linear_attention", out, state, entry_q_start, entry_seat, entries, heads, heads, dim, vdim)) return rc;
     // the decays: a buffer with one value per token, head and key channel, or one fixed value a head
     KVA_REQUIRE(y && ((alpha && alpha_stride >= heads * dim) || (!alpha && head_decay)), "gated_linear_attention: missing operand");
     KVA_REQUIRE(act == 0 || act == 1, "gated_linear_attention: activation %d is neither none (0) nor silu (1)", act);
     if (entries == 0) return KVA_OK;
     if (dim <= 128) {
-        RecArgs a{out, state, (size_t)seat_stride, state_off, entry_q_start, entry_seat, heads, heads, dim, vdim, REC_CHUNK, below};
+        RecArgs a{out, state, (size_t)seat_stride, state_off, entry_q_start, entry_seat, heads, heads, dim, vdim, REC_CHUNK, below, odd};
         const dim3 grid(heads * ((vdim + REG_BLOCK_COLS - 1) / REG_BLOCK_COLS), entries);
 #define KVA_GLA_REG(RP)                                                                                                \
     hipLaunchKernelGGL(gated_linear_attention_reg_kernel<RP>, grid, dim3(REG_THREADS), 0, stream, a, y, y_dtype,          \
@@ -800,7 +802,7 @@ extern "C" int kva_gated_linear_attention(float *out, float *state, long long se
     }
     const int chunk = rec_chunk(dim, 3);
     KVA_REQUIRE(chunk > 0, "gated_linear_attention: key size %d does not fit the LDS", dim);
-    RecArgs a{out, state, (size_t)seat_stride, state_off, entry_q_start, entry_seat, heads, heads, dim, vdim, chunk, below};
+    RecArgs a{out, state, (size_t)seat_stride, state_off, entry_q_start, entry_seat, heads, heads, dim, vdim, chunk, below, odd};
     const size_t lds = ((size_t)dim * REC_COLS + (size_t)chunk * dim * 3) * sizeof(float);
     const int slices = (vdim + REC_COLS - 1) / REC_COLS;
     hipLaunchKernelGGL(gated_linear_attention_kernel, dim3(heads * slices, entries), dim3(KVA_WAVE), lds, stream, a, y,

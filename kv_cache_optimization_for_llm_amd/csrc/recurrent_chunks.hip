@@ -22,6 +22,8 @@
 // against 64 bits, the walk -> all in 32 bits -> this: 3.9e-7 -> 8.8e-7 -> 0.8e-7 with keys that share half of their
 // square, 2.2e-7 -> 7e-7 -> 1.1e-7 with nine tenths and decays from 0.9 up.  Decays only ever enter as products of decays
 // between two tokens (at most 1, no logarithms, no quotients): a decay of zero or of anything else is as exact as in the walk.
+// Where anything of an entry's inputs to a head is infinite or not a number, `prepare` says so and that (entry, head) is left
+// to the walk behind these kernels: zeros above a diagonal would carry it to tokens in front of it.
 // Order of sums: chunks are counted from the step's first token of the request, so here - unlike in the walk - the
 // last bits of a token's result depend on how the request was cut into steps.  The 32-bit path therefore walks.
 //
@@ -32,8 +34,9 @@
 // chunk and two trips through LDS; with operands row by row instead of in operand order and a head's workgroups spread
 // over the dies it took twice as long.  `prepare` and `outputs` are short of workgroups (256) more than of anything else.
 #include "recurrent.h"
+#include <float.h>
 
-#define CK 64                       // tokens a chunk
+#define CK REC_CHUNK_TOKENS         // tokens a chunk
 #define CK_PAD 4                    // a row in LDS is that much longer: rows start in different banks
 
 typedef float ck_f32x4 __attribute__((ext_vector_type(4)));
@@ -48,6 +51,7 @@ struct ChunkArgs {
     int heads, kv_heads, vdim;
     int shortest;                   // entries of fewer tokens are left to the walk
     float *work;                    // per (chunk, head) a block of ck_block() floats
+    int *odd;                       // per (chunk, head): whether an input is infinite or not a number
 };
 
 // A (chunk, head)'s block: W [CK][D], Qd [CK][D], Kd^T [D][CK], P [CK][CK], U^T [vdim][CK] (64-bit, linear attention uses half
@@ -69,8 +73,7 @@ template <int D>
 struct ChunkBlock {
     float *w, *q, *kt, *p, *ut, *st, *g;
     __device__ inline ChunkBlock(const ChunkArgs &a, int q0, int e, int chunk, int head) {
-        // entry e's chunks begin at q0 / CK + e: sums of ceil(n / CK) never exceed that
-        w = a.work + ((size_t)(q0 / CK + e + chunk) * a.heads + head) * ck_block(D, a.vdim);
+        w = a.work + ((size_t)(rec_first_chunk(q0, e) + chunk) * a.heads + head) * ck_block(D, a.vdim);
         q = w + CK * D;
         kt = q + CK * D;
         p = kt + CK * D;
@@ -132,6 +135,8 @@ struct ChunkInput {
     double q_mul;
 };
 
+__device__ inline bool ck_odd(float x) { return !(fabsf(x) <= FLT_MAX); }
+
 // Where the four elements of a lane's share of 16 tokens lie next to each other: tokens g, g + 4, g + 8, g + 12 at 4 g.
 __device__ inline int ck_place(int x) { return 4 * (x % 4) + x / 4; }
 
@@ -164,6 +169,7 @@ chunk_prepare_kernel(ChunkArgs a, ChunkInput in) {
     const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid / KVA_WAVE), lane = tid % KVA_WAVE;
     const int r = lane % 16, g = lane / 16, b0 = wave * 16;
     ChunkBlock<D> out(a, q0, e, chunk, head);
+    bool odd = false;               // an input of this thread's is not a number, or infinite
 
     // ---- the chunk's tokens; rows behind the last one are zero (decay 1): they change nothing
     if (DELTA) {
@@ -179,6 +185,8 @@ chunk_prepare_kernel(ChunkArgs a, ChunkInput in) {
 #pragma unroll
         for (int j = 0; j < PER; ++j) {
             const int x = tid + 256 * j, t = x / (D / 4), i = x % (D / 4) * 4;
+#pragma unroll
+            for (int c = 0; c < 4; ++c) odd |= ck_odd(lq[j][c]) || ck_odd(lk[j][c]);
             ck_st(&Q[t][i], t < m ? lq[j] : ck_f32x4{0.f, 0.f, 0.f, 0.f});
             ck_st(&Kx[t][i], t < m ? lk[j] : ck_f32x4{0.f, 0.f, 0.f, 0.f});
         }
@@ -196,6 +204,7 @@ chunk_prepare_kernel(ChunkArgs a, ChunkInput in) {
 #pragma unroll
             for (int j = 0; j < AT; ++j) {
                 const int x = tid + 256 * (j0 + j), t = x / D, i = x % D;
+                odd |= ck_odd(lq[j]) || ck_odd(lk[j]);
                 Q[t][i] = t < m ? rec_act(lq[j], in.act) * (float)in.q_mul : 0.f;
                 Kx[t][i] = t < m ? rec_act(lk[j], in.act) : 0.f;
             }
@@ -213,6 +222,7 @@ chunk_prepare_kernel(ChunkArgs a, ChunkInput in) {
 #pragma unroll
             for (int j = 0; j < AT; ++j) {
                 const int x = tid + 256 * (j0 + j), t = x / D, i = x % D;
+                odd |= ck_odd(la[j]);
                 Al[CD ? t : 0][i] = t < m ? la[j] : 1.f;
             }
         }
@@ -226,6 +236,7 @@ chunk_prepare_kernel(ChunkArgs a, ChunkInput in) {
             else if (!CD)
                 d = expf(-expf(in.a_log[head]) * rec_softplus(rec_ld(in.y, in.y_dtype, yrow + in.decay_off + head) + in.dt_bias[head]));
         }
+        odd |= ck_odd(b) || ck_odd(d);
         beta[tid] = b;
         gs[tid] = d;
         nq[tid] = nk[tid] = 1.0;
@@ -395,9 +406,14 @@ chunk_prepare_kernel(ChunkArgs a, ChunkInput in) {
         for (int s = 0; s < 4; ++s)
 #pragma unroll
             for (int c = 0; c < 4; ++c) {
+                odd |= ck_odd(v[s][c]);
                 if (!DELTA) v[s][c] = rec_act(v[s][c], in.act);
                 if (16 * s + ck_token(g, c) >= m) v[s][c] = 0.f;
             }
+    };
+    auto note_odd = [&] {
+        const int any = __syncthreads_or(odd ? 1 : 0);
+        if (tid == 0) a.odd[(size_t)(rec_first_chunk(q0, e) + chunk) * a.heads + head] = any;
     };
     if (!DELTA) {                   // U is V
         for (int tile = wave; tile < a.vdim / 16; tile += 4) {
@@ -406,6 +422,7 @@ chunk_prepare_kernel(ChunkArgs a, ChunkInput in) {
 #pragma unroll
             for (int s = 0; s < 4; ++s) ck_st(out.ut + ck_frag(tile, s, 4, lane), v[s]);
         }
+        note_odd();
         return;
     }
 
@@ -487,6 +504,7 @@ chunk_prepare_kernel(ChunkArgs a, ChunkInput in) {
             ck_st(uv + ck_frag(tile, I, 4, lane), acc);
         }
     }
+    note_odd();
 }
 
 // One workgroup a (request, head, 16 value columns), chunk after chunk.  A wavefront keeps D / 64 tiles of 16 rows of
@@ -507,7 +525,7 @@ chunk_states_kernel(ChunkArgs a) {
     __shared__ __attribute__((aligned(32))) R Ut[16 * CK];
     const int e = blockIdx.y, head = blockIdx.x % a.heads, tile = blockIdx.x / a.heads;
     const int q0 = a.entry_q_start[e], n = a.entry_q_start[e + 1] - q0;
-    if (n < a.shortest) return;
+    if (n < a.shortest || rec_odd_entry(a.odd, q0, e, n, a.heads, head)) return;
     const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid / KVA_WAVE), lane = tid % KVA_WAVE;
     const int r = lane % 16, g = lane / 16, chunks = (n + CK - 1) / CK, col = 16 * tile + r;
     float *Sg = a.state + (size_t)a.entry_seat[e] * a.seat_stride + a.state_off + (size_t)head * D * a.vdim;
@@ -584,7 +602,7 @@ chunk_outputs_kernel(ChunkArgs a) {
     using R = typename CkSum<DELTA>::type;
     const int e = blockIdx.z, head = blockIdx.y, chunk = blockIdx.x;
     const int q0 = a.entry_q_start[e], n = a.entry_q_start[e + 1] - q0;
-    if (n < a.shortest || chunk * CK >= n) return;
+    if (n < a.shortest || chunk * CK >= n || rec_odd_entry(a.odd, q0, e, n, a.heads, head)) return;
     const int m = min(CK, n - chunk * CK), row0 = q0 + chunk * CK, tiles = a.vdim / 16;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / KVA_WAVE), lane = threadIdx.x % KVA_WAVE, r = lane % 16, g = lane / 16;
     const ChunkBlock<D> b(a, q0, e, chunk, head);
@@ -647,7 +665,7 @@ static void ck_launch(const ChunkArgs &a, const ChunkInput &in, int longest, int
 }
 
 static int ck_check(const char *what, const ChunkArgs &a, int dim, int longest, int entries, int tokens, long long work_floats) {
-    KVA_REQUIRE(a.out && a.state && a.entry_q_start && a.entry_seat && a.work, "%s: missing operand", what);
+    KVA_REQUIRE(a.out && a.state && a.entry_q_start && a.entry_seat && a.work && a.odd, "%s: missing operand", what);
     KVA_REQUIRE(ck_fits(dim, a.vdim), "%s: chunks are built for key sizes 64 and 128 and value sizes that are multiples of 16, not %d x %d", what, dim, a.vdim);
     KVA_REQUIRE(a.heads > 0 && a.heads <= 65535 && a.kv_heads > 0 && a.heads % a.kv_heads == 0, "%s: %d heads over %d key heads", what, a.heads, a.kv_heads);
     KVA_REQUIRE(entries > 0 && entries <= 65535 && longest > 0 && longest <= tokens && a.shortest >= 1, "%s: %d entries of up to %d tokens", what, entries, longest);
@@ -665,8 +683,8 @@ extern "C" int kva_gated_delta_rule_chunks(float *out, float *state, long long s
                                            const float *channel_decay, int decay_stride, const int *entry_q_start,
                                            const int *entry_seat, int entries, int heads, int kv_heads, int dim, int vdim,
                                            int tokens, int shortest, int longest, float *work, long long work_floats,
-                                           hipStream_t stream) {
-    const ChunkArgs a{out, state, (size_t)seat_stride, state_off, entry_q_start, entry_seat, heads, kv_heads, vdim, shortest, work};
+                                           int *odd, hipStream_t stream) {
+    const ChunkArgs a{out, state, (size_t)seat_stride, state_off, entry_q_start, entry_seat, heads, kv_heads, vdim, shortest, work, odd};
     if (int rc = ck_check("gated_delta_rule", a, dim, longest, entries, tokens, work_floats)) return rc;
     KVA_REQUIRE(qkv && y && ((a_log && dt_bias) || (channel_decay && decay_stride >= heads * dim)), "gated_delta_rule: missing operand");
     KVA_REQUIRE((uintptr_t)qkv % 16 == 0 && conv_stride % 4 == 0, "gated_delta_rule: rows of q, k and v must start at multiples of 16 bytes");
@@ -684,8 +702,8 @@ extern "C" int kva_gated_linear_attention_chunks(float *out, float *state, long 
                                                  const float *alpha, int alpha_stride, float q_mul, const float *head_decay,
                                                  int act, const int *entry_q_start, const int *entry_seat, int entries,
                                                  int heads, int dim, int vdim, int tokens, int shortest, int longest,
-                                                 float *work, long long work_floats, hipStream_t stream) {
-    const ChunkArgs a{out, state, (size_t)seat_stride, state_off, entry_q_start, entry_seat, heads, heads, vdim, shortest, work};
+                                                 float *work, long long work_floats, int *odd, hipStream_t stream) {
+    const ChunkArgs a{out, state, (size_t)seat_stride, state_off, entry_q_start, entry_seat, heads, heads, vdim, shortest, work, odd};
     if (int rc = ck_check("gated_linear_attention", a, dim, longest, entries, tokens, work_floats)) return rc;
     KVA_REQUIRE(y && ((alpha && alpha_stride >= heads * dim) || (!alpha && head_decay)), "gated_linear_attention: missing operand");
     KVA_REQUIRE(act == 0 || act == 1, "gated_linear_attention: activation %d is neither none (0) nor silu (1)", act);

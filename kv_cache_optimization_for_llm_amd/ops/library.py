@@ -95,10 +95,10 @@ _HIP_SIGNATURES = {
     "kva_upload": [P, P, LL, P],
     "kva_latent_prompt": [P, P, I, I, P, P, P, P, P, I, P, P, P, I, P, P, I, P, P, I, I, I, I, I, I, I, I, F, P],
     "kva_latent_prompt_supported": [I, I, I, I],
-    "kva_gated_delta_rule": [P, P, LL, I, P, I, P, I, I, I, I, P, P, F, P, I, P, P, I, I, I, I, I, I, P],
-    "kva_gated_linear_attention": [P, P, LL, I, P, I, I, I, I, I, P, I, F, P, I, P, P, I, I, I, I, I, P],
-    "kva_gated_delta_rule_chunks": [P, P, LL, I, P, I, P, I, I, I, I, P, P, F, P, I, P, P, I, I, I, I, I, I, I, I, P, LL, P],
-    "kva_gated_linear_attention_chunks": [P, P, LL, I, P, I, I, I, I, I, P, I, F, P, I, P, P, I, I, I, I, I, I, I, P, LL, P],
+    "kva_gated_delta_rule": [P, P, LL, I, P, I, P, I, I, I, I, P, P, F, P, I, P, P, I, I, I, I, I, I, P, P],
+    "kva_gated_linear_attention": [P, P, LL, I, P, I, I, I, I, I, P, I, F, P, I, P, P, I, I, I, I, I, P, P],
+    "kva_gated_delta_rule_chunks": [P, P, LL, I, P, I, P, I, I, I, I, P, P, F, P, I, P, P, I, I, I, I, I, I, I, I, P, LL, P, P],
+    "kva_gated_linear_attention_chunks": [P, P, LL, I, P, I, I, I, I, I, P, I, F, P, I, P, P, I, I, I, I, I, I, I, P, LL, P, P],
     "kva_head_norm_gate": [P, I, I, I, P, I, P, F, P, I, I, I, I, I, I, I, I, F, I, P],
     "kva_moe_route": [P, P, P, P, I, I, I, I, I, I, I, I, I, F, F, I, P],
     "kva_moe_router": [P, P, P, P, I, P, P, P, I, I, I, I, I, I, I, I, I, I, I, F, F, P, P, I, I, I, I, P],

@@ -365,6 +365,46 @@ def test_chunks_are_as_close_to_64_bits_as_the_walk(rule, decays, share, gpu):
     assert all(c <= w for c, w in zip(error[False], error[True])), error
 
 
+@pytest.mark.parametrize("bad", [float("nan"), float("inf"), -float("inf")])
+@pytest.mark.parametrize("where, at", [("q", 64), ("k", 69), ("v", 5), ("v", 199), ("decay", 140), ("beta", 70)])
+@pytest.mark.parametrize("rule", ["delta", "delta, channel", "linear"])
+def test_tokens_in_front_of_one_that_is_not_a_number_stay_as_they_are(rule, where, at, bad, gpu):
+    """An input of one token and head, in an entry that goes in chunks beside one that does not: every read-out and state is what
+    the walk over the tokens gives, numbers or not; tokens in front and other heads are numbers."""
+    heads, dim, vdim, n = 3, 64, 32, 200
+    g = torch.Generator().manual_seed(at)
+    T, F32 = n + 7, torch.float32
+    q, k, v = (torch.randn(T, heads, w, generator=g).to(torch.bfloat16).to(F32) for w in (dim, dim, vdim))
+    alpha = torch.rand(T, heads, dim, generator=g) ** 0.2
+    y = torch.randn(T, 2 * heads, generator=g).to(torch.bfloat16)
+    if where in ("q", "k", "v"):
+        {"q": q, "k": k, "v": v}[where][at, 1, 3] = bad
+    elif where == "decay":
+        alpha[at, 1, 3] = bad
+        y[at, heads + 1] = bad
+    else:
+        y[at, 1] = bad
+    got = {}
+    for lengths in ([n, 7], None):
+        state = torch.zeros((2, heads * dim * vdim), dtype=F32, device="cuda")
+        out = torch.full((T, heads * vdim), -7.0, dtype=F32, device="cuda")
+        tail = (out, state, 0, ints([0, n, T]), ints([1, 0]))
+        if rule == "linear":
+            rows = torch.cat([x.reshape(T, -1) for x in (q, k, v)], dim=1).to(torch.bfloat16).to("cuda")
+            K.gated_linear_attention(rows, 0, heads * dim, 2 * heads * dim, dev(alpha.view(T, -1)), dim ** -0.5, *tail, heads, dim, vdim,
+                                     lengths=lengths)
+        else:
+            rows = dev(torch.cat([x.reshape(T, -1) for x in (q, k, v)], dim=1))
+            K.gated_delta_rule(rows, y.to("cuda"), 0, heads, dev(torch.zeros(heads)), dev(torch.zeros(heads)), *tail, heads, heads, dim, vdim,
+                               channel_decay=dev(alpha.view(T, -1)) if "channel" in rule else None, lengths=lengths)
+        got[lengths is None] = (out.view(T, heads, vdim).cpu(), state.view(2, heads, dim, vdim).cpu())
+    out, state = got[False]
+    assert out[:at].isfinite().all() and out[:, [0, 2]].isfinite().all() and out[n:].isfinite().all()
+    assert state[0].isfinite().all() and state[1][[0, 2]].isfinite().all()
+    for x, walked in zip(got[False], got[True]):
+        torch.testing.assert_close(x, walked, rtol=1e-4, atol=1e-5, equal_nan=True)
+
+
 def test_a_seat_used_again_after_zeroing_forgets_and_a_far_token_is_remembered(gpu):
     """A value written at the first position with a key of its own comes back 700 tokens later when
     nothing decays (both recurrences); the same seat zeroed gives a fresh request's numbers."""
