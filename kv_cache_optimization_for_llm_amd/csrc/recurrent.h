@@ -19,15 +19,27 @@ __device__ inline float rec_silu(float z) { return z / (1.f + expf(-z)); }
 __device__ inline float rec_softplus(float z) { return fmaxf(z, 0.f) + log1pf(expf(-fabsf(z))); }
 __device__ inline float rec_act(float z, int act) { return act == 1 ? rec_silu(z) : z; }
 
-// Long entries' chunks of 64 tokens (recurrent_chunks.hip) are numbered through, entry e's from here on: sums of
-// ceil(n / 64) never exceed that.
+// The chunks of 64 tokens (recurrent_chunks.hip) of all entries of `shortest` tokens and more are numbered through.
 #define REC_CHUNK_TOKENS 64
-__device__ inline int rec_first_chunk(int q0, int e) { return q0 / REC_CHUNK_TOKENS + e; }
+
+__device__ inline int rec_chunks_of(const int *__restrict__ entry_q_start, int e, int shortest) {
+    const int n = entry_q_start[e + 1] - entry_q_start[e];
+    return n >= shortest ? (n + REC_CHUNK_TOKENS - 1) / REC_CHUNK_TOKENS : 0;
+}
+
+// The number of the first one of entry e.  Asked by whole wavefronts.
+__device__ inline int rec_first_chunk(const int *__restrict__ entry_q_start, int e, int shortest) {
+    int before = 0;
+    for (int x = threadIdx.x % KVA_WAVE; x < e; x += KVA_WAVE) before += rec_chunks_of(entry_q_start, x, shortest);
+#pragma unroll
+    for (int o = KVA_WAVE / 2; o > 0; o >>= 1) before += __shfl_xor(before, o, KVA_WAVE);
+    return before;
+}
 
 // Whether an input of (an entry's n tokens, head) is infinite or not a number, as chunk_prepare_kernel leaves it per
-// chunk in `odd` [chunks][heads].  Asked by whole wavefronts.
-__device__ inline bool rec_odd_entry(const int *__restrict__ odd, int q0, int e, int n, int heads, int head) {
-    const int first = rec_first_chunk(q0, e), chunks = (n + REC_CHUNK_TOKENS - 1) / REC_CHUNK_TOKENS;
+// chunk (from `first` on) in `odd` [chunks][heads].  Asked by whole wavefronts.
+__device__ inline bool rec_odd_entry(const int *__restrict__ odd, int first, int n, int heads, int head) {
+    const int chunks = (n + REC_CHUNK_TOKENS - 1) / REC_CHUNK_TOKENS;
     int seen = 0;
     for (int c = threadIdx.x % KVA_WAVE; c < chunks; c += KVA_WAVE) seen |= odd[(size_t)(first + c) * heads + head];
     return __ballot(seen != 0) != 0;

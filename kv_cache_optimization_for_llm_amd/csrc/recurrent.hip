@@ -239,6 +239,10 @@ struct RecArgs {
     const int *odd;             // ... unless they hold something that is not a number (rec_odd_entry)
 };
 
+__device__ inline bool rec_left_to_chunks(const RecArgs &a, int e, int n, int head) {
+    return n >= a.below && !(a.odd && rec_odd_entry(a.odd, rec_first_chunk(a.entry_q_start, e, a.below), n, a.heads, head));
+}
+
 // Gated delta rule.  q, k, v are the convolution's fp32 output rows [T, conv_stride]: q at
 // column 0 (kv_heads x dim), k behind it, v behind that (heads x vdim).  beta and the decay's input
 // are columns of the projection y.
@@ -253,7 +257,7 @@ gated_delta_rule_kernel(RecArgs a, const float *__restrict__ qkv, int conv_strid
     const int head = blockIdx.x / slices, col = (blockIdx.x % slices) * REC_COLS + c;
     const int e = blockIdx.y;
     const int q0 = a.entry_q_start[e], n = a.entry_q_start[e + 1] - q0;
-    if (n <= 0 || (n >= a.below && !(a.odd && rec_odd_entry(a.odd, q0, e, n, a.heads, head)))) return;
+    if (n <= 0 || rec_left_to_chunks(a, e, n, head)) return;
     const int d = a.dim, dv = a.vdim, kvh = head / (a.heads / a.kv_heads);
     const bool on = col < dv;
     float *S = lds, *qs = S + d * REC_COLS, *ks = qs + a.chunk * d, *bs = ks + a.chunk * d, *gs = bs + a.chunk;
@@ -338,7 +342,7 @@ gated_linear_attention_kernel(RecArgs a, const void *__restrict__ y, int y_dtype
     const int head = blockIdx.x / slices, col = (blockIdx.x % slices) * REC_COLS + c;
     const int e = blockIdx.y;
     const int q0 = a.entry_q_start[e], n = a.entry_q_start[e + 1] - q0;
-    if (n <= 0 || (n >= a.below && !(a.odd && rec_odd_entry(a.odd, q0, e, n, a.heads, head)))) return;
+    if (n <= 0 || rec_left_to_chunks(a, e, n, head)) return;
     const int d = a.dim, dv = a.vdim;
     const bool on = col < dv;
     float *S = lds, *qs = S + d * REC_COLS, *ks = qs + a.chunk * d, *as = ks + a.chunk * d;
@@ -433,7 +437,7 @@ gated_delta_rule_reg_kernel(RecArgs a, const float *__restrict__ qkv, int conv_s
     const int col = block_col0 + wave * REG_COLS + c;
     const int e = blockIdx.y;
     const int q0 = a.entry_q_start[e], n = a.entry_q_start[e + 1] - q0;
-    if (n <= 0 || (n >= a.below && !(a.odd && rec_odd_entry(a.odd, q0, e, n, a.heads, head)))) return;
+    if (n <= 0 || rec_left_to_chunks(a, e, n, head)) return;
     const int d = a.dim, dv = a.vdim, kvh = head / (a.heads / a.kv_heads);
     const bool on = col < dv;
     float *Sg = a.state + (size_t)a.entry_seat[e] * a.seat_stride + a.state_off + (size_t)head * d * dv;
@@ -608,7 +612,7 @@ gated_linear_attention_reg_kernel(RecArgs a, const void *__restrict__ y, int y_d
     const int col = block_col0 + wave * REG_COLS + c;
     const int e = blockIdx.y;
     const int q0 = a.entry_q_start[e], n = a.entry_q_start[e + 1] - q0;
-    if (n <= 0 || (n >= a.below && !(a.odd && rec_odd_entry(a.odd, q0, e, n, a.heads, head)))) return;
+    if (n <= 0 || rec_left_to_chunks(a, e, n, head)) return;
     const int d = a.dim, dv = a.vdim;
     const bool on = col < dv;
     float *Sg = a.state + (size_t)a.entry_seat[e] * a.seat_stride + a.state_off + (size_t)head * d * dv;

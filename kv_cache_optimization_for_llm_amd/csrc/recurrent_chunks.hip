@@ -49,7 +49,7 @@ struct ChunkArgs {
     int state_off;
     const int *entry_q_start, *entry_seat;
     int heads, kv_heads, vdim;
-    int shortest;                   // entries of fewer tokens are left to the walk
+    int entries, shortest, chunks;  // entries of fewer tokens than `shortest` are left to the walk, the others have so many chunks
     float *work;                    // per (chunk, head) a block of ck_block() floats
     int *odd;                       // per (chunk, head): whether an input is infinite or not a number
 };
@@ -72,8 +72,8 @@ __device__ inline size_t ck_frag(int rowtile, int coltile, int coltiles, int lan
 template <int D>
 struct ChunkBlock {
     float *w, *q, *kt, *p, *ut, *st, *g;
-    __device__ inline ChunkBlock(const ChunkArgs &a, int q0, int e, int chunk, int head) {
-        w = a.work + ((size_t)(rec_first_chunk(q0, e) + chunk) * a.heads + head) * ck_block(D, a.vdim);
+    __device__ inline ChunkBlock(const ChunkArgs &a, int number, int head) {
+        w = a.work + ((size_t)number * a.heads + head) * ck_block(D, a.vdim);
         q = w + CK * D;
         kt = q + CK * D;
         p = kt + CK * D;
@@ -82,6 +82,33 @@ struct ChunkBlock {
         g = st + (size_t)a.vdim * D;
     }
 };
+
+// Chunk `number`: the `chunk`th of entry `entry`, whose first one has the number `first`.  Asked by whole wavefronts;
+// 64 entries a turn.
+struct ChunkPlace {
+    int entry, chunk, first;
+};
+__device__ inline ChunkPlace ck_find(const ChunkArgs &a, int number) {
+    const int lane = threadIdx.x % KVA_WAVE;
+    if (a.entries == 1) return {number < rec_chunks_of(a.entry_q_start, 0, a.shortest) ? 0 : -1, number, 0};
+    for (int e0 = 0, before = 0; e0 < a.entries; e0 += KVA_WAVE) {
+        const int mine = e0 + lane < a.entries ? rec_chunks_of(a.entry_q_start, e0 + lane, a.shortest) : 0;
+        int upto = mine;
+#pragma unroll
+        for (int o = 1; o < KVA_WAVE; o <<= 1) {
+            const int other = __shfl_up(upto, o, KVA_WAVE);
+            if (lane >= o) upto += other;
+        }
+        const unsigned long long past = __ballot(number < before + upto);
+        if (past) {
+            const int owner = __builtin_amdgcn_readfirstlane(__ffsll(past) - 1);
+            const int first = __builtin_amdgcn_readfirstlane(before + __shfl(upto - mine, owner, KVA_WAVE));
+            return {e0 + owner, number - first, first};
+        }
+        before += __shfl(upto, KVA_WAVE - 1, KVA_WAVE);
+    }
+    return {-1, 0, 0};              // (more chunks asked for than the entries have)
+}
 
 template <bool DELTA> __device__ inline int ck_channel(int g, int c) { return DELTA ? g + 4 * c : 4 * g + c; }
 __device__ inline int ck_token(int g, int c) { return g + 4 * c; }
@@ -162,13 +189,15 @@ chunk_prepare_kernel(ChunkArgs a, ChunkInput in) {
     __shared__ float beta[CK];
     auto &Q = QT.q;
     auto &T = QT.t;
-    const int e = blockIdx.z, head = blockIdx.y, chunk = blockIdx.x;
+    const int head = blockIdx.y;
+    const ChunkPlace place = ck_find(a, blockIdx.x);
+    const int e = place.entry, chunk = place.chunk;
+    if (e < 0) return;
     const int q0 = a.entry_q_start[e], n = a.entry_q_start[e + 1] - q0;
-    if (n < a.shortest || chunk * CK >= n) return;
     const int m = min(CK, n - chunk * CK), row0 = q0 + chunk * CK, kvh = head / (a.heads / a.kv_heads);
     const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid / KVA_WAVE), lane = tid % KVA_WAVE;
     const int r = lane % 16, g = lane / 16, b0 = wave * 16;
-    ChunkBlock<D> out(a, q0, e, chunk, head);
+    ChunkBlock<D> out(a, blockIdx.x, head);
     bool odd = false;               // an input of this thread's is not a number, or infinite
 
     // ---- the chunk's tokens; rows behind the last one are zero (decay 1): they change nothing
@@ -413,7 +442,7 @@ chunk_prepare_kernel(ChunkArgs a, ChunkInput in) {
     };
     auto note_odd = [&] {
         const int any = __syncthreads_or(odd ? 1 : 0);
-        if (tid == 0) a.odd[(size_t)(rec_first_chunk(q0, e) + chunk) * a.heads + head] = any;
+        if (tid == 0) a.odd[(size_t)blockIdx.x * a.heads + head] = any;
     };
     if (!DELTA) {                   // U is V
         for (int tile = wave; tile < a.vdim / 16; tile += 4) {
@@ -525,7 +554,9 @@ chunk_states_kernel(ChunkArgs a) {
     __shared__ __attribute__((aligned(32))) R Ut[16 * CK];
     const int e = blockIdx.y, head = blockIdx.x % a.heads, tile = blockIdx.x / a.heads;
     const int q0 = a.entry_q_start[e], n = a.entry_q_start[e + 1] - q0;
-    if (n < a.shortest || rec_odd_entry(a.odd, q0, e, n, a.heads, head)) return;
+    if (n < a.shortest) return;
+    const int first = __builtin_amdgcn_readfirstlane(rec_first_chunk(a.entry_q_start, e, a.shortest));
+    if (first + (n + CK - 1) / CK > a.chunks || rec_odd_entry(a.odd, first, n, a.heads, head)) return;
     const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid / KVA_WAVE), lane = tid % KVA_WAVE;
     const int r = lane % 16, g = lane / 16, chunks = (n + CK - 1) / CK, col = 16 * tile + r;
     float *Sg = a.state + (size_t)a.entry_seat[e] * a.seat_stride + a.state_off + (size_t)head * D * a.vdim;
@@ -539,7 +570,7 @@ chunk_states_kernel(ChunkArgs a) {
         R4 uv;
     } o[2];
     auto fetch = [&](Operands &x, int chunk) {
-        const ChunkBlock<D> b(a, q0, e, min(chunk, chunks - 1), head);
+        const ChunkBlock<D> b(a, first + min(chunk, chunks - 1), head);
         x.uv = ck_ld(reinterpret_cast<const R *>(b.ut) + ck_frag(tile, wave, 4, lane));
         if (DELTA)
 #pragma unroll
@@ -552,7 +583,7 @@ chunk_states_kernel(ChunkArgs a) {
         }
     };
     auto step = [&](const Operands &x, Operands &next, int chunk) {
-        const ChunkBlock<D> b(a, q0, e, chunk, head);
+        const ChunkBlock<D> b(a, first + chunk, head);
 #pragma unroll
         for (int t = 0; t < MT; ++t) {
             if (DELTA) ck_st(&St[ck_frag(0, wave * MT + t, STEPS, lane)], S[t]);
@@ -600,12 +631,15 @@ __global__ void __launch_bounds__(256)
 chunk_outputs_kernel(ChunkArgs a) {
     constexpr int STEPS = D / 16;
     using R = typename CkSum<DELTA>::type;
-    const int e = blockIdx.z, head = blockIdx.y, chunk = blockIdx.x;
+    const int head = blockIdx.y;
+    const ChunkPlace place = ck_find(a, blockIdx.x);
+    const int e = place.entry, chunk = place.chunk;
+    if (e < 0) return;
     const int q0 = a.entry_q_start[e], n = a.entry_q_start[e + 1] - q0;
-    if (n < a.shortest || chunk * CK >= n || rec_odd_entry(a.odd, q0, e, n, a.heads, head)) return;
+    if (rec_odd_entry(a.odd, place.first, n, a.heads, head)) return;
     const int m = min(CK, n - chunk * CK), row0 = q0 + chunk * CK, tiles = a.vdim / 16;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / KVA_WAVE), lane = threadIdx.x % KVA_WAVE, r = lane % 16, g = lane / 16;
-    const ChunkBlock<D> b(a, q0, e, chunk, head);
+    const ChunkBlock<D> b(a, blockIdx.x, head);
     for (int tile = 2 * wave; tile < tiles; tile += 8) {
         const int second = min(tile + 1, tiles - 1);        // (an odd last tile twice: the second result is dropped)
         ck_f64x4 acc[CK / 16][2];
@@ -649,49 +683,49 @@ chunk_outputs_kernel(ChunkArgs a) {
 // Sizes these kernels are built for; other ones walk.
 static bool ck_fits(int dim, int vdim) { return (dim == 64 || dim == 128) && vdim > 0 && vdim % 16 == 0; }
 
-// floats of workspace for a step of `tokens` tokens in `entries` entries; 0: not for these sizes
-extern "C" long long kva_recurrent_chunks_workspace(int tokens, int entries, int heads, int dim, int vdim) {
-    if (!ck_fits(dim, vdim) || tokens < 0 || entries < 0 || heads <= 0) return 0;
-    return (long long)(tokens / CK + entries) * heads * (long long)ck_block(dim, vdim);
+// floats of workspace for so many chunks of 64 tokens; 0: not for these sizes
+extern "C" long long kva_recurrent_chunks_workspace(int chunks, int heads, int dim, int vdim) {
+    if (!ck_fits(dim, vdim) || chunks < 0 || heads <= 0) return 0;
+    return (long long)chunks * heads * (long long)ck_block(dim, vdim);
 }
 
 template <int D, bool DELTA>
-static void ck_launch(const ChunkArgs &a, const ChunkInput &in, int longest, int entries, hipStream_t stream) {
-    const dim3 grid((longest + CK - 1) / CK, a.heads, entries);
+static void ck_launch(const ChunkArgs &a, const ChunkInput &in, hipStream_t stream) {
+    const dim3 grid(a.chunks, a.heads);
     if (in.channel_decay) hipLaunchKernelGGL((chunk_prepare_kernel<D, DELTA, true>), grid, dim3(256), 0, stream, a, in);
     else hipLaunchKernelGGL((chunk_prepare_kernel<D, DELTA, false>), grid, dim3(256), 0, stream, a, in);
-    hipLaunchKernelGGL((chunk_states_kernel<D, DELTA>), dim3(a.heads * (a.vdim / 16), entries), dim3(256), 0, stream, a);
+    hipLaunchKernelGGL((chunk_states_kernel<D, DELTA>), dim3(a.heads * (a.vdim / 16), a.entries), dim3(256), 0, stream, a);
     hipLaunchKernelGGL((chunk_outputs_kernel<D, DELTA>), grid, dim3(256), 0, stream, a);
 }
 
-static int ck_check(const char *what, const ChunkArgs &a, int dim, int longest, int entries, int tokens, long long work_floats) {
+static int ck_check(const char *what, const ChunkArgs &a, int dim, long long work_floats) {
     KVA_REQUIRE(a.out && a.state && a.entry_q_start && a.entry_seat && a.work && a.odd, "%s: missing operand", what);
     KVA_REQUIRE(ck_fits(dim, a.vdim), "%s: chunks are built for key sizes 64 and 128 and value sizes that are multiples of 16, not %d x %d", what, dim, a.vdim);
     KVA_REQUIRE(a.heads > 0 && a.heads <= 65535 && a.kv_heads > 0 && a.heads % a.kv_heads == 0, "%s: %d heads over %d key heads", what, a.heads, a.kv_heads);
-    KVA_REQUIRE(entries > 0 && entries <= 65535 && longest > 0 && longest <= tokens && a.shortest >= 1, "%s: %d entries of up to %d tokens", what, entries, longest);
+    KVA_REQUIRE(a.entries > 0 && a.entries <= 65535 && a.chunks > 0 && a.shortest >= 1, "%s: %d chunks in %d entries", what, a.chunks, a.entries);
     KVA_REQUIRE((uintptr_t)a.work % 32 == 0, "%s: the workspace must start at a multiple of 32 bytes", what);
     KVA_REQUIRE(a.heads * (long long)(a.vdim / 16) < (1LL << 31), "%s: %d heads of %d values", what, a.heads, a.vdim);
-    KVA_REQUIRE(work_floats >= kva_recurrent_chunks_workspace(tokens, entries, a.heads, dim, a.vdim), "%s: the workspace is too small", what);
+    KVA_REQUIRE(work_floats >= kva_recurrent_chunks_workspace(a.chunks, a.heads, dim, a.vdim), "%s: the workspace is too small", what);
     return KVA_OK;
 }
 
-// The same operands as kva_gated_delta_rule; entries of fewer than `shortest` tokens are left alone, no entry has more
-// than `longest` of the step's `tokens`.
+// The same operands as kva_gated_delta_rule; entries of fewer than `shortest` tokens are left alone, the others have
+// `chunks` chunks of 64 tokens (the last one of each may be shorter) between them.  `odd`: int32 [chunks, heads].
 extern "C" int kva_gated_delta_rule_chunks(float *out, float *state, long long seat_stride, int state_off, const float *qkv,
                                            int conv_stride, const void *y, int y_dtype, int y_stride, int beta_off,
                                            int decay_off, const float *a_log, const float *dt_bias, float unit_eps,
                                            const float *channel_decay, int decay_stride, const int *entry_q_start,
                                            const int *entry_seat, int entries, int heads, int kv_heads, int dim, int vdim,
-                                           int tokens, int shortest, int longest, float *work, long long work_floats,
+                                           int shortest, int chunks, float *work, long long work_floats,
                                            int *odd, hipStream_t stream) {
-    const ChunkArgs a{out, state, (size_t)seat_stride, state_off, entry_q_start, entry_seat, heads, kv_heads, vdim, shortest, work, odd};
-    if (int rc = ck_check("gated_delta_rule", a, dim, longest, entries, tokens, work_floats)) return rc;
+    const ChunkArgs a{out, state, (size_t)seat_stride, state_off, entry_q_start, entry_seat, heads, kv_heads, vdim, entries, shortest, chunks, work, odd};
+    if (int rc = ck_check("gated_delta_rule", a, dim, work_floats)) return rc;
     KVA_REQUIRE(qkv && y && ((a_log && dt_bias) || (channel_decay && decay_stride >= heads * dim)), "gated_delta_rule: missing operand");
     KVA_REQUIRE((uintptr_t)qkv % 16 == 0 && conv_stride % 4 == 0, "gated_delta_rule: rows of q, k and v must start at multiples of 16 bytes");
     const ChunkInput in{qkv, y, conv_stride, y_dtype, y_stride, 0, kv_heads * dim, 2 * kv_heads * dim, beta_off, decay_off, 0,
                         a_log, dt_bias, channel_decay, nullptr, decay_stride, unit_eps, 1.0 / sqrt((double)dim)};
-    if (dim == 64) ck_launch<64, true>(a, in, longest, entries, stream);
-    else ck_launch<128, true>(a, in, longest, entries, stream);
+    if (dim == 64) ck_launch<64, true>(a, in, stream);
+    else ck_launch<128, true>(a, in, stream);
     KVA_CHECK_LAUNCH("gated_delta_rule_chunks");
     return KVA_OK;
 }
@@ -701,16 +735,16 @@ extern "C" int kva_gated_linear_attention_chunks(float *out, float *state, long 
                                                  const void *y, int y_dtype, int y_stride, int q_off, int k_off, int v_off,
                                                  const float *alpha, int alpha_stride, float q_mul, const float *head_decay,
                                                  int act, const int *entry_q_start, const int *entry_seat, int entries,
-                                                 int heads, int dim, int vdim, int tokens, int shortest, int longest,
+                                                 int heads, int dim, int vdim, int shortest, int chunks,
                                                  float *work, long long work_floats, int *odd, hipStream_t stream) {
-    const ChunkArgs a{out, state, (size_t)seat_stride, state_off, entry_q_start, entry_seat, heads, heads, vdim, shortest, work, odd};
-    if (int rc = ck_check("gated_linear_attention", a, dim, longest, entries, tokens, work_floats)) return rc;
+    const ChunkArgs a{out, state, (size_t)seat_stride, state_off, entry_q_start, entry_seat, heads, heads, vdim, entries, shortest, chunks, work, odd};
+    if (int rc = ck_check("gated_linear_attention", a, dim, work_floats)) return rc;
     KVA_REQUIRE(y && ((alpha && alpha_stride >= heads * dim) || (!alpha && head_decay)), "gated_linear_attention: missing operand");
     KVA_REQUIRE(act == 0 || act == 1, "gated_linear_attention: activation %d is neither none (0) nor silu (1)", act);
     const ChunkInput in{nullptr, y, 0, y_dtype, y_stride, q_off, k_off, v_off, 0, 0, act, nullptr, nullptr, alpha, head_decay,
                         alpha_stride, 0.f, q_mul};
-    if (dim == 64) ck_launch<64, false>(a, in, longest, entries, stream);
-    else ck_launch<128, false>(a, in, longest, entries, stream);
+    if (dim == 64) ck_launch<64, false>(a, in, stream);
+    else ck_launch<128, false>(a, in, stream);
     KVA_CHECK_LAUNCH("gated_linear_attention_chunks");
     return KVA_OK;
 }

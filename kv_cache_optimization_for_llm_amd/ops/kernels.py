@@ -7,6 +7,7 @@ a tensor that is not on the GPU, or a missing kernel library, is an error.
 from __future__ import annotations
 
 import ctypes
+import math
 from typing import Optional
 
 import torch
@@ -1783,36 +1784,36 @@ DELTA_RULE_CHUNKS_FROM = 96
 LINEAR_ATTENTION_CHUNKS_FROM = 160
 
 
-def recurrent_chunk_floats(dim: int, vdim: int) -> int:
-    """Floats of workspace a chunk of 64 tokens takes per head (csrc/recurrent_chunks.hip: ``ck_block``)."""
-    return 3 * 64 * dim + 64 * 64 + vdim * (2 * 64 + dim) + dim
+def recurrent_chunk_elements(chunks_from: int, heads: int, dim: int, vdim: int) -> int:
+    """32-bit elements of workspace that entries in chunks take a token at most (csrc/recurrent_chunks.hip: ``ck_block`` per
+    chunk of 64 tokens and head; an entry's last chunk may hold a single token)."""
+    block = 3 * 64 * dim + 64 * 64 + vdim * (2 * 64 + dim) + dim + 1
+    worst = max(-(-n // 64) / n for n in (chunks_from, (chunks_from + 62) // 64 * 64 + 1))
+    return math.ceil(heads * block * worst)
 
 
 def _recurrent_plan(lengths, chunks_from: int, entries: int, tokens: int, heads: int, dim: int, vdim: int,
                     dtype: torch.dtype, what: str):
-    """(entries from this many tokens on go in chunks, the longest entry, floats of workspace) for
+    """(entries from this many tokens on go in chunks, how many chunks they have, floats of workspace) for
     entries of ``lengths`` tokens (host numbers; ``None``: not known, all walk)."""
+    none = (1 << 30, 0, 0)
     if lengths is None:
-        return 1 << 30, 0, 0
+        return none
     lengths = [int(n) for n in lengths]
     if len(lengths) != entries or sum(lengths) != tokens:
         raise KernelError(f"{what}: one length per entry, of all the rows together")
-    longest = max(lengths, default=0)
-    work = 0
     # (32-bit projections: a token's bits do not depend on how its request was cut, so they walk)
-    if dtype == torch.bfloat16 and longest >= chunks_from:
-        work = int(hip_lib().kva_recurrent_chunks_workspace(tokens, entries, heads, dim, vdim))
-    if work == 0:
-        return 1 << 30, 0, 0
-    return int(chunks_from), longest, work
+    chunks = sum(-(-n // 64) for n in lengths if n >= chunks_from) if dtype == torch.bfloat16 else 0
+    floats = int(hip_lib().kva_recurrent_chunks_workspace(chunks, heads, dim, vdim))
+    return (int(chunks_from), chunks, floats) if floats else none
 
 
-def _recurrent_chunks(what: str, operands: tuple, tokens: int, below: int, longest: int, floats: int, entries: int, heads: int, device):
+def _recurrent_chunks(what: str, operands: tuple, below: int, chunks: int, floats: int, heads: int, device):
     """Runs the entries of ``below`` tokens and more in chunks.  What the walk behind them, which takes the others, must be told:
     per (chunk, head) whether an input is not a number - such entries it takes as well."""
     work = torch.empty(floats, dtype=torch.float32, device=device)
-    odd = torch.empty((tokens // 64 + entries) * heads, dtype=torch.int32, device=device)
-    check(getattr(hip_lib(), f"kva_{what}_chunks")(*operands, tokens, below, longest, _dev(work, "work"), floats, _dev(odd, "odd"),
+    odd = torch.empty(chunks * heads, dtype=torch.int32, device=device)
+    check(getattr(hip_lib(), f"kva_{what}_chunks")(*operands, below, chunks, _dev(work, "work"), floats, _dev(odd, "odd"),
                                                    _stream()), what)
     return odd
 
@@ -1849,7 +1850,7 @@ def gated_delta_rule(qkv: torch.Tensor, y: torch.Tensor, beta_off: int, decay_of
         raise KernelError("gated_delta_rule: decay columns inside y, one rate and one bias per head")
     seat_stride = _state_row(state, state_off, heads * dim * vdim, "gated_delta_rule")
     qs, seat, entries = _entries((entry_q_start, entry_seat), "gated_delta_rule")
-    below, longest, floats = _recurrent_plan(lengths, DELTA_RULE_CHUNKS_FROM, entries, tokens, heads, dim, vdim, y.dtype,
+    below, chunks, floats = _recurrent_plan(lengths, DELTA_RULE_CHUNKS_FROM, entries, tokens, heads, dim, vdim, y.dtype,
                                              "gated_delta_rule")
     if qkv.data_ptr() % 16:         # (the chunks read 16 bytes at a time, the walk element by element)
         below, floats = 1 << 30, 0
@@ -1858,7 +1859,7 @@ def gated_delta_rule(qkv: torch.Tensor, y: torch.Tensor, beta_off: int, decay_of
                 _opt(a_log, "a_log", torch.float32), _opt(dt_bias, "dt_bias", torch.float32), float(unit_eps),
                 _opt(channel_decay, "channel_decay"), channel_decay.shape[1] if channel_decay is not None else 0, qs, seat,
                 entries, heads, kv_heads, dim, vdim)
-    odd = _recurrent_chunks("gated_delta_rule", operands, tokens, below, longest, floats, entries, heads, out.device) if floats else None
+    odd = _recurrent_chunks("gated_delta_rule", operands, below, chunks, floats, heads, out.device) if floats else None
     check(hip_lib().kva_gated_delta_rule(*operands, below, _opt(odd, "odd", torch.int32), _stream()), "gated_delta_rule")
     return out
 
@@ -1892,13 +1893,13 @@ def gated_linear_attention(y: torch.Tensor, q_off: int, k_off: int, v_off: int, 
             raise KernelError("gated_linear_attention: q, k or v columns lie outside y")
     seat_stride = _state_row(state, state_off, heads * dim * vdim, "gated_linear_attention")
     qs, seat, entries = _entries((entry_q_start, entry_seat), "gated_linear_attention")
-    below, longest, floats = _recurrent_plan(lengths, LINEAR_ATTENTION_CHUNKS_FROM, entries, tokens, heads, dim, vdim,
+    below, chunks, floats = _recurrent_plan(lengths, LINEAR_ATTENTION_CHUNKS_FROM, entries, tokens, heads, dim, vdim,
                                              y.dtype, "gated_linear_attention")
     operands = (_dev(out, "out"), _dev(state, "state"), seat_stride, int(state_off), _dev(y, "y"), dtype_code(y.dtype),
                 y.shape[1], int(q_off), int(k_off), int(v_off), _opt(alpha, "alpha"), alpha.shape[1] if alpha is not None else 0,
                 float(q_mul), _opt(head_decay, "head_decay"), 1 if activation == "silu" else 0, qs, seat,
                 entries, heads, dim, vdim)
-    odd = _recurrent_chunks("gated_linear_attention", operands, tokens, below, longest, floats, entries, heads, out.device) if floats else None
+    odd = _recurrent_chunks("gated_linear_attention", operands, below, chunks, floats, heads, out.device) if floats else None
     check(hip_lib().kva_gated_linear_attention(*operands, below, _opt(odd, "odd", torch.int32), _stream()), "gated_linear_attention")
     return out
 

@@ -97,8 +97,8 @@ _HIP_SIGNATURES = {
     "kva_latent_prompt_supported": [I, I, I, I],
     "kva_gated_delta_rule": [P, P, LL, I, P, I, P, I, I, I, I, P, P, F, P, I, P, P, I, I, I, I, I, I, P, P],
     "kva_gated_linear_attention": [P, P, LL, I, P, I, I, I, I, I, P, I, F, P, I, P, P, I, I, I, I, I, P, P],
-    "kva_gated_delta_rule_chunks": [P, P, LL, I, P, I, P, I, I, I, I, P, P, F, P, I, P, P, I, I, I, I, I, I, I, I, P, LL, P, P],
-    "kva_gated_linear_attention_chunks": [P, P, LL, I, P, I, I, I, I, I, P, I, F, P, I, P, P, I, I, I, I, I, I, I, P, LL, P, P],
+    "kva_gated_delta_rule_chunks": [P, P, LL, I, P, I, P, I, I, I, I, P, P, F, P, I, P, P, I, I, I, I, I, I, I, P, LL, P, P],
+    "kva_gated_linear_attention_chunks": [P, P, LL, I, P, I, I, I, I, I, P, I, F, P, I, P, P, I, I, I, I, I, I, P, LL, P, P],
     "kva_head_norm_gate": [P, I, I, I, P, I, P, F, P, I, I, I, I, I, I, I, I, F, I, P],
     "kva_moe_route": [P, P, P, P, I, I, I, I, I, I, I, I, I, F, F, I, P],
     "kva_moe_router": [P, P, P, P, I, P, P, P, I, I, I, I, I, I, I, I, I, I, I, F, F, P, P, I, I, I, I, P],
@@ -155,7 +155,7 @@ def hip_lib():
         lib.kva_sample_workspace_bytes.restype = LL
         lib.kva_state_space_workspace.argtypes = [I, I, I, I, I]
         lib.kva_state_space_workspace.restype = LL
-        lib.kva_recurrent_chunks_workspace.argtypes = [I, I, I, I, I]
+        lib.kva_recurrent_chunks_workspace.argtypes = [I, I, I, I]
         lib.kva_recurrent_chunks_workspace.restype = LL
         lib._path = path
         _hip = lib

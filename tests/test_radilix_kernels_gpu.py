@@ -405,6 +405,39 @@ def test_tokens_in_front_of_one_that_is_not_a_number_stay_as_they_are(rule, wher
         torch.testing.assert_close(x, walked, rtol=1e-4, atol=1e-5, equal_nan=True)
 
 
+def test_entries_in_chunks_among_many_that_are_not(gpu, monkeypatch):
+    """Chunks are numbered over the long entries alone, 64 entries of the step at a time: long ones at either end of such a run, alone
+    in it or not in it at all give what they give alone, and only they take workspace."""
+    heads, dim, vdim = 2, 64, 16
+    lens = [1] * 130
+    for e, n in ((0, 96), (63, 200), (64, 129), (100, 97), (129, 128)):
+        lens[e] = n
+    starts = np.cumsum([0] + lens)
+    g = torch.Generator().manual_seed(3)
+    y = torch.randn(int(starts[-1]), heads * (2 * dim + vdim), generator=g).to(torch.bfloat16).to("cuda")
+    alpha = dev(torch.rand(int(starts[-1]), heads * dim, generator=g) ** 0.2)
+    monkeypatch.setattr(K, "LINEAR_ATTENTION_CHUNKS_FROM", 96)
+    offs = (0, heads * dim, 2 * heads * dim)
+
+    def run(first, last):
+        rows = slice(int(starts[first]), int(starts[last]))
+        state = torch.zeros((last - first, heads * dim * vdim), dtype=torch.float32, device="cuda")
+        out = torch.full((rows.stop - rows.start, heads * vdim), float("nan"), dtype=torch.float32, device="cuda")
+        K.gated_linear_attention(y[rows].contiguous(), *offs, alpha[rows].contiguous(), dim ** -0.5, out, state, 0,
+                                 ints(starts[first:last + 1] - starts[first]), ints(range(last - first)), heads, dim, vdim,
+                                 lengths=lens[first:last])
+        return out, state
+    whole, states = run(0, len(lens))
+    for e in range(len(lens)):
+        out, state = run(e, e + 1)
+        assert torch.equal(out, whole[starts[e]:starts[e + 1]]) and torch.equal(state[0], states[e]), (e, lens[e])
+    # two blocks of 64 tokens for 96, 97 and 128 tokens, three for 129, four for 200
+    assert K._recurrent_plan(lens, 96, len(lens), sum(lens), heads, dim, vdim, torch.bfloat16, "")[1] == 13
+    most = K.recurrent_chunk_elements(96, heads, dim, vdim)
+    for n in range(96, 700):
+        assert K._recurrent_plan([n], 96, 1, n, heads, dim, vdim, torch.bfloat16, "")[2] <= most * n
+
+
 def test_a_seat_used_again_after_zeroing_forgets_and_a_far_token_is_remembered(gpu):
     """A value written at the first position with a key of its own comes back 700 tokens later when
     nothing decays (both recurrences); the same seat zeroed gives a fresh request's numbers."""
