@@ -1776,24 +1776,63 @@ def causal_conv_act(y: torch.Tensor, col_off: int, weight: torch.Tensor, out: to
     return out
 
 
-# Under bf16 projections an entry of so many tokens and more goes through the recurrence in chunks of 64.  The walk takes
-# about 0.35 us a token with the delta rule (8 heads of 128 x 128) and 0.2 with linear attention (16 of 64 x 128), the
-# chunks' three launches 37 and 30 us for a first chunk: 64 / 128 / 2,048 tokens 27 / 49 / 724 against 37 / 42 / 102 us,
-# and 16 / 27 / 547 against 31 / 32 / 75.
-DELTA_RULE_CHUNKS_FROM = 96
-LINEAR_ATTENTION_CHUNKS_FROM = 160
+# Under bf16 projections an entry of so many tokens and more goes through the recurrence in chunks of 64: by (key size, a decay
+# per key channel), for heads of up to 128 values and for wider ones (or one number for all).  The walk takes 0.2 to 0.5 us a
+# token one after the other, the chunks' launches 35 to 110 us at first.  us a call, walk / chunks, one entry of 128 / 192 / 256
+# tokens: delta rule, 8 heads of 128 x 128 49/58 70/62 91/66, x 256 49/79 70/83 91/89, channel decays 53/79 75/82 99/86; of 64 x
+# 128 36/41 52/43 68/45; linear attention, 8 heads of 128 x 128 43/69 62/70 81/72, fixed decays 55/57 80/58 105/59; of 64 x 128
+# 27/42 38/42 49/43, fixed decays 33/37 48/38 62/38.  2,048 tokens: 550 to 1,110 against 70 to 210 in all of these.
+DELTA_RULE_CHUNKS_FROM = {(128, False): (176, 256), (128, True): (224, 304), (64, False): (160, 208), (64, True): (192, 240)}
+LINEAR_ATTENTION_CHUNKS_FROM = {(128, False): (144, 208), (128, True): (240, 320), (64, False): (160, 192), (64, True): (224, 288)}
+
+# What a step of several entries costs either way, by (delta rule, key size, a decay per key channel), in us: the walk per token one
+# after the other; per token and 16 value columns of a head, and per entry and 16 columns, where workgroups fill the chip; the
+# chunks at first, per chunk one after the other, per (chunk, head) and for 16 more columns of it where they fill the chip.
+# (8 heads: one prompt of 64 to 2,048 tokens, 32 of 256, 256 of one.)  Walks of many entries run side by side and a walk of
+# short entries stands behind the chunks, so many prompts at once, or a long one among many decoded tokens, may do better without.
+_RECURRENT_COSTS = {
+    (True, 128, False): (0.345, 0.00077, 0.0130, 52.0, 3.3, 0.096, 0.0274), (True, 64, False): (0.254, 0.00039, 0.0060, 37.0, 1.9, 0.137, 0.0063),
+    (True, 128, True): (0.370, 0.00083, 0.0130, 72.0, 3.3, 0.183, 0.0271), (True, 64, True): (0.270, 0.00041, 0.0052, 46.0, 1.9, 0.172, 0.0070),
+    (False, 128, False): (0.410, 0.00114, 0.0102, 53.0, 1.9, 0.049, 0.0236), (False, 64, False): (0.230, 0.00039, 0.0052, 35.0, 1.1, 0.064, 0.0085),
+    (False, 128, True): (0.310, 0.00099, 0.0101, 65.0, 1.9, 0.193, 0.0263), (False, 64, True): (0.190, 0.00033, 0.0051, 39.0, 1.2, 0.140, 0.0055)}
+_RECURRENT_FULL = 25.0      # us of a walk's work from which on it, and not a single entry's tokens in a row, may be what counts
+
+
+def recurrent_chunks_pay(lengths, chunks_from: int, heads: int, dim: int, vdim: int, delta: bool, channel: bool) -> bool:
+    """Whether the entries of ``chunks_from`` tokens and more of a step should go in chunks."""
+    long = [n for n in lengths if n >= chunks_from]
+    if not long:
+        return False
+    chain, token, entry, first, then, block, columns = _RECURRENT_COSTS[delta, dim, channel]
+    cols = heads * -(-vdim // 16)
+    work = cols * (token * sum(lengths) + entry * len(lengths))
+    if work < _RECURRENT_FULL:
+        return True
+    chunks = [-(-n // 64) for n in long]
+    behind = cols * (token * (sum(lengths) - sum(long)) + entry * (len(lengths) - len(long)))
+    # (these times are good to 5 %)
+    return max(first + then * max(chunks), sum(chunks) * (heads * block + cols * columns)) + behind < 0.95 * max(chain * max(long), work)
 
 
 def recurrent_chunk_elements(chunks_from: int, heads: int, dim: int, vdim: int) -> int:
     """32-bit elements of workspace that entries in chunks take a token at most (csrc/recurrent_chunks.hip: ``ck_block`` per
     chunk of 64 tokens and head; an entry's last chunk may hold a single token)."""
+    if not chunks_from:
+        return 0
     block = 3 * 64 * dim + 64 * 64 + vdim * (2 * 64 + dim) + dim + 1
     worst = max(-(-n // 64) / n for n in (chunks_from, (chunks_from + 62) // 64 * 64 + 1))
     return math.ceil(heads * block * worst)
 
 
-def _recurrent_plan(lengths, chunks_from: int, entries: int, tokens: int, heads: int, dim: int, vdim: int,
-                    dtype: torch.dtype, what: str):
+def recurrent_chunks_from(table, dim: int, vdim: int, channel: bool) -> int:
+    """An entry's tokens from which on it may go in chunks (``DELTA_RULE_CHUNKS_FROM``, ``LINEAR_ATTENTION_CHUNKS_FROM``); 0: none
+    does with these sizes."""
+    if dim not in (64, 128) or vdim % 16:
+        return 0
+    return table if isinstance(table, int) else table[dim, channel][vdim > 128]
+
+
+def _recurrent_plan(lengths, entries: int, tokens: int, heads: int, dim: int, vdim: int, dtype: torch.dtype, delta: bool, channel: bool):
     """(entries from this many tokens on go in chunks, how many chunks they have, floats of workspace) for
     entries of ``lengths`` tokens (host numbers; ``None``: not known, all walk)."""
     none = (1 << 30, 0, 0)
@@ -1801,11 +1840,14 @@ def _recurrent_plan(lengths, chunks_from: int, entries: int, tokens: int, heads:
         return none
     lengths = [int(n) for n in lengths]
     if len(lengths) != entries or sum(lengths) != tokens:
-        raise KernelError(f"{what}: one length per entry, of all the rows together")
+        raise KernelError(f"{'gated_delta_rule' if delta else 'gated_linear_attention'}: one length per entry, of all the rows together")
+    chunks_from = recurrent_chunks_from(DELTA_RULE_CHUNKS_FROM if delta else LINEAR_ATTENTION_CHUNKS_FROM, dim, vdim, channel)
     # (32-bit projections: a token's bits do not depend on how its request was cut, so they walk)
-    chunks = sum(-(-n // 64) for n in lengths if n >= chunks_from) if dtype == torch.bfloat16 else 0
+    if dtype != torch.bfloat16 or not chunks_from or not recurrent_chunks_pay(lengths, chunks_from, heads, dim, vdim, delta, channel):
+        return none
+    chunks = sum(-(-n // 64) for n in lengths if n >= chunks_from)
     floats = int(hip_lib().kva_recurrent_chunks_workspace(chunks, heads, dim, vdim))
-    return (int(chunks_from), chunks, floats) if floats else none
+    return (chunks_from, chunks, floats) if floats else none
 
 
 def _recurrent_chunks(what: str, operands: tuple, below: int, chunks: int, floats: int, heads: int, device):
@@ -1850,8 +1892,7 @@ def gated_delta_rule(qkv: torch.Tensor, y: torch.Tensor, beta_off: int, decay_of
         raise KernelError("gated_delta_rule: decay columns inside y, one rate and one bias per head")
     seat_stride = _state_row(state, state_off, heads * dim * vdim, "gated_delta_rule")
     qs, seat, entries = _entries((entry_q_start, entry_seat), "gated_delta_rule")
-    below, chunks, floats = _recurrent_plan(lengths, DELTA_RULE_CHUNKS_FROM, entries, tokens, heads, dim, vdim, y.dtype,
-                                             "gated_delta_rule")
+    below, chunks, floats = _recurrent_plan(lengths, entries, tokens, heads, dim, vdim, y.dtype, True, channel_decay is not None)
     if qkv.data_ptr() % 16:         # (the chunks read 16 bytes at a time, the walk element by element)
         below, floats = 1 << 30, 0
     operands = (_dev(out, "out"), _dev(state, "state"), seat_stride, int(state_off), _dev(qkv, "qkv"), qkv.shape[1],
@@ -1893,8 +1934,7 @@ def gated_linear_attention(y: torch.Tensor, q_off: int, k_off: int, v_off: int, 
             raise KernelError("gated_linear_attention: q, k or v columns lie outside y")
     seat_stride = _state_row(state, state_off, heads * dim * vdim, "gated_linear_attention")
     qs, seat, entries = _entries((entry_q_start, entry_seat), "gated_linear_attention")
-    below, chunks, floats = _recurrent_plan(lengths, LINEAR_ATTENTION_CHUNKS_FROM, entries, tokens, heads, dim, vdim,
-                                             y.dtype, "gated_linear_attention")
+    below, chunks, floats = _recurrent_plan(lengths, entries, tokens, heads, dim, vdim, y.dtype, False, alpha is not None)
     operands = (_dev(out, "out"), _dev(state, "state"), seat_stride, int(state_off), _dev(y, "y"), dtype_code(y.dtype),
                 y.shape[1], int(q_off), int(k_off), int(v_off), _opt(alpha, "alpha"), alpha.shape[1] if alpha is not None else 0,
                 float(q_mul), _opt(head_decay, "head_decay"), 1 if activation == "silu" else 0, qs, seat,

@@ -47,9 +47,10 @@ def _names(defaults: Dict[str, str], given: Optional[Dict[str, str]], prefix: st
     return {key: prefix + name for key, name in names.items()}
 
 
-def _chunk_elements(mixer, chunks_from: int) -> int:
+def _chunk_elements(mixer, table, channel: bool) -> int:
     """Elements a token that the recurrence's kernels for long entries keep."""
-    return K.recurrent_chunk_elements(chunks_from, mixer.num_heads, mixer.head_dim, mixer.value_dim)
+    H, d, dv = mixer.num_heads, mixer.head_dim, mixer.value_dim
+    return K.recurrent_chunk_elements(K.recurrent_chunks_from(table, d, dv, channel), H, d, dv)
 
 
 @MIXERS.register("gated_linear_attention")
@@ -109,7 +110,7 @@ class GatedLinearAttention(ProjectedMixer):
         return self.num_heads * self.head_dim * self.value_dim
 
     def activation_elements(self) -> int:
-        return 3 * self.num_heads * self.head_dim + 5 * self.inner_width + self.hidden_size + _chunk_elements(self, K.LINEAR_ATTENTION_CHUNKS_FROM)
+        return 3 * self.num_heads * self.head_dim + 5 * self.inner_width + self.hidden_size + _chunk_elements(self, K.LINEAR_ATTENTION_CHUNKS_FROM, True)
 
     def forward_inner(self, y, col0, ctx: MixerContext, state_off, out, out_col0, mul) -> None:
         batch, T = ctx.batch, y.shape[0]
@@ -232,7 +233,7 @@ class GatedDeltaRule(ProjectedMixer):
         return self.num_heads * self.head_dim * self.value_dim + self.conv_channels * (self.conv_taps - 1)
 
     def activation_elements(self) -> int:
-        return 3 * self.conv_channels + 4 * self.inner_width + self.hidden_size + _chunk_elements(self, K.DELTA_RULE_CHUNKS_FROM)
+        return 3 * self.conv_channels + 4 * self.inner_width + self.hidden_size + _chunk_elements(self, K.DELTA_RULE_CHUNKS_FROM, self.channel_decay)
 
     def forward_inner(self, y, col0, ctx: MixerContext, state_off, out, out_col0, mul) -> None:
         batch, T = ctx.batch, y.shape[0]
@@ -315,7 +316,7 @@ class LightningAttention(ProjectedMixer):
         return self.num_heads * self.head_dim * self.value_dim
 
     def activation_elements(self) -> int:
-        return 2 * self.num_heads * self.head_dim + 5 * self.inner_width + self.hidden_size + _chunk_elements(self, K.LINEAR_ATTENTION_CHUNKS_FROM)
+        return 2 * self.num_heads * self.head_dim + 5 * self.inner_width + self.hidden_size + _chunk_elements(self, K.LINEAR_ATTENTION_CHUNKS_FROM, False)
 
     def forward_inner(self, y, col0, ctx: MixerContext, state_off, out, out_col0, mul) -> None:
         batch, T = ctx.batch, y.shape[0]

@@ -212,3 +212,25 @@ def test_portions_that_share_an_item():
             for mean in range(1, 5000, 83):
                 step = max([s for s in MEAN_KEYS_STEPS if s <= mean], default=0)
                 assert choose_portion_waves(n, mean, head_dim) == choose_portion_waves(n, step, head_dim)
+
+
+def test_recurrences_go_in_chunks_where_that_is_the_faster_way():
+    """One entry from the table's lines on; many prompts at once or a long one among many decoded tokens by what both ways cost."""
+    from kv_cache_optimization_for_llm_amd.ops import kernels as K
+
+    def chunks(lengths, heads, dim, vdim, delta, channel=False):
+        table = K.DELTA_RULE_CHUNKS_FROM if delta else K.LINEAR_ATTENTION_CHUNKS_FROM
+        return K.recurrent_chunks_pay(lengths, K.recurrent_chunks_from(table, dim, vdim, channel), heads, dim, vdim, delta, channel)
+    # (us, walk / chunks: 38/59, 75/67; 53/79, 99/87; 33/44, 149/53; 56/57, 85/61)
+    for shape, at in (((8, 128, 128, True), 176), ((8, 128, 128, True, True), 224), ((16, 64, 128, False, True), 224), ((16, 128, 128, False), 144)):
+        assert chunks([at], *shape) and not chunks([at - 1], *shape)
+        assert chunks([at, 1], *shape) and not chunks([at - 1, 1], *shape)
+    # (248/308, 123/184, 243/328; 186/144, 717/218; 338/432, 435/502, 404/322, 1,160/590)
+    for lengths, shape in (([512] + [1] * 256, (8, 128, 128, True)), ([176] + [1] * 128, (8, 128, 128, True)), ([512] + [1] * 256, (8, 128, 128, True, True)),
+                           ([200] * 40, (16, 64, 128, False, True)), ([225] * 40, (8, 128, 128, True, True))):
+        assert not chunks(lengths, *shape)
+    for lengths, shape in (([512] + [1] * 64, (8, 128, 128, True)), ([2048] + [1] * 64, (8, 128, 128, True)), ([256] * 32, (8, 128, 128, True)),
+                           ([200] * 40, (16, 128, 128, False)), ([2048], (32, 128, 128, True))):
+        assert chunks(lengths, *shape)
+    assert K.recurrent_chunks_from(K.DELTA_RULE_CHUNKS_FROM, 96, 128, False) == 0 == K.recurrent_chunks_from(K.DELTA_RULE_CHUNKS_FROM, 64, 40, True)
+    assert not K.recurrent_chunks_pay([], 64, 8, 128, 128, True, False)

@@ -368,9 +368,11 @@ def test_chunks_are_as_close_to_64_bits_as_the_walk(rule, decays, share, gpu):
 @pytest.mark.parametrize("bad", [float("nan"), float("inf"), -float("inf")])
 @pytest.mark.parametrize("where, at", [("q", 64), ("k", 69), ("v", 5), ("v", 199), ("decay", 140), ("beta", 70)])
 @pytest.mark.parametrize("rule", ["delta", "delta, channel", "linear"])
-def test_tokens_in_front_of_one_that_is_not_a_number_stay_as_they_are(rule, where, at, bad, gpu):
+def test_tokens_in_front_of_one_that_is_not_a_number_stay_as_they_are(rule, where, at, bad, gpu, monkeypatch):
     """An input of one token and head, in an entry that goes in chunks beside one that does not: every read-out and state is what
     the walk over the tokens gives, numbers or not; tokens in front and other heads are numbers."""
+    for name in ("DELTA_RULE_CHUNKS_FROM", "LINEAR_ATTENTION_CHUNKS_FROM"):
+        monkeypatch.setattr(K, name, 64)
     heads, dim, vdim, n = 3, 64, 32, 200
     g = torch.Generator().manual_seed(at)
     T, F32 = n + 7, torch.float32
@@ -432,10 +434,10 @@ def test_entries_in_chunks_among_many_that_are_not(gpu, monkeypatch):
         out, state = run(e, e + 1)
         assert torch.equal(out, whole[starts[e]:starts[e + 1]]) and torch.equal(state[0], states[e]), (e, lens[e])
     # two blocks of 64 tokens for 96, 97 and 128 tokens, three for 129, four for 200
-    assert K._recurrent_plan(lens, 96, len(lens), sum(lens), heads, dim, vdim, torch.bfloat16, "")[1] == 13
+    assert K._recurrent_plan(lens, len(lens), sum(lens), heads, dim, vdim, torch.bfloat16, False, True)[1] == 13
     most = K.recurrent_chunk_elements(96, heads, dim, vdim)
     for n in range(96, 700):
-        assert K._recurrent_plan([n], 96, 1, n, heads, dim, vdim, torch.bfloat16, "")[2] <= most * n
+        assert K._recurrent_plan([n], 1, n, heads, dim, vdim, torch.bfloat16, False, True)[2] <= most * n
 
 
 def test_a_seat_used_again_after_zeroing_forgets_and_a_far_token_is_remembered(gpu):
