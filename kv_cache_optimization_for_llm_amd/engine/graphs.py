@@ -230,7 +230,9 @@ class PortionGraphs:
     MAX_TOKENS = 4096          # tokens of one captured step
     MAX_LOGIT_ROWS = 64        # a graph keeps its logits: [rows, vocabulary] fp32
     MAX_SHAPES = 32            # captured shapes kept (least recently used goes first) ...
-    MAX_KEPT_TOKENS = 16384    # ... and the tokens of all of them: a graph keeps its step's activations
+    # ... and the tokens of all of them: a graph keeps its step's activations.  What its step takes beside those a token
+    # (workspaces, which go by contexts or by chunks) counts as the tokens that take as much.
+    MAX_KEPT_TOKENS = 16384
     MAX_SEEN = 4096
     # A capture costs some 6 ms of host time and a place among the shapes kept.  Under a load of random
     # prompt lengths most shapes come twice at most: captured at their second step, 500 captures in
@@ -268,6 +270,18 @@ class PortionGraphs:
             self.seen[key] = tuple(batch._items.keys())
             self.times[key] = 1
 
+    def make_room(self, lens: Sequence[int], bucket: int) -> Optional[int]:
+        """Drops the graphs used longest ago until a step of ``lens`` tokens with contexts up to ``bucket`` may be kept beside the
+        others; the tokens it counts as, or ``None`` when it is too large for that by itself."""
+        workspace = self.model.step_workspace_bytes(lens, bucket)
+        kept = int(sum(lens)) + -(-workspace // self.model.token_activation_bytes())
+        if kept > self.MAX_KEPT_TOKENS:
+            return None
+        while self.slots and (len(self.slots) >= self.MAX_SHAPES or
+                              sum(s.kept for s in self.slots.values()) + kept > self.MAX_KEPT_TOKENS):
+            self.slots.popitem(last=False)
+        return kept
+
     def run(self, key: tuple, tokens: np.ndarray, seats: np.ndarray, starts: np.ndarray,
             slot_maps: Sequence[np.ndarray]) -> Optional[torch.Tensor]:
         """Logits ``[wanted places, vocab]`` of the step, or ``None`` when the shape is new (the
@@ -281,11 +295,12 @@ class PortionGraphs:
             if self.times[key] < self.CAPTURE_AT:
                 return None
             lens, rows, bucket, _ = key
-            while self.slots and (len(self.slots) >= self.MAX_SHAPES or
-                                  sum(s.T for s in self.slots.values()) + sum(lens) > self.MAX_KEPT_TOKENS):
-                self.slots.popitem(last=False)
+            kept = self.make_room(lens, bucket)
+            if kept is None:
+                return None
             slot = self.slots[key] = _PortionSlot(lens, rows, bucket, variants, len(self.cache.groups),
                                                   self.device, self.feedback)
+            slot.kept = kept
         else:
             self.slots.move_to_end(key)
         slot.fill(tokens, seats, starts, slot_maps)

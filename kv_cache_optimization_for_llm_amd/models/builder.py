@@ -114,6 +114,7 @@ class Model:
         self.token_input_slot = 1 + max((slot for _, slot in self.calls), default=-1)
         self.embedding: Optional[torch.Tensor] = None
         self.head: Optional[Linear] = None
+        self.positions = int(spec.max_positions)
 
     # ---- what the cache manager has to provide
     @property
@@ -158,14 +159,24 @@ class Model:
     def step_activation_bytes(self, tokens: int, logit_rows: Optional[int] = None) -> int:
         """Upper estimate of the device memory one step of ``tokens`` tokens needs beside weights
         and cache: the residual stream and a branch output, twice the widest layer's intermediate
-        results (one layer's are freed while the next one's are made) and fp32 logits at
+        results (one layer's are freed while the next one's are made), a layer's workspace and fp32 logits at
         ``logit_rows`` places (default: every token).  The engine reserves this much once, and
         leaves it out when it sizes the cache pool from leftover memory."""
+        rows = int(tokens if logit_rows is None else logit_rows)
+        workspace = max((sum(part.workspace_limit(int(tokens), self.positions) for part in b.parts()) for b in self.blocks), default=0)
+        return int(tokens) * self.token_activation_bytes() + workspace + rows * 4 * self.spec.vocab_size
+
+    def token_activation_bytes(self) -> int:
+        """What of that goes by tokens."""
         elem = max(torch.empty((), dtype=self.dtype).element_size(), torch.empty((), dtype=self.stream_dtype).element_size())
         widest = max((sum(part.activation_elements() for part in b.parts()) for b in self.blocks), default=0)
         widest += max((op.activation_elements() for op in self.stream_ops), default=0)
-        rows = int(tokens if logit_rows is None else logit_rows)
-        return int(tokens) * ((2 + int(self.spec.streams)) * self.spec.hidden_size + 2 * widest) * elem + rows * 4 * self.spec.vocab_size
+        return ((2 + int(self.spec.streams)) * self.spec.hidden_size + 2 * widest) * elem
+
+    def step_workspace_bytes(self, lens, context: int) -> int:
+        """What one step with entries of ``lens`` tokens and contexts up to ``context`` takes beside them: its widest layer's
+        workspace, which the next layer's takes the place of."""
+        return max((sum(part.workspace_bytes(lens, context) for part in b.parts()) for b in self.blocks), default=0)
 
     def graph_safe(self) -> bool:
         """Whether every part may be captured into a HIP graph."""
@@ -181,6 +192,7 @@ class Model:
     def limit_positions(self, positions: int) -> None:
         """Tells every part that keeps something per position (tables of a position encoding) that
         no position at or past ``positions`` will be asked for."""
+        self.positions = int(positions)
         for b in self.blocks:
             for part in (*b.parts(), getattr(b.mixer, "position", None)):
                 limit = getattr(part, "limit_positions", None)

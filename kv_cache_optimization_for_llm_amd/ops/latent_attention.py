@@ -52,14 +52,29 @@ EXPAND_CONTEXTS = 16
 EXPAND_BYTES = 512 << 20
 
 
+def expanded_bytes(shortest: int, entries: int, max_context: int, heads: int, dim: int, rot: int, vdim: int, rank: int, window: int,
+                   dtype) -> int:
+    """Bytes of expanded keys and values over which a step's prompt portions attend; 0: they attend over the cached rows.  A
+    captured step knows its contexts to the power of two above them (at least 256): every step goes by that, so that it
+    asks for the same work items with and without."""
+    context = 1 << max(8, (max_context - 1).bit_length())
+    size = entries * context * (heads * (dim + vdim) + rot) * 2
+    return size if (dtype == torch.bfloat16 and window <= 0 and heads <= 1024 and shortest >= EXPAND_FROM
+                    and context <= EXPAND_CONTEXTS * shortest and size <= EXPAND_BYTES
+                    and K.latent_prompt_supported(dim, rot, vdim, rank)) else 0
+
+
+def expanded_bytes_limit(tokens: int, positions: int, heads: int, dim: int, rot: int, vdim: int) -> int:
+    """The most any step of up to ``tokens`` tokens and contexts of up to ``positions`` expands."""
+    if tokens < EXPAND_FROM:
+        return 0
+    rows = min(EXPAND_CONTEXTS * tokens, (tokens // EXPAND_FROM) << max(8, (positions - 1).bit_length()))
+    return min(EXPAND_BYTES, rows * (heads * (dim + vdim) + rot) * 2)
+
+
 def expands(batch, heads: int, dim: int, rot: int, vdim: int, rank: int, window: int, dtype) -> bool:
-    """Whether a step's prompt portions attend over expanded keys and values.  A captured step knows its contexts to the power
-    of two above them (at least 256): every step goes by that, so that it asks for the same work items with and without."""
-    context = 1 << max(8, (batch.max_context - 1).bit_length())
-    return (dtype == torch.bfloat16 and window <= 0 and heads <= 1024 and batch.min_q_len >= EXPAND_FROM
-            and context <= EXPAND_CONTEXTS * batch.min_q_len
-            and batch.num_entries * context * (heads * (dim + vdim) + rot) * 2 <= EXPAND_BYTES
-            and K.latent_prompt_supported(dim, rot, vdim, rank))
+    """Whether a step's prompt portions attend over expanded keys and values."""
+    return expanded_bytes(batch.min_q_len, batch.num_entries, batch.max_context, heads, dim, rot, vdim, rank, window, dtype) > 0
 
 
 def latent_attention(q_lat: torch.Tensor, out: torch.Tensor, kv, batch, scale: float, window: int = 0,

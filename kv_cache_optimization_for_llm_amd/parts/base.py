@@ -259,6 +259,15 @@ class Part:
         sizing memory; 0 when negligible)."""
         return 0
 
+    def workspace_bytes(self, lens, context: int) -> int:
+        """Bytes this part takes beside them for a step whose entries have ``lens`` tokens and end at positions up to
+        ``context``."""
+        return 0
+
+    def workspace_limit(self, tokens: int, positions: int) -> int:
+        """The most that can be for steps of up to ``tokens`` tokens and requests of up to ``positions`` positions."""
+        return 0
+
 
 class Norm(Part):
     def forward(self, x: torch.Tensor, out: Optional[torch.Tensor] = None,

@@ -92,6 +92,12 @@ class SideBySide(Mixer):
     def activation_elements(self) -> int:
         return sum(c.activation_elements() for c in self.children)
 
+    def workspace_bytes(self, lens, context: int) -> int:
+        return sum(c.workspace_bytes(lens, context) for c in self.children)
+
+    def workspace_limit(self, tokens: int, positions: int) -> int:
+        return sum(c.workspace_limit(tokens, positions) for c in self.children)
+
     def forward(self, x: torch.Tensor, ctx: MixerContext) -> torch.Tensor:
         y = self.w_in(x)
         ctx.x = x

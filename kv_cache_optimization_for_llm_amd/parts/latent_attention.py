@@ -131,8 +131,18 @@ class LatentAttention(Mixer):
     def activation_elements(self) -> int:
         H = self.num_heads
         return (self.proj.out_features if self.proj is not None else 0) + H * (self.key_dim + self.rank + self.value_dim) \
-            + H * (self.head_dim + self.value_dim) + self.rot_dim \
             + (self.q_rank + H * (self.head_dim + self.rot_dim) if self.q_rank else 0) + self.hidden_size
+
+    def workspace_bytes(self, lens, context: int) -> int:
+        if self.up_kv is None:
+            return 0
+        return lat_ops.expanded_bytes(min(lens), len(lens), context, self.num_heads, self.head_dim, self.rot_dim, self.value_dim,
+                                      self.rank, self.window, self.up_kv.dtype)
+
+    def workspace_limit(self, tokens: int, positions: int) -> int:
+        if self.up_kv is None or self.window > 0:
+            return 0
+        return lat_ops.expanded_bytes_limit(tokens, positions, self.num_heads, self.head_dim, self.rot_dim, self.value_dim)
 
     def forward(self, x, ctx: MixerContext, tail=None):
         if isinstance(x, NormedRows):

@@ -47,14 +47,27 @@ def _names(defaults: Dict[str, str], given: Optional[Dict[str, str]], prefix: st
     return {key: prefix + name for key, name in names.items()}
 
 
-def _chunk_elements(mixer, table, channel: bool) -> int:
-    """Elements a token that the recurrence's kernels for long entries keep."""
-    H, d, dv = mixer.num_heads, mixer.head_dim, mixer.value_dim
-    return K.recurrent_chunk_elements(K.recurrent_chunks_from(table, d, dv, channel), H, d, dv)
+class _InChunks:
+    """What a mixer whose long entries go in chunks keeps for them."""
+
+    delta_rule = channel_decay = False
+
+    def workspace_bytes(self, lens, context: int) -> int:
+        _, chunks, floats = K._recurrent_plan(lens, len(lens), int(sum(lens)), self.num_heads, self.head_dim, self.value_dim,
+                                              self.input_weight().dtype, self.delta_rule, self.channel_decay)
+        return 4 * (floats + chunks * self.num_heads)
+
+    def workspace_limit(self, tokens: int, positions: int) -> int:
+        if self.input_weight().dtype != torch.bfloat16:
+            return 0
+        table = K.DELTA_RULE_CHUNKS_FROM if self.delta_rule else K.LINEAR_ATTENTION_CHUNKS_FROM
+        H, d, dv = self.num_heads, self.head_dim, self.value_dim
+        return 4 * tokens * K.recurrent_chunk_elements(K.recurrent_chunks_from(table, d, dv, self.channel_decay), H, d, dv)
 
 
 @MIXERS.register("gated_linear_attention")
-class GatedLinearAttention(ProjectedMixer):
+class GatedLinearAttention(_InChunks, ProjectedMixer):
+    channel_decay = True
     graph_safe = True
 
     def __init__(self, prefix: str, *, hidden_size: int, num_heads: int, head_dim: int, value_dim: int, tau: float,
@@ -110,7 +123,7 @@ class GatedLinearAttention(ProjectedMixer):
         return self.num_heads * self.head_dim * self.value_dim
 
     def activation_elements(self) -> int:
-        return 3 * self.num_heads * self.head_dim + 5 * self.inner_width + self.hidden_size + _chunk_elements(self, K.LINEAR_ATTENTION_CHUNKS_FROM, True)
+        return 3 * self.num_heads * self.head_dim + 5 * self.inner_width + self.hidden_size
 
     def forward_inner(self, y, col0, ctx: MixerContext, state_off, out, out_col0, mul) -> None:
         batch, T = ctx.batch, y.shape[0]
@@ -127,7 +140,8 @@ class GatedLinearAttention(ProjectedMixer):
 
 
 @MIXERS.register("gated_delta_rule")
-class GatedDeltaRule(ProjectedMixer):
+class GatedDeltaRule(_InChunks, ProjectedMixer):
+    delta_rule = True
     graph_safe = True
 
     def __init__(self, prefix: str, *, hidden_size: int, num_heads: int, num_kv_heads: int, head_dim: int,
@@ -233,7 +247,7 @@ class GatedDeltaRule(ProjectedMixer):
         return self.num_heads * self.head_dim * self.value_dim + self.conv_channels * (self.conv_taps - 1)
 
     def activation_elements(self) -> int:
-        return 3 * self.conv_channels + 4 * self.inner_width + self.hidden_size + _chunk_elements(self, K.DELTA_RULE_CHUNKS_FROM, self.channel_decay)
+        return 3 * self.conv_channels + 4 * self.inner_width + self.hidden_size
 
     def forward_inner(self, y, col0, ctx: MixerContext, state_off, out, out_col0, mul) -> None:
         batch, T = ctx.batch, y.shape[0]
@@ -266,7 +280,7 @@ class GatedDeltaRule(ProjectedMixer):
 
 
 @MIXERS.register("lightning_attention")
-class LightningAttention(ProjectedMixer):
+class LightningAttention(_InChunks, ProjectedMixer):
     """Linear attention with one fixed decay a head: ``S_t = decay_h S_(t-1) + k_t v_t^T``, ``o_t = S_t^T
     (query_scale q_t)`` where q, k and v are the ``activation`` (silu) of their projections.  The heads'
     read-outs are normed TOGETHER (one RMS norm over ``heads * value_dim`` elements with a weight of
@@ -316,7 +330,7 @@ class LightningAttention(ProjectedMixer):
         return self.num_heads * self.head_dim * self.value_dim
 
     def activation_elements(self) -> int:
-        return 2 * self.num_heads * self.head_dim + 5 * self.inner_width + self.hidden_size + _chunk_elements(self, K.LINEAR_ATTENTION_CHUNKS_FROM, False)
+        return 2 * self.num_heads * self.head_dim + 5 * self.inner_width + self.hidden_size
 
     def forward_inner(self, y, col0, ctx: MixerContext, state_off, out, out_col0, mul) -> None:
         batch, T = ctx.batch, y.shape[0]

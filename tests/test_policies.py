@@ -234,3 +234,38 @@ def test_recurrences_go_in_chunks_where_that_is_the_faster_way():
         assert chunks(lengths, *shape)
     assert K.recurrent_chunks_from(K.DELTA_RULE_CHUNKS_FROM, 96, 128, False) == 0 == K.recurrent_chunks_from(K.DELTA_RULE_CHUNKS_FROM, 64, 40, True)
     assert not K.recurrent_chunks_pay([], 64, 8, 128, 128, True, False)
+
+
+def test_a_steps_workspace_is_reserved_and_counts_against_the_graphs_kept(monkeypatch):
+    """Keys and values expanded per head go by entries x contexts, not by tokens: the engine's estimate covers every step that
+    expands, and a captured step counts as the tokens whose activations take as much."""
+    from collections import OrderedDict
+    from types import SimpleNamespace
+
+    import torch
+    from kv_cache_optimization_for_llm_amd.engine.graphs import PortionGraphs
+    from kv_cache_optimization_for_llm_amd.ops import kernels as K
+    from kv_cache_optimization_for_llm_amd.ops import latent_attention as lat
+    monkeypatch.setattr(K, "latent_prompt_supported", lambda *sizes: True)
+    for heads, tokens, positions in ((16, 512, 8192), (16, 8192, 8192), (16, 100, 3000), (128, 2048, 40000), (64, 4096, 700), (16, 63, 8192)):
+        limit, seen = lat.expanded_bytes_limit(tokens, positions, heads, 128, 64, 128), 0
+        for entries in (1, 2, 3, 7, 20, 64, 128):
+            for shortest in (1, 63, 64, 100, 255, 256, 512, tokens // entries):
+                for context in (shortest, 256, 300, 1024, 4097, 16 * shortest, positions):
+                    if entries * shortest <= tokens and shortest <= context <= positions:
+                        seen = max(seen, lat.expanded_bytes(shortest, entries, context, heads, 128, 64, 128, 512, 0, torch.bfloat16))
+        assert (seen > 0) == (tokens >= 64) and seen <= limit <= lat.EXPAND_BYTES
+    # 64 KB of activations a token; a portion of 512 tokens expands its context of 8,192 positions, 8,320 bytes each: 1,040 tokens more
+    model = SimpleNamespace(token_activation_bytes=lambda: 65536, step_workspace_bytes=lambda lens, context:
+                            lat.expanded_bytes(min(lens), len(lens), context, 16, 128, 64, 128, 512, 0, torch.bfloat16))
+    graphs = PortionGraphs(model, None, "cpu")
+    assert isinstance(graphs.slots, OrderedDict)
+    for i in range(40):
+        kept = graphs.make_room((512,), 8192)
+        assert kept == 512 + 1040
+        graphs.slots[i] = SimpleNamespace(kept=kept)
+        assert sum(s.kept for s in graphs.slots.values()) <= graphs.MAX_KEPT_TOKENS
+    assert list(graphs.slots) == list(range(30, 40))
+    assert graphs.make_room((512,) + (1,) * 8, 8192) == 520 and len(graphs.slots) == 10        # (decoded tokens beside it: nothing expanded)
+    model.step_workspace_bytes = lambda lens, context: 17000 * 65536
+    assert graphs.make_room((512,), 8192) is None and len(graphs.slots) == 10
