@@ -9,22 +9,26 @@
 // mask row are penalised first (l > 0 ? l / p : l * p).
 //
 // How: two launches, and the logits are read once.
-//   1. sample_scan_kernel, one workgroup per (chunk of a row, row): the tokens, up to 4,096 at a time, are loaded
-//      into registers (16 bytes a lane where rows are aligned for it), the workgroup's best (value, id) is found,
-//      then the sum of exp((l - maximum) / T); one record per chunk.
-//   2. sample_pick_kernel, one workgroup per row: joins the chunk records (row maximum, argmax),
+//   1. sample_scan_kernel, one wavefront per (chunk of a row, row): the tokens, up to 1,280 at a time, are loaded
+//      into registers, the best (value, id) is found, then the sum of exp((l - maximum) / T); one record per chunk.
+//   2. sample_pick_kernel, one wavefront per row: joins the chunk records (row maximum, argmax),
 //      rescales the chunk sums to the row maximum, finds the chunk that holds the target by a
 //      wavefront prefix scan and reads that one chunk again, 64 neighbouring tokens a load: the 64 that
 //      hold the target are found by their sums, the token by a prefix scan over the lanes.  The chosen
 //      token is also marked in the request's mask row when there is one.
+// The order of all sums follows from the vocabulary and the number of chunks alone: a row draws the same token alone
+// and among others.
 //
-// 64 rows of 128,256 logits (33 MB), half of them at a temperature: both kernels 14 us in a graph.  With 128 workgroups
-// a row whose threads took four tokens each, one by one, and a single wavefront that walked its spans of the chunk: 30.
+// Both kernels in a graph, 128 chunks of a row of 128,256 logits, us, greedy / at a temperature: 1 row 5.5 / 10.9, 16 rows 6.5 /
+// 12.4, 64 rows (33 MB) 8.6 / 17.3, 128 rows 14.8 / 24.0.  With 128 workgroups a row whose threads took four tokens each, one by
+// one, and a single wavefront that walked its spans of the chunk: 64 rows 13.8 / 35.2.
 #include "common.h"
 #include <math.h>
 
-#define SAMPLE_THREADS 256
-#define SCAN_TOKENS 4096         // tokens a workgroup holds in registers at a time
+#define SCAN_WAVES 4             // chunks a workgroup of the first kernel takes, a wavefront each, where there are enough
+// Tokens a lane holds in registers at a time: chunks of up to 256 tokens (a small vocabulary's) and others, 1,280 a turn.
+#define HELD_FEW 4
+#define HELD_MANY 20
 #define SAMPLE_MAX_CHUNKS 1024
 #define KVA_NO_TOKEN (-1)       // what a row gets whose logits name no token
 
@@ -121,18 +125,18 @@ struct ChunkRecord {
     float sum;
 };
 
-// grid (chunks, rows).  VEC: rows and chunks start at multiples of 16 bytes.
-template <bool VEC>
-__global__ void __launch_bounds__(SAMPLE_THREADS)
-sample_scan_kernel(const float *__restrict__ logits, int vocab, int chunk_tokens,
+typedef float sample_f32x4 __attribute__((ext_vector_type(4), aligned(4)));     // (rows may start at any multiple of 4 bytes)
+
+// grid (chunks / wavefronts of a workgroup, rows).  VEC: rows and chunks start at, and end before, multiples of 16 bytes.
+template <int HELD, bool VEC>
+__global__ void __launch_bounds__(KVA_WAVE * SCAN_WAVES)
+sample_scan_kernel(const float *__restrict__ logits, int vocab, int chunk_tokens, int chunks,
                    const unsigned char *__restrict__ penalty_mask, const int *__restrict__ row_seat,
                    float penalty, const float *__restrict__ inv_temperature,
                    ChunkRecord *__restrict__ records) {
-    constexpr int WAVES = SAMPLE_THREADS / KVA_WAVE;
-    __shared__ Best wave_b[2][WAVES];
-    __shared__ float wave_s[2][WAVES];
-    const int row = blockIdx.y, chunk = blockIdx.x, chunks = gridDim.x;
-    const int lane = threadIdx.x % KVA_WAVE, wave = threadIdx.x / KVA_WAVE;
+    const int row = blockIdx.y, lane = threadIdx.x % KVA_WAVE;
+    const int chunk = __builtin_amdgcn_readfirstlane(blockIdx.x * (blockDim.x / KVA_WAVE) + threadIdx.x / KVA_WAVE);
+    if (chunk >= chunks) return;
     const int begin = chunk * chunk_tokens;
     const int end = min(begin + chunk_tokens, vocab);
     const float *rl = logits + (size_t)row * vocab;
@@ -141,14 +145,17 @@ sample_scan_kernel(const float *__restrict__ logits, int vocab, int chunk_tokens
     const bool sampled = inv_t > 0.f;
     Best b{-INFINITY, vocab};
     Online o{-INFINITY, 0.f};
-    for (int base = begin, turn = 0; base < end; base += SCAN_TOKENS, turn ^= 1) {
-        // thread t's tokens: 4 t .. 4 t + 3 of every 1,024 (their loads side by side); past the end: -inf, no weight
-        float l[SCAN_TOKENS / SAMPLE_THREADS];
+    for (int base = begin; base < end; base += HELD * KVA_WAVE) {
+        // lane t's tokens: 4 t .. 4 t + 3 of every 256 (their loads side by side); past the end: -inf, no weight
+        float l[HELD];
 #pragma unroll
-        for (int j = 0; j < SCAN_TOKENS / SAMPLE_THREADS; j += 4) {
-            const int t = base + j * SAMPLE_THREADS + 4 * threadIdx.x;
+        for (int j = 0; j < HELD; j += 4) {
+            const int t = base + j * KVA_WAVE + 4 * lane;
             if (VEC) {
                 const float4 v = t < end ? *reinterpret_cast<const float4 *>(rl + t) : make_float4(-INFINITY, -INFINITY, -INFINITY, -INFINITY);
+                l[j] = v.x; l[j + 1] = v.y; l[j + 2] = v.z; l[j + 3] = v.w;
+            } else if (t + 3 < end) {
+                const sample_f32x4 v = *reinterpret_cast<const sample_f32x4 *>(rl + t);
                 l[j] = v.x; l[j + 1] = v.y; l[j + 2] = v.z; l[j + 3] = v.w;
             } else {
 #pragma unroll
@@ -157,35 +164,25 @@ sample_scan_kernel(const float *__restrict__ logits, int vocab, int chunk_tokens
         }
         Best mine{-INFINITY, vocab};
 #pragma unroll
-        for (int j = 0; j < SCAN_TOKENS / SAMPLE_THREADS; ++j) {
-            const int t = base + j / 4 * 4 * SAMPLE_THREADS + 4 * threadIdx.x + j % 4;
+        for (int j = 0; j < HELD; ++j) {
+            const int t = base + j / 4 * 4 * KVA_WAVE + 4 * lane + j % 4;
             if (mk != nullptr && t < end) l[j] = penalised(l[j], mk, t, penalty);
-            if (l[j] > mine.value) mine = Best{l[j], t};        // (a thread's tokens come in ascending order: the first of equal ones)
+            if (l[j] > mine.value) mine = Best{l[j], t};        // (a lane's tokens come in ascending order: the first of equal ones)
         }
         mine = wave_best(mine);
-        if (lane == 0) wave_b[turn][wave] = mine;
-        __syncthreads();
-#pragma unroll
-        for (int w = 0; w < WAVES; ++w) mine = better(mine, wave_b[turn][w]);
         b = better(b, mine);
-        if (!sampled) continue;                                 // (the row's: the whole workgroup)
+        if (!sampled || !(mine.value > -INFINITY)) continue;    // (the row's; the same in all lanes)
         float s = 0.f;
-        if (mine.value > -INFINITY)
 #pragma unroll
-            for (int j = 0; j < SCAN_TOKENS / SAMPLE_THREADS; ++j) s += token_weight(l[j], mine.value, inv_t);
-        s = wave_sum_valu(s);
-        if (lane == 0) wave_s[turn][wave] = s;
-        __syncthreads();
-        s = 0.f;
-#pragma unroll
-        for (int w = 0; w < WAVES; ++w) s += wave_s[turn][w];
-        o.join(Online{mine.value, s}, inv_t);
+        for (int j = 0; j < HELD; ++j) s += token_weight(l[j], mine.value, inv_t);
+        o.join(Online{mine.value, wave_sum_valu(s)}, inv_t);
     }
-    if (threadIdx.x == 0) records[(size_t)row * chunks + chunk] = ChunkRecord{b.value, b.index, o.m, o.s};
+    if (lane == 0) records[(size_t)row * chunks + chunk] = ChunkRecord{b.value, b.index, o.m, o.s};
 }
 
-// grid (rows).  Every wavefront joins the records by itself (they agree); the chunk's tokens are shared out.
-__global__ void __launch_bounds__(SAMPLE_THREADS)
+// grid (rows), one wavefront
+template <int HELD>
+__global__ void __launch_bounds__(KVA_WAVE)
 sample_pick_kernel(const float *__restrict__ logits, int vocab, int chunk_tokens, int chunks,
                    const unsigned char *penalty_mask, const int *__restrict__ row_seat,
                    float penalty, const float *__restrict__ inv_temperature,
@@ -193,10 +190,7 @@ sample_pick_kernel(const float *__restrict__ logits, int vocab, int chunk_tokens
                    const unsigned int *__restrict__ rng_key, const unsigned int *__restrict__ rng_step,
                    unsigned char *mark_mask /* may be penalty_mask */, const int *__restrict__ mark_seat,
                    int *__restrict__ out_tokens, int *__restrict__ host_tokens) {
-    constexpr int WAVES = SAMPLE_THREADS / KVA_WAVE, GROUPS = SCAN_TOKENS / SAMPLE_THREADS;
-    __shared__ float wave_s[2][WAVES];
-    __shared__ int found_by[2][WAVES];
-    const int row = blockIdx.x, lane = threadIdx.x % KVA_WAVE, wave = __builtin_amdgcn_readfirstlane(threadIdx.x / KVA_WAVE);
+    const int row = blockIdx.x, lane = threadIdx.x;
     const ChunkRecord *rec = records + (size_t)row * chunks;
     // this lane's chunks: a contiguous run, so that lane order is chunk order
     const int per_lane = (chunks + KVA_WAVE - 1) / KVA_WAVE;
@@ -254,65 +248,41 @@ sample_pick_kernel(const float *__restrict__ logits, int vocab, int chunk_tokens
             chunk = __shfl(chunk, owner, KVA_WAVE);
             before = __shfl(before, owner, KVA_WAVE);
         }
-        // inside the chunk, 4,096 tokens at a time, a quarter a wavefront, lane = token: of 64 neighbouring tokens the
-        // sum first, the place inside only where the target is
+        // inside the chunk, 1,280 tokens at a time, lane = token: of 64 neighbouring tokens the sum first, the place
+        // inside only where the target is
         const int begin = chunk * chunk_tokens, end = min(begin + chunk_tokens, vocab);
         const float *rl = logits + (size_t)row * vocab;
         const unsigned char *mk = mask_row(penalty_mask, row_seat, row, vocab);
         float inner = target - before;
         token = end - 1;                     // past every reach (rounding): the chunk's last token
-        for (int base = begin, turn = 0; base < end; base += SCAN_TOKENS, turn ^= 1) {
-            float w[GROUPS];
-            const int first = base + wave * (SCAN_TOKENS / WAVES) + lane;
+        bool done = false;
+        for (int base = begin; base < end && !done; base += HELD * KVA_WAVE) {
+            float w[HELD], sums[HELD];
+            const int first = base + lane;
 #pragma unroll
-            for (int i = 0; i < GROUPS; ++i) w[i] = first + KVA_WAVE * i < end ? rl[first + KVA_WAVE * i] : -INFINITY;
-            float all = 0.f;
+            for (int i = 0; i < HELD; ++i) w[i] = first + KVA_WAVE * i < end ? rl[first + KVA_WAVE * i] : -INFINITY;
 #pragma unroll
-            for (int i = 0; i < GROUPS; ++i) {
+            for (int i = 0; i < HELD; ++i) {
                 if (mk != nullptr && first + KVA_WAVE * i < end) w[i] = penalised(w[i], mk, first + KVA_WAVE * i, penalty);
                 w[i] = token_weight(w[i], top, inv_t);
             }
-            float sums[GROUPS];
 #pragma unroll
-            for (int i = 0; i < GROUPS; ++i) {
-                sums[i] = wave_sum_valu(w[i]);
-                all += sums[i];
-            }
-            if (lane == 0) wave_s[turn][wave] = all;
-            __syncthreads();
-            float here = inner;
-            for (int v = 0; v < wave; ++v) here -= wave_s[turn][v];
-            int found = -1;
-            if (here < all && (wave == 0 || here >= 0.f)) {       // (an earlier wavefront's share holds it: negative)
-                float run = 0.f;
-                bool done = false;
+            for (int i = 0; i < HELD; ++i) sums[i] = wave_sum_valu(w[i]);
+            float run = 0.f;
 #pragma unroll
-                for (int i = 0; i < GROUPS; ++i) {
-                    if (!done && here < run + sums[i]) {
-                        const float reach = run + wave_prefix_sum(w[i]);
-                        const int at = first_lane(here < reach);
-                        // (rounding between the sum and the scan: the last of the 64 that weighs anything)
-                        const unsigned long long weighs = __ballot(w[i] > 0.f);
-                        found = first - lane + KVA_WAVE * i + (at >= 0 ? at : weighs ? 63 - __clzll((long long)weighs) : 0);
-                        done = true;
-                    }
-                    run += sums[i];
+            for (int i = 0; i < HELD; ++i) {
+                if (!done && inner < run + sums[i]) {
+                    const int at = first_lane(inner < run + wave_prefix_sum(w[i]));
+                    // (rounding between the sum and the scan: the last of the 64 that weighs anything)
+                    const unsigned long long weighs = __ballot(w[i] > 0.f);
+                    token = base + KVA_WAVE * i + (at >= 0 ? at : weighs ? 63 - __clzll((long long)weighs) : 0);
+                    done = true;
                 }
+                run += sums[i];
             }
-            if (lane == 0) found_by[turn][wave] = found;
-            __syncthreads();
-            int hit = -1;
-#pragma unroll
-            for (int v = WAVES - 1; v >= 0; --v) hit = found_by[turn][v] >= 0 ? found_by[turn][v] : hit;
-            if (hit >= 0) {
-                token = hit;
-                break;
-            }
-#pragma unroll
-            for (int v = 0; v < WAVES; ++v) inner -= wave_s[turn][v];
+            inner -= run;
         }
     }
-    if (wave != 0) return;
     // A row without a finite best logit (all NaN, all -inf) has no token to name, greedy or sampled,
     // and neither has a temperature row whose weights do not add up to a positive finite total.
     // Such a row gets KVA_NO_TOKEN (-1): the host sees it and ends the request with an error, and
@@ -384,12 +354,16 @@ extern "C" int kva_sample(int *out_tokens, const float *logits, int rows, int vo
     if (rows == 0) return KVA_OK;
     // chunks start at multiples of four tokens (the last ones may be empty)
     const int chunk_tokens = ((vocab + chunks - 1) / chunks + 3) / 4 * 4;
-    const bool vec = vocab % 4 == 0 && (uintptr_t)logits % 16 == 0;
     ChunkRecord *records = (ChunkRecord *)workspace;
     const float *inv_t = any_sampled ? inv_temperature : nullptr;
-    hipLaunchKernelGGL(vec ? sample_scan_kernel<true> : sample_scan_kernel<false>, dim3(chunks, rows), dim3(SAMPLE_THREADS), 0, stream, logits,
-                       vocab, chunk_tokens, penalty_mask, row_seat, penalty, inv_t, records);
-    hipLaunchKernelGGL(sample_pick_kernel, dim3(rows), dim3(SAMPLE_THREADS), 0, stream, logits, vocab,
+    const int waves = (long long)rows * chunks >= 2048 ? SCAN_WAVES : 1;      // (fewer: a compute unit each)
+    const dim3 grid((chunks + waves - 1) / waves, rows), block(KVA_WAVE * waves);
+    const bool few = chunk_tokens <= HELD_FEW * KVA_WAVE;
+    const bool vec = vocab % 4 == 0 && (uintptr_t)logits % 16 == 0;
+    const auto scan = few ? (vec ? sample_scan_kernel<HELD_FEW, true> : sample_scan_kernel<HELD_FEW, false>)
+                          : (vec ? sample_scan_kernel<HELD_MANY, true> : sample_scan_kernel<HELD_MANY, false>);
+    hipLaunchKernelGGL(scan, grid, block, 0, stream, logits, vocab, chunk_tokens, chunks, penalty_mask, row_seat, penalty, inv_t, records);
+    hipLaunchKernelGGL(few ? sample_pick_kernel<HELD_FEW> : sample_pick_kernel<HELD_MANY>, dim3(rows), dim3(KVA_WAVE), 0, stream, logits, vocab,
                        chunk_tokens, chunks, penalty_mask, row_seat, penalty, inv_t, records, seed, rng_key,
                        rng_step, mark_mask, mark_seat, out_tokens, host_mapped);
     KVA_CHECK_LAUNCH("sample");

@@ -96,12 +96,6 @@ class Sampler:
         self._args_views: dict = {}
         self._args_next = 0
 
-    def chunks_for(self, rows: int) -> int:
-        """Workgroups a row of the first kernel: about eight a compute unit over all rows, never more tokens each than
-        it holds in registers (both kernels over 64 rows of 128,256: 14.2 us with 32 workgroups a row, 17 with 16 or 64, 24
-        with 128)."""
-        return min(self.chunks, max(-(-self.vocab_size // 4096), 2048 // max(rows, 1)))
-
     def _row_arguments(self, n: int):
         """(a staging array [5, n] of int32 in pinned memory to fill, the same as uint32 and as float, the device arrays
         its rows go to by :func:`ops.kernels.upload`, what to tell when it has been sent) for the next sampling of n
@@ -190,7 +184,7 @@ class Sampler:
             staging.sent = event
             K.upload(staging.pinned, self._args_dev)
         try:
-            K.sample(logits, out, chunks=self.chunks_for(n), inv_temperature=inv_t, seed=self.seed, rng_key=key,
+            K.sample(logits, out, chunks=self.chunks, inv_temperature=inv_t, seed=self.seed, rng_key=key,
                      rng_step=step, penalty_mask=self.mask if use_mask else None, row_seat=seat_t,
                      penalty=self.penalty, mark_mask=self.mask if mark_seat is not None else None,
                      mark_seat=mark_seat, host_tokens=host if self._kernel_writes_host else None)

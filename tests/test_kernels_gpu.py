@@ -906,6 +906,27 @@ def test_sampler_at_the_edges_of_what_a_workgroup_holds(vocab, chunks, gpu):
             assert w[got] > 0 and (cdf[got - 1] if got else 0.0) - 1e-5 <= u <= cdf[got] + 1e-5, r
 
 
+@pytest.mark.parametrize("chunks", [1, 2])
+@pytest.mark.parametrize("vocab", [1279, 1280, 1281, 2560, 2561])
+def test_sampler_at_the_edges_of_what_a_wavefront_holds(vocab, chunks, gpu):
+    test_sampler_at_the_edges_of_what_a_workgroup_holds(vocab, chunks, gpu)
+
+
+@pytest.mark.parametrize("vocab", [128256, 32003, 160001])
+def test_a_row_draws_the_same_token_alone_and_among_others(vocab, gpu):
+    """Flat rows: a token's share of the cumulative weights is a hundred roundings wide, so that of some hundred draws several lie
+    where another order of the sums would choose the neighbour."""
+    from kv_cache_optimization_for_llm_amd.sampling.sampler import Sampler, SampleRow
+    rows = 100
+    lg = (torch.rand(rows, vocab, generator=torch.Generator().manual_seed(vocab)) * 1e-3).to(gpu)
+    sampler = Sampler(vocab, rows, gpu, seed=5)
+    for step in range(4):
+        which = [SampleRow(r, 0.8, rng_key=8 * r, rng_step=step) for r in range(rows)]
+        alone = [int(sampler.sample(lg[r:r + 1], which[r:r + 1])[0]) for r in range(rows)]
+        for n in (2, 17, 33, 64, rows):
+            assert [int(t) for t in sampler.sample(lg[:n].contiguous(), which[:n])] == alone[:n], n
+
+
 def test_sampler_distribution_and_boundaries(gpu):
     """python/sampling_reference.py:110-134: top-8 frequencies within 5 % over 40 000 draws."""
     vocab = 5000
