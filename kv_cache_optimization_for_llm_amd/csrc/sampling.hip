@@ -317,14 +317,6 @@ extern "C" int kva_host_memory_is_mapped(void *host) {
     return dev != nullptr ? 1 : 0;
 }
 
-// Queues a copy from pinned host memory.
-extern "C" int kva_upload(void *device, const void *host, long long bytes, hipStream_t stream) {
-    KVA_REQUIRE(device && host && bytes >= 0, "upload: missing operand");
-    const hipError_t e = hipMemcpyAsync(device, host, (size_t)bytes, hipMemcpyHostToDevice, stream);
-    KVA_REQUIRE(e == hipSuccess, "upload: %s", hipGetErrorString(e));
-    return KVA_OK;
-}
-
 // host_tokens (optional): pinned host memory (hipHostMalloc, torch's pin_memory) with room for a token
 // per row; the kernel that chooses the tokens writes them there as well, which saves the copy
 // that would otherwise follow it on the stream.  Refused unless the runtime says the memory is

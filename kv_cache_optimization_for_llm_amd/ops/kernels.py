@@ -1075,15 +1075,6 @@ def host_memory_is_mapped(t: torch.Tensor) -> bool:
     return bool(hip_lib().kva_host_memory_is_mapped(ctypes.c_void_p(t.data_ptr())))
 
 
-def upload(host: torch.Tensor, device: torch.Tensor) -> None:
-    """Queues the copy of a pinned host tensor into a device tensor of its shape and type on the current stream; the
-    host tensor must stay as it is until the stream has passed it."""
-    if host.is_cuda or not host.is_contiguous() or host.shape != device.shape or host.dtype != device.dtype:
-        raise KernelError("upload: a pinned host tensor of the device tensor's shape and type")
-    check(hip_lib().kva_upload(_dev(device, "device"), ctypes.c_void_p(host.data_ptr()), host.numel() * host.element_size(), _stream()),
-          "upload")
-
-
 def sample(logits: torch.Tensor, out_tokens: torch.Tensor, *, chunks: int = 128,
            inv_temperature: Optional[torch.Tensor] = None, seed: int = 0,
            rng_key: Optional[torch.Tensor] = None, rng_step: Optional[torch.Tensor] = None,

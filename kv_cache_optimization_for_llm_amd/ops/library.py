@@ -92,7 +92,6 @@ _HIP_SIGNATURES = {
     "kva_sample": [P, P, I, I, I, P, P, F, P, U, P, P, I, P, P, P, P, P],
     "kva_mark_tokens": [P, P, P, I, I, P],
     "kva_causal_conv_act": [P, I, I, P, I, I, I, P, I, P, LL, I, P, P, I, I, I, I, P, P, I, P],
-    "kva_upload": [P, P, LL, P],
     "kva_latent_prompt": [P, P, I, I, P, P, P, P, P, I, P, P, P, I, P, P, I, P, P, I, I, I, I, I, I, I, I, F, P],
     "kva_latent_prompt_supported": [I, I, I, I],
     "kva_gated_delta_rule": [P, P, LL, I, P, I, P, I, I, I, I, P, P, F, P, I, P, P, I, I, I, I, I, I, P, P],

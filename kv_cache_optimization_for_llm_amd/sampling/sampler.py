@@ -97,11 +97,10 @@ class Sampler:
         self._args_next = 0
 
     def _row_arguments(self, n: int):
-        """(a staging array [5, n] of int32 in pinned memory to fill, the same as uint32 and as float, the device arrays
-        its rows go to by :func:`ops.kernels.upload`, what to tell when it has been sent) for the next sampling of n
-        rows.  Slices and views are made once per number of rows: they cost more than what is done with them."""
+        """(a staging array to fill, the device arrays its rows go to) for the next sampling of n rows.  Slices and views are
+        made once per number of rows: they cost more than what is done with them."""
         if self._args_dev is None or self._args_dev.shape[1] < n:
-            cap = max(64, n)
+            cap = max(64, 1 << (n - 1).bit_length())
             self._args_dev = torch.zeros((5, cap), dtype=torch.int32, device=self.device)
             self._args_host = [_Staging(cap) for _ in range(3)]
             self._args_views.clear()
@@ -181,8 +180,10 @@ class Sampler:
                 # every token a request emits is marked in its mask row, by the launch that chooses it
                 staging.i32[4, :n] = [r.seat for r in rows]
                 mark_seat = dev_mark
+            # (torch's own copy: its allocator then knows that the block is in use until the copy has left it, also when this
+            # sampler goes away or takes larger ones before)
             staging.sent = event
-            K.upload(staging.pinned, self._args_dev)
+            self._args_dev.copy_(staging.pinned, non_blocking=True)
         try:
             K.sample(logits, out, chunks=self.chunks, inv_temperature=inv_t, seed=self.seed, rng_key=key,
                      rng_step=step, penalty_mask=self.mask if use_mask else None, row_seat=seat_t,
