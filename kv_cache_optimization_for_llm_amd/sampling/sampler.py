@@ -170,8 +170,8 @@ class Sampler:
             staging, (dev_t, dev_key, dev_step, dev_seat, dev_mark) = self._row_arguments(n)
             if any_sampled:
                 staging.f32[0, :n] = [1.0 / r.temperature if r.temperature > 0 else 0.0 for r in rows]
-                staging.u32[1, :n] = [r.rng_key & 0xFFFFFFFF for r in rows]
-                staging.u32[2, :n] = [r.rng_step & 0xFFFFFFFF for r in rows]
+                staging.u32[1, :n] = [int(r.rng_key) & 0xFFFFFFFF for r in rows]
+                staging.u32[2, :n] = [int(r.rng_step) & 0xFFFFFFFF for r in rows]
                 inv_t, key, step = dev_t, dev_key, dev_step
             if use_mask:
                 staging.i32[3, :n] = [r.seat if r.apply_penalty else -1 for r in rows]

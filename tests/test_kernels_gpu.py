@@ -952,6 +952,15 @@ def test_row_arguments_stay_until_their_copy_has_left_them(how, gpu):
     del others
 
 
+def test_sampler_takes_keys_and_steps_of_any_integer_type(gpu):
+    from kv_cache_optimization_for_llm_amd.sampling.sampler import Sampler, SampleRow
+    lg = torch.randn(1, 4000, generator=torch.Generator().manual_seed(1)).to(gpu)
+    sampler = Sampler(4000, 1, gpu, seed=5)
+    want = int(sampler.sample(lg, [SampleRow(0, 1.0, rng_key=(1 << 32) - 16, rng_step=70000)])[0])
+    for key, step in ((-16, 70000), (np.int32(-16), np.int32(70000)), (np.int64(-16), np.uint32(70000)), (np.uint32((1 << 32) - 16), np.int64(70000))):
+        assert int(sampler.sample(lg, [SampleRow(0, 1.0, rng_key=key, rng_step=step)])[0]) == want
+
+
 def test_sampler_distribution_and_boundaries(gpu):
     """python/sampling_reference.py:110-134: top-8 frequencies within 5 % over 40 000 draws."""
     vocab = 5000
