@@ -15,8 +15,11 @@
 //   rows x outputs x K    3 x 128,256 x 2,048: 480 -> 260 (4.0 TB/s)     3 x 16,384 x 2,048: 147 -> 33 (4.1 TB/s)
 //                         3 x 2,048 x 8,192: 544 -> 19 (3.5 TB/s)        3 x 3,072 x 2,048: 141 -> 11
 //                         32 x 2,048 x 8,192: 545 -> 58                  64 x 2,048 x 8,192: 559 -> 59 (the tiles: 167)
+//                         64 x 128,256 x 2,048: 532 -> 352 (96 TFLOP/s; the few-rows kernel: 941)
 //                         402 x 16,384 x 2,048: 449 -> 329 (82 TFLOP/s)  402 x 2,048 x 8,192: 556 -> 167 (81)
 //                         2,048 x 16,384 x 2,048: 1,748 -> 1,319 (104)
+// Not so for K up to 128 and tens of thousands of outputs (2,000 x 16,384 x 128: 130 -> 143, 64 x 128,256 x 64: 29 -> 26, 2,000 x
+// 128,256 x 64: 591 -> 703): a tile's result takes longer than its products.  No model here has such a product.
 // The few-rows kernel stays below the 6 TB/s of a plain read stream: a load takes 64 bytes from each of 16 rows.
 #include "common.h"
 
@@ -24,16 +27,15 @@ typedef float gf_f32x4 __attribute__((ext_vector_type(4)));
 
 #define GF_STEP 16                  // columns of K that one 16-byte load a lane covers
 #define GF_MAX_PARTS 16
-#define GF_ROWS_UP_TO 64            // rows up to which the few-rows kernel runs: one row of tiles does not fill the chip
+#define GF_ROWS_UP_TO 64            // rows up to which the few-rows kernel may run (gf_few_rows)
 #define GF_BM 64                    // the tile kernel: rows a workgroup, columns of K a round, padding of a row in LDS
 #define GF_BK 32
 #define GF_PAD 4
 
-// Columns of K a part takes: a sixteenth of K in whole rounds of the tile kernel, at least 64 - so at most 16 parts.
+// Columns of K a part takes: a sixteenth of K in whole rounds of the tile kernel - so at most 16 parts.
 static inline int gf_part(int K) {
     const int rounds = (K + GF_BK - 1) / GF_BK;
-    const int part = (rounds + GF_MAX_PARTS - 1) / GF_MAX_PARTS * GF_BK;
-    return part < 64 ? 64 : part;
+    return (rounds + GF_MAX_PARTS - 1) / GF_MAX_PARTS * GF_BK;
 }
 
 // Parts of the front half: an output is (sum of the front parts, in order) + (sum of the others, in order).
@@ -201,19 +203,19 @@ gemm_f32_tile_kernel(float *__restrict__ C, const float *__restrict__ A, const f
         }
     };
     // Two rounds at a time: while one is multiplied from its LDS buffer the next one waits in registers and the one
-    // after that is asked for.  The front half is never the shorter one: its rounds are both halves' (the back half's
-    // last ones may be zeros).
+    // after that is asked for.  The front half is never the shorter one: its barriers are both halves'.
     fetch(0, lo);
     fetch(1, lo + GF_BK);
     for (int d = 0; d < split; d += 2 * GF_BK) {
         put(0);
         __syncthreads();
         fetch(0, lo + d + 2 * GF_BK);
-        round(0);
+        if (lo + d < hi) round(0);
+        if (d + GF_BK >= split) break;                               // (of the front half, which no half is longer than)
         put(1);
         __syncthreads();
         fetch(1, lo + d + 3 * GF_BK);
-        round(1);
+        if (lo + d + GF_BK < hi) round(1);
     }
     __syncthreads();
     if (left != part)                                                // a last, shorter part
@@ -226,7 +228,8 @@ gemm_f32_tile_kernel(float *__restrict__ C, const float *__restrict__ A, const f
     // the back half's sums to the front half, through LDS (the operands there have been read)
     gf_f32x4 *over = reinterpret_cast<gf_f32x4 *>(&lds[0]);
     static_assert(sizeof(lds) >= sizeof(gf_f32x4) * 256 * NT * 2, "the back half's sums fit where the operands were");
-    if (back)
+    const bool halves = split < K;                                   // (else there is nothing in the back half)
+    if (back && halves)
 #pragma unroll
         for (int i = 0; i < NT; ++i)
 #pragma unroll
@@ -241,7 +244,8 @@ gemm_f32_tile_kernel(float *__restrict__ C, const float *__restrict__ A, const f
         for (int i = 0; i < NT; ++i) {
             const int n = n0 + wn + 16 * i + 4 * g;
             float *c = C + (size_t)m * ldc + n;
-            const gf_f32x4 o = over[(i * 2 + j) * 256 + tid];
+            gf_f32x4 o = {0.f, 0.f, 0.f, 0.f};
+            if (halves) o = over[(i * 2 + j) * 256 + tid];
             gf_f32x4 v;
 #pragma unroll
             for (int e = 0; e < 4; ++e) v[e] = tot[i][j][e] + o[e];
@@ -254,13 +258,21 @@ gemm_f32_tile_kernel(float *__restrict__ C, const float *__restrict__ A, const f
     }
 }
 
+// Whether few rows go to the kernel that streams W.  It makes 32 rows a pass over W and shares nothing between its
+// workgroups; from some number of outputs on the tiles fill the chip and are the faster ones (K = 2,048, few-rows kernel / tiles,
+// us): 17-32 rows, 8,192 outputs 28-33 / 46, 16,384 52-65 / 50, 128,256 399-492 / 350; 33-64 rows, 4,096 28-33 / 45, 6,144 42-48 /
+// 46, 8,192 51-62 / 46, 32,768 195-242 / 92, 128,256 754-941 / 345; K = 300 and 8,192 alike.
+static bool gf_few_rows(int M, int N) {
+    return M <= 16 || (M <= GF_ROWS_UP_TO && (long long)N * ((M + 31) / 32) < 14336);
+}
+
 template <bool VEC>
 static void gf_launch(float *C, const float *A, const float *W, int M, int N, int K, int lda, int ldw, int ldc,
                       hipStream_t stream) {
     const int part = gf_part(K), parts = (K + part - 1) / part;
-    if (M <= GF_ROWS_UP_TO) {
+    if (gf_few_rows(M, N)) {
         const int out = M <= 8 ? 8 : 16;
-        const dim3 grid((N + out - 1) / out, (M + 31) / 32), block(KVA_WAVE * (M <= 8 ? (parts + 1) / 2 : parts));
+        const dim3 grid((N + out - 1) / out, (M + 31) / 32), block(KVA_WAVE * (M <= 8 ? (parts + 1) / 2 : M <= 16 ? parts : max(4, parts)));    // (four for the sums' last step)
         if (M <= 8)
             hipLaunchKernelGGL((gemm_f32_rows_kernel<1, 2, true, VEC>), grid, block, 0, stream, C, A, W, M, N, K, lda, ldw, ldc, part);
         else if (M <= 16)

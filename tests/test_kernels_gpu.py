@@ -200,6 +200,16 @@ def test_gemm_f32_rows_are_the_same_bits_in_every_kernel(n, k, gpu):
     assert torch.equal(odd, rows[65])
 
 
+@pytest.mark.parametrize("n, k", [(7167, 40), (7168, 32), (14335, 48), (14336, 31), (20000, 96)])
+def test_gemm_f32_rows_are_the_same_bits_where_the_kernel_changes(n, k, gpu):
+    """16, 17, 32, 33, 64 and 65 rows of about as many outputs as send few rows to the tiles; sums of one to three parts."""
+    a, w = rnd(65, k).to(gpu), rnd(n, k, seed=1).to(gpu)
+    got = {m: K.gemm_nt_f32(a[:m], w, torch.full((m, n), float("nan"), device=gpu)) for m in (1, 16, 17, 32, 33, 64, 65)}
+    for m, rows in got.items():
+        assert torch.equal(rows, got[65][:m]), m
+    close(got[65], a.double() @ w.double().t(), torch.float32, "gemm_nt_f32")
+
+
 def rope_reference(x, pos, inv, heads, d, rot):
     cos, sin = plain.rope_cos_sin(pos, inv)
     x = x.view(len(pos), heads, d).clone()
