@@ -62,9 +62,7 @@ _LDS_MANY_GROUPS_WIDE_HEADS = 512
 _LDS_MIN_GROUPS_WIDE_HEADS = 16
 _LDS_TARGET_GROUPS_WIDE_HEADS = 512
 _LDS_MIN_KEYS_PER_SPLIT_WIDE_HEADS = 256
-# where the choice can change (a step shape that has a graph is told apart by these too)
-# (choose_portion_waves knows the mean to the step below it; the lines above are among them.  Few: every step is a line
-# between shapes that are captured apart)
+# where the choice can change: choose_portion_waves knows the mean to the step below it, the lines above are among them
 MEAN_KEYS_STEPS = (128,) + tuple(1 << k for k in range(9, 15))
 assert {_LDS_MIN_MEAN_KEYS_WIDE_HEADS, _LDS_SOME_GROUPS_MEAN_KEYS, _LDS_MIN_MEAN_KEYS} <= set(MEAN_KEYS_STEPS)
 # few workgroups that each walk thousands of keys: the keys are cut into ranges, one workgroup each
@@ -77,40 +75,56 @@ CHUNKS_IN_TUNED_KERNELS = True
 _ROWS_TWO_TILES = 32 * 1024          # (token, head) rows of a step from which the general rows kernel takes two tiles an item
 
 
-def choose_portion_waves(waves: int, mean_keys: float, head_dim: int) -> int:
+def choose_portion_waves(waves: int, mean_keys: float, head_dim: int, own_keys: float = 0.0, page_size: int = 16, group: int = 4,
+                         visible: int = 0) -> int:
     """Wavefronts of a workgroup (1: none of this, 2 or 4) that share an item of two row tiles of prompt portions, each an
-    equal share of what the item sees, for ``waves`` (item, kv head) pairs whose rows visit ``mean_keys`` keys on average.
+    equal share of what the item sees, for ``waves`` (item, kv head) pairs whose rows visit ``mean_keys`` keys on average,
+    ``own_keys`` of them of their own portions, and see about ``visible`` of them at most (0: all).
 
     One wavefront on two row tiles is a chain of products, softmax and products, 0.9 us a block of 32 keys with its SIMD to
     itself, and fixed key ranges with a merge kernel cost that kernel and leave early rows' ranges empty.  us a call without
     -> with, 32 heads of 64 over 8: one prompt of 256 / 512 / 1,024 / 1,536 / 2,048 / 2,304 / 2,560 tokens 14 / 26 / 22 / 34 /
     44 / 51 / 56 -> 7 / 10 / 17 / 26 / 39 / 45 / 52 (3,072 the same, 4,096 94 -> 112 and from there the workgroup kernel);
     three of 509 20 -> 15; 256 tokens behind 1,024 / 4,096 / 8,000 24 / 35 / 49 -> 12 / 26 / 42, 1,024 behind 2,000 / 6,000
-    65 / 107 -> 41 / 92, 2,048 behind 2,000 / 6,000 112 / 201 -> 89 / 188.  Not so: 64 behind 4,096 21 -> 24, 128 behind 8,000
-    32 -> 41, 512 behind 30,000 194 -> 199, eight of 200 10.4 -> 12.2 (a tie at four of 512).  Heads of 32 and 96 alike.
-    (512 to 767 pairs from 2,048 keys on stay with the workgroup kernel and its key ranges, which the tests of portions deep in
-    a prompt rest on, though 512 tokens behind 2,000 / 4,096 / 7,000 would go 41 / 52 / 70 -> 23 / 36 / 53.)
+    65 / 107 -> 41 / 92, 2,048 behind 2,000 / 6,000 112 / 201 -> 89 / 188.  Not so, and kept out: shares of a block or two (four
+    of 64 6.7 -> 7.2, sixteen 8.2 -> 9.2), few pairs far behind, which more workgroups with a range each serve better (33
+    tokens behind 1,024 12.5 -> 15.2, 64 behind 4,096 21 -> 24, 128 behind 8,000 32 -> 41; 8 heads over 8, 300 tokens behind 1,000
+    13.9 -> 17.5, 767 behind 2,000 25.8 -> 28.6), 512 behind 30,000 194 -> 199, 1,536 behind 20,000 358 -> 389, eight of 200
+    10.4 -> 12.2.  Heads of 32 and 96 alike; pages of other sizes than 16, whose keys are looked up one by one, less far
+    (128 behind 4,000 37 -> 52).  Behind a window key ranges of the whole context are mostly empty: 64 behind 2,000 with 256
+    visible 15.5 -> 9.  (512 to 767 pairs from 2,048 keys on stay with the workgroup kernel and its key ranges, which the tests
+    of portions deep in a prompt rest on, though 512 / 640 tokens behind 2,000 would go 45 / 49 -> 26 / 33, behind 4,000 52 / 59 ->
+    37 / 51 and 640 behind 8,000 93 -> 86.)
 
     Heads of 128 hold a SIMD's registers with one wavefront, so what there is to win ends earlier: 32 heads, 256 / 512 / 768
     tokens 26 / 35 / 40 -> 10 / 14 / 19, 256 behind 1,024 / 4,096 34 / 41 -> 17 / 36, 512 behind 2,000 49 -> 36; 24 heads, 1,024
-    tokens 42 -> 22, four of 256 behind 1,000 57 -> 38; but four of 256 (32 heads) 13 -> 16, behind 1,000 38 -> 43, eight of
-    100 9.6 -> 11.9, 512 behind 7,000 90 -> 104."""
+    tokens 42 -> 22, four of 256 behind 1,000 57 -> 38; but four of 64 7.2 -> 8.1, four of 256 (32 heads) 13 -> 16, behind 1,000
+    38 -> 43, eight of 100 9.6 -> 11.9, eight of 100 behind 3,000 (16 heads) 63 -> 72, 512 behind 7,000 90 -> 104."""
     if head_dim > 128:
         return 1
     keys = max((step for step in MEAN_KEYS_STEPS if step <= mean_keys), default=0)
+    bound = 0 < visible < keys
+    if bound:
+        keys = max((step for step in MEAN_KEYS_STEPS if step <= visible), default=0)
+    least = max(keys, min(own_keys, visible) if visible > 0 else own_keys)
+    far = keys if page_size == 16 else keys * 5 // 4
+    if bound and waves <= 1024 and keys < 512:
+        return 2 if least >= 48 else 1
     if head_dim > 96:
         if waves <= 256 and keys >= 512:
-            return 4 if keys <= 12 * waves else 1
+            return 4 if waves >= (64 if keys == 512 else 96) and far <= 12 * waves else 1
         if waves <= 256:
-            return 2 if waves >= 128 else 1
-        return 2 if waves < 1024 and waves <= 12 * keys and keys <= 4 * waves else 1
+            return 2 if waves >= 128 and least >= 48 else 1
+        return 2 if waves < 1024 and waves <= 12 * keys and keys <= (3 if group == 1 and keys >= 2048 else 4) * waves else 1
     if 512 <= waves < 768 and keys >= _LDS_MIN_MEAN_KEYS:
         return 1
+    if least < 64:
+        return 2 if 128 <= waves < (768 if page_size == 16 else 1024) and least >= 48 else 1
     if waves <= 512:
         if keys >= 512:
-            return 4 if keys <= 16 * waves else 1
+            return 4 if waves >= (64 if group > 1 else 128) and far <= (16 if group > 1 or head_dim > 64 else 10) * waves else 1
         return 2 if waves >= 128 else 1
-    if waves > 2560 or (waves > 1024 and waves > 12 * keys):
+    if waves > 2560 or (waves > 1024 and (waves > 12 * keys or (keys >= 16384 and page_size == 16 and head_dim >= 64))):
         return 1
     return 4 if waves * keys >= 3 << 20 else 2
 
@@ -370,12 +384,12 @@ def choose_lds_splits(groups: int, max_context: int, max_splits: int = None, hea
     return _cut_keys(min(want, max(1, max_context // min_keys)), max_context, max_splits)
 
 
-def _plan_for(batch, kv, num_q_heads: int, num_kv_heads: int, head_dim: int, max_parts: int = 0) -> list:
+def _plan_for(batch, kv, num_q_heads: int, num_kv_heads: int, head_dim: int, max_parts: int = 0, visible: int = 0) -> list:
     plans = batch.attention_plans
-    key = (num_q_heads, num_kv_heads, head_dim, kv.page_size, max_parts)
+    key = (num_q_heads, num_kv_heads, head_dim, kv.page_size, max_parts, visible)
     plan = plans.get(key)
     if plan is None:
-        plan = plans[key] = _plan(batch, num_q_heads // num_kv_heads, num_kv_heads, head_dim, kv.page_size, max_parts)
+        plan = plans[key] = _plan(batch, num_q_heads // num_kv_heads, num_kv_heads, head_dim, kv.page_size, max_parts, visible)
     return plan
 
 
@@ -469,7 +483,7 @@ def paged_attention(qkv: torch.Tensor, out: torch.Tensor, kv, batch, num_q_heads
                                    head_dim, scale, window)
     if chunk > 0:
         window = -chunk         # the tuned kernels take both masks in one number: below zero, chunks of so many positions
-    plan = _plan_for(batch, kv, num_q_heads, num_kv_heads, head_dim, max_parts)
+    plan = _plan_for(batch, kv, num_q_heads, num_kv_heads, head_dim, max_parts, window if window >= 0 else max(1, -window // 2))
     for launch in plan:
         if launch[0] == "wave":
             _, (item_entry, item_row0, meta), tiles, splits, per, pair, covers_all, keep_cached, waves = launch
@@ -488,8 +502,27 @@ def paged_attention(qkv: torch.Tensor, out: torch.Tensor, kv, batch, num_q_heads
     return out
 
 
-def _plan(batch, group: int, num_kv_heads: int, head_dim: int, page_size: int, max_parts: int = 0) -> list:
-    """The launches of one attention call over ``batch``: ("wave", items, row tiles, splits, keys per
+def portion_choice(lens, mean_keys: float, group: int, num_kv_heads: int, head_dim: int, page_size: int, visible: int = 0) -> tuple:
+    """(:func:`choose_portion_waves`, whether prompt portions go to the workgroup kernel) for a step whose entries have ``lens``
+    tokens: all that the step's mean number of keys decides, and so what tells captured shapes of the same entries apart."""
+    rows = [n * group for n in lens]
+    if max(rows) <= 16:
+        return 1, False
+    mixed = min(rows) <= 16
+    long = [n for n in rows if not mixed or n > 16]
+    tiles = K.attention_mfma_row_tiles(head_dim, True)
+    if tiles == 2:
+        # (its own tokens are known exactly, keys in front of a portion to the step of MEAN_KEYS_STEPS)
+        own_keys = sum(n * n for n in long) / (2 * group * sum(long))
+        sharing = choose_portion_waves(sum(-(-n // 32) for n in long) * num_kv_heads, mean_keys, head_dim, own_keys, page_size, group, visible)
+        if sharing > 1:
+            return sharing, False
+    groups = sum(-(-n // 128) for n in long) * num_kv_heads
+    return 1, bool(K.attention_lds_supported(head_dim, page_size)) and use_lds_kernel(groups, mean_keys, head_dim)
+
+
+def _plan(batch, group: int, num_kv_heads: int, head_dim: int, page_size: int, max_parts: int = 0, visible: int = 0) -> list:
+    """The launches of one attention call over ``batch`` (``visible`` > 0: a token sees about so many keys at most): ("wave", items, row tiles, splits, keys per
     split, pair, covers all rows, keep cached, wavefronts of a workgroup that share an item) and
     ("lds", item records, splits, keys per split, covers all rows)."""
     plan = []
@@ -520,22 +553,19 @@ def _plan(batch, group: int, num_kv_heads: int, head_dim: int, page_size: int, m
     # two row tiles per wave, so each key and value loaded serves 32 query rows
     tiles = K.attention_mfma_row_tiles(head_dim, True)
     starts = batch.h_entry_q_start.tolist()
-    rows = [(end - start) * group for start, end in zip(starts, starts[1:])]
-    count = sum(-(-n // (16 * tiles)) for n in rows if not mixed or n > 16) * num_kv_heads
-    mean_keys = batch.mean_keys_of_long_entries()
-    sharing = choose_portion_waves(count, mean_keys, head_dim)
-    if tiles == 2 and sharing > 1:
+    sharing, by_workgroup = portion_choice([end - start for start, end in zip(starts, starts[1:])], batch.mean_keys_of_long_entries(),
+                                           group, num_kv_heads, head_dim, page_size, visible)
+    if sharing > 1:
         items = batch.attention_items(group, tiles, which)
         plan.append(("wave", items, tiles, sharing, 0, False, which == "all", False, sharing))
         if mixed:
             decoded("short")
         return plan
     done = False
-    if K.attention_lds_supported(head_dim, page_size):
+    if by_workgroup:
         items = batch.attention_items(group, 8, which)
-        groups = items[0].shape[0] * num_kv_heads
-        if items[2] is not None and use_lds_kernel(groups, mean_keys, head_dim):
-            splits, per = choose_lds_splits(groups, batch.max_context, head_dim=head_dim)
+        if items[2] is not None:
+            splits, per = choose_lds_splits(items[0].shape[0] * num_kv_heads, batch.max_context, head_dim=head_dim)
             plan.append(("lds", items[2], splits, per, which == "all"))
             done = True
     if not done:

@@ -269,3 +269,22 @@ def test_a_steps_workspace_is_reserved_and_counts_against_the_graphs_kept(monkey
     assert graphs.make_room((512,) + (1,) * 8, 8192) == 520 and len(graphs.slots) == 10        # (decoded tokens beside it: nothing expanded)
     model.step_workspace_bytes = lambda lens, context: 17000 * 65536
     assert graphs.make_room((512,), 8192) is None and len(graphs.slots) == 10
+
+
+def test_portions_that_do_better_without_sharing_an_item():
+    """Measured (us, without / with): short shares, few pairs far behind, pages looked up key by key, windows; and a captured step's
+    shape, which names the step below the mean and the tokens of its entries, decides all of it."""
+    from kv_cache_optimization_for_llm_amd.ops.attention import MEAN_KEYS_STEPS, choose_portion_waves
+    for args in ((256, 32.5, 64, 32.0), (1024, 32.5, 64, 32.0), (800, 50, 80, 50.0), (256, 32.5, 128, 32.0), (40, 1017, 64, 16.5), (64, 4032, 64, 32.0),
+                 (80, 1150, 64, 150.0, 16, 1), (192, 2384, 64, 383.0, 16, 1), (1536, 20768, 64, 768.0), (128, 4064, 64, 64.0, 32), (304, 8150, 64, 150.0, 8),
+                 (512, 3050, 128, 50.0, 16, 1), (512, 2500, 128, 500.0, 16, 1), (40, 1017, 128, 16.5), (2048, 1024, 64, 1024.0, 16, 4, 128)):
+        assert choose_portion_waves(*args) == 1, args
+    for args, waves in (((512, 256.5, 64, 256.0), 2), ((256, 128.5, 64, 128.0), 2), ((256, 1152, 64, 128.0), 4), ((200, 2100, 64, 100.0), 4), ((512, 2256, 128, 256.0), 2),
+                        ((128, 64.5, 64, 64.0), 2), ((1536, 20768, 64, 768.0, 8), 4), ((64, 2032, 64, 32.0, 16, 4, 256), 2), ((64, 300, 64, 32.0, 16, 4, 256), 1),
+                        ((128, 1064, 128, 64.0, 16, 4, 1024), 4)):
+        assert choose_portion_waves(*args) == waves, args
+    for n in range(1, 3000, 131):
+        for mean in (20, 127, 129, 300, 511, 513, 900, 1500, 3000, 7000, 30000):
+            step = max([s for s in MEAN_KEYS_STEPS if s <= mean], default=0)
+            for rest in ((64, 30.0), (64, 50.0, 8), (128, 100.0, 16, 1), (64, 20.0, 16, 4, 256), (64, 400.0, 16, 2, 128), (128, 100.0, 32, 4, 700)):
+                assert choose_portion_waves(n, mean, *rest) == choose_portion_waves(n, step, *rest)
