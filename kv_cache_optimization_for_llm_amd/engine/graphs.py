@@ -220,12 +220,13 @@ class _PortionSlot:
 class PortionGraphs:
     """Graphs for steps that hold prompt portions (alone or beside decoded tokens).
 
-    A shape is (tokens per entry, wanted places, context bucket, the step (MEAN_KEYS_STEPS) below the mean number of
-    keys the portions' rows visit, by which the attention kernel is chosen): everything the forward pass decides on the
-    host.  Its first step runs eagerly and tells which sets of attention work items the pass asks
-    for; the step at which it has come ``CAPTURE_AT`` times is captured over static buffers; later
-    ones upload their indices and replay.  Logits come back in the shape's static buffer: they hold
-    until its next step."""
+    A shape is (tokens per entry, wanted places, context bucket, what each head layout of the model's attention calls decides
+    by the mean number of keys the portions' rows visit): everything the forward pass decides on the host.  The choices and
+    not a step of the mean: portions of 64 to 512 tokens beside a decoded context of 8,192 are 2 or 3 shapes by the choices and
+    were 5 or 6 by the steps, each with first steps that are not replayed and a place among those kept.  Its first step runs
+    eagerly and tells which sets of attention work items the pass asks for; the step at which it has come ``CAPTURE_AT`` times
+    is captured over static buffers; later ones upload their indices and replay.  Logits come back in the shape's static
+    buffer: they hold until its next step."""
 
     MAX_TOKENS = 4096          # tokens of one captured step
     MAX_LOGIT_ROWS = 64        # a graph keeps its logits: [rows, vocabulary] fp32
@@ -245,12 +246,12 @@ class PortionGraphs:
         self.seen: Dict[tuple, tuple] = {}
         self.times: Dict[tuple, int] = {}            # steps a seen shape has come (while it has no graph)
         self.slots: "OrderedDict[tuple, _PortionSlot]" = OrderedDict()
+        self.layouts: tuple = ()                     # of the attention calls, as portion_choice takes them; from eager steps
         self.replays = 0
         self.captures = 0
 
-    @staticmethod
-    def shape_key(lens: Sequence[int], starts: Sequence[int], rows: Sequence[int]) -> Optional[tuple]:
-        from ..ops.attention import MEAN_KEYS_STEPS
+    def shape_key(self, lens: Sequence[int], starts: Sequence[int], rows: Sequence[int]) -> Optional[tuple]:
+        from ..ops.attention import portion_choice
         T = int(sum(lens))
         if T > PortionGraphs.MAX_TOKENS or len(rows) > PortionGraphs.MAX_LOGIT_ROWS:
             return None
@@ -258,11 +259,15 @@ class PortionGraphs:
         long = ln > 1
         mean_keys = float(((st[long] + (ln[long] + 1) / 2) * ln[long]).sum() / ln[long].sum())
         bucket = context_bucket(int(max(s + n for s, n in zip(starts, lens))))
-        return (tuple(int(n) for n in lens), tuple(int(r) for r in rows), bucket,
-                tuple(mean_keys >= t for t in MEAN_KEYS_STEPS))
+        lens = tuple(int(n) for n in lens)
+        return (lens, tuple(int(r) for r in rows), bucket, tuple(portion_choice(lens, mean_keys, *layout) for layout in self.layouts))
 
     def note(self, key: tuple, batch: StepBatch) -> None:
         """After the eager run of a shape: the sets of attention items its forward pass used."""
+        layouts = {(q // kv, kv, dim, page, visible) for q, kv, dim, page, _, visible in batch.attention_plans}
+        if not layouts <= set(self.layouts):
+            self.layouts = tuple(sorted(layouts | set(self.layouts)))
+            key = self.shape_key(key[0], batch.h_entry_start_pos.tolist(), key[1])
         if key not in self.seen:
             if len(self.seen) >= self.MAX_SEEN:
                 self.seen.clear()

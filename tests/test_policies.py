@@ -288,3 +288,31 @@ def test_portions_that_do_better_without_sharing_an_item():
             step = max([s for s in MEAN_KEYS_STEPS if s <= mean], default=0)
             for rest in ((64, 30.0), (64, 50.0, 8), (128, 100.0, 16, 1), (64, 20.0, 16, 4, 256), (64, 400.0, 16, 2, 128), (128, 100.0, 32, 4, 700)):
                 assert choose_portion_waves(n, mean, *rest) == choose_portion_waves(n, step, *rest)
+
+
+def test_captured_shapes_are_told_apart_by_what_is_decided():
+    """Steps of the same entries whose attention is decided alike share a shape, whatever their mean number of keys; those decided
+    otherwise do not.  The head layouts come from the first eager step, which is noted under the shape its next step asks for."""
+    from types import SimpleNamespace
+
+    import numpy as np
+    from kv_cache_optimization_for_llm_amd.engine.graphs import PortionGraphs
+    from kv_cache_optimization_for_llm_amd.ops.attention import portion_choice
+    for heads, dim in ((32, 64), (32, 128), (24, 128)):
+        graphs = PortionGraphs(None, None, "cpu")
+        lens, rows = (512,) + (1,) * 8, tuple(range(511, 520))
+
+        def key(start):
+            return graphs.shape_key(lens, [start] + [8000] * 8, rows)
+        batch = SimpleNamespace(attention_plans={(heads, 8, dim, 16, 0, 0): [], (heads, 8, dim, 16, 12, 0): [], (heads, 8, dim, 16, 0, 256): []},
+                                h_entry_start_pos=np.asarray([1536] + [8000] * 8, dtype=np.int32), _items={})
+        graphs.note(key(1536), batch)
+        assert list(graphs.seen) == [key(1536)] and graphs.times[key(1536)] == 1
+        assert len(graphs.layouts) == 2
+        keys, choices = {}, set()
+        for start in range(0, 7680, 128):
+            decided = tuple(portion_choice(lens, start + 256.5, heads // 8, 8, dim, 16, visible) for visible in (0, 256))
+            assert keys.setdefault(key(start), decided) == decided
+            choices.add(decided)
+        assert len(keys) == len(choices) <= 3
+    assert PortionGraphs(None, None, "cpu").shape_key([5000], [0], [4999]) is None
