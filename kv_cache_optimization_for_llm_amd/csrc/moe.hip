@@ -771,9 +771,13 @@ extern "C" int kva_moe_expert_rows(void *out, int out_dtype, const void *x, cons
     if (max_tiles == 0) return KVA_OK;
     MoeRows a{sorted_slot, tile_expert, slot_weight, top, N, K, mode, act, tiled, gated, limit};
     if (group > 1) {
-        // 256 outputs a workgroup (two workgroups a compute unit) where that leaves no unit idle; 128 where it would:
-        // 8,192 slots of 4 experts, 1,024 x 2,048 (256 workgroups of the wide kind) 75 against 56 us, 2,048 x 1,024 (512)
-        // 43 against 53; 3,356 slots of 16 experts, 1,536 x 2,048 (258) 59 against 44
+        // 256 outputs a workgroup (two workgroups a compute unit) where that leaves no unit idle; 128 where it would.  The line goes
+        // by the groups the list has room for, 5 to 40 % more than the split puts in use (the more the more experts).  us, 128 / 256
+        // outputs, by wide workgroups with room / in use: 160 slots an expert of 1,536 x 2,048, 16 experts 47/60 (216 / 174), 32
+        // 84/74 (432 / 324); 1,024 x 2,048, 32 experts 48/61 (288 / 212), 64 118/96 (576 / 412), 128 228/190 (1,148 / 872); 800 slots
+        // of 1,024 x 2,048, 4 experts 39/58 (116 / 112), 16 87/76 (464 / 440).  Above, wide takes 0.8 to 0.95 of the time, but for a
+        // second turn of few workgroups (550 to 700 in use): 83/89, 128/133, 165/164.  Between 300 and 400 with room it would do as
+        // well (82/73 at 368 / 308) or better.
         const int groups = max_tiles / group, wide = (N + 255) / 256, narrow = (N + 127) / 128;
         KVA_REQUIRE((long long)narrow * groups <= 0x7fffffff, "moe_expert_rows: too many workgroups");
         if (group == 8 && (long long)wide * groups >= 400)
