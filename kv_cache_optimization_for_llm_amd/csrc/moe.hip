@@ -756,10 +756,11 @@ extern "C" int kva_moe_group_supported(int group, int K) { return (group == 4 ||
 extern "C" int kva_moe_expert_rows(void *out, int out_dtype, const void *x, const void *w, int dtype,
                                    const int *sorted_slot, const int *tile_expert, const float *slot_weight,
                                    int max_tiles, int top, int N, int K, int mode, int act, int gated, float limit,
-                                   int group, int tiled, hipStream_t stream) {
+                                   int group, int wide, int tiled, hipStream_t stream) {
     KVA_REQUIRE(!tiled || (dtype == KVA_BF16 && K % 32 == 0 && N % 16 == 0), "moe_expert_rows: no operand order for %d x %d", N, K);
     KVA_REQUIRE(group == 1 || (dtype == KVA_BF16 && kva_moe_group_supported(group, K) && max_tiles % group == 0),
                 "moe_expert_rows: no kernel for groups of %d tiles, %d of them, with K = %d", group, max_tiles, K);
+    KVA_REQUIRE(!wide || group == 8, "moe_expert_rows: 256 outputs a workgroup go with groups of 8 tiles, not %d", group);
     KVA_REQUIRE(act != 4 || gated, "moe_expert_rows: the clamped activation is a gated one");
     KVA_REQUIRE(!gated || (mode == 0 && N % 2 == 0), "moe_expert_rows: gate and up rows come in pairs, in the first product");
     KVA_REQUIRE(out && x && w && sorted_slot && tile_expert, "moe_expert_rows: missing operand");
@@ -771,24 +772,17 @@ extern "C" int kva_moe_expert_rows(void *out, int out_dtype, const void *x, cons
     if (max_tiles == 0) return KVA_OK;
     MoeRows a{sorted_slot, tile_expert, slot_weight, top, N, K, mode, act, tiled, gated, limit};
     if (group > 1) {
-        // 256 outputs a workgroup (two workgroups a compute unit) where that leaves no unit idle; 128 where it would.  The line goes
-        // by the groups the list has room for, 5 to 40 % more than the split puts in use (the more the more experts).  us, 128 / 256
-        // outputs, by wide workgroups with room / in use: 160 slots an expert of 1,536 x 2,048, 16 experts 47/60 (216 / 174), 32
-        // 84/74 (432 / 324); 1,024 x 2,048, 32 experts 48/61 (288 / 212), 64 118/96 (576 / 412), 128 228/190 (1,148 / 872); 800 slots
-        // of 1,024 x 2,048, 4 experts 39/58 (116 / 112), 16 87/76 (464 / 440).  Above, wide takes 0.8 to 0.95 of the time, but for a
-        // second turn of few workgroups (550 to 700 in use): 83/89, 128/133, 165/164.  Between 300 and 400 with room it would do as
-        // well (82/73 at 368 / 308) or better.
-        const int groups = max_tiles / group, wide = (N + 255) / 256, narrow = (N + 127) / 128;
-        KVA_REQUIRE((long long)narrow * groups <= 0x7fffffff, "moe_expert_rows: too many workgroups");
-        if (group == 8 && (long long)wide * groups >= 400)
-            hipLaunchKernelGGL((moe_expert_rows_lds_kernel<4, 8, 3>), dim3(wide * groups), dim3(256), 0, stream, a, out, out_dtype,
-                               (const bf16_t *)x, (const bf16_t *)w, wide, groups);
+        const int groups = max_tiles / group, blocks = wide ? (N + 255) / 256 : (N + 127) / 128;
+        KVA_REQUIRE((long long)blocks * groups <= 0x7fffffff, "moe_expert_rows: too many workgroups");
+        if (wide)
+            hipLaunchKernelGGL((moe_expert_rows_lds_kernel<4, 8, 3>), dim3(blocks * groups), dim3(256), 0, stream, a, out, out_dtype,
+                               (const bf16_t *)x, (const bf16_t *)w, blocks, groups);
         else if (group == 8)
-            hipLaunchKernelGGL((moe_expert_rows_lds_kernel<4, 4, 4>), dim3(narrow * groups), dim3(256), 0, stream, a, out, out_dtype,
-                               (const bf16_t *)x, (const bf16_t *)w, narrow, groups);
+            hipLaunchKernelGGL((moe_expert_rows_lds_kernel<4, 4, 4>), dim3(blocks * groups), dim3(256), 0, stream, a, out, out_dtype,
+                               (const bf16_t *)x, (const bf16_t *)w, blocks, groups);
         else
-            hipLaunchKernelGGL((moe_expert_rows_lds_kernel<2, 4, 4>), dim3(narrow * groups), dim3(256), 0, stream, a, out, out_dtype,
-                               (const bf16_t *)x, (const bf16_t *)w, narrow, groups);
+            hipLaunchKernelGGL((moe_expert_rows_lds_kernel<2, 4, 4>), dim3(blocks * groups), dim3(256), 0, stream, a, out, out_dtype,
+                               (const bf16_t *)x, (const bf16_t *)w, blocks, groups);
     } else if (dtype == KVA_BF16 && K % 32 == 0) {
         // few tiles: 16 outputs a workgroup, so that enough of them stream the matrices; many: 64 outputs and
         // four row tiles, which share what they load

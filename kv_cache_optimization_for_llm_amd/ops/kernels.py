@@ -2193,6 +2193,18 @@ def moe_group(slots: int, experts: int, dtype: torch.dtype, *inner: int) -> int:
     return 1
 
 
+def moe_wide(outputs: int, tiles: int, group: int, experts: int) -> bool:
+    """Whether a workgroup of the experts' products takes a group of 8 tiles against 256 ``outputs``, two workgroups a compute unit,
+    or against 128.  128 are the faster ones while the chip takes them at once, up to 512 workgroups: 256 of the wide kind in use
+    (by wide workgroups in use, us, 128 / 256 outputs: 1,024 x 2,048 64 38/59, 160 45/59, 256 48/61, 308 82/73, 440 87/76, 616
+    155/150, 924 210/168; 2,048 x 1,024 224 31/42, 256 32/43, 304 52/50, 472 59/53, 904 129/112; the same numbers from 4 to 128
+    experts; a second turn of few wide workgroups, 590 to 700, ties or loses up to 8 %).  How many groups are in use is the
+    split's affair: of the ``tiles`` that the list has room for, half a group an expert stays empty on average.  Of 392 steps around
+    the line, of 4 to 128 experts, this one takes the slower kind by more than 10 % in 45, of 148 that it sends the other way one;
+    400 with room took it in 162 (up to 1.34 times as long)."""
+    return group == 8 and -(-outputs // 256) * (2 * (tiles // 8) - experts) > 2 * 288
+
+
 def moe_align(idx: torch.Tensor, experts: int, sorted_slot: torch.Tensor, tile_expert: torch.Tensor, group: int = 1) -> None:
     """The slots ``idx.view(-1)`` that name one of the first ``experts`` router outputs, sorted by
     expert into ``sorted_slot`` (every tile of 16 places belongs to one expert, -1 pads) with the
@@ -2273,8 +2285,8 @@ def moe_expert_rows(x: torch.Tensor, w: torch.Tensor, out: torch.Tensor, sorted_
         _dev(out, "out"), dtype_code(out.dtype), _dev(x, "x"), _dev(w, "w"), dtype_code(x.dtype),
         _dev(sorted_slot, "sorted_slot", torch.int32), _dev(tile_expert, "tile_expert", torch.int32),
         _opt(slot_weight, "slot_weight"), tiles, int(top), w.shape[1], w.shape[2], 0 if activation is not None else 1,
-        EXPERT_ACTIVATIONS.get(activation, 0), 1 if gated else 0, float(limit), int(group), 1 if tiled else 0, _stream()),
-        "moe_expert_rows")
+        EXPERT_ACTIVATIONS.get(activation, 0), 1 if gated else 0, float(limit), int(group),
+        1 if moe_wide(w.shape[1], tiles, group, w.shape[0]) else 0, 1 if tiled else 0, _stream()), "moe_expert_rows")
     return out
 
 

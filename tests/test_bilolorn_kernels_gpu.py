@@ -500,6 +500,35 @@ def test_experts_products_in_tiles_and_in_groups_of_tiles(rows, width, ff, exper
         close(out, want, 3e-2, "second product")
 
 
+@pytest.mark.parametrize("rows, width, ff, experts, top, gated", [(7, 96, 36, 5, 2, True), (700, 128, 132, 9, 4, True), (513, 256, 256, 2, 1, False),
+                                                                  (1500, 544, 264, 8, 3, False)])
+def test_experts_products_are_the_same_against_128_and_256_outputs_a_workgroup(rows, width, ff, experts, top, gated, gpu, monkeypatch):
+    """Bit for bit: an output's products are added up in the same order.  Outputs below, at and behind multiples of 128 and 256."""
+    g = torch.Generator().manual_seed(rows)
+    idx = torch.rand((rows, experts), generator=g).argsort(-1)[:, :top].to(torch.int32).contiguous()
+    x, ff_pad = rnd((rows, width), 1, torch.bfloat16), (ff + 31) // 32 * 32
+    up = rnd((experts, (2 if gated else 1) * ff, width), 2, torch.bfloat16, width ** -0.5)
+    down = rnd((experts, width, ff_pad), 3, torch.bfloat16, ff ** -0.5)
+    wgt = torch.rand((rows, top), generator=g).to(gpu)
+    tiles = K.moe_tiles(rows * top, experts, 8)
+    slot = torch.empty(tiles * K.MOE_TILE, dtype=torch.int32, device=gpu)
+    tile_expert = torch.empty(tiles, dtype=torch.int32, device=gpu)
+    K.moe_align(idx.to(gpu), experts, slot, tile_expert, 8)
+    hidden = rnd((tiles * K.MOE_TILE, ff_pad), 4, torch.bfloat16).to(gpu)
+    for tiled in (False, True)[:2 if up.shape[1] % 16 == 0 else 1]:
+        lay = K.moe_tiled_weight if tiled else (lambda w: w)
+        got = []
+        for wide in (False, True):
+            monkeypatch.setattr(K, "moe_wide", lambda *sizes: wide)
+            act = torch.zeros((tiles * K.MOE_TILE, ff), dtype=torch.bfloat16, device=gpu)
+            K.moe_expert_rows(x.to(gpu), lay(up.to(gpu)), act, slot, tile_expert, top, activation="silu" if gated else "relu2", gated=gated,
+                              group=8, tiled=tiled)
+            out = torch.full((rows * top, width), float("nan"), dtype=torch.float32, device=gpu)
+            K.moe_expert_rows(hidden, lay(down.to(gpu)), out, slot, tile_expert, top, slot_weight=wgt, group=8, tiled=tiled)
+            got.append((act[slot >= 0].cpu(), out.cpu()))
+        assert torch.equal(got[0][0], got[1][0]) and torch.equal(got[0][1], got[1][1]) and got[0][0].any() and got[0][1].isfinite().all()
+
+
 @pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
 @pytest.mark.parametrize("rows, width, ff, experts, top, shared", [(1, 64, 32, 6, 2, 48), (33, 40, 20, 3, 1, 0), (300, 128, 96, 9, 4, 64)])
 def test_table_experts_with_and_without_the_expert_every_token_uses(rows, width, ff, experts, top, shared, dtype, gpu):

@@ -316,3 +316,14 @@ def test_captured_shapes_are_told_apart_by_what_is_decided():
             choices.add(decided)
         assert len(keys) == len(choices) <= 3
     assert PortionGraphs(None, None, "cpu").shape_key([5000], [0], [4999]) is None
+
+
+def test_experts_products_take_256_outputs_a_workgroup_where_128_would_not_fit_the_chip_at_once():
+    """By the groups that are in use, measured (us, 128 / 256 outputs), not by those the list has room for."""
+    from kv_cache_optimization_for_llm_amd.ops.kernels import moe_tiles, moe_wide
+    for slots, experts, outputs, wide in ((8192, 4, 1024, False), (8192, 4, 2048, True),                    # 56/75, 53/43
+                                          (3356, 16, 1536, False), (6400, 16, 1536, True), (12800, 16, 768, True),      # 44/59, 82/71, 84/73
+                                          (7680, 32, 1024, True), (5120, 32, 1024, False), (10240, 64, 512, False),     # 82/73, 48/61, 48/61
+                                          (15360, 64, 512, True), (20480, 128, 512, True), (10240, 64, 768, True)):     # 80/73, 120/100, 86/75
+        assert moe_wide(outputs, moe_tiles(slots, experts, 8), 8, experts) == wide, (slots, experts, outputs)
+    assert not moe_wide(4096, moe_tiles(20000, 16, 4), 4, 16)
