@@ -329,7 +329,8 @@ extern "C" int kva_heads_matmul_mfma(void *out, int o_row, int o_head, const voi
                 "heads_matmul_mfma: strides do not fit %d heads of %d -> %d", heads, K, N);
     HEADS_OPTIONS(gate, ro);
     if (rows == 0) return KVA_OK;
-    if (rows > HM_LDS_ROWS && N >= 64) {
+    // (loads that go straight to LDS want their 16 bytes at multiples of 16; those to registers take any address)
+    if (rows > HM_LDS_ROWS && N >= 64 && (((uintptr_t)x | (uintptr_t)w) & 15) == 0) {
         const int n_blocks = (N + 127) / 128, cols = n_blocks + (rot > 0 ? 1 : 0);
         // the smaller tile where the larger would leave compute units without work
         const bool small = (long long)n_blocks * heads * ((rows + 127) / 128) < 512;

@@ -771,7 +771,9 @@ extern "C" int kva_moe_expert_rows(void *out, int out_dtype, const void *x, cons
     KVA_REQUIRE(max_tiles >= 0 && max_tiles <= 65535, "moe_expert_rows: %d tiles are too many for one launch", max_tiles);
     if (max_tiles == 0) return KVA_OK;
     MoeRows a{sorted_slot, tile_expert, slot_weight, top, N, K, mode, act, tiled, gated, limit};
-    if (group > 1) {
+    // (operands at other addresses than multiples of 16: loads that go straight to LDS do not take those, the kernels below do,
+    // over a list in groups as over any other)
+    if (group > 1 && (((uintptr_t)x | (uintptr_t)w) & 15) == 0) {
         const int groups = max_tiles / group, blocks = wide ? (N + 255) / 256 : (N + 127) / 128;
         KVA_REQUIRE((long long)blocks * groups <= 0x7fffffff, "moe_expert_rows: too many workgroups");
         if (wide)

@@ -529,6 +529,33 @@ def test_experts_products_are_the_same_against_128_and_256_outputs_a_workgroup(r
         assert torch.equal(got[0][0], got[1][0]) and torch.equal(got[0][1], got[1][1]) and got[0][0].any() and got[0][1].isfinite().all()
 
 
+@pytest.mark.parametrize("x_at, w_at", [(1, 0), (0, 1), (4, 2)])
+@pytest.mark.parametrize("group", [4, 8])
+def test_products_of_many_rows_take_operands_at_any_address(group, x_at, w_at, gpu):
+    """Experts' products and products per head whose operands start at no multiple of 16 bytes go through registers, not straight to
+    LDS: the same numbers but for the order of the sums, the results rounded to bf16 (2^-9 of a result, each)."""
+    def at(t, offset):
+        flat = torch.empty(t.numel() + offset, dtype=t.dtype, device=gpu)
+        flat[offset:].copy_(t.reshape(-1))
+        return flat[offset:].view(t.shape)
+    rows, width, ff, experts, top = 700, 96, 136, 3, 2
+    x, up = rnd((rows, width), 1, torch.bfloat16).to(gpu), rnd((experts, ff, width), 2, torch.bfloat16, width ** -0.5).to(gpu)
+    idx = torch.rand((rows, experts), generator=torch.Generator().manual_seed(group)).argsort(-1)[:, :top].to(torch.int32).contiguous()
+    tiles = K.moe_tiles(rows * top, experts, group)
+    slot = torch.empty(tiles * K.MOE_TILE, dtype=torch.int32, device=gpu)
+    tile_expert = torch.empty(tiles, dtype=torch.int32, device=gpu)
+    K.moe_align(idx.to(gpu), experts, slot, tile_expert, group)
+    got = []
+    for dx, dw in ((0, 0), (x_at, w_at)):
+        act = torch.zeros((tiles * K.MOE_TILE, ff), dtype=torch.bfloat16, device=gpu)
+        K.moe_expert_rows(at(x, dx), at(up, dw), act, slot, tile_expert, top, activation="relu2", group=group)
+        heads = torch.zeros((rows, 3, ff), dtype=torch.bfloat16, device=gpu)
+        K.heads_matmul(at(x, dx).view(rows, 3, 32), at(rnd((3, ff, 32), 3, torch.bfloat16, 0.2), dw), heads)
+        got.append((act.double().cpu(), heads.double().cpu()))
+    for a, b in zip(*got):
+        assert a.any() and (a - b).norm() <= 2.0 ** -8 * a.norm()
+
+
 @pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
 @pytest.mark.parametrize("rows, width, ff, experts, top, shared", [(1, 64, 32, 6, 2, 48), (33, 40, 20, 3, 1, 0), (300, 128, 96, 9, 4, 64)])
 def test_table_experts_with_and_without_the_expert_every_token_uses(rows, width, ff, experts, top, shared, dtype, gpu):
