@@ -805,6 +805,152 @@ extern "C" int kva_moe_expert_rows(void *out, int out_dtype, const void *x, cons
     return KVA_OK;
 }
 
+// ---- few tokens ------------------------------------------------------------------------------
+// Up to 16 tokens: a tile has a row for every one of them, so nothing is sorted.  A workgroup takes 16 outputs of one unit: an
+// expert, or (fewer slots than experts) the expert of a slot, whose first slot's workgroups take it; one more unit is the expert
+// that every token uses, in the same launch.  Which tokens chose the expert is read from idx by the lanes themselves, or (mode 0)
+// looked up in a table by token id, in which case one workgroup leaves idx and the weights for whoever comes next.  A token's
+// choices are distinct.  The four wavefronts take a quarter of K each; all of a quarter's loads (up to 16 steps of 32) are on
+// their way at once, since a workgroup is as long as its chain of trips to memory: list, rows, matrix one after another, with
+// eight loads in flight, and a list's launch in front took the times on the left.
+//  mode 0: out[slot] = act(W[e] x[token]) (x's type),   mode 1: out[slot] = W[e] x[slot] * weight[slot] (fp32).
+struct MoeFew {
+    const int *idx;
+    MoeTable tab;
+    int *idx_out;
+    const float *slot_weight;
+    int tokens, top, experts, units, by_slot, N, K, mode, act, gated;
+    float limit;
+    const bf16_t *shared_x, *shared_w;      // rows a token; a matrix in tiles of 16 rows (first product: gates' tiles, then ups')
+    void *shared_out;
+    int shared_N, shared_K, shared_act;
+    float shared_limit;
+};
+
+__device__ inline float moe_gated(float gate, float up, int act, float limit) {
+    return act == 4 ? kva_gated_activate(gate, up, KVA_ACT_SWISH_CLAMPED, limit) : moe_activate(gate, act) * up;
+}
+
+__device__ inline uint32_t moe_pack(float a, float b) { return __builtin_bit_cast(uint32_t, pack_bf16(a, b)); }
+
+template <int AHEAD>
+__global__ void __launch_bounds__(256)
+moe_few_rows_kernel(MoeFew a, void *__restrict__ out, const bf16_t *__restrict__ x, const bf16_t *__restrict__ w) {
+    __shared__ float red[3][KVA_WAVE][4];
+    const int lane = threadIdx.x % KVA_WAVE, wave = __builtin_amdgcn_readfirstlane(threadIdx.x / KVA_WAVE), r = lane & 15, g = lane >> 4;
+    const int unit = blockIdx.y, slots = a.tokens * a.top;
+    const bool shared = unit == a.units;
+    if (a.tab.table && unit == 0 && blockIdx.x == 0)
+        for (int s = threadIdx.x; s < slots; s += 256) {
+            a.idx_out[s] = moe_slot_expert(nullptr, s, a.tab);
+            a.tab.wgt[s] = a.tab.weight;
+        }
+    const int N = shared ? a.shared_N : a.N, K = shared ? a.shared_K : a.K, n0 = 16 * blockIdx.x;
+    if (n0 >= N) return;
+    int slot = -1, e = 0;               // this lane's token's slot with the expert
+    if (shared) {
+        slot = r < a.tokens ? r : -1;
+    } else {
+        int *idx = const_cast<int *>(a.idx);
+        e = __builtin_amdgcn_readfirstlane(a.by_slot ? moe_slot_expert(idx, unit, a.tab) : unit);
+        if (r < a.tokens)
+            for (int k = g; k < a.top; k += 4)
+                if (moe_slot_expert(idx, r * a.top + k, a.tab) == e) slot = r * a.top + k;
+        slot = max(slot, __shfl_xor(slot, 16, KVA_WAVE));
+        slot = max(slot, __shfl_xor(slot, 32, KVA_WAVE));
+        const unsigned long long chose = __ballot(slot >= 0);
+        if (e < 0 || e >= a.experts || !chose) return;
+        if (a.by_slot && __shfl(slot, __ffsll(chose) - 1, KVA_WAVE) != unit) return;
+    }
+    const bool pairs = shared && a.mode == 0;       // 8 gate rows and 8 up rows of two tiles
+    const bf16_t *xrow = (shared ? a.shared_x : x) + (size_t)(shared || a.mode == 0 ? min(r, a.tokens - 1) : max(slot, 0)) * K + 8 * g;
+    const bf16_t *wrow = shared ? a.shared_w : w + (size_t)e * N * K;
+    if (pairs) wrow += (size_t)((r >> 3) * (N / 32) + n0 / 32) * 16 * K + 8 * (16 * g + n0 / 2 % 16 + (r & 7));
+    else wrow += (size_t)n0 * K + 8 * lane;
+    const int steps = K / 32, per = (steps + 3) / 4, s0 = wave * per, s1 = min(steps, s0 + per);
+    f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+    for (int s = s0; s < s1; s += AHEAD) {
+        Frag8 wf[AHEAD], xf[AHEAD];
+#pragma unroll
+        for (int i = 0; i < AHEAD; ++i) wf[i].u4 = *reinterpret_cast<const uint4 *>(wrow + (size_t)min(s + i, s1 - 1) * 512);
+#pragma unroll
+        for (int i = 0; i < AHEAD; ++i) xf[i].u4 = *reinterpret_cast<const uint4 *>(xrow + 32 * min(s + i, s1 - 1));
+#pragma unroll
+        for (int i = 0; i < AHEAD; ++i)
+            if (s + i < s1) acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf[i].v, xf[i].v, acc, 0, 0, 0);
+    }
+    if (wave > 0) *reinterpret_cast<f32x4 *>(red[wave - 1][lane]) = acc;
+    __syncthreads();
+    if (wave > 0) return;
+    float v[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) v[i] = ((acc[i] + red[0][lane][i]) + red[1][lane][i]) + red[2][lane][i];
+    if (pairs) {                        // lanes of g and g + 2: outputs n0 / 2 + 4 g .. + 3, gates and ups
+        float up[4];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) up[i] = __shfl_xor(v[i], 32, KVA_WAVE);
+        if (g >= 2 || slot < 0) return;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) v[i] = moe_gated(v[i], up[i], a.shared_act, a.shared_limit);
+        *reinterpret_cast<uint2 *>(reinterpret_cast<uint16_t *>(a.shared_out) + (size_t)slot * (N / 2) + n0 / 2 + 4 * g) =
+            make_uint2(moe_pack(v[0], v[1]), moe_pack(v[2], v[3]));
+        return;
+    }
+    if (slot < 0) return;
+    const int n = n0 + 4 * g;
+    if (a.slot_weight && !shared) {
+        const float weight = a.slot_weight[slot];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) v[i] *= weight;
+    }
+    if (a.mode == 1) {
+        *reinterpret_cast<float4 *>((shared ? reinterpret_cast<float *>(a.shared_out) : reinterpret_cast<float *>(out)) + (size_t)slot * N + n) =
+            make_float4(v[0], v[1], v[2], v[3]);
+    } else if (a.gated) {
+        *reinterpret_cast<uint32_t *>(reinterpret_cast<uint16_t *>(out) + (size_t)slot * (N / 2) + n / 2) =
+            moe_pack(moe_gated(v[0], v[1], a.act, a.limit), moe_gated(v[2], v[3], a.act, a.limit));
+    } else {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) v[i] = moe_activate(v[i], a.act);
+        *reinterpret_cast<uint2 *>(reinterpret_cast<uint16_t *>(out) + (size_t)slot * N + n) =
+            make_uint2(moe_pack(v[0], v[1]), moe_pack(v[2], v[3]));
+    }
+}
+
+extern "C" int kva_moe_few_max_tokens(void) { return 16; }
+
+extern "C" int kva_moe_few_rows(void *out, const void *x, const void *w, const int *idx, const int *table, int table_rows, int table_top,
+                                const int *ids, const int *feedback, float table_weight, int *idx_out, float *wgt_out,
+                                int tokens, int top, int experts, int N, int K, int mode, int act, int gated, float limit,
+                                const float *slot_weight, const void *shared_x, const void *shared_w, void *shared_out,
+                                int shared_N, int shared_K, int shared_act, float shared_limit, hipStream_t stream) {
+    KVA_REQUIRE(out && x && w && (idx || table) && tokens >= 0 && tokens <= 16 && top > 0 && experts > 0,
+                "moe_few_rows: missing operand, or more than 16 tokens (%d)", tokens);
+    KVA_REQUIRE(N > 0 && N % 16 == 0 && K > 0 && K % 32 == 0, "moe_few_rows: no operand order for %d x %d", N, K);
+    KVA_REQUIRE(mode == 0 || mode == 1, "moe_few_rows: the first product (0) or the second (1)");
+    KVA_REQUIRE(!table || (mode == 0 && ids && idx_out && wgt_out && table_rows > 0 && table_top == top),
+                "moe_few_rows: a table goes with the first product, with ids and places for what it says");
+    KVA_REQUIRE(act >= 0 && act <= 5 && (act != 4 || gated) && (!gated || mode == 0), "moe_few_rows: bad activation");
+    KVA_REQUIRE(!shared_w || (shared_x && shared_out && shared_N > 0 && shared_N % (mode == 0 ? 32 : 16) == 0 && shared_K > 0 && shared_K % 32 == 0 &&
+                              shared_act >= 0 && shared_act <= 5),
+                "moe_few_rows: no operand order for %d x %d of the expert every token uses", shared_N, shared_K);
+    KVA_REQUIRE((((uintptr_t)out | (uintptr_t)x | (uintptr_t)w | (uintptr_t)shared_x | (uintptr_t)shared_w | (uintptr_t)shared_out) & 15) == 0,
+                "moe_few_rows: operands start at multiples of 16 bytes");
+    if (tokens == 0) return KVA_OK;
+    const int slots = tokens * top, by_slot = slots < experts, units = by_slot ? slots : experts;
+    KVA_REQUIRE(units < 65535, "moe_few_rows: too many workgroups");
+    const MoeFew a{idx, MoeTable{table, ids, feedback, table_rows, top, table_weight, wgt_out}, idx_out, slot_weight, tokens, top, experts,
+                   units, by_slot, N, K, mode, act, gated, limit, (const bf16_t *)shared_x, (const bf16_t *)shared_w, shared_out, shared_N,
+                   shared_K, shared_act, shared_limit};
+    const int wide = shared_w && shared_N > N ? shared_N : N, deep = shared_w && shared_K > K ? shared_K : K, per = (deep / 32 + 3) / 4;
+    const dim3 grid((wide + 15) / 16, units + (shared_w ? 1 : 0));
+    if (per > 8) hipLaunchKernelGGL(moe_few_rows_kernel<16>, grid, dim3(256), 0, stream, a, out, (const bf16_t *)x, (const bf16_t *)w);
+    else if (per > 4) hipLaunchKernelGGL(moe_few_rows_kernel<8>, grid, dim3(256), 0, stream, a, out, (const bf16_t *)x, (const bf16_t *)w);
+    else hipLaunchKernelGGL(moe_few_rows_kernel<4>, grid, dim3(256), 0, stream, a, out, (const bf16_t *)x, (const bf16_t *)w);
+    KVA_CHECK_LAUNCH("moe_few_rows");
+    return KVA_OK;
+}
+
 // ---- weighted sum --------------------------------------------------------------------------
 __device__ inline float moe_ld(const void *p, int dtype, size_t i) {
     return dtype == KVA_BF16 ? bf16_bits_to_float(reinterpret_cast<const uint16_t *>(p)[i])
@@ -813,7 +959,7 @@ __device__ inline float moe_ld(const void *p, int dtype, size_t i) {
 
 __global__ void __launch_bounds__(256)
 moe_combine_kernel(void *__restrict__ out, const void *__restrict__ x, int dtype, const float *__restrict__ rows,
-                   const int *__restrict__ idx, const float *__restrict__ wgt, const void *__restrict__ extra,
+                   const int *__restrict__ idx, const float *__restrict__ wgt, const void *__restrict__ extra, int extra_dtype,
                    const float *__restrict__ extra_gate, int extra_gate_stride, int width, int top, int experts) {
     const size_t t = blockIdx.x;
     // (optional) the addend enters times sigmoid(extra_gate[t * stride]), one number a token (a column of a wider array)
@@ -836,7 +982,7 @@ moe_combine_kernel(void *__restrict__ out, const void *__restrict__ x, int dtype
             }
             if (extra) {
 #pragma unroll
-                for (int e = 0; e < 4; ++e) acc[e] += eg * moe_ld(extra, dtype, t * width + j + e);
+                for (int e = 0; e < 4; ++e) acc[e] += eg * moe_ld(extra, extra_dtype, t * width + j + e);
             }
             if (dtype == KVA_BF16) {
                 const uint2 o = make_uint2((uint32_t)float_to_bf16_bits(acc[0]) | ((uint32_t)float_to_bf16_bits(acc[1]) << 16),
@@ -857,20 +1003,19 @@ moe_combine_kernel(void *__restrict__ out, const void *__restrict__ x, int dtype
                                                     : reinterpret_cast<const float *>(x)[t * width + j]);
         }
         // what an expert that every token uses returned, with weight 1
-        if (extra) acc += eg * (dtype == KVA_BF16 ? bf16_bits_to_float(reinterpret_cast<const uint16_t *>(extra)[t * width + j])
-                                                  : reinterpret_cast<const float *>(extra)[t * width + j]);
+        if (extra) acc += eg * moe_ld(extra, extra_dtype, t * width + j);
         if (dtype == KVA_BF16) reinterpret_cast<uint16_t *>(out)[t * width + j] = float_to_bf16_bits(acc);
         else reinterpret_cast<float *>(out)[t * width + j] = acc;
     }
 }
 
 extern "C" int kva_moe_combine(void *out, const void *x, int dtype, const float *rows, const int *idx,
-                               const float *wgt, const void *extra, const float *extra_gate, int extra_gate_stride,
+                               const float *wgt, const void *extra, int extra_dtype, const float *extra_gate, int extra_gate_stride,
                                int tokens, int width, int top, int experts, hipStream_t stream) {
     KVA_REQUIRE(out && x && rows && idx && wgt && width > 0 && top > 0, "moe_combine: missing operand");
     KVA_REQUIRE(dtype == KVA_BF16 || dtype == KVA_F32, "moe_combine: unsupported dtype %d", dtype);
     if (tokens <= 0) return KVA_OK;
-    hipLaunchKernelGGL(moe_combine_kernel, dim3(tokens), dim3(256), 0, stream, out, x, dtype, rows, idx, wgt, extra, extra_gate,
+    hipLaunchKernelGGL(moe_combine_kernel, dim3(tokens), dim3(256), 0, stream, out, x, dtype, rows, idx, wgt, extra, extra_dtype, extra_gate,
                        extra_gate_stride, width, top, experts);
     KVA_CHECK_LAUNCH("moe_combine");
     return KVA_OK;

@@ -19,14 +19,48 @@ __device__ inline void st_from_float(void *p, int dtype, size_t i, float v) {
     else reinterpret_cast<uint16_t *>(p)[i] = float_to_bf16_bits(v);
 }
 
+// A branch output that is still the rows of routed experts: y[t] = sum_k rows[t top + k] (+ sigmoid(gate[t]) extra[t]).  The
+// kernels that let a branch output into the stream form it on the way, in 32 bits: a launch of its own for the sum wrote it
+// rounded and read it back (2,048 tokens of 2,048, four choices: 13-15 us of 27-32 with the norm behind it; one token: 4.8 of 9.5).
+struct ExpertSum {
+    const float *rows, *gate;
+    int top, gate_stride;
+};
+
+// W neighbouring columns from j on of row t; y: the extra row's elements (zeros without one) on the way in, the sum on the way out
+template <int W>
+__device__ inline void expert_sum(const ExpertSum &er, bool extra, size_t t, int width, int j, float (&y)[W]) {
+    const float eg = extra && er.gate ? 1.f / (1.f + expf(-er.gate[t * er.gate_stride])) : 1.f;
+    float sum[W];
+#pragma unroll
+    for (int e = 0; e < W; ++e) sum[e] = 0.f;
+    const float *row = er.rows + t * er.top * width + j;
+#pragma unroll 4
+    for (int k = 0; k < er.top; ++k, row += width) {
+        if constexpr (W % 4 == 0) {
+#pragma unroll
+            for (int e = 0; e < W; e += 4) {
+                const float4 f = *reinterpret_cast<const float4 *>(row + e);
+                sum[e] += f.x; sum[e + 1] += f.y; sum[e + 2] += f.z; sum[e + 3] += f.w;
+            }
+        } else {
+#pragma unroll
+            for (int e = 0; e < W; ++e) sum[e] += row[e];
+        }
+    }
+#pragma unroll
+    for (int e = 0; e < W; ++e) y[e] = sum[e] + (extra ? eg * y[e] : 0.f);
+}
+
 // One workgroup per output row.  x <- x + d1 + d2 (written back unless rows are gathered), then
 // out_k = (x - mean) / sqrt(var + eps) * w_k with the variance as the mean of squared deviations.
-// With rms != 0 the mean is not taken off: out_k = x / sqrt(mean(x^2) + eps) * w_k.
+// With rms != 0 the mean is not taken off: out_k = x / sqrt(mean(x^2) + eps) * w_k.  With `er` the second
+// addend is what routed experts returned (d2 then is its extra row, or absent).
 __global__ void __launch_bounds__(256)
 layernorm_kernel(void *__restrict__ out1, void *__restrict__ out2, int out_dtype, void *__restrict__ x, int x_dtype,
                  const void *__restrict__ d1, int d1_dtype, const void *__restrict__ d2, int d2_dtype,
                  const void *__restrict__ w1, const void *__restrict__ w2, int w_dtype,
-                 const int *__restrict__ row_idx, int width, float eps, int rms, float delta_scale) {
+                 const int *__restrict__ row_idx, int width, float eps, int rms, float delta_scale, ExpertSum er) {
     extern __shared__ float row_s[];
     __shared__ float red_s[4];
     const int r = blockIdx.x;
@@ -34,18 +68,20 @@ layernorm_kernel(void *__restrict__ out1, void *__restrict__ out2, int out_dtype
     float sum = 0.f;
     for (int j = threadIdx.x; j < width; j += blockDim.x) {
         float v = ld_as_float(x, x_dtype, src + j);
+        const bool two = d2 || er.rows;
+        float b[1] = {d2 ? ld_as_float(d2, d2_dtype, src + j) : 0.f};
+        if (er.rows) expert_sum<1>(er, d2 != nullptr, src / width, width, j, b);
         if (delta_scale == 1.0f) {
             if (d1) v += ld_as_float(d1, d1_dtype, src + j);
-            if (d2) v += ld_as_float(d2, d2_dtype, src + j);
-        } else if (d1 || d2) {
+            if (two) v += b[0];
+        } else if (d1 || two) {
             // the branch outputs are added up first, and their sum enters the stream times a constant
-            const float b = (d1 ? ld_as_float(d1, d1_dtype, src + j) : 0.f) + (d2 ? ld_as_float(d2, d2_dtype, src + j) : 0.f);
-            v += delta_scale * b;
+            v += delta_scale * ((d1 ? ld_as_float(d1, d1_dtype, src + j) : 0.f) + b[0]);
         }
-        if ((d1 || d2) && !row_idx) {
+        if ((d1 || two) && !row_idx) {
             st_from_float(x, x_dtype, src + j, v);
             v = ld_as_float(x, x_dtype, src + j);       // what the stream holds from now on
-        } else if (d1 || d2) {
+        } else if (d1 || two) {
             if (x_dtype == KVA_BF16) v = bf16_bits_to_float(float_to_bf16_bits(v));
         }
         row_s[j] = v;
@@ -105,7 +141,7 @@ __global__ void __launch_bounds__(256)
 layernorm_vec_kernel(void *__restrict__ out1, void *__restrict__ out2, int out_dtype, void *__restrict__ x, int x_dtype,
                      const void *__restrict__ d1, int d1_dtype, const void *__restrict__ d2, int d2_dtype,
                      const void *__restrict__ w1, const void *__restrict__ w2, int w_dtype,
-                     const int *__restrict__ row_idx, int width, float eps, int rms, float delta_scale) {
+                     const int *__restrict__ row_idx, int width, float eps, int rms, float delta_scale, ExpertSum er) {
     __shared__ float red_s[4];
     const int r = blockIdx.x;
     const size_t src = (size_t)(row_idx ? row_idx[r] : r) * width, dst = (size_t)r * width;
@@ -118,12 +154,13 @@ layernorm_vec_kernel(void *__restrict__ out1, void *__restrict__ out2, int out_d
         for (int i = 0; i < 8; ++i) v[c][i] = 0.f;
         if (j >= width) continue;
         ld8_as_float(x, x_dtype, src + j, v[c]);
-        if (d1 || d2) {
+        if (d1 || d2 || er.rows) {
             float a[8], b[8];
 #pragma unroll
             for (int i = 0; i < 8; ++i) a[i] = b[i] = 0.f;
             if (d1) ld8_as_float(d1, d1_dtype, src + j, a);
             if (d2) ld8_as_float(d2, d2_dtype, src + j, b);
+            if (er.rows) expert_sum<8>(er, d2 != nullptr, src / width, width, j, b);
 #pragma unroll
             for (int i = 0; i < 8; ++i) {
                 // (scaled: the branch outputs are added up first, and their sum enters the stream times a constant)
@@ -169,16 +206,20 @@ layernorm_vec_kernel(void *__restrict__ out1, void *__restrict__ out2, int out_d
 extern "C" int kva_layernorm(void *out1, void *out2, int out_dtype, void *x, int x_dtype, const void *d1,
                              int d1_dtype, const void *d2, int d2_dtype, const void *w1, const void *w2,
                              int w_dtype, const int *row_idx, int rows, int width, float eps, int rms,
-                             float delta_scale, hipStream_t stream) {
+                             float delta_scale, const float *expert_rows, const float *gate, int top, int gate_stride,
+                             hipStream_t stream) {
+    KVA_REQUIRE(!expert_rows || (top > 0 && gate_stride >= 0), "layernorm: experts' rows come so many a token");
     KVA_REQUIRE(rows >= 0 && width > 0 && width <= 16000, "layernorm: width %d must lie in 1..16000", width);
     KVA_REQUIRE(out1 && x && w1 && (out2 == nullptr) == (w2 == nullptr), "layernorm: an output without its weight");
     KVA_REQUIRE(eps >= 0.f, "layernorm: negative eps");
     if (rows == 0) return KVA_OK;
-    const uintptr_t all = (uintptr_t)out1 | (uintptr_t)out2 | (uintptr_t)x | (uintptr_t)d1 | (uintptr_t)d2 | (uintptr_t)w1 | (uintptr_t)w2;
+    const ExpertSum er{expert_rows, gate, top, gate_stride};
+    const uintptr_t all = (uintptr_t)out1 | (uintptr_t)out2 | (uintptr_t)x | (uintptr_t)d1 | (uintptr_t)d2 | (uintptr_t)w1 |
+                          (uintptr_t)w2 | (uintptr_t)expert_rows;
     if (width % 8 == 0 && width <= 8192 && all % 16 == 0) {
 #define KVA_LAYERNORM_VEC(PER)                                                                                          \
     hipLaunchKernelGGL(layernorm_vec_kernel<PER>, dim3(rows), dim3(256), 0, stream, out1, out2, out_dtype, x, x_dtype, d1,  \
-                       d1_dtype, d2, d2_dtype, w1, w2, w_dtype, row_idx, width, eps, rms, delta_scale)
+                       d1_dtype, d2, d2_dtype, w1, w2, w_dtype, row_idx, width, eps, rms, delta_scale, er)
         if (width <= 2048) KVA_LAYERNORM_VEC(1);
         else if (width <= 4096) KVA_LAYERNORM_VEC(2);
         else KVA_LAYERNORM_VEC(4);
@@ -187,7 +228,7 @@ extern "C" int kva_layernorm(void *out1, void *out2, int out_dtype, void *x, int
         return KVA_OK;
     }
     hipLaunchKernelGGL(layernorm_kernel, dim3(rows), dim3(256), (size_t)width * sizeof(float), stream, out1, out2,
-                       out_dtype, x, x_dtype, d1, d1_dtype, d2, d2_dtype, w1, w2, w_dtype, row_idx, width, eps, rms, delta_scale);
+                       out_dtype, x, x_dtype, d1, d1_dtype, d2, d2_dtype, w1, w2, w_dtype, row_idx, width, eps, rms, delta_scale, er);
     KVA_CHECK_LAUNCH("layernorm");
     return KVA_OK;
 }
@@ -760,7 +801,7 @@ extern "C" int kva_hyper_fill(float *x, const void *first, int dtype, int stream
 // enter goes through its norm into the stream, an optional second addend (fp32, as it is) follows it, and
 // the new row is normed for the next branch.  n(v) = (v - mean) / sqrt(mean((v - mean)^2) + eps) * w (+ b);
 // without `center` the mean is not taken off.  Without a post weight y enters as it is; without `out` the
-// stream is only updated.  With row_idx only the named rows are read, and nothing is written back: the
+// stream is only updated.  With `er` the branch output is what routed experts returned (y then is its extra row, or absent).  With row_idx only the named rows are read, and nothing is written back: the
 // model's last norm.
 struct SideNorm {
     const void *w, *b;
@@ -771,19 +812,25 @@ struct SideNorm {
 __global__ void __launch_bounds__(256)
 sandwich_step_kernel(float *__restrict__ x, const void *__restrict__ y, int y_dtype, SideNorm post,
                      const float *__restrict__ addend, SideNorm pre, void *__restrict__ out, int out_dtype,
-                     const int *__restrict__ row_idx, int width) {
+                     const int *__restrict__ row_idx, int width, ExpertSum er) {
     extern __shared__ float row_s[];
     __shared__ float red_s[4];
     const int r = blockIdx.x, waves = blockDim.x / KVA_WAVE;
     const size_t row = (size_t)(row_idx ? row_idx[r] : r) * width;
+    const bool enters = y || er.rows;
+    auto branch = [&](int j) {                      // the branch output's element j
+        float b[1] = {y ? ld_as_float(y, y_dtype, row + j) : 0.f};
+        if (er.rows) expert_sum<1>(er, y != nullptr, row / width, width, j, b);
+        return b[0];
+    };
     float mean = 0.f, inv = 1.f;
-    if (y && post.w) {
+    if (enters && post.w) {
         float sum = 0.f;
-        for (int j = threadIdx.x; j < width; j += blockDim.x) sum += ld_as_float(y, y_dtype, row + j);
+        for (int j = threadIdx.x; j < width; j += blockDim.x) sum += branch(j);
         if (post.center) mean = block_sum(sum, red_s, waves) / (float)width;
         float sq = 0.f;
         for (int j = threadIdx.x; j < width; j += blockDim.x) {
-            const float d = ld_as_float(y, y_dtype, row + j) - mean;
+            const float d = branch(j) - mean;
             sq += d * d;
         }
         inv = 1.0f / sqrtf(block_sum(sq, red_s, waves) / (float)width + post.eps);
@@ -791,13 +838,13 @@ sandwich_step_kernel(float *__restrict__ x, const void *__restrict__ y, int y_dt
     float sum = 0.f;
     for (int j = threadIdx.x; j < width; j += blockDim.x) {
         float v = x[row + j];
-        if (y) {
-            const float yv = ld_as_float(y, y_dtype, row + j);
+        if (enters) {
+            const float yv = branch(j);
             v += post.w ? (yv - mean) * inv * ld_as_float(post.w, post.w_dtype, j) + (post.b ? ld_as_float(post.b, post.w_dtype, j) : 0.f)
                         : yv;
         }
         if (addend) v += addend[row + j];
-        if (!row_idx && (y || addend)) x[row + j] = v;
+        if (!row_idx && (enters || addend)) x[row + j] = v;
         row_s[j] = v;
         sum += v;
     }
@@ -834,13 +881,13 @@ template <int THREADS, int ITERS>
 __global__ void __launch_bounds__(THREADS)
 sandwich_step_vec_kernel(float *__restrict__ x, const void *__restrict__ y, int y_dtype, SideNorm post,
                          const float *__restrict__ addend, SideNorm pre, void *__restrict__ out, int out_dtype,
-                         const int *__restrict__ row_idx, int width) {
+                         const int *__restrict__ row_idx, int width, ExpertSum er) {
     constexpr int WAVES = THREADS / KVA_WAVE;
     __shared__ float red_s[4][WAVES];
     const int r = blockIdx.x;
     const size_t row = (size_t)(row_idx ? row_idx[r] : r) * width;
     float v[ITERS][4], yv[ITERS][4], av[ITERS][4], pw[ITERS][4], pb[ITERS][4], nw[ITERS][4], nb[ITERS][4];
-    const bool norm_y = y && post.w;
+    const bool enters = y || er.rows, norm_y = enters && post.w;
 #pragma unroll
     for (int it = 0; it < ITERS; ++it) {
         const int j = (threadIdx.x + it * THREADS) * 4;
@@ -849,6 +896,7 @@ sandwich_step_vec_kernel(float *__restrict__ x, const void *__restrict__ y, int 
         if (j >= width) continue;
         hyper_ld4(x, KVA_F32, row + j, v[it]);
         if (y) hyper_ld4(y, y_dtype, row + j, yv[it]);
+        if (er.rows) expert_sum<4>(er, y != nullptr, row / width, width, j, yv[it]);
         if (addend) hyper_ld4(addend, KVA_F32, row + j, av[it]);
         if (norm_y) hyper_ld4(post.w, post.w_dtype, j, pw[it]);
         if (norm_y && post.b) hyper_ld4(post.b, post.w_dtype, j, pb[it]);
@@ -888,7 +936,7 @@ sandwich_step_vec_kernel(float *__restrict__ x, const void *__restrict__ y, int 
             v[it][e] = (v[it][e] + yv[it][e]) + av[it][e];
             sum += v[it][e];
         }
-        if (!row_idx && (y || addend) && j < width)
+        if (!row_idx && (enters || addend) && j < width)
             *reinterpret_cast<float4 *>(x + row + j) = make_float4(v[it][0], v[it][1], v[it][2], v[it][3]);
     }
     if (!out) return;
@@ -924,23 +972,26 @@ sandwich_step_vec_kernel(float *__restrict__ x, const void *__restrict__ y, int 
 extern "C" int kva_sandwich_step(float *x, const void *y, int y_dtype, const void *post_w, const void *post_b, int post_dtype,
                                  int post_center, float post_eps, const float *addend, const void *pre_w, const void *pre_b,
                                  int pre_dtype, int pre_center, float pre_eps, void *out, int out_dtype, const int *row_idx,
-                                 int rows, int width, hipStream_t stream) {
+                                 int rows, int width, const float *expert_rows, const float *gate, int top, int gate_stride,
+                                 hipStream_t stream) {
     KVA_REQUIRE(x && rows >= 0 && width > 0 && width <= 16000, "sandwich_step: width %d must lie in 1..16000", width);
-    KVA_REQUIRE(y || (!post_w && !post_b), "sandwich_step: a norm without the branch output it norms");
+    KVA_REQUIRE(!expert_rows || (top > 0 && gate_stride >= 0), "sandwich_step: experts' rows come so many a token");
+    KVA_REQUIRE(y || expert_rows || (!post_w && !post_b), "sandwich_step: a norm without the branch output it norms");
     KVA_REQUIRE(!post_b || post_w, "sandwich_step: a norm's bias without its weight");
     KVA_REQUIRE(!out || (pre_w && pre_eps >= 0.f), "sandwich_step: the read-out needs a norm");
     KVA_REQUIRE(post_eps >= 0.f, "sandwich_step: negative eps");
-    KVA_REQUIRE(y || addend || out, "sandwich_step: nothing to do");
+    KVA_REQUIRE(y || expert_rows || addend || out, "sandwich_step: nothing to do");
     KVA_REQUIRE(!row_idx || out, "sandwich_step: rows are gathered for the read-out only");
     if (rows == 0) return KVA_OK;
     const SideNorm post{post_w, post_b, post_dtype, post_center, post_eps}, pre{pre_w, pre_b, pre_dtype, pre_center, pre_eps};
+    const ExpertSum er{expert_rows, gate, top, gate_stride};
     // (which kernel runs depends on width and alignment alone, never on the rows: a row's numbers are the same in any batch)
     const bool aligned = aligned16(x) && aligned16(y) && aligned16(post_w) && aligned16(post_b) && aligned16(addend) &&
-                         aligned16(pre_w) && aligned16(pre_b) && aligned16(out);
+                         aligned16(pre_w) && aligned16(pre_b) && aligned16(out) && aligned16(expert_rows);
     if (width % 4 == 0 && width <= 8192 && aligned) {
 #define KVA_SANDWICH(THREADS, ITERS)                                                                                     \
     hipLaunchKernelGGL((sandwich_step_vec_kernel<THREADS, ITERS>), dim3(rows), dim3(THREADS), 0, stream, x, y, y_dtype,  \
-                       post, addend, pre, out, out_dtype, row_idx, width)
+                       post, addend, pre, out, out_dtype, row_idx, width, er)
         if (width <= 1024) KVA_SANDWICH(256, 1);
         else if (width <= 2048) KVA_SANDWICH(512, 1);
         else if (width <= 4096) KVA_SANDWICH(512, 2);
@@ -948,7 +999,7 @@ extern "C" int kva_sandwich_step(float *x, const void *y, int y_dtype, const voi
 #undef KVA_SANDWICH
     } else {
         hipLaunchKernelGGL(sandwich_step_kernel, dim3(rows), dim3(256), (size_t)width * sizeof(float), stream, x, y, y_dtype, post,
-                           addend, pre, out, out_dtype, row_idx, width);
+                           addend, pre, out, out_dtype, row_idx, width, er);
     }
     KVA_CHECK_LAUNCH("sandwich_step");
     return KVA_OK;
@@ -969,15 +1020,10 @@ struct TanhNorm {
     float alpha;
 };
 
-struct TanhRows {
-    const float *rows, *gate;
-    int top, gate_stride;
-};
-
 template <bool VEC>
 __global__ void __launch_bounds__(256)
 tanh_step_kernel(float *__restrict__ x, const void *__restrict__ y, int y_dtype, const float *__restrict__ y_bias,
-                 TanhRows er, TanhNorm post, TanhNorm pre, void *__restrict__ out, int out_dtype, const int *__restrict__ row_idx,
+                 ExpertSum er, TanhNorm post, TanhNorm pre, void *__restrict__ out, int out_dtype, const int *__restrict__ row_idx,
                  int width, size_t n) {
     constexpr int W = VEC ? 4 : 1;
     const size_t i = ((size_t)blockIdx.x * blockDim.x + threadIdx.x) * W;
@@ -996,21 +1042,7 @@ tanh_step_kernel(float *__restrict__ x, const void *__restrict__ y, int y_dtype,
     const bool enters = y || er.rows;
     if (enters) {
         if (y) load(y, y_dtype, at, yv);
-        if (er.rows) {
-            const size_t t = at / width;
-            const float eg = y && er.gate ? 1.f / (1.f + expf(-er.gate[t * er.gate_stride])) : 1.f;
-            float sum[W];
-#pragma unroll
-            for (int e = 0; e < W; ++e) sum[e] = 0.f;
-            for (int k = 0; k < er.top; ++k) {
-                float f[W];
-                load(er.rows, KVA_F32, (t * er.top + k) * width + j, f);
-#pragma unroll
-                for (int e = 0; e < W; ++e) sum[e] += f[e];
-            }
-#pragma unroll
-            for (int e = 0; e < W; ++e) yv[e] = sum[e] + (y ? eg * yv[e] : 0.f);
-        }
+        if (er.rows) expert_sum<W>(er, y != nullptr, at / width, width, j, yv);
         if (y_bias) load(y_bias, KVA_F32, j, yb);
         if (post.w) {
             load(post.w, post.dtype, j, pw);
@@ -1060,7 +1092,7 @@ extern "C" int kva_tanh_step(float *x, const void *y, int y_dtype, const float *
     if (rows == 0) return KVA_OK;
     const TanhNorm post{post_w, post_b, post_dtype, post_alpha}, pre{pre_w, pre_b, pre_dtype, pre_alpha};
     const size_t n = (size_t)rows * width;
-    const TanhRows er{expert_rows, gate, top, gate_stride};
+    const ExpertSum er{expert_rows, gate, top, gate_stride};
     const bool vec = width % 4 == 0 && aligned16(x) && aligned16(y) && aligned16(y_bias) && aligned16(expert_rows) && aligned16(post_w) &&
                      aligned16(post_b) && aligned16(pre_w) && aligned16(pre_b) && aligned16(out);
     if (vec)

@@ -316,6 +316,7 @@ class Model:
                         raise TypeError("an operation between layers adds pending branch outputs as they are, not times "
                                         "a constant or under a norm")
                     pending = () if delta is None else (tuple(delta) if isinstance(delta, (tuple, list)) else (delta,))
+                    pending = tuple(K.added_up(d) for d in pending)
                     hidden, delta = op.forward(hidden, pending, first[id(op)]), None
             # the norm that reads the residual stream after this block
             if i + 1 == len(self.calls):

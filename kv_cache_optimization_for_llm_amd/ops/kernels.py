@@ -533,8 +533,8 @@ def layernorm(x: torch.Tensor, weight: torch.Tensor, eps: float, out: torch.Tens
               out2: Optional[torch.Tensor] = None, rms: bool = False, delta_scale: float = 1.0) -> torch.Tensor:
     """``out = (x - mean) / sqrt(var + eps) * weight`` per row (``rms``: without taking the mean
     off).  ``deltas`` (up to two tensors of x's shape, any of the two storage types) are added to
-    ``x`` first, in place (not written back when ``row_idx`` gathers rows); with a ``delta_scale``
-    other than 1 their sum is multiplied by it before it enters ``x``.  ``weight2`` / ``out2``:
+    ``x`` first, in place (not written back when ``row_idx`` gathers rows); one of them may be
+    :class:`ExpertRows`, whose sum is formed on the way; with a ``delta_scale`` other than 1 their sum is multiplied by it before it enters ``x``.  ``weight2`` / ``out2``:
     a second normalised copy with another weight from the same statistics.  ``x`` may be fp32
     while ``out`` is bf16."""
     width = x.shape[-1]
@@ -550,21 +550,26 @@ def layernorm(x: torch.Tensor, weight: torch.Tensor, eps: float, out: torch.Tens
     for d in deltas:
         if d.shape != x.shape:
             raise KernelError("layernorm: a delta must have x's shape")
-    d1 = deltas[0] if deltas else None
-    d2 = deltas[1] if len(deltas) > 1 else None
+    d1, d2, experts = None, None, [d for d in deltas if isinstance(d, ExpertRows)]
+    if len(experts) > 1:
+        raise KernelError("layernorm: one branch output of experts' rows, the other added up")
+    if experts:
+        d1, d2 = next((d for d in deltas if d is not experts[0]), None), experts[0].extra
+    elif deltas:
+        d1, d2 = deltas[0], (deltas[1] if len(deltas) > 1 else None)
     check(hip_lib().kva_layernorm(
         _dev(out, "out"), _opt(out2, "out2"), dtype_code(out.dtype), _dev(x, "x"), dtype_code(x.dtype),
         _opt(d1, "delta"), dtype_code(d1.dtype) if d1 is not None else 0,
         _opt(d2, "delta"), dtype_code(d2.dtype) if d2 is not None else 0,
         _dev(weight, "weight"), _opt(weight2, "weight2"), dtype_code(weight.dtype),
         _opt(row_idx, "row_idx", torch.int32), rows, width, float(eps), 1 if rms else 0, float(delta_scale),
-        _stream()), "layernorm")
+        *_expert_rows_args(experts[0] if experts else None), _stream()), "layernorm")
     return out
 
 
 def stream_join(x: torch.Tensor, other: torch.Tensor, out: torch.Tensor, deltas=()) -> torch.Tensor:
     """``out[t] = [x[t] + deltas ; other[t]]`` in out's type; ``x`` takes the sum in place."""
-    deltas = [d for d in deltas if d is not None]
+    deltas = [added_up(d) for d in deltas if d is not None]
     rows, wx = x.shape
     if other.dim() != 2 or other.shape[0] != rows or out.shape != (rows, wx + other.shape[1]) or len(deltas) > 2 \
             or any(d.shape != x.shape for d in deltas):
@@ -695,18 +700,21 @@ def sandwich_step(x: torch.Tensor, *, y: Optional[torch.Tensor] = None, post=Non
     """What lies between two branches that have norms on both sides, over a residual stream ``x`` fp32 ``[T,
     width]``: ``x += n_post(y) (+ addend)``, then ``out = n_pre(x)``.  ``post`` and ``pre`` are ``(weight, bias or
     None, eps, center)``: ``(v - mean) / sqrt(var + eps) * weight + bias``, without ``center`` the mean is not taken
-    off.  Without ``post`` the branch output enters as it is; ``addend`` (fp32) always does.  ``row_idx``: only
-    these rows are read out, and nothing is written back."""
+    off.  Without ``post`` the branch output enters as it is; ``addend`` (fp32) always does.  ``y`` may be
+    :class:`ExpertRows`: the sum is formed on the way.  ``row_idx``: only these rows are read out, and nothing is
+    written back."""
     T, width = x.shape
     if x.dim() != 2 or x.dtype != torch.float32:
         raise KernelError(f"sandwich_step: x {tuple(x.shape)} is not an fp32 [T, width] stream")
     if (y is not None and y.shape != x.shape) or (addend is not None and (addend.shape != x.shape or addend.dtype != torch.float32)):
         raise KernelError("sandwich_step: the branch output and the addend (fp32) have the stream's shape")
+    experts = y if isinstance(y, ExpertRows) else None
+    enters, y = y is not None, experts.extra if experts is not None else y
     for norm in (post, pre):
         if norm is not None and (norm[0].shape != (width,) or (norm[1] is not None and (
                 norm[1].shape != (width,) or norm[1].dtype != norm[0].dtype))):
             raise KernelError("sandwich_step: a norm has a weight [width] and a bias of its shape and type, or none")
-    if (post is not None and y is None) or (out is None) != (pre is None):
+    if (post is not None and not enters) or (out is None) != (pre is None):
         raise KernelError("sandwich_step: the first norm goes with a branch output, the second with an output")
     rows = T
     if out is not None:
@@ -724,7 +732,7 @@ def sandwich_step(x: torch.Tensor, *, y: Optional[torch.Tensor] = None, post=Non
     check(hip_lib().kva_sandwich_step(
         _dev(x, "x"), _opt(y, "y"), dtype_code(y.dtype) if y is not None else 0, *args(post, "post norm"), _opt(addend, "addend"),
         *args(pre, "pre norm"), _opt(out, "out"), dtype_code(out.dtype) if out is not None else 0,
-        _opt(row_idx, "row_idx", torch.int32), rows, width, _stream()), "sandwich_step")
+        _opt(row_idx, "row_idx", torch.int32), rows, width, *_expert_rows_args(experts), _stream()), "sandwich_step")
     return out
 
 
@@ -740,19 +748,14 @@ def tanh_step(x: torch.Tensor, *, y: Optional[torch.Tensor] = None, y_bias: Opti
         raise KernelError(f"tanh_step: x {tuple(x.shape)} is not an fp32 [T, width] stream")
     if y is not None and y.shape != x.shape:
         raise KernelError("tanh_step: the branch output has the stream's shape")
-    rows_of, gate, top, gate_stride = None, None, 0, 0
-    if isinstance(y, ExpertRows):
-        if y.rows.shape != (T * y.top, width) or y.rows.dtype != torch.float32:
-            raise KernelError(f"tanh_step: experts' rows {tuple(y.rows.shape)} are not fp32 [T * top, width]")
-        rows_of, top = y.rows, y.top
-        gate, gate_stride = y.gate_column()
-        y = y.extra
-    if y_bias is not None and ((y is None and rows_of is None) or y_bias.shape != (width,) or y_bias.dtype != torch.float32):
+    experts = y if isinstance(y, ExpertRows) else None
+    enters, y = y is not None, experts.extra if experts is not None else y
+    if y_bias is not None and (not enters or y_bias.shape != (width,) or y_bias.dtype != torch.float32):
         raise KernelError("tanh_step: a product's bias is fp32 [width] and goes with the product")
     for norm in (post, pre):
         if norm is not None and (norm[0].shape != (width,) or norm[1].shape != (width,) or norm[1].dtype != norm[0].dtype):
             raise KernelError("tanh_step: a norm has a weight [width] and a bias of its shape and type")
-    if (post is not None and y is None and rows_of is None) or (out is None) != (pre is None):
+    if (post is not None and not enters) or (out is None) != (pre is None):
         raise KernelError("tanh_step: the first norm goes with a branch output, the second with an output")
     rows = T
     if out is not None:
@@ -770,8 +773,7 @@ def tanh_step(x: torch.Tensor, *, y: Optional[torch.Tensor] = None, y_bias: Opti
     check(hip_lib().kva_tanh_step(
         _dev(x, "x"), _opt(y, "y"), dtype_code(y.dtype) if y is not None else 0, _opt(y_bias, "y_bias"), *args(post, "post norm"),
         *args(pre, "pre norm"), _opt(out, "out"), dtype_code(out.dtype) if out is not None else 0,
-        _opt(row_idx, "row_idx", torch.int32), rows, width, _opt(rows_of, "rows"),
-        None if gate is None else _dev(gate, "gate", torch.float32, contiguous=False), top, int(gate_stride), _stream()), "tanh_step")
+        _opt(row_idx, "row_idx", torch.int32), rows, width, *_expert_rows_args(experts), _stream()), "tanh_step")
     return out
 
 
@@ -2290,6 +2292,50 @@ def moe_expert_rows(x: torch.Tensor, w: torch.Tensor, out: torch.Tensor, sorted_
     return out
 
 
+def moe_few_max_tokens() -> int:
+    """Up to so many tokens :func:`moe_few_rows` takes."""
+    return int(hip_lib().kva_moe_few_max_tokens())
+
+
+def moe_few_rows(x: torch.Tensor, w: torch.Tensor, out: torch.Tensor, idx: torch.Tensor, *, activation: Optional[str] = None,
+                 slot_weight: Optional[torch.Tensor] = None, gated: bool = False, limit: float = 0.0, table=None,
+                 shared=None) -> torch.Tensor:
+    """:func:`moe_expert_rows` for a few bf16 tokens (:func:`moe_few_max_tokens`) without a sorted list, over matrices in operand
+    order: tokens' experts are read from ``idx`` ``[T, top]``, distinct in a row.  First product (``activation`` given): row t of
+    ``x`` ``[T, K]`` to row ``t * top + k`` of ``out`` ``[T * top, N or N / 2]``; the second: row ``t * top + k`` of ``x`` to the
+    same row of ``out``, fp32.  ``table`` (first product): ``(table [rows, top], ids [T], feedback or None, wgt [T, top])`` -
+    ``idx`` and ``wgt`` (``1 / top`` each) are filled from it as :func:`moe_table_align` does.  ``shared``: ``(x, w, out, activation,
+    limit)`` of an expert that every token uses, in the same launch: ``w`` a :class:`TiledWeight` (first product: of joined gate and
+    up matrices, ``out`` bf16 ``[T, I]``; the second: ``out`` fp32 ``[T, N]``)."""
+    tokens, top = idx.shape
+    experts, n, k = w.shape
+    first = activation is not None
+    n_out = n // 2 if gated else n
+    if x.dtype != torch.bfloat16 or w.dtype != torch.bfloat16 or x.shape != (tokens if first else tokens * top, k) \
+            or out.shape != (tokens * top, n_out) or out.dtype != (torch.bfloat16 if first else torch.float32) or (gated and not first):
+        raise KernelError(f"moe_few_rows: x {tuple(x.shape)}, w {tuple(w.shape)}, out {tuple(out.shape)} do not fit {tokens} tokens of {top}")
+    if slot_weight is not None and (slot_weight.numel() != tokens * top or slot_weight.dtype != torch.float32):
+        raise KernelError("moe_few_rows: one fp32 weight per (token, choice) slot")
+    if first and activation not in EXPERT_ACTIVATIONS:
+        raise KernelError(f"moe_few_rows: activation {activation!r} is not one of {sorted(EXPERT_ACTIVATIONS)}")
+    tab, ids, feedback, wgt = table if table is not None else (None, None, None, None)
+    if tab is not None and (not first or tab.dim() != 2 or tab.shape[1] != top or ids.shape != (tokens,) or wgt.shape != (tokens, top)):
+        raise KernelError("moe_few_rows: a table [rows, top] goes with the first product, ids [T] and weights [T, top]")
+    sx, sw, sout, sact, slimit = shared if shared is not None else (None, None, None, None, 0.0)
+    if sw is not None and (not isinstance(sw, TiledWeight) or sx.shape != (tokens, sw.k) or sx.dtype != torch.bfloat16
+                           or sout.shape != (tokens, sw.n // 2 if first else sw.n) or sout.dtype != out.dtype
+                           or (first and sact not in EXPERT_ACTIVATIONS) or (not first and sw.n != n)):
+        raise KernelError("moe_few_rows: the expert every token uses does not fit")
+    check(hip_lib().kva_moe_few_rows(
+        _dev(out, "out"), _dev(x, "x"), _dev(w, "w"), _dev(idx, "idx", torch.int32), _opt(tab, "table", torch.int32),
+        tab.shape[0] if tab is not None else 0, top, _opt(ids, "ids", torch.int32), _opt(feedback, "feedback", torch.int32),
+        1.0 / top, _dev(idx, "idx", torch.int32) if tab is not None else None, _opt(wgt, "wgt", torch.float32), tokens, top, experts, n, k,
+        0 if first else 1, EXPERT_ACTIVATIONS.get(activation, 0), 1 if gated else 0, float(limit), _opt(slot_weight, "slot_weight"),
+        _opt(sx, "shared x"), _opt(sw.data, "shared w") if sw is not None else None, _opt(sout, "shared out"), sw.n if sw is not None else 0,
+        sw.k if sw is not None else 0, EXPERT_ACTIVATIONS.get(sact, 0), float(slimit), _stream()), "moe_few_rows")
+    return out
+
+
 SMALL_PRODUCT_MAX_K = 8192
 
 
@@ -2320,9 +2366,9 @@ def small_product_f32(x: torch.Tensor, w: torch.Tensor, out: torch.Tensor, bias:
 
 class ExpertRows:
     """What routed experts returned, not added up yet: ``rows`` (fp32 ``[T * top, width]``, weighted) and, optionally, the
-    output ``extra`` of an expert every token uses, times ``sigmoid(extra_gate[t])`` (fp32, a column) if that is there.
-    Whoever reads the sum next may form it in its own pass (:func:`tanh_step`); :meth:`sum` forms it with
-    :func:`moe_combine`."""
+    output ``extra`` (either storage type) of an expert every token uses, times ``sigmoid(extra_gate[t])`` (fp32, a column) if that
+    is there.  Whoever reads the sum next may form it in its own pass (:func:`tanh_step`, :func:`sandwich_step`,
+    :func:`layernorm`); :meth:`sum` forms it with :func:`moe_combine`."""
 
     def __init__(self, x, rows, idx, wgt, experts: int, extra=None, extra_gate=None):
         self.x, self.rows, self.idx, self.wgt, self.experts, self.extra, self.extra_gate = x, rows, idx, wgt, experts, extra, extra_gate
@@ -2349,12 +2395,30 @@ class ExpertRows:
                            extra_gate=self.extra_gate)
 
 
+def added_up(y):
+    """A branch output as a tensor: what routed experts returned is added up."""
+    return y.sum() if isinstance(y, ExpertRows) else y
+
+
+def _expert_rows_args(e: Optional[ExpertRows]) -> tuple:
+    """(rows, the extra row's gate, choices a token, elements from one gate to the next) as the kernels that form the sum take them."""
+    if e is None:
+        return None, None, 0, 0
+    tokens, width = e.shape
+    if e.rows.shape != (tokens * e.top, width) or e.rows.dtype != torch.float32 or (e.extra is not None and e.extra.shape != (tokens, width)):
+        raise KernelError(f"experts' rows {tuple(e.rows.shape)} are not fp32 [T * top, width] of {tuple(e.shape)}")
+    gate, stride = e.gate_column()
+    if gate is not None and (gate.shape != (tokens,) or gate.dtype != torch.float32):
+        raise KernelError("experts' rows: the gate of the extra row is fp32, one number a token")
+    return _dev(e.rows, "rows"), None if gate is None else _dev(gate, "gate", torch.float32, contiguous=False), e.top, int(stride)
+
+
 def moe_combine(x: torch.Tensor, rows: torch.Tensor, idx: torch.Tensor, wgt: torch.Tensor, experts: int,
                 out: torch.Tensor, extra: Optional[torch.Tensor] = None,
                 extra_gate: Optional[torch.Tensor] = None) -> torch.Tensor:
     """``out[t] = sum over the token's choices`` of the slot's row of ``rows`` (fp32 ``[T * top, width]``,
     already weighted) or, for a choice past the real ``experts`` (an identity expert), ``wgt * x[t]``;
-    ``extra`` (x's shape and type: what an expert that every token uses returned) is added last - times
+    ``extra`` (x's shape, x's type or fp32: what an expert that every token uses returned) is added last - times
     ``sigmoid(extra_gate[t])`` with ``extra_gate`` (fp32, one number a token; it may be a column of a wider array)."""
     if extra_gate is not None and (extra is None or extra_gate.numel() != x.shape[0] or extra_gate.dtype != torch.float32):
         raise KernelError("moe_combine: the addend's gate is fp32, one number a token")
@@ -2369,10 +2433,11 @@ def moe_combine(x: torch.Tensor, rows: torch.Tensor, idx: torch.Tensor, wgt: tor
     top = idx.shape[1]
     if out.shape != x.shape or out.dtype != x.dtype or rows.shape != (tokens * top, width) or rows.dtype != torch.float32 \
             or idx.shape != (tokens, top) or wgt.shape != (tokens, top) \
-            or (extra is not None and (extra.shape != x.shape or extra.dtype != x.dtype)):
+            or (extra is not None and (extra.shape != x.shape or extra.dtype not in (x.dtype, torch.float32))):
         raise KernelError(f"moe_combine: x {tuple(x.shape)}, rows {tuple(rows.shape)}, idx {tuple(idx.shape)} do not fit")
     check(hip_lib().kva_moe_combine(_dev(out, "out"), _dev(x, "x"), dtype_code(x.dtype), _dev(rows, "rows"),
                                     _dev(idx, "idx", torch.int32), _dev(wgt, "wgt", torch.float32), _opt(extra, "extra"),
+                                    dtype_code(extra.dtype) if extra is not None else 0,
                                     None if extra_gate is None else _dev(extra_gate, "extra_gate", contiguous=False),
                                     int(gate_stride), tokens, width, top, int(experts), _stream()), "moe_combine")
     return out
@@ -2397,7 +2462,7 @@ KERNEL_CLASSES = {
     "sample": "sampling", "mark_tokens": "sampling",
     "causal_conv_act": "recurrent mixers", "gated_delta_rule": "recurrent mixers",
     "gated_linear_attention": "recurrent mixers", "head_norm_gate": "elementwise",
-    "moe_route": "routed experts", "moe_router": "routed experts", "moe_align": "routed experts", "moe_table_align": "routed experts", "moe_expert_rows": "routed experts",
+    "moe_route": "routed experts", "moe_router": "routed experts", "moe_align": "routed experts", "moe_table_align": "routed experts", "moe_expert_rows": "routed experts", "moe_few_rows": "routed experts",
     "moe_combine": "routed experts", "small_product_f32": "small fp32 products",
     "norm_into_stream": "norm", "table_gate": "elementwise",
     "hyper_step": "norm", "sandwich_step": "norm", "hyper_fill": "embedding", "bias_act": "activation",

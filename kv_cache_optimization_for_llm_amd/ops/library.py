@@ -45,7 +45,7 @@ _HIP_SIGNATURES = {
     "kva_rope_kv_write": [P, P, P, P, P, P, P, I, I, I, I, I, I, I, I, P],
     "kva_attention_rowwise": [P, P, I, P, P, P, I, P, P, I, I, I, I, I, I, F, I, I, I, P, I, P],
     "kva_latent_attention_rowwise": [P, P, P, P, I, P, P, I, I, I, I, I, F, I, I, P, I, P],
-    "kva_layernorm": [P, P, I, P, I, P, I, P, I, P, P, I, P, I, I, F, I, F, P],
+    "kva_layernorm": [P, P, I, P, I, P, I, P, I, P, P, I, P, I, I, F, I, F, P, P, I, I, P],
     "kva_stream_join": [P, I, P, I, P, I, P, I, P, I, I, I, I, P],
     "kva_act_mul": [P, P, I, I, I, F, I, P],
     "kva_head_gate": [P, P, I, I, I, I, I, P],
@@ -106,14 +106,16 @@ _HIP_SIGNATURES = {
     "kva_moe_group_supported": [I, I],
     "kva_moe_table_align": [P, P, P, P, P, I, P, P, I, I, F, I, I, I, I, P],
     "kva_moe_expert_rows": [P, I, P, P, I, P, P, P, I, I, I, I, I, I, I, F, I, I, I, P],
-    "kva_moe_combine": [P, P, I, P, P, P, P, P, I, I, I, I, I, P],
+    "kva_moe_few_max_tokens": [],
+    "kva_moe_few_rows": [P, P, P, P, P, I, I, P, P, F, P, P, I, I, I, I, I, I, I, I, F, P, P, P, P, I, I, I, F, P],
+    "kva_moe_combine": [P, P, I, P, P, P, P, I, P, I, I, I, I, I, P],
     "kva_small_product_f32": [P, P, I, I, P, I, I, I, I, P, F, P, I, P],
     "kva_norm_into_stream": [P, I, P, I, P, I, P, I, I, I, F, P],
     "kva_table_gate": [P, P, I, P, I, I, I, I, P, P, I, I, I, P],
     "kva_bias_act": [P, P, I, P, I, I, I, P],
     "kva_hyper_step": [P, I, P, I, P, P, F, P, P, P, I, F, P, I, P, I, I, P],
     "kva_latent_attention_merge": [P, P, P, P, I, I, I, I, P],
-    "kva_sandwich_step": [P, P, I, P, P, I, I, F, P, P, P, I, I, F, P, I, P, I, I, P],
+    "kva_sandwich_step": [P, P, I, P, P, I, I, F, P, P, P, I, I, F, P, I, P, I, I, P, P, I, I, P],
     "kva_tanh_step": [P, P, I, P, P, P, I, F, P, P, I, F, P, I, P, I, I, P, P, I, I, P],
     "kva_pair_embed": [P, P, I, I, F, P, I, I, I, I, P, P, I, F, P, P, P, I, P, P, I, I, I, P],
     "kva_maps_encode_cache": [P, I, P, P, P, P, P, P, P, I, I, I, I, I, I, I, I, P, I, P],

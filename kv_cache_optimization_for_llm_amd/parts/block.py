@@ -78,6 +78,9 @@ class ParallelBlock(Block):
         super().__init__(mixer, feed_forward, norms)
         self.mixer_norm = self.norms["mixer"]
         self.ffn_norm = self.norms.get("feed_forward")
+        # (a norm of the other kind, or an operation between layers, adds the rows up first)
+        if self.has_ffn and hasattr(feed_forward, "leaves_rows"):
+            feed_forward.leaves_rows = True
 
     def first_norm(self) -> Optional[Norm]:
         return None             # the stream is handed over as it is, with its pending branch outputs
@@ -187,8 +190,8 @@ class SandwichNormBlock(Block):
         # a pass of tanh norms adds the bias of the product whose output it lets in
         if kinds == {"tanh"} and isinstance(mixer, ProjectedMixer):
             mixer.leaves_out_bias = True
-        if kinds == {"tanh"} and hasattr(feed_forward, "leaves_rows"):
-            feed_forward.leaves_rows = True        # ... and adds up what routed experts returned
+        if hasattr(feed_forward, "leaves_rows"):
+            feed_forward.leaves_rows = True        # every pass adds up what routed experts returned
 
     def first_norm(self) -> Optional[Norm]:
         return None

@@ -70,6 +70,11 @@ class SwiGLU(FeedForward):
 
     fuses_tail = True
 
+    def tiled_for_experts(self) -> bool:
+        """Whether the matrices' tiles can be read by the kernel that runs a few tokens' routed experts."""
+        return self.gate_up.tiled is not None and self.down.tiled is not None and self.intermediate_size % 16 == 0 \
+            and self.hidden_size % 16 == 0
+
     def activation_elements(self) -> int:
         # gate and up, their gated product, the down projection
         return 3 * self.intermediate_size + self.hidden_size

@@ -162,6 +162,10 @@ class RoutedExperts(FeedForward):
             self.w_up = self.w_down = None
         # matrices of the matrix-core kernels lie in operand order: what a wavefront loads at once is one run of bytes
         self.tiled = self.experts > 0 and K.moe_can_tile(self.w_up) and K.moe_can_tile(self.w_down)
+        # a few tokens take no sorted list (ops.kernels.moe_few_rows): a token's choices must be distinct there, as a router's are
+        ordered = None if self.table is None else self.table.sort(dim=1).values
+        self.lists_few = not self.tiled or (ordered is not None and bool((ordered[:, 1:] == ordered[:, :-1]).any())) \
+            or (self.shared is not None and not self.shared.tiled_for_experts())
         if self.tiled:
             self.w_up, self.w_down = K.moe_tiled_weight(self.w_up), K.moe_tiled_weight(self.w_down)
 
@@ -187,6 +191,26 @@ class RoutedExperts(FeedForward):
         # the shared expert's gate: one number a token, in 32-bit; its sigmoid is taken where the rows are added
         return product[:, self.outputs] if self.shared_gate is not None else None
 
+    def _few(self, x) -> bool:
+        return not self.lists_few and x.dtype == torch.bfloat16 and 0 < x.shape[0] <= K.moe_few_max_tokens()
+
+    def _few_rows(self, x, idx, wgt, table) -> tuple:
+        """(the experts' rows, the rows of the expert every token uses or None), both products in a launch each."""
+        T, dev, sh = x.shape[0], x.device, self.shared
+        act = torch.empty((T * self.top, self.intermediate_size), dtype=x.dtype, device=dev)
+        rows = torch.empty((T * self.top, self.hidden_size), dtype=torch.float32, device=dev)
+        first = second = extra = None
+        if sh is not None:
+            mid = torch.empty((T, sh.intermediate_size), dtype=x.dtype, device=dev)
+            extra = torch.empty((T, self.hidden_size), dtype=torch.float32, device=dev)
+            first = (x, sh.gate_up.tiled, mid, sh.activation, sh.limit)
+            second = (mid, sh.down.tiled, extra, None, 0.0)
+        before, behind = (wgt, None) if self.weight_input else (None, wgt)
+        K.moe_few_rows(x, self.w_up, act, idx, activation=self.activation, slot_weight=before, gated=self.gated, limit=self.limit,
+                       table=table, shared=first)
+        K.moe_few_rows(act, self.w_down, rows, idx, slot_weight=behind, shared=second)
+        return rows, extra
+
     # an arrangement whose next pass over the output can add the experts' rows up sets this: they are then handed on
     # as ops.kernels.ExpertRows
     leaves_rows = False
@@ -196,8 +220,15 @@ class RoutedExperts(FeedForward):
         idx = torch.empty((T, self.top), dtype=torch.int32, device=dev)
         wgt = torch.empty((T, self.top), dtype=torch.float32, device=dev)
         slots, gate = T * self.top, None
+        few = self._few(x)
         group = K.moe_group(slots, self.experts, x.dtype, self.hidden_size, self.intermediate_size) if self.experts else 1
-        if self.by_table:
+        table = None
+        if self.by_table and few:
+            # (the weights are equal ones: where they stand on the experts' inputs, they do before the launch that looks them up)
+            table = (self.table, ctx.batch.token_ids, getattr(ctx.batch, "feedback", None), wgt)
+            if self.weight_input:
+                wgt.fill_(1.0 / self.top)
+        elif self.by_table:
             sorted_slot, tile_expert = self._sorted(slots, group, dev)
             K.moe_table_align(self.table, ctx.batch.token_ids, idx, wgt, self.experts, sorted_slot, tile_expert,
                               getattr(ctx.batch, "feedback", None), group)
@@ -205,7 +236,7 @@ class RoutedExperts(FeedForward):
             # one launch for the router's product and the choice, and for few tokens the sorted list too
             rest = torch.empty((T, 1), dtype=torch.float32, device=dev) if self.shared_gate is not None else None
             listed = {}
-            if self.experts:
+            if self.experts and not few:
                 sorted_slot, tile_expert = self._sorted(slots, group, dev)
                 if T <= K.MOE_ROUTER_LIST_TOKENS:
                     listed = dict(sorted_slot=sorted_slot, tile_expert=tile_expert)
@@ -213,24 +244,27 @@ class RoutedExperts(FeedForward):
                          self.renormalise, self.over_chosen, scores=self.scores, groups=self.groups,
                          keep_groups=self.keep_groups, group_top=self.group_top, weight_scale=self.weight_scale,
                          sum_eps=self.sum_eps, experts=self.experts, group=group, **listed)
-            if self.experts and not listed:
+            if self.experts and not listed and not few:
                 K.moe_align(idx, self.experts, sorted_slot, tile_expert, group)
             gate = rest[:, 0] if rest is not None else None
         else:
             gate = self._route(x, idx, wgt)
-            if self.experts:
+            if self.experts and not few:
                 sorted_slot, tile_expert = self._sorted(slots, group, dev)
                 K.moe_align(idx, self.experts, sorted_slot, tile_expert, group)
+        if few:
+            rows, extra = self._few_rows(x, idx, wgt, table)
         if RoutedExperts.on_route is not None and not torch.cuda.is_current_stream_capturing():
             RoutedExperts.on_route(self, idx)
-        rows = torch.empty((slots, self.hidden_size), dtype=torch.float32, device=dev)
-        if self.experts:
-            act = torch.empty((sorted_slot.shape[0], self.intermediate_size), dtype=x.dtype, device=dev)
-            first, second = (wgt, None) if self.weight_input else (None, wgt)
-            K.moe_expert_rows(x, self.w_up, act, sorted_slot, tile_expert, self.top, activation=self.activation,
-                              slot_weight=first, gated=self.gated, limit=self.limit, group=group, tiled=self.tiled)
-            K.moe_expert_rows(act, self.w_down, rows, sorted_slot, tile_expert, self.top, slot_weight=second, group=group,
-                              tiled=self.tiled)
-        extra = self.shared.forward(x, ctx) if self.shared is not None else None
+        if not few:
+            rows = torch.empty((slots, self.hidden_size), dtype=torch.float32, device=dev)
+            if self.experts:
+                act = torch.empty((sorted_slot.shape[0], self.intermediate_size), dtype=x.dtype, device=dev)
+                first, second = (wgt, None) if self.weight_input else (None, wgt)
+                K.moe_expert_rows(x, self.w_up, act, sorted_slot, tile_expert, self.top, activation=self.activation,
+                                  slot_weight=first, gated=self.gated, limit=self.limit, group=group, tiled=self.tiled)
+                K.moe_expert_rows(act, self.w_down, rows, sorted_slot, tile_expert, self.top, slot_weight=second, group=group,
+                                  tiled=self.tiled)
+            extra = self.shared.forward(x, ctx) if self.shared is not None else None
         out = K.ExpertRows(x, rows, idx, wgt, self.experts, extra, gate)
         return out if self.leaves_rows and self.identity == 0 else out.sum()

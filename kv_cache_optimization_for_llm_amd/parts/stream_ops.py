@@ -65,6 +65,7 @@ class AddFirst(Part):
         if isinstance(delta, PendingNorm) and delta.addend is None:
             return hidden, dataclasses.replace(delta, addend=first)
         outputs = () if delta is None else (tuple(delta) if isinstance(delta, (tuple, list)) else (delta,))
+        outputs = tuple(K.added_up(d) for d in outputs)
         if getattr(delta, "scale", 1.0) != 1.0 or not all(isinstance(d, torch.Tensor) for d in outputs):
             raise TypeError("pending branch outputs are added as they are here, or under their norm")
         for y in outputs:
