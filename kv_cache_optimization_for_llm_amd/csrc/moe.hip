@@ -374,6 +374,23 @@ struct MoeRouter {
     int tokens, N, K, x_stride;
 };
 
+// steps s0 .. s1 - 1 of a part, four steps' loads on their way at once
+__device__ inline f32x4 moe_router_part(const bf16_t *wrow, const bf16_t *xrow, int s0, int s1) {
+    f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+    for (int s = s0; s < s1; s += 4) {
+        Frag8 xf[4], wf[4];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            xf[i].u4 = *reinterpret_cast<const uint4 *>(xrow + 32 * min(s + i, s1 - 1));
+            wf[i].u4 = *reinterpret_cast<const uint4 *>(wrow + 32 * min(s + i, s1 - 1));
+        }
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+            if (s + i < s1) acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf[i].v, xf[i].v, acc, 0, 0, 0);
+    }
+    return acc;
+}
+
 template <int PL>
 __global__ void __launch_bounds__(1024)
 moe_router_kernel(MoeRouter m, MoeRoute a, int *__restrict__ sorted_slot, int *__restrict__ tile_expert, int experts, int capacity,
@@ -393,13 +410,7 @@ moe_router_kernel(MoeRouter m, MoeRoute a, int *__restrict__ sorted_slot, int *_
         if (on) {
             const bf16_t *wrow = m.w + (size_t)min(16 * tile + r, m.N - 1) * m.K + 8 * g;
             const int s1 = min(steps, (kp + 1) * per);
-#pragma unroll 8
-            for (int s = kp * per; s < s1; ++s) {
-                Frag8 xf, wf;
-                xf.u4 = *reinterpret_cast<const uint4 *>(xrow + 32 * s);
-                wf.u4 = *reinterpret_cast<const uint4 *>(wrow + 32 * s);
-                acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf.v, xf.v, acc, 0, 0, 0);
-            }
+            acc = moe_router_part(wrow, xrow, kp * per, s1);
         }
         __syncthreads();
 #pragma unroll
@@ -810,10 +821,25 @@ extern "C" int kva_moe_expert_rows(void *out, int out_dtype, const void *x, cons
 // expert, or (fewer slots than experts) the expert of a slot, whose first slot's workgroups take it; one more unit is the expert
 // that every token uses, in the same launch.  Which tokens chose the expert is read from idx by the lanes themselves, or (mode 0)
 // looked up in a table by token id, in which case one workgroup leaves idx and the weights for whoever comes next.  A token's
-// choices are distinct.  The four wavefronts take a quarter of K each; all of a quarter's loads (up to 16 steps of 32) are on
-// their way at once, since a workgroup is as long as its chain of trips to memory: list, rows, matrix one after another, with
-// eight loads in flight, and a list's launch in front took the times on the left.
+// choices are distinct.  The four wavefronts take a quarter of K each, eight steps of 32 on their way at once: a workgroup is as long
+// as its chain of trips to memory.  (Lists, rows and matrix one after another, a list's launch in front, and a tile of 16 places
+// an expert: 8 tokens of 16 experts of 768 x 2,048, four each and a shared one, 19.6 + 7.6 and 16.4 + 4.8 us; now 20.7 and 10.3,
+// 4.7 TB/s; one token of four experts of 1,024 x 2,048 11.9 and 8.2, now 6.5 and 5.6.  All 16 steps at once: 22.7 and 10.3.)
+// Two tiles of outputs a workgroup share the rows where there are enough workgroups without: 16 tokens of 64 experts, 6,240 and
+// 8,320 workgroups, 78 / 41 -> 67 / 37 us; 1,632 and 2,176 of them 20.8 / 10.3 -> 21.6 / 9.9.
+//
+// ROUTED (mode 0): the router's product and the choice are made here too, by every workgroup for itself, in the order of sums
+// of the router's own launch: 16 parts of K.  A router of up to 16 outputs is 64 KB that all workgroups read from L2 while
+// their matrix is on its way; the launch it saves took 6-8 us.
 //  mode 0: out[slot] = act(W[e] x[token]) (x's type),   mode 1: out[slot] = W[e] x[slot] * weight[slot] (fp32).
+struct MoeFewRouter {
+    const bf16_t *w;                // [N, K], N up to 16
+    const float *bias;
+    float *rest, *wgt;              // outputs past the router's [tokens, N - outputs]; weights [tokens, top]
+    int N;
+    MoeRoute rule;
+};
+
 struct MoeFew {
     const int *idx;
     MoeTable tab;
@@ -833,10 +859,12 @@ __device__ inline float moe_gated(float gate, float up, int act, float limit) {
 
 __device__ inline uint32_t moe_pack(float a, float b) { return __builtin_bit_cast(uint32_t, pack_bf16(a, b)); }
 
-template <int AHEAD>
+template <int AHEAD, int NT, bool ROUTED>
 __global__ void __launch_bounds__(256)
-moe_few_rows_kernel(MoeFew a, void *__restrict__ out, const bf16_t *__restrict__ x, const bf16_t *__restrict__ w) {
-    __shared__ float red[3][KVA_WAVE][4];
+moe_few_rows_kernel(MoeFew a, MoeFewRouter ro, void *__restrict__ out, const bf16_t *__restrict__ x, const bf16_t *__restrict__ w) {
+    __shared__ float red[3][NT][KVA_WAVE][4];
+    __shared__ __attribute__((aligned(16))) float part[ROUTED ? 16 : 1][KVA_WAVE][4], logits[ROUTED ? 16 : 1][16], choice[4][KVA_WAVE], wgt_s[ROUTED ? 256 : 1];
+    __shared__ int idx_s[ROUTED ? 256 : 1];
     const int lane = threadIdx.x % KVA_WAVE, wave = __builtin_amdgcn_readfirstlane(threadIdx.x / KVA_WAVE), r = lane & 15, g = lane >> 4;
     const int unit = blockIdx.y, slots = a.tokens * a.top;
     const bool shared = unit == a.units;
@@ -845,86 +873,155 @@ moe_few_rows_kernel(MoeFew a, void *__restrict__ out, const bf16_t *__restrict__
             a.idx_out[s] = moe_slot_expert(nullptr, s, a.tab);
             a.tab.wgt[s] = a.tab.weight;
         }
-    const int N = shared ? a.shared_N : a.N, K = shared ? a.shared_K : a.K, n0 = 16 * blockIdx.x;
-    if (n0 >= N) return;
-    int slot = -1, e = 0;               // this lane's token's slot with the expert
+    const int N = shared ? a.shared_N : a.N, K = shared ? a.shared_K : a.K, first = 16 * NT * blockIdx.x;
+    if (first >= N) return;
+    int slot = -1, e = unit;            // this lane's token's slot with the expert
+    const int steps = K / 32, per = (steps + 3) / 4, s0 = wave * per, s1 = min(steps, s0 + per);
+    const bool pairs = shared && a.mode == 0;       // 8 gate rows and 8 up rows of two tiles
+    const bf16_t *wrow[NT], *xrow;
+    Frag8 wf[NT][AHEAD], xf[AHEAD];
+    auto rows = [&]() {
+        xrow = (shared ? a.shared_x : x) + (size_t)(shared || a.mode == 0 ? min(r, a.tokens - 1) : max(slot, 0)) * K + 8 * g;
+#pragma unroll
+        for (int t = 0; t < NT; ++t) {
+            const int n0 = min(first + 16 * t, N - 16);
+            wrow[t] = shared ? a.shared_w : w + (size_t)e * N * K;
+            if (pairs) wrow[t] += (size_t)((r >> 3) * (N / 32) + n0 / 32) * 16 * K + 8 * (16 * g + n0 / 2 % 16 + (r & 7));
+            else wrow[t] += (size_t)n0 * K + 8 * lane;
+        }
+    };
+    auto load = [&](int s) {
+#pragma unroll
+        for (int i = 0; i < AHEAD; ++i)
+#pragma unroll
+            for (int t = 0; t < NT; ++t) wf[t][i].u4 = *reinterpret_cast<const uint4 *>(wrow[t] + (size_t)max(0, min(s + i, s1 - 1)) * 512);
+#pragma unroll
+        for (int i = 0; i < AHEAD; ++i) xf[i].u4 = *reinterpret_cast<const uint4 *>(xrow + 32 * max(0, min(s + i, s1 - 1)));
+    };
+    if constexpr (ROUTED) {
+        rows();                         // (the expert is the unit's number: its matrix comes while the choice is made)
+        const bf16_t *rx = x + (size_t)min(r, a.tokens - 1) * a.K + 8 * g, *rw = ro.w + (size_t)min(r, ro.N - 1) * a.K + 8 * g;
+        const int all = a.K / 32, each = (all + 15) / 16;
+        f32x4 sums[4];
+#pragma unroll
+        for (int j = 0; j < 4; ++j) sums[j] = moe_router_part(rw, rx, (4 * wave + j) * each, min(all, (4 * wave + j + 1) * each));
+        load(s0);
+#pragma unroll
+        for (int j = 0; j < 4; ++j) *reinterpret_cast<f32x4 *>(part[4 * wave + j][lane]) = sums[j];
+        __syncthreads();
+        {                               // element i of lane l: token l % 16, output 4 (l / 16) + i
+            const int l = threadIdx.x / 4, n = 4 * (l / 16) + threadIdx.x % 4;
+            float v = part[0][l][threadIdx.x % 4];
+#pragma unroll
+            for (int p = 1; p < 16; ++p) v += part[p][l][threadIdx.x % 4];
+            if (n < ro.N) logits[l % 16][n] = v + (ro.bias ? ro.bias[n] : 0.f);
+        }
+        __syncthreads();
+        for (int t = wave; t < a.tokens; t += 4)
+            moe_route_token<1>(ro.rule, logits[t], idx_s + t * a.top, wgt_s + t * a.top, choice[wave]);
+        __syncthreads();
+        if (unit == 0 && blockIdx.x == 0) {
+            for (int s = threadIdx.x; s < slots; s += 256) {
+                a.idx_out[s] = idx_s[s];
+                ro.wgt[s] = wgt_s[s];
+            }
+            const int more = ro.N - ro.rule.outputs;
+            for (int i = threadIdx.x; i < more * a.tokens; i += 256) ro.rest[i] = logits[i / more][ro.rule.outputs + i % more];
+        }
+    }
     if (shared) {
         slot = r < a.tokens ? r : -1;
     } else {
         int *idx = const_cast<int *>(a.idx);
-        e = __builtin_amdgcn_readfirstlane(a.by_slot ? moe_slot_expert(idx, unit, a.tab) : unit);
+        auto chosen = [&](int s) { return ROUTED ? idx_s[s] : moe_slot_expert(idx, s, a.tab); };
+        if (a.by_slot) e = __builtin_amdgcn_readfirstlane(chosen(unit));
         if (r < a.tokens)
             for (int k = g; k < a.top; k += 4)
-                if (moe_slot_expert(idx, r * a.top + k, a.tab) == e) slot = r * a.top + k;
+                if (chosen(r * a.top + k) == e) slot = r * a.top + k;
         slot = max(slot, __shfl_xor(slot, 16, KVA_WAVE));
         slot = max(slot, __shfl_xor(slot, 32, KVA_WAVE));
         const unsigned long long chose = __ballot(slot >= 0);
         if (e < 0 || e >= a.experts || !chose) return;
         if (a.by_slot && __shfl(slot, __ffsll(chose) - 1, KVA_WAVE) != unit) return;
     }
-    const bool pairs = shared && a.mode == 0;       // 8 gate rows and 8 up rows of two tiles
-    const bf16_t *xrow = (shared ? a.shared_x : x) + (size_t)(shared || a.mode == 0 ? min(r, a.tokens - 1) : max(slot, 0)) * K + 8 * g;
-    const bf16_t *wrow = shared ? a.shared_w : w + (size_t)e * N * K;
-    if (pairs) wrow += (size_t)((r >> 3) * (N / 32) + n0 / 32) * 16 * K + 8 * (16 * g + n0 / 2 % 16 + (r & 7));
-    else wrow += (size_t)n0 * K + 8 * lane;
-    const int steps = K / 32, per = (steps + 3) / 4, s0 = wave * per, s1 = min(steps, s0 + per);
-    f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+    if constexpr (!ROUTED) {
+        rows();
+        load(s0);
+    }
+    f32x4 acc[NT];
+#pragma unroll
+    for (int t = 0; t < NT; ++t) acc[t] = f32x4{0.f, 0.f, 0.f, 0.f};
     for (int s = s0; s < s1; s += AHEAD) {
-        Frag8 wf[AHEAD], xf[AHEAD];
-#pragma unroll
-        for (int i = 0; i < AHEAD; ++i) wf[i].u4 = *reinterpret_cast<const uint4 *>(wrow + (size_t)min(s + i, s1 - 1) * 512);
-#pragma unroll
-        for (int i = 0; i < AHEAD; ++i) xf[i].u4 = *reinterpret_cast<const uint4 *>(xrow + 32 * min(s + i, s1 - 1));
+        if (s > s0) load(s);
 #pragma unroll
         for (int i = 0; i < AHEAD; ++i)
-            if (s + i < s1) acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf[i].v, xf[i].v, acc, 0, 0, 0);
+            if (s + i < s1)
+#pragma unroll
+                for (int t = 0; t < NT; ++t) acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf[t][i].v, xf[i].v, acc[t], 0, 0, 0);
     }
-    if (wave > 0) *reinterpret_cast<f32x4 *>(red[wave - 1][lane]) = acc;
+    if (wave > 0)
+#pragma unroll
+        for (int t = 0; t < NT; ++t) *reinterpret_cast<f32x4 *>(red[wave - 1][t][lane]) = acc[t];
     __syncthreads();
     if (wave > 0) return;
-    float v[4];
+    const float weight = shared || slot < 0 ? 1.f : ROUTED && a.slot_weight ? wgt_s[slot] : a.slot_weight ? a.slot_weight[slot] : 1.f;
 #pragma unroll
-    for (int i = 0; i < 4; ++i) v[i] = ((acc[i] + red[0][lane][i]) + red[1][lane][i]) + red[2][lane][i];
-    if (pairs) {                        // lanes of g and g + 2: outputs n0 / 2 + 4 g .. + 3, gates and ups
-        float up[4];
+    for (int t = 0; t < NT; ++t) {
+        const int n0 = first + 16 * t, n = n0 + 4 * g;
+        if (n0 >= N) return;
+        float v[4];
 #pragma unroll
-        for (int i = 0; i < 4; ++i) up[i] = __shfl_xor(v[i], 32, KVA_WAVE);
-        if (g >= 2 || slot < 0) return;
+        for (int i = 0; i < 4; ++i) v[i] = (((acc[t][i] + red[0][t][lane][i]) + red[1][t][lane][i]) + red[2][t][lane][i]) * weight;
+        if (pairs) {                    // lanes of g and g + 2: outputs n0 / 2 + 4 g .. + 3, gates and ups
+            float up[4];
 #pragma unroll
-        for (int i = 0; i < 4; ++i) v[i] = moe_gated(v[i], up[i], a.shared_act, a.shared_limit);
-        *reinterpret_cast<uint2 *>(reinterpret_cast<uint16_t *>(a.shared_out) + (size_t)slot * (N / 2) + n0 / 2 + 4 * g) =
-            make_uint2(moe_pack(v[0], v[1]), moe_pack(v[2], v[3]));
-        return;
-    }
-    if (slot < 0) return;
-    const int n = n0 + 4 * g;
-    if (a.slot_weight && !shared) {
-        const float weight = a.slot_weight[slot];
+            for (int i = 0; i < 4; ++i) up[i] = __shfl_xor(v[i], 32, KVA_WAVE);
+            if (g >= 2 || slot < 0) continue;
 #pragma unroll
-        for (int i = 0; i < 4; ++i) v[i] *= weight;
-    }
-    if (a.mode == 1) {
-        *reinterpret_cast<float4 *>((shared ? reinterpret_cast<float *>(a.shared_out) : reinterpret_cast<float *>(out)) + (size_t)slot * N + n) =
-            make_float4(v[0], v[1], v[2], v[3]);
-    } else if (a.gated) {
-        *reinterpret_cast<uint32_t *>(reinterpret_cast<uint16_t *>(out) + (size_t)slot * (N / 2) + n / 2) =
-            moe_pack(moe_gated(v[0], v[1], a.act, a.limit), moe_gated(v[2], v[3], a.act, a.limit));
-    } else {
+            for (int i = 0; i < 4; ++i) v[i] = moe_gated(v[i], up[i], a.shared_act, a.shared_limit);
+            *reinterpret_cast<uint2 *>(reinterpret_cast<uint16_t *>(a.shared_out) + (size_t)slot * (N / 2) + n0 / 2 + 4 * g) =
+                make_uint2(moe_pack(v[0], v[1]), moe_pack(v[2], v[3]));
+        } else if (slot < 0) {
+        } else if (a.mode == 1) {
+            *reinterpret_cast<float4 *>((shared ? reinterpret_cast<float *>(a.shared_out) : reinterpret_cast<float *>(out)) + (size_t)slot * N + n) =
+                make_float4(v[0], v[1], v[2], v[3]);
+        } else if (a.gated) {
+            *reinterpret_cast<uint32_t *>(reinterpret_cast<uint16_t *>(out) + (size_t)slot * (N / 2) + n / 2) =
+                moe_pack(moe_gated(v[0], v[1], a.act, a.limit), moe_gated(v[2], v[3], a.act, a.limit));
+        } else {
 #pragma unroll
-        for (int i = 0; i < 4; ++i) v[i] = moe_activate(v[i], a.act);
-        *reinterpret_cast<uint2 *>(reinterpret_cast<uint16_t *>(out) + (size_t)slot * N + n) =
-            make_uint2(moe_pack(v[0], v[1]), moe_pack(v[2], v[3]));
+            for (int i = 0; i < 4; ++i) v[i] = moe_activate(v[i], a.act);
+            *reinterpret_cast<uint2 *>(reinterpret_cast<uint16_t *>(out) + (size_t)slot * N + n) =
+                make_uint2(moe_pack(v[0], v[1]), moe_pack(v[2], v[3]));
+        }
     }
 }
 
 extern "C" int kva_moe_few_max_tokens(void) { return 16; }
 
+// whether the first product makes the choice itself (every expert its unit, one tile of router outputs, a place for every slot)
+extern "C" int kva_moe_few_routes(int router_N, int slots, int experts) {
+    return router_N > 0 && router_N <= 16 && slots >= experts && slots <= 256;
+}
+
 extern "C" int kva_moe_few_rows(void *out, const void *x, const void *w, const int *idx, const int *table, int table_rows, int table_top,
                                 const int *ids, const int *feedback, float table_weight, int *idx_out, float *wgt_out,
                                 int tokens, int top, int experts, int N, int K, int mode, int act, int gated, float limit,
                                 const float *slot_weight, const void *shared_x, const void *shared_w, void *shared_out,
-                                int shared_N, int shared_K, int shared_act, float shared_limit, hipStream_t stream) {
-    KVA_REQUIRE(out && x && w && (idx || table) && tokens >= 0 && tokens <= 16 && top > 0 && experts > 0,
+                                int shared_N, int shared_K, int shared_act, float shared_limit, const void *router_w, int router_N,
+                                const float *router_bias, const float *correction, float *rest, int outputs, int renormalise,
+                                int over_chosen, int sigmoid_scores, int groups, int keep_groups, int group_top, float weight_scale,
+                                float sum_eps, hipStream_t stream) {
+    // router_w: the router's product and the choice here (idx_out, wgt_out; slot_weight then means: weights stand on the inputs)
+    const MoeFewRouter ro{(const bf16_t *)router_w, router_bias, rest, wgt_out, router_N,
+                          MoeRoute{correction, outputs, top, renormalise, over_chosen, sigmoid_scores, groups, keep_groups, group_top, weight_scale, sum_eps}};
+    if (router_w) {
+        KVA_REQUIRE(mode == 0 && !table && idx_out && wgt_out && outputs <= router_N && (outputs == router_N || rest) &&
+                        kva_moe_few_routes(router_N, tokens * top, experts) && ((uintptr_t)router_w & 15) == 0,
+                    "moe_few_rows: no choice of %d outputs here", router_N);
+        if (int rc = moe_route_check(ro.rule)) return rc;
+    }
+    KVA_REQUIRE(out && x && w && (idx || table || router_w) && tokens >= 0 && tokens <= 16 && top > 0 && experts > 0,
                 "moe_few_rows: missing operand, or more than 16 tokens (%d)", tokens);
     KVA_REQUIRE(N > 0 && N % 16 == 0 && K > 0 && K % 32 == 0, "moe_few_rows: no operand order for %d x %d", N, K);
     KVA_REQUIRE(mode == 0 || mode == 1, "moe_few_rows: the first product (0) or the second (1)");
@@ -943,10 +1040,15 @@ extern "C" int kva_moe_few_rows(void *out, const void *x, const void *w, const i
                    units, by_slot, N, K, mode, act, gated, limit, (const bf16_t *)shared_x, (const bf16_t *)shared_w, shared_out, shared_N,
                    shared_K, shared_act, shared_limit};
     const int wide = shared_w && shared_N > N ? shared_N : N, deep = shared_w && shared_K > K ? shared_K : K, per = (deep / 32 + 3) / 4;
-    const dim3 grid((wide + 15) / 16, units + (shared_w ? 1 : 0));
-    if (per > 8) hipLaunchKernelGGL(moe_few_rows_kernel<16>, grid, dim3(256), 0, stream, a, out, (const bf16_t *)x, (const bf16_t *)w);
-    else if (per > 4) hipLaunchKernelGGL(moe_few_rows_kernel<8>, grid, dim3(256), 0, stream, a, out, (const bf16_t *)x, (const bf16_t *)w);
-    else hipLaunchKernelGGL(moe_few_rows_kernel<4>, grid, dim3(256), 0, stream, a, out, (const bf16_t *)x, (const bf16_t *)w);
+    const int tiles = (wide + 15) / 16, rows = units + (shared_w ? 1 : 0), nt = !router_w && tiles * rows > 4096 ? 2 : 1;
+    const dim3 grid((tiles + nt - 1) / nt, rows);
+#define KVA_MOE_FEW(AHEAD, NT, ROUTED) \
+    hipLaunchKernelGGL((moe_few_rows_kernel<AHEAD, NT, ROUTED>), grid, dim3(256), 0, stream, a, ro, out, (const bf16_t *)x, (const bf16_t *)w)
+    if (router_w) KVA_MOE_FEW(8, 1, true);
+    else if (nt == 2) KVA_MOE_FEW(8, 2, false);
+    else if (per > 4) KVA_MOE_FEW(8, 1, false);
+    else KVA_MOE_FEW(4, 1, false);
+#undef KVA_MOE_FEW
     KVA_CHECK_LAUNCH("moe_few_rows");
     return KVA_OK;
 }

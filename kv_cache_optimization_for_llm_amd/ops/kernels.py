@@ -2297,16 +2297,23 @@ def moe_few_max_tokens() -> int:
     return int(hip_lib().kva_moe_few_max_tokens())
 
 
+def moe_few_routes(x: torch.Tensor, router: torch.Tensor, slots: int, experts: int) -> bool:
+    """Whether :func:`moe_few_rows` makes the choice for rows like ``x`` itself (``router``)."""
+    return moe_router_supported(x, router) and bool(hip_lib().kva_moe_few_routes(router.shape[0], int(slots), int(experts)))
+
+
 def moe_few_rows(x: torch.Tensor, w: torch.Tensor, out: torch.Tensor, idx: torch.Tensor, *, activation: Optional[str] = None,
                  slot_weight: Optional[torch.Tensor] = None, gated: bool = False, limit: float = 0.0, table=None,
-                 shared=None) -> torch.Tensor:
+                 shared=None, router: Optional[dict] = None) -> torch.Tensor:
     """:func:`moe_expert_rows` for a few bf16 tokens (:func:`moe_few_max_tokens`) without a sorted list, over matrices in operand
     order: tokens' experts are read from ``idx`` ``[T, top]``, distinct in a row.  First product (``activation`` given): row t of
     ``x`` ``[T, K]`` to row ``t * top + k`` of ``out`` ``[T * top, N or N / 2]``; the second: row ``t * top + k`` of ``x`` to the
     same row of ``out``, fp32.  ``table`` (first product): ``(table [rows, top], ids [T], feedback or None, wgt [T, top])`` -
     ``idx`` and ``wgt`` (``1 / top`` each) are filled from it as :func:`moe_table_align` does.  ``shared``: ``(x, w, out, activation,
     limit)`` of an expert that every token uses, in the same launch: ``w`` a :class:`TiledWeight` (first product: of joined gate and
-    up matrices, ``out`` bf16 ``[T, I]``; the second: ``out`` fp32 ``[T, N]``)."""
+    up matrices, ``out`` bf16 ``[T, I]``; the second: ``out`` fp32 ``[T, N]``).  ``router`` (first product, where
+    :func:`moe_few_routes` says so): ``idx`` and ``wgt`` are made here; :func:`moe_router`'s arguments ``w``, ``bias``,
+    ``correction``, ``outputs``, ``wgt``, ``rest`` and its rule's keywords.  A ``slot_weight`` then is ``wgt`` itself."""
     tokens, top = idx.shape
     experts, n, k = w.shape
     first = activation is not None
@@ -2326,13 +2333,28 @@ def moe_few_rows(x: torch.Tensor, w: torch.Tensor, out: torch.Tensor, idx: torch
                            or sout.shape != (tokens, sw.n // 2 if first else sw.n) or sout.dtype != out.dtype
                            or (first and sact not in EXPERT_ACTIVATIONS) or (not first and sw.n != n)):
         raise KernelError("moe_few_rows: the expert every token uses does not fit")
+    rw, rule = None, (None, 0, None, None, None, 1, 0, 0, 0, 1, 1, 1, 1.0, 0.0)
+    if router is not None:
+        rw, wgt, rest, outputs, kw = router["w"], router["wgt"], router.get("rest"), int(router["outputs"]), router
+        if not first or tab is not None or rw.dim() != 2 or rw.shape[1] != k or rw.dtype != torch.bfloat16 or wgt.shape != (tokens, top) \
+                or not 0 < outputs <= rw.shape[0] or (rest is None) != (outputs == rw.shape[0]) \
+                or (rest is not None and rest.shape != (tokens, rw.shape[0] - outputs)) or (slot_weight is not None and slot_weight is not wgt) \
+                or kw.get("scores", "softmax") not in ("softmax", "sigmoid"):
+            raise KernelError(f"moe_few_rows: the router {tuple(rw.shape)} does not fit")
+        for name, n_values in (("bias", rw.shape[0]), ("correction", outputs)):
+            if kw.get(name) is not None and kw[name].shape != (n_values,):
+                raise KernelError(f"moe_few_rows: the router's {name} has one value an output")
+        rule = (_dev(rw, "router"), rw.shape[0], _opt(kw.get("bias"), "bias", torch.float32), _opt(kw.get("correction"), "correction", torch.float32),
+                _opt(rest, "rest", torch.float32), outputs, 1 if kw.get("renormalise") else 0, 1 if kw.get("over_chosen") else 0,
+                1 if kw.get("scores", "softmax") == "sigmoid" else 0, int(kw.get("groups", 1)), int(kw.get("keep_groups", 1)),
+                int(kw.get("group_top", 2)), float(kw.get("weight_scale", 1.0)), float(kw.get("sum_eps", 0.0)))
     check(hip_lib().kva_moe_few_rows(
         _dev(out, "out"), _dev(x, "x"), _dev(w, "w"), _dev(idx, "idx", torch.int32), _opt(tab, "table", torch.int32),
         tab.shape[0] if tab is not None else 0, top, _opt(ids, "ids", torch.int32), _opt(feedback, "feedback", torch.int32),
-        1.0 / top, _dev(idx, "idx", torch.int32) if tab is not None else None, _opt(wgt, "wgt", torch.float32), tokens, top, experts, n, k,
+        1.0 / top, _dev(idx, "idx", torch.int32) if tab is not None or rw is not None else None, _opt(wgt, "wgt", torch.float32), tokens, top, experts, n, k,
         0 if first else 1, EXPERT_ACTIVATIONS.get(activation, 0), 1 if gated else 0, float(limit), _opt(slot_weight, "slot_weight"),
         _opt(sx, "shared x"), _opt(sw.data, "shared w") if sw is not None else None, _opt(sout, "shared out"), sw.n if sw is not None else 0,
-        sw.k if sw is not None else 0, EXPERT_ACTIVATIONS.get(sact, 0), float(slimit), _stream()), "moe_few_rows")
+        sw.k if sw is not None else 0, EXPERT_ACTIVATIONS.get(sact, 0), float(slimit), *rule, _stream()), "moe_few_rows")
     return out
 
 

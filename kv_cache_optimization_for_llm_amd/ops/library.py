@@ -107,7 +107,9 @@ _HIP_SIGNATURES = {
     "kva_moe_table_align": [P, P, P, P, P, I, P, P, I, I, F, I, I, I, I, P],
     "kva_moe_expert_rows": [P, I, P, P, I, P, P, P, I, I, I, I, I, I, I, F, I, I, I, P],
     "kva_moe_few_max_tokens": [],
-    "kva_moe_few_rows": [P, P, P, P, P, I, I, P, P, F, P, P, I, I, I, I, I, I, I, I, F, P, P, P, P, I, I, I, F, P],
+    "kva_moe_few_rows": [P, P, P, P, P, I, I, P, P, F, P, P, I, I, I, I, I, I, I, I, F, P, P, P, P, I, I, I, F,
+                         P, I, P, P, P, I, I, I, I, I, I, I, F, F, P],
+    "kva_moe_few_routes": [I, I, I],
     "kva_moe_combine": [P, P, I, P, P, P, P, I, P, I, I, I, I, I, P],
     "kva_small_product_f32": [P, P, I, I, P, I, I, I, I, P, F, P, I, P],
     "kva_norm_into_stream": [P, I, P, I, P, I, P, I, I, I, F, P],

@@ -194,7 +194,7 @@ class RoutedExperts(FeedForward):
     def _few(self, x) -> bool:
         return not self.lists_few and x.dtype == torch.bfloat16 and 0 < x.shape[0] <= K.moe_few_max_tokens()
 
-    def _few_rows(self, x, idx, wgt, table) -> tuple:
+    def _few_rows(self, x, idx, wgt, table, router) -> tuple:
         """(the experts' rows, the rows of the expert every token uses or None), both products in a launch each."""
         T, dev, sh = x.shape[0], x.device, self.shared
         act = torch.empty((T * self.top, self.intermediate_size), dtype=x.dtype, device=dev)
@@ -207,7 +207,7 @@ class RoutedExperts(FeedForward):
             second = (mid, sh.down.tiled, extra, None, 0.0)
         before, behind = (wgt, None) if self.weight_input else (None, wgt)
         K.moe_few_rows(x, self.w_up, act, idx, activation=self.activation, slot_weight=before, gated=self.gated, limit=self.limit,
-                       table=table, shared=first)
+                       table=table, shared=first, router=router)
         K.moe_few_rows(act, self.w_down, rows, idx, slot_weight=behind, shared=second)
         return rows, extra
 
@@ -222,7 +222,9 @@ class RoutedExperts(FeedForward):
         slots, gate = T * self.top, None
         few = self._few(x)
         group = K.moe_group(slots, self.experts, x.dtype, self.hidden_size, self.intermediate_size) if self.experts else 1
-        table = None
+        table = router = None
+        rule = dict(scores=self.scores, groups=self.groups, keep_groups=self.keep_groups, group_top=self.group_top,
+                    weight_scale=self.weight_scale, sum_eps=self.sum_eps)
         if self.by_table and few:
             # (the weights are equal ones: where they stand on the experts' inputs, they do before the launch that looks them up)
             table = (self.table, ctx.batch.token_ids, getattr(ctx.batch, "feedback", None), wgt)
@@ -235,25 +237,27 @@ class RoutedExperts(FeedForward):
         elif K.moe_router_supported(x, self.router):
             # one launch for the router's product and the choice, and for few tokens the sorted list too
             rest = torch.empty((T, 1), dtype=torch.float32, device=dev) if self.shared_gate is not None else None
+            gate = rest[:, 0] if rest is not None else None
             listed = {}
             if self.experts and not few:
                 sorted_slot, tile_expert = self._sorted(slots, group, dev)
                 if T <= K.MOE_ROUTER_LIST_TOKENS:
                     listed = dict(sorted_slot=sorted_slot, tile_expert=tile_expert)
-            K.moe_router(x, self.router, self.router_bias, self.correction, self.outputs, self.top, idx, wgt, rest,
-                         self.renormalise, self.over_chosen, scores=self.scores, groups=self.groups,
-                         keep_groups=self.keep_groups, group_top=self.group_top, weight_scale=self.weight_scale,
-                         sum_eps=self.sum_eps, experts=self.experts, group=group, **listed)
+            if few and K.moe_few_routes(x, self.router, slots, self.experts):
+                router = dict(w=self.router, bias=self.router_bias, correction=self.correction, outputs=self.outputs, wgt=wgt, rest=rest,
+                              renormalise=self.renormalise, over_chosen=self.over_chosen, **rule)
+            else:
+                K.moe_router(x, self.router, self.router_bias, self.correction, self.outputs, self.top, idx, wgt, rest,
+                             self.renormalise, self.over_chosen, experts=self.experts, group=group, **rule, **listed)
             if self.experts and not listed and not few:
                 K.moe_align(idx, self.experts, sorted_slot, tile_expert, group)
-            gate = rest[:, 0] if rest is not None else None
         else:
             gate = self._route(x, idx, wgt)
             if self.experts and not few:
                 sorted_slot, tile_expert = self._sorted(slots, group, dev)
                 K.moe_align(idx, self.experts, sorted_slot, tile_expert, group)
         if few:
-            rows, extra = self._few_rows(x, idx, wgt, table)
+            rows, extra = self._few_rows(x, idx, wgt, table, router)
         if RoutedExperts.on_route is not None and not torch.cuda.is_current_stream_capturing():
             RoutedExperts.on_route(self, idx)
         if not few:

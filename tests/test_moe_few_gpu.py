@@ -39,11 +39,12 @@ def oracle(x, idx, wgt, state, ff, act, gated, weight_input, shared, gate):
 
 
 # (tokens; width, experts' and shared width: steps of 32 of K that do not divide by four, one step, more than 16 a wavefront;
-#  experts below and above the number of slots; every choice of token and expert counts from one choice to all of them)
+#  experts below and above the number of slots; routers of up to 16 outputs inside the first product, larger ones in front; every choice of token and expert counts from one choice to all of them)
 @pytest.mark.parametrize("T, W, ff, experts, top, shared, router, gated, act, on_input", [
     (1, 64, 32, 4, 4, 0, "learned", False, "gelu", False), (1, 2048, 96, 16, 4, 32, "table", True, "silu", False),
     (16, 96, 160, 16, 3, 96, "learned", True, "silu", True), (5, 2560, 64, 40, 2, 64, "learned", True, "silu", False),
     (16, 64, 4128, 3, 1, 0, "table", False, "relu2", False), (2, 128, 64, 2, 2, 160, "table", True, "silu", True),
+    (16, 2048, 64, 15, 15, 64, "learned", True, "silu", True), (3, 544, 64, 5, 2, 32, "learned", True, "silu", False),
     (17, 64, 32, 4, 2, 32, "learned", True, "silu", False)])
 def test_experts_over_a_few_tokens(T, W, ff, experts, top, shared, router, gated, act, on_input, gpu, monkeypatch):
     learned = router == "learned"
@@ -55,11 +56,14 @@ def test_experts_over_a_few_tokens(T, W, ff, experts, top, shared, router, gated
         state["p.table"] = torch.stack([torch.randperm(experts, generator=torch.Generator().manual_seed(i))[:top] for i in range(50)]).int()
     part.load({k: v.to(gpu) for k, v in state.items()})
     x, ids = rnd((T, W), 77), torch.randint(0, 50, (T,), dtype=torch.int32)
-    seen, calls, few = [], [], K.moe_few_rows
+    seen, calls, routed, few, front = [], [], [], K.moe_few_rows, K.moe_router
+    monkeypatch.setattr(K, "moe_router", lambda *a, **k: routed.append("router") or front(*a, **k))
     monkeypatch.setattr(RoutedExperts, "on_route", lambda p, idx: seen.append(idx.cpu()))
     monkeypatch.setattr(K, "moe_few_rows", lambda *a, **k: calls.append(1) or few(*a, **k))
     got = part.forward(x.to(gpu), MixerContext(batch=_Batch(ids.to(gpu)))).double().cpu()
     assert len(calls) == (2 if T <= K.moe_few_max_tokens() else 0)
+    inside = learned and T <= 16 and T * top >= experts and experts + bool(shared) <= 16
+    assert ("router" in routed) == (learned and not inside)
     idx = seen[0]
     if learned:
         wgt = torch.sigmoid((x.double() @ state["p.router"].double().T).gather(1, idx.long()))
