@@ -15,13 +15,15 @@
 //   rows x outputs x K    3 x 128,256 x 2,048: 480 -> 260 (4.0 TB/s)     3 x 16,384 x 2,048: 147 -> 33 (4.1 TB/s)
 //                         3 x 2,048 x 8,192: 544 -> 19 (3.5 TB/s)        3 x 3,072 x 2,048: 141 -> 11
 //                         32 x 2,048 x 8,192: 545 -> 58                  64 x 2,048 x 8,192: 559 -> 59 (the tiles: 167)
-//                         64 x 128,256 x 2,048: 532 -> 352 (96 TFLOP/s; the few-rows kernel: 941)
-//                         402 x 16,384 x 2,048: 449 -> 329 (82 TFLOP/s)  402 x 2,048 x 8,192: 556 -> 167 (81)
-//                         2,048 x 16,384 x 2,048: 1,748 -> 1,319 (104)
-// Not so for K up to 128 and tens of thousands of outputs (2,000 x 16,384 x 128: 130 -> 143, 64 x 128,256 x 64: 29 -> 26, 2,000 x
-// 128,256 x 64: 591 -> 703): a tile's result takes longer than its products.  No model here has such a product.
+// and of those with more rows, plain FMAs -> tiles through registers, K's halves on eight wavefronts -> the ring:
+//                         64 x 128,256 x 2,048: 532 -> 369 -> 310        402 x 16,384 x 2,048: 449 -> 340 -> 250 (108 TFLOP/s)
+//                         517 x 16,384 x 2,048: 424 -> 287 (121)         517 x 2,048 x 8,192: 308 -> 178 (97)
+//                         517 x 3,072 x 2,048: 85 -> 66                  517 x 2,048 x 2,048: 85 -> 50
+//                         100 x 2,048 x 8,192: 165 -> 85                 2,048 x 16,384 x 2,048: 1,748 -> 1,304 -> 1,009 (136)
+// With K up to 128 a tile's result takes longer than its products: 2,000 x 16,384 x 128 130 -> 162 -> 105.
 // The few-rows kernel stays below the 6 TB/s of a plain read stream: a load takes 64 bytes from each of 16 rows.
 #include "common.h"
+#include "lds_product.h"
 
 typedef float gf_f32x4 __attribute__((ext_vector_type(4)));
 
@@ -126,7 +128,7 @@ gemm_f32_rows_kernel(float *__restrict__ C, const float *__restrict__ A, const f
     }
 }
 
-// Many rows: bound by the matrix cores (a 32-bit product takes 16 times the cycles of a 16-bit one).  A workgroup
+// Many rows that start at any address: bound by the matrix cores and by loads of single elements.  A workgroup
 // takes 64 rows x 32 NT outputs: four wavefronts (32 x 16 NT each) the front half of the parts, four the back half -
 // two wavefronts a SIMD where the tiles are about as many as the compute units.  32 columns of both operands of
 // each half go through LDS at a time (rows 36 elements apart: the 16 rows of an operand read start in different
@@ -137,7 +139,7 @@ struct GfTile {
     float a[2][GF_BM][GF_BK + GF_PAD], w[2][32 * NT][GF_BK + GF_PAD];
 };
 
-template <int NT, bool VEC>
+template <int NT>
 __global__ void __launch_bounds__(512)
 gemm_f32_tile_kernel(float *__restrict__ C, const float *__restrict__ A, const float *__restrict__ W, int M, int N,
                      int K, int lda, int ldw, int ldc, int part, int mtiles, int tiles) {
@@ -160,9 +162,9 @@ gemm_f32_tile_kernel(float *__restrict__ C, const float *__restrict__ A, const f
     const int lrow = tid / 8, lk = tid % 8 * 4;                      // 32 rows a pass, 8 lanes a row
     auto fetch = [&](int set, int k0) {                              // (past the half's end: zeros)
 #pragma unroll
-        for (int i = 0; i < AL; ++i) la[set][i] = gf_load<VEC, false>(A, m0 + lrow + 32 * i, M, k0 + lk, hi, lda);
+        for (int i = 0; i < AL; ++i) la[set][i] = gf_load<false, false>(A, m0 + lrow + 32 * i, M, k0 + lk, hi, lda);
 #pragma unroll
-        for (int i = 0; i < WL; ++i) lw[set][i] = gf_load<VEC, false>(W, n0 + lrow + 32 * i, N, k0 + lk, hi, ldw);
+        for (int i = 0; i < WL; ++i) lw[set][i] = gf_load<false, false>(W, n0 + lrow + 32 * i, N, k0 + lk, hi, ldw);
     };
     auto put = [&](int set) {
 #pragma unroll
@@ -249,28 +251,171 @@ gemm_f32_tile_kernel(float *__restrict__ C, const float *__restrict__ A, const f
             gf_f32x4 v;
 #pragma unroll
             for (int e = 0; e < 4; ++e) v[e] = tot[i][j][e] + o[e];
-            if (VEC && n + 3 < N) *reinterpret_cast<gf_f32x4 *>(c) = v;
-            else
 #pragma unroll
-                for (int e = 0; e < 4; ++e)
-                    if (n + e < N) c[e] = v[e];
+            for (int e = 0; e < 4; ++e)
+                if (n + e < N) c[e] = v[e];
         }
     }
 }
 
+// Many rows, every row of both operands at a multiple of 16 bytes: bound by the matrix cores (a 32-bit product takes 16 times the
+// cycles of a 16-bit one; they give 142-152 TFLOP/s to one wavefront a SIMD, 156 to two), and by how evenly tiles divide among the
+// compute units.  A workgroup of four wavefronts takes 16 MT rows
+// x 64 outputs, a wavefront all of its rows x 16; MT is chosen so that the fullest compute unit has the least to do (gf_rows_a_tile).
+// 32 columns of both operands are a stage; they go straight to LDS (buffer loads, 16 bytes a lane, the eight 16-byte pieces of
+// a row in the order piece ^ row % 8, so that the rows of an operand read lie in different banks), STAGES - 1 stages on their
+// way or waiting.  16 columns' operands are read into registers while the 16 before are multiplied, over the one barrier a stage
+// too: a wavefront that has its SIMD to itself keeps it busy.  Workgroups of one stripe of outputs are neighbours on one die,
+// whose L2 then holds that stripe of W for all of their rows.
+template <int MT, int STAGES>
+__global__ void __launch_bounds__(256, 2)
+gemm_f32_ring_kernel(float *__restrict__ C, const float *__restrict__ A, const float *__restrict__ W, int M, int N,
+                     int K, int lda, int ldw, int ldc, int part, int mtiles, int tiles) {
+    constexpr int PIECES = 2 * MT + 8, LOADS = (PIECES + 3) / 4;     // of 1 KiB: 8 rows of 32; a wavefront's
+    __shared__ __align__(16) float ring[STAGES][PIECES * 256];       // rows of A, then rows of W
+    const int per = (tiles + 7) / 8, tile = (int)(blockIdx.x % 8) * per + (int)(blockIdx.x / 8);
+    if (tile >= tiles) return;                                       // (the whole workgroup)
+    const int m0 = tile % mtiles * 16 * MT, n0 = tile / mtiles * 64;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / KVA_WAVE), lane = threadIdx.x % KVA_WAVE, r = lane % 16, g = lane / 16;
+    const float *atile = A + (size_t)m0 * lda, *wtile = W + (size_t)n0 * ldw;
+    const int arows = min(16 * MT, M - m0), wrows = min(64, N - n0);
+    const Buffer abuf = buffer_at(atile, ((size_t)(arows - 1) * lda + K) * sizeof(float)),
+                 wbuf = buffer_at(wtile, ((size_t)(wrows - 1) * ldw + K) * sizeof(float));
+    int from[LOADS], to[LOADS];
+#pragma unroll
+    for (int i = 0; i < LOADS; ++i) {
+        // (one piece too few for all wavefronts: the last one again, so that all have as many loads on their way)
+        const int piece = min(wave + 4 * i, PIECES - 1);
+        from[i] = 4 * (piece < 2 * MT ? min(8 * piece + lane / 8, arows - 1) * lda : min(8 * (piece - 2 * MT) + lane / 8, wrows - 1) * ldw);
+        to[i] = piece * 256;
+    }
+    const int column = 4 * ((lane % 8) ^ (lane / 8));
+    auto load = [&](int i, int slot, int k0) {                       // (past the end: what is there is left out of the products)
+        buffer_to_lds(to[i] < 2 * MT * 256 ? abuf : wbuf, from[i] + 4 * min(k0 + column, K - 4), 0, &ring[slot][to[i]]);
+    };
+    gf_f32x4 acc[MT], tot[MT], front[MT], a[2][MT], w[2];
+#pragma unroll
+    for (int j = 0; j < MT; ++j) acc[j] = tot[j] = front[j] = gf_f32x4{0.f, 0.f, 0.f, 0.f};
+    auto read = [&](int i, int set, int slot) {                      // half `set` of a stage: W's rows, then A's
+        const float *base = &ring[slot][r * 32 + 4 * ((4 * set + g) ^ (r & 7))];
+        if (i == 0) w[set] = *reinterpret_cast<const gf_f32x4 *>(base + (2 * MT + 2 * wave) * 256);
+        else a[set][i - 1] = *reinterpret_cast<const gf_f32x4 *>(base + 2 * (i - 1) * 256);
+    };
+    const int rounds = (K + GF_BK - 1) / GF_BK, split = gf_half((K + part - 1) / part) * part;
+    auto cut = [&](int set, int k0) {                                // columns past the end are left out
+        if (k0 + 4 * g >= K) {
+            w[set] = gf_f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+            for (int j = 0; j < MT; ++j) a[set][j] = gf_f32x4{0.f, 0.f, 0.f, 0.f};
+        }
+    };
+    // 16 columns' products, and behind the i-th of them what `behind(i)` asks for: a wavefront waits where the next product is not
+    // taken yet, so one load at a time is issued while a product runs
+    auto products = [&](int set, auto behind) {
+#pragma unroll
+        for (int i = 0; i < 4 * MT; ++i) {
+            acc[i % MT] = __builtin_amdgcn_mfma_f32_16x16x4f32(w[set][i / MT], a[set][i % MT][i / MT], acc[i % MT], 0, 0, 0);
+            behind(i);
+            __builtin_amdgcn_sched_barrier(0);
+        }
+    };
+    __builtin_amdgcn_s_waitcnt(0xc07f);     // (arguments' loads have arrived: the waits below are for operands alone, and counted)
+#pragma unroll
+    for (int s = 0; s < STAGES - 1; ++s)
+#pragma unroll
+        for (int i = 0; i < LOADS; ++i) load(i, s, s * GF_BK);
+    wait_and_meet<(STAGES - 2) * LOADS>();
+#pragma unroll
+    for (int i = 0; i <= MT; ++i) read(i, 0, 0);
+    int slot = 0, left = part;                                       // columns of the current part still to come
+    auto round = [&](int t, bool ends) {                             // (`ends`: a constant where this is put in)
+        const int k0 = t * GF_BK, next = slot + 1 == STAGES ? 0 : slot + 1, before = slot == 0 ? STAGES - 1 : slot - 1;
+        if (ends) cut(0, k0);
+        products(0, [&](int i) {
+            if (i <= MT) read(i, 1, slot);
+        });
+        if (ends) cut(1, k0 + GF_STEP);
+        products(1, [&](int i) {
+            // the next stage is there; the slot of the stage before is free: every wavefront has multiplied with it
+            if (i == 0) wait_and_meet<(STAGES - 3) * LOADS>();
+            if (i <= MT) read(i, 0, next);
+            else if (i <= MT + LOADS) load(i - MT - 1, before, k0 + (STAGES - 1) * GF_BK);
+            if (i == 4 * MT - 1)                                     // (what had no product to be behind)
+#pragma unroll
+                for (int j = 4 * MT - MT - 1; j < LOADS; ++j) load(j, before, k0 + (STAGES - 1) * GF_BK);
+        });
+        slot = next;
+        left -= GF_BK;
+        if (left == 0 || t + 1 == rounds) {
+            left = part;
+#pragma unroll
+            for (int j = 0; j < MT; ++j) {
+#pragma unroll
+                for (int c = 0; c < 4; ++c) tot[j][c] += acc[j][c];
+                acc[j] = gf_f32x4{0.f, 0.f, 0.f, 0.f};
+            }
+            if (k0 + GF_BK == split)                                 // the front half is done
+#pragma unroll
+                for (int j = 0; j < MT; ++j) {
+                    front[j] = tot[j];
+                    tot[j] = gf_f32x4{0.f, 0.f, 0.f, 0.f};
+                }
+        }
+    };
+    for (int t = 0; t + 1 < rounds; ++t) round(t, false);
+    round(rounds - 1, true);
+    wait_and_meet<0>();                                              // nothing is on its way to LDS any more
+    if (rounds * GF_BK < split)                                      // (one part, and a short one: it is the front half)
+#pragma unroll
+        for (int j = 0; j < MT; ++j) {
+            front[j] = tot[j];
+            tot[j] = gf_f32x4{0.f, 0.f, 0.f, 0.f};
+        }
+    const int n = n0 + 16 * wave + 4 * g;
+#pragma unroll
+    for (int j = 0; j < MT; ++j) {
+        const int m = m0 + 16 * j + r;
+        if (m >= M) continue;
+        float *c = C + (size_t)m * ldc + n;
+        gf_f32x4 v;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) v[e] = front[j][e] + tot[j][e];
+        if (n + 3 < N) *reinterpret_cast<gf_f32x4 *>(c) = v;
+        else
+#pragma unroll
+            for (int e = 0; e < 4; ++e)
+                if (n + e < N) c[e] = v[e];
+    }
+}
+
+// Rows a tile of the ring kernel takes (16 times the result): the compute unit with the most tiles is what a launch waits for.
+// (us by rows a tile, 16 / 32 / 48 / 64 / 80 / 112 / 128: 517 x 16,384 x 2,048 350 300 292 301 292 287 322; 517 x 2,048 x 8,192
+// 197 198 203 256 178 237 264; 250 x 16,384 x 2,048 182 153 167 137 169 176 133; 70 x 3,072 x 2,048 18 24 33 39 48 63 70.)
+static int gf_rows_a_tile(int M, int N) {
+    int best = 1;
+    long long least = -1;
+    for (int mt = 1; mt <= 8; ++mt) {
+        const long long tiles = (long long)((M + 16 * mt - 1) / (16 * mt)) * ((N + 63) / 64), cost = (tiles + 255) / 256 * (2 * mt + 1);
+        if (least < 0 || cost <= least) { least = cost; best = mt; }
+    }
+    return best;
+}
+
 // Whether few rows go to the kernel that streams W.  It makes 32 rows a pass over W and shares nothing between its
-// workgroups; from some number of outputs on the tiles fill the chip and are the faster ones (K = 2,048, few-rows kernel / tiles,
-// us): 17-32 rows, 8,192 outputs 28-33 / 46, 16,384 52-65 / 50, 128,256 399-492 / 350; 33-64 rows, 4,096 28-33 / 45, 6,144 42-48 /
-// 46, 8,192 51-62 / 46, 32,768 195-242 / 92, 128,256 754-941 / 345; K = 300 and 8,192 alike.
-static bool gf_few_rows(int M, int N) {
-    return M <= 16 || (M <= GF_ROWS_UP_TO && (long long)N * ((M + 31) / 32) < 14336);
+// workgroups; from some number of outputs on the kernels for many rows fill the chip and are the faster ones.  Few-rows kernel / ring,
+// us, K = 2,048: 17-32 rows, 4,096 outputs 16-18 / 17, 6,144 26-32 / 18, 16,384 53-64 / 36; 33-64 rows, 2,048 17 / 17, 3,072
+// 26-31 / 17, 32,768 194-241 / 68-89; K = 300 alike; K = 8,192: 17-32 rows, 2,048 46-58 / 84, 4,096 54-64 / 90; 33-64 rows, 2,048
+// 60 / 85, 4,096 99-123 / 90.  Rows that start at no multiple of 16 bytes have tiles a third slower: few-rows kernel / tiles, 17-32
+// rows, 8,192 outputs 28-33 / 46, 16,384 52-65 / 50; 33-64 rows, 4,096 28-33 / 45, 6,144 42-48 / 46, 8,192 51-62 / 46.
+static bool gf_few_rows(int M, int N, bool vec) {
+    return M <= 16 || (M <= GF_ROWS_UP_TO && (long long)N * ((M + 31) / 32) <= (vec ? 4096 : 14336));
 }
 
 template <bool VEC>
 static void gf_launch(float *C, const float *A, const float *W, int M, int N, int K, int lda, int ldw, int ldc,
                       hipStream_t stream) {
     const int part = gf_part(K), parts = (K + part - 1) / part;
-    if (gf_few_rows(M, N)) {
+    if (gf_few_rows(M, N, VEC)) {
         const int out = M <= 8 ? 8 : 16;
         const dim3 grid((N + out - 1) / out, (M + 31) / 32), block(KVA_WAVE * (M <= 8 ? (parts + 1) / 2 : M <= 16 ? parts : max(4, parts)));    // (four for the sums' last step)
         if (M <= 8)
@@ -281,11 +426,29 @@ static void gf_launch(float *C, const float *A, const float *W, int M, int N, in
             hipLaunchKernelGGL((gemm_f32_rows_kernel<2, 2, false, VEC>), grid, block, 0, stream, C, A, W, M, N, K, lda, ldw, ldc, part);
         return;
     }
+    if (VEC) {
+        const int mt = gf_rows_a_tile(M, N), mtiles = (M + 16 * mt - 1) / (16 * mt), tiles = mtiles * ((N + 63) / 64);
+#define GF_RING(MT, STAGES)                                                                                              \
+    hipLaunchKernelGGL((gemm_f32_ring_kernel<MT, STAGES>), dim3((tiles + 7) / 8 * 8), dim3(256), 0, stream, C, A, W, M, N, K, lda, ldw, \
+                       ldc, part, mtiles, tiles)
+        switch (mt) {
+            case 1: GF_RING(1, 4); break;
+            case 2: GF_RING(2, 4); break;
+            case 3: GF_RING(3, 4); break;
+            case 4: GF_RING(4, 4); break;
+            case 5: GF_RING(5, 4); break;
+            case 6: GF_RING(6, 3); break;
+            case 7: GF_RING(7, 3); break;
+            default: GF_RING(8, 3); break;
+        }
+#undef GF_RING
+        return;
+    }
     const int mtiles = (M + GF_BM - 1) / GF_BM, wide = mtiles * ((N + 127) / 128), narrow = mtiles * ((N + 63) / 64);
     if (wide >= 256)
-        hipLaunchKernelGGL((gemm_f32_tile_kernel<4, VEC>), dim3((wide + 7) / 8 * 8), dim3(512), 0, stream, C, A, W, M, N, K, lda, ldw, ldc, part, mtiles, wide);
+        hipLaunchKernelGGL((gemm_f32_tile_kernel<4>), dim3((wide + 7) / 8 * 8), dim3(512), 0, stream, C, A, W, M, N, K, lda, ldw, ldc, part, mtiles, wide);
     else
-        hipLaunchKernelGGL((gemm_f32_tile_kernel<2, VEC>), dim3((narrow + 7) / 8 * 8), dim3(512), 0, stream, C, A, W, M, N, K, lda, ldw, ldc, part, mtiles, narrow);
+        hipLaunchKernelGGL((gemm_f32_tile_kernel<2>), dim3((narrow + 7) / 8 * 8), dim3(512), 0, stream, C, A, W, M, N, K, lda, ldw, ldc, part, mtiles, narrow);
 }
 
 extern "C" int kva_gemm_nt_f32(float *C, const float *A, const float *W, int M, int N, int K,
@@ -294,8 +457,8 @@ extern "C" int kva_gemm_nt_f32(float *C, const float *A, const float *W, int M, 
     KVA_REQUIRE(lda >= K && ldw >= K && ldc >= N, "gemm_f32: leading dimensions too small");
     if (M == 0) return KVA_OK;
     KVA_REQUIRE((M + GF_BM - 1) / GF_BM <= 65535, "gemm_f32: M=%d is too large for one launch", M);
-    // 16-byte loads and stores where every row of all three starts at a multiple of 16 bytes
-    const bool vec = K % 4 == 0 && lda % 4 == 0 && ldw % 4 == 0 && ldc % 4 == 0 &&
+    // 16-byte loads and stores where every row of all three starts at a multiple of 16 bytes (and a tile's rows lie within 2 GiB)
+    const bool vec = lda <= 1 << 21 && ldw <= 1 << 21 && K % 4 == 0 && lda % 4 == 0 && ldw % 4 == 0 && ldc % 4 == 0 &&
                      ((uintptr_t)A | (uintptr_t)W | (uintptr_t)C) % 16 == 0;
     if (vec) gf_launch<true>(C, A, W, M, N, K, lda, ldw, ldc, stream);
     else gf_launch<false>(C, A, W, M, N, K, lda, ldw, ldc, stream);

@@ -25,6 +25,16 @@ __device__ __forceinline__ void load_to_lds(const void *from, void *to) {
     __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) unsigned int *)from,
                                      (__attribute__((address_space(3))) unsigned int *)to, 16, 0, 0);
 }
+// The same from a buffer that starts at `base` (the same in all lanes): bytes `offset` (a lane's own) + `shared` from there on.  The
+// compiler counts operand reads from LDS that are still on their way past these loads; past load_to_lds, which it takes for one
+// that may read LDS itself, it waits for all of them.  Nothing is read past `bytes`.
+typedef __amdgpu_buffer_rsrc_t Buffer;
+__device__ __forceinline__ Buffer buffer_at(const void *base, size_t bytes) {
+    return __builtin_amdgcn_make_buffer_rsrc(const_cast<void *>(base), 0, (int)(bytes < 0xffffffffull ? bytes : 0xffffffffull), 0x00027000);
+}
+__device__ __forceinline__ void buffer_to_lds(Buffer from, int offset, int shared, void *to) {
+    __builtin_amdgcn_raw_ptr_buffer_load_lds(from, (__attribute__((address_space(3))) void *)to, 16, offset, shared, 0, 0);
+}
 // The wavefront's loads but the last N have arrived; then all wavefronts' have.  Nothing that reads or writes memory
 // moves across.
 template <int N>

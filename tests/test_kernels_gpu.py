@@ -210,6 +210,25 @@ def test_gemm_f32_rows_are_the_same_bits_where_the_kernel_changes(n, k, gpu):
     close(got[65], a.double() @ w.double().t(), torch.float32, "gemm_nt_f32")
 
 
+@pytest.mark.parametrize("m, n", [(65, 68), (100, 3000), (130, 4500), (190, 10000), (517, 2048), (402, 3072), (517, 3072), (250, 16384), (129, 8196)])
+@pytest.mark.parametrize("k", [4, 36, 96, 2052])
+def test_gemm_f32_every_height_of_a_tile(m, n, k, gpu):
+    """Tiles of 16 to 128 rows, remainders of rows, outputs and columns: the bits of a row alone, and nothing of a neighbouring row (whose
+    first elements lie behind a row's last ones)."""
+    a, w = rnd(m, k).to(gpu), rnd(n, k, seed=1).to(gpu)
+    a[m // 2 + 1], w[n // 3 + 1] = float("nan"), float("inf")
+    got = K.gemm_nt_f32(a, w, torch.full((m, n), 7.0, device=gpu))
+    for row in (0, m // 2, m - 1):
+        one = K.gemm_nt_f32(a[row:row + 1].contiguous(), w, torch.empty(1, n, device=gpu))
+        assert torch.equal(one[0].nan_to_num(nan=5.0), got[row].nan_to_num(nan=5.0)), row
+    rows, outputs = [i for i in range(m) if i != m // 2 + 1], [i for i in range(n) if i != n // 3 + 1]
+    want = a[rows].double() @ w[outputs].double().t()
+    # as above: K products and additions of relative error 2^-24 each
+    bound = 2.0 ** -24 * max(4.0, (2.0 * k) ** 0.5) * (a[rows].double().pow(2) @ w[outputs].double().pow(2).t()).sqrt().mean()
+    assert (got[rows][:, outputs] - want).double().pow(2).mean().sqrt() <= bound
+    assert got[m // 2 + 1, outputs].isnan().all()
+
+
 def rope_reference(x, pos, inv, heads, d, rot):
     cos, sin = plain.rope_cos_sin(pos, inv)
     x = x.view(len(pos), heads, d).clone()
