@@ -12,8 +12,8 @@
 //
 // us a call, weights from memory, against one kernel of 64 x 64 tiles and plain FMAs for every M (before -> now;
 // relative error against 64 bits at K = 2,048 / 8,192: 8e-7 / 1.6e-6 -> 2.1e-7 / 4.1e-7):
-//   rows x outputs x K    3 x 128,256 x 2,048: 480 -> 260 (4.0 TB/s)     3 x 16,384 x 2,048: 147 -> 33 (4.1 TB/s)
-//                         3 x 2,048 x 8,192: 544 -> 19 (3.5 TB/s)        3 x 3,072 x 2,048: 141 -> 11
+//   rows x outputs x K    3 x 128,256 x 2,048: 480 -> 231 -> 189 (5.6 TB/s)  3 x 16,384 x 2,048: 147 -> 35 -> 30 (4.5)
+//                         3 x 2,048 x 8,192: 544 -> 20 -> 18 (3.8 TB/s)  3 x 2,048 x 2,048: 7.6 -> 6.7
 //                         32 x 2,048 x 8,192: 545 -> 58                  64 x 2,048 x 8,192: 559 -> 59 (the tiles: 167)
 // and of those with more rows, plain FMAs -> tiles through registers, K's halves on eight wavefronts -> the ring:
 //                         64 x 128,256 x 2,048: 532 -> 369 -> 310        402 x 16,384 x 2,048: 449 -> 340 -> 250 (108 TFLOP/s)
@@ -21,7 +21,6 @@
 //                         517 x 3,072 x 2,048: 85 -> 66                  517 x 2,048 x 2,048: 85 -> 50
 //                         100 x 2,048 x 8,192: 165 -> 85                 2,048 x 16,384 x 2,048: 1,748 -> 1,304 -> 1,009 (136)
 // With K up to 128 a tile's result takes longer than its products: 2,000 x 16,384 x 128 130 -> 162 -> 105.
-// The few-rows kernel stays below the 6 TB/s of a plain read stream: a load takes 64 bytes from each of 16 rows.
 #include "common.h"
 #include "lds_product.h"
 
@@ -44,14 +43,13 @@ static inline int gf_part(int K) {
 __host__ __device__ inline int gf_half(int parts) { return (parts + 1) / 2; }
 
 // four neighbouring elements of a row, zeros past the row's end or for a row that is not there
-template <bool VEC, bool STREAMED>
+template <bool VEC>
 __device__ inline gf_f32x4 gf_load(const float *__restrict__ p, int row, int rows, int k, int K, int ld) {
     gf_f32x4 v = {0.f, 0.f, 0.f, 0.f};
     if (row < rows) {
         const float *a = p + (size_t)row * ld + k;
         if (VEC) {
-            if (k < K) v = STREAMED ? __builtin_nontemporal_load(reinterpret_cast<const gf_f32x4 *>(a))
-                                    : *reinterpret_cast<const gf_f32x4 *>(a);      // (K is a multiple of 4)
+            if (k < K) v = *reinterpret_cast<const gf_f32x4 *>(a);      // (K is a multiple of 4)
         } else {
 #pragma unroll
             for (int e = 0; e < 4; ++e)
@@ -66,7 +64,10 @@ __device__ inline gf_f32x4 gf_load(const float *__restrict__ p, int row, int row
 // product); the parts are added in order through LDS.  PAIR: up to 8 rows and 8 outputs a workgroup, a wavefront
 // takes two parts - operand rows 0-7 the first, 8-15 the second, on both sides, so that the products wanted are
 // the two blocks on the diagonal.  That puts twice the workgroups on a narrow matrix (128 of them would leave
-// half the chip without a share of the stream).
+// half the chip without a share of the stream); from 8,192 outputs on there are enough, and twice the rows a workgroup are the
+// faster way (3 rows, K = 2,048, pairs / not: 6,144 outputs 15.0 / 16.4 us, 8,192 18.3 / 18.4, 16,384 33.7 / 29.8, 128,256 216 /
+// 189).  W goes through the caches: its loads take half a line of 128 bytes each, and with the non-temporal hint the line was
+// asked for twice (128,256 outputs 231 -> 216 us, 2,048 x 8,192 20.1 -> 18.7).
 template <int MT, int DEPTH, bool PAIR, bool VEC>
 __global__ void __launch_bounds__(KVA_WAVE * GF_MAX_PARTS)
 gemm_f32_rows_kernel(float *__restrict__ C, const float *__restrict__ A, const float *__restrict__ W, int M, int N,
@@ -88,9 +89,9 @@ gemm_f32_rows_kernel(float *__restrict__ C, const float *__restrict__ A, const f
 #pragma unroll
         for (int d = 0; d < DEPTH; ++d) {
             const int k = lo + (s0 + d) * GF_STEP + 4 * g;          // (past the part's end: zeros)
-            w[buf][d] = gf_load<VEC, true>(W, wr, N, k, hi, ldw);
+            w[buf][d] = gf_load<VEC>(W, wr, N, k, hi, ldw);
 #pragma unroll
-            for (int t = 0; t < MT; ++t) x[buf][d][t] = gf_load<VEC, false>(A, ar + 16 * t, M, k, hi, lda);
+            for (int t = 0; t < MT; ++t) x[buf][d][t] = gf_load<VEC>(A, ar + 16 * t, M, k, hi, lda);
         }
     };
     auto products = [&](int buf, int s0) {
@@ -162,9 +163,9 @@ gemm_f32_tile_kernel(float *__restrict__ C, const float *__restrict__ A, const f
     const int lrow = tid / 8, lk = tid % 8 * 4;                      // 32 rows a pass, 8 lanes a row
     auto fetch = [&](int set, int k0) {                              // (past the half's end: zeros)
 #pragma unroll
-        for (int i = 0; i < AL; ++i) la[set][i] = gf_load<false, false>(A, m0 + lrow + 32 * i, M, k0 + lk, hi, lda);
+        for (int i = 0; i < AL; ++i) la[set][i] = gf_load<false>(A, m0 + lrow + 32 * i, M, k0 + lk, hi, lda);
 #pragma unroll
-        for (int i = 0; i < WL; ++i) lw[set][i] = gf_load<false, false>(W, n0 + lrow + 32 * i, N, k0 + lk, hi, ldw);
+        for (int i = 0; i < WL; ++i) lw[set][i] = gf_load<false>(W, n0 + lrow + 32 * i, N, k0 + lk, hi, ldw);
     };
     auto put = [&](int set) {
 #pragma unroll
@@ -416,9 +417,9 @@ static void gf_launch(float *C, const float *A, const float *W, int M, int N, in
                       hipStream_t stream) {
     const int part = gf_part(K), parts = (K + part - 1) / part;
     if (gf_few_rows(M, N, VEC)) {
-        const int out = M <= 8 ? 8 : 16;
-        const dim3 grid((N + out - 1) / out, (M + 31) / 32), block(KVA_WAVE * (M <= 8 ? (parts + 1) / 2 : M <= 16 ? parts : max(4, parts)));    // (four for the sums' last step)
-        if (M <= 8)
+        const int out = M <= 8 && N < 8192 ? 8 : 16;
+        const dim3 grid((N + out - 1) / out, (M + 31) / 32), block(KVA_WAVE * (out == 8 ? (parts + 1) / 2 : M <= 16 ? parts : max(4, parts)));    // (four for the sums' last step)
+        if (out == 8)
             hipLaunchKernelGGL((gemm_f32_rows_kernel<1, 2, true, VEC>), grid, block, 0, stream, C, A, W, M, N, K, lda, ldw, ldc, part);
         else if (M <= 16)
             hipLaunchKernelGGL((gemm_f32_rows_kernel<1, 2, false, VEC>), grid, block, 0, stream, C, A, W, M, N, K, lda, ldw, ldc, part);
