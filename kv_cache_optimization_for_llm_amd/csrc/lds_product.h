@@ -126,6 +126,107 @@ struct LdsProduct {
     }
 };
 
+// The same product with a stage's operands in registers while the ones before are multiplied: what a wavefront reads for the next
+// 32 elements of K, and the loads that go to LDS, are issued one at a time behind products, over the one barrier a stage.
+// Operands come from buffers (a base and byte offsets of 32 bits).  The experts' products use it, the two before and with it, the
+// activation chosen once a workgroup (us): 64 experts of 1,536 x 2,048, 32,768 slots 302 -> 244; 16 experts, 8,192 slots 83 -> 71;
+// 4 experts, 9,976 slots 73 -> 63; tiles of 64 x 128, 2,048 slots of 16 experts 47 -> 38.  One workgroup a compute unit would want more
+// stages: two of them cover a load's way with their products (1.35 PFLOP/s from K = 2,048 on, either struct).
+template <int RT, int NT, int STAGES>
+struct RingProduct {
+    static constexpr int ROWS = 32 * RT, OUTS = 32 * NT;
+    static constexpr int XI = ROWS * LDSP_K / 8 / 256, WI = OUTS * LDSP_K / 8 / 256, LOADS = XI + WI;
+    struct Shared {
+        bf16_t x[STAGES][ROWS * LDSP_K], w[STAGES][OUTS * LDSP_K];
+    };
+    Buffer xbuf, wbuf;
+    int xo[XI], wo[WI];             // bytes
+    int wmul;                       // elements of w's storage that go by per element of K
+    bool w_swizzled;
+
+    __device__ __forceinline__ static int row(int i) { return threadIdx.x / 4 + 64 * i; }
+    __device__ __forceinline__ static int element() { return 8 * ((threadIdx.x % 4) ^ (threadIdx.x / 16 % 4)); }
+    __device__ __forceinline__ void plain_w(const bf16_t *w, int N, int K, int n0) {
+        const int rows = min(OUTS, N - n0);
+        wmul = 1;
+        w_swizzled = true;
+        wbuf = buffer_at(w + (size_t)n0 * K, (size_t)rows * K * 2);
+#pragma unroll
+        for (int i = 0; i < WI; ++i) wo[i] = 2 * (min(row(i), rows - 1) * K + element());
+    }
+    __device__ __forceinline__ void tiled_w(const bf16_t *w, int N, int K, int n0) {
+        const int rows = min(OUTS, N - n0);
+        wmul = 16;
+        w_swizzled = false;
+        wbuf = buffer_at(w + (size_t)n0 * K, (size_t)rows * K * 2);
+#pragma unroll
+        for (int i = 0; i < WI; ++i)
+            wo[i] = 2 * (min(16 * (int)(threadIdx.x / KVA_WAVE + 4 * i), rows - 16) * K + 8 * (int)(threadIdx.x % KVA_WAVE));
+    }
+
+    __device__ __forceinline__ void run(Shared &s, int K, f32x4 (&acc)[NT][RT]) const {
+        const int lane = threadIdx.x % KVA_WAVE, wave = __builtin_amdgcn_readfirstlane(threadIdx.x / KVA_WAVE), r = lane & 15, g = lane >> 4;
+        const int wr = wave & 1, wn = wave >> 1;
+        const int swizzled = r * LDSP_K + 8 * (g ^ (r / 4)), xat = wr * RT * 512 + swizzled, wat = wn * NT * 512 + (w_swizzled ? swizzled : 8 * lane);
+        const int last = K - LDSP_K;
+        auto load = [&](int i, int slot, int k0) {
+            const int k = min(k0, last);
+            if (i < XI) buffer_to_lds(xbuf, xo[i], 2 * k, &s.x[slot][(wave + 4 * i) * 512]);
+            else buffer_to_lds(wbuf, wo[i - XI], 2 * k * wmul, &s.w[slot][(wave + 4 * (i - XI)) * 512]);
+        };
+        b16x8 xf[2][RT], wf[2][NT];
+        auto read = [&](int i, int set, int slot) {
+            if (i < RT) xf[set][i] = *reinterpret_cast<const b16x8 *>(&s.x[slot][xat + i * 512]);
+            else wf[set][i - RT] = *reinterpret_cast<const b16x8 *>(&s.w[slot][wat + (i - RT) * 512]);
+        };
+#pragma unroll
+        for (int nt = 0; nt < NT; ++nt)
+#pragma unroll
+            for (int rt = 0; rt < RT; ++rt) acc[nt][rt] = f32x4{0.f, 0.f, 0.f, 0.f};
+        __builtin_amdgcn_s_waitcnt(0xc07f);
+#pragma unroll
+        for (int t = 0; t < STAGES; ++t)
+#pragma unroll
+            for (int i = 0; i < LOADS; ++i) load(i, t, t * LDSP_K);
+        wait_and_meet<(STAGES - 1) * LOADS>();
+#pragma unroll
+        for (int i = 0; i < RT + NT; ++i) read(i, 0, 0);
+        int slot = 0;
+        // round t: the operands of stage t are in `set`; stage t + 1 is read, stage t + STAGES goes where stage t was
+        auto round = [&](int set, int k0) {
+            const int next = slot + 1 == STAGES ? 0 : slot + 1;
+            // every wavefront has read stage t (into registers), stage t + 1 has arrived
+            asm volatile("" ::: "memory");
+            __builtin_amdgcn_sched_barrier(0);
+            __builtin_amdgcn_s_waitcnt((((STAGES - 2) * LOADS) & 15) | (((STAGES - 2) * LOADS) >> 4 << 14) | 0x70);
+            __builtin_amdgcn_s_barrier();
+            __builtin_amdgcn_sched_barrier(0);
+            asm volatile("" ::: "memory");
+#pragma unroll
+            for (int i = 0; i < NT * RT; ++i) {
+                acc[i / RT][i % RT] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf[set][i / RT], xf[set][i % RT], acc[i / RT][i % RT], 0, 0, 0);
+                // a read behind every second product (LDS takes longer for one than a product lasts), the loads between them
+                constexpr int READS = RT + NT, EVERY = NT * RT >= 2 * READS + 2 ? 2 : 1;
+                if (i % EVERY == 0 && i / EVERY < READS) read(i / EVERY, 1 - set, next);
+                if (EVERY == 2 ? i % 2 == 1 && i / 2 < LOADS : i >= READS && i < READS + LOADS)
+                    load(EVERY == 2 ? i / 2 : i - READS, slot, k0 + STAGES * LDSP_K);
+                if (EVERY == 1 && i == NT * RT - 1)     // (what had no product to be behind)
+#pragma unroll
+                    for (int j = NT * RT - READS; j < LOADS; ++j) load(j, slot, k0 + STAGES * LDSP_K);
+                __builtin_amdgcn_sched_barrier(0);
+            }
+            slot = next;
+        };
+        int k0 = 0;
+        for (; k0 + LDSP_K < K; k0 += 2 * LDSP_K) {
+            round(0, k0);
+            round(1, k0 + LDSP_K);
+        }
+        if (k0 < K) round(0, k0);
+        wait_and_meet<0>();
+    }
+};
+
 // Workgroup id -> place in the work list such that neighbours of the list run on one of the 8 dies (the hardware
 // deals workgroups out in turn): what they share is read into one L2.
 __device__ __forceinline__ int die_order(int id, int total) {

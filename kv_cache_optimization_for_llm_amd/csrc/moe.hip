@@ -27,6 +27,7 @@
 #include "attention_frag.h"
 #include "lds_product.h"
 #include <math.h>
+#include <type_traits>
 
 #define MOE_TILE 16
 #define MOE_MAX_EXPERTS 1024
@@ -657,48 +658,56 @@ moe_expert_rows_mfma_kernel(MoeRows a, void *__restrict__ out, int out_dtype, co
     }
 }
 
-// Eight neighbouring results of a place from n on (n a multiple of 8), the slot's weight (or 1) at hand: as moe_store
-// and moe_store_gated do one by one.
-__device__ inline void moe_store8(const MoeRows &a, void *__restrict__ out, int out_dtype, int place, int slot, float weight, int n, const float *v) {
+// Eight neighbouring results of the first product, a place's from n on (n a multiple of 8), the slot's weight (or 1) at hand: as
+// moe_store and moe_store_gated do one by one.  `aligned`: rows start at multiples of 16 bytes.
+template <int ACT, bool GATED>
+__device__ inline void moe_store8(const MoeRows &a, void *__restrict__ out, int place, float weight, int n, const float *v, bool aligned) {
     float f[8];
 #pragma unroll
     for (int i = 0; i < 8; ++i) f[i] = v[i] * weight;
-    if (a.gated) {
+    if (GATED) {
 #pragma unroll
         for (int i = 0; i < 4; ++i)
-            f[i] = a.act == 4 ? kva_gated_activate(f[2 * i], f[2 * i + 1], KVA_ACT_SWISH_CLAMPED, a.limit) : moe_activate(f[2 * i], a.act) * f[2 * i + 1];
-    } else if (a.mode == 0) {
+            f[i] = ACT == 4 ? kva_gated_activate(f[2 * i], f[2 * i + 1], KVA_ACT_SWISH_CLAMPED, a.limit) : moe_activate(f[2 * i], ACT) * f[2 * i + 1];
+    } else {
 #pragma unroll
-        for (int i = 0; i < 8; ++i) f[i] = moe_activate(f[i], a.act);
+        for (int i = 0; i < 8; ++i) f[i] = moe_activate(f[i], ACT);
     }
-    const int width = a.gated ? a.N / 2 : a.N, at = a.gated ? n / 2 : n, count = a.gated ? 4 : 8;
-    const size_t first = (size_t)(a.mode == 0 ? place : slot) * width + at;
-    if (n + 8 <= a.N && width % 8 == 0 && (reinterpret_cast<uintptr_t>(out) & 15) == 0) {
-        if (out_dtype == KVA_BF16) {
-            uint16_t *o = reinterpret_cast<uint16_t *>(out) + first;
-            const Frag8 h = {.p2 = {pack_bf16(f[0], f[1]), pack_bf16(f[2], f[3]), pack_bf16(f[4], f[5]), pack_bf16(f[6], f[7])}};
-            if (a.gated) *reinterpret_cast<uint2 *>(o) = h.u2[0];
-            else *reinterpret_cast<uint4 *>(o) = h.u4;
-        } else {
-            float4 *o = reinterpret_cast<float4 *>(reinterpret_cast<float *>(out) + first);
-            o[0] = make_float4(f[0], f[1], f[2], f[3]);
-            if (!a.gated) o[1] = make_float4(f[4], f[5], f[6], f[7]);
-        }
+    const int width = GATED ? a.N / 2 : a.N, at = GATED ? n / 2 : n, count = GATED ? 4 : 8;
+    uint16_t *o = reinterpret_cast<uint16_t *>(out) + (size_t)place * width + at;
+    if (aligned && n + 8 <= a.N) {
+        const Frag8 h = {.p2 = {pack_bf16(f[0], f[1]), pack_bf16(f[2], f[3]), pack_bf16(f[4], f[5]), pack_bf16(f[6], f[7])}};
+        if (GATED) *reinterpret_cast<uint2 *>(o) = h.u2[0];
+        else *reinterpret_cast<uint4 *>(o) = h.u4;
         return;
     }
 #pragma unroll
-    for (int i = 0; i < 8; ++i) {
-        if (i >= count || at + i >= width) continue;
-        if (out_dtype == KVA_BF16) reinterpret_cast<uint16_t *>(out)[first + i] = float_to_bf16_bits(f[i]);
-        else reinterpret_cast<float *>(out)[first + i] = f[i];
-    }
+    for (int i = 0; i < 8; ++i)
+        if (i < count && at + i < width) o[i] = float_to_bf16_bits(f[i]);
 }
 
+// four of the second one, to the slot's row (fp32)
+__device__ inline void moe_store4(const MoeRows &a, void *__restrict__ out, int slot, float weight, int n, const float *v, bool aligned) {
+    float *o = reinterpret_cast<float *>(out) + (size_t)slot * a.N + n;
+    if (aligned && n + 4 <= a.N) {
+        *reinterpret_cast<float4 *>(o) = make_float4(v[0] * weight, v[1] * weight, v[2] * weight, v[3] * weight);
+        return;
+    }
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+        if (n + i < a.N) o[i] = v[i] * weight;
+}
+
+// (one variable in LDS: with several the compiler tells them apart, and waits for all loads on their way to one before it reads it)
 template <int RT, int NT, int STAGES>
-union MoeLds {
-    static constexpr int STRIDE = 128 + 4;          // a row of results in LDS
-    typename LdsProduct<RT, NT, STAGES>::Shared operands;
-    float results[LdsProduct<RT, NT, STAGES>::ROWS * STRIDE];
+struct MoeLds {
+    static constexpr int STRIDE = 128 + 4, ROWS = RingProduct<RT, NT, STAGES>::ROWS;         // a row of results in LDS
+    union {
+        typename RingProduct<RT, NT, STAGES>::Shared operands;
+        float results[ROWS * STRIDE];
+    };
+    int slot_of[ROWS];
+    float weight_of[ROWS];
 };
 
 // matrix cores, many rows an expert: a workgroup takes a group of 2 RT tiles of one expert (32 RT rows) and 32 NT
@@ -708,10 +717,8 @@ template <int RT, int NT, int STAGES>
 __global__ void __launch_bounds__(256, 2)
 moe_expert_rows_lds_kernel(MoeRows a, void *__restrict__ out, int out_dtype, const bf16_t *__restrict__ x,
                            const bf16_t *__restrict__ w, int n_blocks, int groups) {
-    typedef LdsProduct<RT, NT, STAGES> Product;
+    typedef RingProduct<RT, NT, STAGES> Product;
     __shared__ __align__(16) MoeLds<RT, NT, STAGES> shared;
-    __shared__ int slot_of[Product::ROWS];
-    __shared__ float weight_of[Product::ROWS];
     const int lane = threadIdx.x % KVA_WAVE, wave = threadIdx.x / KVA_WAVE, r = lane & 15, g = lane >> 4;
     int used = 0;
     for (int g0 = 0; g0 < groups; g0 += KVA_WAVE)
@@ -724,15 +731,16 @@ moe_expert_rows_lds_kernel(MoeRows a, void *__restrict__ out, int out_dtype, con
     if (e < 0) return;
     const int wr = wave & 1, wn = wave >> 1;
     Product p;
+    p.xbuf = buffer_at(x, 0xffffffffull);
 #pragma unroll
     for (int i = 0; i < Product::XI; ++i) {
         const int place = first * MOE_TILE + p.row(i), slot = a.sorted_slot[place];
-        p.xp[i] = x + (a.mode == 0 ? (size_t)(slot < 0 ? 0 : slot / a.top) : (size_t)place) * a.K + p.element();
+        p.xo[i] = 2 * ((a.mode == 0 ? (slot < 0 ? 0 : slot / a.top) : place) * a.K + p.element());
     }
     if (threadIdx.x < Product::ROWS) {
         const int slot = a.sorted_slot[first * MOE_TILE + threadIdx.x];
-        slot_of[threadIdx.x] = slot;
-        weight_of[threadIdx.x] = a.slot_weight && slot >= 0 ? a.slot_weight[slot] : 1.f;
+        shared.slot_of[threadIdx.x] = slot;
+        shared.weight_of[threadIdx.x] = a.slot_weight && slot >= 0 ? a.slot_weight[slot] : 1.f;
     }
     const bf16_t *we = w + (size_t)e * a.N * a.K;
     if (a.tiled) p.tiled_w(we, a.N, a.K, n0);
@@ -740,25 +748,52 @@ moe_expert_rows_lds_kernel(MoeRows a, void *__restrict__ out, int out_dtype, con
     f32x4 acc[NT][RT];
     p.run(shared.operands, a.K, acc);
     // The results go out by rows, through LDS in 32 bits (where the operands were): four tiles of either half of the
-    // outputs at a time, then 8 neighbouring outputs a thread.
+    // outputs at a time, then 8 neighbouring outputs a thread.  The activation is chosen once, in front: choosing it for every
+    // element was most of the 25 us that 4,096 x 4,096 outputs cost beside their sums.
+    const bool aligned = (a.gated ? a.N / 2 : a.N) % 8 == 0 && (reinterpret_cast<uintptr_t>(out) & 15) == 0;
+    auto store = [&](auto act, auto gated) {
 #pragma unroll
-    for (int part = 0; part < NT / 4; ++part) {
-        if (part > 0) __syncthreads();
+        for (int part = 0; part < NT / 4; ++part) {
+            if (part > 0) __syncthreads();
 #pragma unroll
-        for (int nt = 0; nt < 4; ++nt)
+            for (int nt = 0; nt < 4; ++nt)
 #pragma unroll
-            for (int rt = 0; rt < RT; ++rt)
-                *reinterpret_cast<f32x4 *>(&shared.results[((wr * RT + rt) * 16 + r) * MoeLds<RT, NT, STAGES>::STRIDE + wn * 64 + nt * 16 + 4 * g]) =
-                    acc[4 * part + nt][rt];
-        __syncthreads();
-        const int c = 8 * (threadIdx.x % 16), n = n0 + c / 64 * 16 * NT + part * 64 + c % 64;
-        if (n < a.N)
-            for (int row = threadIdx.x / 16; row < Product::ROWS; row += 16) {
-                const int slot = slot_of[row];
-                if (slot >= 0)
-                    moe_store8(a, out, out_dtype, first * MOE_TILE + row, slot, weight_of[row], n, &shared.results[row * MoeLds<RT, NT, STAGES>::STRIDE + c]);
-            }
+                for (int rt = 0; rt < RT; ++rt)
+                    *reinterpret_cast<f32x4 *>(&shared.results[((wr * RT + rt) * 16 + r) * MoeLds<RT, NT, STAGES>::STRIDE + wn * 64 + nt * 16 + 4 * g]) =
+                        acc[4 * part + nt][rt];
+            __syncthreads();
+            // (second product: 4 outputs a thread, so that a store takes whole lines)
+            constexpr int AT_ONCE = decltype(act)::value < 0 ? 4 : 8, ACROSS = 128 / AT_ONCE;
+            const int c = AT_ONCE * (threadIdx.x % ACROSS), n = n0 + c / 64 * 16 * NT + part * 64 + c % 64;
+            if (n < a.N)
+                for (int row = threadIdx.x / ACROSS; row < Product::ROWS; row += 256 / ACROSS) {
+                    const int slot = shared.slot_of[row];
+                    const float *v = &shared.results[row * MoeLds<RT, NT, STAGES>::STRIDE + c];
+                    if (slot < 0) continue;
+                    if constexpr (AT_ONCE == 8)
+                        moe_store8<decltype(act)::value, decltype(gated)::value>(a, out, first * MOE_TILE + row, shared.weight_of[row], n, v, aligned);
+                    else moe_store4(a, out, slot, shared.weight_of[row], n, v, aligned);
+                }
+        }
+    };
+#define KVA_MOE_STORE(ACT)                                                                  \
+    case ACT:                                                                               \
+        if (a.gated) store(std::integral_constant<int, ACT>{}, std::true_type{});           \
+        else store(std::integral_constant<int, ACT>{}, std::false_type{});                  \
+        break
+    if (a.mode == 1) {
+        store(std::integral_constant<int, -1>{}, std::false_type{});
+        return;
     }
+    switch (a.act) {
+        KVA_MOE_STORE(0);
+        KVA_MOE_STORE(1);
+        KVA_MOE_STORE(2);
+        KVA_MOE_STORE(3);
+        KVA_MOE_STORE(5);
+        default: store(std::integral_constant<int, 4>{}, std::true_type{});         // (the clamped activation is a gated one)
+    }
+#undef KVA_MOE_STORE
 }
 
 // groups of so many tiles of 16 rows have a kernel of their own (for operands in bf16 whose K is a multiple of 32)
@@ -783,8 +818,8 @@ extern "C" int kva_moe_expert_rows(void *out, int out_dtype, const void *x, cons
     if (max_tiles == 0) return KVA_OK;
     MoeRows a{sorted_slot, tile_expert, slot_weight, top, N, K, mode, act, tiled, gated, limit};
     // (operands at other addresses than multiples of 16: loads that go straight to LDS do not take those, the kernels below do,
-    // over a list in groups as over any other)
-    if (group > 1 && (((uintptr_t)x | (uintptr_t)w) & 15) == 0) {
+    // over a list in groups as over any other; and their rows lie within 2 GiB)
+    if (group > 1 && (((uintptr_t)x | (uintptr_t)w) & 15) == 0 && (long long)max_tiles * MOE_TILE * K * 2 <= 0x7fffffffll) {
         const int groups = max_tiles / group, blocks = wide ? (N + 255) / 256 : (N + 127) / 128;
         KVA_REQUIRE((long long)blocks * groups <= 0x7fffffff, "moe_expert_rows: too many workgroups");
         if (wide)
