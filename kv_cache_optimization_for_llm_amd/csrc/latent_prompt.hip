@@ -28,7 +28,8 @@
 #define LP_DIM 128                  // a head's plain query / key elements, rotated ones, values
 #define LP_ROT 64
 #define LP_VDIM 128
-#define LP_KEYS 32                  // keys a block
+static_assert(LP_DIM == LP_VDIM, "expanded keys and values lie in rows of one size");
+#define LP_KEYS 64                  // keys a block
 #define LP_ROWS 64                  // tokens a workgroup
 
 struct LatentPrompt {
@@ -36,7 +37,7 @@ struct LatentPrompt {
     const bf16_t *q;                // token t, head h: LP_DIM plain elements, then LP_ROT to be rotated, at t q_row + h q_head
     const bf16_t *cache;            // [pages, page_size, rank + rot]
     const bf16_t *w;                // [heads (dim + vdim), rank] in operand order: all heads' U_k, then all heads' U_v
-    bf16_t *kv, *rot;               // expanded: [entries * context, heads (dim + vdim)] and [entries * context, rot]
+    bf16_t *kv, *rot;               // expanded: [entries, keys' heads then values' heads, context, 128] and [entries * context, rot]
     const int *block_table, *entry_seat, *entry_q_start, *entry_start_pos;
     const float *cos, *sin, *sinks; // tables [positions, rot / 2]; one number a head, or none
     const bf16_t *gates;            // or none: one a head at t gate_row + h, or one an element at t gate_row + h gate_head + i
@@ -88,7 +89,8 @@ latent_expand_kernel(LatentPrompt a) {
     __syncthreads();
     const int c = 8 * (threadIdx.x % 32);
     for (int row = threadIdx.x / 32; row < Product::ROWS && m0 + row < keys; row += 8)
-        *reinterpret_cast<uint4 *>(a.kv + (base + m0 + row) * N + n0 + c) = *reinterpret_cast<const uint4 *>(&shared.results[row * STRIDE + c]);
+        *reinterpret_cast<uint4 *>(a.kv + (((size_t)e * 2 * a.heads + (n0 + c) / LP_DIM) * a.context + m0 + row) * LP_DIM + c % LP_DIM) =
+            *reinterpret_cast<const uint4 *>(&shared.results[row * STRIDE + c]);
 }
 
 // 8 keys of value element 16 dt + r as the second product's operand (see latent_attention_mfma.hip: lat_values)
@@ -131,124 +133,180 @@ __device__ __forceinline__ void lp_rotate(Frag8 (&f)[2], const float *cos, const
         for (int i = 0; i < 8; ++i) f[s].h[i] = float_to_bf16_bits(y[s][i]);
 }
 
+// A workgroup takes 64 tokens of one head, 64 keys at a time through LDS; a wavefront 32 of the tokens (wave % 2) and 32 of the keys
+// (wave / 2), and the two halves of the keys are added up at the end.  What bounds it is what the wavefronts read from LDS: 20 KiB
+// of keys and values for 40 products of 16 cycles.  (16 tokens and all keys a wavefront read the same for 20: 2,048 tokens of 16
+// heads 72 us.)  Blocks of keys go through registers, the next ones on their way over the products.
 __global__ void __launch_bounds__(256, 2)
 latent_prompt_kernel(LatentPrompt a, int tiles) {
     constexpr int KD = LP_DIM + LP_ROT, KS = KD / 32, NDT = LP_VDIM / 16;
     constexpr int KSTRIDE = KD + 8, VSTRIDE = LP_VDIM + 24;     // (rows of either kind of read on banks of their own)
-    __shared__ __align__(16) bf16_t Ks[2][LP_KEYS * KSTRIDE];
-    __shared__ __align__(16) bf16_t Vs[2][LP_KEYS * VSTRIDE];
-    const int e = blockIdx.y, head = blockIdx.x % a.heads, tile = tiles - 1 - (int)(blockIdx.x / a.heads);
+    __shared__ __align__(16) union {
+        struct {
+            bf16_t k[LP_KEYS * KSTRIDE], v[LP_KEYS * VSTRIDE];
+        } b;
+        struct {
+            float o[2][2][NDT][KVA_WAVE][4], m[2][2][KVA_WAVE], l[2][2][KVA_WAVE];
+        } half;                                                 // of the wavefronts with the second half of the keys
+    } lds;
+    // The workgroups that the chip takes at once: the longest and the shortest on one compute unit.  More of them: the longest first.
+    const int e = blockIdx.y, head = blockIdx.x % a.heads, at = blockIdx.x / a.heads, front = (tiles + 1) / 2;
+    const int tile = at < front || gridDim.x * gridDim.y > 512 ? tiles - 1 - at : at - front;
     const int q0 = a.entry_q_start[e], n = a.entry_q_start[e + 1] - q0, start = a.entry_start_pos[e];
     if (tile * LP_ROWS >= n) return;
     const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid / KVA_WAVE), lane = tid % KVA_WAVE, r = lane & 15, g = lane >> 4;
-    const int first = tile * LP_ROWS + 16 * wave;               // the wavefront's first token
-    const int mine = min(first + r, n - 1), pos = start + mine;
-    const int hi = first < n ? start + min(first + 15, n - 1) : -1;     // newest key of the wavefront's tokens, and of the workgroup's
+    const int rows = wave & 1, keys = wave >> 1;
+    const int first = tile * LP_ROWS + 32 * rows;               // the wavefront's first token
+    int mine[2];
+#pragma unroll
+    for (int rt = 0; rt < 2; ++rt) mine[rt] = min(first + 16 * rt + r, n - 1);
+    const int hi = first < n ? start + min(first + 31, n - 1) : -1;     // newest key of the wavefront's tokens, and of the workgroup's
     const int end = start + min(tile * LP_ROWS + LP_ROWS, n);           // (one past it)
-    const int N = a.heads * (LP_DIM + LP_VDIM);
-    const bf16_t *kv = a.kv + (size_t)e * a.context * N + head * LP_DIM, *rot = a.rot + (size_t)e * a.context * LP_ROT;
+    const bf16_t *kv = a.kv + ((size_t)e * 2 * a.heads + head) * a.context * LP_DIM, *rot = a.rot + (size_t)e * a.context * LP_ROT;
 
-    Frag8 qf[KS];
-    {
-        const bf16_t *q = a.q + (size_t)(q0 + mine) * a.q_row + (size_t)head * a.q_head + 8 * g;
+    Frag8 qf[2][KS];
 #pragma unroll
-        for (int ks = 0; ks < KS; ++ks) qf[ks].u4 = *reinterpret_cast<const uint4 *>(q + 32 * ks);
-        Frag8 turned[2] = {qf[KS - 2], qf[KS - 1]};
-        lp_rotate(turned, a.cos + (size_t)pos * (LP_ROT / 2), a.sin + (size_t)pos * (LP_ROT / 2), g, a.interleaved != 0);
-        qf[KS - 2] = turned[0];
-        qf[KS - 1] = turned[1];
+    for (int rt = 0; rt < 2; ++rt) {
+        const bf16_t *q = a.q + (size_t)(q0 + mine[rt]) * a.q_row + (size_t)head * a.q_head + 8 * g;
+#pragma unroll
+        for (int ks = 0; ks < KS; ++ks) qf[rt][ks].u4 = *reinterpret_cast<const uint4 *>(q + 32 * ks);
+        Frag8 turned[2] = {qf[rt][KS - 2], qf[rt][KS - 1]};
+        const size_t table = (size_t)(start + mine[rt]) * (LP_ROT / 2);
+        lp_rotate(turned, a.cos + table, a.sin + table, g, a.interleaved != 0);
+        qf[rt][KS - 2] = turned[0];
+        qf[rt][KS - 1] = turned[1];
     }
-    // a block's pieces on their way: rows tid / 16 and 16 further of keys and values, row tid / 8 of the rotated parts
-    uint4 k_lo, k_hi, v_lo, v_hi, turned_k;
+    // a block's pieces on their way: rows tid / 16 and 16, 32, 48 further of keys and values, tid / 8 and 32 further of the rotated parts
+    kva_u32x4 kx[4], vx[4], tx[2];
     auto load = [&](int k0) {
-        const bf16_t *lo = kv + (size_t)min(k0 + tid / 16, end - 1) * N + 8 * (tid % 16);
-        const bf16_t *up = kv + (size_t)min(k0 + tid / 16 + 16, end - 1) * N + 8 * (tid % 16);
-        k_lo = *reinterpret_cast<const uint4 *>(lo);
-        v_lo = *reinterpret_cast<const uint4 *>(lo + a.heads * LP_DIM);
-        k_hi = *reinterpret_cast<const uint4 *>(up);
-        v_hi = *reinterpret_cast<const uint4 *>(up + a.heads * LP_DIM);
-        turned_k = *reinterpret_cast<const uint4 *>(rot + (size_t)min(k0 + tid / 8, end - 1) * LP_ROT + 8 * (tid % 8));
-    };
-    f32x4 o[NDT];
 #pragma unroll
-    for (int dt = 0; dt < NDT; ++dt) o[dt] = f32x4{0.f, 0.f, 0.f, 0.f};
-    float m = -INFINITY, l = 0.f;                               // m in the base-2 domain, l this lane's part
+        for (int j = 0; j < 4; ++j) {
+            const bf16_t *row = kv + (size_t)min(k0 + tid / 16 + 16 * j, end - 1) * LP_DIM + 8 * (tid % 16);
+            kx[j] = *reinterpret_cast<const kva_u32x4 *>(row);
+            vx[j] = *reinterpret_cast<const kva_u32x4 *>(row + (size_t)a.heads * a.context * LP_DIM);
+        }
+#pragma unroll
+        for (int j = 0; j < 2; ++j)
+            tx[j] = *reinterpret_cast<const kva_u32x4 *>(rot + (size_t)min(k0 + tid / 8 + 32 * j, end - 1) * LP_ROT + 8 * (tid % 8));
+    };
+    f32x4 o[2][NDT];
+    float m[2] = {-INFINITY, -INFINITY}, l[2] = {0.f, 0.f};     // m in the base-2 domain, l this lane's part
+#pragma unroll
+    for (int rt = 0; rt < 2; ++rt)
+#pragma unroll
+        for (int dt = 0; dt < NDT; ++dt) o[rt][dt] = f32x4{0.f, 0.f, 0.f, 0.f};
     const float scale2 = a.scale * LP_LOG2E;
     load(0);
-    for (int k0 = 0, buf = 0; k0 < end; k0 += LP_KEYS, buf ^= 1) {
-        bf16_t *kp = &Ks[buf][tid / 16 * KSTRIDE + 8 * (tid % 16)], *vp = &Vs[buf][tid / 16 * VSTRIDE + 8 * (tid % 16)];
-        *reinterpret_cast<uint4 *>(kp) = k_lo;
-        *reinterpret_cast<uint4 *>(kp + 16 * KSTRIDE) = k_hi;
-        *reinterpret_cast<uint4 *>(vp) = v_lo;
-        *reinterpret_cast<uint4 *>(vp + 16 * VSTRIDE) = v_hi;
-        *reinterpret_cast<uint4 *>(&Ks[buf][tid / 8 * KSTRIDE + LP_DIM + 8 * (tid % 8)]) = turned_k;
-        __syncthreads();            // (a buffer was read last two turns ago: every wavefront has passed the barrier between)
+    for (int k0 = 0; k0 < end; k0 += LP_KEYS) {
+        __syncthreads();                                        // every wavefront is done with the block before
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            *reinterpret_cast<kva_u32x4 *>(&lds.b.k[(tid / 16 + 16 * j) * KSTRIDE + 8 * (tid % 16)]) = kx[j];
+            *reinterpret_cast<kva_u32x4 *>(&lds.b.v[(tid / 16 + 16 * j) * VSTRIDE + 8 * (tid % 16)]) = vx[j];
+        }
+#pragma unroll
+        for (int j = 0; j < 2; ++j)
+            *reinterpret_cast<kva_u32x4 *>(&lds.b.k[(tid / 8 + 32 * j) * KSTRIDE + LP_DIM + 8 * (tid % 8)]) = tx[j];
+        __syncthreads();
         if (k0 + LP_KEYS < end) load(k0 + LP_KEYS);
-        if (k0 > hi) continue;                                  // (the wavefront's tokens see none of these)
-        f32x4 s[2] = {f32x4{0.f, 0.f, 0.f, 0.f}, f32x4{0.f, 0.f, 0.f, 0.f}};
+        const int kb = k0 + 32 * keys;
+        if (kb > hi) continue;                                  // (the wavefront's tokens see none of these)
+        const bf16_t *kp = &lds.b.k[(32 * keys + r) * KSTRIDE + 8 * g];
+        f32x4 s[2][2];
+#pragma unroll
+        for (int rt = 0; rt < 2; ++rt)
+#pragma unroll
+            for (int t = 0; t < 2; ++t) s[rt][t] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
         for (int ks = 0; ks < KS; ++ks)
 #pragma unroll
             for (int t = 0; t < 2; ++t) {
                 Frag8 k;
-                k.u4 = *reinterpret_cast<const uint4 *>(&Ks[buf][(16 * t + r) * KSTRIDE + 32 * ks + 8 * g]);
-                s[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(k.v, qf[ks].v, s[t], 0, 0, 0);
-            }
-        const bool whole = k0 + LP_KEYS - 1 <= start + first;   // all of the wavefront's tokens see all of the keys
-        float sv[8], mx = -INFINITY;
+                k.u4 = *reinterpret_cast<const uint4 *>(kp + 16 * t * KSTRIDE + 32 * ks);
 #pragma unroll
-        for (int t = 0; t < 2; ++t)
+                for (int rt = 0; rt < 2; ++rt) s[rt][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(k.v, qf[rt][ks].v, s[rt][t], 0, 0, 0);
+            }
+        Frag8 pf[2];
+#pragma unroll
+        for (int rt = 0; rt < 2; ++rt) {
+            const int pos = start + mine[rt];
+            const bool whole = kb + 31 <= start + first + 16 * rt;      // all of the tile's tokens see all of the keys
+            float sv[8], mx = -INFINITY;
+#pragma unroll
+            for (int t = 0; t < 2; ++t)
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    float x = s[rt][t][i] * scale2;
+                    if (!whole) x = kb + 16 * t + 4 * g + i <= pos ? x : -INFINITY;
+                    sv[4 * t + i] = x;
+                    mx = fmaxf(mx, x);
+                }
+            const float bm = quad_rows_max(mx);
+            // (the reference of the exponentials moves only when a maximum has grown by more than 2^8)
+            if (__builtin_amdgcn_ballot_w64(bm > m[rt] + 8.f) != 0) {
+                const float m_new = fmaxf(m[rt], bm), corr = __builtin_amdgcn_exp2f(m[rt] - ((m_new == -INFINITY) ? 0.f : m_new));     // exp2(-inf) = 0
+                l[rt] *= corr;
+#pragma unroll
+                for (int dt = 0; dt < NDT; ++dt)
+#pragma unroll
+                    for (int c = 0; c < 4; ++c) o[rt][dt][c] *= corr;
+                m[rt] = m_new;
+            }
+            const float ref = m[rt] == -INFINITY ? 0.f : m[rt];
+#pragma unroll
+            for (int j = 0; j < 8; j += 2) {
+                const float p0 = __builtin_amdgcn_exp2f(sv[j] - ref), p1 = __builtin_amdgcn_exp2f(sv[j + 1] - ref);
+                l[rt] += p0 + p1;
+                pf[rt].p2[j / 2] = pack_bf16(p0, p1);
+            }
+        }
+        const bf16_t *get = &lds.b.v[(32 * keys + 4 * g + (r >> 2)) * VSTRIDE + 4 * (r & 3)];
+#pragma unroll
+        for (int dt = 0; dt < NDT; ++dt) {
+            const Frag8 v = lp_values<VSTRIDE>(get, dt);
+#pragma unroll
+            for (int rt = 0; rt < 2; ++rt) o[rt][dt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(v.v, pf[rt].v, o[rt][dt], 0, 0, 0);
+        }
+    }
+    __syncthreads();
+    if (keys == 1) {
+#pragma unroll
+        for (int rt = 0; rt < 2; ++rt) {
+            lds.half.m[rows][rt][lane] = m[rt];
+            lds.half.l[rows][rt][lane] = l[rt];
+#pragma unroll
+            for (int dt = 0; dt < NDT; ++dt) *reinterpret_cast<f32x4 *>(lds.half.o[rows][rt][dt][lane]) = o[rt][dt];
+        }
+    }
+    __syncthreads();
+    if (keys == 1) return;
+#pragma unroll
+    for (int rt = 0; rt < 2; ++rt) {
+        const float other = lds.half.m[rows][rt][lane], both = fmaxf(m[rt], other), ref = both == -INFINITY ? 0.f : both;
+        const float c0 = __builtin_amdgcn_exp2f(m[rt] - ref), c1 = __builtin_amdgcn_exp2f(other - ref);
+        const float sum = quad_rows_sum(l[rt] * c0 + lds.half.l[rows][rt][lane] * c1);
+        if (first + 16 * rt + r >= n) continue;
+        float mul = 1.f / sum;
+        if (a.sinks) {                                          // one more term of the denominator, with no key and no value
+            const float sk = a.sinks[head] * LP_LOG2E, m_new = fmaxf(both, sk), corr = __builtin_amdgcn_exp2f(both - m_new);
+            mul = corr / (sum * corr + __builtin_amdgcn_exp2f(sk - m_new));
+        }
+        const bf16_t *gate = a.gates ? a.gates + (size_t)(q0 + mine[rt]) * a.gate_row : nullptr;
+        if (gate && !a.gate_per_element) mul *= 1.f / (1.f + expf(-to_float(gate[head])));
+        bf16_t *out = a.out + ((size_t)(q0 + mine[rt]) * a.heads + head) * LP_VDIM;
+#pragma unroll
+        for (int dt = 0; dt < NDT; ++dt) {
+            const int c = 16 * dt + 4 * g;
+            const f32x4 more = *reinterpret_cast<const f32x4 *>(lds.half.o[rows][rt][dt][lane]);
+            float v[4];
 #pragma unroll
             for (int i = 0; i < 4; ++i) {
-                float x = s[t][i] * scale2;
-                if (!whole) x = k0 + 16 * t + 4 * g + i <= pos ? x : -INFINITY;
-                sv[4 * t + i] = x;
-                mx = fmaxf(mx, x);
+                v[i] = (o[rt][dt][i] * c0 + more[i] * c1) * mul;
+                if (gate && a.gate_per_element) v[i] *= 1.f / (1.f + expf(-to_float(gate[(size_t)head * a.gate_head + c + i])));
             }
-        const float bm = quad_rows_max(mx);
-        // (the reference of the exponentials moves only when a maximum has grown by more than 2^8)
-        if (__builtin_amdgcn_ballot_w64(bm > m + 8.f) != 0) {
-            const float m_new = fmaxf(m, bm), corr = __builtin_amdgcn_exp2f(m - ((m_new == -INFINITY) ? 0.f : m_new));     // exp2(-inf) = 0
-            l *= corr;
-#pragma unroll
-            for (int dt = 0; dt < NDT; ++dt)
-#pragma unroll
-                for (int c = 0; c < 4; ++c) o[dt][c] *= corr;
-            m = m_new;
+            const b16x2 lo = pack_bf16(v[0], v[1]), hi2 = pack_bf16(v[2], v[3]);
+            *reinterpret_cast<uint2 *>(out + c) = make_uint2(__builtin_bit_cast(unsigned, lo), __builtin_bit_cast(unsigned, hi2));
         }
-        const float ref = m == -INFINITY ? 0.f : m;
-        Frag8 pf;
-#pragma unroll
-        for (int j = 0; j < 8; j += 2) {
-            const float p0 = __builtin_amdgcn_exp2f(sv[j] - ref), p1 = __builtin_amdgcn_exp2f(sv[j + 1] - ref);
-            l += p0 + p1;
-            pf.p2[j / 2] = pack_bf16(p0, p1);
-        }
-        const bf16_t *get = &Vs[buf][(4 * g + (r >> 2)) * VSTRIDE + 4 * (r & 3)];
-#pragma unroll
-        for (int dt = 0; dt < NDT; ++dt) o[dt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(lp_values<VSTRIDE>(get, dt).v, pf.v, o[dt], 0, 0, 0);
-    }
-    l = quad_rows_sum(l);
-    if (first + r >= n) return;
-    float mul = 1.f / l;
-    if (a.sinks) {                                              // one more term of the denominator, with no key and no value
-        const float sk = a.sinks[head] * LP_LOG2E, m_new = fmaxf(m, sk), corr = __builtin_amdgcn_exp2f(m - m_new);
-        mul = corr / (l * corr + __builtin_amdgcn_exp2f(sk - m_new));
-    }
-    const bf16_t *gate = a.gates ? a.gates + (size_t)(q0 + mine) * a.gate_row : nullptr;
-    if (gate && !a.gate_per_element) mul *= 1.f / (1.f + expf(-to_float(gate[head])));
-    bf16_t *out = a.out + ((size_t)(q0 + mine) * a.heads + head) * LP_VDIM;
-#pragma unroll
-    for (int dt = 0; dt < NDT; ++dt) {
-        const int c = 16 * dt + 4 * g;
-        float v[4];
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            v[i] = o[dt][i] * mul;
-            if (gate && a.gate_per_element) v[i] *= 1.f / (1.f + expf(-to_float(gate[(size_t)head * a.gate_head + c + i])));
-        }
-        const b16x2 lo = pack_bf16(v[0], v[1]), hi2 = pack_bf16(v[2], v[3]);
-        *reinterpret_cast<uint2 *>(out + c) = make_uint2(__builtin_bit_cast(unsigned, lo), __builtin_bit_cast(unsigned, hi2));
     }
 }
 
