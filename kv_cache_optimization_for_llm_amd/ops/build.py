@@ -1,7 +1,7 @@
 """Compiles the HIP kernels (gfx950) and the host allocators into two shared libraries.
 
 ``libkva_hip.so``  - every ``csrc/*.hip`` file, compiled with hipcc for gfx950.
-``libkva_host.so`` - ``csrc/host/*.cpp``, plain C++ (no GPU runtime needed to load it).
+``libkva_host.so`` - ``csrc/host/*.cpp``, C++ without a GPU runtime; one function takes Python objects.
 
 Libraries are kept in ``<package>/_lib`` when that folder can be written, otherwise in a
 per-user folder under the system's temporary directory.  A stamp file holds a hash of the
@@ -14,6 +14,7 @@ import os
 import shutil
 import subprocess
 import sys
+import sysconfig
 import tempfile
 import time
 from concurrent.futures import ThreadPoolExecutor
@@ -188,7 +189,7 @@ def build_host(force: bool = False) -> str:
     lib = os.path.join(out_dir, name)
     tmp = lib + f".tmp{os.getpid()}"
     _say(f"compiling host allocators into {out_dir}")
-    _run([cxx, *HOST_FLAGS, *_host_sources(), "-o", tmp], "compiling " + name)
+    _run([cxx, *HOST_FLAGS, "-I", sysconfig.get_paths()["include"], *_host_sources(), "-o", tmp], "compiling " + name)
     os.replace(tmp, lib)
     with open(lib + ".stamp", "w") as f:
         f.write(digest + "\n")

@@ -219,3 +219,19 @@ def host_lib():
             fn.restype = res
         _host = lib
         return _host
+
+
+_sample_rows = None
+
+
+def sample_rows():
+    """``kva_sample_rows`` of the host library (it takes Python objects and is called with the interpreter's lock held),
+    or None where the library was built without the interpreter's headers."""
+    global _sample_rows
+    if _sample_rows is None:
+        host_lib()
+        fn = getattr(ctypes.PyDLL(build.build_host()), "kva_sample_rows", False)
+        if fn:
+            fn.argtypes, fn.restype = [ctypes.py_object, LL, P, LL, I], I
+        _sample_rows = fn
+    return _sample_rows or None

@@ -23,6 +23,7 @@ import numpy as np
 import torch
 
 from ..ops import kernels as K
+from ..ops.library import sample_rows
 
 
 def counter_uniform(seed: int, key: int, step: int) -> float:
@@ -54,6 +55,23 @@ class _Staging:
         self.i32 = self.pinned.numpy()
         self.u32, self.f32 = self.i32.view(np.uint32), self.i32.view(np.float32)
         self.sent = None                    # an event behind the copy
+
+
+def _read_rows(rows: Sequence[SampleRow], n: int, staging: Optional[_Staging], seats: bool) -> int:
+    """Bit 0: a row has a temperature, bit 1: a row asks for the penalty.  ``staging`` takes the rows' arguments, with ``seats``
+    the seats too."""
+    native = sample_rows()
+    if native is not None:
+        return native(rows, n, staging.pinned.data_ptr() if staging is not None else None,
+                      staging.i32.shape[1] if staging is not None else 0, 1 if seats else 0)
+    if staging is not None:
+        staging.f32[0, :n] = [1.0 / r.temperature if r.temperature > 0 else 0.0 for r in rows]
+        staging.u32[1, :n] = [int(r.rng_key) & 0xFFFFFFFF for r in rows]
+        staging.u32[2, :n] = [int(r.rng_step) & 0xFFFFFFFF for r in rows]
+        if seats:
+            staging.i32[3, :n] = [r.seat if r.apply_penalty else -1 for r in rows]
+            staging.i32[4, :n] = [r.seat for r in rows]
+    return (1 if any(r.temperature > 0 for r in rows) else 0) | (2 if any(r.apply_penalty for r in rows) else 0)
 
 
 class PendingTokens:
@@ -161,24 +179,20 @@ class Sampler:
         if n == 0:
             event.record()
             return PendingTokens(host, event, 0)
-        any_sampled = any(r.temperature > 0 for r in rows)
-        use_mask = self.mask is not None and any(r.apply_penalty for r in rows)
+        flags = _read_rows(rows, n, None, False)
+        any_sampled, use_mask = bool(flags & 1), self.mask is not None and bool(flags & 2)
         inv_t = key = step = seat_t = mark_seat = None
         if any_sampled or self.mask is not None:
             # the per-row arguments go up in one copy from pinned memory (five small pageable
             # tensors, each copied by itself, were 0.4 ms of host time apiece in a serving loop)
             staging, (dev_t, dev_key, dev_step, dev_seat, dev_mark) = self._row_arguments(n)
+            _read_rows(rows, n, staging, self.mask is not None)
             if any_sampled:
-                staging.f32[0, :n] = [1.0 / r.temperature if r.temperature > 0 else 0.0 for r in rows]
-                staging.u32[1, :n] = [int(r.rng_key) & 0xFFFFFFFF for r in rows]
-                staging.u32[2, :n] = [int(r.rng_step) & 0xFFFFFFFF for r in rows]
                 inv_t, key, step = dev_t, dev_key, dev_step
             if use_mask:
-                staging.i32[3, :n] = [r.seat if r.apply_penalty else -1 for r in rows]
                 seat_t = dev_seat
             if self.mask is not None:
                 # every token a request emits is marked in its mask row, by the launch that chooses it
-                staging.i32[4, :n] = [r.seat for r in rows]
                 mark_seat = dev_mark
             # (torch's own copy: its allocator then knows that the block is in use until the copy has left it, also when this
             # sampler goes away or takes larger ones before)

@@ -1,0 +1,44 @@
+"""Per-row arguments of a sampling: the native reader against the comprehensions it stands for, bit for bit."""
+import types
+
+import numpy as np
+import pytest
+import torch
+
+from kv_cache_optimization_for_llm_amd.ops.library import sample_rows
+from kv_cache_optimization_for_llm_amd.sampling import sampler as S
+
+
+def staging(rows):
+    s = types.SimpleNamespace(pinned=torch.full((5, rows), -7, dtype=torch.int32))
+    s.i32 = s.pinned.numpy()
+    s.u32, s.f32 = s.i32.view(np.uint32), s.i32.view(np.float32)
+    return s
+
+
+ROWS = [S.SampleRow(0), S.SampleRow(3, 0.8, 8, 100), S.SampleRow(7, -1.0, -5, 1 << 40, True), S.SampleRow(np.int64(2), np.float32(1.5), np.int64(-1), np.uint8(9)),
+        S.SampleRow(5, 2, (1 << 70) + 3, 7.9, np.bool_(True)), S.SampleRow(1, float("nan"), True, 2), S.SampleRow(4, 1e-45, np.uint32(0xFFFFFFFF), -(1 << 33))]
+
+
+@pytest.mark.parametrize("rows, room", [([], 1), (ROWS[:1], 1), (ROWS, 7), (tuple(ROWS * 20), 256)])
+@pytest.mark.parametrize("seats", [False, True])
+def test_native_reader_against_the_comprehensions(rows, room, seats, monkeypatch):
+    assert sample_rows() is not None
+    got, want = staging(room), staging(room)
+    with np.errstate(over="ignore"):
+        flags = S._read_rows(rows, len(rows), got, seats)
+        assert flags == S._read_rows(rows, len(rows), None, False)
+        monkeypatch.setattr(S, "sample_rows", lambda: None)
+        assert flags == S._read_rows(rows, len(rows), want, seats)
+    assert np.array_equal(got.i32, want.i32)
+
+
+def test_what_the_comprehensions_raise_is_raised():
+    with pytest.raises(AttributeError):
+        S._read_rows([types.SimpleNamespace(temperature=0.5)], 1, staging(1), False)
+    with pytest.raises(TypeError):
+        S._read_rows([S.SampleRow(0, None)], 1, staging(1), False)
+    with pytest.raises((ValueError, TypeError)):
+        S._read_rows([S.SampleRow(0, 0.5, "x")], 1, staging(1), False)
+    with pytest.raises(OverflowError):
+        S._read_rows([S.SampleRow(1 << 40, 0.5)], 1, staging(1), True)
