@@ -230,6 +230,12 @@ _SHARED_FOUR_BELOW_WIDE = 257
 _SHARED_FOUR_FROM_SHORT_WIDE = 127
 _SHARED_FOUR_FROM = 128             # more (item, kv head) pairs than this ...
 _SHARED_FOUR_BELOW = 512            # ... and fewer than this: four ranges in one workgroup
+# ... and from so many keys on at 512 pairs too, which the chip still takes at once, two workgroups a compute unit.  Steps of 64 requests,
+# 6 layers of the 1B sizes, contexts alike / down to half / down to a tenth, a wavefront a pair -> four: at 1,000 keys 622 / 620 / 621 ->
+# 623 / 600 / 580 us, 1,400 681 / 667 / 665 -> 672 / 648 / 615, 2,000 740 / 739 / 735 -> 755 / 696 / 664, 3,000 884 / 817 / 753 -> 870 /
+# 814 / 755: what one wavefront takes for the longest context is what a step waits for.  72 to 96 requests lose 1-6 % with contexts
+# alike and gain 1-5 % where they differ most: not there.
+_SHARED_FOUR_FULL_FROM = 1024
 _SHARED_SHORT_CONTEXT = 1024        # up to this many keys already from ...
 _SHARED_FOUR_FROM_SHORT = 63        # ... this many pairs (8 / 12 / 16 requests at 768 keys 0.854 / 0.912 / 0.959 ->
                                     # 0.852 / 0.900 / 0.945 ms; but 8 at 2,048 keys 0.930 -> 0.978, 16 at 8,192 1.56 -> 1.73)
@@ -298,6 +304,8 @@ def choose_decode_ranges(num_items: int, num_kv_heads: int, max_context: int, he
     """(key ranges, keys per range, wavefronts per workgroup) for decoded tokens."""
     pairs = max(1, num_items * num_kv_heads)
     below = _SHARED_FOUR_BELOW if max_context < _SHARED_LONG_CONTEXT else _SHARED_FOUR_BELOW_LONG
+    if _SHARED_FOUR_FULL_FROM <= max_context < _SHARED_LONG_CONTEXT:
+        below = _SHARED_FOUR_BELOW + 1
     wide = head_dim > _SHARED_TUNED_HEAD_DIM
     if wide:
         below = _SHARED_FOUR_BELOW_WIDE

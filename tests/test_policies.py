@@ -55,6 +55,9 @@ def test_where_decoded_tokens_need_no_merge_launch():
         assert choose_decode_ranges(items, 8, 768, 64, KERNEL_MAX_SPLITS) == (4, 192, 4)
     assert choose_decode_ranges(64, 8, 768, 64, KERNEL_MAX_SPLITS) == (1, 0, 1)          # enough wavefronts as they are
     assert choose_decode_ranges(64, 8, 8192, 64, KERNEL_MAX_SPLITS) == (4, 2048, 4)      # but not for long contexts
+    for context, want in ((1023, 1), (1024, 4), (4095, 4)):                                # as many as the chip takes at once, long enough
+        assert choose_decode_ranges(64, 8, context, 64, KERNEL_MAX_SPLITS)[2] == want
+        assert choose_decode_ranges(65, 8, context, 64, KERNEL_MAX_SPLITS) == (1, 0, 1)
     assert choose_decode_ranges(20, 8, 100, 64, KERNEL_MAX_SPLITS) == (2, 64, 2)
     # many ranges share a workgroup only where the merge has much to read
     assert choose_decode_ranges(8, 8, 8192, 64, KERNEL_MAX_SPLITS) == (16, 512, 4)
