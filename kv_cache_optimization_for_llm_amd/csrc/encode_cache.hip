@@ -150,7 +150,7 @@ qk_encode_cache_vec_kernel(bf16_t *__restrict__ qkv, int row_stride, int k_off, 
     const int slot = slot_mapping ? slot_mapping[t] : -1;
     const int page = slot >= 0 ? slot / page_size : 0, off = slot >= 0 ? slot % page_size : 0;
     const int total = (num_q_heads + num_kv_heads) * vecs;
-    for (int w0 = 0; w0 < total; w0 += blockDim.x) {              // (uniform trip count: the lanes of a head shuffle)
+    for (int w0 = blockIdx.y * blockDim.x; w0 < total; w0 += blockDim.x * gridDim.y) {    // (uniform trip count: the lanes of a head shuffle)
         const int w = w0 + threadIdx.x;
         const bool on = w < total;
         const int head = on ? w / vecs : 0, j = on ? w % vecs : 0;
@@ -217,7 +217,7 @@ qk_encode_cache_vec_kernel(bf16_t *__restrict__ qkv, int row_stride, int k_off, 
     if (slot >= 0) {
         const bf16_t *v = row + v_off;
         const bf16_t *vb = bias ? bias + (size_t)(num_q_heads + num_kv_heads) * head_dim : nullptr;
-        for (int w = threadIdx.x; w < num_kv_heads * value_dim; w += blockDim.x) {
+        for (int w = blockIdx.y * blockDim.x + threadIdx.x; w < num_kv_heads * value_dim; w += blockDim.x * gridDim.y) {
             const int kvh = w / value_dim, j = w % value_dim;
             v_cache[(((size_t)page * num_kv_heads + kvh) * value_dim + j) * page_size + off] =
                 vb ? from_float<bf16_t>(to_float(v[w]) + to_float(vb[w])) : v[w];
@@ -254,7 +254,8 @@ extern "C" int kva_qk_encode_cache(void *qkv, int row_stride, int k_off, int v_o
                            (interleaved || rot == 0 ? 0 : (uintptr_t)cos_table | (uintptr_t)sin_table);
     if (dtype == KVA_BF16 && head_dim % 8 == 0 && (vecs & (vecs - 1)) == 0 && vecs <= KVA_WAVE &&
         (interleaved || rot % 16 == 0) && row_stride % 8 == 0 && k_off % 8 == 0 && (wide & 15) == 0) {
-        hipLaunchKernelGGL(qk_encode_cache_vec_kernel, dim3(tokens), dim3(256), 0, stream, (bf16_t *)qkv, row_stride,
+        // (a workgroup a turn over the heads: a second turn behind the first was a second chain of trips to memory)
+        hipLaunchKernelGGL(qk_encode_cache_vec_kernel, dim3(tokens, ((num_q_heads + num_kv_heads) * vecs + 255) / 256), dim3(256), 0, stream, (bf16_t *)qkv, row_stride,
                            k_off, v_off, (bf16_t *)k_cache, (bf16_t *)v_cache, cos_table, sin_table, positions,
                            slot_mapping, num_q_heads, num_kv_heads, head_dim, value_dim, rot, interleaved, unit_eps,
                            page_size, (const bf16_t *)bias, q_weight, k_weight, norm_first);
@@ -449,7 +450,7 @@ maps_encode_cache_vec_kernel(const bf16_t *__restrict__ qkv, int row_stride, bf1
     const int slot = slot_mapping ? slot_mapping[t] : -1;
     const int page = slot >= 0 ? slot / page_size : 0, off = slot >= 0 ? slot % page_size : 0;
     const int vecs = dim / 8, maps = 2 * heads + (slot >= 0 ? 2 * kv_heads : 0);
-    for (int w = threadIdx.x; w < maps * vecs; w += blockDim.x) {
+    for (int w = blockIdx.y * blockDim.x + threadIdx.x; w < maps * vecs; w += blockDim.x * gridDim.y) {
         const int m = w / vecs, j = w % vecs;
         const int at = m * dim + 8 * j;
         const uint4 in = *reinterpret_cast<const uint4 *>(row + at);
@@ -487,7 +488,7 @@ maps_encode_cache_vec_kernel(const bf16_t *__restrict__ qkv, int row_stride, bf1
     }
     if (slot >= 0) {
         const int v_off = 2 * (heads + kv_heads) * dim;
-        for (int w = threadIdx.x; w < kv_heads * value_dim; w += blockDim.x)
+        for (int w = blockIdx.y * blockDim.x + threadIdx.x; w < kv_heads * value_dim; w += blockDim.x * gridDim.y)
             v_cache[((size_t)page * kv_heads * value_dim + w) * page_size + off] =
                 bias ? from_float<bf16_t>(to_float(row[v_off + w]) + bias[v_off + w]) : row[v_off + w];
     }
@@ -513,7 +514,7 @@ extern "C" int kva_maps_encode_cache(const void *qkv, int row_stride, void *q_ro
     if (rot == 0) cos_table = sin_table = reinterpret_cast<const float *>(qkv);     // never read
     if (dtype == KVA_BF16 && interleaved && dim % 8 == 0 && row_stride % 8 == 0 &&
         ((reinterpret_cast<uintptr_t>(qkv) | reinterpret_cast<uintptr_t>(q_rows) | reinterpret_cast<uintptr_t>(bias)) & 15) == 0)
-        hipLaunchKernelGGL(maps_encode_cache_vec_kernel, dim3(tokens), dim3(256), 0, stream, (const bf16_t *)qkv, row_stride,
+        hipLaunchKernelGGL(maps_encode_cache_vec_kernel, dim3(tokens, (2 * (heads + kv_heads) * (dim / 8) + 255) / 256), dim3(256), 0, stream, (const bf16_t *)qkv, row_stride,
                            (bf16_t *)q_rows, (bf16_t *)k_cache, (bf16_t *)v_cache, cos_table, sin_table, positions,
                            slot_mapping, heads, kv_heads, dim, value_dim, rot, page_size, bias);
     else if (dtype == KVA_F32)
