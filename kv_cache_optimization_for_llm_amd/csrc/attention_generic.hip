@@ -47,8 +47,10 @@ template <> struct Vec4<bf16_t> {
 // 4 keys) a lane reads its value element of 4 keys at once, a row of the transposed page, and 32 keys' loads are under way
 // together; a head's additions keep their order in every variant, so its bits do too.  One key's values a load, one head a
 // wavefront -> this, fp32, us: 603 tokens of 32 heads of 64 over 8 key heads at up to 201 / 2,000 keys 253 / 731 -> 35 / 78,
-// one token at 200 / 2,000 keys 34 / 307 -> 11 / 75 (bound by the chains: 64 dependent additions a block for the score,
-// 64 for the values), heads of 128 at 2,000 keys 659 -> 185.
+// one token at 200 / 2,000 keys 34 / 307 -> 11 / 77 (bound by the chains: 64 dependent additions a block for the score,
+// 64 for the values), heads of 128 at 2,000 keys 659 -> 185.  A head alone, which is what few rows get, has all of a block's
+// loads under way together instead of a quarter and a half of them: 3 tokens at up to 200 keys 11.3 -> 10.6 (heads of 128 17.0 ->
+// 15.5), one at 2,000 77 -> 66; several heads a wavefront have no registers for it and other wavefronts to hide behind.
 template <typename T, int H>
 __global__ void __launch_bounds__(KVA_WAVE)
 attention_rowwise_kernel(T *__restrict__ out, const T *__restrict__ q, int q_row_stride,
@@ -60,6 +62,8 @@ attention_rowwise_kernel(T *__restrict__ out, const T *__restrict__ q, int q_row
     __shared__ __attribute__((aligned(16))) float q_s[H][ATTN_MAX_HEAD_DIM];
     __shared__ __attribute__((aligned(16))) float p_s[H][KVA_WAVE];
     __shared__ long long voff_s[KVA_WAVE];
+    // (of a head alone all of a key's elements, and all values of a block, are asked for before the first is used)
+    constexpr int KEY_LOADS = H == 1 ? 16 : 4, FOURS = H == 1 ? 16 : 8;
 
     const int t = blockIdx.x;
     const int qh = blockIdx.y * H;
@@ -101,7 +105,7 @@ attention_rowwise_kernel(T *__restrict__ out, const T *__restrict__ q, int q_row
             float dot[H];
 #pragma unroll
             for (int h = 0; h < H; ++h) dot[h] = 0.f;
-#pragma unroll 4
+#pragma unroll KEY_LOADS
             for (int j = 0; j < head_dim; j += 4) {
                 float kv[4];
                 Vec4<T>::load(kpage + kva_k_at(krow, j, page_size, kc), kv);     // (4 elements never straddle a chunk)
@@ -145,19 +149,19 @@ attention_rowwise_kernel(T *__restrict__ out, const T *__restrict__ q, int q_row
 #pragma unroll
                 for (int h = 0; h < H; ++h) a[h] = acc[c][h] * corr[h];
                 if (fours) {
-                    for (int i0 = 0; i0 <= last; i0 += 32) {
-                        float v[8][4];
+                    for (int i0 = 0; i0 <= last; i0 += 4 * FOURS) {
+                        float v[FOURS][4];
 #pragma unroll
-                        for (int g = 0; g < 8; ++g) Vec4<T>::load(vcol + voff_s[i0 + 4 * g], v[g]);
-                        const uint32_t these = (uint32_t)(seen >> i0);
-                        if (these != 0xffffffffu) {
+                        for (int g = 0; g < FOURS; ++g) Vec4<T>::load(vcol + voff_s[i0 + 4 * g], v[g]);
+                        const unsigned long long these = seen >> i0;
+                        if (seen != ~0ull) {
 #pragma unroll
-                            for (int g = 0; g < 8; ++g)
+                            for (int g = 0; g < FOURS; ++g)
 #pragma unroll
                                 for (int u = 0; u < 4; ++u) v[g][u] = (these >> (4 * g + u)) & 1 ? v[g][u] : 0.f;
                         }
 #pragma unroll
-                        for (int g = 0; g < 8; ++g)
+                        for (int g = 0; g < FOURS; ++g)
 #pragma unroll
                             for (int h = 0; h < H; ++h) {
                                 const float4 p = *reinterpret_cast<const float4 *>(&p_s[h][i0 + 4 * g]);
