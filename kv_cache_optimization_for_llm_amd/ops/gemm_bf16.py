@@ -91,6 +91,20 @@ def use_gemv(m: int, n: int, k: int) -> bool:
     return not (n >= GEMV_WIDE_N and k >= GEMV_LONG_K[m] and K.gemm_skinny_supported(m, n, k))
 
 
+# A few outputs past a multiple of 256 (a mixer's gates and decays behind its projections) cost the library's tiles a turn of the
+# compute units, or its better tiles: taken as a product of their own behind the others, K = 2,048, whole -> in two, us: 2,048
+# rows, 8,208 outputs 83 -> 61, 6,160 59 -> 53, 4,128 42 -> 41; 4,096 rows, 8,208 141 -> 111, 4,128 82 -> 61, 5,152 94 -> 95;
+# 6,000 rows, 8,208 220 -> 163; 1,203 rows, 8,208 50 -> 44, 6,160 37 -> 40; 512 rows, 8,208 26 -> 29, 12,304 36 -> 35.  The small
+# product takes 6-10 us, so from 2^23 results on (32 of them at most in the last tile, as measured).
+CUT_OUTPUTS, CUT_REST, CUT_RESULTS = 256, 32, 1 << 23
+
+
+def vendor_cut(m: int, n: int) -> int:
+    """How many of ``n`` outputs the first of two library products takes; 0: one product takes all."""
+    rest = n % CUT_OUTPUTS
+    return n - rest if 0 < rest <= CUT_REST and n > CUT_OUTPUTS and m * n >= CUT_RESULTS else 0
+
+
 def decode_tune_rows(max_rows: int) -> list:
     """Row counts for which a server with ``max_rows`` seats has the vendor library's algorithms
     timed at start-up: the powers of two from 32 and ``max_rows`` itself.  A row count that was not
@@ -120,6 +134,9 @@ def linear_bf16(x: torch.Tensor, w: torch.Tensor, out: torch.Tensor, tiled=None)
         return K.gemv(x, w, out)
     if tiled is not None and use_skinny(x.shape[0], w.shape[0], w.shape[1]):
         return K.gemm_skinny(x, tiled, out)
+    cut = vendor_cut(*out.shape) if out.is_contiguous() else 0
+    if cut and K.gemm_vendor(x, w[:cut], out[:, :cut], columns=True) and K.gemm_vendor(x, w[cut:], out[:, cut:], columns=True):
+        return out
     if K.gemm_vendor(x, w, out):
         return out
     # a shape the library's heuristic has nothing for: the framework's route to the same library

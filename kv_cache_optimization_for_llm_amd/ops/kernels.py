@@ -1307,17 +1307,20 @@ def gemm_vendor_init() -> None:
     check(hip_lib().kva_gemm_vendor_init(), "gemm_vendor_init")
 
 
-def gemm_vendor(x: torch.Tensor, w: torch.Tensor, out: torch.Tensor) -> bool:
+def gemm_vendor(x: torch.Tensor, w: torch.Tensor, out: torch.Tensor, *, columns: bool = False) -> bool:
     """out = x @ w^T by the vendor GEMM library (bf16 operands, fp32 accumulation, bf16 or fp32
-    result).  False when the library has no algorithm for the shape: nothing was launched."""
+    result; with ``columns`` ``out`` is columns of a wider array).  False when the library has no algorithm for the
+    shape: nothing was launched."""
     m, k = x.shape
     n = w.shape[0]
     if w.shape[1] != k or out.shape != (m, n) or x.dtype != torch.bfloat16 or w.dtype != torch.bfloat16 \
             or out.dtype not in (torch.bfloat16, torch.float32):
         raise KernelError(f"gemm_vendor: x {tuple(x.shape)} {x.dtype}, w {tuple(w.shape)} {w.dtype}, out "
                           f"{tuple(out.shape)} {out.dtype} do not fit")
-    code = hip_lib().kva_gemm_vendor(_dev(out, "out"), _dev(x, "x"), _dev(w, "w"), m, n, k, k, n,
-                                     1 if out.dtype == torch.float32 else 0, _stream())
+    if columns and (out.stride(1) != 1 or out.stride(0) < n):
+        raise KernelError("gemm_vendor: rows of the result are contiguous and do not overlap")
+    code = hip_lib().kva_gemm_vendor(_dev(out, "out", contiguous=not columns), _dev(x, "x"), _dev(w, "w"), m, n, k, k,
+                                     out.stride(0) if columns else n, 1 if out.dtype == torch.float32 else 0, _stream())
     if code == 1:
         return False
     check(code, "gemm_vendor")

@@ -325,3 +325,20 @@ def test_vendor_product_keeps_the_fastest_algorithm_and_the_same_result(gpu):
     assert (out40.double().cpu() - want40).abs().max() / want40.abs().max() <= 2 ** -8
     with pytest.raises(K.KernelError):
         K.gemm_vendor_tune(m, [ws[0], rnd(n, k + 32, seed=1).to(gpu)])
+
+
+@pytest.mark.parametrize("m, n, k", [(2048, 4128, 64), (3000, 2824, 96), (2000, 4128, 64), (2048, 4129, 32)])
+@pytest.mark.parametrize("out_dtype", [torch.bfloat16, torch.float32])
+def test_a_few_outputs_past_a_multiple_of_256_in_a_product_of_their_own(m, n, k, out_dtype, gpu):
+    """Both sides of where the product is cut in two, by rows and by what is left of the outputs; nothing else of the result is written."""
+    from kv_cache_optimization_for_llm_amd.ops.gemm_bf16 import linear_bf16, vendor_cut
+    assert vendor_cut(m, n) == {(2048, 4128): 4096, (3000, 2824): 2816}.get((m, n), 0)
+    g = torch.Generator().manual_seed(m + n)
+    x, w = torch.randn((m, k), generator=g).bfloat16(), torch.randn((n, k), generator=g).bfloat16()
+    room = torch.full((m + 2, n), 7.0, dtype=out_dtype, device=gpu)
+    linear_bf16(x.to(gpu), w.to(gpu), room[1:m + 1])
+    want = x.float() @ w.float().t()
+    # fp32 sums of K exact products; a bf16 result is rounded once (2^-9 of it)
+    bound = want.abs() * (2.0 ** -8 if out_dtype == torch.bfloat16 else 0) + 2.0 ** -20 * k * 4
+    assert ((room[1:m + 1].float().cpu() - want).abs() <= bound).all()
+    assert (room[0] == 7.0).all() and (room[m + 1] == 7.0).all()
