@@ -415,7 +415,8 @@ def rotates_in_kernel(batch, kv, num_q_heads: int, num_kv_heads: int, head_dim: 
 
 def paged_attention(qkv: torch.Tensor, out: torch.Tensor, kv, batch, num_q_heads: int,
                     num_kv_heads: int, head_dim: int, scale: float, window: int = 0, rope=None,
-                    max_parts: int = 0, keep_first: int = 0, sinks=None, value_dim: int = None, chunk: int = 0):
+                    max_parts: int = 0, keep_first: int = 0, sinks=None, value_dim: int = None, chunk: int = 0,
+                    leave_partials: bool = False):
     """Causal GQA attention of the step's tokens over the paged cache.  ``qkv`` is the fused
     projection output ``[T, (nq + 2 nkv) d]`` (or just its Q part) whose first ``nq * d`` columns
     are the (already position-encoded) queries; keys and values are read from ``kv``.
@@ -431,6 +432,8 @@ def paged_attention(qkv: torch.Tensor, out: torch.Tensor, kv, batch, num_q_heads
     ``max_parts`` > 0: the caller can take the output of one or two decoded tokens as up to so
     many partial results a row (``ops.kernels.AttentionPartials``, returned instead of ``out``,
     which is then not written) - where the keys are cut that way no merge kernel runs.
+    ``leave_partials``: the caller takes however many partial results a row there are, of however many tokens,
+    where one launch leaves them for all rows; the keys are cut as without it.
 
     ``keep_first`` (with a window: the first so many positions stay visible behind it), ``sinks``
     (fp32 per query head: one more term exp(sink) in every denominator), a ``value_dim`` other
@@ -495,7 +498,8 @@ def paged_attention(qkv: torch.Tensor, out: torch.Tensor, kv, batch, num_q_heads
     for launch in plan:
         if launch[0] == "wave":
             _, (item_entry, item_row0, meta), tiles, splits, per, pair, covers_all, keep_cached, waves = launch
-            left = max_parts > 0 and len(plan) == 1 and covers_all and 2 <= splits // waves <= max_parts
+            left = len(plan) == 1 and covers_all and splits // waves >= 2 \
+                and (leave_partials or 0 < splits // waves <= max_parts)
             got = K.attention_mfma(qkv, stride, out, kv.k_cache, kv.v_cache, kv.block_table, item_entry, item_row0,
                                    batch.entry_seat, batch.entry_q_start, batch.entry_start_pos, num_q_heads,
                                    num_kv_heads, head_dim, scale, window, splits, per, tiles, pair, meta,

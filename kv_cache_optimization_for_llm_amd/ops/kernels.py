@@ -1213,6 +1213,26 @@ def attention_mfma(q: torch.Tensor, q_row_stride: int, out: torch.Tensor, k_cach
     return AttentionPartials(part_o, part_ml, tokens, num_q_heads) if left else out
 
 
+def attention_merge_gated(x: AttentionPartials, out: torch.Tensor, out_off: int, gate: Optional[torch.Tensor] = None, gate_off: int = 0,
+                          activation: str = "sigmoid", mul: float = 1.0) -> torch.Tensor:
+    """The output that ``x`` stands for, times ``mul`` and times ``activation`` (``"sigmoid"`` or ``"silu"``) of columns ``gate_off ..``
+    of the bf16 rows ``gate`` if given, into columns ``out_off ..`` of the bf16 rows ``out``: the merge and
+    :func:`head_norm_gate` without a norm in one launch."""
+    width = x.heads * x.head_dim
+    if out.dim() != 2 or out.shape[0] != x.tokens or out.dtype != torch.bfloat16 or not 0 <= out_off <= out.shape[1] - width:
+        raise KernelError(f"attention_merge_gated: {x.tokens} rows of {x.heads} heads of {x.head_dim} do not fit out {tuple(out.shape)}")
+    if gate is not None and (gate.dim() != 2 or gate.shape[0] != x.tokens or gate.dtype != torch.bfloat16
+                             or not 0 <= gate_off <= gate.shape[1] - width):
+        raise KernelError(f"attention_merge_gated: gate {tuple(gate.shape)} does not fit")
+    if activation not in ("sigmoid", "silu"):
+        raise KernelError(f"attention_merge_gated: activation {activation!r} is neither 'sigmoid' nor 'silu'")
+    check(hip_lib().kva_attention_merge_gated(
+        _dev(out, "out"), out.shape[1], int(out_off), _dev(x.part_o, "part_o"), _dev(x.part_ml, "part_ml"), x.tokens, x.heads, x.head_dim,
+        x.parts, _opt(gate, "gate"), gate.shape[1] if gate is not None else 0, int(gate_off), 1 if activation == "sigmoid" else 0,
+        float(mul), _stream()), "attention_merge_gated")
+    return out
+
+
 def attention_mfma_rope_supported(head_dim: int, page_size: int, group: int) -> bool:
     """Whether the decode attention kernel that rotates and caches inside takes this geometry
     (``group``: query heads per kv head)."""
@@ -2200,13 +2220,12 @@ def moe_group(slots: int, experts: int, dtype: torch.dtype, *inner: int) -> int:
 
 def moe_wide(outputs: int, tiles: int, group: int, experts: int) -> bool:
     """Whether a workgroup of the experts' products takes a group of 8 tiles against 256 ``outputs``, two workgroups a compute unit,
-    or against 128.  128 are the faster ones while the chip takes them at once, up to 512 workgroups: 256 of the wide kind in use
-    (by wide workgroups in use, us, 128 / 256 outputs: 1,024 x 2,048 64 38/59, 160 45/59, 256 48/61, 308 82/73, 440 87/76, 616
-    155/150, 924 210/168; 2,048 x 1,024 224 31/42, 256 32/43, 304 52/50, 472 59/53, 904 129/112; the same numbers from 4 to 128
-    experts; a second turn of few wide workgroups, 590 to 700, ties or loses up to 8 %).  How many groups are in use is the
-    split's affair: of the ``tiles`` that the list has room for, half a group an expert stays empty on average.  Of 392 steps around
-    the line, of 4 to 128 experts, this one takes the slower kind by more than 10 % in 45, of 148 that it sends the other way one;
-    400 with room took it in 162 (up to 1.34 times as long)."""
+    or against 128.  128 are no slower while the chip takes them at once, up to 512 workgroups: 256 of the wide kind in use
+    (by wide workgroups in use, us, 128 / 256 outputs, the matrices' outputs x K: 1,536 x 2,048 144 32/31, 258 48/52, 288 49/51, 330
+    53/55, 438 69/59, 624 93/82, 1,194 178/151; 2,048 x 2,048 192 40/32, 256 39/36, 312 67/60, 440 81/69, 832 136/120; 2,048 x 1,024
+    192 23/23, 256 25/25, 328 35/36, 440 44/39, 584 72/64, 1,088 131/108; 2,048 x 768 192 20/21, 256 22/23, 328 30/31, 448 38/32, 576
+    56/44; the same numbers for 4, 16 and 64 experts).  How many groups are in use is the split's affair: of the ``tiles`` that the
+    list has room for, half a group an expert stays empty on average."""
     return group == 8 and -(-outputs // 256) * (2 * (tiles // 8) - experts) > 2 * 288
 
 
@@ -2479,7 +2498,7 @@ KERNEL_CLASSES = {
     "layernorm": "norm", "stream_join": "elementwise", "head_gate": "elementwise", "act_mul": "activation",
     "qk_encode_cache": "rope + cache write", "latent_encode_cache": "rope + cache write",
     "heads_matmul": "per-head products",
-    "attention_mfma_rope": "attention",
+    "attention_mfma_rope": "attention", "attention_merge_gated": "attention",
     "latent_prompt": "attention (matrix cores)",
     "gemm_nt_f32": "gemm fp32", "gemm_vendor": "gemm (vendor library)",
     "gemm_skinny": "gemm (few rows)", "gemm_skinny_qkv_rope": "gemm (few rows)",

@@ -58,6 +58,7 @@ _HIP_SIGNATURES = {
     "kva_heads_matmul": [P, I, I, P, I, I, P, I, I, I, I, P, I, I, I, P, I, I, P, I, I, P, P, P, I, I, I, P],
     "kva_heads_matmul_mfma_supported": [I, I, I],
     "kva_heads_matmul_mfma": [P, I, I, P, I, I, P, I, I, I, I, P, I, I, I, P, I, I, P, I, I, P, P, P, I, I, P],
+    "kva_attention_merge_gated": [P, I, I, P, P, I, I, I, I, P, I, I, I, F, P],
     "kva_attention_mfma": [P, P, P, P, I, P, P, P, I, P, P, P, I, I, P, P, P, I, I, I, I, I, F, I, I, I, I, I, I, I, P],
     "kva_attention_mfma_rope": [P, P, P, P, I, P, P, P, I, P, I, I, I, I, I, I, F, I, I, I, I, P, P, P, I, P],
     "kva_attention_mfma_rope_supported": [I, I, I],

@@ -280,9 +280,14 @@ class GatedGQAAttention(ProjectedMixer):
                           k_weight=self.k_weight, norm_first=self.qk_norm == "before_rotation")
         direct = self.gate is None and mul == 1.0 and out_col0 == 0 and out.shape[1] == self.inner_width
         heads = out if direct else torch.empty((y.shape[0], self.inner_width), dtype=y.dtype, device=y.device)
-        attn_ops.paged_attention(qkv, heads, kv, batch, self.num_heads, self.num_kv_heads, self.head_dim, self.scale,
-                                 self.window, keep_first=self.keep_first, value_dim=self.value_dim, sinks=self.sinks)
-        if not direct:
+        # (partial results go straight to the launch that gates them)
+        got = attn_ops.paged_attention(qkv, heads, kv, batch, self.num_heads, self.num_kv_heads, self.head_dim, self.scale,
+                                       self.window, keep_first=self.keep_first, value_dim=self.value_dim, sinks=self.sinks,
+                                       leave_partials=not direct and out.dtype == torch.bfloat16 and y.is_contiguous() and out.is_contiguous())
+        if isinstance(got, K.AttentionPartials):
+            K.attention_merge_gated(got, out, out_col0, y if self.gate is not None else None, col0 + self.qkv_width,
+                                    self.gate or "sigmoid", mul)
+        elif not direct:
             if self.gate is None:
                 # the heads times the constant, into their columns of the wider buffer
                 K.head_norm_gate(heads, None, 0.0, None, 0, out, out_col0, self.num_heads, self.value_dim, None, mul)
