@@ -7,19 +7,19 @@
 // 128 + 64 / 128.  Expanding a key costs 2 rank (dim + vdim) per head once, as much as 85 tokens looking at it save.
 // Two kernels:
 //   * latent_expand_kernel: the entries' whole contexts (cached rows, by page) times [U_k ; U_v], rounded to
-//     bf16, one row [heads x dim | heads x vdim] a position; the rotated key parts, which all heads share, are laid
-//     side by side in the same launch.
-//   * latent_prompt_kernel: a workgroup takes 64 tokens of an entry and one head, a wavefront 16 of the tokens.  As in
-//     latent_attention_mfma.hip everything is transposed, S^T = K Q^T and O^T = V^T P^T; blocks of 32 keys go through LDS
-//     for the four wavefronts (the next one's loads in flight), V^T is read there with the transposing load.  The
+//     bf16, keys' heads and then values' heads one after the other, a position a row of 128 elements; the rotated key parts,
+//     which all heads share, are laid side by side in the same launch.
+//   * latent_prompt_kernel: a workgroup takes 64 tokens of an entry and one head, a wavefront 32 of the tokens and half of
+//     the keys.  As in latent_attention_mfma.hip everything is transposed, S^T = K Q^T and O^T = V^T P^T; blocks of 64 keys go
+//     through LDS for the four wavefronts (the next one's loads in flight), V^T is read there with the transposing load.  The
 //     queries' rotation happens as they are loaded, sink and output gate where the result is normalised.
-// A SIMD issues matrix products (20 of 16 cycles a block and wavefront) or the softmax's vector work (about as
-// much), and LDS gives the four wavefronts 20 KiB each a block (640 cycles): the three are about even.  The
+// A SIMD issues matrix products (40 of 16 cycles a block and wavefront) or the softmax's vector work (about as
+// much), and LDS gives the four wavefronts 20 KiB each a block (640 cycles).  The
 // workgroups with the most keys are launched first; a head's workgroups are on one die where the heads are a
 // multiple of eight, whose L2 holds its keys and values.
 //
 // us a layer, one prompt of 2,048 tokens, 16 heads of 128 + 64 / 128, rank 512: over the cached rows 183, the products
-// per head in front and behind 38 + 21; expanded 18 + 67 (21.5 GFLOP in the second: 320 TFLOP/s).
+// per head in front and behind 38 + 21; expanded 18 + 69 (21.5 GFLOP in the second: 312 TFLOP/s).
 #include "common.h"
 #include "lds_product.h"
 #include <math.h>

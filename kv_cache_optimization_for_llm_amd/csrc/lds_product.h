@@ -1,5 +1,6 @@
 // A bf16 product of many rows on the matrix cores, operands through LDS: the middle of kernels that differ in
-// where their operands' rows lie and in what they do with the result (experts' products, products per head).
+// where their operands' rows lie and in what they do with the result.  LdsProduct: products per head and expanded keys and
+// values, whose rows lie anywhere; RingProduct, further down: experts' products, whose rows are reached from one base.
 //
 // A workgroup of four wavefronts takes 32 RT rows of x and 32 NT outputs (rows of w), a wavefront half of
 // either.  32 elements of K of both operands are a stage; STAGES of them stand in LDS in a ring.  They get there
@@ -8,8 +9,8 @@
 // times that.  K (a multiple of 32) is added in ascending order into one accumulator an output.
 //
 // Before, operands went through registers, one stage of 64 elements ahead, 128 x 128 at a time, and results to memory
-// one by one: experts' products of 8,192 slots of 16 experts, 1,536 x 2,048 / 2,048 x 768: 122 / 61 -> 78 / 60 us; of 4
-// experts, 1,024 x 2,048 / 2,048 x 1,024: 132 / 70 -> 56 / 43; 2,048 slots of 16: 67 / 29 -> 36 / 22.  The middle alone
+// one by one (LdsProduct, which the experts' products used then): of 8,192 slots of 16 experts, 1,536 x 2,048 / 2,048 x 768:
+// 122 / 61 -> 78 / 60 us; of 4 experts, 1,024 x 2,048 / 2,048 x 1,024: 132 / 70 -> 56 / 43; 2,048 slots of 16: 67 / 29 -> 36 / 22.  The middle alone
 // (4,096 x 4,096 x 2,048, w in operand order): 1.23 PFLOP/s; without its loads 1.61, without its reads 1.41.
 //
 // What bounds it: a wavefront reads (RT + NT) KiB of operands from LDS for RT NT products of 16 cycles; four of them
