@@ -1069,6 +1069,10 @@ moe_few_rows_kernel(MoeFew a, MoeFewRouter ro, void *__restrict__ out, const bf1
                 make_uint2(moe_pack(v[0], v[1]), moe_pack(v[2], v[3]));
         } else if (slot < 0) {
         } else if (a.mode == 1) {
+            // (rounded as the product's bf16 rows are where it runs alone: what comes behind is the same for few tokens and many)
+            if (shared)
+#pragma unroll
+                for (int i = 0; i < 4; ++i) v[i] = bf16_bits_to_float(float_to_bf16_bits(v[i]));
             *reinterpret_cast<float4 *>((shared ? reinterpret_cast<float *>(a.shared_out) : reinterpret_cast<float *>(out)) + (size_t)slot * N + n) =
                 make_float4(v[0], v[1], v[2], v[3]);
         } else if (a.gated) {
