@@ -657,9 +657,9 @@ attention_mfma_rope_kernel(bf16_t *__restrict__ out, float *__restrict__ part_o,
 // the first MERGE_EARLY splits are loaded before the weights are known, so that the kernel makes
 // one trip to memory, not two.
 //
-// GATED (every row of a launch): the row times `mul` and, with a gate, times its activation of gate[token, off + head head_dim
-// + j], into columns of a wider output - what a launch of its own did behind this one, over the rounded row (a prompt of 2,048
-// tokens and four decoded ones, six layers of it: 5,933 -> 5,784 us).
+// GATED (every row of a launch): the row, rounded as it would be in memory, times `mul` and, with a gate, times its activation of
+// gate[token, off + head head_dim + j], into columns of a wider output - what a launch of its own did behind this one, to the
+// bit (a prompt of 2,048 tokens and four decoded ones, six layers of it: 5,933 -> 5,784 us).
 #define MERGE_EARLY 32
 struct MergeGate {
     const bf16_t *p;                // or null: the row times `mul` alone
@@ -737,7 +737,7 @@ attention_merge_kernel(MergeGate mg, bf16_t *__restrict__ out, const float *__re
 #pragma unroll 8
         for (int s = s0; s < splits; ++s) acc += po[(size_t)s * head_dim + j] * w_s[s];
         if constexpr (GATED) {
-            float v = acc * inv;
+            float v = bf16_bits_to_float(float_to_bf16_bits(acc * inv));
             if (mg.p) {
                 const float z = j == lane ? early_gate : to_float(mg.p[token * mg.stride + mg.off + column + j]);
                 v *= (mg.sigmoid ? 1.f : z) / (1.f + expf(-z));

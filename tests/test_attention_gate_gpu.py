@@ -1,6 +1,7 @@
 """Partial results of decoded tokens merged and gated in one launch, against float64 over the same partial results.
 
-Tolerance: one rounding to bf16 (2^-9 of a value; 2^-8 allowed) and 2^-20 of the largest for the fp32 sums over up to 256 ranges."""
+Tolerance: the merged row and the gated one are each rounded to bf16's 8 significant bits, half of the last place or 2^-8 of the
+value at most, and 2^-20 of the largest for the fp32 sums over up to 256 ranges."""
 import pytest
 import torch
 
@@ -28,7 +29,7 @@ def test_partial_results_merged_and_gated(tokens, heads, dim, parts, act, mul, g
         z = gate[:, 16:16 + width].double()
         want = want * (torch.sigmoid(z) if act == "sigmoid" else z * torch.sigmoid(z))
     got = out.double().cpu()
-    assert ((got[:, 8:8 + width] - want).abs() <= 2.0 ** -8 * want.abs() + 2.0 ** -20 * want.abs().max()).all()
+    assert ((got[:, 8:8 + width] - want).abs() <= 2.01 * 2.0 ** -8 * want.abs() + 2.0 ** -20 * want.abs().max()).all()
     assert (got[:, :8] == 7.0).all() and (got[:, 8 + width:] == 7.0).all()
     with pytest.raises(K.KernelError):
         K.attention_merge_gated(x, out, 17, None, 0, "sigmoid", mul)
