@@ -48,6 +48,8 @@ struct MoeRoute {
 
 // one token by one wavefront: `logits` [outputs] (memory or LDS) -> idx and wgt [top]; `choice` is the wavefront's own
 // piece of LDS, KVA_WAVE * PL floats (16-byte aligned; with PL > 1 read with groups only).  A lane takes PL outputs.
+// The choices are `top` different outputs whatever the scores hold (the few-token products rely on it): a score that is
+// not a number counts as the largest, and of equal ones, -inf among them, the lowest index comes first.
 template <int PL>
 __device__ inline void moe_route_token(const MoeRoute &a, const float *logits, int *idx, float *wgt, float *choice) {
     const int lane = threadIdx.x % KVA_WAVE;
@@ -80,6 +82,7 @@ __device__ inline void moe_route_token(const MoeRoute &a, const float *logits, i
             s[j] = a.sigmoid_scores ? (e < a.outputs ? 1.f / (1.f + expf(-logits[e])) : 0.f) : s[j] / sum;
             ch[j] = e < a.outputs ? s[j] + (a.correction ? a.correction[e] : 0.f) : -INFINITY;
         }
+        if (ch[j] != ch[j]) ch[j] = INFINITY;
     }
     if (a.groups > 1) {
         // Outputs form `groups` equal runs of neighbours.  A group's score is the sum of its `group_top`
@@ -154,6 +157,7 @@ __device__ inline void moe_route_token(const MoeRoute &a, const float *logits, i
         return;
     }
     float total = 0.f;
+    unsigned taken = 0u;                // this lane's outputs that are chosen
     for (int k = 0; k < a.top; ++k) {
         // the largest remaining choice score; of equal ones the lowest index
         float bv = -INFINITY, bs = 0.f;
@@ -161,7 +165,7 @@ __device__ inline void moe_route_token(const MoeRoute &a, const float *logits, i
 #pragma unroll
         for (int j = 0; j < PL; ++j) {
             const int e = lane + j * KVA_WAVE;
-            if (e < a.outputs && (ch[j] > bv || (ch[j] == bv && e < be))) { bv = ch[j]; be = e; bs = s[j]; }
+            if (e < a.outputs && !((taken >> j) & 1u) && (ch[j] > bv || (ch[j] == bv && e < be))) { bv = ch[j]; be = e; bs = s[j]; }
         }
 #pragma unroll
         for (int off = KVA_WAVE / 2; off > 0; off >>= 1) {
@@ -171,7 +175,7 @@ __device__ inline void moe_route_token(const MoeRoute &a, const float *logits, i
         }
 #pragma unroll
         for (int j = 0; j < PL; ++j)
-            if (lane + j * KVA_WAVE == be) ch[j] = -INFINITY;
+            if (lane + j * KVA_WAVE == be) taken |= 1u << j;
         total += bs;
         if (lane == 0) {
             idx[k] = be;

@@ -128,3 +128,43 @@ def test_norms_add_up_what_experts_returned(rows, width, top, extra, gate, gpu):
         want = x.double() + norm(branch, w, b)
         assert (out.double().cpu() - norm(want, b, w)[chosen]).abs().max() <= 2e-5 * 8
         assert (stream.double().cpu() - (want if pick is None else x.double())).abs().max() <= 2e-5 * want.abs().max()
+
+
+@pytest.mark.parametrize("outputs, top", [(5, 3), (64, 4), (96, 4), (96, 96)])
+@pytest.mark.parametrize("scores", ["softmax", "sigmoid"])
+def test_a_tokens_choices_are_different_whatever_its_scores_hold(outputs, top, scores, gpu):
+    """Rows: ordinary; one score that is not a number; all of them; and a correction that leaves two outputs above -inf."""
+    logits = rnd((3, outputs), 9, dtype=torch.float32)
+    logits[1, 2], logits[2] = float("nan"), float("nan")
+    hidden = torch.full((outputs,), float("-inf"))
+    hidden[1], hidden[3] = 0.5, 0.0
+    for correction in (None, hidden):
+        idx = torch.full((3, top), -1, dtype=torch.int32, device=gpu)
+        wgt = torch.full((3, top), 7.0, device=gpu)
+        K.moe_route(logits.to(gpu), None if correction is None else correction.to(gpu), top, idx, wgt, scores=scores)
+        idx, wgt = idx.cpu().long(), wgt.cpu()
+        value = torch.softmax(logits, -1) if scores == "softmax" else torch.sigmoid(logits)
+        score = value if correction is None else value + correction
+        score = torch.where(score.isnan(), float("inf"), score)
+        want = torch.sort(score, dim=1, descending=True, stable=True).indices[:, :top]       # (of equal ones the lowest index first)
+        assert torch.equal(idx, want)
+        # fp32 sums over at most 96 outputs, exp and sigmoid within a few units of 2^-23
+        torch.testing.assert_close(wgt, value.gather(1, want), rtol=1e-5, atol=1e-7, equal_nan=True)
+
+
+@pytest.mark.parametrize("experts, top", [(4, 2), (80, 3)])
+def test_a_row_that_is_not_a_number_stays_one_and_leaves_the_others_alone(experts, top, gpu):
+    """A router inside the first product, and one in front of it."""
+    part = RoutedExperts("p.", hidden_size=64, intermediate_size=32, experts=experts, top=top, activation="silu", gated=True, correction=False)
+    part.leaves_rows = True
+    part.load({k: rnd(s.shape, i, 0.1).to(gpu) for i, (k, s) in enumerate(part.tensor_specs().items())})
+    x = rnd((4, 64), 5)
+    x[1, 7] = float("nan")
+    left = part.forward(x.to(gpu), MixerContext(batch=None))
+    idx = left.idx.cpu()
+    assert all(len(set(row.tolist())) == top and 0 <= min(row) and max(row) < experts for row in idx)
+    got = left.rows.view(4, top, 64)
+    assert got[1].isnan().all()
+    for t in (0, 2, 3):
+        alone = part.forward(x[t:t + 1].to(gpu), MixerContext(batch=None))
+        assert torch.equal(alone.idx[0], left.idx[t]) and torch.equal(alone.rows.view(top, 64), got[t])
