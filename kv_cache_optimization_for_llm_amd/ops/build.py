@@ -1,7 +1,8 @@
 """Compiles the HIP kernels (gfx950) and the host allocators into two shared libraries.
 
 ``libkva_hip.so``  - every ``csrc/*.hip`` file, compiled with hipcc for gfx950.
-``libkva_host.so`` - ``csrc/host/*.cpp``, C++ without a GPU runtime; one function takes Python objects.
+``libkva_host.<interpreter>.so`` - ``csrc/host/*.cpp``, C++ without a GPU runtime; one function takes Python objects,
+laid out as the interpreter that compiled it lays them out: every interpreter has a library of its own.
 
 Libraries are kept in ``<package>/_lib`` when that folder can be written, otherwise in a
 per-user folder under the system's temporary directory.  A stamp file holds a hash of the
@@ -120,8 +121,14 @@ def hip_digest() -> str:
     return _digest(_hip_sources() + _headers(), HIP_FLAGS + HIP_LINK_LIBS)
 
 
+def host_name() -> str:
+    return f"libkva_host.{sysconfig.get_config_var('SOABI') or sys.implementation.cache_tag}.so"
+
+
 def host_digest() -> str:
-    return _digest(_host_sources(), HOST_FLAGS)
+    # (built without the interpreter's headers it lacks a function: built again once they are there)
+    headers = os.path.isfile(os.path.join(sysconfig.get_paths()["include"], "Python.h"))
+    return _digest(_host_sources(), HOST_FLAGS + [host_name(), sys.version, f"headers={headers}"])
 
 
 def build_hip(force: bool = False) -> str:
@@ -173,8 +180,8 @@ def build_hip(force: bool = False) -> str:
 
 
 def build_host(force: bool = False) -> str:
-    """Path of an up-to-date ``libkva_host.so`` (the page pool and the buddy allocator)."""
-    name, digest = "libkva_host.so", host_digest()
+    """Path of this interpreter's up-to-date host library (the page pool, the buddy allocator, a sampling's row arguments)."""
+    name, digest = host_name(), host_digest()
     if not force:
         cur = _find_current(name, digest)
         if cur:

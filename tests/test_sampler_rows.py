@@ -5,6 +5,7 @@ import numpy as np
 import pytest
 import torch
 
+from kv_cache_optimization_for_llm_amd.ops import build
 from kv_cache_optimization_for_llm_amd.ops.library import sample_rows
 from kv_cache_optimization_for_llm_amd.sampling import sampler as S
 
@@ -42,3 +43,14 @@ def test_what_the_comprehensions_raise_is_raised():
         S._read_rows([S.SampleRow(0, 0.5, "x")], 1, staging(1), False)
     with pytest.raises(OverflowError):
         S._read_rows([S.SampleRow(1 << 40, 0.5)], 1, staging(1), True)
+
+
+def test_every_interpreter_has_a_host_library_of_its_own(monkeypatch, tmp_path):
+    name, digest, var, paths = build.host_name(), build.host_digest(), build.sysconfig.get_config_var, build.sysconfig.get_paths()
+    with monkeypatch.context() as m:
+        m.setattr(build.sysconfig, "get_config_var", lambda key: "cpython-399-elsewhere" if key == "SOABI" else var(key))
+        assert build.host_name() != name and build.host_digest() != digest
+    with monkeypatch.context() as m:            # built without the headers: not what is asked for once they are there
+        m.setattr(build.sysconfig, "get_paths", lambda: dict(paths, include=str(tmp_path)))
+        assert build.host_name() == name and build.host_digest() != digest
+    assert (build.host_name(), build.host_digest()) == (name, digest)
