@@ -192,7 +192,8 @@ class RoutedExperts(FeedForward):
         return product[:, self.outputs] if self.shared_gate is not None else None
 
     def _few(self, x) -> bool:
-        return not self.lists_few and x.dtype == torch.bfloat16 and 0 < x.shape[0] <= K.moe_few_max_tokens()
+        # (rows that start at no multiple of 16 bytes keep the list: its kernels take them)
+        return not self.lists_few and x.dtype == torch.bfloat16 and 0 < x.shape[0] <= K.moe_few_max_tokens() and x.data_ptr() % 16 == 0
 
     def _few_rows(self, x, idx, wgt, table, router) -> tuple:
         """(the experts' rows, the rows of the expert every token uses or None), both products in a launch each."""

@@ -95,6 +95,21 @@ def test_a_table_that_names_an_expert_twice_keeps_the_list(gpu):
     assert (got - want).abs().max() <= 2.0 ** -7 * want.abs().max()
 
 
+@pytest.mark.parametrize("T", [1, 5, 16])
+def test_rows_at_no_multiple_of_16_bytes_keep_the_list(T, gpu):
+    part = RoutedExperts("p.", hidden_size=64, intermediate_size=32, experts=4, top=2, activation="silu", gated=True, correction=False,
+                         router="table", table_rows=8)
+    state = {k: rnd(s.shape, i, 0.1) for i, (k, s) in enumerate(part.tensor_specs().items())}
+    state["p.table"] = torch.tensor([[t % 4, (t + 1) % 4] for t in range(8)], dtype=torch.int32)
+    part.load({k: v.to(gpu) for k, v in state.items()})
+    x, ids = rnd((T, 64), 5), torch.arange(T, dtype=torch.int32) % 8
+    place = torch.zeros(T * 64 + 1, dtype=torch.bfloat16, device=gpu)[1:].view(T, 64)
+    place.copy_(x)
+    got = part.forward(place, MixerContext(batch=_Batch(ids.to(gpu)))).double().cpu()
+    want = oracle(x, state["p.table"][ids.long()], torch.full((T, 2), 0.5), state, 32, "silu", True, False, 0, None)
+    assert (got - want).abs().max() <= 2.0 ** -7 * want.abs().max()
+
+
 @pytest.mark.parametrize("rows, width, top, extra, gate", [(1, 64, 1, None, False), (3, 2048, 4, "float32", True), (5, 4100, 3, "bfloat16", False),
                                                            (2, 36, 9, "bfloat16", True), (2, 37, 2, "float32", True)])
 def test_norms_add_up_what_experts_returned(rows, width, top, extra, gate, gpu):
