@@ -1,7 +1,7 @@
 // Per-row arguments of a sampling, read from the rows' Python objects into the staging array that goes up to the device.
 // Four list comprehensions over 64 rows took 23 us of a call whose kernels take 18; this takes 4.  Called with the
-// interpreter's lock held (ctypes.PyDLL); an exception set here is raised by the caller.  Without the interpreter's headers
-// the function is absent and the comprehensions run.
+// interpreter's lock held (ctypes.PyDLL).  The comprehensions are what a row's values mean: they run where an exception is set
+// here, and where the function is absent because the interpreter's headers were.
 #if __has_include(<Python.h>)
 #define PY_SSIZE_T_CLEAN
 #include <Python.h>
@@ -67,10 +67,13 @@ bool truth(PyObject *row, PyObject *name, bool *out) {
 
 } // namespace
 
-// Bit 0: a row has a temperature, bit 1: a row asks for the penalty; -1: an exception is set.  With `staging` ([5][stride], n <=
-// stride) its rows get 1 / temperature (0: greedy) in fp32, the low 32 bits of key and step, and - with `seats` - the seat of rows
-// that ask for the penalty (else -1) and the seat.
-extern "C" int kva_sample_rows(PyObject *rows, long long n, int32_t *staging, long long stride, int seats) {
+// Returns bit 0: a row has a temperature (asked for with READ_SAMPLED), bit 1: a row asks for the penalty (READ_PENALTY); -1: an
+// exception is set.  With `staging` ([5][stride], n <= stride) its rows get, with READ_SAMPLED, 1 / temperature (0: greedy) in fp32
+// and the low 32 bits of key and step, with READ_SEATS the seat and, with READ_PENALTY too, the seat of rows that ask for the penalty
+// (else -1).  Nothing else of a row is looked at.
+enum { READ_SAMPLED = 1, READ_PENALTY = 2, READ_SEATS = 4 };
+
+extern "C" int kva_sample_rows(PyObject *rows, long long n, int32_t *staging, long long stride, int want) {
     static const Names names;
     PyObject *list = PySequence_Fast(rows, "the rows of a sampling are a sequence");
     if (!list) return -1;
@@ -84,19 +87,22 @@ extern "C" int kva_sample_rows(PyObject *rows, long long n, int32_t *staging, lo
         PyObject *row = PySequence_Fast_GET_ITEM(list, i);
         Py_INCREF(row);
         double temperature = 0.0;
-        bool penalty = false, ok = real(row, names.temperature, &temperature) && truth(row, names.apply_penalty, &penalty);
-        if (ok && staging) {
+        bool penalty = false, ok = true;
+        if (want & READ_SAMPLED) ok = real(row, names.temperature, &temperature);
+        if (ok && want & READ_PENALTY) ok = truth(row, names.apply_penalty, &penalty);
+        if (ok && staging && want & READ_SAMPLED) {
             const float inverse = temperature > 0.0 ? (float)(1.0 / temperature) : 0.f;
-            __builtin_memcpy(&staging[i], &inverse, sizeof inverse);
             uint32_t key = 0, step = 0;
-            int32_t seat = 0;
-            ok = low_bits(row, names.rng_key, &key) && low_bits(row, names.rng_step, &step) && (!seats || whole32(row, names.seat, &seat));
+            ok = low_bits(row, names.rng_key, &key) && low_bits(row, names.rng_step, &step);
+            __builtin_memcpy(&staging[i], &inverse, sizeof inverse);
             staging[stride + i] = (int32_t)key;
             staging[2 * stride + i] = (int32_t)step;
-            if (seats) {
-                staging[3 * stride + i] = penalty ? seat : -1;
-                staging[4 * stride + i] = seat;
-            }
+        }
+        if (ok && staging && want & READ_SEATS) {
+            int32_t seat = 0;
+            ok = whole32(row, names.seat, &seat);
+            if (want & READ_PENALTY) staging[3 * stride + i] = penalty ? seat : -1;
+            staging[4 * stride + i] = seat;
         }
         Py_DECREF(row);
         flags = ok ? flags | (temperature > 0.0 ? 1 : 0) | (penalty ? 2 : 0) : -1;

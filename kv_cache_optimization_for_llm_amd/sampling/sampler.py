@@ -57,21 +57,28 @@ class _Staging:
         self.sent = None                    # an event behind the copy
 
 
-def _read_rows(rows: Sequence[SampleRow], n: int, staging: Optional[_Staging], seats: bool) -> int:
-    """Bit 0: a row has a temperature, bit 1: a row asks for the penalty.  ``staging`` takes the rows' arguments, with ``seats``
-    the seats too."""
+def _read_rows(rows: Sequence[SampleRow], n: int, staging: Optional[_Staging], seats: bool, *, sampled: bool = True,
+               penalty: bool = True) -> int:
+    """Bit 0: a row has a temperature (``sampled``), bit 1: a row asks for the penalty (``penalty``).  ``staging`` takes the rows'
+    arguments: temperature, key and step with ``sampled``; with ``seats`` the seats, and with ``penalty`` too those of rows that ask
+    for it.  What is not asked for is not read."""
     native = sample_rows()
     if native is not None:
-        return native(rows, n, staging.pinned.data_ptr() if staging is not None else None,
-                      staging.i32.shape[1] if staging is not None else 0, 1 if seats else 0)
+        try:
+            return native(rows, n, staging.pinned.data_ptr() if staging is not None else None,
+                          staging.i32.shape[1] if staging is not None else 0, (1 if sampled else 0) | (2 if penalty else 0) | (4 if seats else 0))
+        except Exception:
+            pass                    # a value that it does not take: below it is taken, or refused with its own error
     if staging is not None:
-        staging.f32[0, :n] = [1.0 / r.temperature if r.temperature > 0 else 0.0 for r in rows]
-        staging.u32[1, :n] = [int(r.rng_key) & 0xFFFFFFFF for r in rows]
-        staging.u32[2, :n] = [int(r.rng_step) & 0xFFFFFFFF for r in rows]
-        if seats:
+        if sampled:
+            staging.f32[0, :n] = [1.0 / r.temperature if r.temperature > 0 else 0.0 for r in rows]
+            staging.u32[1, :n] = [int(r.rng_key) & 0xFFFFFFFF for r in rows]
+            staging.u32[2, :n] = [int(r.rng_step) & 0xFFFFFFFF for r in rows]
+        if seats and penalty:
             staging.i32[3, :n] = [r.seat if r.apply_penalty else -1 for r in rows]
+        if seats:
             staging.i32[4, :n] = [r.seat for r in rows]
-    return (1 if any(r.temperature > 0 for r in rows) else 0) | (2 if any(r.apply_penalty for r in rows) else 0)
+    return (1 if sampled and any(r.temperature > 0 for r in rows) else 0) | (2 if penalty and any(r.apply_penalty for r in rows) else 0)
 
 
 class PendingTokens:
@@ -179,14 +186,14 @@ class Sampler:
         if n == 0:
             event.record()
             return PendingTokens(host, event, 0)
-        flags = _read_rows(rows, n, None, False)
-        any_sampled, use_mask = bool(flags & 1), self.mask is not None and bool(flags & 2)
+        flags = _read_rows(rows, n, None, False, penalty=self.mask is not None)
+        any_sampled, use_mask = bool(flags & 1), bool(flags & 2)
         inv_t = key = step = seat_t = mark_seat = None
         if any_sampled or self.mask is not None:
             # the per-row arguments go up in one copy from pinned memory (five small pageable
             # tensors, each copied by itself, were 0.4 ms of host time apiece in a serving loop)
             staging, (dev_t, dev_key, dev_step, dev_seat, dev_mark) = self._row_arguments(n)
-            _read_rows(rows, n, staging, self.mask is not None)
+            _read_rows(rows, n, staging, self.mask is not None, sampled=any_sampled, penalty=use_mask)
             if any_sampled:
                 inv_t, key, step = dev_t, dev_key, dev_step
             if use_mask:

@@ -45,6 +45,31 @@ def test_what_the_comprehensions_raise_is_raised():
         S._read_rows([S.SampleRow(1 << 40, 0.5)], 1, staging(1), True)
 
 
+def test_what_a_sampling_does_not_need_is_not_read():
+    """Rows need no more than what is asked for, and a seat may be of any type that an array takes."""
+    greedy, seated = types.SimpleNamespace(temperature=0.0), types.SimpleNamespace(seat=3.0)
+    assert S._read_rows([greedy] * 2, 2, None, False, penalty=False) == 0
+    got = staging(2)
+    assert S._read_rows([seated] * 2, 2, got, True, sampled=False, penalty=False) == 0
+    assert got.i32.tolist() == [[-7, -7]] * 4 + [[3, 3]]
+    drawn = types.SimpleNamespace(temperature=0.5, rng_key=4, rng_step=5)
+    got = staging(1)
+    assert S._read_rows([drawn], 1, got, False, penalty=False) == 1
+    assert got.f32[0, 0] == 2.0 and got.i32[1:, 0].tolist() == [4, 5, -7, -7]
+    for asked in (dict(sampled=False), dict(penalty=False)):
+        with pytest.raises(AttributeError):
+            S._read_rows([types.SimpleNamespace()], 1, None, False, **asked)
+
+
+@pytest.mark.gpu
+def test_greedy_rows_need_a_temperature_and_with_a_penalty_a_seat(gpu):
+    logits = torch.randn((3, 300), generator=torch.Generator().manual_seed(1)).to(gpu)
+    best = logits.argmax(1).tolist()
+    assert S.Sampler(300, 4, gpu).sample(logits, [types.SimpleNamespace(temperature=0.0)] * 3).tolist() == best
+    rows = [types.SimpleNamespace(temperature=0.0, apply_penalty=False, seat=i) for i in range(3)]
+    assert S.Sampler(300, 4, gpu, repetition_penalty=1.5).sample(logits, rows).tolist() == best
+
+
 def test_every_interpreter_has_a_host_library_of_its_own(monkeypatch, tmp_path):
     name, digest, var, paths = build.host_name(), build.host_digest(), build.sysconfig.get_config_var, build.sysconfig.get_paths()
     with monkeypatch.context() as m:
