@@ -333,11 +333,12 @@ def test_rows_of_several_entries_in_items_of_both_sizes(heads, rank, rot, page, 
 
 # ---------------------------------------------------------------- feed-forwards
 @pytest.mark.parametrize("interleaved, gate, sink", [(True, "element", True), (False, "head", False), (True, None, True)])
-@pytest.mark.parametrize("heads, rank, page, entries", [(1, 32, 16, [(0, 1)]), (3, 96, 16, [(0, 63), (5, 64), (200, 65)]), (16, 512, 16, [(0, 300), (700, 129)]),
+@pytest.mark.parametrize("heads, rank, page, entries", [(1, 32, 16, [(0, 1)]), (3, 96, 16, [(0, 63), (5, 64), (200, 65)]), (16, 512, 16, [(0, 300), (700, 129)]), (40, 32, 16, [(3, 900)]),
                                                         (4, 512, 48, [(31, 257), (0, 33), (96, 128), (1, 1)])])
 def test_prompts_over_expanded_keys_and_values(heads, rank, page, entries, interleaved, gate, sink, gpu):
-    """Entries (first position, tokens) whose tokens and contexts end inside, at and behind tiles of 64 tokens, blocks of 32 keys
-    and tiles of 128 positions, on pages in no order, a context bound larger than any of them."""
+    """Entries (first position, tokens) whose tokens and contexts end inside, at and behind tiles of 64 tokens, blocks of 64 keys, their
+    halves and tiles of 128 positions, on pages in no order, a context bound larger than any of them; more workgroups than the chip
+    takes at once (40 heads of 900 tokens), which go out in another order."""
     d, rot, dv, T = 128, 64, 128, sum(n for _, n in entries)
     context = max(s + n for s, n in entries) + 37
     blocks = -(-context // page)
@@ -384,6 +385,35 @@ def test_prompts_over_expanded_keys_and_values(heads, rank, page, entries, inter
         got = out[at].double().cpu().view(n, heads, dv)
         # keys, values, rotated queries, probabilities and results are rounded to bf16 (2^-9 each, relative): their squares add up
         assert (got - want).norm() <= 2.0 ** -9 * 5 ** 0.5 * 1.5 * want.norm(), e
+
+
+@pytest.mark.parametrize("heads, start, n", [(2, 0, 100), (2, 5, 100), (3, 39, 64), (40, 3, 900)])
+def test_a_prompts_later_positions_leave_earlier_tokens_alone(heads, start, n, gpu):
+    """Positions that are no numbers: tokens of the 16 beside them that see none of the 32 keys beside theirs have the bits that they have
+    without, in every order that the workgroups are launched in (40 heads of 900 tokens: more than the chip takes at once)."""
+    d, rot, rank, page = 128, 64, 32, 16
+    context, T = start + n + 9, n
+    blocks = -(-context // page)
+    q = rnd((T, heads, d + rot), 1, torch.bfloat16).to(gpu)
+    up = K.moe_tiled_weight(torch.cat([rnd((heads * d, rank), 2, torch.bfloat16, rank ** -0.5), rnd((heads * d, rank), 3, torch.bfloat16, rank ** -0.5)])[None].to(gpu))[0]
+    cos, sin = RotaryEncoding(head_dim=rot, max_positions=2048, theta=10000.0, frequencies="plain_f64", pairing="half").tables(gpu)
+    rows = rnd((blocks * page, rank + rot), 4, torch.bfloat16)
+
+    def run(cache):
+        out = torch.empty((T, heads * d), dtype=torch.bfloat16, device=gpu)
+        one = lambda *v: torch.tensor(v, dtype=torch.int32, device=gpu)
+        return K.latent_prompt(q, cache.view(blocks, page, rank + rot).to(gpu), up, out, torch.arange(blocks, dtype=torch.int32, device=gpu)[None],
+                               one(0), one(0, n), one(start), cos, sin, False, 192 ** -0.5, context, n).cpu()
+    want = run(rows)
+    assert want.isfinite().all()
+    newest = start + torch.clamp(torch.arange(n) // 16 * 16 + 15, max=n - 1)       # of a token's 16
+    for bad in sorted({start, start + n - 1, start + n // 2, start + 17, start + 33, min(64, start + n - 1)}):
+        spoilt = rows.clone()
+        spoilt[bad] = float("nan") if bad % 2 else float("inf")
+        got = run(spoilt)
+        apart = newest < bad // 32 * 32
+        assert torch.equal(got[apart], want[apart]), bad
+        assert not got[bad - start:].isfinite().any(dim=1).any(), bad
 
 
 @pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
