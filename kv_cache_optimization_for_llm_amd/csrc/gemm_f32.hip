@@ -402,21 +402,35 @@ static int gf_rows_a_tile(int M, int N) {
     return best;
 }
 
-// Whether few rows go to the kernel that streams W.  It makes 32 rows a pass over W and shares nothing between its
-// workgroups; from some number of outputs on the kernels for many rows fill the chip and are the faster ones.  Few-rows kernel / ring,
-// us, K = 2,048: 17-32 rows, 4,096 outputs 16-18 / 17, 6,144 26-32 / 18, 16,384 53-64 / 36; 33-64 rows, 2,048 17 / 17, 3,072
-// 26-31 / 17, 32,768 194-241 / 68-89; K = 300 alike; K = 8,192: 17-32 rows, 2,048 46-58 / 84, 4,096 54-64 / 90; 33-64 rows, 2,048
-// 60 / 85, 4,096 99-123 / 90.  Rows that start at no multiple of 16 bytes have tiles a third slower: few-rows kernel / tiles, 17-32
-// rows, 8,192 outputs 28-33 / 46, 16,384 52-65 / 50; 33-64 rows, 4,096 28-33 / 45, 6,144 42-48 / 46, 8,192 51-62 / 46.
-static bool gf_few_rows(int M, int N, bool vec) {
-    return M <= 16 || (M <= GF_ROWS_UP_TO && (long long)N * ((M + 31) / 32) <= (vec ? 4096 : 14336));
+// Whether few rows go to the kernel that streams W.  It makes 32 rows a pass over W, in a workgroup per 16 outputs and pass, and shares
+// nothing between workgroups: its time goes up by half where a compute unit gets a second one, and with the rows of a pass.  The ring
+// takes much the same from 17 to 64 rows, and longer than one such workgroup: a wavefront alone on its SIMD waits for W.  Weights from
+// memory (sets of 800 MB and more), few-rows kernel / ring, us at K = 1,024, 2,048, 4,096, 8,192, 14,336:
+//   one a unit:  17 rows, 2,048 outputs  9.0/14.0  14.1/24.9  25.0/45.2  45.1/88.0  77.9/156    32 rows, 4,096  10.9/14.2  18.6/25.9  31.9/46.3
+//                64 rows, 2,048  10.0/13.8  16.5/24.8  29.5/44.6  55.0/87.4  95.5/154                           59.7/91.9  112/162
+//   up to one and a half (two passes):  33 rows, 2,560  11.4/14.0  18.6/25.1  32.8/45.6  58.8/88.8  102/158     48 rows, 3,072  14.8/14.1
+//                24.7/25.2  44.3/45.8  85.1/89.7  148/158    64 rows, 3,072  16.5/14.1  28.5/25.3  52.0/45.6  99.0/89.1  179/158
+//   up to two:   17 rows, 8,192  16.3/15.4  27.5/27.4  51.0/51.9  93.2/100  166/181      20 rows, 4,608  15.7/14.5  26.6/25.9  48.2/47.1
+//                90.7/92.9  162/163    24 rows, 4,608  95.7/92.5 at 8,192    40 rows, 4,096  15.7/14.5  27.0/25.5  47.5/46.1  90.0/90.9  160/161
+//   more:        17 rows, 10,240  22.0/16.5  37.9/29.4  71.5/57.0  133/107  233/187      33 rows, 6,144  22.5/15.4  39.4/27.4  72.0/50.8
+// Below K = 1,024 the ring is ahead from the second workgroup on (K = 512: 33 rows, 2,560 7.4 / 6.7).  Where the line is wrong it costs 5 % at most
+// (48 rows of 3,072 outputs at K = 1,024; 17 rows of 7,168 at K = 4,096).  Rows that start at no multiple of 16 bytes have tiles that take a third
+// longer than the ring: few-rows kernel / tiles, 17-32 rows, 8,192 outputs 28-33 / 46, 16,384 52-65 / 50; 33-64 rows, 4,096 28-33 / 45, 6,144 42-48 /
+// 46, 8,192 51-62 / 46.
+static bool gf_few_rows(int M, int N, int K, bool vec) {
+    if (M <= 16) return true;
+    if (M > GF_ROWS_UP_TO) return false;
+    const int passes = (M + 31) / 32;
+    const long long streamed = (long long)N * passes;              // 16 of them a workgroup, 4,096 one workgroup a compute unit
+    if (!vec) return streamed <= 14336;
+    return streamed <= 4096 || (streamed <= 6144 && passes == 2 && M <= 48 && K >= 1024) || (streamed <= 8192 && M <= 20 * passes && K >= 6144);
 }
 
 template <bool VEC>
 static void gf_launch(float *C, const float *A, const float *W, int M, int N, int K, int lda, int ldw, int ldc,
                       hipStream_t stream) {
     const int part = gf_part(K), parts = (K + part - 1) / part;
-    if (gf_few_rows(M, N, VEC)) {
+    if (gf_few_rows(M, N, K, VEC)) {
         const int out = M <= 8 && N < 8192 ? 8 : 16;
         const dim3 grid((N + out - 1) / out, (M + 31) / 32), block(KVA_WAVE * (out == 8 ? (parts + 1) / 2 : M <= 16 ? parts : max(4, parts)));    // (four for the sums' last step)
         if (out == 8)

@@ -210,6 +210,16 @@ def test_gemm_f32_rows_are_the_same_bits_where_the_kernel_changes(n, k, gpu):
     close(got[65], a.double() @ w.double().t(), torch.float32, "gemm_nt_f32")
 
 
+@pytest.mark.parametrize("m, n, k", [(48, 3072, 1024), (49, 3072, 1024), (33, 3072, 1020), (20, 8192, 6144), (21, 8192, 6144), (20, 8196, 6144), (40, 4096, 6144),
+                                     (41, 4096, 6144), (40, 4100, 6144)])
+def test_gemm_f32_either_side_of_where_few_rows_end(m, n, k, gpu):
+    """By outputs, rows and K: the bits of a row alone, whichever kernel the rows go to."""
+    a, w = rnd(m, k).to(gpu), rnd(n, k, seed=1).to(gpu)
+    got = K.gemm_nt_f32(a, w, torch.full((m, n), 7.0, device=gpu))
+    for row in (0, m // 2, m - 1):
+        assert torch.equal(K.gemm_nt_f32(a[row:row + 1].contiguous(), w, torch.empty(1, n, device=gpu))[0], got[row]), row
+
+
 @pytest.mark.parametrize("m, n", [(65, 68), (100, 3000), (130, 4500), (190, 10000), (517, 2048), (402, 3072), (517, 3072), (250, 16384), (129, 8196)])
 @pytest.mark.parametrize("k", [4, 36, 96, 2052])
 def test_gemm_f32_every_height_of_a_tile(m, n, k, gpu):
