@@ -920,7 +920,7 @@ extern "C" int kva_moe_expert_rows(void *out, int out_dtype, const void *x, cons
 //
 // ROUTED (mode 0): the router's product and the choice are made here too, by every workgroup for itself, in the order of sums
 // of the router's own launch: 16 parts of K.  A router of up to 16 outputs is 64 KB that all workgroups read from L2 while
-// their matrix is on its way; the launch it saves took 6-8 us.
+// their matrix is on its way; where the workgroups and the tokens are few (the caller's rule) that saves 2 us of a launch's 6-8.
 //  mode 0: out[slot] = act(W[e] x[token]) (x's type),   mode 1: out[slot] = W[e] x[slot] * weight[slot] (fp32).
 struct MoeFewRouter {
     const bf16_t *w;                // [N, K], N up to 16
@@ -1093,7 +1093,7 @@ moe_few_rows_kernel(MoeFew a, MoeFewRouter ro, void *__restrict__ out, const bf1
 
 extern "C" int kva_moe_few_max_tokens(void) { return 16; }
 
-// whether the first product makes the choice itself (every expert its unit, one tile of router outputs, a place for every slot)
+// whether the first product can make the choice itself (every expert its unit, one tile of router outputs, a place for every slot)
 extern "C" int kva_moe_few_routes(int router_N, int slots, int experts) {
     return router_N > 0 && router_N <= 16 && slots >= experts && slots <= 256;
 }

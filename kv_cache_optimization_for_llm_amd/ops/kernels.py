@@ -2319,9 +2319,27 @@ def moe_few_max_tokens() -> int:
     return int(hip_lib().kva_moe_few_max_tokens())
 
 
-def moe_few_routes(x: torch.Tensor, router: torch.Tensor, slots: int, experts: int) -> bool:
-    """Whether :func:`moe_few_rows` makes the choice for rows like ``x`` itself (``router``)."""
-    return moe_router_supported(x, router) and bool(hip_lib().kva_moe_few_routes(router.shape[0], int(slots), int(experts)))
+def moe_few_routes(x: torch.Tensor, router: torch.Tensor, w: torch.Tensor, top: int, shared: Optional["TiledWeight"] = None) -> bool:
+    """Whether :func:`moe_few_rows` makes the choice for rows like ``x`` itself (``router``), in front of experts' matrices ``w`` and
+    the one every token uses (``shared``)."""
+    tokens, experts, outputs = x.shape[0], w.shape[0], max(w.shape[1], shared.n if shared is not None else 0)
+    return moe_router_supported(x, router) and bool(hip_lib().kva_moe_few_routes(router.shape[0], tokens * int(top), experts)) \
+        and moe_choice_inside((experts + (shared is not None)) * -(-outputs // 16), tokens)
+
+
+# Every workgroup of the first product forms the whole choice, and asks for its expert's matrix before it knows whether a token
+# chose it: that saves a launch of 2 us where workgroups and tokens are few, and costs more than that where they are not.  Both products
+# and the choice, us, in a launch of its own / inside (sorted lists, which came before either): 4 of 4 experts of 768 x 2,048 (384
+# workgroups) 1 / 8 / 16 tokens 18.5/15.7 (23) 20.3/19.1 (24) 22.6/24.0 (25), 1 of 4 8 tokens 19.5/18.4 (24), all on one expert 16.5/16.0;
+# with a shared expert (480) 1 / 8 tokens 20.8/18.4 (31) 22.3/21.7 (36), 1 of 4 on one expert 17.7/17.9 (34); 8 of 8 (768) 1 / 8 tokens 26.8/25.7
+# (34) 29.2/29.6 (35), 2 of 8 4 tokens 24.8/25.1 (30), on the same two 17.1/18.5; 4 of 16 (1,536) 4 / 8 / 16 tokens 35.5/47.3 (40)
+# 41.2/54.9 (46) 46.5/64.8 (49), on the same four 21.3/40.4 (28); 4 of 4 of 1,536 x 4,096 (768) 1 token 41.0/42.2 (49); 8 of 8 of 512 x
+# 1,024 (512) 8 tokens 18.1/18.7 (21), 4 of 4 (256) 8 / 16 tokens 15.6/14.5 (20) 16.4/17.0 (21).
+MOE_CHOICE_INSIDE_WORKGROUPS, MOE_CHOICE_INSIDE_CHOICES = 512, 4096      # of the launch; workgroups times tokens: choices made
+
+
+def moe_choice_inside(workgroups: int, tokens: int) -> bool:
+    return workgroups < MOE_CHOICE_INSIDE_WORKGROUPS and workgroups * tokens < MOE_CHOICE_INSIDE_CHOICES
 
 
 def moe_few_rows(x: torch.Tensor, w: torch.Tensor, out: torch.Tensor, idx: torch.Tensor, *, activation: Optional[str] = None,

@@ -244,7 +244,7 @@ class RoutedExperts(FeedForward):
                 sorted_slot, tile_expert = self._sorted(slots, group, dev)
                 if T <= K.MOE_ROUTER_LIST_TOKENS:
                     listed = dict(sorted_slot=sorted_slot, tile_expert=tile_expert)
-            if few and K.moe_few_routes(x, self.router, slots, self.experts):
+            if few and K.moe_few_routes(x, self.router, self.w_up, self.top, self.shared.gate_up.tiled if self.shared is not None else None):
                 router = dict(w=self.router, bias=self.router_bias, correction=self.correction, outputs=self.outputs, wgt=wgt, rest=rest,
                               renormalise=self.renormalise, over_chosen=self.over_chosen, **rule)
             else:

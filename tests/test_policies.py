@@ -330,3 +330,12 @@ def test_experts_products_take_256_outputs_a_workgroup_where_128_would_not_fit_t
                                           (15360, 64, 512, True), (20480, 128, 512, True), (10240, 64, 768, True)):     # 80/73, 120/100, 86/75
         assert moe_wide(outputs, moe_tiles(slots, experts, 8), 8, experts) == wide, (slots, experts, outputs)
     assert not moe_wide(4096, moe_tiles(20000, 16, 4), 4, 16)
+
+
+def test_the_choice_of_experts_is_made_inside_the_first_product_where_workgroups_and_tokens_are_few():
+    """By workgroups of the launch and tokens, measured (us, in a launch of its own / inside)."""
+    from kv_cache_optimization_for_llm_amd.ops.kernels import moe_choice_inside
+    for workgroups, tokens, inside in ((384, 1, True), (384, 8, True), (384, 16, False),            # 18.5/15.7, 20.3/19.1, 22.6/24.0
+                                       (480, 8, True), (480, 16, False), (768, 1, False),           # 22.3/21.7, 25.0/26.8, 41.0/42.2
+                                       (1536, 1, False), (1536, 16, False), (256, 8, True), (256, 16, False)):   # 41.2/47.8, 46.5/64.8, 15.6/14.5, 16.4/17.0
+        assert moe_choice_inside(workgroups, tokens) == inside, (workgroups, tokens)
