@@ -2220,12 +2220,14 @@ def moe_group(slots: int, experts: int, dtype: torch.dtype, *inner: int) -> int:
 
 def moe_wide(outputs: int, tiles: int, group: int, experts: int) -> bool:
     """Whether a workgroup of the experts' products takes a group of 8 tiles against 256 ``outputs``, two workgroups a compute unit,
-    or against 128.  128 are no slower while the chip takes them at once, up to 512 workgroups: 256 of the wide kind in use
-    (by wide workgroups in use, us, 128 / 256 outputs, the matrices' outputs x K: 1,536 x 2,048 144 32/31, 258 48/52, 288 49/51, 330
-    53/55, 438 69/59, 624 93/82, 1,194 178/151; 2,048 x 2,048 192 40/32, 256 39/36, 312 67/60, 440 81/69, 832 136/120; 2,048 x 1,024
-    192 23/23, 256 25/25, 328 35/36, 440 44/39, 584 72/64, 1,088 131/108; 2,048 x 768 192 20/21, 256 22/23, 328 30/31, 448 38/32, 576
-    56/44; the same numbers for 4, 16 and 64 experts).  How many groups are in use is the split's affair: of the ``tiles`` that the
-    list has room for, half a group an expert stays empty on average."""
+    or against 128.  The line, 288 of the wide kind in use, was measured on the products as they were before they read their
+    operands over the barrier; with these the wide kind is ahead or level from about 150 on, so below the line up to 9 % are given
+    up, above it 3 % at most (us by wide workgroups in use, 128 / 256 outputs a workgroup, the matrices' outputs x K, matrices from
+    memory: 1,536 x 2,048 144 30.9/31.2, 192 35.6/32.8, 246 51.0/46.5, 288 51.5/51.6 and 57.5/52.9, 330 67.6/65.7, 432 81.9/69.6, 630 105/95,
+    1,212 194/161; 2,048 x 2,048 192 35.7/32.9, 256 40.0/36.4, 320 69.5/68.4, 384 56.6/57.5 and 70.2/59.5, 512 81.7/66.6, 832 141/127;
+    2,048 x 1,024 192 22.7/23.2, 256 28.0/26.1, 328 46.6/48.1, 432 55.7/47.9, 584 74.8/68.0, 1,088 131/110; 2,048 x 768 192 19.9/20.4,
+    256 23.0/22.3, 320 40.5/36.6, 440 51.4/44.2, 560 61.1/57.1; of 4, 16 and 64 experts).  How many groups are in use is the
+    split's affair: of the ``tiles`` that the list has room for, half a group an expert stays empty on average."""
     return group == 8 and -(-outputs // 256) * (2 * (tiles // 8) - experts) > 2 * 288
 
 
