@@ -137,25 +137,23 @@ __device__ __forceinline__ void lp_rotate(Frag8 (&f)[2], const float *cos, const
 // (wave / 2), and the two halves of the keys are added up at the end.  What bounds it is what the wavefronts read from LDS: 20 KiB
 // of keys and values for 40 products of 16 cycles.  (16 tokens and all keys a wavefront read the same for 20: 2,048 tokens of 16
 // heads 72 us.)  Blocks of keys go through registers, the next ones on their way over the products.
-constexpr int LP_KEY_STRIDE = LP_DIM + LP_ROT + 8, LP_VALUE_STRIDE = LP_VDIM + 24;     // (rows of either kind of read on banks of their own)
-union LpLds {
-    struct {
-        bf16_t k[LP_KEYS * LP_KEY_STRIDE], v[LP_KEYS * LP_VALUE_STRIDE];
-    } b;
-    struct {
-        float o[2][2][LP_VDIM / 16][KVA_WAVE][4], m[2][2][KVA_WAVE], l[2][2][KVA_WAVE];
-    } half;                                                     // of the wavefronts with the second half of the keys
-};
-
-// APART: the wavefront's last 16 tokens see a block of 32 keys that the first 16 do not.  A probability of zero does not leave out a
-// value that is not a number, so the first 16 are given zeros for that block's values.  Portions that start at a multiple of 32, or
-// more than 16 behind one, have no such block (masked all the same, a prompt of 2,048 tokens takes 69.0 us instead of 67.9).
-template <bool APART>
-__device__ __forceinline__ void latent_prompt_tile(const LatentPrompt &a, int tile, LpLds &lds) {
+__global__ void __launch_bounds__(256, 2)
+latent_prompt_kernel(LatentPrompt a, int tiles) {
     constexpr int KD = LP_DIM + LP_ROT, KS = KD / 32, NDT = LP_VDIM / 16;
-    constexpr int KSTRIDE = LP_KEY_STRIDE, VSTRIDE = LP_VALUE_STRIDE;
-    const int e = blockIdx.y, head = blockIdx.x % a.heads;
+    constexpr int KSTRIDE = KD + 8, VSTRIDE = LP_VDIM + 24;     // (rows of either kind of read on banks of their own)
+    __shared__ __align__(16) union {
+        struct {
+            bf16_t k[LP_KEYS * KSTRIDE], v[LP_KEYS * VSTRIDE];
+        } b;
+        struct {
+            float o[2][2][NDT][KVA_WAVE][4], m[2][2][KVA_WAVE], l[2][2][KVA_WAVE];
+        } half;                                                 // of the wavefronts with the second half of the keys
+    } lds;
+    // The workgroups that the chip takes at once: the longest and the shortest on one compute unit.  More of them: the longest first.
+    const int e = blockIdx.y, head = blockIdx.x % a.heads, at = blockIdx.x / a.heads, front = (tiles + 1) / 2;
+    const int tile = at < front || gridDim.x * gridDim.y > 512 ? tiles - 1 - at : at - front;
     const int q0 = a.entry_q_start[e], n = a.entry_q_start[e + 1] - q0, start = a.entry_start_pos[e];
+    if (tile * LP_ROWS >= n) return;
     const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid / KVA_WAVE), lane = tid % KVA_WAVE, r = lane & 15, g = lane >> 4;
     const int rows = wave & 1, keys = wave >> 1;
     const int first = tile * LP_ROWS + 32 * rows;               // the wavefront's first token
@@ -263,12 +261,14 @@ __device__ __forceinline__ void latent_prompt_tile(const LatentPrompt &a, int ti
             }
         }
         const bf16_t *get = &lds.b.v[(32 * keys + 4 * g + (r >> 2)) * VSTRIDE + 4 * (r & 3)];
+        // A portion that starts up to 16 positions behind a multiple of 32 has one block of keys that the wavefront's last 16 tokens see
+        // and the first 16 do not.  A probability of zero does not leave out a value that is not a number: they get zeros for it.
         const unsigned seen = kb <= start + first + 15 ? ~0u : 0u;
 #pragma unroll
         for (int dt = 0; dt < NDT; ++dt) {
             const Frag8 v = lp_values<VSTRIDE>(get, dt);
             Frag8 f = v;
-            if (APART) f.u4 = make_uint4(v.u4.x & seen, v.u4.y & seen, v.u4.z & seen, v.u4.w & seen);
+            f.u4 = make_uint4(v.u4.x & seen, v.u4.y & seen, v.u4.z & seen, v.u4.w & seen);
             o[0][dt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(f.v, pf[0].v, o[0][dt], 0, 0, 0);
             o[1][dt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(v.v, pf[1].v, o[1][dt], 0, 0, 0);
         }
@@ -313,18 +313,6 @@ __device__ __forceinline__ void latent_prompt_tile(const LatentPrompt &a, int ti
             *reinterpret_cast<uint2 *>(out + c) = make_uint2(__builtin_bit_cast(unsigned, lo), __builtin_bit_cast(unsigned, hi2));
         }
     }
-}
-
-__global__ void __launch_bounds__(256, 2)
-latent_prompt_kernel(LatentPrompt a, int tiles) {
-    __shared__ __align__(16) LpLds lds;
-    // The workgroups that the chip takes at once: the longest and the shortest on one compute unit.  More of them: the longest first.
-    const int e = blockIdx.y, at = blockIdx.x / a.heads, front = (tiles + 1) / 2;
-    const int tile = at < front || gridDim.x * gridDim.y > 512 ? tiles - 1 - at : at - front;
-    if (tile * LP_ROWS >= a.entry_q_start[e + 1] - a.entry_q_start[e]) return;
-    const int behind = a.entry_start_pos[e] % 32;
-    if (behind == 0 || behind > 16) latent_prompt_tile<false>(a, tile, lds);
-    else latent_prompt_tile<true>(a, tile, lds);
 }
 
 extern "C" int kva_latent_prompt_supported(int dim, int rot, int vdim, int rank) {
