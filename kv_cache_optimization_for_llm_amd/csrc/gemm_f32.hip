@@ -129,7 +129,8 @@ gemm_f32_rows_kernel(float *__restrict__ C, const float *__restrict__ A, const f
     }
 }
 
-// Many rows that start at any address: bound by the matrix cores and by loads of single elements.  A workgroup
+// Many rows that start at any address, or more than 8 MiB apart: bound by the matrix cores, at odd addresses by loads of
+// single elements.  A workgroup
 // takes 64 rows x 32 NT outputs: four wavefronts (32 x 16 NT each) the front half of the parts, four the back half -
 // two wavefronts a SIMD where the tiles are about as many as the compute units.  32 columns of both operands of
 // each half go through LDS at a time (rows 36 elements apart: the 16 rows of an operand read start in different
@@ -140,7 +141,7 @@ struct GfTile {
     float a[2][GF_BM][GF_BK + GF_PAD], w[2][32 * NT][GF_BK + GF_PAD];
 };
 
-template <int NT>
+template <int NT, bool VEC>
 __global__ void __launch_bounds__(512)
 gemm_f32_tile_kernel(float *__restrict__ C, const float *__restrict__ A, const float *__restrict__ W, int M, int N,
                      int K, int lda, int ldw, int ldc, int part, int mtiles, int tiles) {
@@ -163,9 +164,9 @@ gemm_f32_tile_kernel(float *__restrict__ C, const float *__restrict__ A, const f
     const int lrow = tid / 8, lk = tid % 8 * 4;                      // 32 rows a pass, 8 lanes a row
     auto fetch = [&](int set, int k0) {                              // (past the half's end: zeros)
 #pragma unroll
-        for (int i = 0; i < AL; ++i) la[set][i] = gf_load<false>(A, m0 + lrow + 32 * i, M, k0 + lk, hi, lda);
+        for (int i = 0; i < AL; ++i) la[set][i] = gf_load<VEC>(A, m0 + lrow + 32 * i, M, k0 + lk, hi, lda);
 #pragma unroll
-        for (int i = 0; i < WL; ++i) lw[set][i] = gf_load<false>(W, n0 + lrow + 32 * i, N, k0 + lk, hi, ldw);
+        for (int i = 0; i < WL; ++i) lw[set][i] = gf_load<VEC>(W, n0 + lrow + 32 * i, N, k0 + lk, hi, ldw);
     };
     auto put = [&](int set) {
 #pragma unroll
@@ -252,9 +253,11 @@ gemm_f32_tile_kernel(float *__restrict__ C, const float *__restrict__ A, const f
             gf_f32x4 v;
 #pragma unroll
             for (int e = 0; e < 4; ++e) v[e] = tot[i][j][e] + o[e];
+            if (VEC && n + 3 < N) *reinterpret_cast<gf_f32x4 *>(c) = v;
+            else
 #pragma unroll
-            for (int e = 0; e < 4; ++e)
-                if (n + e < N) c[e] = v[e];
+                for (int e = 0; e < 4; ++e)
+                    if (n + e < N) c[e] = v[e];
         }
     }
 }
@@ -414,23 +417,23 @@ static int gf_rows_a_tile(int M, int N) {
 //                90.7/92.9  162/163    24 rows, 4,608  95.7/92.5 at 8,192    40 rows, 4,096  15.7/14.5  27.0/25.5  47.5/46.1  90.0/90.9  160/161
 //   more:        17 rows, 10,240  22.0/16.5  37.9/29.4  71.5/57.0  133/107  233/187      33 rows, 6,144  22.5/15.4  39.4/27.4  72.0/50.8
 // Below K = 1,024 the ring is ahead from the second workgroup on (K = 512: 33 rows, 2,560 7.4 / 6.7).  Where the line is wrong it costs 5 % at most
-// (48 rows of 3,072 outputs at K = 1,024; 17 rows of 7,168 at K = 4,096).  Rows that start at no multiple of 16 bytes have tiles that take a third
-// longer than the ring: few-rows kernel / tiles, 17-32 rows, 8,192 outputs 28-33 / 46, 16,384 52-65 / 50; 33-64 rows, 4,096 28-33 / 45, 6,144 42-48 /
+// (48 rows of 3,072 outputs at K = 1,024; 17 rows of 7,168 at K = 4,096).  Without the ring the tiles are what many rows go to, and take a third
+// longer: few-rows kernel / tiles, 17-32 rows, 8,192 outputs 28-33 / 46, 16,384 52-65 / 50; 33-64 rows, 4,096 28-33 / 45, 6,144 42-48 /
 // 46, 8,192 51-62 / 46.
-static bool gf_few_rows(int M, int N, int K, bool vec) {
+static bool gf_few_rows(int M, int N, int K, bool ring) {
     if (M <= 16) return true;
     if (M > GF_ROWS_UP_TO) return false;
     const int passes = (M + 31) / 32;
     const long long streamed = (long long)N * passes;              // 16 of them a workgroup, 4,096 one workgroup a compute unit
-    if (!vec) return streamed <= 14336;
+    if (!ring) return streamed <= 14336;
     return streamed <= 4096 || (streamed <= 6144 && passes == 2 && M <= 48 && K >= 1024) || (streamed <= 8192 && M <= 20 * passes && K >= 6144);
 }
 
 template <bool VEC>
 static void gf_launch(float *C, const float *A, const float *W, int M, int N, int K, int lda, int ldw, int ldc,
-                      hipStream_t stream) {
+                      bool ring, hipStream_t stream) {
     const int part = gf_part(K), parts = (K + part - 1) / part;
-    if (gf_few_rows(M, N, K, VEC)) {
+    if (gf_few_rows(M, N, K, ring)) {
         const int out = M <= 8 && N < 8192 ? 8 : 16;
         const dim3 grid((N + out - 1) / out, (M + 31) / 32), block(KVA_WAVE * (out == 8 ? (parts + 1) / 2 : M <= 16 ? parts : max(4, parts)));    // (four for the sums' last step)
         if (out == 8)
@@ -441,7 +444,7 @@ static void gf_launch(float *C, const float *A, const float *W, int M, int N, in
             hipLaunchKernelGGL((gemm_f32_rows_kernel<2, 2, false, VEC>), grid, block, 0, stream, C, A, W, M, N, K, lda, ldw, ldc, part);
         return;
     }
-    if (VEC) {
+    if (ring) {
         const int mt = gf_rows_a_tile(M, N), mtiles = (M + 16 * mt - 1) / (16 * mt), tiles = mtiles * ((N + 63) / 64);
 #define GF_RING(MT, STAGES)                                                                                              \
     hipLaunchKernelGGL((gemm_f32_ring_kernel<MT, STAGES>), dim3((tiles + 7) / 8 * 8), dim3(256), 0, stream, C, A, W, M, N, K, lda, ldw, \
@@ -461,9 +464,9 @@ static void gf_launch(float *C, const float *A, const float *W, int M, int N, in
     }
     const int mtiles = (M + GF_BM - 1) / GF_BM, wide = mtiles * ((N + 127) / 128), narrow = mtiles * ((N + 63) / 64);
     if (wide >= 256)
-        hipLaunchKernelGGL((gemm_f32_tile_kernel<4>), dim3((wide + 7) / 8 * 8), dim3(512), 0, stream, C, A, W, M, N, K, lda, ldw, ldc, part, mtiles, wide);
+        hipLaunchKernelGGL((gemm_f32_tile_kernel<4, VEC>), dim3((wide + 7) / 8 * 8), dim3(512), 0, stream, C, A, W, M, N, K, lda, ldw, ldc, part, mtiles, wide);
     else
-        hipLaunchKernelGGL((gemm_f32_tile_kernel<2>), dim3((narrow + 7) / 8 * 8), dim3(512), 0, stream, C, A, W, M, N, K, lda, ldw, ldc, part, mtiles, narrow);
+        hipLaunchKernelGGL((gemm_f32_tile_kernel<2, VEC>), dim3((narrow + 7) / 8 * 8), dim3(512), 0, stream, C, A, W, M, N, K, lda, ldw, ldc, part, mtiles, narrow);
 }
 
 extern "C" int kva_gemm_nt_f32(float *C, const float *A, const float *W, int M, int N, int K,
@@ -472,11 +475,11 @@ extern "C" int kva_gemm_nt_f32(float *C, const float *A, const float *W, int M, 
     KVA_REQUIRE(lda >= K && ldw >= K && ldc >= N, "gemm_f32: leading dimensions too small");
     if (M == 0) return KVA_OK;
     KVA_REQUIRE((M + GF_BM - 1) / GF_BM <= 65535, "gemm_f32: M=%d is too large for one launch", M);
-    // 16-byte loads and stores where every row of all three starts at a multiple of 16 bytes (and a tile's rows lie within 2 GiB)
-    const bool vec = lda <= 1 << 21 && ldw <= 1 << 21 && K % 4 == 0 && lda % 4 == 0 && ldw % 4 == 0 && ldc % 4 == 0 &&
-                     ((uintptr_t)A | (uintptr_t)W | (uintptr_t)C) % 16 == 0;
-    if (vec) gf_launch<true>(C, A, W, M, N, K, lda, ldw, ldc, stream);
-    else gf_launch<false>(C, A, W, M, N, K, lda, ldw, ldc, stream);
+    // 16-byte loads and stores where every row of all three starts at a multiple of 16 bytes; the ring where a tile's rows lie
+    // within 2 GiB too (its loads have 32-bit offsets)
+    const bool vec = K % 4 == 0 && lda % 4 == 0 && ldw % 4 == 0 && ldc % 4 == 0 && ((uintptr_t)A | (uintptr_t)W | (uintptr_t)C) % 16 == 0;
+    if (vec) gf_launch<true>(C, A, W, M, N, K, lda, ldw, ldc, lda <= 1 << 21 && ldw <= 1 << 21, stream);
+    else gf_launch<false>(C, A, W, M, N, K, lda, ldw, ldc, false, stream);
     KVA_CHECK_LAUNCH("gemm_nt_f32");
     return KVA_OK;
 }

@@ -210,6 +210,22 @@ def test_gemm_f32_rows_are_the_same_bits_where_the_kernel_changes(n, k, gpu):
     close(got[65], a.double() @ w.double().t(), torch.float32, "gemm_nt_f32")
 
 
+@pytest.mark.parametrize("m, n", [(20, 16), (66, 70)])
+def test_gemm_f32_rows_of_more_than_8_mib(m, n, gpu):
+    """Rows that a tile's 32-bit offsets do not reach: in parts of 16 bytes or one by one, alone or among others, the same bits."""
+    k = (1 << 21) + 4
+    g = torch.Generator(device=gpu).manual_seed(m)
+    flat = torch.empty(m * k + 1, device=gpu)
+    a, w = torch.randn((m, k), generator=g, device=gpu), torch.randn((n, k), generator=g, device=gpu)
+    flat[1:].view(m, k).copy_(a)
+    got = K.gemm_nt_f32(a, w, torch.empty(m, n, device=gpu))
+    assert torch.equal(K.gemm_nt_f32(flat[1:].view(m, k), w, torch.empty(m, n, device=gpu)), got)
+    assert torch.equal(K.gemm_nt_f32(a[-1:], w, torch.empty(1, n, device=gpu))[0], got[-1])
+    want = sum(a[:, i:i + 65536].double() @ w[:, i:i + 65536].double().t() for i in range(0, k, 65536))
+    # as above: K products and additions of relative error 2^-24 each, by their root
+    assert (got - want).pow(2).mean().sqrt() <= 2.0 ** -24 * (2.0 * k) ** 0.5 * k ** 0.5
+
+
 @pytest.mark.parametrize("m, n, k", [(48, 3072, 1024), (49, 3072, 1024), (33, 3072, 1020), (20, 8192, 6144), (21, 8192, 6144), (20, 8196, 6144), (40, 4096, 6144),
                                      (41, 4096, 6144), (40, 4100, 6144)])
 def test_gemm_f32_either_side_of_where_few_rows_end(m, n, k, gpu):
