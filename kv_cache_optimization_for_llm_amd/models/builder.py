@@ -236,10 +236,10 @@ class Model:
 
     def tune_products(self, row_counts, say=None) -> List[dict]:
         """For every row count, has the vendor GEMM library's algorithms timed for each shape of
-        bf16 Linear that goes to the library at that many rows (``ops.kernels.gemm_vendor_tune``;
+        bf16 Linear that goes to the library at that many rows (``ops.gemm_bf16.tune_linear``;
         the same projection of all layers shares a shape and the layers' weights are used in
         turn).  Seconds per shape: start-up work.  Returns one record per (rows, shape)."""
-        from ..ops.gemm_bf16 import use_skinny
+        from ..ops.gemm_bf16 import tune_linear, use_skinny
         shapes: Dict[tuple, List[Linear]] = {}
         for lin in self.linears():
             if lin.weight.is_cuda and lin.weight.dtype == torch.bfloat16:
@@ -249,7 +249,7 @@ class Model:
             for (n, k, halves), lins in shapes.items():
                 if lins[0].tiled is not None and (use_skinny(rows, n, k, halves == 2) or use_skinny(rows, n, k)):
                     continue                                    # the few-rows kernel takes these
-                first, best, tried = K.gemm_vendor_tune(rows, [lin.weight for lin in lins[:16]])
+                first, best, tried = tune_linear(rows, [lin.weight for lin in lins[:16]])
                 report.append(dict(rows=rows, n=n, k=k, heuristic_us=round(first, 2), kept_us=round(best, 2),
                                    algorithms_run=tried))
                 if say is not None:

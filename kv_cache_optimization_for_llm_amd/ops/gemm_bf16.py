@@ -95,14 +95,48 @@ def use_gemv(m: int, n: int, k: int) -> bool:
 # compute units, or its better tiles: taken as a product of their own behind the others, K = 2,048, whole -> in two, us: 2,048
 # rows, 8,208 outputs 83 -> 61, 6,160 59 -> 53, 4,128 42 -> 41; 4,096 rows, 8,208 141 -> 111, 4,128 82 -> 61, 5,152 94 -> 95;
 # 6,000 rows, 8,208 220 -> 163; 1,203 rows, 8,208 50 -> 44, 6,160 37 -> 40; 512 rows, 8,208 26 -> 29, 12,304 36 -> 35.  The small
-# product takes 6-10 us, so from 2^23 results on (32 of them at most in the last tile, as measured).
+# product takes 6-10 us, so from 2^23 results on (32 of them at most in the last tile, as measured).  At K = 512 / 1,024 / 4,096: 2,048
+# rows, 8,208 outputs 52 -> 28 / 64 -> 40 / 153 -> 110, 6,160 31 -> 33 / 40 -> 34 / 106 -> 97, 12,304 59 -> 45 / 67 -> 61 / 189 -> 186; 4,096 rows,
+# 4,128 53 -> 31 / 50 -> 39 / 150 -> 103; 1,024 rows, 12,304 31 -> 33 / 41 -> 35 / 113 -> 98.
+# That is by the library's own choice of an algorithm.  Where a server has the algorithms timed (tune_linear) the whole is often the
+# faster way (2,048 rows, K = 2,048, whole / in two, both timed: 6,160 51 / 58, 12,304 95 / 119, but 8,208 79 / 65), so both are.
 CUT_OUTPUTS, CUT_REST, CUT_RESULTS = 256, 32, 1 << 23
+_TIMED_CUTS: dict = {}          # (device, outputs, K, result's type) -> {rows: whether the two were faster}, as the library's algorithms are kept
 
 
 def vendor_cut(m: int, n: int) -> int:
     """How many of ``n`` outputs the first of two library products takes; 0: one product takes all."""
     rest = n % CUT_OUTPUTS
     return n - rest if 0 < rest <= CUT_REST and n > CUT_OUTPUTS and m * n >= CUT_RESULTS else 0
+
+
+def chosen_cut(m: int, n: int, k: int, device, dtype: torch.dtype = torch.bfloat16) -> int:
+    """:func:`vendor_cut`, or 0 where :func:`tune_linear` found the whole product to be faster at this many rows, or at the nearest
+    number above it that was timed, up to twice as many."""
+    cut = vendor_cut(m, n)
+    timed = _TIMED_CUTS.get((device, n, k, dtype)) if cut else None
+    if timed:
+        rows = min((r for r in timed if m <= r <= 2 * m), default=None)
+        if rows is not None and not timed[rows]:
+            return 0
+    return cut
+
+
+def tune_linear(rows: int, weights, out_dtype: torch.dtype = torch.bfloat16) -> tuple:
+    """Has the vendor library's algorithms timed for products of ``rows`` rows with ``weights`` (matrices of one shape), whole and, where
+    :func:`linear_bf16` would cut them, in two; the faster way is kept.  Returns (microseconds by the library's own choice,
+    microseconds of what is kept, algorithms run)."""
+    n, k = weights[0].shape
+    first, best, tried = K.gemm_vendor_tune(rows, weights, out_dtype)
+    cut = vendor_cut(rows, n)
+    if not cut:
+        return first, best, tried
+    parts = [K.gemm_vendor_tune(rows, [w[a:b] for w in weights], out_dtype, columns_of=n) for a, b in ((0, cut), (cut, n))]
+    two = all(p[1] > 0 for p in parts) and (best < 0 or sum(p[1] for p in parts) < best)
+    _TIMED_CUTS.setdefault((weights[0].device, n, k, out_dtype), {})[int(rows)] = two
+    if all(p[0] > 0 for p in parts):
+        first = sum(p[0] for p in parts)                # what runs without the timing
+    return first, sum(p[1] for p in parts) if two else best, tried + sum(p[2] for p in parts)
 
 
 def decode_tune_rows(max_rows: int) -> list:
@@ -134,7 +168,7 @@ def linear_bf16(x: torch.Tensor, w: torch.Tensor, out: torch.Tensor, tiled=None)
         return K.gemv(x, w, out)
     if tiled is not None and use_skinny(x.shape[0], w.shape[0], w.shape[1]):
         return K.gemm_skinny(x, tiled, out)
-    cut = vendor_cut(*out.shape) if out.is_contiguous() else 0
+    cut = chosen_cut(x.shape[0], w.shape[0], w.shape[1], w.device, out.dtype) if out.is_contiguous() else 0
     if cut and K.gemm_vendor(x, w[:cut], out[:, :cut], columns=True) and K.gemm_vendor(x, w[cut:], out[:, cut:], columns=True):
         return out
     if K.gemm_vendor(x, w, out):

@@ -327,12 +327,12 @@ def test_vendor_product_keeps_the_fastest_algorithm_and_the_same_result(gpu):
         K.gemm_vendor_tune(m, [ws[0], rnd(n, k + 32, seed=1).to(gpu)])
 
 
-@pytest.mark.parametrize("m, n, k", [(2048, 4128, 64), (3000, 2824, 96), (2000, 4128, 64), (2048, 4129, 32)])
+@pytest.mark.parametrize("m, n, k", [(2048, 4128, 64), (3000, 2824, 96), (2000, 4128, 64), (2048, 4129, 32), (2048, 4128, 2048), (1025, 8208, 512)])
 @pytest.mark.parametrize("out_dtype", [torch.bfloat16, torch.float32])
 def test_a_few_outputs_past_a_multiple_of_256_in_a_product_of_their_own(m, n, k, out_dtype, gpu):
     """Both sides of where the product is cut in two, by rows and by what is left of the outputs; nothing else of the result is written."""
     from kv_cache_optimization_for_llm_amd.ops.gemm_bf16 import linear_bf16, vendor_cut
-    assert vendor_cut(m, n) == {(2048, 4128): 4096, (3000, 2824): 2816}.get((m, n), 0)
+    assert vendor_cut(m, n) == {(2048, 4128): 4096, (3000, 2824): 2816, (1025, 8208): 8192}.get((m, n), 0)
     g = torch.Generator().manual_seed(m + n)
     x, w = torch.randn((m, k), generator=g).bfloat16(), torch.randn((n, k), generator=g).bfloat16()
     room = torch.full((m + 2, n), 7.0, dtype=out_dtype, device=gpu)
@@ -342,3 +342,23 @@ def test_a_few_outputs_past_a_multiple_of_256_in_a_product_of_their_own(m, n, k,
     bound = want.abs() * (2.0 ** -8 if out_dtype == torch.bfloat16 else 0) + 2.0 ** -20 * k * 4
     assert ((room[1:m + 1].float().cpu() - want).abs() <= bound).all()
     assert (room[0] == 7.0).all() and (room[m + 1] == 7.0).all()
+
+
+def test_a_cut_product_is_timed_both_ways_and_stays_the_same(gpu, monkeypatch):
+    from kv_cache_optimization_for_llm_amd.ops import gemm_bf16 as G
+    monkeypatch.setattr(G, "_TIMED_CUTS", {})
+    m, n, k = 2048, 4128, 96
+    ws = [rnd(n, k, scale=0.05, seed=s).to(gpu) for s in range(2)]
+    x = rnd(m, k, seed=9).to(gpu)
+    want = x.float().cpu() @ ws[1].float().cpu().t()
+    first, best, tried = G.tune_linear(m, ws)
+    assert tried >= 3 and 0 < best and first > 0
+    two = G._TIMED_CUTS[(x.device, n, k, torch.bfloat16)][m]
+    for decided in (two, True, False):
+        G._TIMED_CUTS[(x.device, n, k, torch.bfloat16)][m] = decided
+        seen, one = [], K.gemm_vendor
+        with monkeypatch.context() as patch:
+            patch.setattr(K, "gemm_vendor", lambda a, w, out, **kw: seen.append(w.shape[0]) or one(a, w, out, **kw))
+            got = G.linear_bf16(x, ws[1], torch.full((m, n), 7.0, dtype=torch.bfloat16, device=gpu))
+        assert seen == ([4096, 32] if decided else [4128])
+        assert ((got.float().cpu() - want).abs() <= want.abs() * 2.0 ** -8 + 2.0 ** -20 * k).all()

@@ -339,3 +339,25 @@ def test_the_choice_of_experts_is_made_inside_the_first_product_where_workgroups
                                        (480, 8, True), (480, 16, False), (768, 1, False),           # 22.3/21.7, 25.0/26.8, 41.0/42.2
                                        (1536, 1, False), (1536, 16, False), (256, 8, True), (256, 16, False)):   # 41.2/47.8, 46.5/64.8, 15.6/14.5, 16.4/17.0
         assert moe_choice_inside(workgroups, tokens) == inside, (workgroups, tokens)
+
+
+def test_products_timed_at_start_up_run_the_way_that_was_faster(monkeypatch):
+    """Whole or in two, both timed; rows that were not timed go by the nearest above, up to twice as many; others by the rule."""
+    import torch
+    from kv_cache_optimization_for_llm_amd.ops import gemm_bf16 as G
+    calls, us = [], {}
+    monkeypatch.setattr(G, "_TIMED_CUTS", {})
+    monkeypatch.setattr(G.K, "gemm_vendor_tune", lambda rows, ws, dtype, columns_of=0: calls.append((rows, ws[0].shape[0], columns_of)) or us[ws[0].shape[0]])
+    ws, dev = [torch.empty((8208, 64), dtype=torch.bfloat16)] * 2, torch.device("cpu")
+    assert G.chosen_cut(2048, 8208, 64, dev) == 8192
+    us.update({8208: (84.0, 50.0, 9), 8192: (56.0, 48.0, 8), 16: (8.0, 6.0, 7)})
+    assert G.tune_linear(2048, ws) == (64.0, 50.0, 24) and calls == [(2048, 8208, 0), (2048, 8192, 8208), (2048, 16, 8208)]
+    assert [G.chosen_cut(m, 8208, 64, dev) for m in (2049, 2048, 1500, 1024, 1023, 1022)] == [8192, 0, 0, 0, 8192, 8192 if 1022 * 8208 >= G.CUT_RESULTS else 0]
+    assert G.chosen_cut(2048, 8208, 32, dev) == G.chosen_cut(2048, 8208, 64, dev, torch.float32) == 8192
+    us[8208] = (84.0, 60.0, 9)
+    assert G.tune_linear(1300, ws) == (64.0, 54.0, 24) and G.chosen_cut(1200, 8208, 64, dev) == 8192 and G.chosen_cut(1400, 8208, 64, dev) == 0
+    us[16] = (-1.0, -1.0, 0)                # the library has nothing for the rest: one product
+    assert G.tune_linear(3000, ws) == (84.0, 60.0, 17) and G.chosen_cut(3000, 8208, 64, dev) == 0
+    calls.clear()
+    us[8192 + 64] = (5.0, 4.0, 3)
+    assert G.tune_linear(2048, [torch.empty((8192 + 64, 64))]) == (5.0, 4.0, 3) and calls == [(2048, 8256, 0)]
