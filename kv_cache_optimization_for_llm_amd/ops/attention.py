@@ -230,11 +230,16 @@ _SHARED_FOUR_BELOW_WIDE = 257
 _SHARED_FOUR_FROM_SHORT_WIDE = 127
 _SHARED_FOUR_FROM = 128             # more (item, kv head) pairs than this ...
 _SHARED_FOUR_BELOW = 512            # ... and fewer than this: four ranges in one workgroup
-# ... and from so many keys on at 512 pairs too, which the chip still takes at once, two workgroups a compute unit.  Steps of 64 requests,
-# 6 layers of the 1B sizes, contexts alike / down to half / down to a tenth, a wavefront a pair -> four: at 1,000 keys 622 / 620 / 621 ->
-# 623 / 600 / 580 us, 1,400 681 / 667 / 665 -> 672 / 648 / 615, 2,000 740 / 739 / 735 -> 755 / 696 / 664, 3,000 884 / 817 / 753 -> 870 /
-# 814 / 755: what one wavefront takes for the longest context is what a step waits for.  72 to 96 requests lose 1-6 % with contexts
-# alike and gain 1-5 % where they differ most: not there.
+# The chip takes four wavefronts a pair of two pairs a compute unit at once, 512 pairs: up to there a step waits for the longest
+# context, whose pairs four wavefronts cut in four; from 513 on it waits for a second turn.  Steps of 6 layers of the 1B sizes, a wavefront a
+# pair / four, contexts alike, down to 3/4, to half, to a tenth of the longest:
+#   63 requests (504 pairs)  700 keys 595/591 591/585 589/576 588/564   2,000 749/754 744/727 745/710 741/662   3,000 858/864 854/843 854/803 847/745
+#   64 requests (512)        700 598/597 596/589 593/581 591/568   1,000 635/632 633/622 632/609 628/589   2,000 749/766 745/734 738/701 736/666
+#                            3,000 862/872 858/847 856/808 851/747
+#   65 requests (520)        700 739/754 727/740 725/731 728/713   1,000 758/784 762/772 760/760 760/732   2,000 876/932 882/902 871/868 871/810
+#                            3,000 1,012/1,094 1,005/1,058 996/1,005 986/894
+# (A served step knows the longest context alone, rounded up: contexts alike to the key lose 1-2 % at 2,000 and 3,000 keys on 504 and 512 pairs
+# alike, any others gain up to 12 %.)  Below 1,024 keys 512 pairs stay with a wavefront each, as they were: level where contexts are alike.
 _SHARED_FOUR_FULL_FROM = 1024
 _SHARED_SHORT_CONTEXT = 1024        # up to this many keys already from ...
 _SHARED_FOUR_FROM_SHORT = 63        # ... this many pairs (8 / 12 / 16 requests at 768 keys 0.854 / 0.912 / 0.959 ->
@@ -305,7 +310,7 @@ def choose_decode_ranges(num_items: int, num_kv_heads: int, max_context: int, he
     pairs = max(1, num_items * num_kv_heads)
     below = _SHARED_FOUR_BELOW if max_context < _SHARED_LONG_CONTEXT else _SHARED_FOUR_BELOW_LONG
     if _SHARED_FOUR_FULL_FROM <= max_context < _SHARED_LONG_CONTEXT:
-        below = _SHARED_FOUR_BELOW + 1
+        below = 2 * _COMPUTE_UNITS + 1
     wide = head_dim > _SHARED_TUNED_HEAD_DIM
     if wide:
         below = _SHARED_FOUR_BELOW_WIDE
