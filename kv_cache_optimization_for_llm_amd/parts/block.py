@@ -78,7 +78,7 @@ class ParallelBlock(Block):
         super().__init__(mixer, feed_forward, norms)
         self.mixer_norm = self.norms["mixer"]
         self.ffn_norm = self.norms.get("feed_forward")
-        # (a norm of the other kind, or an operation between layers, adds the rows up first)
+        # (the pass that takes both outputs forms the sum; an operation between layers has it formed first)
         if self.has_ffn and hasattr(feed_forward, "leaves_rows"):
             feed_forward.leaves_rows = True
 

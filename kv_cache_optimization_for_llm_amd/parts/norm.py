@@ -45,7 +45,6 @@ class RMSNorm(Norm):
         if out is None:
             rows = x.shape[0] if row_idx is None else row_idx.shape[0]
             out = torch.empty((rows, self.width), dtype=x.dtype, device=x.device)
-        delta = K.added_up(delta)
         if isinstance(delta, K.PartialSums) and (x.dtype != torch.bfloat16 or self.width % 8):
             delta = delta.materialize()
         return K.rmsnorm(x, self.weight, self.eps, out, delta=delta, row_idx=row_idx)
@@ -141,7 +140,7 @@ class LayerNorm(Norm):
                 raise TypeError(f"{self.prefix}: this norm takes a pending output with its way into the stream's copies")
             if delta is not None and delta.streams != self.streams:
                 raise ValueError(f"{self.prefix}: the pending output belongs to a stream of {delta.streams} copies")
-            enter = {} if delta is None else dict(y=K.added_up(delta.y), mix=delta.mix, out_w=delta.out_w, mult=delta.mult)
+            enter = {} if delta is None else dict(y=delta.y, mix=delta.mix, out_w=delta.out_w, mult=delta.mult)
             return K.hyper_step(x, self.streams, in_w=self._ones, norm_weight=self.weight, norm_bias=self.bias,
                                 eps=self.eps, out=out, row_idx=row_idx, **enter)
         return K.layernorm(x, self.weight, self.eps, out, deltas=self._deltas(delta), row_idx=row_idx,
