@@ -50,8 +50,10 @@ template <> struct Vec4<bf16_t> {
 // one token at 200 / 2,000 keys 34 / 307 -> 11 / 77 (bound by the chains: 64 dependent additions a block for the score,
 // 64 for the values), heads of 128 at 2,000 keys 659 -> 185.  A head alone, which is what few rows get, has all of a block's
 // loads under way together instead of a quarter and a half of them: 3 tokens at up to 200 keys 11.3 -> 10.6 (heads of 128 17.0 ->
-// 15.5), one at 2,000 77 -> 66; several heads a wavefront have no registers for it and other wavefronts to hide behind.
-template <typename T, int H>
+// 15.5), one at 2,000 77 -> 66 (bf16 up to 32 keys 0.2 us more); several heads a wavefront have no registers for it and other
+// wavefronts to hide behind, and heads that are not whole rounds of 64 elements would ask for the rest one load after the other (96
+// elements at 200 keys 15.2 -> 17.0).
+template <typename T, int H, bool ALL = false>
 __global__ void __launch_bounds__(KVA_WAVE)
 attention_rowwise_kernel(T *__restrict__ out, const T *__restrict__ q, int q_row_stride,
                          const T *__restrict__ k_cache, const T *__restrict__ v_cache,
@@ -62,8 +64,8 @@ attention_rowwise_kernel(T *__restrict__ out, const T *__restrict__ q, int q_row
     __shared__ __attribute__((aligned(16))) float q_s[H][ATTN_MAX_HEAD_DIM];
     __shared__ __attribute__((aligned(16))) float p_s[H][KVA_WAVE];
     __shared__ long long voff_s[KVA_WAVE];
-    // (of a head alone all of a key's elements, and all values of a block, are asked for before the first is used)
-    constexpr int KEY_LOADS = H == 1 ? 16 : 4, FOURS = H == 1 ? 16 : 8;
+    // ALL: 64 of a key's elements, and all values of a block, are asked for before the first is used
+    constexpr int KEY_LOADS = ALL ? 16 : 4, FOURS = ALL ? 16 : 8;
 
     const int t = blockIdx.x;
     const int qh = blockIdx.y * H;
@@ -161,7 +163,8 @@ attention_rowwise_kernel(T *__restrict__ out, const T *__restrict__ q, int q_row
                                 for (int u = 0; u < 4; ++u) v[g][u] = (these >> (4 * g + u)) & 1 ? v[g][u] : 0.f;
                         }
 #pragma unroll
-                        for (int g = 0; g < FOURS; ++g)
+                        for (int g = 0; g < FOURS; ++g) {
+                            if (ALL && g == 8 && last < 32) break;      // (no keys in the block's second half)
 #pragma unroll
                             for (int h = 0; h < H; ++h) {
                                 const float4 p = *reinterpret_cast<const float4 *>(&p_s[h][i0 + 4 * g]);
@@ -170,6 +173,7 @@ attention_rowwise_kernel(T *__restrict__ out, const T *__restrict__ q, int q_row
                                 a[h] += p.z * v[g][2];
                                 a[h] += p.w * v[g][3];
                             }
+                        }
                     }
                 } else {
                     for (int i = 0; i <= last; ++i)
@@ -235,17 +239,19 @@ extern "C" int kva_attention_rowwise(void *out, const void *q, int q_row_stride,
     const int together = rows >= 12288 && group % 4 == 0 ? 4
                          : rows >= 6144 && group % 3 == 0 ? 3
                          : rows >= 3072 && group % 2 == 0 ? 2 : 1;
-#define KVA_ROWWISE(T, H)                                                                                              \
-    hipLaunchKernelGGL((attention_rowwise_kernel<T, H>), dim3(tokens, num_q_heads / H), dim3(KVA_WAVE), 0, stream, (T *)out, \
+    // (a head alone whose elements are whole rounds of 64 loads' worth; of others the last round would go one load at a time)
+#define KVA_ROWWISE(T, H, ALL)                                                                                         \
+    hipLaunchKernelGGL((attention_rowwise_kernel<T, H, ALL>), dim3(tokens, num_q_heads / H), dim3(KVA_WAVE), 0, stream, (T *)out, \
                        (const T *)q, q_row_stride, (const T *)k_cache, (const T *)v_cache, block_table, max_blocks,    \
                        tok_seat, tok_pos, num_q_heads, num_kv_heads, head_dim, value_dim, page_size, fours, scale,     \
                        window, keep_first, chunk, sinks)
 #define KVA_ROWWISE_HEADS(T)                                                                                           \
     do {                                                                                                               \
-        if (together == 4) KVA_ROWWISE(T, 4);                                                                          \
-        else if (together == 3) KVA_ROWWISE(T, 3);                                                                     \
-        else if (together == 2) KVA_ROWWISE(T, 2);                                                                     \
-        else KVA_ROWWISE(T, 1);                                                                                        \
+        if (together == 4) KVA_ROWWISE(T, 4, false);                                                                          \
+        else if (together == 3) KVA_ROWWISE(T, 3, false);                                                                     \
+        else if (together == 2) KVA_ROWWISE(T, 2, false);                                                                     \
+        else if (head_dim % 64 == 0) KVA_ROWWISE(T, 1, true);                                                          \
+        else KVA_ROWWISE(T, 1, false);                                                                                 \
     } while (0)
     if (dtype == KVA_F32) KVA_ROWWISE_HEADS(float);
     else if (dtype == KVA_BF16) KVA_ROWWISE_HEADS(bf16_t);
