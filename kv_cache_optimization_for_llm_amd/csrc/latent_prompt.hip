@@ -9,13 +9,14 @@
 //   * latent_expand_kernel: the entries' whole contexts (cached rows, by page) times [U_k ; U_v], rounded to
 //     bf16, keys' heads and then values' heads one after the other, a position a row of 128 elements; the rotated key parts,
 //     which all heads share, are laid side by side in the same launch.
-//   * latent_prompt_kernel: a workgroup takes 64 tokens of an entry and one head, a wavefront 32 of the tokens and half of
-//     the keys.  As in latent_attention_mfma.hip everything is transposed, S^T = K Q^T and O^T = V^T P^T; blocks of 64 keys go
-//     through LDS for the four wavefronts (the next one's loads in flight), V^T is read there with the transposing load.  The
+//   * latent_prompt_kernel: a workgroup takes 64 tokens of an entry and one head, a wavefront 16 of the tokens;
+//     latent_prompt_wide_kernel: a wavefront 32 of the tokens and half of the keys (latent_prompt_wide says where).  As in
+//     latent_attention_mfma.hip everything is transposed, S^T = K Q^T and O^T = V^T P^T; blocks of 32 or 64 keys go through LDS
+//     for the four wavefronts (the next one's loads in flight), V^T is read there with the transposing load.  The
 //     queries' rotation happens as they are loaded, sink and output gate where the result is normalised.
-// A SIMD issues matrix products (40 of 16 cycles a block and wavefront) or the softmax's vector work (about as
-// much), and LDS gives the four wavefronts 20 KiB each a block (640 cycles).  The
-// workgroups with the most keys are launched first (of those that the chip takes at once, the longest beside the shortest); a
+// A SIMD issues matrix products (20 of 16 cycles a block and wavefront; wide: 40) or the softmax's vector work (about as
+// much), and LDS gives the four wavefronts 20 KiB each a block (640 cycles): without the wide form's second use of what is read, the
+// three are about even.  The workgroups with the most keys are launched first (wide: the longest beside the shortest); a
 // head's workgroups are on one die where the heads are a multiple of eight, whose L2 holds its keys and values.
 //
 // us a layer, one prompt of 2,048 tokens, 16 heads of 128 + 64 / 128, rank 512: over the cached rows 183, the products
@@ -29,7 +30,8 @@
 #define LP_ROT 64
 #define LP_VDIM 128
 static_assert(LP_DIM == LP_VDIM, "expanded keys and values lie in rows of one size");
-#define LP_KEYS 64                  // keys a block
+#define LP_BLOCK 32                 // keys a block
+#define LP_WIDE_BLOCK 64            // ... of the wide kernel
 #define LP_ROWS 64                  // tokens a workgroup
 
 struct LatentPrompt {
@@ -133,25 +135,146 @@ __device__ __forceinline__ void lp_rotate(Frag8 (&f)[2], const float *cos, const
         for (int i = 0; i < 8; ++i) f[s].h[i] = float_to_bf16_bits(y[s][i]);
 }
 
-// A workgroup takes 64 tokens of one head, 64 keys at a time through LDS; a wavefront 32 of the tokens (wave % 2) and 32 of the keys
-// (wave / 2), and the two halves of the keys are added up at the end.  What bounds it is what the wavefronts read from LDS: 20 KiB
-// of keys and values for 40 products of 16 cycles.  (16 tokens and all keys a wavefront read the same for 20: 2,048 tokens of 16
-// heads 72 us.)  Blocks of keys go through registers, the next ones on their way over the products.
+// A wavefront takes 16 of the tokens and all keys; blocks of 32 keys go to one half of LDS while the other is read.
 __global__ void __launch_bounds__(256, 2)
 latent_prompt_kernel(LatentPrompt a, int tiles) {
     constexpr int KD = LP_DIM + LP_ROT, KS = KD / 32, NDT = LP_VDIM / 16;
     constexpr int KSTRIDE = KD + 8, VSTRIDE = LP_VDIM + 24;     // (rows of either kind of read on banks of their own)
+    __shared__ __align__(16) bf16_t Ks[2][LP_BLOCK * KSTRIDE];
+    __shared__ __align__(16) bf16_t Vs[2][LP_BLOCK * VSTRIDE];
+    const int e = blockIdx.y, head = blockIdx.x % a.heads, tile = tiles - 1 - (int)(blockIdx.x / a.heads);
+    const int q0 = a.entry_q_start[e], n = a.entry_q_start[e + 1] - q0, start = a.entry_start_pos[e];
+    if (tile * LP_ROWS >= n) return;
+    const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid / KVA_WAVE), lane = tid % KVA_WAVE, r = lane & 15, g = lane >> 4;
+    const int first = tile * LP_ROWS + 16 * wave;               // the wavefront's first token
+    const int mine = min(first + r, n - 1), pos = start + mine;
+    const int hi = first < n ? start + min(first + 15, n - 1) : -1;     // newest key of the wavefront's tokens, and of the workgroup's
+    const int end = start + min(tile * LP_ROWS + LP_ROWS, n);           // (one past it)
+    const bf16_t *kv = a.kv + ((size_t)e * 2 * a.heads + head) * a.context * LP_DIM, *rot = a.rot + (size_t)e * a.context * LP_ROT;
+    const size_t to_values = (size_t)a.heads * a.context * LP_DIM;
+
+    Frag8 qf[KS];
+    {
+        const bf16_t *q = a.q + (size_t)(q0 + mine) * a.q_row + (size_t)head * a.q_head + 8 * g;
+#pragma unroll
+        for (int ks = 0; ks < KS; ++ks) qf[ks].u4 = *reinterpret_cast<const uint4 *>(q + 32 * ks);
+        Frag8 turned[2] = {qf[KS - 2], qf[KS - 1]};
+        lp_rotate(turned, a.cos + (size_t)pos * (LP_ROT / 2), a.sin + (size_t)pos * (LP_ROT / 2), g, a.interleaved != 0);
+        qf[KS - 2] = turned[0];
+        qf[KS - 1] = turned[1];
+    }
+    // a block's pieces on their way: rows tid / 16 and 16 further of keys and values, row tid / 8 of the rotated parts
+    uint4 k_lo, k_hi, v_lo, v_hi, turned_k;
+    auto load = [&](int k0) {
+        const bf16_t *lo = kv + (size_t)min(k0 + tid / 16, end - 1) * LP_DIM + 8 * (tid % 16);
+        const bf16_t *up = kv + (size_t)min(k0 + tid / 16 + 16, end - 1) * LP_DIM + 8 * (tid % 16);
+        k_lo = *reinterpret_cast<const uint4 *>(lo);
+        v_lo = *reinterpret_cast<const uint4 *>(lo + to_values);
+        k_hi = *reinterpret_cast<const uint4 *>(up);
+        v_hi = *reinterpret_cast<const uint4 *>(up + to_values);
+        turned_k = *reinterpret_cast<const uint4 *>(rot + (size_t)min(k0 + tid / 8, end - 1) * LP_ROT + 8 * (tid % 8));
+    };
+    f32x4 o[NDT];
+#pragma unroll
+    for (int dt = 0; dt < NDT; ++dt) o[dt] = f32x4{0.f, 0.f, 0.f, 0.f};
+    float m = -INFINITY, l = 0.f;                               // m in the base-2 domain, l this lane's part
+    const float scale2 = a.scale * LP_LOG2E;
+    load(0);
+    for (int k0 = 0, buf = 0; k0 < end; k0 += LP_BLOCK, buf ^= 1) {
+        bf16_t *kp = &Ks[buf][tid / 16 * KSTRIDE + 8 * (tid % 16)], *vp = &Vs[buf][tid / 16 * VSTRIDE + 8 * (tid % 16)];
+        *reinterpret_cast<uint4 *>(kp) = k_lo;
+        *reinterpret_cast<uint4 *>(kp + 16 * KSTRIDE) = k_hi;
+        *reinterpret_cast<uint4 *>(vp) = v_lo;
+        *reinterpret_cast<uint4 *>(vp + 16 * VSTRIDE) = v_hi;
+        *reinterpret_cast<uint4 *>(&Ks[buf][tid / 8 * KSTRIDE + LP_DIM + 8 * (tid % 8)]) = turned_k;
+        __syncthreads();            // (a buffer was read last two turns ago: every wavefront has passed the barrier between)
+        if (k0 + LP_BLOCK < end) load(k0 + LP_BLOCK);
+        if (k0 > hi) continue;                                  // (the wavefront's tokens see none of these)
+        f32x4 s[2] = {f32x4{0.f, 0.f, 0.f, 0.f}, f32x4{0.f, 0.f, 0.f, 0.f}};
+#pragma unroll
+        for (int ks = 0; ks < KS; ++ks)
+#pragma unroll
+            for (int t = 0; t < 2; ++t) {
+                Frag8 k;
+                k.u4 = *reinterpret_cast<const uint4 *>(&Ks[buf][(16 * t + r) * KSTRIDE + 32 * ks + 8 * g]);
+                s[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(k.v, qf[ks].v, s[t], 0, 0, 0);
+            }
+        const bool whole = k0 + LP_BLOCK - 1 <= start + first;   // all of the wavefront's tokens see all of the keys
+        float sv[8], mx = -INFINITY;
+#pragma unroll
+        for (int t = 0; t < 2; ++t)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                float x = s[t][i] * scale2;
+                if (!whole) x = k0 + 16 * t + 4 * g + i <= pos ? x : -INFINITY;
+                sv[4 * t + i] = x;
+                mx = fmaxf(mx, x);
+            }
+        const float bm = quad_rows_max(mx);
+        // (the reference of the exponentials moves only when a maximum has grown by more than 2^8)
+        if (__builtin_amdgcn_ballot_w64(bm > m + 8.f) != 0) {
+            const float m_new = fmaxf(m, bm), corr = __builtin_amdgcn_exp2f(m - ((m_new == -INFINITY) ? 0.f : m_new));     // exp2(-inf) = 0
+            l *= corr;
+#pragma unroll
+            for (int dt = 0; dt < NDT; ++dt)
+#pragma unroll
+                for (int c = 0; c < 4; ++c) o[dt][c] *= corr;
+            m = m_new;
+        }
+        const float ref = m == -INFINITY ? 0.f : m;
+        Frag8 pf;
+#pragma unroll
+        for (int j = 0; j < 8; j += 2) {
+            const float p0 = __builtin_amdgcn_exp2f(sv[j] - ref), p1 = __builtin_amdgcn_exp2f(sv[j + 1] - ref);
+            l += p0 + p1;
+            pf.p2[j / 2] = pack_bf16(p0, p1);
+        }
+        const bf16_t *get = &Vs[buf][(4 * g + (r >> 2)) * VSTRIDE + 4 * (r & 3)];
+#pragma unroll
+        for (int dt = 0; dt < NDT; ++dt) o[dt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(lp_values<VSTRIDE>(get, dt).v, pf.v, o[dt], 0, 0, 0);
+    }
+    l = quad_rows_sum(l);
+    if (first + r >= n) return;
+    float mul = 1.f / l;
+    if (a.sinks) {                                              // one more term of the denominator, with no key and no value
+        const float sk = a.sinks[head] * LP_LOG2E, m_new = fmaxf(m, sk), corr = __builtin_amdgcn_exp2f(m - m_new);
+        mul = corr / (l * corr + __builtin_amdgcn_exp2f(sk - m_new));
+    }
+    const bf16_t *gate = a.gates ? a.gates + (size_t)(q0 + mine) * a.gate_row : nullptr;
+    if (gate && !a.gate_per_element) mul *= 1.f / (1.f + expf(-to_float(gate[head])));
+    bf16_t *out = a.out + ((size_t)(q0 + mine) * a.heads + head) * LP_VDIM;
+#pragma unroll
+    for (int dt = 0; dt < NDT; ++dt) {
+        const int c = 16 * dt + 4 * g;
+        float v[4];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            v[i] = o[dt][i] * mul;
+            if (gate && a.gate_per_element) v[i] *= 1.f / (1.f + expf(-to_float(gate[(size_t)head * a.gate_head + c + i])));
+        }
+        const b16x2 lo = pack_bf16(v[0], v[1]), hi2 = pack_bf16(v[2], v[3]);
+        *reinterpret_cast<uint2 *>(out + c) = make_uint2(__builtin_bit_cast(unsigned, lo), __builtin_bit_cast(unsigned, hi2));
+    }
+}
+
+// 64 keys at a time through LDS; a wavefront takes 32 of the tokens (wave % 2) and 32 of the keys (wave / 2), and the two halves of
+// the keys are added up at the end.  What bounds it is what the wavefronts read from LDS: 20 KiB of keys and values for 40 products
+// of 16 cycles, twice as many as above.  Blocks of keys go through registers, the next ones on their way over the products.
+__global__ void __launch_bounds__(256, 2)
+latent_prompt_wide_kernel(LatentPrompt a, int tiles) {
+    constexpr int KD = LP_DIM + LP_ROT, KS = KD / 32, NDT = LP_VDIM / 16;
+    constexpr int KSTRIDE = KD + 8, VSTRIDE = LP_VDIM + 24;     // (rows of either kind of read on banks of their own)
     __shared__ __align__(16) union {
         struct {
-            bf16_t k[LP_KEYS * KSTRIDE], v[LP_KEYS * VSTRIDE];
+            bf16_t k[LP_WIDE_BLOCK * KSTRIDE], v[LP_WIDE_BLOCK * VSTRIDE];
         } b;
         struct {
             float o[2][2][NDT][KVA_WAVE][4], m[2][2][KVA_WAVE], l[2][2][KVA_WAVE];
         } half;                                                 // of the wavefronts with the second half of the keys
     } lds;
-    // The workgroups that the chip takes at once: the longest and the shortest on one compute unit.  More of them: the longest first.
+    // (the chip takes all of them at once: the longest and the shortest on one compute unit)
     const int e = blockIdx.y, head = blockIdx.x % a.heads, at = blockIdx.x / a.heads, front = (tiles + 1) / 2;
-    const int tile = at < front || gridDim.x * gridDim.y > 512 ? tiles - 1 - at : at - front;
+    const int tile = at < front ? tiles - 1 - at : at - front;
     const int q0 = a.entry_q_start[e], n = a.entry_q_start[e + 1] - q0, start = a.entry_start_pos[e];
     if (tile * LP_ROWS >= n) return;
     const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid / KVA_WAVE), lane = tid % KVA_WAVE, r = lane & 15, g = lane >> 4;
@@ -197,7 +320,7 @@ latent_prompt_kernel(LatentPrompt a, int tiles) {
         for (int dt = 0; dt < NDT; ++dt) o[rt][dt] = f32x4{0.f, 0.f, 0.f, 0.f};
     const float scale2 = a.scale * LP_LOG2E;
     load(0);
-    for (int k0 = 0; k0 < end; k0 += LP_KEYS) {
+    for (int k0 = 0; k0 < end; k0 += LP_WIDE_BLOCK) {
         __syncthreads();                                        // every wavefront is done with the block before
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
@@ -208,7 +331,7 @@ latent_prompt_kernel(LatentPrompt a, int tiles) {
         for (int j = 0; j < 2; ++j)
             *reinterpret_cast<kva_u32x4 *>(&lds.b.k[(tid / 8 + 32 * j) * KSTRIDE + LP_DIM + 8 * (tid % 8)]) = tx[j];
         __syncthreads();
-        if (k0 + LP_KEYS < end) load(k0 + LP_KEYS);
+        if (k0 + LP_WIDE_BLOCK < end) load(k0 + LP_WIDE_BLOCK);
         const int kb = k0 + 32 * keys;
         if (kb > hi) continue;                                  // (the wavefront's tokens see none of these)
         const bf16_t *kp = &lds.b.k[(32 * keys + r) * KSTRIDE + 8 * g];
@@ -319,6 +442,15 @@ extern "C" int kva_latent_prompt_supported(int dim, int rot, int vdim, int rank)
     return dim == LP_DIM && rot == LP_ROT && vdim == LP_VDIM && rank > 0 && rank % LDSP_K == 0;
 }
 
+// Whether a wavefront takes 32 tokens and half of the keys (or 16 and all of them).  That reads LDS half as often and ends with sums over the
+// halves and two more barriers a block, which long contexts repay, as long as the chip takes all workgroups at once; past that, one more
+// turn of them, four fewer wavefronts a compute unit weigh more.  16 tokens / 32, us with the expansion, rank 512:
+//   one entry of 16 heads from position 0:  64 tokens 16.4/19.2  256 22.1/24.7  512 30.2/32.4  1,000 44.2/44.2  1,400 56.1/55.1  2,048 (512
+//   workgroups) 75.5/68.8  4,096 (1,024) 157/169;  of 8 heads 2,048 70.4/68.4  4,096 (512) 127/112;  of 32 heads 1,000 50.3/50.2  1,400 (704)
+//   69.2/69.2  2,048 (1,024) 98.9/109;  of 64 heads 1,000 (1,024) 73.9/79.6  2,048 202/209
+//   behind 1,024 positions, 16 heads:  64 44.6/45.4  256 49.8/49.7  512 56.2/55.5  1,400 87.8/83.3  four of 512 90.0/89.3  four of 700 (704) 122/125
+static bool latent_prompt_wide(long long workgroups, int longest, int context) { return workgroups <= 512 && context > 1024 && longest >= 256; }
+
 // kv bf16 [entries, 2 heads, context, 128] and rot bf16 [entries * context, rot] are workspace; `context` is no
 // smaller than any entry's first position + tokens, `longest` than its tokens.
 extern "C" int kva_latent_prompt(void *out, const void *q, int q_row, int q_head, const void *cache, const void *w, void *kv,
@@ -341,7 +473,10 @@ extern "C" int kva_latent_prompt(void *out, const void *q, int q_row, int q_head
     const long long expand = (long long)((context + 127) / 128) * heads, tiles = (longest + LP_ROWS - 1) / LP_ROWS;
     KVA_REQUIRE(expand <= 0x7fffffff && tiles * heads <= 0x7fffffff, "latent_prompt: too many workgroups");
     hipLaunchKernelGGL(latent_expand_kernel, dim3((unsigned)expand, entries), dim3(256), 0, stream, a);
-    hipLaunchKernelGGL(latent_prompt_kernel, dim3((unsigned)(tiles * heads), entries), dim3(256), 0, stream, a, (int)tiles);
+    if (latent_prompt_wide(tiles * heads * entries, longest, context))
+        hipLaunchKernelGGL(latent_prompt_wide_kernel, dim3((unsigned)(tiles * heads), entries), dim3(256), 0, stream, a, (int)tiles);
+    else
+        hipLaunchKernelGGL(latent_prompt_kernel, dim3((unsigned)(tiles * heads), entries), dim3(256), 0, stream, a, (int)tiles);
     KVA_CHECK_LAUNCH("latent_prompt");
     return KVA_OK;
 }

@@ -334,11 +334,12 @@ def test_rows_of_several_entries_in_items_of_both_sizes(heads, rank, rot, page, 
 # ---------------------------------------------------------------- feed-forwards
 @pytest.mark.parametrize("interleaved, gate, sink", [(True, "element", True), (False, "head", False), (True, None, True)])
 @pytest.mark.parametrize("heads, rank, page, entries", [(1, 32, 16, [(0, 1)]), (3, 96, 16, [(0, 63), (5, 64), (200, 65)]), (16, 512, 16, [(0, 300), (700, 129)]), (40, 32, 16, [(3, 900)]),
+                                                        (3, 64, 16, [(5, 1200)]), (4, 96, 16, [(900, 300), (1021, 257), (0, 64)]), (6, 32, 16, [(1030, 256), (17, 1)]),
                                                         (4, 512, 48, [(31, 257), (0, 33), (96, 128), (1, 1)])])
 def test_prompts_over_expanded_keys_and_values(heads, rank, page, entries, interleaved, gate, sink, gpu):
     """Entries (first position, tokens) whose tokens and contexts end inside, at and behind tiles of 64 tokens, blocks of 64 keys, their
-    halves and tiles of 128 positions, on pages in no order, a context bound larger than any of them; more workgroups than the chip
-    takes at once (40 heads of 900 tokens), which go out in another order."""
+    halves and tiles of 128 positions, on pages in no order, a context bound larger than any of them; 16 tokens a wavefront or (contexts
+    above 1,024, at least 256 tokens, no more workgroups than the chip takes at once) 32."""
     d, rot, dv, T = 128, 64, 128, sum(n for _, n in entries)
     context = max(s + n for s, n in entries) + 37
     blocks = -(-context // page)
@@ -387,10 +388,10 @@ def test_prompts_over_expanded_keys_and_values(heads, rank, page, entries, inter
         assert (got - want).norm() <= 2.0 ** -9 * 5 ** 0.5 * 1.5 * want.norm(), e
 
 
-@pytest.mark.parametrize("heads, start, n", [(2, 0, 100), (2, 5, 100), (3, 39, 64), (40, 3, 900)])
+@pytest.mark.parametrize("heads, start, n", [(2, 0, 100), (2, 5, 100), (3, 39, 64), (40, 3, 900), (2, 0, 1100), (3, 1029, 260), (2, 1039, 300), (2, 1045, 256)])
 def test_a_prompts_later_positions_leave_earlier_tokens_alone(heads, start, n, gpu):
-    """Positions that are no numbers: tokens of the 16 beside them that see none of the 32 keys beside theirs have the bits that they have
-    without, in every order that the workgroups are launched in (40 heads of 900 tokens: more than the chip takes at once)."""
+    """Positions that are no numbers: tokens that, with the 16 that they go with, see none of the 32 keys beside theirs have the bits that
+    they have without, with 16 tokens a wavefront and with 32."""
     d, rot, rank, page = 128, 64, 32, 16
     context, T = start + n + 9, n
     blocks = -(-context // page)
@@ -407,7 +408,7 @@ def test_a_prompts_later_positions_leave_earlier_tokens_alone(heads, start, n, g
     want = run(rows)
     assert want.isfinite().all()
     newest = start + torch.clamp(torch.arange(n) // 16 * 16 + 15, max=n - 1)       # of a token's 16
-    for bad in sorted({start, start + n - 1, start + n // 2, start + 17, start + 33, min(64, start + n - 1)}):
+    for bad in sorted({start, start + n - 1, start + n // 2, start + 17, start + 33, max(start, min(64, start + n - 1))}):
         spoilt = rows.clone()
         spoilt[bad] = float("nan") if bad % 2 else float("inf")
         got = run(spoilt)
