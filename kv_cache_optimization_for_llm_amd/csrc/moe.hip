@@ -157,7 +157,6 @@ __device__ inline void moe_route_token(const MoeRoute &a, const float *logits, i
         return;
     }
     float total = 0.f;
-    unsigned taken = 0u;                // this lane's outputs that are chosen
     for (int k = 0; k < a.top; ++k) {
         // the largest remaining choice score; of equal ones the lowest index
         float bv = -INFINITY, bs = 0.f;
@@ -165,7 +164,7 @@ __device__ inline void moe_route_token(const MoeRoute &a, const float *logits, i
 #pragma unroll
         for (int j = 0; j < PL; ++j) {
             const int e = lane + j * KVA_WAVE;
-            if (e < a.outputs && !((taken >> j) & 1u) && (ch[j] > bv || (ch[j] == bv && e < be))) { bv = ch[j]; be = e; bs = s[j]; }
+            if (e < a.outputs && (ch[j] > bv || (ch[j] == bv && e < be))) { bv = ch[j]; be = e; bs = s[j]; }
         }
 #pragma unroll
         for (int off = KVA_WAVE / 2; off > 0; off >>= 1) {
@@ -175,7 +174,7 @@ __device__ inline void moe_route_token(const MoeRoute &a, const float *logits, i
         }
 #pragma unroll
         for (int j = 0; j < PL; ++j)
-            if (lane + j * KVA_WAVE == be) taken |= 1u << j;
+            if (lane + j * KVA_WAVE == be) ch[j] = __builtin_nanf("");       // (taken: neither above nor equal to anything)
         total += bs;
         if (lane == 0) {
             idx[k] = be;
