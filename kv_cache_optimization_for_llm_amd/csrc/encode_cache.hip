@@ -254,8 +254,11 @@ extern "C" int kva_qk_encode_cache(void *qkv, int row_stride, int k_off, int v_o
                            (interleaved || rot == 0 ? 0 : (uintptr_t)cos_table | (uintptr_t)sin_table);
     if (dtype == KVA_BF16 && head_dim % 8 == 0 && (vecs & (vecs - 1)) == 0 && vecs <= KVA_WAVE &&
         (interleaved || rot % 16 == 0) && row_stride % 8 == 0 && k_off % 8 == 0 && (wide & 15) == 0) {
-        // (a workgroup a turn over the heads: a second turn behind the first was a second chain of trips to memory)
-        hipLaunchKernelGGL(qk_encode_cache_vec_kernel, dim3(tokens, ((num_q_heads + num_kv_heads) * vecs + 255) / 256), dim3(256), 0, stream, (bf16_t *)qkv, row_stride,
+        // A workgroup a turn over the heads while tokens are few: a second turn behind the first is a second chain of trips to memory
+        // (32 and 8 heads of 64, a token: 7.3 -> 5.1 us).  With many tokens other workgroups are there meanwhile, and the last turn's
+        // mostly idle lanes take room (1,024 tokens 10.7 -> 11.2, 8,192 40.4 -> 44.6).
+        const int turns = tokens <= 512 ? ((num_q_heads + num_kv_heads) * vecs + 255) / 256 : 1;
+        hipLaunchKernelGGL(qk_encode_cache_vec_kernel, dim3(tokens, turns), dim3(256), 0, stream, (bf16_t *)qkv, row_stride,
                            k_off, v_off, (bf16_t *)k_cache, (bf16_t *)v_cache, cos_table, sin_table, positions,
                            slot_mapping, num_q_heads, num_kv_heads, head_dim, value_dim, rot, interleaved, unit_eps,
                            page_size, (const bf16_t *)bias, q_weight, k_weight, norm_first);
@@ -513,11 +516,14 @@ extern "C" int kva_maps_encode_cache(const void *qkv, int row_stride, void *q_ro
     if (tokens == 0) return KVA_OK;
     if (rot == 0) cos_table = sin_table = reinterpret_cast<const float *>(qkv);     // never read
     if (dtype == KVA_BF16 && interleaved && dim % 8 == 0 && row_stride % 8 == 0 &&
-        ((reinterpret_cast<uintptr_t>(qkv) | reinterpret_cast<uintptr_t>(q_rows) | reinterpret_cast<uintptr_t>(bias)) & 15) == 0)
-        hipLaunchKernelGGL(maps_encode_cache_vec_kernel, dim3(tokens, (2 * (heads + kv_heads) * (dim / 8) + 255) / 256), dim3(256), 0, stream, (const bf16_t *)qkv, row_stride,
+        ((reinterpret_cast<uintptr_t>(qkv) | reinterpret_cast<uintptr_t>(q_rows) | reinterpret_cast<uintptr_t>(bias)) & 15) == 0) {
+        // (as above; with more than two turns' worth of maps a token they stay the faster way: 32 and 8 heads of two maps of 64, 8,192 tokens
+        // 130 -> 116 us, 16 and 4, a turn and a quarter, 40.1 -> 42.8 and at 1,024 tokens 10.8 -> 10.2)
+        const int items = 2 * (heads + kv_heads) * (dim / 8), turns = tokens <= 1024 || items > 512 ? (items + 255) / 256 : 1;
+        hipLaunchKernelGGL(maps_encode_cache_vec_kernel, dim3(tokens, turns), dim3(256), 0, stream, (const bf16_t *)qkv, row_stride,
                            (bf16_t *)q_rows, (bf16_t *)k_cache, (bf16_t *)v_cache, cos_table, sin_table, positions,
                            slot_mapping, heads, kv_heads, dim, value_dim, rot, page_size, bias);
-    else if (dtype == KVA_F32)
+    } else if (dtype == KVA_F32)
         hipLaunchKernelGGL(maps_encode_cache_kernel<float>, dim3(tokens), dim3(256), 0, stream, (const float *)qkv, row_stride,
                            (float *)q_rows, (float *)k_cache, (float *)v_cache, cos_table, sin_table, positions,
                            slot_mapping, heads, kv_heads, dim, value_dim, rot, interleaved, page_size, bias);

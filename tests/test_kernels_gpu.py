@@ -1076,3 +1076,47 @@ def test_the_read_probes_take_their_ranges_and_refuse_bad_ones(gpu):
         K.stream_mixed(None, None, 5, sink)
     with pytest.raises(K.KernelError):
         K.stream_mixed(own, shared, 0, sink)
+
+
+@pytest.mark.parametrize("heads, kv_heads, d, tokens", [(32, 8, 64, 512), (32, 8, 64, 513), (40, 16, 64, 700), (3, 1, 128, 600)])
+def test_a_heads_encoding_does_not_depend_on_the_tokens_beside_it(heads, kv_heads, d, tokens, gpu):
+    """Either side of where a token's heads go to one workgroup instead of one a turn: rows, keys and values of a token alone."""
+    width, pages = (heads + 2 * kv_heads) * d, -(-tokens // 16)
+    y = rnd(tokens, width).to(torch.bfloat16).to(gpu)
+    pos = torch.arange(tokens, dtype=torch.int32, device=gpu)
+    angle = torch.rand((tokens, d // 2), generator=torch.Generator().manual_seed(3)).to(gpu) * 6
+    cos, sin = angle.cos(), angle.sin()
+
+    def run(at):
+        k = torch.full((pages, kv_heads, d // 8, 16, 8), 7.0, dtype=torch.bfloat16, device=gpu)
+        v = torch.full((pages, kv_heads, d, 16), 7.0, dtype=torch.bfloat16, device=gpu)
+        rows = y[at].clone()
+        K.qk_encode_cache(rows, pos[at], heads, kv_heads, d, d, cos, sin, False, 1e-6, k, v, pos[at])
+        return rows, k, v
+    rows, k, v = run(slice(0, tokens))
+    for t in (0, 17, tokens - 1):
+        one, k1, v1 = run(slice(t, t + 1))
+        assert torch.equal(one[0], rows[t]), t
+        assert torch.equal(k1[t // 16, :, :, t % 16], k[t // 16, :, :, t % 16]) and torch.equal(v1[t // 16, ..., t % 16], v[t // 16, ..., t % 16]), t
+
+
+@pytest.mark.parametrize("heads, kv_heads, d, tokens", [(16, 4, 64, 1024), (16, 4, 64, 1025), (32, 8, 64, 1025), (3, 1, 32, 1030)])
+def test_a_maps_encoding_does_not_depend_on_the_tokens_beside_it(heads, kv_heads, d, tokens, gpu):
+    width, pages, dv = 2 * (heads + kv_heads) * d + kv_heads * 2 * d, -(-tokens // 16), 2 * d
+    y = rnd(tokens, width).to(torch.bfloat16).to(gpu)
+    pos = torch.arange(tokens, dtype=torch.int32, device=gpu)
+    angle = torch.rand((tokens, d // 2), generator=torch.Generator().manual_seed(3)).to(gpu) * 6
+    cos, sin = angle.cos(), angle.sin()
+
+    def run(at):
+        k = torch.full((pages, kv_heads, 2 * d // 8, 16, 8), 7.0, dtype=torch.bfloat16, device=gpu)
+        v = torch.full((pages, kv_heads, dv, 16), 7.0, dtype=torch.bfloat16, device=gpu)
+        rows = y[at].contiguous()
+        q = torch.full((rows.shape[0], 4 * heads * d), 7.0, dtype=torch.bfloat16, device=gpu)
+        K.maps_encode_cache(rows, q, pos[at], heads, kv_heads, d, dv, cos, sin, True, k, v, pos[at])
+        return q, k, v
+    q, k, v = run(slice(0, tokens))
+    for t in (0, 17, tokens - 1):
+        one, k1, v1 = run(slice(t, t + 1))
+        assert torch.equal(one[0], q[t]), t
+        assert torch.equal(k1[t // 16, :, :, t % 16], k[t // 16, :, :, t % 16]) and torch.equal(v1[t // 16, ..., t % 16], v[t // 16, ..., t % 16]), t
