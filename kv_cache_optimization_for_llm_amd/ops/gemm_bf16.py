@@ -91,23 +91,23 @@ def use_gemv(m: int, n: int, k: int) -> bool:
     return not (n >= GEMV_WIDE_N and k >= GEMV_LONG_K[m] and K.gemm_skinny_supported(m, n, k))
 
 
-# A few outputs past a multiple of 256 (a mixer's gates and decays behind its projections) cost the library's tiles a turn of the
-# compute units, or its better tiles: taken as a product of their own behind the others, K = 2,048, whole -> in two, us: 2,048
-# rows, 8,208 outputs 83 -> 61, 6,160 59 -> 53, 4,128 42 -> 41; 4,096 rows, 8,208 141 -> 111, 4,128 82 -> 61, 5,152 94 -> 95;
-# 6,000 rows, 8,208 220 -> 163; 1,203 rows, 8,208 50 -> 44, 6,160 37 -> 40; 512 rows, 8,208 26 -> 29, 12,304 36 -> 35.  The small
-# product takes 6-10 us, so from 2^23 results on (32 of them at most in the last tile, as measured).  At K = 512 / 1,024 / 4,096: 2,048
-# rows, 8,208 outputs 52 -> 28 / 64 -> 40 / 153 -> 110, 6,160 31 -> 33 / 40 -> 34 / 106 -> 97, 12,304 59 -> 45 / 67 -> 61 / 189 -> 186; 4,096 rows,
-# 4,128 53 -> 31 / 50 -> 39 / 150 -> 103; 1,024 rows, 12,304 31 -> 33 / 41 -> 35 / 113 -> 98.
-# That is by the library's own choice of an algorithm.  Where a server has the algorithms timed (tune_linear) the whole is often the
-# faster way (2,048 rows, K = 2,048, whole / in two, both timed: 6,160 51 / 58, 12,304 95 / 119, but 8,208 79 / 65), so both are.
-CUT_OUTPUTS, CUT_REST, CUT_RESULTS = 256, 32, 1 << 23
+# A few outputs past a multiple of 256 (a mixer's gates and decays behind its projections) cost the library a column of tiles, and where that
+# column begins one more turn of the compute units (tiles of 256 x 256), most of a turn: there the rest is a product of its own.  Whole ->
+# in two, by the library's own choice of algorithms, us at K = 512 / 1,024 / 2,048 / 4,096, 16 outputs past: 2,048 rows, 8,192 outputs 52 -> 28
+# / 58 -> 40 / 75 -> 62 / 128 -> 107, 16,384 74 -> 44 / 97 -> 66 / 144 -> 112 / 287 -> 201; 4,096 rows, 4,096 52 -> 27 / 46 -> 39 / 74 -> 62 / 127 ->
+# 107, 12,288 119 -> 61 / 110 -> 93 / 195 -> 157 / 351 -> 289; 1,600 rows, 9,216 39 -> 27 / 44 -> 38 / 68 -> 60 / 116 -> 105.  Where it begins no
+# turn the two are sometimes ahead and as often behind (2,048 rows, 6,144 31 -> 33 / 38 -> 34 / 55 -> 54 / 88 -> 94, 10,240 63 -> 48 / 54 -> 57 / 84 ->
+# 90 / 148 -> 158; 1,203 rows, 7,168 25 -> 30 / 28 -> 36 / 43 -> 52 / 67 -> 75): one product there.  Up to 32 outputs past, as measured, and from
+# 2^23 results on.  Where a server has the algorithms timed (tune_linear) the whole may be the faster way, so both are.
+CUT_OUTPUTS, CUT_REST, CUT_RESULTS, CUT_ROWS, COMPUTE_UNITS = 256, 32, 1 << 23, 256, 256
 _TIMED_CUTS: dict = {}          # (device, outputs, K, result's type) -> {rows: whether the two were faster}, as the library's algorithms are kept
 
 
 def vendor_cut(m: int, n: int) -> int:
     """How many of ``n`` outputs the first of two library products takes; 0: one product takes all."""
-    rest = n % CUT_OUTPUTS
-    return n - rest if 0 < rest <= CUT_REST and n > CUT_OUTPUTS and m * n >= CUT_RESULTS else 0
+    rows, columns, rest = -(-m // CUT_ROWS), n // CUT_OUTPUTS, n % CUT_OUTPUTS
+    turns = [-(-rows * c // COMPUTE_UNITS) for c in (columns, columns + 1)]
+    return n - rest if 0 < rest <= CUT_REST and columns and m * n >= CUT_RESULTS and turns[1] > turns[0] else 0
 
 
 def chosen_cut(m: int, n: int, k: int, device, dtype: torch.dtype = torch.bfloat16) -> int:

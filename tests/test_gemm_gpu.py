@@ -327,12 +327,13 @@ def test_vendor_product_keeps_the_fastest_algorithm_and_the_same_result(gpu):
         K.gemm_vendor_tune(m, [ws[0], rnd(n, k + 32, seed=1).to(gpu)])
 
 
-@pytest.mark.parametrize("m, n, k", [(2048, 4128, 64), (3000, 2824, 96), (2000, 4128, 64), (2048, 4129, 32), (2048, 4128, 2048), (1025, 8208, 512)])
+@pytest.mark.parametrize("m, n, k", [(4096, 4128, 64), (2000, 8224, 96), (2048, 4128, 64), (4096, 4129, 32), (2048, 8208, 2048), (1793, 8193, 512)])
 @pytest.mark.parametrize("out_dtype", [torch.bfloat16, torch.float32])
 def test_a_few_outputs_past_a_multiple_of_256_in_a_product_of_their_own(m, n, k, out_dtype, gpu):
-    """Both sides of where the product is cut in two, by rows and by what is left of the outputs; nothing else of the result is written."""
+    """Both sides of where the product is cut in two, by turns of tiles and by what is left of the outputs; nothing else of the result is
+    written."""
     from kv_cache_optimization_for_llm_amd.ops.gemm_bf16 import linear_bf16, vendor_cut
-    assert vendor_cut(m, n) == {(2048, 4128): 4096, (3000, 2824): 2816, (1025, 8208): 8192}.get((m, n), 0)
+    assert vendor_cut(m, n) == {(4096, 4128): 4096, (2000, 8224): 8192, (2048, 8208): 8192, (1793, 8193): 8192}.get((m, n), 0)
     g = torch.Generator().manual_seed(m + n)
     x, w = torch.randn((m, k), generator=g).bfloat16(), torch.randn((n, k), generator=g).bfloat16()
     room = torch.full((m + 2, n), 7.0, dtype=out_dtype, device=gpu)
@@ -347,7 +348,7 @@ def test_a_few_outputs_past_a_multiple_of_256_in_a_product_of_their_own(m, n, k,
 def test_a_cut_product_is_timed_both_ways_and_stays_the_same(gpu, monkeypatch):
     from kv_cache_optimization_for_llm_amd.ops import gemm_bf16 as G
     monkeypatch.setattr(G, "_TIMED_CUTS", {})
-    m, n, k = 2048, 4128, 96
+    m, n, k = 2048, 8208, 96
     ws = [rnd(n, k, scale=0.05, seed=s).to(gpu) for s in range(2)]
     x = rnd(m, k, seed=9).to(gpu)
     want = x.float().cpu() @ ws[1].float().cpu().t()
@@ -360,5 +361,5 @@ def test_a_cut_product_is_timed_both_ways_and_stays_the_same(gpu, monkeypatch):
         with monkeypatch.context() as patch:
             patch.setattr(K, "gemm_vendor", lambda a, w, out, **kw: seen.append(w.shape[0]) or one(a, w, out, **kw))
             got = G.linear_bf16(x, ws[1], torch.full((m, n), 7.0, dtype=torch.bfloat16, device=gpu))
-        assert seen == ([4096, 32] if decided else [4128])
+        assert seen == ([8192, 16] if decided else [8208])
         assert ((got.float().cpu() - want).abs() <= want.abs() * 2.0 ** -8 + 2.0 ** -20 * k).all()

@@ -349,15 +349,18 @@ def test_products_timed_at_start_up_run_the_way_that_was_faster(monkeypatch):
     monkeypatch.setattr(G, "_TIMED_CUTS", {})
     monkeypatch.setattr(G.K, "gemm_vendor_tune", lambda rows, ws, dtype, columns_of=0: calls.append((rows, ws[0].shape[0], columns_of)) or us[ws[0].shape[0]])
     ws, dev = [torch.empty((8208, 64), dtype=torch.bfloat16)] * 2, torch.device("cpu")
+    # the rest begins a turn of the compute units, or does not, or is too much for the small product
+    assert [G.vendor_cut(m, n) for m, n in ((2048, 8208), (1793, 8208), (1792, 8208), (2049, 8208), (4096, 4128), (2048, 4128), (4096, 4129), (2048, 8192))] \
+        == [8192, 8192, 0, 0, 4096, 0, 0, 0]
     assert G.chosen_cut(2048, 8208, 64, dev) == 8192
     us.update({8208: (84.0, 50.0, 9), 8192: (56.0, 48.0, 8), 16: (8.0, 6.0, 7)})
     assert G.tune_linear(2048, ws) == (64.0, 50.0, 24) and calls == [(2048, 8208, 0), (2048, 8192, 8208), (2048, 16, 8208)]
-    assert [G.chosen_cut(m, 8208, 64, dev) for m in (2049, 2048, 1500, 1024, 1023, 1022)] == [8192, 0, 0, 0, 8192, 8192 if 1022 * 8208 >= G.CUT_RESULTS else 0]
+    assert [G.chosen_cut(m, 8208, 64, dev) for m in (4096, 2048, 1793, 1792)] == [8192, 0, 0, 0]
     assert G.chosen_cut(2048, 8208, 32, dev) == G.chosen_cut(2048, 8208, 64, dev, torch.float32) == 8192
     us[8208] = (84.0, 60.0, 9)
-    assert G.tune_linear(1300, ws) == (64.0, 54.0, 24) and G.chosen_cut(1200, 8208, 64, dev) == 8192 and G.chosen_cut(1400, 8208, 64, dev) == 0
+    assert G.tune_linear(1900, ws) == (64.0, 54.0, 24) and G.chosen_cut(1800, 8208, 64, dev) == 8192 and G.chosen_cut(1901, 8208, 64, dev) == 0
     us[16] = (-1.0, -1.0, 0)                # the library has nothing for the rest: one product
-    assert G.tune_linear(3000, ws) == (84.0, 60.0, 17) and G.chosen_cut(3000, 8208, 64, dev) == 0
+    assert G.tune_linear(4096, ws) == (84.0, 60.0, 17) and G.chosen_cut(4096, 8208, 64, dev) == 0
     calls.clear()
     us[8192 + 64] = (5.0, 4.0, 3)
     assert G.tune_linear(2048, [torch.empty((8192 + 64, 64))]) == (5.0, 4.0, 3) and calls == [(2048, 8256, 0)]
