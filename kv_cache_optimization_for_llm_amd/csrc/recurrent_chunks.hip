@@ -11,7 +11,7 @@
 // The u_i are the solution of a unit lower triangular system with right-hand sides beta v and beta D_0 k, so
 //   U = Uv - W S,    O = Qd S + P U,    S <- diag(G) S + Kd^T U
 // with Uv, W, Qd, P, Kd, G of a chunk known without S.  Three kernels: `prepare` makes those, all chunks side by side;
-// `states` hands S on from chunk to chunk, a head's value columns 16 to a workgroup, and leaves the S each chunk
+// `states` hands S on from chunk to chunk, a head's value columns 4, 8 or 16 to a workgroup, and leaves the S each chunk
 // starts from and its U; `outputs` makes O, all chunks side by side again.
 //
 // Inputs, outputs and the state between steps are 32-bit as in the walk.  What the walk does not have is the sums over
@@ -28,11 +28,12 @@
 // last bits of a token's result depend on how the request was cut into steps.  The 32-bit path therefore walks.
 //
 // us a call, the walk -> these three kernels (in 32 bits alone), one prompt of 2,048 / 8,192 tokens:
-//   delta rule, 8 heads of 128 x 128 over 4 key heads:  715 / 2,831 -> 154 / 600 (101 / 373)
+//   delta rule, 8 heads of 128 x 128 over 4 key heads:  715 / 2,831 -> 119 / 447 (in 32 bits and 16 columns a workgroup 101 / 373)
 //   linear attention, 16 heads of 64 x 128:             584 / 2,317 -> 89 / 377 (73 / 334)
 // A 64-bit product takes two to three times the cycles of a 32-bit one.  `states` is a chain: 64 of them a wavefront and
-// chunk and two trips through LDS; with operands row by row instead of in operand order and a head's workgroups spread
-// over the dies it took twice as long.  `prepare` and `outputs` are short of workgroups (256) more than of anything else.
+// chunk and two trips through LDS (102 us of 154 with 16 columns a workgroup; with 4 on the smaller instruction 63: the same
+// number of instructions, each a third as long); with operands row by row instead of in operand order and a head's workgroups
+// spread over the dies it took twice as long.  `prepare` and `outputs` are short of workgroups (256) more than of anything else.
 #include "recurrent.h"
 #include <float.h>
 
@@ -624,6 +625,110 @@ chunk_states_kernel(ChunkArgs a) {
         for (int c = 0; c < 4; ++c) Sg[(size_t)(16 * (wave * MT + t) + ck_channel<DELTA>(g, c)) * a.vdim + col] = (float)S[t][c];
 }
 
+// The delta rule's states with 4 NB value columns to a workgroup instead of 16, for launches that would leave units idle:
+// v_mfma_f64_4x4x4_4b_f64 makes 16 rows of 4 columns (its four blocks are four groups of rows against the same columns), 9.6 ns an
+// instruction where 16 x 16 take 30.4, so a quarter of the columns is a third of a chunk's products.  An operand's rows are held
+// as by the 16 x 16 one; a result is one number a lane: lane (g, b, j) has row 4 b + g of column j.  S^T and U^T stand in
+// LDS with the four rows g + 4 c of (16 rows, column) next to each other, as a lane (g, any b, j) takes them for the next product.
+template <int D, int NB>
+__global__ void __launch_bounds__(256)
+chunk_states_narrow_kernel(ChunkArgs a) {
+    constexpr int STEPS = D / 16, MT = D / 64;
+    __shared__ __attribute__((aligned(32))) double St[NB][D * 4];
+    __shared__ __attribute__((aligned(32))) double Ut[NB][CK * 4];
+    const int e = blockIdx.y, head = blockIdx.x % a.heads, part = blockIdx.x / a.heads;
+    const int q0 = a.entry_q_start[e], n = a.entry_q_start[e + 1] - q0;
+    if (n < a.shortest) return;
+    const int first = __builtin_amdgcn_readfirstlane(rec_first_chunk(a.entry_q_start, e, a.shortest));
+    if (first + (n + CK - 1) / CK > a.chunks || rec_odd_entry(a.odd, first, n, a.heads, head)) return;
+    const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid / KVA_WAVE), lane = tid % KVA_WAVE;
+    const int g = lane / 16, b = lane / 4 % 4, j = lane % 4, chunks = (n + CK - 1) / CK;
+    const int tile = 4 * NB * part / 16, sub = 4 * NB * part % 16 + j;          // of 16 columns; the lane's first one among them
+    float *Sg = a.state + (size_t)a.entry_seat[e] * a.seat_stride + a.state_off + (size_t)head * D * a.vdim + 16 * tile + sub;
+    double S[MT][NB];               // row 16 (wave MT + t) + 4 b + g of the columns
+#pragma unroll
+    for (int t = 0; t < MT; ++t)
+#pragma unroll
+        for (int c = 0; c < NB; ++c) S[t][c] = Sg[(size_t)(16 * (wave * MT + t) + 4 * b + g) * a.vdim + 4 * c];
+    struct Operands {
+        ck_f32x4 w[STEPS], kt[MT][CK / 16];
+        float dec[MT];
+        double uv[NB];
+    } o[2];
+    // (in operand order the lane's element of 16 rows and its column)
+    auto at = [&](int s, int steps, int c) { return ck_frag(tile, s, steps, sub + 4 * c + 16 * g) + b; };
+    auto fetch = [&](Operands &x, int chunk) {
+        const ChunkBlock<D> k(a, first + min(chunk, chunks - 1), head);
+#pragma unroll
+        for (int c = 0; c < NB; ++c) x.uv[c] = reinterpret_cast<const double *>(k.ut)[at(wave, 4, c)];
+#pragma unroll
+        for (int s = 0; s < STEPS; ++s) x.w[s] = ck_ld(k.w + ck_frag(wave, s, STEPS, lane));
+#pragma unroll
+        for (int t = 0; t < MT; ++t) {
+#pragma unroll
+            for (int s = 0; s < CK / 16; ++s) x.kt[t][s] = ck_ld(k.kt + ck_frag(wave * MT + t, s, 4, lane));
+            x.dec[t] = k.g[16 * (wave * MT + t) + 4 * g + b];
+        }
+    };
+    auto step = [&](const Operands &x, Operands &next, int chunk) {
+        const ChunkBlock<D> k(a, first + chunk, head);
+#pragma unroll
+        for (int t = 0; t < MT; ++t)
+#pragma unroll
+            for (int c = 0; c < NB; ++c) {
+                St[c][((wave * MT + t) * 16 + 4 * g + j) * 4 + b] = S[t][c];
+                k.st[at(wave * MT + t, STEPS, c)] = (float)S[t][c];
+            }
+        __syncthreads();
+        fetch(next, chunk + 1);
+        double y[NB][4];            // chains of products: one alone waits for its own results
+#pragma unroll
+        for (int c = 0; c < NB; ++c)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) y[c][i] = 0.0;
+#pragma unroll
+        for (int s = 0; s < STEPS; ++s)
+#pragma unroll
+            for (int c = 0; c < NB; ++c) {
+                const ck_f64x4 z = ck_ld(&St[c][(16 * s + 4 * g + j) * 4]);
+#pragma unroll
+                for (int i = 0; i < 4; ++i) y[c][i] = __builtin_amdgcn_mfma_f64_4x4x4f64((double)x.w[s][i], z[i], y[c][i], 0, 0, 0);
+            }
+#pragma unroll
+        for (int c = 0; c < NB; ++c) {
+            const double u = x.uv[c] - ((y[c][0] + y[c][1]) + (y[c][2] + y[c][3]));
+            reinterpret_cast<double *>(k.ut)[at(wave, 4, c)] = u;
+            Ut[c][(16 * wave + 4 * g + j) * 4 + b] = u;
+        }
+        __syncthreads();
+#pragma unroll
+        for (int t = 0; t < MT; ++t)
+#pragma unroll
+            for (int c = 0; c < NB; ++c) {
+                double lo = S[t][c] * x.dec[t], hi = 0.0;
+#pragma unroll
+                for (int s = 0; s < CK / 16; ++s) {
+                    const ck_f64x4 z = ck_ld(&Ut[c][(16 * s + 4 * g + j) * 4]);
+#pragma unroll
+                    for (int i = 0; i < 4; i += 2) {
+                        lo = __builtin_amdgcn_mfma_f64_4x4x4f64((double)x.kt[t][s][i], z[i], lo, 0, 0, 0);
+                        hi = __builtin_amdgcn_mfma_f64_4x4x4f64((double)x.kt[t][s][i + 1], z[i + 1], hi, 0, 0, 0);
+                    }
+                }
+                S[t][c] = lo + hi;
+            }
+    };
+    fetch(o[0], 0);
+    for (int chunk = 0; chunk < chunks; chunk += 2) {
+        step(o[0], o[1], chunk);
+        if (chunk + 1 < chunks) step(o[1], o[0], chunk + 1);
+    }
+#pragma unroll
+    for (int t = 0; t < MT; ++t)
+#pragma unroll
+        for (int c = 0; c < NB; ++c) Sg[(size_t)(16 * (wave * MT + t) + 4 * b + g) * a.vdim + 4 * c] = (float)S[t][c];
+}
+
 // One workgroup a (chunk, head), a wavefront every fourth 32 value columns, for all 64 tokens: O = Qd S + P U, every
 // operand from where the other two kernels left it, in operand order.
 template <int D, bool DELTA>
@@ -694,7 +799,14 @@ static void ck_launch(const ChunkArgs &a, const ChunkInput &in, hipStream_t stre
     const dim3 grid(a.chunks, a.heads);
     if (in.channel_decay) hipLaunchKernelGGL((chunk_prepare_kernel<D, DELTA, true>), grid, dim3(256), 0, stream, a, in);
     else hipLaunchKernelGGL((chunk_prepare_kernel<D, DELTA, false>), grid, dim3(256), 0, stream, a, in);
-    hipLaunchKernelGGL((chunk_states_kernel<D, DELTA>), dim3(a.heads * (a.vdim / 16), a.entries), dim3(256), 0, stream, a);
+    // A chain's length is its chunks whatever the workgroups hold, so the columns go to as many as a turn of the 256 units takes.
+    // All three kernels at 4 / 8 / 16 columns a workgroup, heads of 128 x 128, us: 64 workgroups of 16 columns (8 heads, 2,048 tokens)
+    // 121 / 139 / 160, 128 (16 heads) 194 / 182 / 199, 256 (32 heads) 400 / 383 / 333; of 64 x 64: 16 (4 heads, 2,048) 72 / 79 / 93,
+    // 128 (32 heads, 1,024) 98 / 95 / 101.
+    const int tiles = a.heads * (a.vdim / 16), entries = min(a.entries, a.chunks);
+    if (DELTA && (long long)tiles * entries <= 64) hipLaunchKernelGGL((chunk_states_narrow_kernel<D, 1>), dim3(tiles * 4, a.entries), dim3(256), 0, stream, a);
+    else if (DELTA && (long long)tiles * entries <= 128) hipLaunchKernelGGL((chunk_states_narrow_kernel<D, 2>), dim3(tiles * 2, a.entries), dim3(256), 0, stream, a);
+    else hipLaunchKernelGGL((chunk_states_kernel<D, DELTA>), dim3(tiles, a.entries), dim3(256), 0, stream, a);
     hipLaunchKernelGGL((chunk_outputs_kernel<D, DELTA>), grid, dim3(256), 0, stream, a);
 }
 

@@ -268,6 +268,32 @@ def test_gated_delta_rule_in_chunks(heads, kv_heads, dim, vdim, decays, portions
     assert (states[True][:, :4] == 0).all()
 
 
+@pytest.mark.parametrize("dim", [64, 128])
+def test_delta_rule_chunks_with_few_and_many_columns_a_workgroup(dim, gpu):
+    """Heads with the same inputs, so few (2), some (12) and many (18) of them that a workgroup takes 4, 8 and 16 value columns.
+    Sums are formed in 64 bits in every form and rounded once to 32 (2^-24 of a value): a few such roundings apart."""
+    vdim, lens = 128, [130, 321]
+    g = torch.Generator().manual_seed(dim)
+    n = sum(lens)
+    q, k, v = (torch.randn(n, d, generator=g) for d in (dim, dim, vdim))
+    b = (torch.randn(n, 1, generator=g) * 2).to(torch.bfloat16)
+    got = {}
+    for heads in (2, 12, 18):
+        rows = torch.cat([q, k] + [v] * heads, dim=1)
+        state = torch.full((len(lens), heads * dim * vdim), 0.25, dtype=torch.float32, device="cuda")
+        out = torch.empty((n, heads * vdim), dtype=torch.float32, device="cuda")
+        for part in range(len(lens)):       # one entry a call: heads x 8 tiles of 16 columns
+            at = slice(sum(lens[:part]), sum(lens[:part + 1]))
+            K.gated_delta_rule(dev(rows[at]), b[at].repeat(1, heads).to("cuda"), 0, 0, dev(torch.full((heads,), -1.0)), dev(torch.zeros(heads)),
+                               out[at], state, 0, ints([0, lens[part]]), ints([part]), heads, 1, dim, vdim, lengths=[lens[part]])
+        got[heads] = (out.cpu().view(n, heads, vdim), state.cpu().view(len(lens), heads, dim, vdim))
+    want = [x.to(F) for x in got[18]]
+    for heads, pair in got.items():
+        for x, w in zip(pair, want):
+            w = w[:, :1].expand(x.shape)
+            assert rms(x.to(F) - w) <= 2.0 ** -22 * rms(w), heads
+
+
 def test_gated_delta_rule_rows_at_any_address_walk(gpu):
     """Rows that do not start at a multiple of 16 bytes are not read by the chunks."""
     heads, dim, vdim, n = 2, 64, 16, 200
