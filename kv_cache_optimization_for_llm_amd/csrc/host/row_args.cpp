@@ -67,22 +67,16 @@ bool truth(PyObject *row, PyObject *name, bool *out) {
 
 } // namespace
 
-// Returns bit 0: a row has a temperature (asked for with READ_SAMPLED), bit 1: a row asks for the penalty (READ_PENALTY); -1: an
-// exception is set.  With `staging` ([5][stride], n <= stride) its rows get, with READ_SAMPLED, 1 / temperature (0: greedy) in fp32
-// and the low 32 bits of key and step, with READ_SEATS the seat and, with READ_PENALTY too, the seat of rows that ask for the penalty
-// (else -1).  Nothing else of a row is looked at.
-enum { READ_SAMPLED = 1, READ_PENALTY = 2, READ_SEATS = 4 };
+enum { READ_SAMPLED = 1, READ_PENALTY = 2, READ_SEATS = 4, READ_AS_USED = 8, READ_KEYS = 16 };
 
-extern "C" int kva_sample_rows(PyObject *rows, long long n, int32_t *staging, long long stride, int want) {
+// One pass over the rows: READ_KEYS the keys and steps alone, whatever else is asked for as below.
+static int read_rows(PyObject *list, long long n, int32_t *staging, long long stride, int want) {
     static const Names names;
-    PyObject *list = PySequence_Fast(rows, "the rows of a sampling are a sequence");
-    if (!list) return -1;
     int flags = 0;
     for (long long i = 0; i < n && flags >= 0; ++i) {
         if (i >= PySequence_Fast_GET_SIZE(list)) {
             PyErr_SetString(PyExc_ValueError, "fewer rows than logits");
-            flags = -1;
-            break;
+            return -1;
         }
         PyObject *row = PySequence_Fast_GET_ITEM(list, i);
         Py_INCREF(row);
@@ -92,9 +86,11 @@ extern "C" int kva_sample_rows(PyObject *rows, long long n, int32_t *staging, lo
         if (ok && want & READ_PENALTY) ok = truth(row, names.apply_penalty, &penalty);
         if (ok && staging && want & READ_SAMPLED) {
             const float inverse = temperature > 0.0 ? (float)(1.0 / temperature) : 0.f;
+            __builtin_memcpy(&staging[i], &inverse, sizeof inverse);
+        }
+        if (ok && staging && want & READ_KEYS) {
             uint32_t key = 0, step = 0;
             ok = low_bits(row, names.rng_key, &key) && low_bits(row, names.rng_step, &step);
-            __builtin_memcpy(&staging[i], &inverse, sizeof inverse);
             staging[stride + i] = (int32_t)key;
             staging[2 * stride + i] = (int32_t)step;
         }
@@ -106,6 +102,25 @@ extern "C" int kva_sample_rows(PyObject *rows, long long n, int32_t *staging, lo
         }
         Py_DECREF(row);
         flags = ok ? flags | (temperature > 0.0 ? 1 : 0) | (penalty ? 2 : 0) : -1;
+    }
+    return flags;
+}
+
+// Returns bit 0: a row has a temperature (asked for with READ_SAMPLED), bit 1: a row asks for the penalty (READ_PENALTY); -1: an
+// exception is set.  With `staging` ([5][stride], n <= stride) its rows get, with READ_SAMPLED, 1 / temperature (0: greedy) in fp32
+// and the low 32 bits of key and step, with READ_SEATS the seat and, with READ_PENALTY too, the seat of rows that ask for the penalty
+// (else -1).  Nothing else of a row is looked at.  READ_AS_USED, with `staging`: keys and steps only where a row has a temperature,
+// the penalty's seats only where a row asks for it.
+extern "C" int kva_sample_rows(PyObject *rows, long long n, int32_t *staging, long long stride, int want) {
+    PyObject *list = PySequence_Fast(rows, "the rows of a sampling are a sequence");
+    if (!list) return -1;
+    int flags;
+    if (want & READ_AS_USED && staging) {
+        flags = read_rows(list, n, staging, stride, want & (READ_SAMPLED | READ_PENALTY));
+        const int rest = (flags & 1 ? READ_KEYS : 0) | (want & READ_SEATS ? READ_SEATS | (flags & 2 ? READ_PENALTY : 0) : 0);
+        if (flags >= 0 && rest && read_rows(list, n, staging, stride, rest) < 0) flags = -1;
+    } else {
+        flags = read_rows(list, n, staging, stride, want | (want & READ_SAMPLED ? READ_KEYS : 0));
     }
     Py_DECREF(list);
     return flags;

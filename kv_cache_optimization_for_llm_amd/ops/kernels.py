@@ -1121,6 +1121,63 @@ def sample(logits: torch.Tensor, out_tokens: torch.Tensor, *, chunks: int = 128,
     return out_tokens
 
 
+class StreamEvent:
+    """An event that native code can record behind its launches; waiting for it does not hold the interpreter's lock."""
+
+    def __init__(self):
+        handle = ctypes.c_void_p()
+        self.handle, self._lib = None, hip_lib()
+        check(self._lib.kva_event_create(ctypes.byref(handle)), "event")
+        self.handle = handle.value
+
+    def record(self) -> None:
+        check(self._lib.kva_event_record(self.handle, _stream()), "event")
+
+    def synchronize(self) -> None:
+        check(self._lib.kva_event_synchronize(self.handle), "event")
+
+    def __del__(self):
+        if self.handle is not None:
+            self._lib.kva_event_destroy(self.handle)
+
+
+_SAMPLE_BY_VALUE = None
+
+
+def sample_rows_by_value() -> int:
+    """Most rows of :func:`sample_by_value`."""
+    global _SAMPLE_BY_VALUE
+    if _SAMPLE_BY_VALUE is None:
+        _SAMPLE_BY_VALUE = int(hip_lib().kva_sample_rows_by_value())
+    return _SAMPLE_BY_VALUE
+
+
+def sample_by_value(logits: torch.Tensor, out_tokens: torch.Tensor, row_args: int, stride: int, *, chunks: int = 128,
+                    any_sampled: bool = False, seed: int = 0, penalty_mask: Optional[torch.Tensor] = None, penalty: float = 1.0,
+                    mark_mask: Optional[torch.Tensor] = None, host_tokens: Optional[torch.Tensor] = None,
+                    behind: Optional[StreamEvent] = None) -> torch.Tensor:
+    """:func:`sample` for up to :func:`sample_rows_by_value` rows whose arguments are on the host: ``row_args`` is the address
+    of int32 ``[5, stride]`` with 1 / temperature (as fp32), key, step, seat of the penalty (-1: none) and seat to mark
+    (-1: none), and may be written again as soon as this returns.  Arrays of an option that is not used are not read.
+    ``behind`` is recorded behind the kernels (not without rows)."""
+    rows, vocab = logits.shape
+    if out_tokens.shape != (rows,) or not 0 <= rows <= min(stride, sample_rows_by_value()):
+        raise KernelError(f"sample: one output token and one set of arguments per row, up to {sample_rows_by_value()}")
+    for mask in (penalty_mask, mark_mask):
+        if mask is not None and (mask.dim() != 2 or mask.shape[1] != vocab):
+            raise KernelError("sample: masks are [seats, vocab]")
+    if host_tokens is not None and (host_tokens.is_cuda or host_tokens.dtype != torch.int32 or host_tokens.dim() != 1
+                                    or host_tokens.shape[0] < rows or not host_tokens.is_contiguous()):
+        raise KernelError("sample: host_tokens must be a pinned host int32 vector with a place per row")
+    ws = torch.empty(4 * max(1, rows * chunks), dtype=torch.float32, device=logits.device)     # (a record is 16 bytes)
+    check(hip_lib().kva_sample_by_value(
+        _dev(out_tokens, "out_tokens", torch.int32), _dev(logits, "logits", torch.float32), rows, vocab, chunks,
+        _opt(penalty_mask, "penalty_mask", torch.uint8), float(penalty), row_args, stride, int(seed) & 0xFFFFFFFF,
+        1 if any_sampled else 0, ws.data_ptr(), _opt(mark_mask, "mark_mask", torch.uint8),
+        host_tokens.data_ptr() if host_tokens is not None else None, behind.handle if behind is not None else None, _stream()), "sample")
+    return out_tokens
+
+
 def mark_tokens(mask: torch.Tensor, seats: torch.Tensor, tokens: torch.Tensor) -> None:
     n = seats.shape[0]
     if tokens.shape != (n,) or mask.dim() != 2:

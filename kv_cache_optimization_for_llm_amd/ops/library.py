@@ -91,6 +91,12 @@ _HIP_SIGNATURES = {
     "kva_gemm_vendor_forget": [I, I, I, I, I, I],
     "kva_host_memory_is_mapped": [P],
     "kva_sample": [P, P, I, I, I, P, P, F, P, U, P, P, I, P, P, P, P, P],
+    "kva_sample_rows_by_value": [],
+    "kva_sample_by_value": [P, P, I, I, I, P, F, P, I, U, I, P, P, P, P, P],
+    "kva_event_create": [POINTER(P)],
+    "kva_event_record": [P, P],
+    "kva_event_synchronize": [P],
+    "kva_event_destroy": [P],
     "kva_mark_tokens": [P, P, P, I, I, P],
     "kva_causal_conv_act": [P, I, I, P, I, I, I, P, I, P, LL, I, P, P, I, I, I, I, P, P, I, P],
     "kva_latent_prompt": [P, P, I, I, P, P, P, P, P, I, P, P, P, I, P, P, I, P, P, I, I, I, I, I, I, I, I, F, P],

@@ -48,12 +48,14 @@ class SampleRow:
 
 
 class _Staging:
-    """Per-row arguments on their way up: pinned memory, seen as int32, uint32 and float32 ``[5, rows]``."""
+    """Per-row arguments, seen as int32, uint32 and float32 ``[5, rows]``: on their way up in pinned memory, or (``pin`` off) as
+    the launches take them."""
 
-    def __init__(self, rows: int):
-        self.pinned = torch.zeros((5, rows), dtype=torch.int32, pin_memory=True)
+    def __init__(self, rows: int, pin: bool = True):
+        self.pinned = torch.zeros((5, rows), dtype=torch.int32, pin_memory=pin)
         self.i32 = self.pinned.numpy()
         self.u32, self.f32 = self.i32.view(np.uint32), self.i32.view(np.float32)
+        self.address = self.pinned.data_ptr()
         self.sent = None                    # an event behind the copy
 
 
@@ -81,11 +83,26 @@ def _read_rows(rows: Sequence[SampleRow], n: int, staging: Optional[_Staging], s
     return (1 if sampled and any(r.temperature > 0 for r in rows) else 0) | (2 if penalty and any(r.apply_penalty for r in rows) else 0)
 
 
+def _read_rows_as_used(rows: Sequence[SampleRow], n: int, staging: _Staging, mask: bool) -> int:
+    """What a sampling of these rows uses of them, in ``staging``, and :func:`_read_rows`'s bits: their temperatures, keys and steps
+    where one is above 0, with ``mask`` their seats and, where one asks for it, the seats of the penalty."""
+    native = sample_rows()
+    if native is not None:
+        try:
+            return native(rows, n, staging.address, staging.i32.shape[1], 8 | (7 if mask else 1))
+        except Exception:
+            pass
+    flags = _read_rows(rows, n, None, False, penalty=mask)
+    if flags & 1 or mask:
+        _read_rows(rows, n, staging, mask, sampled=bool(flags & 1), penalty=bool(flags & 2))
+    return flags
+
+
 class PendingTokens:
     """Sampled tokens on their way to the host: the kernel that chooses them writes them into
     pinned memory as well, and :meth:`wait` blocks until the stream has passed it."""
 
-    def __init__(self, host: torch.Tensor, event: "torch.cuda.Event", n: int):
+    def __init__(self, host: torch.Tensor, event: "K.StreamEvent", n: int):
         self._host, self._event, self._n = host, event, n
         self._value: Optional[np.ndarray] = None
 
@@ -113,9 +130,12 @@ class Sampler:
             self.mask = torch.zeros((max_seqs, vocab_size), dtype=torch.uint8, device=device)
         # pinned landing buffers for sample_async, used in turn (two samplings may be in flight)
         self._landing: List[torch.Tensor] = []
+        self._events: list = []             # one a landing buffer, recorded behind the sampling that fills it
         self._kernel_writes_host = False
         self._landing_next = 0
-        # per-row arguments of a sampling (temperatures, random-stream keys and steps, seats)
+        # per-row arguments of a sampling (temperatures, random-stream keys and steps, seats): of a few rows they travel with
+        # the launches, of more they go up in a copy
+        self._args_few: Optional[_Staging] = None
         self._args_dev: Optional[torch.Tensor] = None
         self._args_host: List[_Staging] = []
         self._args_views: dict = {}
@@ -125,7 +145,7 @@ class Sampler:
         """(a staging array to fill, the device arrays its rows go to) for the next sampling of n rows.  Slices and views are
         made once per number of rows: they cost more than what is done with them."""
         if self._args_dev is None or self._args_dev.shape[1] < n:
-            cap = max(64, 1 << (n - 1).bit_length())
+            cap = 1 << (n - 1).bit_length()
             self._args_dev = torch.zeros((5, cap), dtype=torch.int32, device=self.device)
             self._args_host = [_Staging(cap) for _ in range(3)]
             self._args_views.clear()
@@ -174,18 +194,33 @@ class Sampler:
             out = torch.empty(max(n, 1), dtype=torch.int32, device=self.device)
         if out.dtype != torch.int32 or out.dim() != 1 or out.shape[0] < n:
             raise ValueError("sample: out must be a device int32 vector with a place per row")
-        out = out[:n]
+        if out.shape[0] != n:
+            out = out[:n]
         if len(self._landing) < 3 or self._landing[0].shape[0] < n:
             size = max(64, n)
             self._landing = [torch.zeros(size, dtype=torch.int32, pin_memory=True) for _ in range(3)]
+            self._events = [K.StreamEvent() for _ in range(3)]
             # where the runtime does not map pinned memory for the device, a copy follows the kernels instead
             self._kernel_writes_host = self.KERNEL_WRITES_HOST and all(K.host_memory_is_mapped(t) for t in self._landing)
-        host = self._landing[self._landing_next]
+        host, event = self._landing[self._landing_next], self._events[self._landing_next]
         self._landing_next = (self._landing_next + 1) % len(self._landing)
-        event = torch.cuda.Event()
         if n == 0:
             event.record()
             return PendingTokens(host, event, 0)
+        landing = host if self._kernel_writes_host else None
+        if n <= K.sample_rows_by_value():
+            args = self._args_few
+            if args is None:
+                args = self._args_few = _Staging(K.sample_rows_by_value(), pin=False)
+            flags = _read_rows_as_used(rows, n, args, self.mask is not None)
+            # every token a request emits is marked in its mask row, by the launch that chooses it
+            K.sample_by_value(logits, out, args.address, args.i32.shape[1], chunks=self.chunks, any_sampled=bool(flags & 1), seed=self.seed,
+                              penalty_mask=self.mask if flags & 2 else None, penalty=self.penalty, mark_mask=self.mask,
+                              host_tokens=landing, behind=event)
+            if landing is None:
+                host[:n].copy_(out, non_blocking=True)
+                event.record()
+            return PendingTokens(host, event, n)
         flags = _read_rows(rows, n, None, False, penalty=self.mask is not None)
         any_sampled, use_mask = bool(flags & 1), bool(flags & 2)
         inv_t = key = step = seat_t = mark_seat = None
@@ -199,18 +234,18 @@ class Sampler:
             if use_mask:
                 seat_t = dev_seat
             if self.mask is not None:
-                # every token a request emits is marked in its mask row, by the launch that chooses it
                 mark_seat = dev_mark
             # (torch's own copy: its allocator then knows that the block is in use until the copy has left it, also when this
             # sampler goes away or takes larger ones before)
-            staging.sent = event
+            staging.sent = torch.cuda.Event()
             self._args_dev.copy_(staging.pinned, non_blocking=True)
+            staging.sent.record()
         try:
             K.sample(logits, out, chunks=self.chunks, inv_temperature=inv_t, seed=self.seed, rng_key=key,
                      rng_step=step, penalty_mask=self.mask if use_mask else None, row_seat=seat_t,
                      penalty=self.penalty, mark_mask=self.mask if mark_seat is not None else None,
-                     mark_seat=mark_seat, host_tokens=host if self._kernel_writes_host else None)
-            if not self._kernel_writes_host:
+                     mark_seat=mark_seat, host_tokens=landing)
+            if landing is None:
                 host[:n].copy_(out, non_blocking=True)
         finally:
             event.record()

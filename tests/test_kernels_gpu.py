@@ -1007,6 +1007,38 @@ def test_row_arguments_stay_until_their_copy_has_left_them(how, gpu):
     del others
 
 
+@pytest.mark.parametrize("penalty", [1.0, 1.3])
+def test_rows_with_the_launch_and_rows_in_a_copy(penalty, gpu):
+    """As many rows as a launch's arguments take, one more, and all of them behind a long step: every row draws what it draws
+    alone, and with a penalty leaves the same mask."""
+    from kv_cache_optimization_for_llm_amd.sampling.sampler import Sampler, SampleRow
+    vocab, most = 2500, K.sample_rows_by_value()
+    rows = 3 * most
+    lg = (torch.randn(rows, vocab, generator=torch.Generator().manual_seed(4)) * 2).to(gpu)
+    which = [SampleRow(r, (0.0, 0.9, 0.7)[r % 3], rng_key=8 * r, rng_step=9, apply_penalty=r % 2 == 0) for r in range(rows)]
+
+    def fresh():
+        s = Sampler(vocab, rows, gpu, seed=5, repetition_penalty=penalty)
+        s.mark(list(range(rows)), lg.argmax(1).tolist())
+        return s
+    one = fresh()
+    want = [int(one.sample(lg[r:r + 1], which[r:r + 1])[0]) for r in range(rows)]
+    busy = torch.randn(4096, 4096, device=gpu)
+    for n in (most, most + 1, rows):
+        sampler, part = fresh(), lg[:n].contiguous()
+        torch.cuda.synchronize()
+        for _ in range(50):
+            busy = busy @ busy * 1e-3
+        pending = sampler.sample_async(part, which[:n])
+        if penalty == 1.0:                  # (a mask's marks would change the second one's draws)
+            others = [sampler.sample_async(part, which[:n]) for _ in range(2)]
+            assert all(o.wait().tolist() == want[:n] for o in others), n
+        else:
+            torch.cuda.synchronize()
+            assert torch.equal(sampler.mask[:n], one.mask[:n])
+        assert pending.wait().tolist() == want[:n], n
+
+
 def test_sampler_takes_keys_and_steps_of_any_integer_type(gpu):
     from kv_cache_optimization_for_llm_amd.sampling.sampler import Sampler, SampleRow
     lg = torch.randn(1, 4000, generator=torch.Generator().manual_seed(1)).to(gpu)

@@ -34,6 +34,19 @@ def test_native_reader_against_the_comprehensions(rows, room, seats, monkeypatch
     assert np.array_equal(got.i32, want.i32)
 
 
+@pytest.mark.parametrize("rows", [ROWS, ROWS[:1] * 3, [r for r in ROWS if not r.apply_penalty], []])
+@pytest.mark.parametrize("mask", [False, True])
+def test_what_is_used_in_one_call(rows, mask, monkeypatch):
+    got, want = S._Staging(8, pin=False), S._Staging(8, pin=False)
+    with np.errstate(over="ignore"):
+        flags = S._read_rows_as_used(rows, len(rows), got, mask)
+        monkeypatch.setattr(S, "sample_rows", lambda: None)
+        assert flags == S._read_rows_as_used(rows, len(rows), want, mask)
+    if not flags & 1:                       # (no temperature: nothing of the first array is used)
+        want.i32[0] = got.i32[0]
+    assert np.array_equal(got.i32, want.i32)
+
+
 def test_what_the_comprehensions_raise_is_raised():
     with pytest.raises(AttributeError):
         S._read_rows([types.SimpleNamespace(temperature=0.5)], 1, staging(1), False)
