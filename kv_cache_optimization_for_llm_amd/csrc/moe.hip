@@ -1288,9 +1288,9 @@ small_product_f32_kernel(float *__restrict__ out, const void *__restrict__ x, in
                 float f[8];
                 moe_ld8(w, w_dtype, (size_t)n * K + k, f);
 #pragma unroll
-                for (int i = 0; i < 8; ++i) acc += xs[k + i] * f[i];
+                for (int i = 0; i < 8; ++i) acc = __builtin_fmaf(xs[k + i], f[i], acc);
             }
-            for (int k = K8; k < K; ++k) acc += xs[k] * moe_ld(w, w_dtype, (size_t)n * K + k);
+            for (int k = K8; k < K; ++k) acc = __builtin_fmaf(xs[k], moe_ld(w, w_dtype, (size_t)n * K + k), acc);
             out[t * N + n] = small_product_finish(acc, bias, n, decay_inv_tau, rate_log, rate_group);
         }
     }

@@ -140,7 +140,7 @@ causal_conv_act_kernel(ConvArgs a) {
 #pragma unroll
                 for (int j = 0; j < TAPS; ++j) {
                     const int src = i - (TAPS - 1) + j;
-                    acc[v] += w[j][v] * (src >= 0 ? in[src >= 0 ? src : 0][v] : old[src < 0 ? TAPS - 1 + src : 0][v]);
+                    acc[v] = rec_fma(w[j][v], src >= 0 ? in[src >= 0 ? src : 0][v] : old[src < 0 ? TAPS - 1 + src : 0][v], acc[v]);
                 }
             }
             conv_store<VEC>(a, (size_t)(q0 + first + i), c, acc);
@@ -499,8 +499,8 @@ gated_delta_rule_reg_kernel(RecArgs a, const float *__restrict__ qkv, int conv_s
             float sq = 0.f, sk = 0.f;
             if (tt < m)
                 for (int i = part; i < DP; i += 4) {
-                    sq += qs[tt * DS + i] * qs[tt * DS + i];
-                    sk += ks[tt * DS + i] * ks[tt * DS + i];
+                    sq = rec_fma(qs[tt * DS + i], qs[tt * DS + i], sq);
+                    sk = rec_fma(ks[tt * DS + i], ks[tt * DS + i], sk);
                 }
             sq += __shfl_xor(sq, 1, KVA_WAVE); sq += __shfl_xor(sq, 2, KVA_WAVE);
             sk += __shfl_xor(sk, 1, KVA_WAVE); sk += __shfl_xor(sk, 2, KVA_WAVE);
@@ -540,39 +540,39 @@ gated_delta_rule_reg_kernel(RecArgs a, const float *__restrict__ qkv, int conv_s
                     Sd[4 * j + 1] = al.y * S[4 * j + 1];
                     Sd[4 * j + 2] = al.z * S[4 * j + 2];
                     Sd[4 * j + 3] = al.w * S[4 * j + 3];
-                    d0 += Sd[4 * j] * kk[j].x;
-                    d1 += Sd[4 * j + 1] * kk[j].y;
-                    d2 += Sd[4 * j + 2] * kk[j].z;
-                    d3 += Sd[4 * j + 3] * kk[j].w;
+                    d0 = rec_fma(Sd[4 * j], kk[j].x, d0);
+                    d1 = rec_fma(Sd[4 * j + 1], kk[j].y, d1);
+                    d2 = rec_fma(Sd[4 * j + 2], kk[j].z, d2);
+                    d3 = rec_fma(Sd[4 * j + 3], kk[j].w, d3);
                 } else {
-                    d0 += S[4 * j] * kk[j].x;
-                    d1 += S[4 * j + 1] * kk[j].y;
-                    d2 += S[4 * j + 2] * kk[j].z;
-                    d3 += S[4 * j + 3] * kk[j].w;
+                    d0 = rec_fma(S[4 * j], kk[j].x, d0);
+                    d1 = rec_fma(S[4 * j + 1], kk[j].y, d1);
+                    d2 = rec_fma(S[4 * j + 2], kk[j].z, d2);
+                    d3 = rec_fma(S[4 * j + 3], kk[j].w, d3);
                 }
-                p0 += S[4 * j] * qp[j].x;
-                p1 += S[4 * j + 1] * qp[j].y;
-                p2 += S[4 * j + 2] * qp[j].z;
-                p3 += S[4 * j + 3] * qp[j].w;
+                p0 = rec_fma(S[4 * j], qp[j].x, p0);
+                p1 = rec_fma(S[4 * j + 1], qp[j].y, p1);
+                p2 = rec_fma(S[4 * j + 2], qp[j].z, p2);
+                p3 = rec_fma(S[4 * j + 3], qp[j].w, p3);
             }
             d0 += d1; p0 += p1; d2 += d3; p2 += p3;
             float both[2] = {d0 + d2, p0 + p2};
             row16_sum_each<2>(both);
             if (tt > 0 && r == 0) os[(tt - 1) * REG_BLOCK_COLS + wave * REG_COLS + c] = both[1] * mqp;
             if (last) break;
-            const float u = beta * (v - g * both[0]);
+            const float u = beta * rec_fma(-g, both[0], v);
 #pragma unroll
             for (int j = 0; j < RP / 4; ++j) {
                 if constexpr (CD) {
-                    S[4 * j] = Sd[4 * j] + kk[j].x * u;
-                    S[4 * j + 1] = Sd[4 * j + 1] + kk[j].y * u;
-                    S[4 * j + 2] = Sd[4 * j + 2] + kk[j].z * u;
-                    S[4 * j + 3] = Sd[4 * j + 3] + kk[j].w * u;
+                    S[4 * j] = rec_fma(kk[j].x, u, Sd[4 * j]);
+                    S[4 * j + 1] = rec_fma(kk[j].y, u, Sd[4 * j + 1]);
+                    S[4 * j + 2] = rec_fma(kk[j].z, u, Sd[4 * j + 2]);
+                    S[4 * j + 3] = rec_fma(kk[j].w, u, Sd[4 * j + 3]);
                 } else {
-                    S[4 * j] = g * S[4 * j] + kk[j].x * u;
-                    S[4 * j + 1] = g * S[4 * j + 1] + kk[j].y * u;
-                    S[4 * j + 2] = g * S[4 * j + 2] + kk[j].z * u;
-                    S[4 * j + 3] = g * S[4 * j + 3] + kk[j].w * u;
+                    S[4 * j] = rec_fma(kk[j].x, u, g * S[4 * j]);
+                    S[4 * j + 1] = rec_fma(kk[j].y, u, g * S[4 * j + 1]);
+                    S[4 * j + 2] = rec_fma(kk[j].z, u, g * S[4 * j + 2]);
+                    S[4 * j + 3] = rec_fma(kk[j].w, u, g * S[4 * j + 3]);
                 }
                 qp[j] = qq[j];
             }
@@ -671,14 +671,14 @@ gated_linear_attention_reg_kernel(RecArgs a, const void *__restrict__ y, int y_d
 #pragma unroll
             for (int j = 0; j < RP / 4; ++j) {
                 const float4 kk = k4[REG_LANES * j], qq = q4[REG_LANES * j], al = a4[REG_LANES * j];
-                S[4 * j] = al.x * S[4 * j] + kk.x * v;
-                S[4 * j + 1] = al.y * S[4 * j + 1] + kk.y * v;
-                S[4 * j + 2] = al.z * S[4 * j + 2] + kk.z * v;
-                S[4 * j + 3] = al.w * S[4 * j + 3] + kk.w * v;
-                o[0] += S[4 * j] * qq.x;
-                o[1] += S[4 * j + 1] * qq.y;
-                o[2] += S[4 * j + 2] * qq.z;
-                o[3] += S[4 * j + 3] * qq.w;
+                S[4 * j] = rec_fma(kk.x, v, al.x * S[4 * j]);
+                S[4 * j + 1] = rec_fma(kk.y, v, al.y * S[4 * j + 1]);
+                S[4 * j + 2] = rec_fma(kk.z, v, al.z * S[4 * j + 2]);
+                S[4 * j + 3] = rec_fma(kk.w, v, al.w * S[4 * j + 3]);
+                o[0] = rec_fma(S[4 * j], qq.x, o[0]);
+                o[1] = rec_fma(S[4 * j + 1], qq.y, o[1]);
+                o[2] = rec_fma(S[4 * j + 2], qq.z, o[2]);
+                o[3] = rec_fma(S[4 * j + 3], qq.w, o[3]);
             }
         };
         int tt = 0;
@@ -819,16 +819,6 @@ extern "C" int kva_gated_linear_attention(float *out, float *state, long long se
 // out[t, out_off + h dv + j] = (x[t, h, j] / sqrt(mean_j x^2 + eps) * w[j], or x as it is without a
 // weight) * act(gate[t, gate_off + h dv + j]) * mul;  act: 0 silu, 1 sigmoid.  One wavefront a head.
 // gate_first: the gate multiplies what is normed, n(x * act(gate)), instead of the norm's result.
-struct HeadGate {
-    const void *p;
-    int dtype, stride, off, act, first;
-    __device__ float at(size_t t, int i) const {
-        if (!p) return 1.f;
-        const float g = rec_ld(p, dtype, t * stride + off + i);
-        return act == 1 ? rec_sigmoid(g) : rec_silu(g);
-    }
-};
-
 __global__ void __launch_bounds__(256)
 head_norm_gate_kernel(void *__restrict__ out, int out_dtype, int out_stride, int out_off, const void *__restrict__ x,
                       int x_dtype, const float *__restrict__ w, float eps, HeadGate gate, int heads, int dv, float mul,
@@ -896,22 +886,6 @@ head_norm_gate_wide_kernel(void *__restrict__ out, int out_dtype, int out_stride
 // lanes of them, with every row at a multiple of 16 bytes.
 #define HNG_KEEP 4
 
-__device__ inline void hng_ld8(const void *p, int dtype, size_t i, float (&f)[8]) {
-    if (dtype == KVA_BF16) {
-        const uint4 v = *reinterpret_cast<const uint4 *>(reinterpret_cast<const uint16_t *>(p) + i);
-        const uint32_t u[4] = {v.x, v.y, v.z, v.w};
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            f[2 * j] = __uint_as_float(u[j] << 16);
-            f[2 * j + 1] = __uint_as_float(u[j] & 0xffff0000u);
-        }
-    } else {
-        const float4 a = *reinterpret_cast<const float4 *>(reinterpret_cast<const float *>(p) + i);
-        const float4 b = *reinterpret_cast<const float4 *>(reinterpret_cast<const float *>(p) + i + 4);
-        f[0] = a.x; f[1] = a.y; f[2] = a.z; f[3] = a.w; f[4] = b.x; f[5] = b.y; f[6] = b.z; f[7] = b.w;
-    }
-}
-
 template <bool WIDE>
 __global__ void __launch_bounds__(256)
 head_norm_gate_vec_kernel(void *__restrict__ out, int out_dtype, int out_stride, int out_off, const void *__restrict__ x,
@@ -942,7 +916,7 @@ head_norm_gate_vec_kernel(void *__restrict__ out, int out_dtype, int out_stride,
         for (int i = 0; i < 8; ++i) {
             if (gate.p) gt[k][i] = gate.act == 1 ? rec_sigmoid(gt[k][i]) : rec_silu(gt[k][i]);
             if (gate.first) v[k][i] *= gt[k][i];
-            sq += v[k][i] * v[k][i];
+            sq = rec_fma(v[k][i], v[k][i], sq);
         }
     }
     float inv = 1.f;

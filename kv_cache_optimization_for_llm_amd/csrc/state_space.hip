@@ -221,14 +221,14 @@ state_space_token_kernel(SsmArgs a) {
         for (int k = 0; k < SSM_TOKEN_ROWS; ++k) {
             const int r = r0 + 16 * k;
             const float w = b[k] * dt;
-            S[k].x = keep * S[k].x + w * x[0];
-            S[k].y = keep * S[k].y + w * x[1];
-            S[k].z = keep * S[k].z + w * x[2];
-            S[k].w = keep * S[k].w + w * x[3];
-            o[0] += S[k].x * c[k];
-            o[1] += S[k].y * c[k];
-            o[2] += S[k].z * c[k];
-            o[3] += S[k].w * c[k];
+            S[k].x = __builtin_fmaf(w, x[0], keep * S[k].x);
+            S[k].y = __builtin_fmaf(w, x[1], keep * S[k].y);
+            S[k].z = __builtin_fmaf(w, x[2], keep * S[k].z);
+            S[k].w = __builtin_fmaf(w, x[3], keep * S[k].w);
+            o[0] = __builtin_fmaf(S[k].x, c[k], o[0]);
+            o[1] = __builtin_fmaf(S[k].y, c[k], o[1]);
+            o[2] = __builtin_fmaf(S[k].z, c[k], o[2]);
+            o[3] = __builtin_fmaf(S[k].w, c[k], o[3]);
             if (on && r < n) *reinterpret_cast<float4 *>(Sg + (size_t)r * dv) = S[k];
         }
     }
@@ -243,7 +243,7 @@ state_space_token_kernel(SsmArgs a) {
         v.x += red[w][cg].x; v.y += red[w][cg].y; v.z += red[w][cg].z; v.w += red[w][cg].w;
     }
     *reinterpret_cast<float4 *>(a.out + (size_t)q0 * a.heads * dv + head * dv + col) =
-        make_float4(v.x + skip * x[0], v.y + skip * x[1], v.z + skip * x[2], v.w + skip * x[3]);
+        make_float4(__builtin_fmaf(skip, x[0], v.x), __builtin_fmaf(skip, x[1], v.y), __builtin_fmaf(skip, x[2], v.z), __builtin_fmaf(skip, x[3], v.w));
 }
 
 // ---- chunks of 64 tokens on the matrix cores -------------------------------------------------------------

@@ -2185,6 +2185,103 @@ def head_norm_gate(x: torch.Tensor, weight: Optional[torch.Tensor], eps: float, 
     return out
 
 
+# One token of every request through a recurrent mixer in one launch: the same numbers as the functions above, called one after the
+# other (csrc/recurrent_token.hip).  Each returns False where the sizes or addresses are not what it is built for: nothing was done.
+def _token_rows(what: str, y: torch.Tensor, col0: int, cols: int, out: torch.Tensor, out_off: int, inner: int, entries: int) -> None:
+    if y.dim() != 2 or not 0 <= col0 <= y.shape[1] - cols or out.dim() != 2 or out.shape[0] != y.shape[0] \
+            or not 0 <= out_off <= out.shape[1] - inner or entries != y.shape[0]:
+        raise KernelError(f"{what}: one row of y {tuple(y.shape)} and of out {tuple(out.shape)} per entry, wide enough for what they hold")
+
+
+def _vectors(what: str, *pairs) -> None:
+    for t, shape in pairs:
+        if t is not None and (tuple(t.shape) != shape or t.dtype != torch.float32):
+            raise KernelError(f"{what}: fp32 {shape} expected, not {t.dtype} {tuple(t.shape)}")
+
+
+def _token_launch(fn, what: str, *args) -> bool:
+    if not fn(1, *args):
+        return False
+    check(fn(0, *args), what)
+    return True
+
+
+def gated_delta_rule_token(y: torch.Tensor, conv_col: int, conv_weight: torch.Tensor, state: torch.Tensor, state_off: int, conv_off: int,
+                           beta_off: int, decay_off: int, a_log: Optional[torch.Tensor], dt_bias: Optional[torch.Tensor],
+                           channel_decay: Optional[torch.Tensor], unit_eps: float, norm_weight: torch.Tensor, norm_eps: float,
+                           gate: torch.Tensor, gate_off: int, activation: str, out: torch.Tensor, out_off: int, mul: float,
+                           entry_q_start: torch.Tensor, entry_seat: torch.Tensor, heads: int, kv_heads: int, dim: int, vdim: int) -> bool:
+    """:func:`causal_conv_act` (silu), :func:`gated_delta_rule` and :func:`head_norm_gate` for entries of one token."""
+    what, channels, inner = "gated_delta_rule_token", 2 * kv_heads * dim + heads * vdim, heads * vdim
+    qs, seat, entries = _entries((entry_q_start, entry_seat), what)
+    _token_rows(what, y, conv_col, channels, out, out_off, inner, entries)
+    if conv_weight.dim() != 2 or gate.dim() != 2 or gate.shape[0] != y.shape[0] or not 0 <= gate_off <= gate.shape[1] - inner \
+            or not 0 <= beta_off <= y.shape[1] - heads or (channel_decay is None and not 0 <= decay_off <= y.shape[1] - heads):
+        raise KernelError(f"{what}: columns lie outside their rows")
+    taps = conv_weight.shape[1]
+    _vectors(what, (conv_weight, (channels, taps)), (norm_weight, (vdim,)), (channel_decay, (y.shape[0], heads * dim)),
+             (None if channel_decay is not None else a_log, (heads,)), (None if channel_decay is not None else dt_bias, (heads,)))
+    _state_row(state, conv_off, channels * (taps - 1), what)
+    stride = _state_row(state, state_off, heads * dim * vdim, what)
+    return _token_launch(
+        hip_lib().kva_delta_token, what, _dev(y, "y"), dtype_code(y.dtype), y.shape[1], int(conv_col), _dev(conv_weight, "conv_weight"), taps,
+        _dev(state, "state"), stride, int(state_off), int(conv_off), int(beta_off), int(decay_off), _opt(a_log, "a_log"),
+        _opt(dt_bias, "dt_bias"), _opt(channel_decay, "channel_decay"), heads * dim, float(unit_eps), _dev(norm_weight, "norm_weight"),
+        float(norm_eps), _dev(gate, "gate"), dtype_code(gate.dtype), gate.shape[1], int(gate_off), HEAD_GATES[activation], _dev(out, "out"),
+        dtype_code(out.dtype), out.shape[1], int(out_off), float(mul), qs, seat, entries, heads, kv_heads, dim, vdim, _stream())
+
+
+def gated_linear_attention_token(y: torch.Tensor, q_off: int, k_off: int, v_off: int, a_off: int, a2: torch.Tensor, a2_bias: torch.Tensor,
+                                 tau: float, q_mul: float, state: torch.Tensor, state_off: int, norm_weight: torch.Tensor, norm_eps: float,
+                                 gate_off: int, activation: str, out: torch.Tensor, out_off: int, mul: float,
+                                 entry_q_start: torch.Tensor, entry_seat: torch.Tensor, heads: int, dim: int, vdim: int) -> bool:
+    """:func:`small_product_f32` (a decay per channel from ``a2`` and the columns ``a_off ..``), :func:`gated_linear_attention` and
+    :func:`head_norm_gate` (the gate in the columns ``gate_off ..``) for entries of one token."""
+    what, inner = "gated_linear_attention_token", heads * vdim
+    qs, seat, entries = _entries((entry_q_start, entry_seat), what)
+    _token_rows(what, y, min(q_off, k_off, v_off, a_off, gate_off), 1, out, out_off, inner, entries)
+    rank = a2.shape[1]
+    for off, n in ((q_off, heads * dim), (k_off, heads * dim), (v_off, inner), (gate_off, inner), (a_off, rank)):
+        if off + n > y.shape[1]:
+            raise KernelError(f"{what}: columns lie outside y")
+    if tuple(a2.shape) != (heads * dim, rank):
+        raise KernelError(f"{what}: the decays' matrix {tuple(a2.shape)} is not [heads * dim, rank]")
+    _vectors(what, (a2_bias, (heads * dim,)), (norm_weight, (vdim,)))
+    stride = _state_row(state, state_off, heads * dim * vdim, what)
+    return _token_launch(
+        hip_lib().kva_linear_token, what, _dev(y, "y"), dtype_code(y.dtype), y.shape[1], int(q_off), int(k_off), int(v_off), int(a_off), rank,
+        _dev(a2, "a2"), dtype_code(a2.dtype), _dev(a2_bias, "a2_bias"), 1.0 / float(tau), float(q_mul), _dev(state, "state"), stride,
+        int(state_off), _dev(norm_weight, "norm_weight"), float(norm_eps), _dev(y, "y"), dtype_code(y.dtype), y.shape[1], int(gate_off),
+        HEAD_GATES[activation], _dev(out, "out"), dtype_code(out.dtype), out.shape[1], int(out_off), float(mul), qs, seat, entries, heads,
+        dim, vdim, _stream())
+
+
+def state_space_token(y: torch.Tensor, conv_col: int, conv_weight: torch.Tensor, conv_bias: Optional[torch.Tensor], state: torch.Tensor,
+                      state_off: int, conv_off: int, dt_off: int, a_log: torch.Tensor, dt_bias: torch.Tensor, skip: torch.Tensor,
+                      norm_weight: torch.Tensor, norm_eps: float, gate_off: int, out: torch.Tensor, out_off: int, mul: float,
+                      entry_q_start: torch.Tensor, entry_seat: torch.Tensor, heads: int, groups: int, state_size: int, vdim: int,
+                      norm_groups: int) -> bool:
+    """:func:`causal_conv_act` (silu, rows in y's type), :func:`state_space` and :func:`head_norm_gate` (silu in front of the norm of
+    ``norm_groups`` parts, the gate in the columns ``gate_off ..``) for entries of one token."""
+    what, inner = "state_space_token", heads * vdim
+    channels = inner + 2 * groups * state_size
+    qs, seat, entries = _entries((entry_q_start, entry_seat), what)
+    _token_rows(what, y, conv_col, channels, out, out_off, inner, entries)
+    if conv_weight.dim() != 2 or not 0 <= gate_off <= y.shape[1] - inner or not 0 <= dt_off <= y.shape[1] - heads:
+        raise KernelError(f"{what}: columns lie outside y")
+    taps = conv_weight.shape[1]
+    _vectors(what, (conv_weight, (channels, taps)), (conv_bias, (channels,)), (norm_weight, (inner,)), (a_log, (heads,)),
+             (dt_bias, (heads,)), (skip, (heads,)))
+    _state_row(state, conv_off, channels * (taps - 1), what)
+    stride = _state_row(state, state_off, heads * state_size * vdim, what)
+    return _token_launch(
+        hip_lib().kva_space_token, what, _dev(y, "y"), dtype_code(y.dtype), y.shape[1], int(conv_col), _dev(conv_weight, "conv_weight"),
+        _opt(conv_bias, "conv_bias"), taps, _dev(state, "state"), stride, int(state_off), int(conv_off), int(dt_off), _dev(a_log, "a_log"),
+        _dev(dt_bias, "dt_bias"), _dev(skip, "skip"), _dev(norm_weight, "norm_weight"), float(norm_eps), int(gate_off), _dev(out, "out"),
+        dtype_code(out.dtype), out.shape[1], int(out_off), float(mul), qs, seat, entries, heads, groups, state_size, vdim,
+        int(norm_groups), _stream())
+
+
 # --------------------------------------------------------------------------------------
 # Routed experts.
 MOE_TILE = 16

@@ -98,6 +98,9 @@ _HIP_SIGNATURES = {
     "kva_event_synchronize": [P],
     "kva_event_destroy": [P],
     "kva_mark_tokens": [P, P, P, I, I, P],
+    "kva_delta_token": [I, P, I, I, I, P, I, P, LL, I, I, I, I, P, P, P, I, F, P, F, P, I, I, I, I, P, I, I, I, F, P, P, I, I, I, I, I, P],
+    "kva_linear_token": [I, P, I, I, I, I, I, I, I, P, I, P, F, F, P, LL, I, P, F, P, I, I, I, I, P, I, I, I, F, P, P, I, I, I, I, P],
+    "kva_space_token": [I, P, I, I, I, P, P, I, P, LL, I, I, I, P, P, P, P, F, I, P, I, I, I, F, P, P, I, I, I, I, I, I, P],
     "kva_causal_conv_act": [P, I, I, P, I, I, I, P, I, P, LL, I, P, P, I, I, I, I, P, P, I, P],
     "kva_latent_prompt": [P, P, I, I, P, P, P, P, P, I, P, P, P, I, P, P, I, P, P, I, I, I, I, I, I, I, I, F, P],
     "kva_latent_prompt_supported": [I, I, I, I],

@@ -127,6 +127,11 @@ class GatedLinearAttention(_InChunks, ProjectedMixer):
 
     def forward_inner(self, y, col0, ctx: MixerContext, state_off, out, out_col0, mul) -> None:
         batch, T = ctx.batch, y.shape[0]
+        if batch.max_q_len == 1 and K.gated_linear_attention_token(
+                y, col0 + self.q_off, col0 + self.k_off, col0 + self.v_off, col0 + self.a_off, self.a2, self.a2_bias, self.tau,
+                self.query_scale, ctx.state, state_off, self.norm_weight, self.norm_eps, col0 + self.g_off, "silu", out, out_col0, mul,
+                batch.entry_q_start, batch.entry_seat, self.num_heads, self.head_dim, self.value_dim):
+            return
         # the decays: the low-rank projection's second half, its bias, sigmoid and power in one 32-bit pass
         alpha = K.small_product_f32(y[:, col0 + self.a_off:col0 + self.a_off + self.rank], self.a2,
                                     torch.empty((T, self.num_heads * self.head_dim), dtype=torch.float32, device=y.device),
@@ -253,28 +258,33 @@ class GatedDeltaRule(_InChunks, ProjectedMixer):
         batch, T = ctx.batch, y.shape[0]
         lengths = np.diff(batch.h_entry_q_start)
         s_elems = self.num_heads * self.head_dim * self.value_dim
+        decays, gate, gate_off = None, y, col0 + self.g_off
+        if self.channel_decay:
+            # bias, softplus, the head's rate and the exponential in the second product's epilogue
+            d0 = col0 + self.decay_off
+            decays = K.small_product_f32(y[:, d0:d0 + self.decay_cols], self.a2,
+                                         torch.empty((T, self.num_heads * self.head_dim), dtype=torch.float32, device=y.device),
+                                         bias=self.dt_bias, rate_log=self.a_log)
+        if self.low_rank_gate:
+            gate, gate_off = self.g2(y[:, gate_off:gate_off + self.gate_cols].contiguous()), 0
+        if batch.max_q_len == 1 and K.gated_delta_rule_token(
+                y, col0, self.conv_weight, ctx.state, state_off, state_off + s_elems, col0 + self.beta_off, col0 + self.decay_off,
+                None if decays is not None else self.a_log, None if decays is not None else self.dt_bias, decays, self.unit_eps,
+                self.norm_weight, self.norm_eps, gate, gate_off, self.gate, out, out_col0, mul, batch.entry_q_start, batch.entry_seat,
+                self.num_heads, self.num_kv_heads, self.head_dim, self.value_dim):
+            return
         qkv = torch.empty((T, self.conv_channels), dtype=torch.float32, device=y.device)
         K.causal_conv_act(y, col0, self.conv_weight, qkv, ctx.state, state_off + s_elems, batch.entry_q_start,
                           batch.entry_seat, batch.max_q_len)
         o = torch.empty((T, self.inner_width), dtype=torch.float32, device=y.device)
-        if self.channel_decay:
-            # bias, softplus, the head's rate and the exponential in the second product's epilogue
-            d0 = col0 + self.decay_off
-            g = K.small_product_f32(y[:, d0:d0 + self.decay_cols], self.a2,
-                                    torch.empty((T, self.num_heads * self.head_dim), dtype=torch.float32, device=y.device),
-                                    bias=self.dt_bias, rate_log=self.a_log)
+        if decays is not None:
             K.gated_delta_rule(qkv, y, col0 + self.beta_off, 0, None, None, o, ctx.state, state_off,
                                batch.entry_q_start, batch.entry_seat, self.num_heads, self.num_kv_heads,
-                               self.head_dim, self.value_dim, self.unit_eps, channel_decay=g, lengths=lengths)
+                               self.head_dim, self.value_dim, self.unit_eps, channel_decay=decays, lengths=lengths)
         else:
             K.gated_delta_rule(qkv, y, col0 + self.beta_off, col0 + self.decay_off, self.a_log, self.dt_bias, o,
                                ctx.state, state_off, batch.entry_q_start, batch.entry_seat, self.num_heads,
                                self.num_kv_heads, self.head_dim, self.value_dim, self.unit_eps, lengths=lengths)
-        if self.low_rank_gate:
-            g0 = col0 + self.g_off
-            gate, gate_off = self.g2(y[:, g0:g0 + self.gate_cols].contiguous()), 0
-        else:
-            gate, gate_off = y, col0 + self.g_off
         K.head_norm_gate(o, self.norm_weight, self.norm_eps, gate, gate_off, out, out_col0, self.num_heads,
                          self.value_dim, self.gate, mul)
 
@@ -572,6 +582,11 @@ class StateSpaceDuality(ProjectedMixer):
     def forward_inner(self, y, col0, ctx: MixerContext, state_off, out, out_col0, mul) -> None:
         batch, T = ctx.batch, y.shape[0]
         s_elems = self.num_heads * self.state_size * self.value_dim
+        if batch.max_q_len == 1 and K.state_space_token(
+                y, col0 + self.conv_off, self.conv_weight, self.conv_bias, ctx.state, state_off, state_off + s_elems, col0 + self.dt_off,
+                self.a_log, self.dt_bias, self.skip, self.norm_weight, self.norm_eps, col0 + self.z_off, out, out_col0, mul,
+                batch.entry_q_start, batch.entry_seat, self.num_heads, self.groups, self.state_size, self.value_dim, self.norm_groups):
+            return
         xbc = torch.empty((T, self.conv_channels), dtype=y.dtype, device=y.device)
         K.causal_conv_act(y, col0 + self.conv_off, self.conv_weight, xbc, ctx.state, state_off + s_elems, batch.entry_q_start,
                           batch.entry_seat, batch.max_q_len, out_bias=self.conv_bias)
