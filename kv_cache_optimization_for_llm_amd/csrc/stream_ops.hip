@@ -19,6 +19,51 @@ __device__ inline void st_from_float(void *p, int dtype, size_t i, float v) {
     else reinterpret_cast<uint16_t *>(p)[i] = float_to_bf16_bits(v);
 }
 
+// Loads whose numbers are wanted later.  LATE: the bits now, the numbers then - a load that is turned into numbers inside a branch (on
+// whether there is one) is waited for there, and a kernel over a few rows is as long as its trips to memory.  That pays where the types
+// are known when the kernel is compiled; where they are not, choosing between two readings of the bits costs more than the waits
+// (2,048 rows of 4,096 25 -> 28 us, one row of 2,048 3.3 -> 3.6).  Nothing loaded is zeros either way.  us, numbers made as they are loaded
+// -> this, bf16 operands, 1 / 2,048 rows of 2,048: step between branches with layer norms 3.7 / 14.8 -> 3.3 / 12.7 (the sum over four
+// experts' rows in it 4.3 / 30.2 -> 3.8 / 25.8), with tanh norms 3.5 / 14.6 -> 2.8 / 12.0 (4.0 / 29.7 -> 3.3 / 25.4), layer norm of a bf16
+// stream with two outputs added 3.7 / 11.6 -> 3.0 / 9.6, one copy of the stream 4.0 / 11.9 -> 3.2 / 10.1.
+template <int N, bool LATE>             // neighbouring elements at a multiple of 16 (fp32) or 2 N (bf16) bytes
+struct RawRow {
+    uint32_t u[N] = {};
+    __device__ inline void load(const void *p, int dtype, size_t i) {
+        if (dtype == KVA_F32) {
+#pragma unroll
+            for (int k = 0; k < N; k += 4) {
+                const uint4 v = *reinterpret_cast<const uint4 *>(reinterpret_cast<const uint32_t *>(p) + i + k);
+                u[k] = v.x; u[k + 1] = v.y; u[k + 2] = v.z; u[k + 3] = v.w;
+            }
+        } else {
+            uint32_t w[N / 2];
+            if constexpr (N == 4) {
+                const uint2 v = *reinterpret_cast<const uint2 *>(reinterpret_cast<const uint16_t *>(p) + i);
+                w[0] = v.x; w[1] = v.y;
+            } else {
+                const uint4 v = *reinterpret_cast<const uint4 *>(reinterpret_cast<const uint16_t *>(p) + i);
+                w[0] = v.x; w[1] = v.y; w[2] = v.z; w[3] = v.w;
+            }
+#pragma unroll
+            for (int k = 0; k < N; ++k) u[k] = LATE ? w[k / 2] : k % 2 ? w[k / 2] & 0xffff0000u : w[k / 2] << 16;
+        }
+    }
+    __device__ inline void floats(int dtype, float (&f)[N]) const {
+#pragma unroll
+        for (int k = 0; k < N; ++k)
+            f[k] = __uint_as_float(!LATE || dtype == KVA_F32 ? u[k] : k % 2 ? u[k] & 0xffff0000u : u[k] << 16);
+    }
+};
+// The types of most launches, known when the kernel is compiled: branch outputs, weights and results bf16 (SIDE32: of routed
+// experts, whose extra row is fp32; WEIGHTS32: fp32 weights beside them) or all fp32; the stream fp32, or (layer norms) bf16 like the rest.
+enum { TYPES_ANY = 0, TYPES_BF16 = 1, TYPES_SIDE32 = 2, TYPES_F32 = 3, TYPES_STREAM16 = 4, TYPES_WEIGHTS32 = 5 };
+static inline bool type_or_absent(const void *p, int dtype, int want) { return p == nullptr || dtype == want; }
+#define KVA_BY_TYPES(types, KERNEL, ...)                                                                                             \
+    (types == TYPES_BF16 ? KERNEL<__VA_ARGS__, TYPES_BF16, Experts> : types == TYPES_SIDE32 ? KERNEL<__VA_ARGS__, TYPES_SIDE32, Experts>  \
+     : types == TYPES_F32 ? KERNEL<__VA_ARGS__, TYPES_F32, Experts> : types == TYPES_WEIGHTS32 ? KERNEL<__VA_ARGS__, TYPES_WEIGHTS32, Experts>  \
+     : KERNEL<__VA_ARGS__, TYPES_ANY, Experts>)
+
 // A branch output that is still the rows of routed experts: y[t] = sum_k rows[t top + k] (+ sigmoid(gate[t]) extra[t]).  The
 // kernels that let a branch output into the stream form it on the way, in 32 bits: a launch of its own for the sum wrote it
 // rounded and read it back (2,048 tokens of 2,048, four choices: 13-15 us of 27-32 with the norm behind it; one token: 4.8 of 9.5).
@@ -38,7 +83,7 @@ __device__ inline void expert_sum(const NoExperts &, bool, size_t, int, int, flo
 // W neighbouring columns from j on of row t; y: the extra row's elements (zeros without one) on the way in, the sum on the way out
 template <int W>
 __device__ inline void expert_sum(const ExpertSum &er, bool extra, size_t t, int width, int j, float (&y)[W]) {
-    const float eg = extra && er.gate ? 1.f / (1.f + expf(-er.gate[t * er.gate_stride])) : 1.f;
+    float eg = extra && er.gate ? er.gate[t * er.gate_stride] : 0.f;
     float sum[W];
 #pragma unroll
     for (int e = 0; e < W; ++e) sum[e] = 0.f;
@@ -56,6 +101,7 @@ __device__ inline void expert_sum(const ExpertSum &er, bool extra, size_t t, int
             for (int e = 0; e < W; ++e) sum[e] += row[e];
         }
     }
+    eg = extra && er.gate ? 1.f / (1.f + expf(-eg)) : 1.f;
 #pragma unroll
     for (int e = 0; e < W; ++e) y[e] = sum[e] + (extra ? eg * y[e] : 0.f);
 }
@@ -115,22 +161,6 @@ layernorm_kernel(void *__restrict__ out1, void *__restrict__ out2, int out_dtype
 // Rows of a multiple of 8 elements up to 8,192, every operand at a multiple of 16 bytes: a thread holds PER times 8 neighbouring
 // elements in registers from the sum to the outputs.  (One element a time, what was added up written and read back through
 // memory, 2,048 rows of 2,048 with a branch added took 54 us; so they take 10.)
-__device__ inline void ld8_as_float(const void *p, int dtype, size_t i, float (&o)[8]) {
-    if (dtype == KVA_F32) {
-        const float4 *f = reinterpret_cast<const float4 *>(reinterpret_cast<const float *>(p) + i);
-        const float4 a = f[0], b = f[1];
-        o[0] = a.x; o[1] = a.y; o[2] = a.z; o[3] = a.w; o[4] = b.x; o[5] = b.y; o[6] = b.z; o[7] = b.w;
-    } else {
-        const uint4 v = *reinterpret_cast<const uint4 *>(reinterpret_cast<const uint16_t *>(p) + i);
-        const uint32_t w[4] = {v.x, v.y, v.z, v.w};
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            o[2 * j] = bf16_bits_to_float((uint16_t)(w[j] & 0xffffu));
-            o[2 * j + 1] = bf16_bits_to_float((uint16_t)(w[j] >> 16));
-        }
-    }
-}
-
 __device__ inline void st8_from_float(void *p, int dtype, size_t i, const float (&v)[8]) {
     if (dtype == KVA_F32) {
         float4 *f = reinterpret_cast<float4 *>(reinterpret_cast<float *>(p) + i);
@@ -145,30 +175,44 @@ __device__ inline void st8_from_float(void *p, int dtype, size_t i, const float 
     }
 }
 
-template <int PER, typename Experts>
+template <int PER, int TYPES, typename Experts>
 __global__ void __launch_bounds__(256)
 layernorm_vec_kernel(void *__restrict__ out1, void *__restrict__ out2, int out_dtype, void *__restrict__ x, int x_dtype,
                      const void *__restrict__ d1, int d1_dtype, const void *__restrict__ d2, int d2_dtype,
                      const void *__restrict__ w1, const void *__restrict__ w2, int w_dtype,
                      const int *__restrict__ row_idx, int width, float eps, int rms, float delta_scale, Experts er) {
+    constexpr bool LATE = TYPES != TYPES_ANY;
+    if constexpr (LATE) {
+        x_dtype = TYPES == TYPES_STREAM16 ? KVA_BF16 : KVA_F32;
+        d1_dtype = out_dtype = TYPES == TYPES_F32 ? KVA_F32 : KVA_BF16;
+        w_dtype = TYPES == TYPES_F32 || TYPES == TYPES_WEIGHTS32 ? KVA_F32 : KVA_BF16;
+        d2_dtype = TYPES == TYPES_F32 || TYPES == TYPES_SIDE32 ? KVA_F32 : KVA_BF16;
+    }
     __shared__ float red_s[4];
     const int r = blockIdx.x;
     const size_t src = (size_t)(row_idx ? row_idx[r] : r) * width, dst = (size_t)r * width;
     float v[PER][8], w[8];
+    RawRow<8, LATE> xr[PER], ar[PER], br[PER], w1r[PER], w2r[PER];
+#pragma unroll
+    for (int c = 0; c < PER; ++c) {
+        const int j = (c * 256 + (int)threadIdx.x) * 8;
+        if (j >= width) continue;
+        xr[c].load(x, x_dtype, src + j);
+        if (d1) ar[c].load(d1, d1_dtype, src + j);
+        if (d2) br[c].load(d2, d2_dtype, src + j);
+        w1r[c].load(w1, w_dtype, j);
+        if (w2) w2r[c].load(w2, w_dtype, j);
+    }
     float sum = 0.f;
 #pragma unroll
     for (int c = 0; c < PER; ++c) {
         const int j = (c * 256 + (int)threadIdx.x) * 8;
-#pragma unroll
-        for (int i = 0; i < 8; ++i) v[c][i] = 0.f;
+        xr[c].floats(x_dtype, v[c]);
         if (j >= width) continue;
-        ld8_as_float(x, x_dtype, src + j, v[c]);
         if (d1 || d2 || er.rows) {
             float a[8], b[8];
-#pragma unroll
-            for (int i = 0; i < 8; ++i) a[i] = b[i] = 0.f;
-            if (d1) ld8_as_float(d1, d1_dtype, src + j, a);
-            if (d2) ld8_as_float(d2, d2_dtype, src + j, b);
+            ar[c].floats(d1_dtype, a);
+            br[c].floats(d2_dtype, b);
             if (er.rows) expert_sum<8>(er, d2 != nullptr, src / width, width, j, b);
 #pragma unroll
             for (int i = 0; i < 8; ++i) {
@@ -199,12 +243,12 @@ layernorm_vec_kernel(void *__restrict__ out1, void *__restrict__ out2, int out_d
         const int j = (c * 256 + (int)threadIdx.x) * 8;
         if (j >= width) continue;
         float n[8];
-        ld8_as_float(w1, w_dtype, j, w);
+        w1r[c].floats(w_dtype, w);
 #pragma unroll
         for (int i = 0; i < 8; ++i) n[i] = v[c][i] * inv * w[i];
         st8_from_float(out1, out_dtype, dst + j, n);
         if (out2) {
-            ld8_as_float(w2, w_dtype, j, w);
+            w2r[c].floats(w_dtype, w);
 #pragma unroll
             for (int i = 0; i < 8; ++i) n[i] = v[c][i] * inv * w[i];
             st8_from_float(out2, out_dtype, dst + j, n);
@@ -224,10 +268,17 @@ extern "C" int kva_layernorm(void *out1, void *out2, int out_dtype, void *x, int
     if (rows == 0) return KVA_OK;
     const uintptr_t all = (uintptr_t)out1 | (uintptr_t)out2 | (uintptr_t)x | (uintptr_t)d1 | (uintptr_t)d2 | (uintptr_t)w1 |
                           (uintptr_t)w2 | (uintptr_t)expert_rows;
+    int types = TYPES_ANY;
+    if (x_dtype == KVA_F32 && type_or_absent(d1, d1_dtype, KVA_BF16) && w_dtype == KVA_BF16 && out_dtype == KVA_BF16)
+        types = type_or_absent(d2, d2_dtype, KVA_BF16) ? TYPES_BF16 : TYPES_SIDE32;
+    else if (x_dtype == w_dtype && out_dtype == w_dtype && type_or_absent(d1, d1_dtype, w_dtype) && type_or_absent(d2, d2_dtype, w_dtype))
+        types = w_dtype == KVA_F32 ? TYPES_F32 : TYPES_STREAM16;
+    else if (x_dtype == KVA_F32 && w_dtype == KVA_F32 && out_dtype == KVA_BF16 && type_or_absent(d1, d1_dtype, KVA_BF16) && type_or_absent(d2, d2_dtype, KVA_BF16))
+        types = TYPES_WEIGHTS32;
     auto launch = [&](auto er) {
         typedef decltype(er) Experts;
 #define KVA_LAYERNORM_VEC(PER)                                                                                          \
-    hipLaunchKernelGGL((layernorm_vec_kernel<PER, Experts>), dim3(rows), dim3(256), 0, stream, out1, out2, out_dtype, x, x_dtype, d1,  \
+    hipLaunchKernelGGL((types == TYPES_STREAM16 ? layernorm_vec_kernel<PER, TYPES_STREAM16, Experts> : KVA_BY_TYPES(types, layernorm_vec_kernel, PER)), dim3(rows), dim3(256), 0, stream, out1, out2, out_dtype, x, x_dtype, d1,  \
                        d1_dtype, d2, d2_dtype, w1, w2, w_dtype, row_idx, width, eps, rms, delta_scale, er)
         if (width % 8 == 0 && width <= 8192 && all % 16 == 0) {
             if (width <= 2048) KVA_LAYERNORM_VEC(1);
@@ -632,18 +683,20 @@ __device__ inline void hyper_ld4(const void *p, int dtype, size_t i, float (&f)[
     }
 }
 
-template <int S, int ITERS>
+template <int S, int ITERS, bool NARROW>
 __global__ void __launch_bounds__(256)
 hyper_step_vec_kernel(float *__restrict__ x, const void *__restrict__ y, int y_dtype, const float *__restrict__ mix,
                       const float *__restrict__ out_w, float mult, const float *__restrict__ in_w,
                       const void *__restrict__ nw, const void *__restrict__ nb, int w_dtype, float eps,
                       void *__restrict__ out, int out_dtype, const int *__restrict__ row_idx, int width) {
+    if constexpr (NARROW) y_dtype = w_dtype = out_dtype = KVA_BF16;
     __shared__ float red_s[4];
     __shared__ HyperCoefficients co;
     const int r = blockIdx.x;
     const size_t row = (size_t)(row_idx ? row_idx[r] : r);
     float *xr = x + row * S * width;
     float v[ITERS][S][4], yv[ITERS][4], wv[ITERS][4], bv[ITERS][4];
+    RawRow<4, NARROW> yr[ITERS], wr[ITERS], br[ITERS];
 #pragma unroll
     for (int it = 0; it < ITERS; ++it) {
         const int j = (threadIdx.x + it * 256) * 4;
@@ -653,11 +706,15 @@ hyper_step_vec_kernel(float *__restrict__ x, const void *__restrict__ y, int y_d
             const float4 t = on ? *reinterpret_cast<const float4 *>(xr + (size_t)s * width + j) : make_float4(0.f, 0.f, 0.f, 0.f);
             v[it][s][0] = t.x; v[it][s][1] = t.y; v[it][s][2] = t.z; v[it][s][3] = t.w;
         }
+        if (on && y) yr[it].load(y, y_dtype, row * width + j);
+        if (on && out) wr[it].load(nw, w_dtype, j);
+        if (on && out && nb) br[it].load(nb, w_dtype, j);
+    }
 #pragma unroll
-        for (int e = 0; e < 4; ++e) yv[it][e] = wv[it][e] = bv[it][e] = 0.f;
-        if (on && y) hyper_ld4(y, y_dtype, row * width + j, yv[it]);
-        if (on && out) hyper_ld4(nw, w_dtype, j, wv[it]);
-        if (on && out && nb) hyper_ld4(nb, w_dtype, j, bv[it]);
+    for (int it = 0; it < ITERS; ++it) {
+        yr[it].floats(y_dtype, yv[it]);
+        wr[it].floats(w_dtype, wv[it]);
+        br[it].floats(w_dtype, bv[it]);
     }
     if (threadIdx.x < S * S) co.mix[threadIdx.x] = y ? mix[threadIdx.x] : 0.f;
     if (threadIdx.x < S) {
@@ -735,9 +792,10 @@ static bool hyper_step_vec(float *x, const void *y, int y_dtype, const float *mi
     if (width % 4 || ((reinterpret_cast<uintptr_t>(x) | reinterpret_cast<uintptr_t>(y) | reinterpret_cast<uintptr_t>(norm_w) |
                        reinterpret_cast<uintptr_t>(norm_b) | reinterpret_cast<uintptr_t>(out)) & 15))
         return false;
+    const bool narrow = out && w_dtype == KVA_BF16 && out_dtype == KVA_BF16 && type_or_absent(y, y_dtype, KVA_BF16);
 #define KVA_HYPER_VEC(ITERS)                                                                                               \
-    hipLaunchKernelGGL((hyper_step_vec_kernel<S, ITERS>), dim3(rows), dim3(256), 0, stream, x, y, y_dtype, mix, out_w, mult,  \
-                       in_w, norm_w, norm_b, w_dtype, eps, out, out_dtype, row_idx, width)
+    hipLaunchKernelGGL((narrow ? hyper_step_vec_kernel<S, ITERS, true> : hyper_step_vec_kernel<S, ITERS, false>), dim3(rows), dim3(256), \
+                       0, stream, x, y, y_dtype, mix, out_w, mult, in_w, norm_w, norm_b, w_dtype, eps, out, out_dtype, row_idx, width)
     if (width <= 1024) KVA_HYPER_VEC(1);
     else if (width <= 2048 && S <= 8) KVA_HYPER_VEC(2);
     else if (width <= 4096 && S <= 4) KVA_HYPER_VEC(4);
@@ -890,31 +948,47 @@ __device__ inline float sandwich_sum(float v, float *line) {
     return total;
 }
 
-template <int THREADS, int ITERS, typename Experts>
+template <int THREADS, int ITERS, int TYPES, typename Experts>
 __global__ void __launch_bounds__(THREADS)
 sandwich_step_vec_kernel(float *__restrict__ x, const void *__restrict__ y, int y_dtype, SideNorm post,
                          const float *__restrict__ addend, SideNorm pre, void *__restrict__ out, int out_dtype,
                          const int *__restrict__ row_idx, int width, Experts er) {
+    constexpr bool LATE = TYPES != TYPES_ANY;
+    if constexpr (LATE) {
+        y_dtype = TYPES == TYPES_BF16 || TYPES == TYPES_WEIGHTS32 ? KVA_BF16 : KVA_F32;
+        post.w_dtype = pre.w_dtype = TYPES == TYPES_F32 || TYPES == TYPES_WEIGHTS32 ? KVA_F32 : KVA_BF16;
+        out_dtype = TYPES == TYPES_F32 ? KVA_F32 : KVA_BF16;
+    }
     constexpr int WAVES = THREADS / KVA_WAVE;
     __shared__ float red_s[4][WAVES];
     const int r = blockIdx.x;
     const size_t row = (size_t)(row_idx ? row_idx[r] : r) * width;
     float v[ITERS][4], yv[ITERS][4], av[ITERS][4], pw[ITERS][4], pb[ITERS][4], nw[ITERS][4], nb[ITERS][4];
     const bool enters = y || er.rows, norm_y = enters && post.w;
+    RawRow<4, LATE> raw[ITERS][7];
 #pragma unroll
     for (int it = 0; it < ITERS; ++it) {
         const int j = (threadIdx.x + it * THREADS) * 4;
-#pragma unroll
-        for (int e = 0; e < 4; ++e) v[it][e] = yv[it][e] = av[it][e] = pw[it][e] = pb[it][e] = nw[it][e] = nb[it][e] = 0.f;
         if (j >= width) continue;
-        hyper_ld4(x, KVA_F32, row + j, v[it]);
-        if (y) hyper_ld4(y, y_dtype, row + j, yv[it]);
-        if (er.rows) expert_sum<4>(er, y != nullptr, row / width, width, j, yv[it]);
-        if (addend) hyper_ld4(addend, KVA_F32, row + j, av[it]);
-        if (norm_y) hyper_ld4(post.w, post.w_dtype, j, pw[it]);
-        if (norm_y && post.b) hyper_ld4(post.b, post.w_dtype, j, pb[it]);
-        if (out) hyper_ld4(pre.w, pre.w_dtype, j, nw[it]);
-        if (out && pre.b) hyper_ld4(pre.b, pre.w_dtype, j, nb[it]);
+        raw[it][0].load(x, KVA_F32, row + j);
+        if (y) raw[it][1].load(y, y_dtype, row + j);
+        if (addend) raw[it][2].load(addend, KVA_F32, row + j);
+        if (norm_y) raw[it][3].load(post.w, post.w_dtype, j);
+        if (norm_y && post.b) raw[it][4].load(post.b, post.w_dtype, j);
+        if (out) raw[it][5].load(pre.w, pre.w_dtype, j);
+        if (out && pre.b) raw[it][6].load(pre.b, pre.w_dtype, j);
+    }
+#pragma unroll
+    for (int it = 0; it < ITERS; ++it) {
+        const int j = (threadIdx.x + it * THREADS) * 4;
+        raw[it][0].floats(KVA_F32, v[it]);
+        raw[it][1].floats(y_dtype, yv[it]);
+        raw[it][2].floats(KVA_F32, av[it]);
+        raw[it][3].floats(post.w_dtype, pw[it]);
+        raw[it][4].floats(post.w_dtype, pb[it]);
+        raw[it][5].floats(pre.w_dtype, nw[it]);
+        raw[it][6].floats(pre.w_dtype, nb[it]);
+        if (er.rows && j < width) expert_sum<4>(er, y != nullptr, row / width, width, j, yv[it]);
     }
     if (norm_y) {
         float mean = 0.f;
@@ -982,6 +1056,14 @@ sandwich_step_vec_kernel(float *__restrict__ x, const void *__restrict__ y, int 
     }
 }
 
+static int step_types(const void *y, int y_dtype, const void *post_w, int post_dtype, const void *pre_w, int pre_dtype, const void *out, int out_dtype) {
+    const bool y16 = type_or_absent(y, y_dtype, KVA_BF16), out16 = type_or_absent(out, out_dtype, KVA_BF16);
+    if (out16 && type_or_absent(post_w, post_dtype, KVA_BF16) && type_or_absent(pre_w, pre_dtype, KVA_BF16)) return y16 ? TYPES_BF16 : TYPES_SIDE32;
+    if (!type_or_absent(post_w, post_dtype, KVA_F32) || !type_or_absent(pre_w, pre_dtype, KVA_F32)) return TYPES_ANY;
+    if (type_or_absent(y, y_dtype, KVA_F32) && type_or_absent(out, out_dtype, KVA_F32)) return TYPES_F32;
+    return y16 && out16 ? TYPES_WEIGHTS32 : TYPES_ANY;
+}
+
 extern "C" int kva_sandwich_step(float *x, const void *y, int y_dtype, const void *post_w, const void *post_b, int post_dtype,
                                  int post_center, float post_eps, const float *addend, const void *pre_w, const void *pre_b,
                                  int pre_dtype, int pre_center, float pre_eps, void *out, int out_dtype, const int *row_idx,
@@ -1000,10 +1082,11 @@ extern "C" int kva_sandwich_step(float *x, const void *y, int y_dtype, const voi
     // (which kernel runs depends on width and alignment alone, never on the rows: a row's numbers are the same in any batch)
     const bool aligned = aligned16(x) && aligned16(y) && aligned16(post_w) && aligned16(post_b) && aligned16(addend) &&
                          aligned16(pre_w) && aligned16(pre_b) && aligned16(out) && aligned16(expert_rows);
+    const int types = step_types(y, y_dtype, post_w, post_dtype, pre_w, pre_dtype, out, out_dtype);
     auto launch = [&](auto er) {
         typedef decltype(er) Experts;
 #define KVA_SANDWICH(THREADS, ITERS)                                                                                     \
-    hipLaunchKernelGGL((sandwich_step_vec_kernel<THREADS, ITERS, Experts>), dim3(rows), dim3(THREADS), 0, stream, x, y, y_dtype,  \
+    hipLaunchKernelGGL(KVA_BY_TYPES(types, sandwich_step_vec_kernel, THREADS, ITERS), dim3(rows), dim3(THREADS), 0, stream, x, y, y_dtype,  \
                        post, addend, pre, out, out_dtype, row_idx, width, er)
         if (width % 4 == 0 && width <= 8192 && aligned) {
             if (width <= 1024) KVA_SANDWICH(256, 1);
@@ -1037,39 +1120,55 @@ struct TanhNorm {
     float alpha;
 };
 
-template <bool VEC>
+template <bool VEC, int TYPES>
 __global__ void __launch_bounds__(256)
 tanh_step_kernel(float *__restrict__ x, const void *__restrict__ y, int y_dtype, const float *__restrict__ y_bias,
                  ExpertSum er, TanhNorm post, TanhNorm pre, void *__restrict__ out, int out_dtype, const int *__restrict__ row_idx,
                  int width, size_t n) {
     constexpr int W = VEC ? 4 : 1;
+    constexpr bool LATE = TYPES != TYPES_ANY;
+    if constexpr (LATE) {
+        y_dtype = TYPES == TYPES_BF16 || TYPES == TYPES_WEIGHTS32 ? KVA_BF16 : KVA_F32;
+        post.dtype = pre.dtype = TYPES == TYPES_F32 || TYPES == TYPES_WEIGHTS32 ? KVA_F32 : KVA_BF16;
+        out_dtype = TYPES == TYPES_F32 ? KVA_F32 : KVA_BF16;
+    }
     const size_t i = ((size_t)blockIdx.x * blockDim.x + threadIdx.x) * W;
     if (i >= n) return;
     const size_t r = i / width;
     const int j = (int)(i % width);
     const size_t at = row_idx ? (size_t)row_idx[r] * width + j : i;
     float v[W], yv[W], yb[W], pw[W], pb[W], nw[W], nb[W];
-    auto load = [&](const void *p, int dtype, size_t k, float (&f)[W]) {
-        if constexpr (VEC) hyper_ld4(p, dtype, k, f);
-        else f[0] = ld_as_float(p, dtype, k);
-    };
-#pragma unroll
-    for (int e = 0; e < W; ++e) yv[e] = yb[e] = pw[e] = pb[e] = nw[e] = nb[e] = 0.f;
-    load(x, KVA_F32, at, v);
-    const bool enters = y || er.rows;
-    if (enters) {
-        if (y) load(y, y_dtype, at, yv);
-        if (er.rows) expert_sum<W>(er, y != nullptr, at / width, width, j, yv);
-        if (y_bias) load(y_bias, KVA_F32, j, yb);
-        if (post.w) {
-            load(post.w, post.dtype, j, pw);
-            load(post.b, post.dtype, j, pb);
+    const bool enters = y || er.rows, norm_y = enters && post.w;
+    if constexpr (VEC) {
+        RawRow<4, LATE> raw[7];
+        raw[0].load(x, KVA_F32, at);
+        if (y) raw[1].load(y, y_dtype, at);
+        if (enters && y_bias) raw[2].load(y_bias, KVA_F32, j);
+        if (norm_y) {
+            raw[3].load(post.w, post.dtype, j);
+            raw[4].load(post.b, post.dtype, j);
         }
+        if (out) {
+            raw[5].load(pre.w, pre.dtype, j);
+            raw[6].load(pre.b, pre.dtype, j);
+        }
+        raw[0].floats(KVA_F32, v);
+        raw[1].floats(y_dtype, yv);
+        raw[2].floats(KVA_F32, yb);
+        raw[3].floats(post.dtype, pw);
+        raw[4].floats(post.dtype, pb);
+        raw[5].floats(pre.dtype, nw);
+        raw[6].floats(pre.dtype, nb);
+    } else {
+        v[0] = x[at];
+        yv[0] = y ? ld_as_float(y, y_dtype, at) : 0.f;
+        yb[0] = enters && y_bias ? y_bias[j] : 0.f;
+        pw[0] = norm_y ? ld_as_float(post.w, post.dtype, j) : 0.f;
+        pb[0] = norm_y ? ld_as_float(post.b, post.dtype, j) : 0.f;
+        nw[0] = out ? ld_as_float(pre.w, pre.dtype, j) : 0.f;
+        nb[0] = out ? ld_as_float(pre.b, pre.dtype, j) : 0.f;
     }
-    if (out) {
-        load(pre.w, pre.dtype, j, nw);
-        load(pre.b, pre.dtype, j, nb);
-    }
+    if (er.rows) expert_sum<W>(er, y != nullptr, at / width, width, j, yv);
     if (enters) {
 #pragma unroll
         for (int e = 0; e < W; ++e) v[e] += post.w ? tanhf(post.alpha * (yv[e] + yb[e])) * pw[e] + pb[e] : yv[e] + yb[e];
@@ -1112,12 +1211,14 @@ extern "C" int kva_tanh_step(float *x, const void *y, int y_dtype, const float *
     const ExpertSum er{expert_rows, gate, top, gate_stride};
     const bool vec = width % 4 == 0 && aligned16(x) && aligned16(y) && aligned16(y_bias) && aligned16(expert_rows) && aligned16(post_w) &&
                      aligned16(post_b) && aligned16(pre_w) && aligned16(pre_b) && aligned16(out);
-    if (vec)
-        hipLaunchKernelGGL(tanh_step_kernel<true>, dim3((unsigned)((n / 4 + 255) / 256)), dim3(256), 0, stream, x, y, y_dtype,
-                           y_bias, er, post, pre, out, out_dtype, row_idx, width, n);
-    else
-        hipLaunchKernelGGL(tanh_step_kernel<false>, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, stream, x, y, y_dtype,
-                           y_bias, er, post, pre, out, out_dtype, row_idx, width, n);
+    const int types = step_types(y, y_dtype, post_w, post_dtype, pre_w, pre_dtype, out, out_dtype);
+    const auto kernel = !vec ? tanh_step_kernel<false, TYPES_ANY> : types == TYPES_BF16 ? tanh_step_kernel<true, TYPES_BF16>
+                        : types == TYPES_SIDE32 ? tanh_step_kernel<true, TYPES_SIDE32> : types == TYPES_F32 ? tanh_step_kernel<true, TYPES_F32>
+                        : types == TYPES_WEIGHTS32 ? tanh_step_kernel<true, TYPES_WEIGHTS32>                                                                                        : tanh_step_kernel<true, TYPES_ANY>;
+    // (a few rows: wavefronts spread over more units)
+    const int threads = vec && n / 4 <= 64 * 1024 ? 64 : 256, per = vec ? 4 * threads : threads;
+    hipLaunchKernelGGL(kernel, dim3((unsigned)((n + per - 1) / per)), dim3(threads), 0, stream, x, y, y_dtype, y_bias, er, post, pre, out,
+                       out_dtype, row_idx, width, n);
     KVA_CHECK_LAUNCH("tanh_step");
     return KVA_OK;
 }
