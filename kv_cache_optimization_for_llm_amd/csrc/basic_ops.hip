@@ -183,74 +183,61 @@ extern "C" int kva_embed_gather_prep(void *hidden, void *scaled, float *sumsq, c
     return KVA_OK;
 }
 
-#define RMS_VEC_CACHE 4   // vectors of 8 a thread keeps between the passes
-// 8 elements of the branch output that is added to the stream: from the bf16 delta, or (parts > 0)
-// the sum of `parts` fp32 partial products [parts][rows][width], rounded to bf16 as the product
-// itself would have been
-__device__ inline void load_delta8(const bf16_t *dl, const float *parts_row, int parts, size_t part_stride, int i,
-                                   float (&d)[8]) {
-    if (parts > 0) {
-        sum_ranges8(parts_row, parts, part_stride, i, d);
-    } else {
-        unpack8(*reinterpret_cast<const uint4 *>(dl + i), d);
-    }
+// A row's elements in registers, PER times 8 neighbouring ones a thread: a row's loads are asked for at once, the weight in front of
+// the sum over the workgroup, and what was added up is not read back.  us with a branch added, a loop over the row -> this: bf16, 2,048
+// rows of 2,048 / 8,192 10.9 / 43.9 -> 10.8 / 34.0; fp32 (element by element before) 3 rows 3.8 / 8.8 -> 2.9 / 4.4, 2,048 rows 19.0 /
+// 71.6 -> 14.9 / 53.5.
+template <typename T>
+__device__ inline void row_load8(const T *p, float (&f)[8]) { load_weight8<T>(p, f); }
+__device__ inline void row_store8(bf16_t *p, const float (&f)[8]) { *reinterpret_cast<uint4 *>(p) = pack8(f); }
+__device__ inline void row_store8(float *p, const float (&f)[8]) {
+    reinterpret_cast<float4 *>(p)[0] = make_float4(f[0], f[1], f[2], f[3]);
+    reinterpret_cast<float4 *>(p)[1] = make_float4(f[4], f[5], f[6], f[7]);
 }
 
-template <typename TW>
-__global__ void rmsnorm_vec_kernel(bf16_t *__restrict__ out, bf16_t *__restrict__ hidden,
-                                   const bf16_t *__restrict__ delta, const float *__restrict__ delta_parts,
-                                   int parts, size_t part_stride, const TW *__restrict__ weight,
-                                   const int *__restrict__ row_idx, int width, float eps) {
+template <typename T, typename TW, int PER>
+__global__ void __launch_bounds__(1024)
+rmsnorm_vec_kernel(T *__restrict__ out, T *__restrict__ hidden, const T *__restrict__ delta, const float *__restrict__ delta_parts,
+                   int parts, size_t part_stride, const TW *__restrict__ weight, const int *__restrict__ row_idx, int width, float eps) {
     __shared__ float scratch[16];
     const int orow = blockIdx.x;
     const int irow = row_idx ? row_idx[orow] : orow;
-    bf16_t *x = hidden + (size_t)irow * width;
-    const bf16_t *dl = delta ? delta + (size_t)irow * width : nullptr;
+    T *x = hidden + (size_t)irow * width;
     const float *pr = parts > 0 ? delta_parts + (size_t)irow * width : nullptr;
-    const bool adds = dl != nullptr || parts > 0;
-    const bool write_back = adds && !row_idx;
-    bf16_t *y = out + (size_t)orow * width;
-    float cache[RMS_VEC_CACHE][8];
+    const bool adds = delta != nullptr || parts > 0, write_back = adds && !row_idx;
+    float v[PER][8], d[PER][8], w[PER][8];
+#pragma unroll
+    for (int c = 0; c < PER; ++c) {
+        const int i = (c * blockDim.x + threadIdx.x) * 8;
+        if (i >= width) continue;
+        row_load8<T>(x + i, v[c]);
+        if (delta) row_load8<T>(delta + (size_t)irow * width + i, d[c]);
+    }
     float ss = 0.f;
-    int c = 0;
-    for (int i = threadIdx.x * 8; i < width; i += blockDim.x * 8, ++c) {
-        float v[8];
-        unpack8(*reinterpret_cast<const uint4 *>(x + i), v);
+#pragma unroll
+    for (int c = 0; c < PER; ++c) {
+        const int i = (c * blockDim.x + threadIdx.x) * 8;
+        if (i >= width) continue;
+        if constexpr (sizeof(T) == 2)
+            if (parts > 0) sum_ranges8(pr, parts, part_stride, i, d[c]);
         if (adds) {
-            float d[8];
-            load_delta8(dl, pr, parts, part_stride, i, d);
 #pragma unroll
-            for (int j = 0; j < 8; ++j) v[j] = bf16_bits_to_float(float_to_bf16_bits(v[j] + d[j]));
-            if (write_back) *reinterpret_cast<uint4 *>(x + i) = pack8(v);
+            for (int j = 0; j < 8; ++j) v[c][j] = to_float(from_float<T>(v[c][j] + d[c][j]));
+            if (write_back) row_store8(x + i, v[c]);
         }
 #pragma unroll
-        for (int j = 0; j < 8; ++j) ss += v[j] * v[j];
-        if (c < RMS_VEC_CACHE) {
-#pragma unroll
-            for (int j = 0; j < 8; ++j) cache[c][j] = v[j];
-        }
+        for (int j = 0; j < 8; ++j) ss += v[c][j] * v[c][j];
+        row_load8<TW>(weight + i, w[c]);            // (wanted behind the sum)
     }
     const float total = block_sum(ss, scratch, blockDim.x / KVA_WAVE);
     const float r = (float)sqrt((double)total / (double)width + (double)eps);
-    c = 0;
-    for (int i = threadIdx.x * 8; i < width; i += blockDim.x * 8, ++c) {
-        float v[8], w[8];
-        if (c < RMS_VEC_CACHE) {
 #pragma unroll
-            for (int j = 0; j < 8; ++j) v[j] = cache[c][j];
-        } else {
-            unpack8(*reinterpret_cast<const uint4 *>(x + i), v);
-            if (adds && !write_back) {
-                float d[8];
-                load_delta8(dl, pr, parts, part_stride, i, d);
+    for (int c = 0; c < PER; ++c) {
+        const int i = (c * blockDim.x + threadIdx.x) * 8;
+        if (i >= width) continue;
 #pragma unroll
-                for (int j = 0; j < 8; ++j) v[j] = bf16_bits_to_float(float_to_bf16_bits(v[j] + d[j]));
-            }
-        }
-        load_weight8<TW>(weight + i, w);
-#pragma unroll
-        for (int j = 0; j < 8; ++j) v[j] = (v[j] / r) * w[j];
-        *reinterpret_cast<uint4 *>(y + i) = pack8(v);
+        for (int j = 0; j < 8; ++j) v[c][j] = (v[c][j] / r) * w[c][j];
+        row_store8(out + (size_t)orow * width + i, v[c]);
     }
 }
 
@@ -265,36 +252,46 @@ extern "C" int kva_rmsnorm(void *out, void *hidden, const void *delta, const voi
                                dtype == KVA_BF16 && width % 8 == 0),
                 "rmsnorm: partial products stand in for a bf16 delta of a width that is a multiple of 8");
     if (out_rows == 0) return KVA_OK;
-    if (dtype == KVA_BF16 && width % 8 == 0) {
+    const uintptr_t all = (uintptr_t)out | (uintptr_t)hidden | (uintptr_t)delta | (uintptr_t)weight | (uintptr_t)delta_parts;
+    KVA_REQUIRE((dtype == KVA_BF16 || dtype == KVA_F32) && (weight_dtype == KVA_BF16 || weight_dtype == KVA_F32),
+                "rmsnorm: unsupported dtypes %d / %d", dtype, weight_dtype);
+    if (width % 8 == 0 && width <= 8 * 8 * 1024 && (dtype == KVA_BF16 || all % 16 == 0)) {
         // Many rows (prompt portions): 256 threads walk a row of up to 8,184 columns in several turns and
         // the workgroups overlap each other's waits.  Few rows (decode steps): a thread per 8 columns
         // where a workgroup allows, every load of the row asked for at once (4,096 columns, 64 rows:
         // 5.3 -> 4.5 us, with partial products in 8 ranges 9.2 -> 7.0; 2,048 rows: 18.6 -> 20.9, so not there).
         int threads = width >= 8192 ? 1024 : (width >= 2048 ? 256 : (width >= 1024 ? 128 : 64));
         if (out_rows <= 256) threads = std::min(1024, std::max(64, (width / 8 + 63) / 64 * 64));
-        dim3 vgrid(out_rows), vblock(threads);
+        const int per = (width / 8 + threads - 1) / threads;                 // 1 .. 8
         const size_t part_stride = (size_t)part_rows * width;
-        if (weight_dtype == KVA_BF16)
-            hipLaunchKernelGGL(rmsnorm_vec_kernel<bf16_t>, vgrid, vblock, 0, stream, (bf16_t *)out,
-                               (bf16_t *)hidden, (const bf16_t *)delta, delta_parts, parts, part_stride,
-                               (const bf16_t *)weight, row_idx, width, eps);
-        else if (weight_dtype == KVA_F32)
-            hipLaunchKernelGGL(rmsnorm_vec_kernel<float>, vgrid, vblock, 0, stream, (bf16_t *)out,
-                               (bf16_t *)hidden, (const bf16_t *)delta, delta_parts, parts, part_stride,
-                               (const float *)weight, row_idx, width, eps);
-        else KVA_REQUIRE(false, "rmsnorm: unsupported weight dtype %d", weight_dtype);
+#define RMS_LAUNCH(T, TW, PER)                                                                                                        \
+    hipLaunchKernelGGL((rmsnorm_vec_kernel<T, TW, PER>), dim3(out_rows), dim3(threads), 0, stream, (T *)out, (T *)hidden, (const T *)delta, \
+                       delta_parts, parts, part_stride, (const TW *)weight, row_idx, width, eps)
+#define RMS_VEC(T, TW)                                                                              \
+    do {                                                                                            \
+        if (per == 1) RMS_LAUNCH(T, TW, 1);                                                         \
+        else if (per == 2) RMS_LAUNCH(T, TW, 2);                                                    \
+        else if (per <= 4) RMS_LAUNCH(T, TW, 4);                                                    \
+        else RMS_LAUNCH(T, TW, 8);                                                                  \
+    } while (0)
+        if (dtype == KVA_BF16 && weight_dtype == KVA_BF16) RMS_VEC(bf16_t, bf16_t);
+        else if (dtype == KVA_BF16) RMS_VEC(bf16_t, float);
+        else if (weight_dtype == KVA_F32) RMS_VEC(float, float);
+        else RMS_VEC(float, bf16_t);
+#undef RMS_VEC
+#undef RMS_LAUNCH
         KVA_CHECK_LAUNCH("rmsnorm");
         return KVA_OK;
     }
+    KVA_REQUIRE(parts == 0, "rmsnorm: partial products go with rows of up to 65,536");
     dim3 grid(out_rows), block(width >= 2048 ? 512 : 256);
 #define LAUNCH(T, TW)                                                                      \
     hipLaunchKernelGGL((rmsnorm_kernel<T, TW>), grid, block, 0, stream, (T *)out, (T *)hidden, \
                        (const T *)delta, (const TW *)weight, row_idx, width, eps)
     if (dtype == KVA_F32 && weight_dtype == KVA_F32) LAUNCH(float, float);
     else if (dtype == KVA_BF16 && weight_dtype == KVA_BF16) LAUNCH(bf16_t, bf16_t);
-    else if (dtype == KVA_BF16 && weight_dtype == KVA_F32) LAUNCH(bf16_t, float);
-    else if (dtype == KVA_F32 && weight_dtype == KVA_BF16) LAUNCH(float, bf16_t);
-    else KVA_REQUIRE(false, "rmsnorm: unsupported dtypes %d / %d", dtype, weight_dtype);
+    else if (dtype == KVA_BF16) LAUNCH(bf16_t, float);
+    else LAUNCH(float, bf16_t);
 #undef LAUNCH
     KVA_CHECK_LAUNCH("rmsnorm");
     return KVA_OK;
@@ -474,18 +471,19 @@ __global__ void silu_mul_kernel(T *__restrict__ out, const T *__restrict__ gate_
     }
 }
 
-__global__ void silu_mul_vec_kernel(bf16_t *__restrict__ out, const bf16_t *__restrict__ gate_up, int inter) {
+template <typename T>
+__global__ void silu_mul_vec_kernel(T *__restrict__ out, const T *__restrict__ gate_up, int inter) {
     const int row = blockIdx.y;
-    const bf16_t *g = gate_up + (size_t)row * 2 * inter;
-    const bf16_t *u = g + inter;
-    bf16_t *o = out + (size_t)row * inter;
+    const T *g = gate_up + (size_t)row * 2 * inter;
+    const T *u = g + inter;
+    T *o = out + (size_t)row * inter;
     for (int i = (blockIdx.x * blockDim.x + threadIdx.x) * 8; i < inter; i += gridDim.x * blockDim.x * 8) {
         float gv[8], uv[8];
-        unpack8(*reinterpret_cast<const uint4 *>(g + i), gv);
-        unpack8(*reinterpret_cast<const uint4 *>(u + i), uv);
+        row_load8<T>(g + i, gv);
+        row_load8<T>(u + i, uv);
 #pragma unroll
         for (int j = 0; j < 8; ++j) gv[j] = gv[j] * (1.f / (1.f + expf(-gv[j]))) * uv[j];
-        *reinterpret_cast<uint4 *>(o + i) = pack8(gv);
+        row_store8(o + i, gv);
     }
 }
 
@@ -494,10 +492,14 @@ extern "C" int kva_silu_mul(void *out, const void *gate_up, int rows, int inter,
     KVA_REQUIRE(rows >= 0 && inter > 0, "silu_mul: bad sizes");
     KVA_REQUIRE(rows <= 65535, "silu_mul: at most 65535 rows per call, got %d", rows);
     if (rows == 0) return KVA_OK;
-    if (dtype == KVA_BF16 && inter % 8 == 0) {
-        int vbx = (inter / 8 + 255) / 256;
-        hipLaunchKernelGGL(silu_mul_vec_kernel, dim3(vbx, rows), dim3(256), 0, stream, (bf16_t *)out,
-                           (const bf16_t *)gate_up, inter);
+    // fp32: 2,048 rows of 2,048 / 8,192 12.6 / 41.8 -> 11.3 / 36.2 us with 32 bytes a thread, 517 rows 4.3 / 12.7 -> 4.2 / 11.6; 64 rows
+    // of 2,048 2.1 -> 2.3, so a few go element by element, over more units.
+    if (inter % 8 == 0 && (dtype == KVA_BF16 || (dtype == KVA_F32 && (((uintptr_t)out | (uintptr_t)gate_up) & 15) == 0 && (long long)rows * inter >= 1 << 20))) {
+        const dim3 vgrid((inter / 8 + 255) / 256, rows);
+        if (dtype == KVA_BF16)
+            hipLaunchKernelGGL(silu_mul_vec_kernel<bf16_t>, vgrid, dim3(256), 0, stream, (bf16_t *)out, (const bf16_t *)gate_up, inter);
+        else
+            hipLaunchKernelGGL(silu_mul_vec_kernel<float>, vgrid, dim3(256), 0, stream, (float *)out, (const float *)gate_up, inter);
         KVA_CHECK_LAUNCH("silu_mul");
         return KVA_OK;
     }

@@ -17,6 +17,7 @@
 // slot skips the write.
 #include "common.h"
 #include "kv_layout.h"
+#include <algorithm>
 
 template <typename T>
 __global__ void rope_kv_write_kernel(T *__restrict__ qkv, T *__restrict__ k_cache,
@@ -88,34 +89,39 @@ __global__ void rope_kv_write_kernel(T *__restrict__ qkv, T *__restrict__ k_cach
     }
 }
 
-// bf16, full rotary (rot_dim == head_dim), head_dim a multiple of 16: a thread rotates 8 pairs at a
-// time with 16-byte loads and stores.
-__device__ inline void rk_unpack8(const uint4 &v, float (&f)[8]) {
-    const uint32_t w[4] = {v.x, v.y, v.z, v.w};
+// Full rotary (rot_dim == head_dim), head_dim a multiple of 16: a thread rotates as many pairs at a time as 16 bytes hold elements.
+// Few tokens: a token's heads go to several workgroups (3 tokens of 32 + 2 x 8 heads of 64 / 128, fp32 2.6 / 2.6 us, pair by
+// pair in one workgroup 4.5 / 7.2; bf16 3.0 / 3.1, in one workgroup 3.1 / 4.1).
+template <typename T>
+struct RopeVec {
+    static constexpr int N = 16 / sizeof(T);
+    __device__ static inline void load(const T *p, float (&f)[N]) {
+        const uint4 v = *reinterpret_cast<const uint4 *>(p);
+        const uint32_t w[4] = {v.x, v.y, v.z, v.w};
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-        f[2 * i] = bf16_bits_to_float((uint16_t)(w[i] & 0xffffu));
-        f[2 * i + 1] = bf16_bits_to_float((uint16_t)(w[i] >> 16));
+        for (int i = 0; i < N; ++i)
+            f[i] = __uint_as_float(N == 4 ? w[i % 4] : i % 2 ? w[i / 2] & 0xffff0000u : w[i / 2] << 16);
     }
-}
-
-__device__ inline uint4 rk_pack8(const float (&f)[8]) {
-    uint32_t w[4];
+    __device__ static inline void store(T *p, const float (&f)[N]) {
+        uint32_t w[4];
 #pragma unroll
-    for (int i = 0; i < 4; ++i)
-        w[i] = (uint32_t)float_to_bf16_bits(f[2 * i]) | ((uint32_t)float_to_bf16_bits(f[2 * i + 1]) << 16);
-    return make_uint4(w[0], w[1], w[2], w[3]);
-}
+        for (int i = 0; i < 4; ++i)
+            w[i] = N == 4 ? __float_as_uint(f[i % N])
+                          : (uint32_t)float_to_bf16_bits(f[2 * i % N]) | ((uint32_t)float_to_bf16_bits(f[(2 * i + 1) % N]) << 16);
+        *reinterpret_cast<uint4 *>(p) = make_uint4(w[0], w[1], w[2], w[3]);
+    }
+};
 
-__global__ void rope_kv_write_vec_kernel(bf16_t *__restrict__ qkv, bf16_t *__restrict__ k_cache,
-                                         bf16_t *__restrict__ v_cache, const float *__restrict__ cos_table,
-                                         const float *__restrict__ sin_table,
+template <typename T>
+__global__ void rope_kv_write_vec_kernel(T *__restrict__ qkv, T *__restrict__ k_cache, T *__restrict__ v_cache,
+                                         const float *__restrict__ cos_table, const float *__restrict__ sin_table,
                                          const int *__restrict__ positions,
                                          const int *__restrict__ slot_mapping, int num_q_heads,
                                          int num_kv_heads, int head_dim, int page_size, int write_cache) {
-    const int t = blockIdx.x;
+    constexpr int N = RopeVec<T>::N;
+    const int t = blockIdx.x, first = blockIdx.y * blockDim.x + threadIdx.x, step = gridDim.y * blockDim.x;
     const int row_width = (num_q_heads + 2 * num_kv_heads) * head_dim;
-    bf16_t *row = qkv + (size_t)t * row_width;
+    T *row = qkv + (size_t)t * row_width;
     const int pos = positions[t];
     const int half = head_dim / 2;
     const float *cs = cos_table + (size_t)pos * half;
@@ -124,37 +130,39 @@ __global__ void rope_kv_write_vec_kernel(bf16_t *__restrict__ qkv, bf16_t *__res
     if (write_cache) slot = slot_mapping[t];
     const int page = slot >= 0 ? slot / page_size : 0;
     const int off = slot >= 0 ? slot % page_size : 0;
-    const int chunks = half / 8;
+    const int chunks = half / N;
     const int qk_heads = num_q_heads + num_kv_heads;
-    for (int w = threadIdx.x; w < qk_heads * chunks; w += blockDim.x) {
-        const int head = w / chunks, p0 = (w % chunks) * 8;
+    for (int w = first; w < qk_heads * chunks; w += step) {
+        const int head = w / chunks, p0 = (w % chunks) * N;
         if (head >= num_q_heads && slot < 0) continue;
-        bf16_t *h = row + (size_t)head * head_dim;
-        float x1[8], x2[8], c[8], s[8], o1[8], o2[8];
-        rk_unpack8(*reinterpret_cast<const uint4 *>(h + p0), x1);
-        rk_unpack8(*reinterpret_cast<const uint4 *>(h + half + p0), x2);
-        const float4 c0 = *reinterpret_cast<const float4 *>(cs + p0), c1 = *reinterpret_cast<const float4 *>(cs + p0 + 4);
-        const float4 s0 = *reinterpret_cast<const float4 *>(sn + p0), s1 = *reinterpret_cast<const float4 *>(sn + p0 + 4);
-        c[0] = c0.x; c[1] = c0.y; c[2] = c0.z; c[3] = c0.w; c[4] = c1.x; c[5] = c1.y; c[6] = c1.z; c[7] = c1.w;
-        s[0] = s0.x; s[1] = s0.y; s[2] = s0.z; s[3] = s0.w; s[4] = s1.x; s[5] = s1.y; s[6] = s1.z; s[7] = s1.w;
+        T *h = row + (size_t)head * head_dim;
+        float x1[N], x2[N], c[N], s[N], o1[N], o2[N];
+        RopeVec<T>::load(h + p0, x1);
+        RopeVec<T>::load(h + half + p0, x2);
 #pragma unroll
-        for (int j = 0; j < 8; ++j) {
+        for (int j = 0; j < N; j += 4) {
+            const float4 cv = *reinterpret_cast<const float4 *>(cs + p0 + j), sv = *reinterpret_cast<const float4 *>(sn + p0 + j);
+            c[j] = cv.x; c[j + 1] = cv.y; c[j + 2] = cv.z; c[j + 3] = cv.w;
+            s[j] = sv.x; s[j + 1] = sv.y; s[j + 2] = sv.z; s[j + 3] = sv.w;
+        }
+#pragma unroll
+        for (int j = 0; j < N; ++j) {
             o1[j] = x1[j] * c[j] - x2[j] * s[j];
             o2[j] = x1[j] * s[j] + x2[j] * c[j];
         }
         if (head >= num_q_heads) {
-            // (head_dim is a multiple of 16 here: p0 and half + p0 are whole chunks of 8)
-            bf16_t *dst = k_cache + ((size_t)page * num_kv_heads + (head - num_q_heads)) * page_size * head_dim;
-            *reinterpret_cast<uint4 *>(dst + kva_k_at(off, p0, page_size, 8)) = rk_pack8(o1);
-            *reinterpret_cast<uint4 *>(dst + kva_k_at(off, half + p0, page_size, 8)) = rk_pack8(o2);
+            // (head_dim is a multiple of 16 here: chunks of 8, of which p0 and half + p0 start one or its second half)
+            T *dst = k_cache + ((size_t)page * num_kv_heads + (head - num_q_heads)) * page_size * head_dim;
+            RopeVec<T>::store(dst + kva_k_at(off, p0, page_size, 8), o1);
+            RopeVec<T>::store(dst + kva_k_at(off, half + p0, page_size, 8), o2);
         } else {
-            *reinterpret_cast<uint4 *>(h + p0) = rk_pack8(o1);
-            *reinterpret_cast<uint4 *>(h + half + p0) = rk_pack8(o2);
+            RopeVec<T>::store(h + p0, o1);
+            RopeVec<T>::store(h + half + p0, o2);
         }
     }
     if (slot >= 0) {
-        const bf16_t *v = row + (size_t)(num_q_heads + num_kv_heads) * head_dim;
-        for (int w = threadIdx.x; w < num_kv_heads * head_dim; w += blockDim.x) {
+        const T *v = row + (size_t)(num_q_heads + num_kv_heads) * head_dim;
+        for (int w = first; w < num_kv_heads * head_dim; w += step) {
             const int kvh = w / head_dim, j = w % head_dim;
             v_cache[(((size_t)page * num_kv_heads + kvh) * head_dim + j) * page_size + off] = v[w];
         }
@@ -175,10 +183,16 @@ extern "C" int kva_rope_kv_write(void *qkv, void *k_cache, void *v_cache, const 
                 "rope_kv_write: cache write asked for without cache, slots or page size");
     if (tokens == 0) return KVA_OK;
     dim3 grid(tokens), block(256);
-    if (dtype == KVA_BF16 && cos_table && rot_dim == head_dim && head_dim % 16 == 0) {
-        hipLaunchKernelGGL(rope_kv_write_vec_kernel, grid, block, 0, stream, (bf16_t *)qkv,
-                           (bf16_t *)k_cache, (bf16_t *)v_cache, cos_table, sin_table, positions,
-                           slot_mapping, num_q_heads, num_kv_heads, head_dim, page_size, write_cache);
+    const uintptr_t all = (uintptr_t)qkv | (uintptr_t)k_cache | (uintptr_t)cos_table | (uintptr_t)sin_table;
+    if (cos_table && rot_dim == head_dim && head_dim % 16 == 0 && (dtype == KVA_BF16 || (dtype == KVA_F32 && all % 16 == 0))) {
+        const int vectors = (num_q_heads + num_kv_heads) * head_dim / 2 / (dtype == KVA_BF16 ? 8 : 4);
+        const dim3 vgrid(tokens, tokens <= 64 ? std::min(65535, (std::max(vectors, num_kv_heads * head_dim) + 255) / 256) : 1);
+        if (dtype == KVA_BF16)
+            hipLaunchKernelGGL(rope_kv_write_vec_kernel<bf16_t>, vgrid, block, 0, stream, (bf16_t *)qkv, (bf16_t *)k_cache, (bf16_t *)v_cache,
+                               cos_table, sin_table, positions, slot_mapping, num_q_heads, num_kv_heads, head_dim, page_size, write_cache);
+        else
+            hipLaunchKernelGGL(rope_kv_write_vec_kernel<float>, vgrid, block, 0, stream, (float *)qkv, (float *)k_cache, (float *)v_cache,
+                               cos_table, sin_table, positions, slot_mapping, num_q_heads, num_kv_heads, head_dim, page_size, write_cache);
         KVA_CHECK_LAUNCH("rope_kv_write");
         return KVA_OK;
     }

@@ -1,0 +1,82 @@
+"""Norms, activations and rotations over rows of 16-byte vectors: the edges of their launches, against 64 bits."""
+import pytest
+import torch
+
+from kv_cache_optimization_for_llm_amd.ops import kernels as K
+
+pytestmark = pytest.mark.gpu
+D = torch.float64
+
+
+def made(shape, dtype, g, shift=0):
+    """A tensor that starts `shift` elements behind an aligned address."""
+    t = torch.randn(shape, generator=g).to(dtype)
+    flat = torch.empty(t.numel() + shift, dtype=dtype, device="cuda")
+    out = flat[shift:].view(shape)
+    out.copy_(t)
+    return out
+
+
+def close(got, want):
+    """fp32 sums of up to 65,536 squares and a handful of roundings, then one of the result."""
+    tol = 2.0 ** -8 if got.dtype == torch.bfloat16 else 1e-5
+    assert (got.to(D) - want).abs().max() <= tol * max(1e-30, float(want.abs().max()))
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("w_dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("rows, width, shift", [(1, 8, 0), (3, 2040, 0), (300, 2048, 0), (2, 2056, 0), (300, 2056, 0), (300, 6152, 0), (2, 8200, 0),
+                                                (2, 40000, 0), (1, 65536, 0), (1, 65544, 0), (3, 2048, 1), (3, 100, 0)])
+def test_rmsnorm(rows, width, shift, w_dtype, dtype, gpu):
+    g = torch.Generator().manual_seed(width)
+    shift = shift if dtype == torch.float32 else 0          # (bf16 rows are aligned by what makes them)
+    w = made((width,), w_dtype, g)
+    for added in (False, True):
+        x, d = made((rows, width), dtype, g, shift), made((rows, width), dtype, g)
+        want = x.to(D) if not added else (x.float() + d.float()).to(dtype).to(D)
+        out = torch.empty((rows, width), dtype=dtype, device="cuda")
+        K.rmsnorm(x, w, 1e-5, out, delta=d if added else None)
+        assert torch.equal(x.to(D), want)
+        normed = want / torch.sqrt((want * want).mean(1, keepdim=True) + 1e-5) * w.to(D)
+        close(out, normed)
+        idx = torch.tensor([rows - 1, 0], dtype=torch.int32, device="cuda")
+        K.rmsnorm(x, w, 1e-5, out2 := torch.empty((2, width), dtype=dtype, device="cuda"), row_idx=idx)
+        close(out2, normed[idx.long()])
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("rows, inter, shift", [(1, 8, 0), (3, 2040, 0), (515, 2040, 0), (515, 2048, 1), (2, 13, 0)])
+def test_silu_mul(rows, inter, shift, dtype, gpu):
+    g = torch.Generator().manual_seed(inter)
+    gu = made((rows, 2 * inter), dtype, g, shift if dtype == torch.float32 else 0)
+    out = K.silu_mul(gu, torch.empty((rows, inter), dtype=dtype, device="cuda"))
+    z = gu.to(D)
+    close(out, z[:, :inter] * torch.sigmoid(z[:, :inter]) * z[:, inter:])
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("tokens, nq, nkv, d, page", [(1, 2, 1, 16, 16), (3, 32, 8, 64, 16), (64, 5, 3, 48, 8), (65, 4, 4, 128, 16), (2, 3, 1, 24, 4), (1, 64, 64, 256, 16)])
+def test_rope_and_cache(tokens, nq, nkv, d, page, dtype, gpu):
+    g = torch.Generator().manual_seed(tokens * d)
+    pages = (tokens + page - 1) // page + 1
+    cos, sin = (torch.randn(100, d // 2, generator=g).cuda() for _ in range(2))
+    pos = torch.randint(0, 100, (tokens,), generator=g).int().cuda()
+    slots = torch.randperm(pages * page, generator=g)[:tokens].int()
+    slots[tokens // 2] = -1 if tokens > 1 else slots[0]
+    qkv = made((tokens, (nq + 2 * nkv) * d), dtype, g)
+    x = qkv.to(D).view(tokens, nq + 2 * nkv, d)
+    kc = torch.zeros((pages, *K.k_page_shape(nkv, d)[:2], page, K.k_chunk(d)), dtype=dtype, device="cuda")
+    vc = torch.zeros((pages, nkv, d, page), dtype=dtype, device="cuda")
+    K.rope_kv_write(qkv, pos, nq, nkv, d, cos, sin, kc, vc, slots.cuda(), page)
+    c, s = cos[pos.long()].to(D)[:, None], sin[pos.long()].to(D)[:, None]
+    u, v = x[..., :d // 2], x[..., d // 2:]
+    turned = torch.cat([u * c - v * s, v * c + u * s], -1)
+    close(qkv.view(tokens, -1, d)[:, :nq], turned[:, :nq])
+    keys = K.pages_to_keys(kc).transpose(1, 2).reshape(pages * page, nkv, d)
+    values = vc.permute(0, 3, 1, 2).reshape(pages * page, nkv, d)
+    on = slots >= 0
+    close(keys[slots[on].long()], turned[on][:, nq:nq + nkv])
+    assert torch.equal(values[slots[on].long()].to(D), x[on][:, nq + nkv:])
+    rest = torch.ones(pages * page, dtype=torch.bool)
+    rest[slots[on].long()] = False
+    assert not keys[rest].any() and not values[rest].any()
