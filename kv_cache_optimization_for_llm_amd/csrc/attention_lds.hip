@@ -6,11 +6,13 @@
 // vector memory path is what it waits for (halving it nearly halves its time).  Here a workgroup
 // of four wavefronts takes 128 consecutive query rows of one request and kv head (row =
 // token * G + head_in_group, as there), each wavefront 32 of them, and every 32-key block is
-// copied from the pages to LDS once for all four: 16 bytes per thread for K and for V^T, in the
-// pages' own layout, rows padded so that the operand reads do not collide on the 32 banks (K rows
-// 16 bytes longer, V^T rows 72 bytes apart).  The copies of
-// block i+1 travel (global -> registers) while block i is computed, are written to the other
-// half of LDS afterwards, and one barrier per block separates the two.
+// copied from the pages to LDS once for all four, in the pages' own layout: two wavefronts a page of K each, two a page of
+// V^T.  That layout is what operands are read in without a bank met twice: 16 keys' chunks of 8 elements of K next to each other
+// are the 64 lanes' 16 bytes in order, 16 value dimensions of 16 keys their 8 bytes.  So the copies need no stop in registers
+// (buffer loads to LDS); LDS_STAGES - 1 blocks are on their way while one is computed, and the page of the one after those is
+// looked up.  One barrier a block says that everybody's share of it has arrived and that the block before is read.
+// One block ahead through registers, 8,190 tokens, 32 heads of 128 over 8: 762 us, 145 of
+// them for that staging; 577 now (0.95 PFLOP/s of the visible half).  2,048 tokens 85 -> 77; 32 heads of 64, 8,190 tokens 398 -> 341.
 //
 // The arithmetic per block is the other kernel's: S^T = K Q^T, online softmax in fp32 per query
 // row with a lazily re-based reference, O^T += V^T P^T with P taken from the registers S^T came
@@ -24,26 +26,25 @@
 // from the cache.
 #include "common.h"
 #include "attention_frag.h"
+#include "lds_product.h"
 #include "kv_layout.h"
 #include <math.h>
 #include <type_traits>
 
+#define LDS_STAGES 3
+#define LDS_BLOCKS 512         // blocks of 32 keys whose pages stand in LDS at a time
+
 template <int D>
 struct LdsGeom {
-    static constexpr int KROW = D * 2 + 16;          // bytes per key row (D bf16 + pad)
-    static constexpr int VROW = 32 * 2 + 8;          // bytes per value-dimension row (32 keys + pad)
-    static constexpr int KBYTES = 32 * KROW;
-    static constexpr int VBYTES = D * VROW;
-    static constexpr int CHUNKS = 4 * D;             // 16-byte chunks of a K tile (and of a V^T tile)
-    static constexpr int PER_THREAD = (CHUNKS + 255) / 256;
-    static constexpr int SB = 1;                     // 32-key blocks per stage (per barrier); 2 measured slower
-    static constexpr int BLOCK_BYTES = KBYTES + VBYTES;
-    static constexpr int STAGE_BYTES = SB * BLOCK_BYTES;
+    static constexpr int PAGE = 16 * D;                  // elements of a page of K or V^T (one kv head)
+    static constexpr int LOADS = D / 32;                 // of 1 KiB a wavefront and block
+    static constexpr int STAGE = 4 * PAGE;               // K of both pages, then V^T of both
 };
+typedef __bf16 b16x4 __attribute__((ext_vector_type(4)));
 
 template <int D>
 __device__ __forceinline__ void
-attention_lds_item(char *lds, bf16_t *__restrict__ out, float *__restrict__ part_o, float *__restrict__ part_ml,
+attention_lds_item(bf16_t *lds, bf16_t *__restrict__ out, float *__restrict__ part_o, float *__restrict__ part_ml,
                    const bf16_t *__restrict__ q, int q_row_stride,
                    const bf16_t *__restrict__ k_cache, const bf16_t *__restrict__ v_cache,
                    const int *__restrict__ block_table, int max_blocks,
@@ -129,108 +130,66 @@ attention_lds_item(char *lds, bf16_t *__restrict__ out, float *__restrict__ part
         for (int dt = 0; dt < NDT; ++dt) o[rt][dt] = f32x4{0.f, 0.f, 0.f, 0.f};
     }
 
-    // ---- copies page -> registers -> LDS.  Chunk c of the K tile is 16 bytes of key c % 16 of page c / 2D, dims 8 (c % 2D) / 16 ..;
-    // chunk c of the V^T tile is 8 keys of value dimension (c % 2D) / 2 in page c / 2D.  A tile
-    // outside the keys the workgroup needs is redirected to the nearest needed one (its page is
-    // certainly mapped); its scores are masked away.
-    // (named registers, not arrays: as arrays the compiler kept them in scratch memory for head sizes
-    // with two chunks per thread, a store and a load of 64 bytes per thread and block)
-    static_assert(Geo::SB == 1 && Geo::PER_THREAD <= 2, "the staging registers below are two chunks of one block");
-    uint4 stage_k0, stage_k1, stage_v0, stage_v1;
-    // which of the block's two pages a thread's chunk lies in is the same for a whole wavefront
-    // (said explicitly, so that the page's address stays scalar arithmetic); its place inside the
-    // page never changes
-    int k_sel[Geo::PER_THREAD], v_sel[Geo::PER_THREAD], k_off[Geo::PER_THREAD], v_off[Geo::PER_THREAD];
-#pragma unroll
-    for (int i = 0; i < Geo::PER_THREAD; ++i) {
-        const int c = tid + i * 256;
-        // K pages are [D / 8][16 keys][8] (kv_layout.h): chunk c of the tile is 16 bytes number c % 2D of page c / 2D
-        k_sel[i] = __builtin_amdgcn_readfirstlane(c / (2 * D));
-        k_off[i] = (c % (2 * D)) * 8;
-        const int rem = c % (2 * D);
-        v_sel[i] = __builtin_amdgcn_readfirstlane(c / (2 * D));
-        v_off[i] = (rem >> 1) * 16 + (rem & 1) * 8;
-    }
-    auto fetch = [&](int b, int kstart) {
-        int pg[2];
-#pragma unroll
-        for (int t = 0; t < 2; ++t) {
-            int tile0 = kstart + t * 16;
-            tile0 = tile0 < lo_tile ? lo_tile : (tile0 > hi_tile ? hi_tile : tile0);
-            pg[t] = bt[__builtin_amdgcn_readfirstlane(tile0 >> 4)];
-        }
-        auto chunk = [&](int i, uint4 &k, uint4 &v) {
-            const int c = tid + i * 256;
-            if (Geo::CHUNKS % 256 == 0 || c < Geo::CHUNKS) {
-                const size_t kpage = ((size_t)(k_sel[i] ? pg[1] : pg[0]) * num_kv_heads + kvh) * (size_t)(16 * D);
-                k = *reinterpret_cast<const uint4 *>(k_cache + kpage + k_off[i]);
-                const size_t vpage = ((size_t)(v_sel[i] ? pg[1] : pg[0]) * num_kv_heads + kvh) * (size_t)(16 * D);
-                v = *reinterpret_cast<const uint4 *>(v_cache + vpage + v_off[i]);
-            }
-        };
-        chunk(0, stage_k0, stage_v0);
-        if (Geo::PER_THREAD > 1) chunk(1, stage_k1, stage_v1);
+    // ---- copies page -> LDS: a wavefront's page of a block (K of the first, of the second, V^T of the first, of the second).  A tile
+    // outside the keys the workgroup needs is redirected to the nearest needed one (its page is certainly mapped); its scores are
+    // masked away.
+    const int wave_s = __builtin_amdgcn_readfirstlane(wave);
+    const bf16_t *cache = wave_s < 2 ? k_cache : v_cache;
+    bf16_t *pages = lds + LDS_STAGES * Geo::STAGE;
+    auto page_of = [&](int block) {         // (of those that stand in LDS; read as bf16 like the operands)
+        union { b16x2 v; int i; } x;
+        x.v = *reinterpret_cast<const b16x2 *>(pages + 2 * (2 * min(block, LDS_BLOCKS - 1) + (wave_s & 1)));
+        return x.i;
     };
-    auto stash = [&](int b, char *buf) {
-        auto chunk = [&](int i, const uint4 &k, const uint4 &v) {
-            const int c = tid + i * 256;
-            if (Geo::CHUNKS % 256 == 0 || c < Geo::CHUNKS) {
-                const int key = (c / (2 * D)) * 16 + (c & 15), kc = (c % (2 * D)) >> 4;     // the page's chunk order: [dim / 8][key]
-                *reinterpret_cast<uint4 *>(buf + key * Geo::KROW + kc * 16) = k;
-                const int t = c / (2 * D), rem = c % (2 * D);
-                // rows of 72 bytes: 18 banks apart, so that the 16 lanes of an 8-byte operand read (rows r = 0..15
-                // of one tile) meet 16 different pairs of the 32 banks; the price is two 8-byte writes here
-                char *vp = buf + Geo::KBYTES + (rem >> 1) * Geo::VROW + (t * 16 + (rem & 1) * 8) * 2;
-                *reinterpret_cast<uint2 *>(vp) = make_uint2(v.x, v.y);
-                *reinterpret_cast<uint2 *>(vp + 8) = make_uint2(v.z, v.w);
-            }
-        };
-        chunk(0, stage_k0, stage_v0);
-        if (Geo::PER_THREAD > 1) chunk(1, stage_k1, stage_v1);
+    // V^T: of every 16 value dimensions first their first 8 keys, then the others, 16 bytes each
+    const int lane_at = wave_s < 2 ? 16 * lane : (lane >> 5) * 512 + r * 32 + (g & 1) * 16;
+    auto fetch = [&](int slot, int page_v) {
+        const int page = __builtin_amdgcn_readfirstlane(page_v);
+        const Buffer from = buffer_at(cache + ((size_t)page * num_kv_heads + kvh) * Geo::PAGE, Geo::PAGE * sizeof(bf16_t));
+#pragma unroll
+        for (int i = 0; i < Geo::LOADS; ++i)
+            buffer_to_lds(from, lane_at, i * 1024, lds + slot * Geo::STAGE + wave_s * Geo::PAGE + i * 512);
     };
 
     const float scale2 = scale * 1.44269504088896340736f;   // exp(x * scale) = exp2(x * scale * log2 e)
     constexpr float REBASE = 8.f;
     const float rebase_raw = REBASE / scale2;
 
-    auto compute_as = [&](auto masked_tag, const char *buf, int kstart) {
+    auto compute_as = [&](auto masked_tag, const bf16_t *buf, int kstart) {
         constexpr bool MASKED = decltype(masked_tag)::value;
         // operands from LDS: K: lane (r, g) holds K[key t*16 + r][ks*32 + g*8 ..]; V^T: lane (r, g)
-        // holds V^T[dt*16 + r][keys t*16 + 4g .. +3] for both tiles of the block
-        Frag8 kf[2][NKS], vf[NDT];
+        // holds V^T[dt*16 + r][keys t*16 + 4g .. +3] for both tiles of the block.  (Read as vectors of bf16: the compiler then knows
+        // that no copy on its way writes what is read here, of which the barrier makes sure, and does not wait for all of them.)
+        Frag8 vf[NDT];
+        auto values = [&](int dt) {
+            union { b16x4 v; uint2 u2; } x[2];
 #pragma unroll
-        for (int t = 0; t < 2; ++t)
-#pragma unroll
-            for (int ks = 0; ks < NKS; ++ks)
-                kf[t][ks].u4 = *reinterpret_cast<const uint4 *>(buf + (t * 16 + r) * Geo::KROW + (ks * 32 + g * 8) * 2);
-#pragma unroll
-        for (int dt = 0; dt < NDT; ++dt)
-#pragma unroll
-            for (int t = 0; t < 2; ++t)
-                vf[dt].u2[t] = *reinterpret_cast<const uint2 *>(buf + Geo::KBYTES + (dt * 16 + r) * Geo::VROW + (t * 16 + 4 * g) * 2);
-
-        // Behind the workgroup's last key a block holds whatever the page held before (or the nearest
-        // needed tile, for a redirected one): P is zero there, and the values are made zero too, so
-        // that nothing non-finite left in a page can reach this request.
-        if (MASKED && kstart + 31 > g_hi) {
-            const int n0 = g_hi + 1 - (kstart + 4 * g), n1 = n0 - 16;
-#pragma unroll
-            for (int dt = 0; dt < NDT; ++dt) {
-                vf[dt].u2[0] = keep_first_keys(vf[dt].u2[0], n0);
-                vf[dt].u2[1] = keep_first_keys(vf[dt].u2[1], n1);
+            for (int t = 0; t < 2; ++t) x[t].v = *reinterpret_cast<const b16x4 *>(buf + (2 + t) * Geo::PAGE + dt * 256 + (g >> 1) * 128 + r * 8 + (g & 1) * 4);
+            // Behind the workgroup's last key a block holds whatever the page held before (or the nearest
+            // needed tile, for a redirected one): P is zero there, and the values are made zero too, so
+            // that nothing non-finite left in a page can reach this request.
+            if (MASKED && kstart + 31 > g_hi) {
+                const int n0 = g_hi + 1 - (kstart + 4 * g);
+                x[0].u2 = keep_first_keys(x[0].u2, n0);
+                x[1].u2 = keep_first_keys(x[1].u2, n0 - 16);
             }
-        }
+            vf[dt].u2[0] = x[0].u2;
+            vf[dt].u2[1] = x[1].u2;
+        };
 
         f32x4 s[RT][2];
 #pragma unroll
-        for (int rt = 0; rt < RT; ++rt)
+        for (int t = 0; t < 2; ++t) {
+            Frag8 kf[NKS];
 #pragma unroll
-            for (int t = 0; t < 2; ++t) {
-                s[rt][t] = f32x4{0.f, 0.f, 0.f, 0.f};
+            for (int ks = 0; ks < NKS; ++ks) kf[ks].v = *reinterpret_cast<const b16x8 *>(buf + t * Geo::PAGE + ks * 512 + lane * 8);
 #pragma unroll
-                for (int ks = 0; ks < NKS; ++ks)
-                    s[rt][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kf[t][ks].v, qf[rt][ks].v, s[rt][t], 0, 0, 0);
-            }
+            for (int rt = 0; rt < RT; ++rt) s[rt][t] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+            for (int ks = 0; ks < NKS; ++ks)
+#pragma unroll
+                for (int rt = 0; rt < RT; ++rt) s[rt][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kf[ks].v, qf[rt][ks].v, s[rt][t], 0, 0, 0);
+        }
         float sv[RT][8], mloc[RT];
         Frag8 pf[RT];
 #pragma unroll
@@ -278,52 +237,50 @@ attention_lds_item(char *lds, bf16_t *__restrict__ out, float *__restrict__ part
                 pf[rt].p2[j / 2] = pack_bf16(p0, p1);
             }
         }
-        // Head sizes above 64: the wavefront whose products are ready goes first (head size 128,
-        // 8,192-token prompt: 807 -> 772 us; head size 64 loses 1 % by it).  A SIMD issues either a
-        // matrix-core product or a vector instruction, from whichever wavefront: timed alone, 8 products
-        // and 24 multiply-adds in one wavefront take 126 ns, the products without the multiply-adds 67 and
-        // the multiply-adds without the products 56, and given to two wavefronts of one SIMD 109; so a key
-        // block costs its products plus its softmax, however the two are interleaved.
-        if (D > 64) __builtin_amdgcn_s_setprio(1);
+        // A SIMD issues either a matrix-core product or a vector instruction, from whichever wavefront: timed alone, 8 products
+        // and 24 multiply-adds in one wavefront take 126 ns, the products without the multiply-adds 67 and the multiply-adds
+        // without the products 56, and given to two wavefronts of one SIMD 109; so a key block costs its products plus its
+        // softmax, however the two are interleaved.  (Nothing in a wavefront's priority during its products: 577 / 577 us.)
+        // Values are read a tile ahead of their products and no further (head size 128, 8,190 tokens: two tiles ahead 605 us, one
+        // 577; left to the compiler's order 613).
+        values(0);
 #pragma unroll
-        for (int rt = 0; rt < RT; ++rt) {
+        for (int dt = 0; dt < NDT; ++dt) {
+            if (dt + 1 < NDT) values(dt + 1);
+            __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-            for (int dt = 0; dt < NDT; ++dt)
+            for (int rt = 0; rt < RT; ++rt)
                 o[rt][dt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vf[dt].v, pf[rt].v, o[rt][dt], 0, 0, 0);
-            ol[rt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ones.v, pf[rt].v, ol[rt], 0, 0, 0);
         }
-        if (D > 64) __builtin_amdgcn_s_setprio(0);
+#pragma unroll
+        for (int rt = 0; rt < RT; ++rt) ol[rt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ones.v, pf[rt].v, ol[rt], 0, 0, 0);
     };
 
-    // ---- the key loop: a stage is SB blocks of 32 keys; one barrier per stage, two LDS buffers.
-    // Loads past the end are redirected inside fetch (never out of the mapped pages) and unused.
-    auto compute = [&](const char *buf, int kstart) {
-        if (wave_valid && kstart < k_end && kstart <= w_hi && kstart + 31 >= w_lo) {
+    // ---- the key loop.  Copies past the end are redirected inside page_of (never out of the mapped pages) and unused.
+    auto compute = [&](const bf16_t *buf, int kstart) {
+        if (wave_valid && kstart <= w_hi && kstart + 31 >= w_lo) {
             const bool masked = kstart < w_hi_lo || kstart + 31 > w_first_pos || !all_rows;
             if (masked) compute_as(std::true_type{}, buf, kstart);
             else compute_as(std::false_type{}, buf, kstart);
         }
     };
-#pragma unroll
-    for (int b = 0; b < Geo::SB; ++b) fetch(b, k_begin + 32 * b);
-#pragma unroll
-    for (int b = 0; b < Geo::SB; ++b) stash(b, lds + b * Geo::BLOCK_BYTES);
-    __syncthreads();
-    int which = 0;
-    for (int kstart = k_begin; kstart < k_end; kstart += 32 * Geo::SB) {
-        const bool more = kstart + 32 * Geo::SB < k_end;       // uniform over the workgroup
-        if (more) {
-#pragma unroll
-            for (int b = 0; b < Geo::SB; ++b) fetch(b, kstart + 32 * (Geo::SB + b));
-        }
-#pragma unroll
-        for (int b = 0; b < Geo::SB; ++b) compute(lds + which * Geo::STAGE_BYTES + b * Geo::BLOCK_BYTES, kstart + 32 * b);
-        if (more) {
-#pragma unroll
-            for (int b = 0; b < Geo::SB; ++b) stash(b, lds + (which ^ 1) * Geo::STAGE_BYTES + b * Geo::BLOCK_BYTES);
-        }
+    for (int k0 = k_begin; k0 < k_end; k0 += 32 * LDS_BLOCKS) {             // uniform over the workgroup
+        const int k1 = min(k_end, k0 + 32 * LDS_BLOCKS);
+        for (int i = tid; i < min(2 * LDS_BLOCKS, (k1 - k0 + 15) / 16 + 2 * LDS_STAGES); i += 256)
+            reinterpret_cast<int *>(pages)[i] = bt[min(max(k0 + 16 * i, lo_tile), hi_tile) >> 4];
         __syncthreads();
-        which ^= 1;
+#pragma unroll
+        for (int b = 0; b < LDS_STAGES - 1; ++b) fetch(b, page_of(b));
+        int slot = 0, block = LDS_STAGES - 1, page = page_of(block);
+        for (int kstart = k0; kstart < k1; kstart += 32) {
+            wait_and_meet<(LDS_STAGES - 2) * Geo::LOADS>();
+            // into the slot that was read in the turn before: every wavefront has passed the barrier since
+            fetch(slot == 0 ? LDS_STAGES - 1 : slot - 1, page);
+            page = page_of(++block);
+            compute(lds + slot * Geo::STAGE, kstart);
+            slot = slot + 1 == LDS_STAGES ? 0 : slot + 1;
+        }
+        wait_and_meet<0>();                 // nothing is on its way any more, nobody reads
     }
 
     // ---- lane (r, g) holds O[row r][dt * 16 + 4g + i]
@@ -367,7 +324,7 @@ attention_lds_body(bf16_t *__restrict__ out, float *__restrict__ part_o, float *
                    const int *__restrict__ item_meta, int num_items, int pair, int num_q_heads,
                    int num_kv_heads, float scale, int window, int splits, int keys_per_split) {
     using Geo = LdsGeom<D>;
-    __shared__ __align__(16) char lds[2 * Geo::STAGE_BYTES];
+    __shared__ __align__(16) bf16_t lds[LDS_STAGES * Geo::STAGE + 4 * LDS_BLOCKS];      // the ring, then pages
     const int kvh = blockIdx.x % num_kv_heads;
     const int w = blockIdx.x / num_kv_heads, split = blockIdx.z;
     attention_lds_item<D>(lds, out, part_o, part_ml, q, q_row_stride, k_cache, v_cache, block_table, max_blocks,
@@ -390,25 +347,19 @@ attention_lds_body(bf16_t *__restrict__ out, float *__restrict__ part_o, float *
     out, part_o, part_ml, q, q_row_stride, k_cache, v_cache, block_table, max_blocks, item_meta,   \
     num_items, pair, num_q_heads, num_kv_heads, scale, window, splits, keys_per_split
 
+// Head sizes up to 64: four wavefronts a SIMD (up to 128 registers each, no spills).
 template <int D>
-__global__ void __launch_bounds__(256) attention_lds_kernel(LDS_KERNEL_PARAMS) {
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4)))
+attention_lds_kernel_4(LDS_KERNEL_PARAMS) {
     attention_lds_body<D>(LDS_KERNEL_ARGS);
 }
 
-// Head sizes up to 64 need a few registers more than three wavefronts per SIMD leave each (168):
-// held to that, the compiler spills a handful of values, and three wavefronts instead of two are
-// worth far more than those cost (the kernel is bound by vector work the wavefronts overlap).
+// Head sizes 96 and 128: left alone the compiler takes over 300 registers, which leaves one wavefront per SIMD and nothing to
+// overlap matrix-core, vector and LDS work with.  Three (168 registers, 13 of them spilled at 128) against two without spills,
+// 8,190 tokens of 32 heads of 128: 577 against 703 us.
 template <int D>
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3)))
 attention_lds_kernel_3(LDS_KERNEL_PARAMS) {
-    attention_lds_body<D>(LDS_KERNEL_ARGS);
-}
-
-// Head sizes 96 and 128: left alone the compiler takes over 300 registers, which leaves one wavefront
-// per SIMD and nothing to overlap matrix-core, vector and LDS work with.
-template <int D>
-__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2)))
-attention_lds_kernel_2(LDS_KERNEL_PARAMS) {
     attention_lds_body<D>(LDS_KERNEL_ARGS);
 }
 
@@ -450,10 +401,10 @@ extern "C" int kva_attention_lds(void *out, float *part_o, float *part_ml, const
                        (const bf16_t *)v_cache, block_table, max_blocks, item_meta, num_items, pair, \
                        num_q_heads, num_kv_heads, scale, window, splits, keys_per_split)
     switch (head_dim) {
-    case 32: LAUNCH(attention_lds_kernel_3, 32); break;
-    case 64: LAUNCH(attention_lds_kernel_3, 64); break;
-    case 96: LAUNCH(attention_lds_kernel_2, 96); break;
-    default: LAUNCH(attention_lds_kernel_2, 128); break;
+    case 32: LAUNCH(attention_lds_kernel_4, 32); break;
+    case 64: LAUNCH(attention_lds_kernel_4, 64); break;
+    case 96: LAUNCH(attention_lds_kernel_3, 96); break;
+    default: LAUNCH(attention_lds_kernel_3, 128); break;
     }
 #undef LAUNCH
     KVA_CHECK_LAUNCH("attention_lds");
