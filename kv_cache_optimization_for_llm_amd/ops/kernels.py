@@ -993,14 +993,15 @@ def latent_prompt(q: torch.Tensor, cache: torch.Tensor, w: torch.Tensor, out: to
         if gates.shape != ((T, heads, vdim) if element else (T, heads)) or gates.dtype != q.dtype or gates.stride(-1) != 1:
             raise KernelError(f"latent_prompt: gates {tuple(gates.shape)} do not fit {T} rows of {heads} heads")
         gate = [_dev(gates, "gates", contiguous=False), gates.stride(0), gates.stride(1) if element else 1, 1 if element else 0]
-    kv = torch.empty((entries * int(context), heads * (dim + vdim)), dtype=q.dtype, device=q.device)
-    turned = torch.empty((entries * int(context), rot), dtype=q.dtype, device=q.device)
+    context = (int(context) + 31) // 32 * 32          # (the workspace lies in tiles of 32 keys)
+    kv = torch.empty((entries * context, heads * (dim + vdim)), dtype=q.dtype, device=q.device)
+    turned = torch.empty((entries * context, rot), dtype=q.dtype, device=q.device)
     check(hip_lib().kva_latent_prompt(
         _dev(out, "out"), _dev(q, "q", contiguous=False), q.stride(0), q.stride(1), _dev(cache, "cache"), _dev(w, "w"), _dev(kv, "kv"),
         _dev(turned, "turned"), _dev(block_table, "block_table", torch.int32), block_table.shape[1],
         _dev(entry_seat, "entry_seat", torch.int32), _dev(entry_q_start, "entry_q_start", torch.int32),
         _dev(entry_start_pos, "entry_start_pos", torch.int32), entries, _dev(cos, "cos", torch.float32), _dev(sin, "sin", torch.float32),
-        1 if interleaved else 0, _opt(sinks, "sinks", torch.float32), *gate, cache.shape[1], heads, rank, int(context), int(longest),
+        1 if interleaved else 0, _opt(sinks, "sinks", torch.float32), *gate, cache.shape[1], heads, rank, context, int(longest),
         float(scale), _stream()), "latent_prompt")
     return out
 
