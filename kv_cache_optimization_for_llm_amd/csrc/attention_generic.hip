@@ -22,6 +22,7 @@
 #include "common.h"
 #include "kv_layout.h"
 #include <math.h>
+#include <type_traits>
 
 #define ATTN_MAX_HEAD_DIM 256
 
@@ -207,12 +208,161 @@ attention_rowwise_kernel(T *__restrict__ out, const T *__restrict__ q, int q_row
     }
 }
 
+// The same for few rows: FEW_BLOCKS wavefronts a token and head, a block of 64 keys each at a time.  Everything of a block is asked for, and its
+// scores and exponentials are made, beside the other blocks'; what stays one after the other are the sums over the values, whose
+// additions keep their order, handed on through LDS from block to block.  So bits are those of the kernel above.
+#define FEW_BLOCKS 4
+#define FEW_MAX_DIM 128
+
+// VC: rounds of 64 value elements
+template <typename T, int VC>
+__global__ void __launch_bounds__(KVA_WAVE * FEW_BLOCKS)
+attention_few_kernel(T *__restrict__ out, const T *__restrict__ q, int q_row_stride, const T *__restrict__ k_cache,
+                     const T *__restrict__ v_cache, const int *__restrict__ block_table, int max_blocks, const int *__restrict__ tok_seat,
+                     const int *__restrict__ tok_pos, int num_q_heads, int num_kv_heads, int head_dim, int value_dim, int page_size,
+                     float scale, int window, int keep_first, int chunk, const float *__restrict__ sinks) {
+    __shared__ __attribute__((aligned(16))) float q_s[FEW_MAX_DIM], p_s[FEW_BLOCKS][KVA_WAVE];
+    __shared__ long long voff_s[FEW_BLOCKS][KVA_WAVE];
+    __shared__ float max_s[FEW_BLOCKS], sum_s[FEW_BLOCKS], acc_s[VC * KVA_WAVE];
+
+    const int t = blockIdx.x, qh = blockIdx.y, tid = threadIdx.x, lane = tid % KVA_WAVE;
+    const int wave = __builtin_amdgcn_readfirstlane(tid / KVA_WAVE), kvh = qh / (num_q_heads / num_kv_heads);
+    const int pos = tok_pos[t];
+    const int *bt = block_table + (size_t)tok_seat[t] * max_blocks;
+    const T *qrow = q + (size_t)t * q_row_stride + (size_t)qh * head_dim;
+    if (tid < head_dim) q_s[tid] = to_float(qrow[tid]);
+    if (tid < VC * KVA_WAVE) acc_s[tid] = 0.f;
+    __syncthreads();
+
+    const int lo = kva_first_visible(pos, window, chunk), end = pos / KVA_WAVE + 1;
+    // a block with no visible key: behind the window and past the kept first positions, or past the token
+    auto visible = [&](int kb) { return kb < end && !(kb * KVA_WAVE + KVA_WAVE <= lo && kb * KVA_WAVE >= keep_first); };
+    float m = -INFINITY, l = 0.f;
+    for (int base = keep_first > 0 ? 0 : lo / KVA_WAVE; base < end; base += FEW_BLOCKS) {       // uniform over the workgroup
+        if ((base + FEW_BLOCKS) * KVA_WAVE <= lo && base * KVA_WAVE >= keep_first) continue;
+        const int kb = base + wave;
+        const bool on = visible(kb);
+        const int key = kb * KVA_WAVE + lane;
+        const bool valid = on && key <= pos && (key >= lo || key < keep_first);
+        const unsigned long long seen = __ballot(valid);
+        float s = -INFINITY, v[VC][16][4];
+        if (on) {
+            // (four keys of a page together; where none of them is visible, the first visible one's place is read and not used)
+            const int group = (seen >> (lane & ~3)) & 15 ? lane : (__ffsll(seen) - 1) & ~3;
+            const int page = bt[key <= pos ? key / page_size : pos / page_size], vkey = kb * KVA_WAVE + group;
+            voff_s[wave][lane] = ((long long)bt[vkey / page_size] * num_kv_heads + kvh) * (long long)value_dim * page_size + vkey % page_size;
+            const T *kpage = k_cache + ((long long)page * num_kv_heads + kvh) * page_size * (long long)head_dim;
+            const int krow = key % page_size, kc = kva_k_chunk(head_dim);
+            float kv[16][4];
+            auto keys = [&](int j0) {
+#pragma unroll
+                for (int j = 0; j < 16; ++j) Vec4<T>::load(kpage + kva_k_at(krow, j0 + 4 * j, page_size, kc), kv[j]);
+            };
+            float dot = 0.f;
+            auto score = [&](int j0) {
+#pragma unroll
+                for (int j = 0; j < 16; ++j) {
+                    const float4 qv = *reinterpret_cast<const float4 *>(&q_s[j0 + 4 * j]);
+                    dot = __builtin_fmaf(qv.x, kv[j][0], dot);
+                    dot = __builtin_fmaf(qv.y, kv[j][1], dot);
+                    dot = __builtin_fmaf(qv.z, kv[j][2], dot);
+                    dot = __builtin_fmaf(qv.w, kv[j][3], dot);
+                }
+            };
+            keys(0);
+            __builtin_amdgcn_wave_barrier();
+#pragma unroll
+            for (int c = 0; c < VC; ++c) {
+                const T *vcol = v_cache + (long long)min(lane + c * KVA_WAVE, value_dim - 1) * page_size;
+#pragma unroll
+                for (int g = 0; g < 16; ++g) Vec4<T>::load(vcol + voff_s[wave][4 * g], v[c][g]);
+            }
+            score(0);
+            for (int j0 = 64; j0 < head_dim; j0 += 64) {
+                keys(j0);
+                score(j0);
+            }
+            if (valid) s = dot * scale;
+        }
+        const float top = wave_max(s);
+        if (lane == 0) max_s[wave] = top;
+        __syncthreads();
+        float corr[FEW_BLOCKS], mine = 0.f, my_corr = 1.f, m_new = m;
+#pragma unroll
+        for (int k = 0; k < FEW_BLOCKS; ++k) {
+            corr[k] = 1.f;
+            if (!visible(base + k)) continue;
+            const float before = m_new;
+            m_new = fmaxf(before, max_s[k]);
+            corr[k] = (before == -INFINITY) ? 0.f : expf(before - m_new);
+            mine = k == wave ? m_new : mine;
+            my_corr = k == wave ? corr[k] : my_corr;
+        }
+        m = m_new;
+        const float p = valid ? expf(s - mine) : 0.f, sum = wave_sum(p);
+        p_s[wave][lane] = p;
+        if (lane == 0) sum_s[wave] = sum;
+        const bool half = pos - kb * KVA_WAVE < 32;             // no keys in the block's second half
+        if (on && seen != ~0ull) {
+#pragma unroll
+            for (int c = 0; c < VC; ++c)
+#pragma unroll
+                for (int g = 0; g < 16; ++g)
+#pragma unroll
+                    for (int u = 0; u < 4; ++u) v[c][g][u] = (seen >> (4 * g + u)) & 1 ? v[c][g][u] : 0.f;
+        }
+        __syncthreads();
+#pragma unroll
+        for (int k = 0; k < FEW_BLOCKS; ++k)
+            if (visible(base + k)) l = __builtin_fmaf(l, corr[k], sum_s[k]);
+#pragma unroll 1
+        for (int k = 0; k < FEW_BLOCKS; ++k) {
+            if (!visible(base + k)) continue;                   // (uniform over the workgroup)
+            if (k == wave) {
+                float a[VC];
+#pragma unroll
+                for (int c = 0; c < VC; ++c) {
+                    a[c] = acc_s[c * KVA_WAVE + lane] * my_corr;
+                    asm volatile("" : "+v"(a[c]));              // (rounded before the first value is added)
+                }
+                auto add = [&](auto first) {
+#pragma unroll
+                    for (int g = decltype(first)::value; g < decltype(first)::value + 8; ++g) {
+                        const float4 w = *reinterpret_cast<const float4 *>(&p_s[wave][4 * g]);
+#pragma unroll
+                        for (int c = 0; c < VC; ++c) {
+                            a[c] = __builtin_fmaf(w.x, v[c][g][0], a[c]);
+                            a[c] = __builtin_fmaf(w.y, v[c][g][1], a[c]);
+                            a[c] = __builtin_fmaf(w.z, v[c][g][2], a[c]);
+                            a[c] = __builtin_fmaf(w.w, v[c][g][3], a[c]);
+                        }
+                    }
+                };
+                add(std::integral_constant<int, 0>{});
+                if (!half) add(std::integral_constant<int, 8>{});
+#pragma unroll
+                for (int c = 0; c < VC; ++c) acc_s[c * KVA_WAVE + lane] = a[c];
+            }
+            __syncthreads();
+        }
+    }
+    float more = 1.f;
+    if (sinks) {
+        // one more term of the denominator, exp(sink), with no key and no value
+        const float s = sinks[qh], m_new = fmaxf(m, s);
+        more = (m == -INFINITY) ? 0.f : expf(m - m_new);
+        l = __builtin_fmaf(l, more, expf(s - m_new));
+    }
+    if (tid < value_dim) out[(size_t)t * num_q_heads * value_dim + (size_t)qh * value_dim + tid] = from_float<T>((sinks ? acc_s[tid] * more : acc_s[tid]) / l);
+}
+
+// `longest`: no token has a position past it (only the choice of kernel goes by it).
 extern "C" int kva_attention_rowwise(void *out, const void *q, int q_row_stride, const void *k_cache,
                                      const void *v_cache, const int *block_table, int max_blocks,
                                      const int *tok_seat, const int *tok_pos, int tokens,
                                      int num_q_heads, int num_kv_heads, int head_dim, int value_dim, int page_size,
-                                     float scale, int window, int keep_first, int chunk, const float *sinks, int dtype,
-                                     hipStream_t stream) {
+                                     float scale, int window, int keep_first, int chunk, const float *sinks, int longest,
+                                     int dtype, hipStream_t stream) {
     KVA_REQUIRE(tokens >= 0 && num_q_heads > 0 && num_kv_heads > 0 && page_size > 0 && max_blocks > 0,
                 "attention: bad sizes");
     KVA_REQUIRE(num_q_heads % num_kv_heads == 0, "attention: %d query heads is not a multiple of %d kv heads",
@@ -239,14 +389,29 @@ extern "C" int kva_attention_rowwise(void *out, const void *q, int q_row_stride,
     const int together = rows >= 12288 && group % 4 == 0 ? 4
                          : rows >= 6144 && group % 3 == 0 ? 3
                          : rows >= 3072 && group % 2 == 0 ? 2 : 1;
+    // Few rows with more than a block of keys: four blocks at a time, whose chains of additions are 6.5 us for two blocks and 2 more for each
+    // one after the other.  One wavefront / four, fp32, us a call: 3 tokens of 32 heads of 64 at 66 / 130 / 201 / 1,000 keys 6.5 / 8.4 / 10.2 /
+    // 42.5 -> 5.6 / 6.2 / 7.0 / 22.9, heads of 128 9.0 / 11.9 / 16.3 / 64.3 -> 7.7 / 8.7 / 10.5 / 36.2; 16 tokens (512 rows) at 201 keys 11.1 -> 8.6
+    // (heads of 128 16.2 -> 13.5); but 32 tokens 13.7 -> 15.8, and at 40 keys, one block, 4.6 -> 5.2.
+    const long long span = window > 0 ? (long long)window + keep_first : chunk > 0 ? chunk : longest;      // keys that a token sees, at most
+    const bool few = fours && rows <= 512 && span > KVA_WAVE && longest > KVA_WAVE && head_dim % 64 == 0 && head_dim <= FEW_MAX_DIM &&
+                     value_dim <= FEW_MAX_DIM;
     // (a head alone whose elements are whole rounds of 64 loads' worth; of others the last round would go one load at a time)
 #define KVA_ROWWISE(T, H, ALL)                                                                                         \
     hipLaunchKernelGGL((attention_rowwise_kernel<T, H, ALL>), dim3(tokens, num_q_heads / H), dim3(KVA_WAVE), 0, stream, (T *)out, \
                        (const T *)q, q_row_stride, (const T *)k_cache, (const T *)v_cache, block_table, max_blocks,    \
                        tok_seat, tok_pos, num_q_heads, num_kv_heads, head_dim, value_dim, page_size, fours, scale,     \
                        window, keep_first, chunk, sinks)
+#define KVA_FEW(T, VC)                                                                                                 \
+    hipLaunchKernelGGL((attention_few_kernel<T, VC>), dim3(tokens, num_q_heads), dim3(KVA_WAVE * FEW_BLOCKS), 0, stream, (T *)out, \
+                       (const T *)q, q_row_stride, (const T *)k_cache, (const T *)v_cache, block_table, max_blocks,    \
+                       tok_seat, tok_pos, num_q_heads, num_kv_heads, head_dim, value_dim, page_size, scale, window,    \
+                       keep_first, chunk, sinks)
 #define KVA_ROWWISE_HEADS(T)                                                                                           \
     do {                                                                                                               \
+        if (few && value_dim <= KVA_WAVE) KVA_FEW(T, 1);                                                               \
+        else if (few) KVA_FEW(T, 2);                                                                                   \
+        else                                                                                                           \
         if (together == 4) KVA_ROWWISE(T, 4, false);                                                                          \
         else if (together == 3) KVA_ROWWISE(T, 3, false);                                                                     \
         else if (together == 2) KVA_ROWWISE(T, 2, false);                                                                     \
@@ -258,6 +423,7 @@ extern "C" int kva_attention_rowwise(void *out, const void *q, int q_row_stride,
     else KVA_REQUIRE(false, "attention: unsupported dtype %d", dtype);
 #undef KVA_ROWWISE_HEADS
 #undef KVA_ROWWISE
+#undef KVA_FEW
     KVA_CHECK_LAUNCH("attention_rowwise");
     return KVA_OK;
 }

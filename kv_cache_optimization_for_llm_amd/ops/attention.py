@@ -483,7 +483,7 @@ def paged_attention(qkv: torch.Tensor, out: torch.Tensor, kv, batch, num_q_heads
                                          value_dim, ranges, per, tiles, chunk)
         return K.attention_rowwise(qkv, stride, out, kv.k_cache, kv.v_cache, kv.block_table,
                                    batch.tok_seat, batch.positions, num_q_heads, num_kv_heads,
-                                   head_dim, scale, window, keep_first, sinks, value_dim, chunk)
+                                   head_dim, scale, window, keep_first, sinks, value_dim, chunk, batch.max_context)
     if rope is not None:
         # decoded tokens whose rotation and cache write are still to be done: ``rope`` = (cos, sin)
         # tables or (None, None); only where rotates_in_kernel() said yes
@@ -496,7 +496,7 @@ def paged_attention(qkv: torch.Tensor, out: torch.Tensor, kv, batch, num_q_heads
     if not tuned:
         return K.attention_rowwise(qkv, stride, out, kv.k_cache, kv.v_cache, kv.block_table,
                                    batch.tok_seat, batch.positions, num_q_heads, num_kv_heads,
-                                   head_dim, scale, window)
+                                   head_dim, scale, window, longest=batch.max_context)
     if chunk > 0:
         window = -chunk         # the tuned kernels take both masks in one number: below zero, chunks of so many positions
     plan = _plan_for(batch, kv, num_q_heads, num_kv_heads, head_dim, max_parts, window if window >= 0 else max(1, -window // 2))

@@ -369,13 +369,14 @@ def attention_rowwise(q: torch.Tensor, q_row_stride: int, out: torch.Tensor, k_c
                       v_cache: torch.Tensor, block_table: torch.Tensor, tok_seat: torch.Tensor,
                       tok_pos: torch.Tensor, num_q_heads: int, num_kv_heads: int, head_dim: int,
                       scale: float, window: int = 0, keep_first: int = 0, sinks: Optional[torch.Tensor] = None,
-                      value_dim: Optional[int] = None, chunk: int = 0) -> torch.Tensor:
+                      value_dim: Optional[int] = None, chunk: int = 0, longest: int = 0) -> torch.Tensor:
     """Causal GQA attention of every token over its request's cached keys; ``q`` is a view whose
     rows are ``q_row_stride`` elements apart (the Q part of a fused QKV buffer).  With a
     ``window`` a query at position i sees key j when ``i - j < window`` or ``j < keep_first``; with a
     ``chunk`` when both lie in the same run of ``chunk`` positions counted from 0;
     ``sinks`` (fp32, one per query head) adds ``exp(sink)`` to every softmax denominator;
-    ``value_dim`` is the size of a value where it differs from a key's."""
+    ``value_dim`` is the size of a value where it differs from a key's.  ``longest``: no request has more keys (0: than its
+    row of the block table has places for); it decides how the work is laid out, not the results."""
     tokens = out.shape[0]
     value_dim = head_dim if value_dim is None else int(value_dim)
     if out.shape != (tokens, num_q_heads * value_dim):
@@ -395,7 +396,8 @@ def attention_rowwise(q: torch.Tensor, q_row_stride: int, out: torch.Tensor, k_c
         _dev(v_cache, "v_cache"), _dev(block_table, "block_table", torch.int32), block_table.shape[1],
         _dev(tok_seat, "tok_seat", torch.int32), _dev(tok_pos, "tok_pos", torch.int32), tokens,
         num_q_heads, num_kv_heads, head_dim, value_dim, page_size, float(scale), int(window), int(keep_first),
-        int(chunk), _opt(sinks, "sinks"), dtype_code(out.dtype), _stream()), "attention_rowwise")
+        int(chunk), _opt(sinks, "sinks"), min(int(longest) or 1 << 30, block_table.shape[1] * page_size), dtype_code(out.dtype),
+        _stream()), "attention_rowwise")
     return out
 
 
