@@ -530,7 +530,7 @@ static int token_check(const char *what, const TokenIO &io, int entries) {
     return KVA_OK;
 }
 
-// Entries of one token each.  `shape`: whether sizes and addresses fit is all that is asked (0 / 1, nothing is launched).
+// Entries of one token each, or none.  `ask`: whether sizes and addresses fit is all that is asked (0 / 1, nothing is launched).
 extern "C" int kva_delta_token(int ask, const void *y, int y_dtype, int y_stride, int conv_col, const float *conv_w, int taps, float *state,
                                long long seat_stride, int state_off, int conv_off, int beta_off, int decay_off, const float *a_log,
                                const float *dt_bias, const float *channel_decay, int decay_stride, float unit_eps, const float *norm_w,

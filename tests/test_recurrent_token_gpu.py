@@ -117,3 +117,23 @@ def test_what_does_not_fit_is_left_alone(gpu):
     assert delta()
     for other in (dict(heads=5), dict(dim=136), dict(vdim=60), dict(taps=5), dict(taps=1), dict(gate_off=4), dict(out_off=4), dict(state_off=2), dict(wide=4)):
         assert not delta(**other), other
+
+
+def test_entries_without_a_token(gpu):
+    """More entries than rows: an entry without a token leaves its seat's state as it is."""
+    g = torch.Generator().manual_seed(1)
+    heads, dim, vdim, rank = 2, 64, 64, 16
+    starts, seats = ints([0, 0, 1, 1, 2]), ints([3, 0, 4, 2])
+    y = numbers((2, 4 * heads * dim + 16), g)
+    a2, bias, norm = numbers((heads * dim, rank), g, scale=0.3), numbers((heads * dim,), g), numbers((vdim,), g)
+    state = numbers((5, heads * dim * vdim), g)
+    got, want = state.clone(), state.clone()
+    out = torch.zeros((2, heads * vdim), device="cuda")
+    ref = out.clone()
+    offs = (0, heads * dim, 2 * heads * dim, 4 * heads * dim)
+    assert K.gated_linear_attention_token(y, *offs, a2, bias, 3.5, 0.125, got, 0, norm, 1e-5, 3 * heads * dim, "silu", out, 0, 1.0, starts, seats,
+                                          heads, dim, vdim)
+    assert K.gated_linear_attention_token(y, *offs, a2, bias, 3.5, 0.125, want, 0, norm, 1e-5, 3 * heads * dim, "silu", ref, 0, 1.0, ints([0, 1, 2]),
+                                          ints([0, 2]), heads, dim, vdim)
+    same([(out, ref), (got, want)])
+    assert torch.equal(got[[1, 3, 4]], state[[1, 3, 4]])
