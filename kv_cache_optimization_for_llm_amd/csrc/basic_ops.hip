@@ -261,7 +261,8 @@ extern "C" int kva_rmsnorm(void *out, void *hidden, const void *delta, const voi
         // where a workgroup allows, every load of the row asked for at once (4,096 columns, 64 rows:
         // 5.3 -> 4.5 us, with partial products in 8 ranges 9.2 -> 7.0; 2,048 rows: 18.6 -> 20.9, so not there).
         int threads = width >= 8192 ? 1024 : (width >= 2048 ? 256 : (width >= 1024 ? 128 : 64));
-        if (out_rows <= 256) threads = std::min(1024, std::max(64, (width / 8 + 63) / 64 * 64));
+        // fp32: as for few rows whatever their number, so that the order of a row's sum follows from its width alone.
+        if (out_rows <= 256 || dtype == KVA_F32) threads = std::min(1024, std::max(64, (width / 8 + 63) / 64 * 64));
         const int per = (width / 8 + threads - 1) / threads;                 // 1 .. 8
         const size_t part_stride = (size_t)part_rows * width;
 #define RMS_LAUNCH(T, TW, PER)                                                                                                        \

@@ -44,6 +44,16 @@ def test_rmsnorm(rows, width, shift, w_dtype, dtype, gpu):
         close(out2, normed[idx.long()])
 
 
+@pytest.mark.parametrize("width", [72, 768, 1096, 2048, 4096, 10000])
+def test_rmsnorm_of_a_row_alone_and_among_others(width, gpu):
+    """fp32: the same bits however many rows there are."""
+    g = torch.Generator().manual_seed(width)
+    w, x = made((width,), torch.float32, g), made((300, width), torch.float32, g)
+    many = K.rmsnorm(x, w, 1e-5, torch.empty_like(x))
+    for n in (1, 256):
+        assert torch.equal(K.rmsnorm(x[:n].contiguous(), w, 1e-5, torch.empty_like(x[:n])), many[:n])
+
+
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
 @pytest.mark.parametrize("rows, inter, shift", [(1, 8, 0), (3, 2040, 0), (515, 2040, 0), (515, 2048, 1), (2, 13, 0)])
 def test_silu_mul(rows, inter, shift, dtype, gpu):
