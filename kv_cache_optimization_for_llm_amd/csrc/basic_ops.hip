@@ -74,20 +74,26 @@ extern "C" int kva_embed_gather(void *out, void *copy, const void *table, const 
 // named twice).
 template <typename T, typename TW>
 __global__ void rmsnorm_kernel(T *__restrict__ out, T *__restrict__ hidden,
-                               const T *__restrict__ delta, const TW *__restrict__ weight,
-                               const int *__restrict__ row_idx, int width, float eps) {
+                               const T *__restrict__ delta, const float *__restrict__ delta_parts, int parts, size_t part_stride,
+                               const TW *__restrict__ weight, const int *__restrict__ row_idx, int width, float eps) {
     __shared__ float scratch[16];
     const int orow = blockIdx.x;
     const int irow = row_idx ? row_idx[orow] : orow;
     T *x = hidden + (size_t)irow * width;
     const T *dl = delta ? delta + (size_t)irow * width : nullptr;
-    const bool write_back = dl && !row_idx;
+    const bool adds = dl || parts > 0, write_back = adds && !row_idx;
+    auto added = [&](int i) {           // of partial products their sum, rounded as the product itself would have been
+        if (dl) return to_float(dl[i]);
+        float sum = 0.f;
+        for (int p = 0; p < parts; ++p) sum += delta_parts[p * part_stride + (size_t)irow * width + i];
+        return to_float(from_float<T>(sum));
+    };
     T *y = out + (size_t)orow * width;
     float ss = 0.f;
     for (int i = threadIdx.x; i < width; i += blockDim.x) {
         float v = to_float(x[i]);
-        if (dl) {
-            const T r = from_float<T>(v + to_float(dl[i]));
+        if (adds) {
+            const T r = from_float<T>(v + added(i));
             if (write_back) x[i] = r;
             v = to_float(r);
         }
@@ -97,7 +103,7 @@ __global__ void rmsnorm_kernel(T *__restrict__ out, T *__restrict__ hidden,
     const float r = (float)sqrt((double)total / (double)width + (double)eps);
     for (int i = threadIdx.x; i < width; i += blockDim.x) {
         float v = to_float(x[i]);
-        if (dl && !write_back) v = to_float(from_float<T>(v + to_float(dl[i])));
+        if (adds && !write_back) v = to_float(from_float<T>(v + added(i)));
         y[i] = from_float<T>((v / r) * to_float(weight[i]));
     }
 }
@@ -284,11 +290,10 @@ extern "C" int kva_rmsnorm(void *out, void *hidden, const void *delta, const voi
         KVA_CHECK_LAUNCH("rmsnorm");
         return KVA_OK;
     }
-    KVA_REQUIRE(parts == 0, "rmsnorm: partial products go with rows of up to 65,536");
     dim3 grid(out_rows), block(width >= 2048 ? 512 : 256);
 #define LAUNCH(T, TW)                                                                      \
     hipLaunchKernelGGL((rmsnorm_kernel<T, TW>), grid, block, 0, stream, (T *)out, (T *)hidden, \
-                       (const T *)delta, (const TW *)weight, row_idx, width, eps)
+                       (const T *)delta, delta_parts, parts, (size_t)part_rows * width, (const TW *)weight, row_idx, width, eps)
     if (dtype == KVA_F32 && weight_dtype == KVA_F32) LAUNCH(float, float);
     else if (dtype == KVA_BF16 && weight_dtype == KVA_BF16) LAUNCH(bf16_t, bf16_t);
     else if (dtype == KVA_BF16) LAUNCH(bf16_t, float);

@@ -54,6 +54,25 @@ def test_rmsnorm_of_a_row_alone_and_among_others(width, gpu):
         assert torch.equal(K.rmsnorm(x[:n].contiguous(), w, 1e-5, torch.empty_like(x[:n])), many[:n])
 
 
+@pytest.mark.parametrize("rows, width, ranges", [(3, 2056, 5), (2, 65536, 2), (2, 65544, 3)])
+def test_rmsnorm_of_partial_products(rows, width, ranges, gpu):
+    """A branch output in ranges of K: their sum in order, rounded to bf16, is added; rows of any length."""
+    g = torch.Generator().manual_seed(width)
+    w, x, parts = made((width,), torch.bfloat16, g), made((rows, width), torch.bfloat16, g), made((ranges, rows, width), torch.float32, g)
+    idx = torch.tensor([rows - 1, 0], dtype=torch.int32, device="cuda")
+    d = torch.zeros((rows, width), device="cuda")
+    for p in parts:
+        d += p
+    want = (x.float() + d.bfloat16().float()).bfloat16().to(D)
+    normed = want / torch.sqrt((want * want).mean(1, keepdim=True) + 1e-5) * w.to(D)
+    out, some = (torch.empty((n, width), dtype=torch.bfloat16, device="cuda") for n in (rows, 2))
+    K.rmsnorm(x, w, 1e-5, some, delta=K.PartialSums(parts), row_idx=idx)
+    close(some, normed[idx.long()])
+    K.rmsnorm(x, w, 1e-5, out, delta=K.PartialSums(parts))
+    assert torch.equal(x.to(D), want)
+    close(out, normed)
+
+
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
 @pytest.mark.parametrize("rows, inter, shift", [(1, 8, 0), (3, 2040, 0), (515, 2040, 0), (515, 2048, 1), (2, 13, 0)])
 def test_silu_mul(rows, inter, shift, dtype, gpu):
