@@ -214,6 +214,23 @@ attention_rowwise_kernel(T *__restrict__ out, const T *__restrict__ q, int q_row
 #define FEW_BLOCKS 4
 #define FEW_MAX_DIM 128
 
+// Whether a block has a key that is seen, which they are, and whose places its lanes read.  Pages that hold none of a token's keys may be given back (behind a
+// window, past the kept first positions): their entries in the table name no page, and only a seen key's entry may be looked up.
+__host__ __device__ inline bool few_block_seen(int kb, int pos, int lo, int keep_first) {
+    return kb <= pos / KVA_WAVE && !(kb * KVA_WAVE + KVA_WAVE <= lo && kb * KVA_WAVE >= keep_first);
+}
+__host__ __device__ inline bool few_key_seen(int key, int pos, int lo, int keep_first) {
+    return key <= pos && (key >= lo || key < keep_first);
+}
+// (`seen`: a bit a lane.)  A key not seen: the place of the first that is, its score goes unused.
+__host__ __device__ inline int few_key_read(unsigned long long seen, int lane) {
+    return (seen >> lane) & 1 ? lane : __builtin_ctzll(seen);
+}
+// Values are read four keys of a page together: where none of them is seen, those around the first seen one.
+__host__ __device__ inline int few_value_read(unsigned long long seen, int lane) {
+    return (seen >> (lane & ~3)) & 15 ? lane : __builtin_ctzll(seen) & ~3;
+}
+
 // VC: rounds of 64 value elements
 template <typename T, int VC>
 __global__ void __launch_bounds__(KVA_WAVE * FEW_BLOCKS)
@@ -236,23 +253,21 @@ attention_few_kernel(T *__restrict__ out, const T *__restrict__ q, int q_row_str
 
     const int lo = kva_first_visible(pos, window, chunk), end = pos / KVA_WAVE + 1;
     // a block with no visible key: behind the window and past the kept first positions, or past the token
-    auto visible = [&](int kb) { return kb < end && !(kb * KVA_WAVE + KVA_WAVE <= lo && kb * KVA_WAVE >= keep_first); };
+    auto visible = [&](int kb) { return few_block_seen(kb, pos, lo, keep_first); };
     float m = -INFINITY, l = 0.f;
     for (int base = keep_first > 0 ? 0 : lo / KVA_WAVE; base < end; base += FEW_BLOCKS) {       // uniform over the workgroup
         if ((base + FEW_BLOCKS) * KVA_WAVE <= lo && base * KVA_WAVE >= keep_first) continue;
         const int kb = base + wave;
-        const bool on = visible(kb);
-        const int key = kb * KVA_WAVE + lane;
-        const bool valid = on && key <= pos && (key >= lo || key < keep_first);
+        const bool valid = few_key_seen(kb * KVA_WAVE + lane, pos, lo, keep_first);
         const unsigned long long seen = __ballot(valid);
+        const bool on = seen != 0;
         float s = -INFINITY, v[VC][16][4];
         if (on) {
-            // (four keys of a page together; where none of them is visible, the first visible one's place is read and not used)
-            const int group = (seen >> (lane & ~3)) & 15 ? lane : (__ffsll(seen) - 1) & ~3;
-            const int page = bt[key <= pos ? key / page_size : pos / page_size], vkey = kb * KVA_WAVE + group;
+            const int kkey = kb * KVA_WAVE + few_key_read(seen, lane), vkey = kb * KVA_WAVE + few_value_read(seen, lane);
+            const int page = bt[kkey / page_size];
             voff_s[wave][lane] = ((long long)bt[vkey / page_size] * num_kv_heads + kvh) * (long long)value_dim * page_size + vkey % page_size;
             const T *kpage = k_cache + ((long long)page * num_kv_heads + kvh) * page_size * (long long)head_dim;
-            const int krow = key % page_size, kc = kva_k_chunk(head_dim);
+            const int krow = kkey % page_size, kc = kva_k_chunk(head_dim);
             float kv[16][4];
             auto keys = [&](int j0) {
 #pragma unroll
@@ -354,6 +369,21 @@ attention_few_kernel(T *__restrict__ out, const T *__restrict__ q, int q_row_str
         l = __builtin_fmaf(l, more, expf(s - m_new));
     }
     if (tid < value_dim) out[(size_t)t * num_q_heads * value_dim + (size_t)qh * value_dim + tid] = from_float<T>((sinks ? acc_s[tid] * more : acc_s[tid]) / l);
+}
+
+// What the few-rows kernel's wavefront over block `kb` reads for a token at `pos`: the keys whose places its 64 lanes look up, for
+// keys and for values (-1: the block is passed by).  On the host; the rule is the kernel's own.
+extern "C" int kva_attention_few_reads(int pos, int window, int keep_first, int chunk, int kb, int *keys, int *values) {
+    const int lo = kva_first_visible(pos, window, chunk);
+    unsigned long long seen = 0;
+    for (int lane = 0; lane < KVA_WAVE; ++lane)
+        if (few_key_seen(kb * KVA_WAVE + lane, pos, lo, keep_first)) seen |= 1ull << lane;
+    KVA_REQUIRE((seen != 0) == few_block_seen(kb, pos, lo, keep_first), "attention: block %d of position %d: the rules for blocks and for keys differ", kb, pos);
+    for (int lane = 0; lane < KVA_WAVE; ++lane) {
+        keys[lane] = seen ? kb * KVA_WAVE + few_key_read(seen, lane) : -1;
+        values[lane] = seen ? kb * KVA_WAVE + few_value_read(seen, lane) : -1;
+    }
+    return KVA_OK;
 }
 
 // `longest`: no token has a position past it (only the choice of kernel goes by it).

@@ -44,6 +44,7 @@ _HIP_SIGNATURES = {
     "kva_cast": [P, P, LL, I, I, P],
     "kva_rope_kv_write": [P, P, P, P, P, P, P, I, I, I, I, I, I, I, I, P],
     "kva_attention_rowwise": [P, P, I, P, P, P, I, P, P, I, I, I, I, I, I, F, I, I, I, P, I, I, P],
+    "kva_attention_few_reads": [I, I, I, I, I, P, P],
     "kva_latent_attention_rowwise": [P, P, P, P, I, P, P, I, I, I, I, I, F, I, I, P, I, P],
     "kva_layernorm": [P, P, I, P, I, P, I, P, I, P, P, I, P, I, I, F, I, F, P, P, I, I, P],
     "kva_stream_join": [P, I, P, I, P, I, P, I, P, I, I, I, I, P],

@@ -18,14 +18,21 @@ def test_four_wavefronts_have_the_bits_of_one(dtype, nq, nkv, d, dv, mask, sink,
     g = torch.Generator(device=gpu).manual_seed(2)
     rnd = lambda *s: torch.randn(*s, generator=g, device=gpu).to(dtype)
     T, page, blocks = len(POSITIONS), 16, 40
-    kc = torch.full((T * blocks, nkv, page, d), float("nan"), dtype=dtype, device=gpu)        # what lies behind a token is no number
-    vc = torch.full((T * blocks, nkv, dv, page), float("nan"), dtype=dtype, device=gpu)
+    # what lies behind a token is no number; pages without a key that is seen are not in the table, as the cache leaves them (and what
+    # such an entry would lead to is a page in front of the others)
+    kc = torch.full((1 + T * blocks, nkv, page, d), float("nan"), dtype=dtype, device=gpu)
+    vc = torch.full((1 + T * blocks, nkv, dv, page), float("nan"), dtype=dtype, device=gpu)[1:]
     table = torch.randperm(T * blocks, generator=torch.Generator().manual_seed(1)).to(torch.int32).view(T, blocks).to(gpu)
     for t, pos in enumerate(POSITIONS):
         at = torch.arange(pos + 1, device=gpu)
-        kc[table[t].long()[at // page], :, at % page] = rnd(pos + 1, nkv, d)
+        kc[1 + table[t].long()[at // page], :, at % page] = rnd(pos + 1, nkv, d)
         vc[table[t].long()[at // page], :, :, at % page] = rnd(pos + 1, nkv, dv)
-    kc = K.keys_to_pages(kc)
+        lo = pos - pos % mask["chunk"] if "chunk" in mask else max(0, pos - mask.get("window", pos + 1) + 1)
+        seen = (at >= lo) | (at < mask.get("keep_first", 0))
+        unseen = torch.ones(blocks, dtype=torch.bool, device=gpu)
+        unseen[at[seen] // page] = False
+        table[t, unseen] = -1
+    kc = K.keys_to_pages(kc)[1:]
     q, sinks = rnd(T, nq * d) * 2, torch.randn(nq, generator=g, device=gpu) if sink else None
     seat, pos = torch.arange(T, dtype=torch.int32, device=gpu), torch.tensor(POSITIONS, dtype=torch.int32, device=gpu)
 
