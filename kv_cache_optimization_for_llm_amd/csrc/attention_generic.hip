@@ -43,6 +43,14 @@ template <> struct Vec4<bf16_t> {
     }
 };
 
+// Multiply-adds are written out, and a product that is rounded by itself is kept apart from the addition behind it, in both kernels of this
+// file: which of them the compiler folds into one is otherwise its own choice in every variant, and a token's bits are to be the same
+// in all of them.
+__device__ inline float attn_rounded(float x) {
+    asm("" : "+v"(x));
+    return x;
+}
+
 // H query heads of one key head go together: a key's and a value's elements are loaded once for all of them, and their
 // sums, which are chains of dependent additions in a fixed order, run side by side.  With `fours` (pages of a multiple of
 // 4 keys) a lane reads its value element of 4 keys at once, a row of the transposed page, and 32 keys' loads are under way
@@ -115,14 +123,14 @@ attention_rowwise_kernel(T *__restrict__ out, const T *__restrict__ q, int q_row
 #pragma unroll
                 for (int h = 0; h < H; ++h) {
                     const float4 qv = *reinterpret_cast<const float4 *>(&q_s[h][j]);
-                    dot[h] += qv.x * kv[0];
-                    dot[h] += qv.y * kv[1];
-                    dot[h] += qv.z * kv[2];
-                    dot[h] += qv.w * kv[3];
+                    dot[h] = __builtin_fmaf(qv.x, kv[0], dot[h]);
+                    dot[h] = __builtin_fmaf(qv.y, kv[1], dot[h]);
+                    dot[h] = __builtin_fmaf(qv.z, kv[2], dot[h]);
+                    dot[h] = __builtin_fmaf(qv.w, kv[3], dot[h]);
                 }
             }
 #pragma unroll
-            for (int h = 0; h < H; ++h) s[h] = dot[h] * scale;
+            for (int h = 0; h < H; ++h) s[h] = attn_rounded(dot[h] * scale);
         }
         __syncthreads();  // the previous block's p_s / voff_s have been consumed
 #pragma unroll
@@ -130,7 +138,7 @@ attention_rowwise_kernel(T *__restrict__ out, const T *__restrict__ q, int q_row
             const float m_new = fmaxf(m[h], wave_max(s[h]));
             corr[h] = (m[h] == -INFINITY) ? 0.f : expf(m[h] - m_new);
             const float p = valid ? expf(s[h] - m_new) : 0.f;
-            l[h] = l[h] * corr[h] + wave_sum(p);
+            l[h] = __builtin_fmaf(l[h], corr[h], wave_sum(p));
             m[h] = m_new;
             p_s[h][lane] = p;
         }
@@ -150,7 +158,7 @@ attention_rowwise_kernel(T *__restrict__ out, const T *__restrict__ q, int q_row
                 const T *vcol = v_cache + (long long)j * page_size;
                 float a[H];
 #pragma unroll
-                for (int h = 0; h < H; ++h) a[h] = acc[c][h] * corr[h];
+                for (int h = 0; h < H; ++h) a[h] = attn_rounded(acc[c][h] * corr[h]);
                 if (fours) {
                     for (int i0 = 0; i0 <= last; i0 += 4 * FOURS) {
                         float v[FOURS][4];
@@ -169,10 +177,10 @@ attention_rowwise_kernel(T *__restrict__ out, const T *__restrict__ q, int q_row
 #pragma unroll
                             for (int h = 0; h < H; ++h) {
                                 const float4 p = *reinterpret_cast<const float4 *>(&p_s[h][i0 + 4 * g]);
-                                a[h] += p.x * v[g][0];
-                                a[h] += p.y * v[g][1];
-                                a[h] += p.z * v[g][2];
-                                a[h] += p.w * v[g][3];
+                                a[h] = __builtin_fmaf(p.x, v[g][0], a[h]);
+                                a[h] = __builtin_fmaf(p.y, v[g][1], a[h]);
+                                a[h] = __builtin_fmaf(p.z, v[g][2], a[h]);
+                                a[h] = __builtin_fmaf(p.w, v[g][3], a[h]);
                             }
                         }
                     }
@@ -181,7 +189,7 @@ attention_rowwise_kernel(T *__restrict__ out, const T *__restrict__ q, int q_row
                         if ((seen >> i) & 1) {
                             const float v = to_float(vcol[voff_s[i]]);
 #pragma unroll
-                            for (int h = 0; h < H; ++h) a[h] += p_s[h][i] * v;
+                            for (int h = 0; h < H; ++h) a[h] = __builtin_fmaf(p_s[h][i], v, a[h]);
                         }
                 }
 #pragma unroll
@@ -195,7 +203,7 @@ attention_rowwise_kernel(T *__restrict__ out, const T *__restrict__ q, int q_row
             // one more term of the denominator, exp(sink), with no key and no value
             const float s = sinks[qh + h], m_new = fmaxf(m[h], s);
             const float more = (m[h] == -INFINITY) ? 0.f : expf(m[h] - m_new);
-            l[h] = l[h] * more + expf(s - m_new);
+            l[h] = __builtin_fmaf(l[h], more, expf(s - m_new));
 #pragma unroll
             for (int c = 0; c < ATTN_MAX_HEAD_DIM / KVA_WAVE; ++c) acc[c][h] *= more;
         }
@@ -297,7 +305,7 @@ attention_few_kernel(T *__restrict__ out, const T *__restrict__ q, int q_row_str
                 keys(j0);
                 score(j0);
             }
-            if (valid) s = dot * scale;
+            if (valid) s = attn_rounded(dot * scale);
         }
         const float top = wave_max(s);
         if (lane == 0) max_s[wave] = top;
@@ -336,10 +344,7 @@ attention_few_kernel(T *__restrict__ out, const T *__restrict__ q, int q_row_str
             if (k == wave) {
                 float a[VC];
 #pragma unroll
-                for (int c = 0; c < VC; ++c) {
-                    a[c] = acc_s[c * KVA_WAVE + lane] * my_corr;
-                    asm volatile("" : "+v"(a[c]));              // (rounded before the first value is added)
-                }
+                for (int c = 0; c < VC; ++c) a[c] = attn_rounded(acc_s[c * KVA_WAVE + lane] * my_corr);
                 auto add = [&](auto first) {
 #pragma unroll
                     for (int g = decltype(first)::value; g < decltype(first)::value + 8; ++g) {

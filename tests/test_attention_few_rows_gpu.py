@@ -41,3 +41,25 @@ def test_four_wavefronts_have_the_bits_of_one(dtype, nq, nkv, d, dv, mask, sink,
         return K.attention_rowwise(q, nq * d, out, kc, vc, table, seat, pos, nq, nkv, d, d ** -0.5, sinks=sinks, value_dim=dv, longest=longest, **mask)
     one, four = run(64), run(601)            # (one block of keys at most: a wavefront; it decides nothing else)
     assert one.isfinite().all() and torch.equal(one, four)
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("nq, nkv, d, dv", [(8, 2, 64, 64), (8, 2, 128, 100), (6, 2, 64, 128), (2, 1, 128, 24), (4, 4, 64, 64)])
+@pytest.mark.parametrize("mask", [{}, dict(window=70, keep_first=3)])
+@pytest.mark.parametrize("page", [16, 6])            # (6: keys one by one, a wavefront a head or several)
+def test_many_rows_have_the_bits_of_few(dtype, nq, nkv, d, dv, mask, page, gpu):
+    """Four, three, two and one query heads a wavefront, as a prompt's tokens take them, against the same tokens alone."""
+    g = torch.Generator(device=gpu).manual_seed(3)
+    rnd = lambda *s: torch.randn(*s, generator=g, device=gpu).to(dtype)
+    T, blocks, times = len(POSITIONS), 601 // page + 1, 12288 // nq // len(POSITIONS) + 1
+    kc, vc = K.keys_to_pages(rnd(blocks, nkv, page, d)), rnd(blocks, nkv, dv, page)
+    table = torch.randperm(blocks, generator=torch.Generator().manual_seed(1)).to(torch.int32).view(1, blocks).to(gpu)
+    q, sinks = rnd(T, nq * d) * 2, torch.randn(nq, generator=g, device=gpu)
+    pos = torch.tensor(POSITIONS, dtype=torch.int32, device=gpu)
+
+    def run(n):
+        out = torch.full((n * T, nq * dv), 7.0, dtype=dtype, device=gpu)
+        return K.attention_rowwise(q.repeat(n, 1), nq * d, out, kc, vc, table, torch.zeros(n * T, dtype=torch.int32, device=gpu), pos.repeat(n), nq, nkv,
+                                   d, d ** -0.5, sinks=sinks, value_dim=dv, **mask)
+    few, many = run(1), run(times)
+    assert few.isfinite().all() and torch.equal(few.repeat(times, 1), many)
