@@ -175,13 +175,14 @@ __device__ inline void st8_from_float(void *p, int dtype, size_t i, const float 
     }
 }
 
-template <int PER, int TYPES, typename Experts>
+// FEW_ROWS: all that a row needs is asked for at once, weights too (types known), in up to 170 registers against 64.
+template <int PER, bool FEW_ROWS, int TYPES, typename Experts>
 __global__ void __launch_bounds__(256)
 layernorm_vec_kernel(void *__restrict__ out1, void *__restrict__ out2, int out_dtype, void *__restrict__ x, int x_dtype,
                      const void *__restrict__ d1, int d1_dtype, const void *__restrict__ d2, int d2_dtype,
                      const void *__restrict__ w1, const void *__restrict__ w2, int w_dtype,
                      const int *__restrict__ row_idx, int width, float eps, int rms, float delta_scale, Experts er) {
-    constexpr bool LATE = TYPES != TYPES_ANY;
+    constexpr bool LATE = TYPES != TYPES_ANY, AHEAD = LATE && FEW_ROWS;
     if constexpr (LATE) {
         x_dtype = TYPES == TYPES_STREAM16 ? KVA_BF16 : KVA_F32;
         d1_dtype = out_dtype = TYPES == TYPES_F32 ? KVA_F32 : KVA_BF16;
@@ -193,20 +194,29 @@ layernorm_vec_kernel(void *__restrict__ out1, void *__restrict__ out2, int out_d
     const size_t src = (size_t)(row_idx ? row_idx[r] : r) * width, dst = (size_t)r * width;
     float v[PER][8], w[8];
     RawRow<8, LATE> xr[PER], ar[PER], br[PER], w1r[PER], w2r[PER];
-#pragma unroll
-    for (int c = 0; c < PER; ++c) {
-        const int j = (c * 256 + (int)threadIdx.x) * 8;
-        if (j >= width) continue;
+    auto ask = [&](int c, int j) {
         xr[c].load(x, x_dtype, src + j);
         if (d1) ar[c].load(d1, d1_dtype, src + j);
         if (d2) br[c].load(d2, d2_dtype, src + j);
+    };
+    auto ask_weights = [&](int c, int j) {
         w1r[c].load(w1, w_dtype, j);
         if (w2) w2r[c].load(w2, w_dtype, j);
+    };
+    if constexpr (AHEAD) {
+#pragma unroll
+        for (int c = 0; c < PER; ++c) {
+            const int j = (c * 256 + (int)threadIdx.x) * 8;
+            if (j >= width) continue;
+            ask(c, j);
+            ask_weights(c, j);
+        }
     }
     float sum = 0.f;
 #pragma unroll
     for (int c = 0; c < PER; ++c) {
         const int j = (c * 256 + (int)threadIdx.x) * 8;
+        if (!AHEAD && j < width) ask(c, j);
         xr[c].floats(x_dtype, v[c]);
         if (j >= width) continue;
         if (d1 || d2 || er.rows) {
@@ -243,6 +253,7 @@ layernorm_vec_kernel(void *__restrict__ out1, void *__restrict__ out2, int out_d
         const int j = (c * 256 + (int)threadIdx.x) * 8;
         if (j >= width) continue;
         float n[8];
+        if (!AHEAD) ask_weights(c, j);
         w1r[c].floats(w_dtype, w);
 #pragma unroll
         for (int i = 0; i < 8; ++i) n[i] = v[c][i] * inv * w[i];
@@ -277,13 +288,18 @@ extern "C" int kva_layernorm(void *out1, void *out2, int out_dtype, void *x, int
         types = TYPES_WEIGHTS32;
     auto launch = [&](auto er) {
         typedef decltype(er) Experts;
-#define KVA_LAYERNORM_VEC(PER)                                                                                          \
-    hipLaunchKernelGGL((types == TYPES_STREAM16 ? layernorm_vec_kernel<PER, TYPES_STREAM16, Experts> : KVA_BY_TYPES(types, layernorm_vec_kernel, PER)), dim3(rows), dim3(256), 0, stream, out1, out2, out_dtype, x, x_dtype, d1,  \
+#define KVA_LAYERNORM_VEC(PER, FEW_ROWS)                                                                                          \
+    hipLaunchKernelGGL((types == TYPES_STREAM16 ? layernorm_vec_kernel<PER, FEW_ROWS, TYPES_STREAM16, Experts>                     \
+                                                : KVA_BY_TYPES(types, layernorm_vec_kernel, PER, FEW_ROWS)), dim3(rows), dim3(256), 0, stream, out1, out2, out_dtype, x, x_dtype, d1,  \
                        d1_dtype, d2, d2_dtype, w1, w2, w_dtype, row_idx, width, eps, rms, delta_scale, er)
         if (width % 8 == 0 && width <= 8192 && all % 16 == 0) {
-            if (width <= 2048) KVA_LAYERNORM_VEC(1);
-            else if (width <= 4096) KVA_LAYERNORM_VEC(2);
-            else KVA_LAYERNORM_VEC(4);
+            // Past 4,096 elements what is held ahead costs workgroups a unit, from three of them on.  Held / as it is used, us, 64 / 512 /
+            // 768 / 1,024 / 2,048 rows of 6,144: fp32 5.3 / 9.5 / 16.3 / 19.8 / 43.6, 5.7 / 9.9 / 13.9 / 17.8 / 37.5; bf16 beside an fp32 stream
+            // 6.3 / 9.1 / 11.1 / 14.3 / 30.4, 6.3 / 9.1 / 10.8 / 13.9 / 28.1; fp32, two outputs, 64 rows of 8,192 6.4, 7.5.
+            if (width <= 2048) KVA_LAYERNORM_VEC(1, true);
+            else if (width <= 4096) KVA_LAYERNORM_VEC(2, true);
+            else if (rows <= 512) KVA_LAYERNORM_VEC(4, true);
+            else KVA_LAYERNORM_VEC(4, false);
         } else {
             hipLaunchKernelGGL(layernorm_kernel<Experts>, dim3(rows), dim3(256), (size_t)width * sizeof(float), stream, out1, out2,
                                out_dtype, x, x_dtype, d1, d1_dtype, d2, d2_dtype, w1, w2, w_dtype, row_idx, width, eps, rms, delta_scale, er);
