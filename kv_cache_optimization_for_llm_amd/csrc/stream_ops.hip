@@ -712,7 +712,7 @@ hyper_step_vec_kernel(float *__restrict__ x, const void *__restrict__ y, int y_d
     const size_t row = (size_t)(row_idx ? row_idx[r] : r);
     float *xr = x + row * S * width;
     float v[ITERS][S][4], yv[ITERS][4], wv[ITERS][4], bv[ITERS][4];
-    RawRow<4, NARROW> yr[ITERS], wr[ITERS], br[ITERS];
+    RawRow<4, NARROW> yr[ITERS], wr[ITERS], br[ITERS];      // (of other types numbers are made as they are loaded: 64 rows of 4,096 6.3 us against 7.0)
 #pragma unroll
     for (int it = 0; it < ITERS; ++it) {
         const int j = (threadIdx.x + it * 256) * 4;
@@ -722,15 +722,25 @@ hyper_step_vec_kernel(float *__restrict__ x, const void *__restrict__ y, int y_d
             const float4 t = on ? *reinterpret_cast<const float4 *>(xr + (size_t)s * width + j) : make_float4(0.f, 0.f, 0.f, 0.f);
             v[it][s][0] = t.x; v[it][s][1] = t.y; v[it][s][2] = t.z; v[it][s][3] = t.w;
         }
-        if (on && y) yr[it].load(y, y_dtype, row * width + j);
-        if (on && out) wr[it].load(nw, w_dtype, j);
-        if (on && out && nb) br[it].load(nb, w_dtype, j);
-    }
+        if constexpr (NARROW) {
+            if (on && y) yr[it].load(y, y_dtype, row * width + j);
+            if (on && out) wr[it].load(nw, w_dtype, j);
+            if (on && out && nb) br[it].load(nb, w_dtype, j);
+        } else {
 #pragma unroll
-    for (int it = 0; it < ITERS; ++it) {
-        yr[it].floats(y_dtype, yv[it]);
-        wr[it].floats(w_dtype, wv[it]);
-        br[it].floats(w_dtype, bv[it]);
+            for (int e = 0; e < 4; ++e) yv[it][e] = wv[it][e] = bv[it][e] = 0.f;
+            if (on && y) hyper_ld4(y, y_dtype, row * width + j, yv[it]);
+            if (on && out) hyper_ld4(nw, w_dtype, j, wv[it]);
+            if (on && out && nb) hyper_ld4(nb, w_dtype, j, bv[it]);
+        }
+    }
+    if constexpr (NARROW) {
+#pragma unroll
+        for (int it = 0; it < ITERS; ++it) {
+            yr[it].floats(y_dtype, yv[it]);
+            wr[it].floats(w_dtype, wv[it]);
+            br[it].floats(w_dtype, bv[it]);
+        }
     }
     if (threadIdx.x < S * S) co.mix[threadIdx.x] = y ? mix[threadIdx.x] : 0.f;
     if (threadIdx.x < S) {
