@@ -445,7 +445,7 @@ space_token_kernel(SpaceToken a) {
     }
     token_keep_order();
     if (tid < channels) put(tid, conv.finish(st, channel(tid)));
-    for (int i = tid + TOKEN_THREADS; i < channels; i += TOKEN_THREADS) {
+    for (int i = tid + blockDim.x; i < channels; i += blockDim.x) {
         conv.load(io, st, q0, channel(i));
         put(i, conv.finish(st, channel(i)));
     }
@@ -603,16 +603,23 @@ extern "C" int kva_space_token(int ask, const void *y, int y_dtype, int y_stride
     const int units = hg * ((vdim + 63) / 64), per = TOKEN_THREADS / 256;
     const bool fits = heads > 0 && groups > 0 && norm_groups > 0 && heads % groups == 0 && (long long)heads * vdim % norm_groups == 0 && width > 0 &&
                       hg * vdim <= SPACE_COLS && hg * vdim % width == 0 && hg * vdim / width << token_lanes(width) <= TOKEN_THREADS &&
-                      n > 0 && n <= TOKEN_MAX_DIM && taps >= 2 && taps <= 4 && units <= 2 * per && token_types(y_dtype, y_dtype, out_dtype) && token_aligned(a.io, width, vdim);
+                      n > 0 && n <= TOKEN_MAX_DIM && taps >= 2 && taps <= 4 && units <= 2 * per && token_types(y_dtype, y_dtype, out_dtype) && token_aligned(a.io, width, vdim) &&
+                      // (fp32 rows, a group's columns in two passes, more workgroups than the chip takes at once: three launches / one, us, 1,024 requests
+                      // of 24 heads of 64 x 64 in 3 groups 188 / 223, 16 heads in 2 groups 125 / 141; 256 requests of 32 heads of 128 x 64 in 4 groups
+                      // 103 / 108, of 24 in 3 50 / 51; 64 requests of the two 34 / 28 and 19 / 14)
+                      (y_dtype != KVA_F32 || units <= per || (long long)groups * entries <= 768);
     if (ask) return fits;
     if (int rc = token_check("space_token", a.io, entries)) return rc;
     KVA_REQUIRE(fits && conv_w && a_log && dt_bias && d_skip, "space_token: sizes, addresses or operands do not fit");
     if (entries == 0) return KVA_OK;
     const dim3 grid(groups, entries);
+    // (all 1,024 where 256 have work: 64 heads of 16 x 64 in groups of their own, 1 / 64 / 256 requests 6.8 / 70 / 280 us; 6.2 / 23 / 73 so, and
+    // 11.7 / 32 / 94 in three launches)
+    const int threads = 256 * min(units, per);
 #define KVA_SPACE_TOKEN(TAPS)                                                                                                       \
     hipLaunchKernelGGL((y_dtype == KVA_BF16 ? (units <= per ? space_token_kernel<bf16_t, 1, TAPS> : space_token_kernel<bf16_t, 2, TAPS>)  \
                                             : (units <= per ? space_token_kernel<float, 1, TAPS> : space_token_kernel<float, 2, TAPS>)),  \
-                       grid, dim3(TOKEN_THREADS), 0, stream, a)
+                       grid, dim3(threads), 0, stream, a)
     if (taps == 2) KVA_SPACE_TOKEN(2);
     else if (taps == 3) KVA_SPACE_TOKEN(3);
     else KVA_SPACE_TOKEN(4);

@@ -76,7 +76,8 @@ def test_linear_attention(heads, dim, vdim, rank, entries, dtype, gpu):
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
 @pytest.mark.parametrize("heads, groups, n, vdim, norm_groups, taps, entries", [(32, 4, 128, 64, 4, 4, 2), (8, 8, 100, 24, 8, 3, 1), (4, 2, 16, 128, 4, 4, 5),
-                                                                               (3, 3, 33, 8, 3, 2, 3), (2, 2, 128, 512, 2, 4, 1), (16, 2, 64, 16, 16, 4, 2)])
+                                                                               (3, 3, 33, 8, 3, 2, 3), (2, 2, 128, 512, 2, 4, 1), (16, 2, 64, 16, 16, 4, 2),
+                                                                               (6, 3, 128, 64, 3, 4, 2), (3, 1, 100, 64, 1, 4, 3)])
 def test_state_space(heads, groups, n, vdim, norm_groups, taps, entries, dtype, gpu):
     g = torch.Generator().manual_seed(heads * n + vdim)
     inner, S = heads * vdim, heads * n * vdim
@@ -117,6 +118,20 @@ def test_what_does_not_fit_is_left_alone(gpu):
     assert delta()
     for other in (dict(heads=5), dict(dim=136), dict(vdim=60), dict(taps=5), dict(taps=1), dict(gate_off=4), dict(out_off=4), dict(state_off=2), dict(wide=4)):
         assert not delta(**other), other
+
+
+def test_state_space_of_many_requests(gpu):
+    """fp32 rows whose groups' columns take two passes stay with the three launches where workgroups are many."""
+    g = torch.Generator().manual_seed(0)
+    H, n, dv, taps = 8, 16, 64, 2
+    inner, S, C = H * dv, H * n * dv, H * dv + 2 * n
+    for dtype, entries, fits in ((torch.float32, 768, True), (torch.float32, 769, False), (torch.bfloat16, 769, True)):
+        y = numbers((entries, inner + C + H), g, dtype)
+        state, out = torch.zeros((entries, S + C), device="cuda"), torch.zeros((entries, inner), dtype=dtype, device="cuda")
+        one = torch.ones(H, device="cuda")
+        assert fits == K.state_space_token(y, inner, numbers((C, taps), g), None, state, 0, S, inner + C, one, one, one, torch.ones(inner, device="cuda"), 1e-5,
+                                           0, out, 0, 1.0, ints(np.arange(entries + 1)), ints(np.arange(entries)), H, 1, n, dv, 1)
+        assert bool(out.any()) == bool(state.any()) == fits
 
 
 def test_entries_without_a_token(gpu):
