@@ -306,7 +306,7 @@ delta_token_kernel(DeltaToken a) {
 }
 
 // ---- gated linear attention: grid (heads, entries) -----------------------------------------------------------------
-// The decays alpha = sigmoid(a2 (a1 columns of y) + bias)^(1 / tau), a channel by a thread, or handed in.
+// The decays alpha = sigmoid(a2 (a1 columns of y) + bias)^(1 / tau), a channel by a thread.
 struct LinearToken {
     TokenIO io;
     int q_off, k_off, v_off, a_off, rank;

@@ -134,21 +134,46 @@ def test_state_space_of_many_requests(gpu):
         assert bool(out.any()) == bool(state.any()) == fits
 
 
+def without_a_token(run, width, state):
+    """``run(state, out, starts, seats)`` over entries some of which have no token, against the others alone: their outputs and states, and
+    seats without a token keep theirs, the convolution's inputs among it."""
+    got, want = state.clone(), state.clone()
+    out = torch.zeros((2, width), device="cuda")
+    ref = out.clone()
+    assert run(got, out, ints([0, 0, 1, 1, 2]), ints([3, 0, 4, 2]))
+    assert run(want, ref, ints([0, 1, 2]), ints([0, 2]))
+    same([(out, ref), (got, want)])
+    assert torch.equal(got[[1, 3, 4]], state[[1, 3, 4]]) and not torch.equal(got[[0, 2]], state[[0, 2]])
+
+
 def test_entries_without_a_token(gpu):
     """More entries than rows: an entry without a token leaves its seat's state as it is."""
     g = torch.Generator().manual_seed(1)
     heads, dim, vdim, rank = 2, 64, 64, 16
-    starts, seats = ints([0, 0, 1, 1, 2]), ints([3, 0, 4, 2])
     y = numbers((2, 4 * heads * dim + 16), g)
     a2, bias, norm = numbers((heads * dim, rank), g, scale=0.3), numbers((heads * dim,), g), numbers((vdim,), g)
-    state = numbers((5, heads * dim * vdim), g)
-    got, want = state.clone(), state.clone()
-    out = torch.zeros((2, heads * vdim), device="cuda")
-    ref = out.clone()
     offs = (0, heads * dim, 2 * heads * dim, 4 * heads * dim)
-    assert K.gated_linear_attention_token(y, *offs, a2, bias, 3.5, 0.125, got, 0, norm, 1e-5, 3 * heads * dim, "silu", out, 0, 1.0, starts, seats,
-                                          heads, dim, vdim)
-    assert K.gated_linear_attention_token(y, *offs, a2, bias, 3.5, 0.125, want, 0, norm, 1e-5, 3 * heads * dim, "silu", ref, 0, 1.0, ints([0, 1, 2]),
-                                          ints([0, 2]), heads, dim, vdim)
-    same([(out, ref), (got, want)])
-    assert torch.equal(got[[1, 3, 4]], state[[1, 3, 4]])
+    without_a_token(lambda state, out, starts, seats: K.gated_linear_attention_token(
+        y, *offs, a2, bias, 3.5, 0.125, state, 0, norm, 1e-5, 3 * heads * dim, "silu", out, 0, 1.0, starts, seats, heads, dim, vdim),
+        heads * vdim, numbers((5, heads * dim * vdim), g))
+
+
+def test_delta_rule_of_entries_without_a_token(gpu):
+    g = torch.Generator().manual_seed(2)
+    heads, dim, vdim, taps = 2, 64, 64, 4
+    C, S = 2 * dim + heads * vdim, heads * dim * vdim
+    y, conv, norm, one = numbers((2, C + 8 + heads * vdim), g), numbers((C, taps), g, scale=0.5), numbers((vdim,), g), torch.ones(heads, device="cuda")
+    without_a_token(lambda state, out, starts, seats: K.gated_delta_rule_token(
+        y, 0, conv, state, 0, S, C, C + heads, one, one, None, 1e-6, norm, 1e-5, y, C + 8, "silu", out, 0, 1.0, starts, seats, heads, 1, dim, vdim),
+        heads * vdim, numbers((5, S + C * (taps - 1)), g))
+
+
+def test_state_space_of_entries_without_a_token(gpu):
+    g = torch.Generator().manual_seed(3)
+    heads, groups, n, vdim, taps = 4, 2, 32, 64, 4
+    inner, S = heads * vdim, heads * n * vdim
+    C = inner + 2 * groups * n
+    y, conv, norm, one = numbers((2, inner + C + 8), g), numbers((C, taps), g, scale=0.5), numbers((inner,), g), torch.ones(heads, device="cuda")
+    without_a_token(lambda state, out, starts, seats: K.state_space_token(
+        y, inner, conv, None, state, 0, S, inner + C, one, one, one, norm, 1e-5, 0, out, 0, 1.0, starts, seats, heads, groups, n, vdim, groups),
+        inner, numbers((5, S + C * (taps - 1)), g))
