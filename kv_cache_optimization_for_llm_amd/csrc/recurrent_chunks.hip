@@ -25,7 +25,9 @@
 // Where anything of an entry's inputs to a head is infinite or not a number, `prepare` says so and that (entry, head) is left
 // to the walk behind these kernels: zeros above a diagonal would carry it to tokens in front of it.
 // Order of sums: chunks are counted from the step's first token of the request, so here - unlike in the walk - the
-// last bits of a token's result depend on how the request was cut into steps.  The 32-bit path therefore walks.
+// last bits of a token's result depend on how the request was cut into steps, and, with the delta rule, now and then on how many
+// entries and heads the step has (how many value columns a workgroup takes orders the sums of 64-bit products).  The 32-bit
+// path therefore walks.
 //
 // us a call, the walk -> these three kernels (in 32 bits alone), one prompt of 2,048 / 8,192 tokens:
 //   delta rule, 8 heads of 128 x 128 over 4 key heads:  715 / 2,831 -> 119 / 447 (in 32 bits and 16 columns a workgroup 101 / 373)
@@ -800,7 +802,7 @@ static void ck_launch(const ChunkArgs &a, const ChunkInput &in, hipStream_t stre
     if (in.channel_decay) hipLaunchKernelGGL((chunk_prepare_kernel<D, DELTA, true>), grid, dim3(256), 0, stream, a, in);
     else hipLaunchKernelGGL((chunk_prepare_kernel<D, DELTA, false>), grid, dim3(256), 0, stream, a, in);
     // A chain's length is its chunks whatever the workgroups hold, so the columns go to as many as a turn of the 256 units takes.
-    // All three kernels at 4 / 8 / 16 columns a workgroup, heads of 128 x 128, us: 64 workgroups of 16 columns (8 heads, 2,048 tokens)
+    // All three kernels at 4 / 8 / 16 columns a workgroup, heads of 128 x 128, us (a run of its own, 2 % above the figures at the top): 64 workgroups of 16 columns (8 heads, 2,048 tokens)
     // 121 / 139 / 160, 128 (16 heads) 194 / 182 / 199, 256 (32 heads) 400 / 383 / 333; of 64 x 64: 16 (4 heads, 2,048) 72 / 79 / 93,
     // 128 (32 heads, 1,024) 98 / 95 / 101.
     const int tiles = a.heads * (a.vdim / 16), entries = min(a.entries, a.chunks);

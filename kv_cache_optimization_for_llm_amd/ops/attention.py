@@ -39,9 +39,11 @@ _WIDE_MIN_WAVES = 1024
 _PAIR_MIN_WAVES = 2048      # two items per wavefront once that still leaves a wavefront per SIMD
 # The workgroup kernel (128 query rows share each key block through LDS) pays one barrier per key
 # block: it wins once there are three workgroups per compute unit, or one per two units when the
-# rows visit thousands of keys each (measured: 2,048-token prompt from position 0 a tie, 4,096 1.5x;
-# portions of 512 tokens of an 8,192-token prompt, 128 workgroups, 5 % faster, and 25 % faster with
-# their keys cut into ranges so that about a thousand workgroups run; portions of 256 tokens no faster).
+# rows visit thousands of keys each and their keys are cut into ranges so that about a thousand workgroups
+# run.  Heads of 64, 32 over 8, us a call, one wavefront an item / two that share it / workgroups: one prompt of
+# 2,048 tokens (512 workgroups) 44 / 39 / 70, 2,304 61 / 46 / 49, 2,560 67 / 53 / 54, 2,816 74 / 60 / 59, 3,072 (768) 80 / 69 / 64, 4,096
+# 108 / 112 / 92, 8,190 459 / 402 / 303; 512 tokens behind 7,680 positions (128 workgroups, 8 key ranges) 78 / 91 / 58, 256
+# behind 4,096 (64) 34 / 44 / 34.
 _LDS_MIN_GROUPS = 128
 _LDS_MANY_GROUPS = 768
 _LDS_MIN_MEAN_KEYS = 2048
@@ -51,12 +53,12 @@ _LDS_SOME_GROUPS_MEAN_KEYS = 1024
 # one wavefront with two row tiles of them fills its SIMD's registers alone.  With keys laid out in
 # chunks of 8 elements across a page (one run of bytes per operand load) the one-wavefront kernel
 # holds out longer than it did: head size 128, one prompt from position 0, 24 heads, one-wavefront
-# against workgroup kernel: 1,024 tokens 31 against 36 us, 2,048 (384 workgroups) 61 against 71,
-# 2,560 (480) 80 against 91, but 3,072 (576) 163 against 112 and 4,096 221 against 161; 32 heads,
-# 2,560 tokens (640 workgroups) 142 against 97.  So: from 512 workgroups on, or where rows visit
-# 2,048 keys or more on average - with the keys cut into shorter ranges also for short portions deep
-# in a context (256 tokens at position 4,096: 48 us in 8 ranges against 71 for the one-wavefront
-# kernel at its best split; 128 at 8,192: 47 against 64; 64 at 8,192: 35 against 41).
+# against workgroup kernel: 1,536 tokens (288 workgroups) 42 against 47 us, 2,048 (384) 57 against 60,
+# 2,560 (480) 72 against 74, but 3,072 (576) 150 against 89 and 4,096 201 against 126; 32 heads, 1,536
+# (384) 44 against 47, 2,048 (512) 64 against 61, 2,560 (640) 129 against 78.  So: from 512 workgroups on,
+# or where rows visit 2,048 keys or more on average - with the keys cut into shorter ranges also for short portions
+# deep in a context (256 tokens at position 4,096: 38 us in 8 ranges against 49 for the one-wavefront
+# kernel; 128 at 8,192: 36 against 47; 64 at 8,192: 30 against 37).
 _LDS_MIN_MEAN_KEYS_WIDE_HEADS = 2048
 _LDS_MANY_GROUPS_WIDE_HEADS = 512
 _LDS_MIN_GROUPS_WIDE_HEADS = 16
@@ -84,22 +86,23 @@ def choose_portion_waves(waves: int, mean_keys: float, head_dim: int, own_keys: 
     One wavefront on two row tiles is a chain of products, softmax and products, 0.9 us a block of 32 keys with its SIMD to
     itself, and fixed key ranges with a merge kernel cost that kernel and leave early rows' ranges empty.  us a call without
     -> with, 32 heads of 64 over 8: one prompt of 256 / 512 / 1,024 / 1,536 / 2,048 / 2,304 / 2,560 tokens 14 / 26 / 22 / 34 /
-    44 / 51 / 56 -> 7 / 10 / 17 / 26 / 39 / 45 / 52 (3,072 the same, 4,096 94 -> 112 and from there the workgroup kernel);
+    44 / 51 / 56 -> 7 / 10 / 17 / 26 / 39 / 45 / 52 (2,816 59 / 59, 3,072 64 -> 69, 4,096 92 -> 112: the workgroup kernel);
     three of 509 20 -> 15; 256 tokens behind 1,024 / 4,096 / 8,000 24 / 35 / 49 -> 12 / 26 / 42, 1,024 behind 2,000 / 6,000
-    65 / 107 -> 41 / 92, 2,048 behind 2,000 / 6,000 112 / 201 -> 89 / 188.  Not so, and kept out: shares of a block or two (four
+    61 / 92 -> 42 / 89, 2,048 behind 2,000 / 4,000 101 / 134 -> 86 / 136 (behind 6,000, where the workgroup kernel is ahead by now, 168 ->
+    183).  Not so, and kept out: shares of a block or two (four
     of 64 6.7 -> 7.2, sixteen 8.2 -> 9.2), few pairs far behind, which more workgroups with a range each serve better (33
     tokens behind 1,024 12.5 -> 15.2, 64 behind 4,096 21 -> 24, 128 behind 8,000 32 -> 41; 8 heads over 8, 300 tokens behind 1,000
-    13.9 -> 17.5, 767 behind 2,000 25.8 -> 28.6), 512 behind 30,000 194 -> 199, 1,536 behind 20,000 358 -> 389, eight of 200
+    13.9 -> 17.5, 767 behind 2,000 25.8 -> 28.6), 512 behind 30,000 194 -> 199, 1,536 behind 20,000 330 -> 393, eight of 200
     10.4 -> 12.2.  Heads of 32 and 96 alike; pages of other sizes than 16, whose keys are looked up one by one, less far
     (128 behind 4,000 37 -> 52).  Behind a window key ranges of the whole context are mostly empty: 64 behind 2,000 with 256
     visible 15.5 -> 9.  (512 to 767 pairs from 2,048 keys on stay with the workgroup kernel and its key ranges, which the tests
-    of portions deep in a prompt rest on, though 512 / 640 tokens behind 2,000 would go 45 / 49 -> 26 / 33, behind 4,000 52 / 59 ->
-    37 / 51 and 640 behind 8,000 93 -> 86.)
+    of portions deep in a prompt rest on, though 512 / 640 tokens behind 2,000 would go 40 / 46 -> 23 / 31 and behind 4,000 48 / 54 ->
+    35 / 49; behind 8,000 60 / 73 -> 60 / 84.)
 
     Heads of 128 hold a SIMD's registers with one wavefront, so what there is to win ends earlier: 32 heads, 256 / 512 / 768
-    tokens 26 / 35 / 40 -> 10 / 14 / 19, 256 behind 1,024 / 4,096 34 / 41 -> 17 / 36, 512 behind 2,000 49 -> 36; 24 heads, 1,024
-    tokens 42 -> 22, four of 256 behind 1,000 57 -> 38; but four of 64 7.2 -> 8.1, four of 256 (32 heads) 13 -> 16, behind 1,000
-    38 -> 43, eight of 100 9.6 -> 11.9, eight of 100 behind 3,000 (16 heads) 63 -> 72, 512 behind 7,000 90 -> 104."""
+    tokens 26 / 34 / 40 -> 10 / 14 / 20, 256 behind 1,024 / 4,096 34 / 38 -> 17 / 38, 512 behind 2,000 46 -> 41; 24 heads, 1,024
+    tokens 42 -> 23, four of 256 behind 1,000 55 -> 38; but four of 64 7.2 -> 8.1, four of 256 (32 heads) 13 -> 16, behind 1,000
+    38 -> 43, eight of 100 9.6 -> 11.9, eight of 100 behind 3,000 (16 heads) 63 -> 72, 512 behind 7,000 83 -> 108."""
     if head_dim > 128:
         return 1
     keys = max((step for step in MEAN_KEYS_STEPS if step <= mean_keys), default=0)
@@ -142,9 +145,8 @@ def use_lds_kernel(groups: int, mean_keys: float, head_dim: int) -> bool:
         return groups >= _LDS_MIN_GROUPS_WIDE_HEADS and mean_keys >= _LDS_MIN_MEAN_KEYS
     if groups >= _LDS_MIN_GROUPS and mean_keys >= _LDS_MIN_MEAN_KEYS:
         return True
-    # Between 512 and 768 workgroups, whole prefill passes at the 1B sizes (one prompt from position 0):
-    # 2,048 tokens (512 workgroups) 5.74 ms with the one-wavefront kernel against 6.03, but 2,304 tokens
-    # 7.15 against 6.90, 2,560 7.66 against 7.36, 2,816 8.58 against 8.08.
+    # Between 512 and 768 workgroups, one prompt of 32 heads of 64 from position 0, one wavefront an item against this kernel: 2,048
+    # tokens (512 workgroups) 44 us against 70, but 2,304 (576) 61 against 49, 2,560 67 against 54, 2,816 74 against 59.
     return groups >= _LDS_SOME_GROUPS and mean_keys >= _LDS_SOME_GROUPS_MEAN_KEYS
 
 
