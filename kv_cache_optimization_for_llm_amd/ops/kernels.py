@@ -2682,7 +2682,8 @@ KERNEL_CLASSES = {
     "gemm_nt_f32": "gemm fp32", "gemm_vendor": "gemm (vendor library)",
     "gemm_skinny": "gemm (few rows)", "gemm_skinny_qkv_rope": "gemm (few rows)",
     "gemv": "gemm (few rows)", "gemv_qkv_rope": "gemm (few rows)", "gemv_merged": "gemm (few rows)",
-    "sample": "sampling", "mark_tokens": "sampling",
+    "gemm_skinny_partials": "gemm (few rows)",
+    "sample": "sampling", "sample_by_value": "sampling", "mark_tokens": "sampling",
     "causal_conv_act": "recurrent mixers", "gated_delta_rule": "recurrent mixers",
     "gated_linear_attention": "recurrent mixers", "head_norm_gate": "elementwise",
     "moe_route": "routed experts", "moe_router": "routed experts", "moe_align": "routed experts", "moe_table_align": "routed experts", "moe_expert_rows": "routed experts", "moe_few_rows": "routed experts",
@@ -2690,7 +2691,8 @@ KERNEL_CLASSES = {
     "norm_into_stream": "norm", "table_gate": "elementwise",
     "hyper_step": "norm", "sandwich_step": "norm", "hyper_fill": "embedding", "bias_act": "activation",
     "tanh_step": "norm", "pair_embed": "embedding", "maps_encode_cache": "rope + cache write", "maps_combine": "elementwise",
-    "state_space": "recurrent mixers",
+    "state_space": "recurrent mixers", "gated_delta_rule_token": "recurrent mixers",
+    "gated_linear_attention_token": "recurrent mixers", "state_space_token": "recurrent mixers",
     "block_gates": "recurrent mixers", "linear_scan_gate": "recurrent mixers", "matrix_memory": "recurrent mixers",
 }
 
