@@ -239,7 +239,7 @@ class Model:
         bf16 Linear that goes to the library at that many rows (``ops.gemm_bf16.tune_linear``;
         the same projection of all layers shares a shape and the layers' weights are used in
         turn).  Seconds per shape: start-up work.  Returns one record per (rows, shape)."""
-        from ..ops.gemm_bf16 import tune_linear, use_skinny
+        from ..ops.gemm_bf16 import SKINNY_WIDE_ROWS, tune_linear, use_skinny
         shapes: Dict[tuple, List[Linear]] = {}
         for lin in self.linears():
             if lin.weight.is_cuda and lin.weight.dtype == torch.bfloat16:
@@ -249,6 +249,9 @@ class Model:
             for (n, k, halves), lins in shapes.items():
                 if lins[0].tiled is not None and (use_skinny(rows, n, k, halves == 2) or use_skinny(rows, n, k)):
                     continue                                    # the few-rows kernel takes these
+                if lins[0].tiled is not None and rows > SKINNY_WIDE_ROWS \
+                        and K.gemm_tiles_plan(rows, n, k, K.TILES_GATED if halves == 2 else K.TILES_PLAIN) >= 0:
+                    continue                                    # the tiles of gemm_tiles.hip take these
                 first, best, tried = tune_linear(rows, [lin.weight for lin in lins[:16]])
                 report.append(dict(rows=rows, n=n, k=k, heuristic_us=round(first, 2), kept_us=round(best, 2),
                                    algorithms_run=tried))

@@ -3,9 +3,10 @@
 ``linear_bf16(x, w, out)`` computes ``out = x @ w^T`` with fp32 accumulation.  ``out`` may be
 bf16 or fp32.  Few rows (decode steps, short portions; how few depends on the matrix, see
 ``use_skinny``) take the hand-written matrix-core kernel that streams a tiled copy of the weight
-once (``csrc/gemm_skinny.hip``).  Other shapes go to the vendor GEMM library (hipBLASLt, called
-directly with the algorithm of a shape looked up once: ``csrc/gemm_vendor.hip``), which is where
-the reference's engine uses cuBLAS.
+once (``csrc/gemm_skinny.hip``).  More than 64 rows go to the tiles over the same copy
+(``csrc/gemm_tiles.hip``, where ``kernels.gemm_tiles_plan`` expects them to be faster) or to the vendor GEMM
+library (hipBLASLt, called directly with the algorithm of a shape looked up once: ``csrc/gemm_vendor.hip``),
+which is where the reference's engine uses cuBLAS.
 """
 from __future__ import annotations
 
@@ -63,7 +64,7 @@ def use_skinny(m: int, n: int, k: int, gated: bool = False, rotated: bool = Fals
 def use_partial_sums(m: int, n: int, k: int) -> bool:
     """17 to 64 rows of a product that goes into the residual stream and that the few-rows kernel
     does not take whole: its shared-X form over ranges of K (``kernels.gemm_skinny_partials``)
-    instead of the vendor library, the norm kernel adding the ranges up."""
+    instead of the vendor library, the norm kernel adding the ranges up.  (More rows: ``Linear._partial_tiles``.)"""
     return SKINNY_MAX_ROWS < m <= SKINNY_WIDE_ROWS and K.gemm_skinny_partial_ranges(m, n, k) >= 1
 
 
@@ -168,6 +169,12 @@ def linear_bf16(x: torch.Tensor, w: torch.Tensor, out: torch.Tensor, tiled=None)
         return K.gemv(x, w, out)
     if tiled is not None and use_skinny(x.shape[0], w.shape[0], w.shape[1]):
         return K.gemm_skinny(x, tiled, out)
+    if tiled is not None and out.dtype == torch.bfloat16 and x.shape[0] > SKINNY_WIDE_ROWS and tiled.halves == 1 \
+            and out.is_contiguous() and out.data_ptr() % 16 == 0 and K.gemm_tiles_takes(x, tiled):
+        # (a product that the library takes in two has its whole turns there: 2,048 rows of 8,208 outputs of 2,048 68 us, 72 in tiles)
+        plan = -1 if vendor_cut(x.shape[0], w.shape[0]) else K.gemm_tiles_plan(x.shape[0], w.shape[0], w.shape[1])
+        if plan >= 0:
+            return K.gemm_tiles(x, tiled, out, plan)
     cut = chosen_cut(x.shape[0], w.shape[0], w.shape[1], w.device, out.dtype) if out.is_contiguous() else 0
     if cut and K.gemm_vendor(x, w[:cut], out[:, :cut], columns=True) and K.gemm_vendor(x, w[cut:], out[:, cut:], columns=True):
         return out

@@ -141,7 +141,7 @@ def embed_gather_prep(table: torch.Tensor, ids: torch.Tensor, hidden: torch.Tens
 
 class PartialSums:
     """A branch output that has not been added up yet: ``parts`` fp32 ``[ranges, rows, width]``, the
-    products of :func:`gemm_skinny_partials` over ranges of K.  It stands where a bf16 ``[rows,
+    products of :func:`gemm_skinny_partials` or :func:`gemm_tiles` over ranges of K.  It stands where a bf16 ``[rows,
     width]`` delta stands; the norm kernel that adds the delta to the stream adds the ranges first
     (and rounds their sum to bf16, as the whole product would have been).  ``materialize()`` gives
     the plain delta."""
@@ -1475,6 +1475,35 @@ class TiledWeight:
         self.data = torch.cat(parts).contiguous()
 
 
+TILES_PLAIN, TILES_PARTS, TILES_GATED = 0, 1, 2
+
+
+def gemm_tiles_plan(m: int, n: int, k: int, form: int = TILES_PLAIN) -> int:
+    """How :func:`gemm_tiles` takes ``m`` rows of a ``[n, k]`` weight (a number for its ``plan``), or -1 where the vendor library is
+    expected to be faster or the kernel does not take the sizes.  ``plan >> 8``: the ranges of K that :data:`TILES_PARTS` leaves
+    (1: the whole product is faster)."""
+    return hip_lib().kva_gemm_tiles_plan(int(m), int(n), int(k), form)
+
+
+def gemm_tiles_takes(x: torch.Tensor, w: "TiledWeight") -> bool:
+    """Whether the rows lie as :func:`gemm_tiles` reads them."""
+    return x.dtype == torch.bfloat16 and x.dim() == 2 and x.shape[1] == w.k and x.is_contiguous() and x.data_ptr() % 16 == 0
+
+
+def gemm_tiles(x: torch.Tensor, w: "TiledWeight", out: torch.Tensor, plan: int, form: int = TILES_PLAIN, activation: str = "silu") -> torch.Tensor:
+    """x @ W^T of more than 64 bf16 rows on the matrix cores over the tiled copy of the weight.  ``out``: bf16 [M, N]; of a joined
+    [gate; up] weight (:data:`TILES_GATED`) bf16 [M, N / 2], act(gate) * up of the 32-bit sums; for :data:`TILES_PARTS` fp32 [ranges, M, N],
+    products over ranges of K."""
+    m, k = x.shape
+    shape = (m, w.n) if form == TILES_PLAIN else (m, w.n // 2) if form == TILES_GATED else (plan >> 8, m, w.n)
+    if not gemm_tiles_takes(x, w) or w.halves != (2 if form == TILES_GATED else 1) or tuple(out.shape) != shape \
+            or out.dtype != (torch.float32 if form == TILES_PARTS else torch.bfloat16):
+        raise KernelError(f"gemm_tiles: x {tuple(x.shape)} {x.dtype}, weight [{w.n}, {w.k}] in {w.halves}, out {tuple(out.shape)} {out.dtype} do not fit")
+    check(hip_lib().kva_gemm_tiles(_dev(out, "out"), _dev(x, "x"), _dev(w.data, "w"), m, w.n, k, form, plan,
+                                   ACTIVATIONS[activation], _stream()), "gemm_tiles")
+    return out
+
+
 class TiledRows:
     """At most 64 rows of ``width`` bf16 columns laid out ``[width / 8, R, 8]`` with ``R`` the row
     count rounded up to a multiple of 16, or 8 for up to 8 rows (the library says which:
@@ -2679,7 +2708,7 @@ KERNEL_CLASSES = {
     "heads_matmul": "per-head products",
     "attention_mfma_rope": "attention", "attention_merge_gated": "attention",
     "latent_prompt": "attention (matrix cores)",
-    "gemm_nt_f32": "gemm fp32", "gemm_vendor": "gemm (vendor library)",
+    "gemm_nt_f32": "gemm fp32", "gemm_vendor": "gemm (vendor library)", "gemm_tiles": "gemm (tiles)",
     "gemm_skinny": "gemm (few rows)", "gemm_skinny_qkv_rope": "gemm (few rows)",
     "gemv": "gemm (few rows)", "gemv_qkv_rope": "gemm (few rows)", "gemv_merged": "gemm (few rows)",
     "gemm_skinny_partials": "gemm (few rows)",

@@ -88,6 +88,8 @@ _HIP_SIGNATURES = {
     "kva_gemm_nt_f32": [P, P, P, I, I, I, I, I, I, P],
     "kva_gemm_vendor": [P, P, P, I, I, I, I, I, I, P],
     "kva_gemm_vendor_init": [],
+    "kva_gemm_tiles_plan": [I, I, I, I],
+    "kva_gemm_tiles": [P, P, P, I, I, I, I, I, I, P],
     "kva_gemm_vendor_tune": [P, P, P, I, I, I, I, I, I, I, P, P, P, P],
     "kva_gemm_vendor_forget": [I, I, I, I, I, I],
     "kva_host_memory_is_mapped": [P],

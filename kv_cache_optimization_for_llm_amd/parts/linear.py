@@ -3,7 +3,7 @@
 The reference calls cublasGemmEx for this (bf16 operands, fp32 accumulate,
 ``base/src/engine.cu:652-671``).  Here:
 
-* bf16 weight, bf16 activations: hand-written MFMA kernels where they exist for the shape,
+* bf16 weight, bf16 activations: hand-written MFMA kernels where they are the faster ones for the shape,
   otherwise the vendor GEMM library (``ops.kernels.gemm_vendor``, as the reference uses cuBLAS);
 * fp32 weight: the true-fp32 kernel ``gemm_nt_f32``; bf16 activations are widened for it and
   the result is rounded back, so a tensor stored in 32-bit is used in 32-bit.
@@ -26,7 +26,8 @@ class Linear:
         self.weight = weight.contiguous()
         self.out_features, self.in_features = weight.shape
         self.halves = halves
-        # a second, tiled copy for the few-rows kernel (decode); the plain layout serves prompts
+        # a second, tiled copy for the few-rows kernel (decode) and the tiles of more than 64 rows; the plain layout
+        # serves the vendor library and one or two rows
         self.tiled = None
         if weight.is_cuda and weight.dtype == torch.bfloat16:
             K.gemm_vendor_init()            # the library's handle and workspace exist before any step
@@ -79,13 +80,14 @@ class Linear:
 
     def into_residual(self, x, tail: BranchTail):
         """hidden += x @ W^T in place and the sum prepared for ``tail.norm`` (NormedRows); or, at
-        17 to 64 rows of a matrix that the few-rows kernel does not take whole, the product as
+        17 rows and more of a matrix that the few-rows kernel does not take whole, the product as
         ``ops.kernels.PartialSums`` for a ``tail.norm`` that says it adds them up
         (``takes_partial_sums``); ``None`` when neither is possible (the caller then takes the
         plain product)."""
+        from ..ops.gemm_bf16 import SKINNY_WIDE_ROWS
         kernel = self.residual_kernel(x.shape[0], x.dtype, tail)
         if kernel is None:
-            return self._partial_sums(x, tail)
+            return self._partial_sums(x, tail) if x.shape[0] <= SKINNY_WIDE_ROWS else self._partial_tiles(x, tail)
         next_w, width, eps = tail.norm.prepared_by_product()
         rows = x.shape[0]
         scaled = torch.empty((rows, self.out_features), dtype=torch.bfloat16, device=x.device)
@@ -119,6 +121,33 @@ class Linear:
                 or self.out_features % 8 or not use_partial_sums(x.shape[0], self.out_features, self.in_features):
             return None
         return K.gemm_skinny_partials(x, self.tiled)
+
+    def _partial_tiles(self, x, tail: Optional[BranchTail]):
+        """More than 64 rows: the product over ranges of K where that is expected to be faster than the whole one, what the norm reads
+        more of included (``kernels.gemm_tiles_plan``)."""
+        if tail is None or not getattr(tail.norm, "takes_partial_sums", False) or self.tiled is None or self.halves != 1 \
+                or not isinstance(x, torch.Tensor) or tail.hidden.dtype != torch.bfloat16 or self.out_features % 8 \
+                or not K.gemm_tiles_takes(x, self.tiled):
+            return None
+        plan = K.gemm_tiles_plan(x.shape[0], self.out_features, self.in_features, K.TILES_PARTS)
+        if plan < 0 or plan >> 8 < 2:
+            return None
+        parts = torch.empty((plan >> 8, x.shape[0], self.out_features), dtype=torch.float32, device=x.device)
+        return K.PartialSums(K.gemm_tiles(x, self.tiled, parts, plan, K.TILES_PARTS))
+
+    def gated_tiles(self, x, activation: str):
+        """act(x gate^T) * (x up^T) of more than 64 rows for a joined [gate; up] weight, the activation applied to the product's sums;
+        ``None`` where the library's product and the activation's own kernel are expected to be faster, or rows and weight are not of
+        the kinds that ``kernels.gemm_tiles`` takes."""
+        from ..ops.gemm_bf16 import SKINNY_WIDE_ROWS
+        if self.tiled is None or self.halves != 2 or not isinstance(x, torch.Tensor) or x.shape[0] <= SKINNY_WIDE_ROWS \
+                or not K.gemm_tiles_takes(x, self.tiled):
+            return None
+        plan = K.gemm_tiles_plan(x.shape[0], self.out_features, self.in_features, K.TILES_GATED)
+        if plan < 0:
+            return None
+        out = torch.empty((x.shape[0], self.out_features // 2), dtype=x.dtype, device=x.device)
+        return K.gemm_tiles(x, self.tiled, out, plan, K.TILES_GATED, activation)
 
     def gated(self, x, out, activation: str = "silu") -> None:
         """``out`` = act(x gate^T) * (x up^T) for a joined [gate; up] weight whose rows

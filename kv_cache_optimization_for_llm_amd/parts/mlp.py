@@ -89,17 +89,19 @@ class SwiGLU(FeedForward):
         # the other in the order the second one's lanes read them (ops.kernels.TiledRows).
         tiled = (up_kernel == Linear.FEW_ROWS and rows <= K.TiledRows.MAX_ROWS and self.intermediate_size % 8 == 0
                  and self.down.residual_kernel(rows, x.dtype, tail) == Linear.FEW_ROWS)
-        if tiled:
-            act = K.TiledRows(rows, self.intermediate_size, x.device)
-        else:
-            act = torch.empty((rows, self.intermediate_size), dtype=x.dtype, device=x.device)
-        if up_kernel is not None:
-            # activation fused into the product; an unfinished input norm is finished there too
-            self.gate_up.gated(x, act, self.activation)
-        elif self.activation == "silu":
-            K.silu_mul(self.gate_up(x), act)
-        else:
-            K.act_mul(self.gate_up(x), act, self.activation, self.limit)
+        act = None
+        if up_kernel is None and self.activation in K.ACTIVATIONS:
+            act = self.gate_up.gated_tiles(x, self.activation)      # (many rows: the activation is applied to the product's sums)
+        if act is None:
+            act = K.TiledRows(rows, self.intermediate_size, x.device) if tiled else \
+                torch.empty((rows, self.intermediate_size), dtype=x.dtype, device=x.device)
+            if up_kernel is not None:
+                # activation fused into the product; an unfinished input norm is finished there too
+                self.gate_up.gated(x, act, self.activation)
+            elif self.activation == "silu":
+                K.silu_mul(self.gate_up(x), act)
+            else:
+                K.act_mul(self.gate_up(x), act, self.activation, self.limit)
         if tail is not None:
             fused = self.down.into_residual(act, tail)
             if fused is not None:
