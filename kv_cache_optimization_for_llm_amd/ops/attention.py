@@ -150,6 +150,26 @@ def use_lds_kernel(groups: int, mean_keys: float, head_dim: int) -> bool:
     return groups >= _LDS_SOME_GROUPS and mean_keys >= _LDS_SOME_GROUPS_MEAN_KEYS
 
 
+# The workgroup kernel's other forms (csrc/attention_lds.hip, with both sides), by workgroups of 128 rows over all kv heads.  Two groups of
+# wavefronts: heads up to 64 from 448 to 699 workgroups whose rows visit 1,024 keys and more (fewer keys: 1,531 and 963 tokens, 632 workgroups, 35 us
+# against 34 by two wavefronts an item; fewer workgroups: 1,536 tokens, 384, 26 against 26), above 96 from 272 to 544 that visit 512 and more, to 659 below 1,024
+# (256 workgroups: 2,048 tokens of 16 heads over 8 42 against 41; 576: 2,304 of 32 71 against 66 in blocks of 64).  Blocks of 64 keys: heads up to
+# 64 from 700 workgroups on (8,190 tokens, 2,048: 318 -> 312), above 96 from 545 to 899 and from 1,100 to 1,535 (1,024 workgroups are two full turns with two a
+# unit, where three a unit make one and a third: 4,096 tokens of 32 heads 148 -> 156; 2,048: 528 -> 537).
+LDS_BLOCKS_OF_32, LDS_BLOCKS_OF_64, LDS_TWO_GROUPS = 0, 1, 2
+_TWO_GROUPS = {False: ((448, 700, 1024, 1 << 30),), True: ((272, 545, 512, 1 << 30), (545, 660, 512, 1024))}       # from, below; mean keys from, below
+_LONG_BLOCKS = {False: ((700, 1 << 30),), True: ((545, 900), (1100, 1536))}
+
+
+def choose_lds_kind(groups: int, mean_keys: float, head_dim: int, by_workgroup: bool) -> int:
+    """Which form of the workgroup kernel takes ``groups`` workgroups of rows that visit ``mean_keys`` keys on average; ``by_workgroup``:
+    they go to that kernel in any case.  (Two groups are also ahead of the one-wavefront kernel, so its lines do not hold there.)"""
+    wide = head_dim > 96
+    if any(a <= groups < b and lo <= mean_keys < hi for a, b, lo, hi in _TWO_GROUPS[wide]):
+        return LDS_TWO_GROUPS
+    return LDS_BLOCKS_OF_64 if by_workgroup and any(a <= groups < b for a, b in _LONG_BLOCKS[wide]) else LDS_BLOCKS_OF_32
+
+
 def _cut_keys(want: int, max_context: int, max_splits: int) -> tuple:
     """``max_context`` keys in at most ``min(want, max_splits)`` ranges of a multiple of 32 keys."""
     splits = min(want, max_splits)
@@ -515,35 +535,43 @@ def paged_attention(qkv: torch.Tensor, out: torch.Tensor, kv, batch, num_q_heads
             if left:
                 return got
         else:
-            _, meta, splits, per, covers_all = launch
+            _, meta, splits, per, covers_all, kind = launch
             K.attention_lds(qkv, stride, out, kv.k_cache, kv.v_cache, kv.block_table, meta, num_q_heads,
-                            num_kv_heads, head_dim, scale, window, False, splits, per, covers_all_rows=covers_all)
+                            num_kv_heads, head_dim, scale, window, False, splits, per, covers_all_rows=covers_all, kind=kind)
     return out
 
 
 def portion_choice(lens, mean_keys: float, group: int, num_kv_heads: int, head_dim: int, page_size: int, visible: int = 0) -> tuple:
-    """(:func:`choose_portion_waves`, whether prompt portions go to the workgroup kernel) for a step whose entries have ``lens``
-    tokens: all that the step's mean number of keys decides, and so what tells captured shapes of the same entries apart."""
+    """(:func:`choose_portion_waves`, 0 or one more than the form of the workgroup kernel that prompt portions go to,
+    :func:`choose_lds_kind`) for a step whose entries have ``lens`` tokens: all that the step's mean number of keys decides, and so what tells
+    captured shapes of the same entries apart."""
     rows = [n * group for n in lens]
     if max(rows) <= 16:
-        return 1, False
+        return 1, 0
     mixed = min(rows) <= 16
     long = [n for n in rows if not mixed or n > 16]
+    groups = sum(-(-n // 128) for n in long) * num_kv_heads
+    workgroups = K.attention_lds_supported(head_dim, page_size)
+    # (behind a window most of a context is skipped: as before)
+    if workgroups and not 0 < visible < mean_keys and choose_lds_kind(groups, mean_keys, head_dim, False) == LDS_TWO_GROUPS:
+        return 1, 1 + LDS_TWO_GROUPS
     tiles = K.attention_mfma_row_tiles(head_dim, True)
     if tiles == 2:
         # (its own tokens are known exactly, keys in front of a portion to the step of MEAN_KEYS_STEPS)
         own_keys = sum(n * n for n in long) / (2 * group * sum(long))
         sharing = choose_portion_waves(sum(-(-n // 32) for n in long) * num_kv_heads, mean_keys, head_dim, own_keys, page_size, group, visible)
         if sharing > 1:
-            return sharing, False
-    groups = sum(-(-n // 128) for n in long) * num_kv_heads
-    return 1, bool(K.attention_lds_supported(head_dim, page_size)) and use_lds_kernel(groups, mean_keys, head_dim)
+            return sharing, 0
+    if not workgroups or not use_lds_kernel(groups, mean_keys, head_dim):
+        return 1, 0
+    kind = choose_lds_kind(groups, mean_keys, head_dim, True)
+    return 1, 1 + (LDS_BLOCKS_OF_32 if kind == LDS_TWO_GROUPS else kind)
 
 
 def _plan(batch, group: int, num_kv_heads: int, head_dim: int, page_size: int, max_parts: int = 0, visible: int = 0) -> list:
     """The launches of one attention call over ``batch`` (``visible`` > 0: a token sees about so many keys at most): ("wave", items, row tiles, splits, keys per
     split, pair, covers all rows, keep cached, wavefronts of a workgroup that share an item) and
-    ("lds", item records, splits, keys per split, covers all rows)."""
+    ("lds", item records, splits, keys per split, covers all rows, form of the kernel)."""
     plan = []
 
     def decoded(which):
@@ -584,8 +612,9 @@ def _plan(batch, group: int, num_kv_heads: int, head_dim: int, page_size: int, m
     if by_workgroup:
         items = batch.attention_items(group, 8, which)
         if items[2] is not None:
-            splits, per = choose_lds_splits(items[0].shape[0] * num_kv_heads, batch.max_context, head_dim=head_dim)
-            plan.append(("lds", items[2], splits, per, which == "all"))
+            kind = by_workgroup - 1
+            splits, per = (1, 0) if kind else choose_lds_splits(items[0].shape[0] * num_kv_heads, batch.max_context, head_dim=head_dim)
+            plan.append(("lds", items[2], splits, per, which == "all", kind))
             done = True
     if not done:
         # whole key ranges as long as that gives a wave per SIMD
