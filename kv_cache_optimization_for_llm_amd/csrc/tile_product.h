@@ -40,12 +40,18 @@ struct TileProduct {
     // rows m0 .. m0 + ROWS - 1 of x (past the last one the last one again); tile_of(j): which tile of w is the workgroup's j-th
     template <class F>
     __device__ __forceinline__ void init(const bf16_t *x, int M, int m0, const bf16_t *w, int tiles, int K, F tile_of) {
-        const int lane = threadIdx.x % KVA_WAVE, wave = __builtin_amdgcn_readfirstlane(threadIdx.x / KVA_WAVE), rows = min(ROWS, M - m0);
-        xbuf = buffer_at(x + (size_t)m0 * K, (size_t)rows * K * 2);
+        const int rows = min(ROWS, M - m0);
+        init(buffer_at(x + (size_t)m0 * K, (size_t)rows * K * 2), [&](int i) { return min(i, rows - 1); }, w, tiles, K, tile_of);
+    }
+    // row_of(i): which row of the buffer is the workgroup's i-th
+    template <class R, class F>
+    __device__ __forceinline__ void init(Buffer x, R row_of, const bf16_t *w, int tiles, int K, F tile_of) {
+        const int lane = threadIdx.x % KVA_WAVE, wave = __builtin_amdgcn_readfirstlane(threadIdx.x / KVA_WAVE);
+        xbuf = x;
         wbuf = buffer_at(w, (size_t)tiles * 16 * K * 2);
 #pragma unroll
         for (int i = 0; i < XI; ++i)
-            xo[i] = 2 * (min(8 * x_piece(wave, i) + lane / 8, rows - 1) * K + 8 * ((lane % 8) ^ (lane / 8)));
+            xo[i] = 2 * (row_of(8 * x_piece(wave, i) + lane / 8) * K + 8 * ((lane % 8) ^ (lane / 8)));
 #pragma unroll
         for (int i = 0; i < WI; ++i) {
             const int piece = w_piece(wave, i);
@@ -55,6 +61,10 @@ struct TileProduct {
 
     // Elements k_begin .. k_end - 1 (both multiples of KS, at least one stage).  acc[nt][rt]: lane (r = lane % 16, g = lane / 16) gets
     // outputs 16 (NT wn + nt) + 4 g .. + 3 of row 16 (RT wr + rt) + r.
+    // PAIRED: rows 2 j and 2 j + 1 of w are the gate and the up row of output j.  Two tiles hold 16 of them, and of each pair of tiles
+    // (nt even) the lane gets the gate and the up rows of outputs 8 (NT wn + nt) + 4 g .. + 3: gates in acc[nt] and ups in acc[nt + 1]
+    // where g < 2, the other way round where g >= 2 (so that the 16 rows read at once lie in different banks).
+    template <bool PAIRED = false>
     __device__ __forceinline__ void run(Shared &s, int k_begin, int k_end, f32x4 (&acc)[NT][RT]) const {
         const int lane = threadIdx.x % KVA_WAVE, wave = __builtin_amdgcn_readfirstlane(threadIdx.x / KVA_WAVE), r = lane & 15, g = lane >> 4;
         const int wk = wave / (WR * WN), wr = wave % WR, wn = wave / WR % WN;
@@ -63,7 +73,8 @@ struct TileProduct {
 #pragma unroll
         for (int j = 0; j < KSUB; ++j)
             xat[j] = (2 * wr * RT + r / 8) * 512 + (r % 8) * 64 + 8 * ((4 * (wk * KSUB + j) + g) ^ (r % 8));
-        const int wat = (wn * NT * STEPS + wk * KSUB) * 512 + 8 * lane;
+        const int wat = (wn * NT * STEPS + wk * KSUB) * 512 + (PAIRED ? r / 8 * STEPS * 512 + 8 * (16 * g + 2 * (r % 8) + r / 8) : 8 * lane);
+        const int odd = PAIRED ? 8 * (1 - 2 * (r / 8)) - STEPS * 512 : 0;       // elements from an even tile's place to the next one's
         auto load = [&](int i, int slot, int k0) {
             const int k = min(k0, last);
             if (i < XI) buffer_to_lds(xbuf, xo[i], 2 * k, &s.x[slot][x_piece(wave, i) * 512]);
@@ -72,7 +83,7 @@ struct TileProduct {
         b16x8 xf[2][RT], wf[2][NT];
         auto read = [&](int i, int set, int slot, int j) {
             if (i < RT) xf[set][i] = *reinterpret_cast<const b16x8 *>(&s.x[slot][xat[j] + i * 1024]);
-            else wf[set][i - RT] = *reinterpret_cast<const b16x8 *>(&s.w[slot][wat + ((i - RT) * STEPS + j) * 512]);
+            else wf[set][i - RT] = *reinterpret_cast<const b16x8 *>(&s.w[slot][wat + ((i - RT) * STEPS + j) * 512 + ((i - RT) % 2 ? odd : 0)]);
         };
 #pragma unroll
         for (int nt = 0; nt < NT; ++nt)

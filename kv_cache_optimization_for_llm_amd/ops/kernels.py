@@ -2506,6 +2506,37 @@ def moe_expert_rows(x: torch.Tensor, w: torch.Tensor, out: torch.Tensor, sorted_
     return out
 
 
+def moe_tiles_plan(slots: int, experts: int, top: int, n: int, k: int, second: bool) -> int:
+    """How :func:`moe_expert_tiles` takes ``slots`` (token, choice) pairs of ``experts``, ``top`` of them a token, against matrices ``[n, k]`` in
+    the first or the second product (a number for its ``plan``), or -1: it does not take the sizes, or :func:`moe_expert_rows` in groups
+    is expected to be faster."""
+    return hip_lib().kva_moe_tiles_plan(int(slots), int(experts), int(top), int(n), int(k), 1 if second else 0)
+
+
+def moe_expert_tiles(x: torch.Tensor, w: torch.Tensor, out: torch.Tensor, sorted_slot: torch.Tensor, tile_expert: torch.Tensor, top: int,
+                     plan: int, *, activation: Optional[str] = None, slot_weight: Optional[torch.Tensor] = None, gated: bool = False,
+                     limit: float = 0.0) -> torch.Tensor:
+    """:func:`moe_expert_rows` for many bf16 rows an expert, matrices in operand order: a workgroup takes as many
+    neighbouring tiles of one expert as ``plan`` (:func:`moe_tiles_plan`) says, of a list with or without groups."""
+    tiles, first = tile_expert.shape[0], activation is not None
+    n_out = w.shape[1] // 2 if gated else w.shape[1]
+    if first and activation not in EXPERT_ACTIVATIONS:
+        raise KernelError(f"moe_expert_tiles: activation {activation!r} is not one of {sorted(EXPERT_ACTIVATIONS)}")
+    if w.dim() != 3 or w.dtype != torch.bfloat16 or x.dtype != torch.bfloat16 or x.dim() != 2 or x.shape[1] != w.shape[2] or out.dim() != 2 \
+            or out.shape[1] != n_out or sorted_slot.shape != (tiles * MOE_TILE,) or (gated and (not first or w.shape[1] % 2)):
+        raise KernelError(f"moe_expert_tiles: x {tuple(x.shape)}, w {tuple(w.shape)}, out {tuple(out.shape)} do not fit")
+    places, rows = (out, x) if first else (x, out)
+    if places.shape[0] != tiles * MOE_TILE or out.dtype != (torch.bfloat16 if first else torch.float32):
+        raise KernelError("moe_expert_tiles: the first product writes a bf16 row per sorted place, the second reads those and writes fp32 rows per slot")
+    if slot_weight is not None and (slot_weight.dtype != torch.float32 or slot_weight.numel() != (rows.shape[0] * int(top) if first else rows.shape[0])):
+        raise KernelError("moe_expert_tiles: one fp32 weight per (token, choice) slot")
+    check(hip_lib().kva_moe_tiles(
+        _dev(out, "out"), _dev(x, "x"), _dev(w, "w"), _dev(sorted_slot, "sorted_slot", torch.int32), _dev(tile_expert, "tile_expert", torch.int32),
+        _opt(slot_weight, "slot_weight"), tiles, w.shape[0], int(top), w.shape[1], w.shape[2], 0 if first else 1,
+        EXPERT_ACTIVATIONS.get(activation, 0), 1 if gated else 0, float(limit), int(plan), _stream()), "moe_tiles")
+    return out
+
+
 def moe_few_max_tokens() -> int:
     """Up to so many tokens :func:`moe_few_rows` takes."""
     return int(hip_lib().kva_moe_few_max_tokens())

@@ -191,6 +191,13 @@ class RoutedExperts(FeedForward):
         # the shared expert's gate: one number a token, in 32-bit; its sigmoid is taken where the rows are added
         return product[:, self.outputs] if self.shared_gate is not None else None
 
+    def _tile_plans(self, x, slots: int):
+        """For both products the plan where a workgroup takes what rows of an expert there are (ops.kernels.moe_expert_tiles), or -1."""
+        if not self.tiled or x.data_ptr() % 16:
+            return -1, -1
+        return tuple(K.moe_tiles_plan(slots, self.experts, self.top, w.shape[1], w.shape[2], second)
+                     for w, second in ((self.w_up, False), (self.w_down, True)))
+
     def _few(self, x) -> bool:
         # (rows that start at no multiple of 16 bytes keep the list: its kernels take them)
         return not self.lists_few and x.dtype == torch.bfloat16 and 0 < x.shape[0] <= K.moe_few_max_tokens() and x.data_ptr() % 16 == 0
@@ -223,6 +230,9 @@ class RoutedExperts(FeedForward):
         slots, gate = T * self.top, None
         few = self._few(x)
         group = K.moe_group(slots, self.experts, x.dtype, self.hidden_size, self.intermediate_size) if self.experts else 1
+        plans = self._tile_plans(x, slots) if group > 1 and not few else (-1, -1)
+        if min(plans) >= 0:
+            group = 1                       # (a list in groups is for moe_expert_rows)
         table = router = None
         rule = dict(scores=self.scores, groups=self.groups, keep_groups=self.keep_groups, group_top=self.group_top,
                     weight_scale=self.weight_scale, sum_eps=self.sum_eps)
@@ -266,10 +276,17 @@ class RoutedExperts(FeedForward):
             if self.experts:
                 act = torch.empty((sorted_slot.shape[0], self.intermediate_size), dtype=x.dtype, device=dev)
                 first, second = (wgt, None) if self.weight_input else (None, wgt)
-                K.moe_expert_rows(x, self.w_up, act, sorted_slot, tile_expert, self.top, activation=self.activation,
-                                  slot_weight=first, gated=self.gated, limit=self.limit, group=group, tiled=self.tiled)
-                K.moe_expert_rows(act, self.w_down, rows, sorted_slot, tile_expert, self.top, slot_weight=second, group=group,
-                                  tiled=self.tiled)
+                if plans[0] >= 0:
+                    K.moe_expert_tiles(x, self.w_up, act, sorted_slot, tile_expert, self.top, plans[0], activation=self.activation,
+                                       slot_weight=first, gated=self.gated, limit=self.limit)
+                else:
+                    K.moe_expert_rows(x, self.w_up, act, sorted_slot, tile_expert, self.top, activation=self.activation,
+                                      slot_weight=first, gated=self.gated, limit=self.limit, group=group, tiled=self.tiled)
+                if plans[1] >= 0:
+                    K.moe_expert_tiles(act, self.w_down, rows, sorted_slot, tile_expert, self.top, plans[1], slot_weight=second)
+                else:
+                    K.moe_expert_rows(act, self.w_down, rows, sorted_slot, tile_expert, self.top, slot_weight=second, group=group,
+                                      tiled=self.tiled)
             extra = self.shared.forward(x, ctx) if self.shared is not None else None
         out = K.ExpertRows(x, rows, idx, wgt, self.experts, extra, gate)
         return out if self.leaves_rows and self.identity == 0 else out.sum()
