@@ -169,6 +169,121 @@ __global__ void rope_kv_write_vec_kernel(T *__restrict__ qkv, T *__restrict__ k_
     }
 }
 
+// Many tokens in bf16: a workgroup takes 16 neighbouring tokens and some of the heads, q's, k's or v's (blockIdx.y).  With a
+// workgroup a token the cache bounds it: neighbouring tokens' keys and values share cache lines, an element of V goes a page's row
+// further than the one before it, and eight dies write 16 and 2 bytes of a line each.  Here a line is one workgroup's, and eight
+// keys that fill eight aligned places of a page go out as 16 bytes of V at a time, turned round in LDS.  A thread keeps its token's
+// cosines and sines over all of its heads.  us, before and now: 1,203 tokens (portions that begin anywhere) / 2,048 of 32 + 2 x 8
+// heads of 64 8.5 / 12.1 -> 7.6 / 8.1 (3 TB/s), 8,190 of 128 75 -> 41 (4.9 TB/s).  (Runs of four and two keys as one store, too: 9.2 at
+// 1,203 tokens, the search for them takes longer than the stores.)
+#define ROPE_TOKENS 16
+#define ROPE_HEADS 2                    // of q or k a thread takes at once
+#define ROPE_V_COLS 256
+
+struct RopeWide {
+    bf16_t *qkv, *k_cache, *v_cache;
+    const float *cos_table, *sin_table;
+    const int *positions, *slot_mapping;        // slot_mapping absent: no cache
+    int tokens, num_q_heads, num_kv_heads, head_dim, page_size;
+    int lanes, q_blocks, k_blocks;              // threads that share a token's chunk; workgroups of 16 tokens' q and k heads
+};
+
+__global__ void __launch_bounds__(256)
+rope_kv_write_wide_kernel(RopeWide a) {
+    __shared__ __attribute__((aligned(16))) uint16_t turn[ROPE_TOKENS][ROPE_V_COLS + 8];
+    const int t0 = blockIdx.x * ROPE_TOKENS, d = a.head_dim, half = d / 2, chunks = half / 8, tid = threadIdx.x;
+    const size_t row_width = (size_t)(a.num_q_heads + 2 * a.num_kv_heads) * d;
+    int block = blockIdx.y;
+    if (block < a.q_blocks + a.k_blocks) {
+        const bool keys = block >= a.q_blocks;
+        if (keys) block -= a.q_blocks;
+        // q: a token's chunks and heads by neighbouring threads, as they lie in the row; k: the tokens, as they lie in the cache
+        const int per = chunks * a.lanes, token = keys ? tid % ROPE_TOKENS : tid / per, rest = keys ? tid / ROPE_TOKENS : tid % per, t = t0 + token;
+        if (token >= ROPE_TOKENS || rest >= per || t >= a.tokens) return;
+        const int chunk = rest % chunks, lane = rest / chunks, p0 = 8 * chunk, heads = keys ? a.num_kv_heads : a.num_q_heads;
+        const int slot = keys ? a.slot_mapping[t] : 0;
+        if (slot < 0) return;
+        bf16_t *row = a.qkv + (size_t)t * row_width + (keys ? (size_t)a.num_q_heads * d : 0);
+        const float *cs = a.cos_table + (size_t)a.positions[t] * half + p0, *sn = a.sin_table + (size_t)a.positions[t] * half + p0;
+        float x1[ROPE_HEADS][8], x2[ROPE_HEADS][8], c[8], s[8];
+        const int head0 = block * a.lanes * ROPE_HEADS + lane;
+#pragma unroll
+        for (int i = 0; i < ROPE_HEADS; ++i) {
+            const bf16_t *h = row + (size_t)min(head0 + i * a.lanes, heads - 1) * d + p0;
+            RopeVec<bf16_t>::load(h, x1[i]);
+            RopeVec<bf16_t>::load(h + half, x2[i]);
+        }
+#pragma unroll
+        for (int j = 0; j < 8; j += 4) {
+            const float4 cv = *reinterpret_cast<const float4 *>(cs + j), sv = *reinterpret_cast<const float4 *>(sn + j);
+            c[j] = cv.x; c[j + 1] = cv.y; c[j + 2] = cv.z; c[j + 3] = cv.w;
+            s[j] = sv.x; s[j + 1] = sv.y; s[j + 2] = sv.z; s[j + 3] = sv.w;
+        }
+#pragma unroll
+        for (int i = 0; i < ROPE_HEADS; ++i) {
+            const int head = head0 + i * a.lanes;
+            if (head >= heads) return;
+            float o1[8], o2[8];
+#pragma unroll
+            for (int j = 0; j < 8; ++j) {
+                o1[j] = fmaf(x1[i][j], c[j], -(x2[i][j] * s[j]));       // (as the compiler contracts it in the other kernels)
+                o2[j] = fmaf(x2[i][j], c[j], x1[i][j] * s[j]);
+            }
+            bf16_t *to1 = row + (size_t)head * d + p0, *to2 = to1 + half;
+            if (keys) {
+                bf16_t *dst = a.k_cache + ((size_t)(slot / a.page_size) * a.num_kv_heads + head) * a.page_size * d;
+                to1 = dst + kva_k_at(slot % a.page_size, p0, a.page_size, 8);
+                to2 = dst + kva_k_at(slot % a.page_size, half + p0, a.page_size, 8);
+            }
+            RopeVec<bf16_t>::store(to1, o1);
+            RopeVec<bf16_t>::store(to2, o2);
+        }
+        return;
+    }
+    const int col0 = (block - a.q_blocks - a.k_blocks) * ROPE_V_COLS, cols = min(ROPE_V_COLS, a.num_kv_heads * d - col0);
+    const bf16_t *v = a.qkv + (size_t)(a.num_q_heads + a.num_kv_heads) * d + col0;
+    int slot[ROPE_TOKENS];
+#pragma unroll
+    for (int i = 0; i < ROPE_TOKENS; ++i) {
+        slot[i] = a.slot_mapping[min(t0 + i, a.tokens - 1)];
+        if (t0 + i >= a.tokens) slot[i] = -1;
+    }
+#pragma unroll
+    for (int i = 0; i < ROPE_TOKENS * ROPE_V_COLS / 8 / 256; ++i) {
+        const int token = tid / (ROPE_V_COLS / 8) + i * (256 / (ROPE_V_COLS / 8)), col = 8 * (tid % (ROPE_V_COLS / 8));
+        if (t0 + token < a.tokens && col < cols)            // (a whole number of 16 columns)
+            *reinterpret_cast<uint4 *>(&turn[token][col]) = *reinterpret_cast<const uint4 *>(v + (size_t)(t0 + token) * row_width + col);
+    }
+    __syncthreads();
+    if (tid >= cols) return;
+    const int kvh = (col0 + tid) / d, j = (col0 + tid) % d;
+    uint32_t pair[ROPE_TOKENS / 2];
+#pragma unroll
+    for (int i = 0; i < ROPE_TOKENS; i += 2) pair[i / 2] = (uint32_t)turn[i][tid] | ((uint32_t)turn[i + 1][tid] << 16);
+    int next = 0;
+#pragma unroll
+    for (int i = 0; i < ROPE_TOKENS; ++i) {
+        if (i < next || slot[i] < 0) continue;              // (the same in all threads)
+        uint16_t *dst = reinterpret_cast<uint16_t *>(a.v_cache) +
+                        (((size_t)(slot[i] / a.page_size) * a.num_kv_heads + kvh) * d + j) * a.page_size + slot[i] % a.page_size;
+        bool run = i + 8 <= ROPE_TOKENS && slot[i] % 8 == 0;
+#pragma unroll
+        for (int k = 1; k < 8; ++k) run = run && slot[(i + k) % ROPE_TOKENS] == slot[i] + k;
+        if (run) {
+            uint32_t w[4];
+#pragma unroll
+            for (int k = 0; k < 4; ++k) {
+                const int at = (i / 2 + k) % (ROPE_TOKENS / 2), then = (at + 1) % (ROPE_TOKENS / 2);
+                w[k] = i % 2 ? (pair[at] >> 16) | (pair[then] << 16) : pair[at];
+            }
+            *reinterpret_cast<uint4 *>(dst) = make_uint4(w[0], w[1], w[2], w[3]);
+            next = i + 8;
+        } else {
+            *dst = (uint16_t)(i % 2 ? pair[i / 2] >> 16 : pair[i / 2] & 0xffffu);
+        }
+    }
+}
+
 extern "C" int kva_rope_kv_write(void *qkv, void *k_cache, void *v_cache, const float *cos_table,
                                  const float *sin_table, const int *positions,
                                  const int *slot_mapping, int tokens, int num_q_heads,
@@ -185,6 +300,20 @@ extern "C" int kva_rope_kv_write(void *qkv, void *k_cache, void *v_cache, const 
     dim3 grid(tokens), block(256);
     const uintptr_t all = (uintptr_t)qkv | (uintptr_t)k_cache | (uintptr_t)cos_table | (uintptr_t)sin_table;
     if (cos_table && rot_dim == head_dim && head_dim % 16 == 0 && (dtype == KVA_BF16 || (dtype == KVA_F32 && all % 16 == 0))) {
+        // (up to 64 tokens are too few workgroups of 16)
+        if (dtype == KVA_BF16 && tokens > 64 && head_dim <= 256 && ((all | (uintptr_t)v_cache) & 15) == 0 && (!write_cache || page_size % 8 == 0)) {
+            const int lanes = 256 / (ROPE_TOKENS * (head_dim / 16)), heads = lanes * ROPE_HEADS;
+            const int q_blocks = (num_q_heads + heads - 1) / heads, k_blocks = write_cache ? (num_kv_heads + heads - 1) / heads : 0;
+            const int v_blocks = write_cache ? (num_kv_heads * head_dim + ROPE_V_COLS - 1) / ROPE_V_COLS : 0;
+            if (q_blocks + k_blocks + v_blocks <= 65535) {
+                const RopeWide a{(bf16_t *)qkv, (bf16_t *)k_cache, (bf16_t *)v_cache, cos_table, sin_table, positions, slot_mapping, tokens, num_q_heads,
+                                 num_kv_heads, head_dim, page_size, lanes, q_blocks, k_blocks};
+                hipLaunchKernelGGL(rope_kv_write_wide_kernel, dim3((tokens + ROPE_TOKENS - 1) / ROPE_TOKENS, q_blocks + k_blocks + v_blocks), block, 0,
+                                   stream, a);
+                KVA_CHECK_LAUNCH("rope_kv_write");
+                return KVA_OK;
+            }
+        }
         const int vectors = (num_q_heads + num_kv_heads) * head_dim / 2 / (dtype == KVA_BF16 ? 8 : 4);
         const dim3 vgrid(tokens, tokens <= 64 ? std::min(65535, (std::max(vectors, num_kv_heads * head_dim) + 255) / 256) : 1);
         if (dtype == KVA_BF16)
