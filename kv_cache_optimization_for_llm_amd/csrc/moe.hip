@@ -429,21 +429,48 @@ struct MoeRouter {
     int tokens, N, K, x_stride;
 };
 
-// steps s0 .. s1 - 1 of a part, four steps' loads on their way at once
-__device__ inline f32x4 moe_router_part(const bf16_t *wrow, const bf16_t *xrow, int s0, int s1) {
-    f32x4 acc = {0.f, 0.f, 0.f, 0.f};
-    for (int s = s0; s < s1; s += 4) {
-        Frag8 xf[4], wf[4];
+// PARTS neighbouring parts of `each` steps of 32 from number part0 on, of `steps` in all: the loads of four steps of every part are on their
+// way at once, and right behind the first ones what `behind()` asks for.  RAGGED: parts are no whole fours of steps, or the last ones are
+// shorter; what lies past a part's end is made zero on both sides.  (With a branch around every product instead the compiler moved its
+// loads into the branch, and a part was a chain of two trips to memory, one part after the other.)
+template <int PARTS, bool RAGGED, class F>
+__device__ __forceinline__ void moe_router_parts_as(const bf16_t *wrow, const bf16_t *xrow, int part0, int each, int steps, f32x4 (&acc)[PARTS], F behind) {
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            xf[i].u4 = *reinterpret_cast<const uint4 *>(xrow + 32 * min(s + i, s1 - 1));
-            wf[i].u4 = *reinterpret_cast<const uint4 *>(wrow + 32 * min(s + i, s1 - 1));
-        }
+    for (int j = 0; j < PARTS; ++j) acc[j] = f32x4{0.f, 0.f, 0.f, 0.f};
+    for (int c = 0; c < each; c += 4) {
+        Frag8 xf[PARTS][4], wf[PARTS][4];
+#pragma unroll
+        for (int j = 0; j < PARTS; ++j)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                const int s = (part0 + j) * each + c + i, at = 32 * (RAGGED ? min(s, steps - 1) : s);
+                xf[j][i].u4 = *reinterpret_cast<const uint4 *>(xrow + at);
+                wf[j][i].u4 = *reinterpret_cast<const uint4 *>(wrow + at);
+            }
+        __builtin_amdgcn_sched_barrier(0);
+        if (c == 0) behind();
+        __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
         for (int i = 0; i < 4; ++i)
-            if (s + i < s1) acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf[i].v, xf[i].v, acc, 0, 0, 0);
+#pragma unroll
+            for (int j = 0; j < PARTS; ++j) {
+                if (RAGGED) {
+                    const uint32_t in = c + i < each && (part0 + j) * each + c + i < steps ? 0xffffffffu : 0u;
+#pragma unroll
+                    for (int q = 0; q < 2; ++q) {
+                        xf[j][i].u2[q].x &= in; xf[j][i].u2[q].y &= in;
+                        wf[j][i].u2[q].x &= in; wf[j][i].u2[q].y &= in;
+                    }
+                }
+                acc[j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf[j][i].v, xf[j][i].v, acc[j], 0, 0, 0);
+            }
     }
-    return acc;
+}
+template <int PARTS, class F>
+__device__ __forceinline__ void moe_router_parts(const bf16_t *wrow, const bf16_t *xrow, int part0, int each, int parts, int steps,
+                                                 f32x4 (&acc)[PARTS], F behind) {
+    if (each % 4 == 0 && each * parts == steps) moe_router_parts_as<PARTS, false>(wrow, xrow, part0, each, steps, acc, behind);
+    else moe_router_parts_as<PARTS, true>(wrow, xrow, part0, each, steps, acc, behind);
 }
 
 template <int PL>
@@ -461,12 +488,9 @@ moe_router_kernel(MoeRouter m, MoeRoute a, int *__restrict__ sorted_slot, int *_
     for (int tile0 = 0; tile0 < tiles; tile0 += 16) {            // (more than 256 outputs: in turns)
         const int tile = tile0 + wave % min(tiles, 16), kp = wave / min(tiles, 16);
         const bool on = tile < tiles && kp < parts;
-        f32x4 acc = {0.f, 0.f, 0.f, 0.f};
-        if (on) {
-            const bf16_t *wrow = m.w + (size_t)min(16 * tile + r, m.N - 1) * m.K + 8 * g;
-            const int s1 = min(steps, (kp + 1) * per);
-            acc = moe_router_part(wrow, xrow, kp * per, s1);
-        }
+        f32x4 sums[1] = {f32x4{0.f, 0.f, 0.f, 0.f}};
+        if (on) moe_router_parts(m.w + (size_t)min(16 * tile + r, m.N - 1) * m.K + 8 * g, xrow, kp, per, parts, steps, sums, []() {});
+        const f32x4 acc = sums[0];
         __syncthreads();
 #pragma unroll
         for (int i = 0; i < 4; ++i) part[wave][lane][i] = acc[i];
@@ -919,7 +943,9 @@ extern "C" int kva_moe_expert_rows(void *out, int out_dtype, const void *x, cons
 //
 // ROUTED (mode 0): the router's product and the choice are made here too, by every workgroup for itself, in the order of sums
 // of the router's own launch: 16 parts of K.  A router of up to 16 outputs is 64 KB that all workgroups read from L2 while
-// their matrix is on its way; where the workgroups and the tokens are few (the caller's rule) that saves 2 us of a launch's 6-8.
+// their matrix is on its way; where the workgroups and the tokens are few (the caller's rule) that saves 2 us of a launch's 6-8.  All of the
+// router's loads, the matrix's first ones and what is added to the scores are on their way at once (228 registers: two
+// workgroups a unit): one token of 4 experts of 1,024 x 2,048 11.5 -> 9.5 us in the model, of 1,536 x 2,048 and a shared one 13.8 -> 12.6.
 //  mode 0: out[slot] = act(W[e] x[token]) (x's type),   mode 1: out[slot] = W[e] x[slot] * weight[slot] (fp32).
 struct MoeFewRouter {
     const bf16_t *w;                // [N, K], N up to 16
@@ -952,7 +978,8 @@ template <int AHEAD, int NT, bool ROUTED>
 __global__ void __launch_bounds__(256)
 moe_few_rows_kernel(MoeFew a, MoeFewRouter ro, void *__restrict__ out, const bf16_t *__restrict__ x, const bf16_t *__restrict__ w) {
     __shared__ float red[3][NT][KVA_WAVE][4];
-    __shared__ __attribute__((aligned(16))) float part[ROUTED ? 16 : 1][KVA_WAVE][4], logits[ROUTED ? 16 : 1][16], choice[4][KVA_WAVE], wgt_s[ROUTED ? 256 : 1];
+    __shared__ __attribute__((aligned(16))) float part[ROUTED ? 16 : 1][KVA_WAVE][4], logits[ROUTED ? 16 : 1][16], choice[4][KVA_WAVE], wgt_s[ROUTED ? 256 : 1],
+        correction_s[ROUTED ? 16 : 1];
     __shared__ int idx_s[ROUTED ? 256 : 1];
     const int lane = threadIdx.x % KVA_WAVE, wave = __builtin_amdgcn_readfirstlane(threadIdx.x / KVA_WAVE), r = lane & 15, g = lane >> 4;
     const int unit = blockIdx.y, slots = a.tokens * a.top;
@@ -991,10 +1018,13 @@ moe_few_rows_kernel(MoeFew a, MoeFewRouter ro, void *__restrict__ out, const bf1
         rows();                         // (the expert is the unit's number: its matrix comes while the choice is made)
         const bf16_t *rx = x + (size_t)min(r, a.tokens - 1) * a.K + 8 * g, *rw = ro.w + (size_t)min(r, ro.N - 1) * a.K + 8 * g;
         const int all = a.K / 32, each = (all + 15) / 16;
+        // (what the choice adds to logits and scores: asked for first, or it is a trip to memory of its own behind the sums)
+        const int own = 4 * (threadIdx.x / 64) + threadIdx.x % 4;
+        const float bias = ro.bias ? ro.bias[min(own, ro.N - 1)] : 0.f;
+        const float correction = ro.rule.correction ? ro.rule.correction[min((int)threadIdx.x, ro.rule.outputs - 1)] : 0.f;
+        __builtin_amdgcn_sched_barrier(0);
         f32x4 sums[4];
-#pragma unroll
-        for (int j = 0; j < 4; ++j) sums[j] = moe_router_part(rw, rx, (4 * wave + j) * each, min(all, (4 * wave + j + 1) * each));
-        load(s0);
+        moe_router_parts(rw, rx, 4 * wave, each, 16, all, sums, [&]() { load(s0); });
 #pragma unroll
         for (int j = 0; j < 4; ++j) *reinterpret_cast<f32x4 *>(part[4 * wave + j][lane]) = sums[j];
         __syncthreads();
@@ -1003,11 +1033,14 @@ moe_few_rows_kernel(MoeFew a, MoeFewRouter ro, void *__restrict__ out, const bf1
             float v = part[0][l][threadIdx.x % 4];
 #pragma unroll
             for (int p = 1; p < 16; ++p) v += part[p][l][threadIdx.x % 4];
-            if (n < ro.N) logits[l % 16][n] = v + (ro.bias ? ro.bias[n] : 0.f);
+            if (n < ro.N) logits[l % 16][n] = v + bias;
         }
+        if (threadIdx.x < 16) correction_s[threadIdx.x] = correction;
         __syncthreads();
+        MoeRoute rule = ro.rule;
+        if (rule.correction) rule.correction = correction_s;
         for (int t = wave; t < a.tokens; t += 4)
-            moe_route_token<1>(ro.rule, logits[t], idx_s + t * a.top, wgt_s + t * a.top, choice[wave]);
+            moe_route_token<1>(rule, logits[t], idx_s + t * a.top, wgt_s + t * a.top, choice[wave]);
         __syncthreads();
         if (unit == 0 && blockIdx.x == 0) {
             for (int s = threadIdx.x; s < slots; s += 256) {

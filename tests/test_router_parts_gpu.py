@@ -1,0 +1,42 @@
+"""The router's product in its 16 parts of K, in a launch of its own and inside the experts' first product (csrc/moe.hip): whole fours of
+steps of 32 a part, fewer, more, and last parts that are shorter or empty."""
+import pytest
+import torch
+
+from kv_cache_optimization_for_llm_amd.ops import kernels as K
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("tokens", [1, 5, 16])
+@pytest.mark.parametrize("width", [32, 96, 544, 1024, 2048, 2080, 4096, 4608])
+def test_the_routers_product_at_any_inner_size(width, tokens, gpu):
+    g = torch.Generator().manual_seed(width + tokens)
+    outputs, extra, top, ff = 6, 2, 6, 32
+    x = torch.randn((tokens, width), generator=g).bfloat16().to(gpu)
+    w = (torch.randn((outputs + extra, width), generator=g) * width ** -0.5).bfloat16().to(gpu)
+    bias, corr = torch.randn(outputs + extra, generator=g).to(gpu), torch.randn(outputs, generator=g).to(gpu)
+    up = K.moe_tiled_weight((torch.randn((outputs, ff, width), generator=g) * width ** -0.5).bfloat16().to(gpu))
+
+    def room():
+        return (torch.full((tokens, top), -9, dtype=torch.int32, device=gpu), torch.zeros((tokens, top), device=gpu),
+                torch.zeros((tokens, extra), device=gpu))
+    idx, wgt, rest = room()
+    K.moe_router(x, w, bias, corr, outputs, top, idx, wgt, rest, experts=outputs)
+    want = x.double().cpu() @ w.double().cpu().T + bias.double().cpu()
+    scores = torch.softmax(want[:, :outputs], -1)
+    # sums of `width` products of numbers around width^-1/2 in 32 bits; every output is chosen, so weights can be put back in order
+    assert (rest.cpu().double() - want[:, outputs:]).abs().max() <= 2.0 ** -19
+    assert torch.equal(idx.cpu().sort(-1).values, torch.arange(outputs, dtype=torch.int32).expand(tokens, -1))
+    assert (wgt.cpu().double() - scores.gather(1, idx.cpu().long())).abs().max() <= 2.0 ** -18
+    if tokens * top >= outputs:
+        inside = room()
+        act = torch.zeros((tokens * top, ff), dtype=torch.bfloat16, device=gpu)
+        K.moe_few_rows(x, up, act, inside[0], activation="silu",
+                       router=dict(w=w, bias=bias, correction=corr, outputs=outputs, wgt=inside[1], rest=inside[2], renormalise=False,
+                                   over_chosen=False, scores="softmax", groups=1, keep_groups=1, group_top=2, weight_scale=1.0, sum_eps=0.0))
+        for a, b in zip(inside, (idx, wgt, rest)):
+            assert torch.equal(a, b)
+        alone = torch.zeros_like(act)
+        K.moe_few_rows(x, up, alone, idx, activation="silu")
+        assert torch.equal(act, alone) and act.any()
