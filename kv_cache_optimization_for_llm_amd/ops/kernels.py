@@ -2748,7 +2748,7 @@ KERNEL_CLASSES = {
     "sample": "sampling", "sample_by_value": "sampling", "mark_tokens": "sampling",
     "causal_conv_act": "recurrent mixers", "gated_delta_rule": "recurrent mixers",
     "gated_linear_attention": "recurrent mixers", "head_norm_gate": "elementwise",
-    "moe_route": "routed experts", "moe_router": "routed experts", "moe_align": "routed experts", "moe_table_align": "routed experts", "moe_expert_rows": "routed experts", "moe_few_rows": "routed experts",
+    "moe_route": "routed experts", "moe_router": "routed experts", "moe_align": "routed experts", "moe_table_align": "routed experts", "moe_expert_rows": "routed experts", "moe_expert_tiles": "routed experts", "moe_few_rows": "routed experts",
     "moe_combine": "routed experts", "small_product_f32": "small fp32 products",
     "norm_into_stream": "norm", "table_gate": "elementwise",
     "hyper_step": "norm", "sandwich_step": "norm", "hyper_fill": "embedding", "bias_act": "activation",
