@@ -236,10 +236,11 @@ class Model:
 
     def tune_products(self, row_counts, say=None) -> List[dict]:
         """For every row count, has the vendor GEMM library's algorithms timed for each shape of
-        bf16 Linear that goes to the library at that many rows (``ops.gemm_bf16.tune_linear``;
+        bf16 Linear that goes to the library at that many rows, or at a row count down to half of it
+        (``ops.gemm_bf16.worth_timing``, ``tune_linear``;
         the same projection of all layers shares a shape and the layers' weights are used in
         turn).  Seconds per shape: start-up work.  Returns one record per (rows, shape)."""
-        from ..ops.gemm_bf16 import SKINNY_WIDE_ROWS, tune_linear, use_skinny
+        from ..ops.gemm_bf16 import tune_linear, worth_timing
         shapes: Dict[tuple, List[Linear]] = {}
         for lin in self.linears():
             if lin.weight.is_cuda and lin.weight.dtype == torch.bfloat16:
@@ -247,11 +248,8 @@ class Model:
         report = []
         for rows in sorted(set(int(r) for r in row_counts)):
             for (n, k, halves), lins in shapes.items():
-                if lins[0].tiled is not None and (use_skinny(rows, n, k, halves == 2) or use_skinny(rows, n, k)):
-                    continue                                    # the few-rows kernel takes these
-                if lins[0].tiled is not None and rows > SKINNY_WIDE_ROWS \
-                        and K.gemm_tiles_plan(rows, n, k, K.TILES_GATED if halves == 2 else K.TILES_PLAIN) >= 0:
-                    continue                                    # the tiles of gemm_tiles.hip take these
+                if not worth_timing(rows, n, k, halves == 2, lins[0].tiled is not None):
+                    continue                                    # hand-written kernels take these
                 first, best, tried = tune_linear(rows, [lin.weight for lin in lins[:16]])
                 report.append(dict(rows=rows, n=n, k=k, heuristic_us=round(first, 2), kept_us=round(best, 2),
                                    algorithms_run=tried))

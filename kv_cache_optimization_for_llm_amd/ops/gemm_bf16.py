@@ -123,6 +123,23 @@ def chosen_cut(m: int, n: int, k: int, device, dtype: torch.dtype = torch.bfloat
     return cut
 
 
+def tiles_plan(m: int, n: int, k: int, gated: bool = False) -> int:
+    """The plan by which ``m`` bf16 rows of a ``[n, k]`` weight with a tiled copy go to ``kernels.gemm_tiles``, or -1: the vendor library
+    takes them (or, up to :data:`SKINNY_WIDE_ROWS` rows, the few-rows kernels).  ``gated``: the joined [gate; up] product with its activation.
+    (A product that the library takes in two has its whole turns there: 2,048 rows of 8,208 outputs of 2,048 68 us, 72 in tiles.)"""
+    if m <= SKINNY_WIDE_ROWS or (not gated and vendor_cut(m, n)):
+        return -1
+    return K.gemm_tiles_plan(m, n, k, K.TILES_GATED if gated else K.TILES_PLAIN)
+
+
+def worth_timing(rows: int, n: int, k: int, gated: bool = False, tiled: bool = True) -> bool:
+    """Whether the vendor library's algorithms are timed for ``rows`` rows: it takes that many, or a row count down to half of them, which
+    what is found serves too.  ``tiled``: the weight has a tiled copy."""
+    def library(m: int) -> bool:
+        return not (use_skinny(m, n, k, gated) or use_skinny(m, n, k)) and tiles_plan(m, n, k, gated) < 0
+    return not tiled or any(library(m) for m in range(rows, (rows + 1) // 2 - 1, -1))
+
+
 def tune_linear(rows: int, weights, out_dtype: torch.dtype = torch.bfloat16) -> tuple:
     """Has the vendor library's algorithms timed for products of ``rows`` rows with ``weights`` (matrices of one shape), whole and, where
     :func:`linear_bf16` would cut them, in two; the faster way is kept.  Returns (microseconds by the library's own choice,
@@ -171,8 +188,7 @@ def linear_bf16(x: torch.Tensor, w: torch.Tensor, out: torch.Tensor, tiled=None)
         return K.gemm_skinny(x, tiled, out)
     if tiled is not None and out.dtype == torch.bfloat16 and x.shape[0] > SKINNY_WIDE_ROWS and tiled.halves == 1 \
             and out.is_contiguous() and out.data_ptr() % 16 == 0 and K.gemm_tiles_takes(x, tiled):
-        # (a product that the library takes in two has its whole turns there: 2,048 rows of 8,208 outputs of 2,048 68 us, 72 in tiles)
-        plan = -1 if vendor_cut(x.shape[0], w.shape[0]) else K.gemm_tiles_plan(x.shape[0], w.shape[0], w.shape[1])
+        plan = tiles_plan(x.shape[0], w.shape[0], w.shape[1])
         if plan >= 0:
             return K.gemm_tiles(x, tiled, out, plan)
     cut = chosen_cut(x.shape[0], w.shape[0], w.shape[1], w.device, out.dtype) if out.is_contiguous() else 0

@@ -139,11 +139,10 @@ class Linear:
         """act(x gate^T) * (x up^T) of more than 64 rows for a joined [gate; up] weight, the activation applied to the product's sums;
         ``None`` where the library's product and the activation's own kernel are expected to be faster, or rows and weight are not of
         the kinds that ``kernels.gemm_tiles`` takes."""
-        from ..ops.gemm_bf16 import SKINNY_WIDE_ROWS
-        if self.tiled is None or self.halves != 2 or not isinstance(x, torch.Tensor) or x.shape[0] <= SKINNY_WIDE_ROWS \
-                or not K.gemm_tiles_takes(x, self.tiled):
+        from ..ops.gemm_bf16 import tiles_plan
+        if self.tiled is None or self.halves != 2 or not isinstance(x, torch.Tensor) or not K.gemm_tiles_takes(x, self.tiled):
             return None
-        plan = K.gemm_tiles_plan(x.shape[0], self.out_features, self.in_features, K.TILES_GATED)
+        plan = tiles_plan(x.shape[0], self.out_features, self.in_features, gated=True)
         if plan < 0:
             return None
         out = torch.empty((x.shape[0], self.out_features // 2), dtype=x.dtype, device=x.device)

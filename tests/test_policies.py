@@ -364,3 +364,60 @@ def test_products_timed_at_start_up_run_the_way_that_was_faster(monkeypatch):
     calls.clear()
     us[8192 + 64] = (5.0, 4.0, 3)
     assert G.tune_linear(2048, [torch.empty((8192 + 64, 64))]) == (5.0, 4.0, 3) and calls == [(2048, 8256, 0)]
+
+
+class _Operand:
+    """As much of a tensor on the GPU as the choice of a product looks at."""
+    is_cuda, device = True, "cuda:0"
+
+    def __init__(self, *shape):
+        import torch
+        self.shape, self.dtype = shape, torch.bfloat16
+
+    def is_contiguous(self):
+        return True
+
+    def data_ptr(self):
+        return 0
+
+    def stride(self, _):
+        return 1
+
+    def __getitem__(self, _):
+        return self
+
+
+def test_the_librarys_algorithms_are_timed_where_the_library_takes_rows(monkeypatch):
+    """What linear_bf16 hands to the library at a row count, or at one that what was timed there serves (down to half of it), is timed; and
+    nothing else is."""
+    from types import SimpleNamespace
+    from kv_cache_optimization_for_llm_amd.models.builder import Model
+    from kv_cache_optimization_for_llm_amd.ops import gemm_bf16 as G
+    taken, timed = [], []
+    monkeypatch.setattr(G, "_TIMED_CUTS", {})
+    monkeypatch.setattr(G.K, "gemm_tiles_takes", lambda x, w: True)
+    for kernel in ("gemm_tiles", "gemm_skinny", "gemv", "gemm_vendor"):
+        monkeypatch.setattr(G.K, kernel, lambda *a, _k=kernel, **kw: taken.append(_k) or True)
+    monkeypatch.setattr(G, "tune_linear", lambda rows, ws: timed.append(rows) or (1.0, 1.0, 1))
+
+    def takes(m, n, k):
+        taken.clear()
+        G.linear_bf16(_Operand(m, k), _Operand(n, k), _Operand(m, n), SimpleNamespace(halves=1))
+        return set(taken)
+
+    # outputs a little past whole columns, which the library takes in two; others that it takes whole at some of the rows; none
+    for n, k, asked in ((8208, 2048, (2048, 1024)), (16400, 2048, (2048,)), (4112, 2048, (4096,)), (6144, 4096, (256, 128, 80)), (3072, 8192, (512,)),
+                        (2048, 2048, (64, 512, 2048)), (2048, 8192, (100, 1203)), (40000, 2048, (96,))):
+        for rows in asked:
+            library = any("gemm_vendor" in takes(m, n, k) for m in range((rows + 1) // 2, rows + 1))
+            timed.clear()
+            lin = SimpleNamespace(weight=_Operand(n, k), tiled=SimpleNamespace(halves=1), out_features=n, in_features=k, halves=1)
+            Model.tune_products(SimpleNamespace(linears=lambda: [lin]), [rows])
+            assert timed == ([rows] if library else []), (rows, n, k)
+    assert takes(2048, 8208, 2048) == {"gemm_vendor"} and takes(256, 6144, 4096) == {"gemm_tiles"} and takes(200, 6144, 4096) == {"gemm_vendor"}
+    # a joined [gate; up] matrix: by the plan of the product with its activation
+    for rows in (96, 300, 8190):
+        timed.clear()
+        lin = SimpleNamespace(weight=_Operand(28672, 4096), tiled=SimpleNamespace(halves=2), out_features=28672, in_features=4096, halves=2)
+        Model.tune_products(SimpleNamespace(linears=lambda: [lin]), [rows])
+        assert timed == ([rows] if any(G.K.gemm_tiles_plan(m, 28672, 4096, G.K.TILES_GATED) < 0 for m in range(max(65, (rows + 1) // 2), rows + 1)) else [])
