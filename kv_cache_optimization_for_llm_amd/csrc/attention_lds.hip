@@ -419,8 +419,8 @@ attention_lds_kernel_3(LDS_KERNEL_PARAMS) {
 
 // Where few workgroups run at once a wavefront's chain through its blocks is the time (0.65 us a block of 32 keys with a SIMD or half of one to
 // itself, 0.3 where four share it).  Blocks of 64 keys, two wavefronts a SIMD: 1.05 us a block.  us, blocks of 32 -> of 64: 32 heads of 64
-// over 8, 3,072 / 4,096 / 6,000 tokens 66 -> 59, 96 -> 88, 193 -> 180; heads of 128, 24 over 8, 3,072 / 4,096 / 6,000 91 -> 84, 131 -> 117, 272 -> 235;
-// 32 over 8, 3,072 100 -> 90.
+// over 8, 3,072 / 4,096 / 6,000 tokens 66 -> 59, 96 -> 88, 193 -> 180; heads of 128, 24 over 8, 3,072 91 -> 84; 32 over 8, 3,072 100 -> 90.
+// (Where either form is behind, and by how much: the lines in ops/attention.py.)
 template <int D>
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2)))
 attention_lds_kernel_64(LDS_KERNEL_PARAMS) {

@@ -150,24 +150,39 @@ def use_lds_kernel(groups: int, mean_keys: float, head_dim: int) -> bool:
     return groups >= _LDS_SOME_GROUPS and mean_keys >= _LDS_SOME_GROUPS_MEAN_KEYS
 
 
-# The workgroup kernel's other forms (csrc/attention_lds.hip, with both sides), by workgroups of 128 rows over all kv heads.  Two groups of
-# wavefronts: heads up to 64 from 448 to 699 workgroups whose rows visit 1,024 keys and more (fewer keys: 1,531 and 963 tokens, 632 workgroups, 35 us
-# against 34 by two wavefronts an item; fewer workgroups: 1,536 tokens, 384, 26 against 26), above 96 from 272 to 544 that visit 512 and more, to 659 below 1,024
-# (256 workgroups: 2,048 tokens of 16 heads over 8 42 against 41; 576: 2,304 of 32 71 against 66 in blocks of 64).  Blocks of 64 keys: heads up to
-# 64 from 700 workgroups on (8,190 tokens, 2,048: 318 -> 312), above 96 from 545 to 899 and from 1,100 to 1,535 (1,024 workgroups are two full turns with two a
-# unit, where three a unit make one and a third: 4,096 tokens of 32 heads 148 -> 156; 2,048: 528 -> 537).
+# The workgroup kernel's other forms (csrc/attention_lds.hip), by workgroups of 128 rows over all kv heads and mean keys.  Where the lines lie comes
+# from 4,400 steps of one to eight portions of 32 heads of 64 and 24 and 32 of 128 over 8: alike and unlike in length, from position 0 and from the
+# same and different ones up to 16,000, a third of them of whole workgroups.
+# Two groups of wavefronts, against what else is chosen (two or four wavefronts an item, or blocks of 32): heads up to 64 from 448 to 699 workgroups,
+# 1,024 to 2,047 keys, 0.85 of its time where every portion is whole workgroups (one prompt of 2,048 tokens 39 -> 34 us; 2,176 42.5 -> 37, 2,400 49 ->
+# 41), and from 640 on otherwise (0.77; below, the last workgroup walks its keys with the mask on, and 2,047 tokens are 42 against 44, 2,143 44 against
+# 47).  Above 96 from 272 to 544 workgroups, 512 to 2,047 keys: 0.71, and 0.84 where whole; the slowest of 257 1.18.  Not from 2,048 keys on: the chain
+# of the furthest portion is halved, where four wavefronts an item or key ranges cut it further, so portions at unlike depths were up to twice as
+# slow (six of 319 behind 512 to 16,000 keys 141 against 283), heads of 128 behind 8,192 keys 428 against 443.  Not above 544: 1.03 to 1.2 where whole.
+# Blocks of 64 keys, against blocks of 32: heads up to 64 from 700 workgroups and 512 keys on 0.93 (odd) and 0.95 (whole), but of 1,025 to 1,299 workgroups only
+# from 4,096 keys on (below 0.92 and 1.03) and of more from 1,024 on; fewer keys 1.0 to 1.3 (sixteen prompts of 200 14 against 18).  Above 96 from 545 to 749
+# workgroups, 512 to 2,047 keys, 0.90 and 0.94, and to 899 from 1,024 on, 0.89 and 0.97; more keys up to 1.25 (3,392 tokens behind 6,000 322 against 403),
+# more workgroups 0.9 to 1.13.
 LDS_BLOCKS_OF_32, LDS_BLOCKS_OF_64, LDS_TWO_GROUPS = 0, 1, 2
-_TWO_GROUPS = {False: ((448, 700, 1024, 1 << 30),), True: ((272, 545, 512, 1 << 30), (545, 660, 512, 1024))}       # from, below; mean keys from, below
-_LONG_BLOCKS = {False: ((700, 1 << 30),), True: ((545, 900), (1100, 1536))}
+_ANY_KEYS = 1 << 30
+# (workgroups from, below; mean keys from, below), by whether heads are above 96
+_TWO_GROUPS = {False: ((448, 700, 1024, 2048),), True: ((272, 545, 512, 2048),)}
+_LONG_BLOCKS = {False: ((700, 1025, 512, _ANY_KEYS), (1025, 1300, 4096, _ANY_KEYS), (1300, _ANY_KEYS, 1024, _ANY_KEYS)),
+                True: ((545, 750, 512, 2048), (750, 900, 1024, 2048))}
+_TWO_GROUPS_RAGGED_FROM = 640           # heads up to 96, portions that end inside a workgroup
 
 
-def choose_lds_kind(groups: int, mean_keys: float, head_dim: int, by_workgroup: bool) -> int:
+def choose_lds_kind(groups: int, mean_keys: float, head_dim: int, by_workgroup: bool, whole: bool = True) -> int:
     """Which form of the workgroup kernel takes ``groups`` workgroups of rows that visit ``mean_keys`` keys on average; ``by_workgroup``:
-    they go to that kernel in any case.  (Two groups are also ahead of the one-wavefront kernel, so its lines do not hold there.)"""
+    they go to that kernel in any case; ``whole``: every portion's rows fill their workgroups.  (Two groups are also ahead of the
+    one-wavefront kernel, so its lines do not hold there.)"""
     wide = head_dim > 96
-    if any(a <= groups < b and lo <= mean_keys < hi for a, b, lo, hi in _TWO_GROUPS[wide]):
+
+    def within(lines) -> bool:
+        return any(a <= groups < b and lo <= mean_keys < hi for a, b, lo, hi in lines[wide])
+    if within(_TWO_GROUPS) and (wide or whole or groups >= _TWO_GROUPS_RAGGED_FROM):
         return LDS_TWO_GROUPS
-    return LDS_BLOCKS_OF_64 if by_workgroup and any(a <= groups < b for a, b in _LONG_BLOCKS[wide]) else LDS_BLOCKS_OF_32
+    return LDS_BLOCKS_OF_64 if by_workgroup and within(_LONG_BLOCKS) else LDS_BLOCKS_OF_32
 
 
 def _cut_keys(want: int, max_context: int, max_splits: int) -> tuple:
@@ -553,7 +568,8 @@ def portion_choice(lens, mean_keys: float, group: int, num_kv_heads: int, head_d
     groups = sum(-(-n // 128) for n in long) * num_kv_heads
     workgroups = K.attention_lds_supported(head_dim, page_size)
     # (behind a window most of a context is skipped: as before)
-    if workgroups and not 0 < visible < mean_keys and choose_lds_kind(groups, mean_keys, head_dim, False) == LDS_TWO_GROUPS:
+    whole = all(n % 128 == 0 for n in long)
+    if workgroups and not 0 < visible < mean_keys and choose_lds_kind(groups, mean_keys, head_dim, False, whole) == LDS_TWO_GROUPS:
         return 1, 1 + LDS_TWO_GROUPS
     tiles = K.attention_mfma_row_tiles(head_dim, True)
     if tiles == 2:
@@ -564,7 +580,7 @@ def portion_choice(lens, mean_keys: float, group: int, num_kv_heads: int, head_d
             return sharing, 0
     if not workgroups or not use_lds_kernel(groups, mean_keys, head_dim):
         return 1, 0
-    kind = choose_lds_kind(groups, mean_keys, head_dim, True)
+    kind = choose_lds_kind(groups, mean_keys, head_dim, True, whole)
     return 1, 1 + (LDS_BLOCKS_OF_32 if kind == LDS_TWO_GROUPS else kind)
 
 
