@@ -11,6 +11,7 @@
 //   2,048 of 8,192: 517 rows 42.8 / 38.1 (26.5 as three ranges, the norm's longer read included), 1,203 53.6 / 45.9 (42.9 as two),
 //     2,048 65.5 / 59.0
 //   5,152 of 2,048: 2,494 rows 59 / 50; 6,144 of 4,096: 192 rows 33.7 / 24.2, 700 49.9 / 38.9, 2,048 80 / 92 (the library's)
+#include "tile_activations.h"
 #include "tile_product.h"
 
 #include <type_traits>
@@ -22,9 +23,6 @@ struct GtArgs {
     void *out;              // bf16 [M, N] ([M, N / 2] gated), or fp32 [splits, M, N]
     int M, N, K, splits, act;
 };
-
-// silu with the hardware's exponential and reciprocal, on 32-bit sums that are rounded to 16 bits next
-__device__ __forceinline__ float gt_silu(float z) { return z * __builtin_amdgcn_rcpf(1.f + __builtin_amdgcn_exp2f(-1.44269504f * z)); }
 
 template <class P, int FORM>
 __global__ void __launch_bounds__(P::THREADS, P::WAVES / 4)
@@ -77,7 +75,7 @@ gemm_tiles_kernel(GtArgs a) {
                 f32x4 v = acc[nt][rt];
                 if constexpr (FORM == GT_GATED) {
 #pragma unroll
-                    for (int q = 0; q < 4; ++q) v[q] = (silu ? gt_silu(v[q]) : kva_activate(v[q], a.act)) * acc[nt + 1][rt][q];
+                    for (int q = 0; q < 4; ++q) v[q] = (silu ? tile_silu(v[q]) : kva_activate(v[q], a.act)) * acc[nt + 1][rt][q];
                 }
                 if constexpr (FORM == GT_PARTS) {       // (N is a multiple of 4)
                     *reinterpret_cast<f32x4 *>(reinterpret_cast<float *>(a.out) + ((size_t)split * a.M + row) * a.N + n) = v;

@@ -9,6 +9,7 @@
 // and around them the first operands' way from memory and the results' to it.  Before (moe.hip's 128 x 256, two workgroups a unit) and
 // now, in the model, us: 2,048 tokens, 4 of 16 experts of 1,536 x 2,048 68 / 62 (830 TFLOP/s), of 2,048 x 768 58 / 48; all of 4
 // of 1,024 x 2,048 with erf-gelu 49.5 / 46; 2,494 tokens, all of 4 of 1,536 x 2,048 65 / 62.
+#include "tile_activations.h"
 #include "tile_product.h"
 #include <math.h>
 #include <type_traits>
@@ -47,8 +48,7 @@ __device__ __forceinline__ float mt_gelu(float z) {
 
 template <int ACT>
 __device__ __forceinline__ float mt_activate(float z) {
-    // (silu with the hardware's exponential and reciprocal, on 32-bit sums that are rounded to 16 bits next)
-    if (ACT == MT_ACT_SILU) return z * __builtin_amdgcn_rcpf(1.f + __builtin_amdgcn_exp2f(-1.44269504f * z));
+    if (ACT == MT_ACT_SILU) return tile_silu(z);
     if (ACT == MT_ACT_GELU) return mt_gelu(z);
     return kva_activate(z, ACT == MT_ACT_RELU ? KVA_ACT_RELU : ACT == MT_ACT_RELU2 ? KVA_ACT_RELU2 : KVA_ACT_GELU_TANH);
 }

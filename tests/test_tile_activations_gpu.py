@@ -1,0 +1,71 @@
+"""The activations that the tiled products apply to their 32-bit sums (``csrc/tile_activations.h``): results whose exact value lies just beside the
+middle of two bf16 numbers are rounded to the right one of them, which asks for an error below the distance from the middle."""
+import pytest
+import torch
+
+from kv_cache_optimization_for_llm_amd.ops import kernels as K
+
+pytestmark = pytest.mark.gpu
+EXACT = {"silu": lambda z: z * torch.sigmoid(z)}
+
+
+def beside_middles(activation, lo, hi, distance, seed):
+    """32-bit numbers between lo and hi whose activation is `distance` to 3 x `distance` of itself away from a middle, and the rounded result."""
+    z = (torch.rand(1 << 23, generator=torch.Generator().manual_seed(seed), dtype=torch.float64) * (hi - lo) + lo).float()
+    y = EXACT[activation](z.double())
+    unit = 2.0 ** (torch.frexp(y).exponent.double() - 8)                    # of bf16's last place
+    away = ((y / unit - torch.floor(y / unit) - 0.5).abs() * unit) / y.abs()
+    z = z[(away >= distance) & (away <= 3 * distance)][:3000]
+    return z, EXACT[activation](z.double()).float().bfloat16()
+
+
+def rows_of(z, width=192):
+    """Rows whose product with ones at columns 0, 64 and 128 is z, exactly: its 24 bits in three bf16 numbers of different stages; column 1 holds a one."""
+    x = torch.zeros((z.numel(), width), dtype=torch.bfloat16)
+    rest = z.clone()
+    for col in (0, 64, 128):
+        x[:, col] = rest.bfloat16()
+        rest = rest - x[:, col].float()
+    assert not rest.any()
+    x[:, 1] = 1.0
+    return x
+
+
+def by_product(z, shape, gpu, width=192, ff=64):
+    w = torch.zeros((2 * ff, width), dtype=torch.bfloat16)
+    w[:ff, [0, 64, 128]] = 1.0
+    w[ff:, 1] = 1.0
+    out = torch.empty((z.numel(), ff), dtype=torch.bfloat16, device=gpu)
+    return K.gemm_tiles(rows_of(z).to(gpu), K.TiledWeight(w.to(gpu), 2), out, shape + 256, K.TILES_GATED, "silu").cpu()
+
+
+def by_experts(z, shape, activation, gated, gpu, width=192, ff=64):
+    w = torch.zeros((1, (2 if gated else 1) * ff, width), dtype=torch.bfloat16)
+    w[0, :, [0, 64, 128]] = 1.0
+    if gated:
+        w[0, 1::2] = 0.0
+        w[0, 1::2, 1] = 1.0
+    tiles = K.moe_tiles(z.numel(), 1, 1)
+    slot, expert = torch.empty(tiles * K.MOE_TILE, dtype=torch.int32, device=gpu), torch.empty(tiles, dtype=torch.int32, device=gpu)
+    K.moe_align(torch.zeros((z.numel(), 1), dtype=torch.int32, device=gpu), 1, slot, expert, 1)
+    out = torch.zeros((tiles * K.MOE_TILE, ff), dtype=torch.bfloat16, device=gpu)
+    K.moe_expert_tiles(rows_of(z).to(gpu), K.moe_tiled_weight(w.to(gpu)), out, slot, expert, 1, shape, activation=activation, gated=gated)
+    slot, got = slot.cpu().long(), torch.empty((z.numel(), ff), dtype=torch.bfloat16)
+    got[slot[slot >= 0]] = out.cpu()[slot >= 0]
+    return got
+
+
+# the exponential 2^-23, the sum and the quotient half a unit of the last place, 2^-24 each: 2^-22 in all
+@pytest.mark.parametrize("lo, hi", [(-87, -20), (-20, -5), (-5, 0), (0, 12)])
+def test_silu_is_as_exact_as_32_bits_allow(lo, hi, gpu):
+    z, want = beside_middles("silu", lo, hi, 2.0 ** -22, 3)
+    assert z.numel() >= 500
+    for got in (by_product(z, 0, gpu), by_product(z, 8, gpu), by_experts(z, 0, "silu", True, gpu)):
+        assert torch.equal(got, want[:, None].expand_as(got)), int((got != want[:, None]).any(1).sum())
+
+
+def test_activations_far_out(gpu):
+    z = torch.tensor([-3e38, -1000.0, -200.0, -88.0, -87.5, -0.0, 0.0, 1e-30, 88.0, 89.0, 1000.0, 3e38])
+    want = EXACT["silu"](z.double()).float().bfloat16()
+    for got in (by_product(z, 8, gpu), by_experts(z, 8, "silu", True, gpu)):
+        assert torch.equal(got, want[:, None].expand_as(got))
