@@ -28,28 +28,10 @@ struct MtArgs {
     float limit;
 };
 
-// z Phi(z), erf-gelu: erfc(u) = t exp(-u^2) 2^P(t), t = 1 / (1 + u / 2), P fitted to log2(exp(u^2) erfc(u) / t) at Chebyshev points
-// for u of 0 to 10 (4e-7).  Over z of -8 to 8 in 32 bits off by 3.8e-7 at most, 1 + erff(z / sqrt 2) by 4.5e-7; that one's two
-// branches for every output cost as long as the products: a tile of 256 x 256 is 20,000 cycles of them.
-__device__ __forceinline__ float mt_gelu(float z) {
-    const float u = fabsf(z) * 0.70710678f, t = __builtin_amdgcn_rcpf(fmaf(0.5f, u, 1.f));
-    float p = 0.11549703776836395f;
-    p = fmaf(p, t, -0.8108638525009155f);
-    p = fmaf(p, t, 2.1482982635498047f);
-    p = fmaf(p, t, -2.5933144092559814f);
-    p = fmaf(p, t, 1.2448766231536865f);
-    p = fmaf(p, t, -0.3467652201652527f);
-    p = fmaf(p, t, 0.6351691484451294f);
-    p = fmaf(p, t, 1.4323792457580566f);
-    p = fmaf(p, t, -1.8252770900726318f);
-    const float c = t * __builtin_amdgcn_exp2f(fmaf(-1.44269504f * u, u, p));
-    return 0.5f * z * (z > 0.f ? 2.f - c : c);
-}
-
 template <int ACT>
 __device__ __forceinline__ float mt_activate(float z) {
     if (ACT == MT_ACT_SILU) return tile_silu(z);
-    if (ACT == MT_ACT_GELU) return mt_gelu(z);
+    if (ACT == MT_ACT_GELU) return tile_gelu(z);
     return kva_activate(z, ACT == MT_ACT_RELU ? KVA_ACT_RELU : ACT == MT_ACT_RELU2 ? KVA_ACT_RELU2 : KVA_ACT_GELU_TANH);
 }
 

@@ -6,7 +6,7 @@ import torch
 from kv_cache_optimization_for_llm_amd.ops import kernels as K
 
 pytestmark = pytest.mark.gpu
-EXACT = {"silu": lambda z: z * torch.sigmoid(z)}
+EXACT = {"silu": lambda z: z * torch.sigmoid(z), "gelu": lambda z: 0.5 * z * torch.special.erfc(-z * 0.5 ** 0.5)}
 
 
 def beside_middles(activation, lo, hi, distance, seed):
@@ -64,8 +64,20 @@ def test_silu_is_as_exact_as_32_bits_allow(lo, hi, gpu):
         assert torch.equal(got, want[:, None].expand_as(got)), int((got != want[:, None]).any(1).sum())
 
 
+# up to 1.5 two roundings of 2^-24 of results that are a fifth of their parts' size or more; below -1 1 + erf cancels, and beyond the exponent's rounding
+# comes in, 2^-23 of numbers up to 8
+@pytest.mark.parametrize("lo, hi, distance", [(-1, 0, 2.0 ** -22), (0, 6, 2.0 ** -22), (-3, -1, 2.0 ** -19)])
+def test_erf_gelu_is_as_exact_as_32_bits_allow(lo, hi, distance, gpu):
+    z, want = beside_middles("gelu", lo, hi, distance, 4)
+    assert z.numel() >= 500
+    got = by_experts(z, 2, "gelu", False, gpu)
+    assert torch.equal(got, want[:, None].expand_as(got)), int((got != want[:, None]).any(1).sum())
+
+
 def test_activations_far_out(gpu):
     z = torch.tensor([-3e38, -1000.0, -200.0, -88.0, -87.5, -0.0, 0.0, 1e-30, 88.0, 89.0, 1000.0, 3e38])
     want = EXACT["silu"](z.double()).float().bfloat16()
     for got in (by_product(z, 8, gpu), by_experts(z, 8, "silu", True, gpu)):
         assert torch.equal(got, want[:, None].expand_as(got))
+    got, want = by_experts(z, 8, "gelu", False, gpu), EXACT["gelu"](z.double()).float().bfloat16()
+    assert torch.equal(got, want[:, None].expand_as(got))
