@@ -4,13 +4,13 @@
 //
 // Prompts, portions and steps of many decoding requests take them: some 65 to 3,000 rows of 1,000 to 30,000 outputs, sizes at
 // which a tile's shape decides how full the 256 compute units are (one workgroup a unit: its stages take most of the LDS).  So
-// there are ten shapes, and gt_plan below takes the one that it expects to be fastest.  The vendor library against these, us
-// (weights from memory, in a graph or with enough work on the way; activation included where the matrix is joined):
-//   2,048 outputs of 2,048 inputs: 96 rows 11.3 / 10.3, 517 14.0 / 12.6, 1,203 20.3 / 16.2, 2,048 21.9 / 19.6
-//   16,384 joined of 2,048: 96 rows 22.4 / 18.7, 517 45 / 36, 1,203 89 / 75, 2,048 125 / 113, 3,072 180 / 160
-//   2,048 of 8,192: 517 rows 42.8 / 38.1 (26.5 as three ranges, the norm's longer read included), 1,203 53.6 / 45.9 (42.9 as two),
-//     2,048 65.5 / 59.0
-//   5,152 of 2,048: 2,494 rows 59 / 50; 6,144 of 4,096: 192 rows 33.7 / 24.2, 700 49.9 / 38.9, 2,048 80 / 92 (the library's)
+// there are ten shapes, and gt_plan below takes the one that it expects to be fastest.  The vendor library against these, us (in a graph, the rows
+// just written by another kernel, weights from memory; activation included where the matrix is joined, and what the norm reads more of where
+// the product is left in ranges):
+//   2,048 outputs of 2,048 inputs: 128 rows 8.6 / 7.4, 512 11.4 / 9.8, 1,203 20.1 / 16.4, 2,048 21.6 / 19.8
+//   16,384 joined of 2,048: 128 rows 24.7 / 21.4, 512 43 / 36, 1,203 88 / 78, 2,048 137 / 127, 4,096 240 / 236
+//   2,048 of 8,192: 128 rows 21.2 / 16.1 (four ranges), 512 34.7 / 28.6 (four), 1,203 64.0 / 47.9 (two), 2,048 77 / 68 (two), 4,096 120 / 116
+//   5,152 of 2,048: 512 rows 24.0 / 19.4, 2,048 50 / 49; 6,144 of 4,096: 128 rows 25.2 / 21.3, 1,024 54 / 51, 2,048 84 (the library's)
 #include "tile_activations.h"
 #include "tile_product.h"
 
@@ -103,10 +103,12 @@ gemm_tiles_kernel(GtArgs a) {
 
 // The shapes: rows and outputs a workgroup, with what a launch of one turn of the units costs beside its stages (us), a stage of 64
 // elements of K, a megabyte of operands, and a megabyte of partial products.  Fitted to 5,600 timings of 19 matrices of the 1B, 3B and 8B
-// layer sizes and others at 65 to 8,190 rows (weights from memory up to 1,000 rows); of the shape they choose the time is within
-// 0.3 % of the best of the ten on average, 9 % at most.  (128 x 128: 0.393 there; 0.41 is what it takes behind a model's other kernels,
-// where 2,048 rows of 2,048 x 8,192 want two ranges of 128 x 256, 9.5 us less of a layer's 274.)  Five more shapes (64 x 128, 64 x 256, 96 x 256, 256 x 128, 128 x 256 by eight
-// wavefronts) were tried and bring nothing on average.
+// layer sizes and others at 65 to 8,190 rows, the same weights again from 1,000 rows on; 128 x 128's stage, 0.393 in that fit, is 0.41 because
+// with weights from memory and the rows just written it takes 0.43.  In those conditions, 609 products of 18 matrices at 65 to
+// 8,190 rows, what is chosen is 1.4 % behind the best of all shapes, ranges and the library on average, 4.5 % at the ninetieth of a hundred and 1.72 times
+// at most (135 to 158 rows of 6,144 x 4,096, where the library's time jumps from 22 us to 38); the same from 0.40 to 0.42, with 0.393 0.05 % more, with all
+// ten shapes fitted to these conditions 0.2 % more.  Five more shapes (64 x 128, 64 x 256, 96 x 256, 256 x 128, 128 x 256 by eight wavefronts) were tried
+// and bring nothing on average.
 struct GtShape {
     int rows, outs;
     float turn, stage, megabyte, part_megabyte;
@@ -170,7 +172,8 @@ static bool gt_sizes(int M, int N, int K, int form) {
 // graph (1B, 3B and 8B sizes):
 // * the joined ones up to where rows x outputs x K make 3.3 million times 65,536: two passes over the sums are gone, 0.68 to 0.98 of library and
 //   activation.  In a layer, 1B sizes, 96 / 517 / 1,203 / 2,048 / 4,096 rows 3.8 / 7.5 / 14 / 8 / 13 us less, 3B 517 / 1,203 / 2,048 13 / 22 / 18, 8B 517 /
-//   1,203 20 / 14; 2,048 rows of 28,672 x 4,096 5 us more;
+//   1,203 20 / 14; 2,048 rows of 28,672 x 4,096 5 us more.  (170 joined products in those conditions: 421 to 512 rows of 28,672 x 4,096 3 to 11 us more than
+//   the library's 105, a turn of 224 workgroups; five slower than it by 2 % and more, and any line through the two estimates loses more elsewhere);
 // * from 155 tiles of 256 x 256 on (2,048 rows x 5,120 outputs) the library's tiles of that size fill the units and run at 1.3 to 1.6
 //   PFLOP/s against 1.2 to 1.4: 8,190 x 4,096 x 14,336 608 / 707 us; except where the outputs are no multiple of 256, 0.86 to 0.96 there;
 // * below, where the expected time is at most 1.1 of the library's; up to 64 tiles 1.3 of it, because the library's
