@@ -158,18 +158,19 @@ def use_lds_kernel(groups: int, mean_keys: float, head_dim: int) -> bool:
 # 41), and from 640 on otherwise (0.77; below, the last workgroup walks its keys with the mask on, and 2,047 tokens are 42 against 44, 2,143 44 against
 # 47).  Above 96 from 272 to 544 workgroups, 512 to 2,047 keys: 0.71, and 0.84 where whole; the slowest of 257 1.18.  Not from 2,048 keys on: the chain
 # of the furthest portion is halved, where four wavefronts an item or key ranges cut it further, so portions at unlike depths were up to twice as
-# slow (six of 319 behind 512 to 16,000 keys 141 against 283), heads of 128 behind 8,192 keys 428 against 443.  Not above 544: 1.03 to 1.2 where whole.
+# slow (six of 319 behind 512 to 16,000 keys 141 against 283), heads of 128 behind 8,192 keys 428 against 443.  Not above 544 where whole: 1.03 to 1.2; to 659
+# otherwise, below 1,024 keys, where they are 0.93 of blocks of 64 (1,601 and 676 tokens 52 against 62, 1,014 and 1,197 48 against 49).
 # Blocks of 64 keys, against blocks of 32: heads up to 64 from 700 workgroups and 512 keys on 0.93 (odd) and 0.95 (whole), but of 1,025 to 1,299 workgroups only
 # from 4,096 keys on (below 0.92 and 1.03) and of more from 1,024 on; fewer keys 1.0 to 1.3 (sixteen prompts of 200 14 against 18).  Above 96 from 545 to 749
 # workgroups, 512 to 2,047 keys, 0.90 and 0.94, and to 899 from 1,024 on, 0.89 and 0.97; more keys up to 1.25 (3,392 tokens behind 6,000 322 against 403),
 # more workgroups 0.9 to 1.13.
 LDS_BLOCKS_OF_32, LDS_BLOCKS_OF_64, LDS_TWO_GROUPS = 0, 1, 2
 _ANY_KEYS = 1 << 30
-# (workgroups from, below; mean keys from, below), by whether heads are above 96
-_TWO_GROUPS = {False: ((448, 700, 1024, 2048),), True: ((272, 545, 512, 2048),)}
+# (workgroups from, below; mean keys from, below), by whether heads are above 96, and for two groups whether portions are whole workgroups
+_TWO_GROUPS = {(False, True): ((448, 700, 1024, 2048),), (False, False): ((640, 700, 1024, 2048),),
+               (True, True): ((272, 545, 512, 2048),), (True, False): ((272, 545, 512, 2048), (545, 660, 512, 1024))}
 _LONG_BLOCKS = {False: ((700, 1025, 512, _ANY_KEYS), (1025, 1300, 4096, _ANY_KEYS), (1300, _ANY_KEYS, 1024, _ANY_KEYS)),
                 True: ((545, 750, 512, 2048), (750, 900, 1024, 2048))}
-_TWO_GROUPS_RAGGED_FROM = 640           # heads up to 96, portions that end inside a workgroup
 
 
 def choose_lds_kind(groups: int, mean_keys: float, head_dim: int, by_workgroup: bool, whole: bool = True) -> int:
@@ -179,10 +180,10 @@ def choose_lds_kind(groups: int, mean_keys: float, head_dim: int, by_workgroup: 
     wide = head_dim > 96
 
     def within(lines) -> bool:
-        return any(a <= groups < b and lo <= mean_keys < hi for a, b, lo, hi in lines[wide])
-    if within(_TWO_GROUPS) and (wide or whole or groups >= _TWO_GROUPS_RAGGED_FROM):
+        return any(a <= groups < b and lo <= mean_keys < hi for a, b, lo, hi in lines)
+    if within(_TWO_GROUPS[wide, bool(whole)]):
         return LDS_TWO_GROUPS
-    return LDS_BLOCKS_OF_64 if by_workgroup and within(_LONG_BLOCKS) else LDS_BLOCKS_OF_32
+    return LDS_BLOCKS_OF_64 if by_workgroup and within(_LONG_BLOCKS[wide]) else LDS_BLOCKS_OF_32
 
 
 def _cut_keys(want: int, max_context: int, max_splits: int) -> tuple:

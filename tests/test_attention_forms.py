@@ -31,6 +31,8 @@ def test_portions_keep_the_kernels_that_are_faster_for_them():
             ([905] * 2, 3581, 4, 64, (4, 0)),                               # behind 256 and 6,000: 126 / 93
             ([2173], 9279, 4, 128, (1, 1)),                                 # 443 / 428 in blocks of 32
             ([200] * 16, 100.5, 4, 64, (1, 1)),                             # 18 in blocks of 64 / 14
+            ([1601, 676], 663, 4, 128, (1, 1 + A.LDS_TWO_GROUPS)),          # 52 / 62 in blocks of 64
+            ([1248] * 2, 624.5, 4, 128, (1, 1 + A.LDS_BLOCKS_OF_64)),       # 42 / 53 in two groups
             ([1000] * 3, 4500.5, 4, 128, (1, 1)),                           # 250 / 211
             ([5885], 7039, 3, 128, (1, 1)),                                 # 528 / 507
             ([3072], 1536.5, 4, 64, (1, 1 + A.LDS_BLOCKS_OF_64))):          # 59 / 66 in blocks of 32
