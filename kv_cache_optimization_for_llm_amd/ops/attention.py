@@ -152,11 +152,11 @@ def use_lds_kernel(groups: int, mean_keys: float, head_dim: int) -> bool:
 
 # The workgroup kernel's other forms (csrc/attention_lds.hip), by workgroups of 128 rows over all kv heads and mean keys.  Where the lines lie comes
 # from 4,400 steps of one to eight portions of 32 heads of 64 and 24 and 32 of 128 over 8: alike and unlike in length, from position 0 and from the
-# same and different ones up to 16,000, a third of them of whole workgroups.
+# same and different ones up to 16,000, two fifths of them whole: every portion's rows a multiple of a wavefront's 32.
 # Two groups of wavefronts, against what else is chosen (two or four wavefronts an item, or blocks of 32): heads up to 64 from 448 to 699 workgroups,
-# 1,024 to 2,047 keys, 0.85 of its time where every portion is whole workgroups (one prompt of 2,048 tokens 39 -> 34 us; 2,176 42.5 -> 37, 2,400 49 ->
-# 41), and from 640 on otherwise (0.77; below, the last workgroup walks its keys with the mask on, and 2,047 tokens are 42 against 44, 2,143 44 against
-# 47).  Above 96 from 272 to 544 workgroups, 512 to 2,047 keys: 0.71, and 0.84 where whole; the slowest of 257 1.18.  Not from 2,048 keys on: the chain
+# 1,024 to 2,047 keys, 0.85 of its time where portions are whole (one prompt of 2,048 tokens 39 -> 34 us; 2,176 42.5 -> 37, 2,400 49 -> 41), and from
+# 640 on otherwise (0.73; below, the last wavefront walks its keys with the mask on, 1.01, and 2,047 tokens are 42 against 44, 2,143 44 against
+# 47).  Above 96 from 272 to 544 workgroups, 512 to 2,047 keys: 0.71, and 0.84 where whole; the slowest of 276 1.18.  Not from 2,048 keys on: the chain
 # of the furthest portion is halved, where four wavefronts an item or key ranges cut it further, so portions at unlike depths were up to twice as
 # slow (six of 319 behind 512 to 16,000 keys 141 against 283), heads of 128 behind 8,192 keys 428 against 443.  Not above 544 where whole: 1.03 to 1.2; to 659
 # otherwise, below 1,024 keys, where they are 0.93 of blocks of 64 (1,601 and 676 tokens 52 against 62, 1,014 and 1,197 48 against 49).
@@ -166,7 +166,7 @@ def use_lds_kernel(groups: int, mean_keys: float, head_dim: int) -> bool:
 # more workgroups 0.9 to 1.13.
 LDS_BLOCKS_OF_32, LDS_BLOCKS_OF_64, LDS_TWO_GROUPS = 0, 1, 2
 _ANY_KEYS = 1 << 30
-# (workgroups from, below; mean keys from, below), by whether heads are above 96, and for two groups whether portions are whole workgroups
+# (workgroups from, below; mean keys from, below), by whether heads are above 96, and for two groups whether portions are whole
 _TWO_GROUPS = {(False, True): ((448, 700, 1024, 2048),), (False, False): ((640, 700, 1024, 2048),),
                (True, True): ((272, 545, 512, 2048),), (True, False): ((272, 545, 512, 2048), (545, 660, 512, 1024))}
 _LONG_BLOCKS = {False: ((700, 1025, 512, _ANY_KEYS), (1025, 1300, 4096, _ANY_KEYS), (1300, _ANY_KEYS, 1024, _ANY_KEYS)),
@@ -175,7 +175,7 @@ _LONG_BLOCKS = {False: ((700, 1025, 512, _ANY_KEYS), (1025, 1300, 4096, _ANY_KEY
 
 def choose_lds_kind(groups: int, mean_keys: float, head_dim: int, by_workgroup: bool, whole: bool = True) -> int:
     """Which form of the workgroup kernel takes ``groups`` workgroups of rows that visit ``mean_keys`` keys on average; ``by_workgroup``:
-    they go to that kernel in any case; ``whole``: every portion's rows fill their workgroups.  (Two groups are also ahead of the
+    they go to that kernel in any case; ``whole``: every portion's rows are a multiple of 32.  (Two groups are also ahead of the
     one-wavefront kernel, so its lines do not hold there.)"""
     wide = head_dim > 96
 
@@ -569,7 +569,7 @@ def portion_choice(lens, mean_keys: float, group: int, num_kv_heads: int, head_d
     groups = sum(-(-n // 128) for n in long) * num_kv_heads
     workgroups = K.attention_lds_supported(head_dim, page_size)
     # (behind a window most of a context is skipped: as before)
-    whole = all(n % 128 == 0 for n in long)
+    whole = all(n % 32 == 0 for n in long)          # (rows of a wavefront)
     if workgroups and not 0 < visible < mean_keys and choose_lds_kind(groups, mean_keys, head_dim, False, whole) == LDS_TWO_GROUPS:
         return 1, 1 + LDS_TWO_GROUPS
     tiles = K.attention_mfma_row_tiles(head_dim, True)

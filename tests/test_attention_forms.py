@@ -33,6 +33,7 @@ def test_portions_keep_the_kernels_that_are_faster_for_them():
             ([200] * 16, 100.5, 4, 64, (1, 1)),                             # 18 in blocks of 64 / 14
             ([1601, 676], 663, 4, 128, (1, 1 + A.LDS_TWO_GROUPS)),          # 52 / 62 in blocks of 64
             ([1248] * 2, 624.5, 4, 128, (1, 1 + A.LDS_BLOCKS_OF_64)),       # 42 / 53 in two groups
+            ([1120] * 3, 560.5, 3, 128, (1, 1 + A.LDS_BLOCKS_OF_64)),       # 41 / 53, rows that end inside a workgroup but not inside a wavefront
             ([1000] * 3, 4500.5, 4, 128, (1, 1)),                           # 250 / 211
             ([5885], 7039, 3, 128, (1, 1)),                                 # 528 / 507
             ([3072], 1536.5, 4, 64, (1, 1 + A.LDS_BLOCKS_OF_64))):          # 59 / 66 in blocks of 32
