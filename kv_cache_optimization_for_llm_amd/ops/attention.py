@@ -164,6 +164,8 @@ def use_lds_kernel(groups: int, mean_keys: float, head_dim: int) -> bool:
 # from 4,096 keys on (below 0.92 and 1.03) and of more from 1,024 on; fewer keys 1.0 to 1.3 (sixteen prompts of 200 14 against 18).  Above 96 from 545 to 749
 # workgroups, 512 to 2,047 keys, 0.90 and 0.94, and to 899 from 1,024 on, 0.89 and 0.97; more keys up to 1.25 (3,392 tokens behind 6,000 322 against 403),
 # more workgroups 0.9 to 1.13.
+# On 4,000 further steps, drawn alike: 0.93 (heads of 64) and 0.82 (128) of the time where the lines change the kernel, 39 of 932 slower by more than
+# 3 %, 1.22 at most (six of 640 behind 1,024).
 LDS_BLOCKS_OF_32, LDS_BLOCKS_OF_64, LDS_TWO_GROUPS = 0, 1, 2
 _ANY_KEYS = 1 << 30
 # (workgroups from, below; mean keys from, below), by whether heads are above 96, and for two groups whether portions are whole
