@@ -168,17 +168,16 @@ static bool gt_sizes(int M, int N, int K, int form) {
 }
 
 // Shape + 256 x ranges of K, or -1: the library is expected to be faster, or takes what these do not.
-// Where the line lies, of the 19 matrices at 65 to 8,190 rows and, "in a layer", of a layer's products and norms over all layers' weights in a
-// graph (1B, 3B and 8B sizes):
-// * the joined ones up to where rows x outputs x K make 3.3 million times 65,536: two passes over the sums are gone, 0.68 to 0.98 of library and
-//   activation.  In a layer, 1B sizes, 96 / 517 / 1,203 / 2,048 / 4,096 rows 3.8 / 7.5 / 14 / 8 / 13 us less, 3B 517 / 1,203 / 2,048 13 / 22 / 18, 8B 517 /
-//   1,203 20 / 14; 2,048 rows of 28,672 x 4,096 5 us more.  (170 joined products in those conditions: 421 to 512 rows of 28,672 x 4,096 3 to 11 us more than
-//   the library's 105, a turn of 224 workgroups; five slower than it by 2 % and more, and any line through the two estimates loses more elsewhere);
+// Where the line lies, of the 19 matrices at 65 to 8,190 rows.  A layer's four products and two norms over all layers' weights in a graph, us by the
+// library (with the activation's pass) / here, 96 / 517 / 1,203 / 2,048 / 4,096 rows: 1B sizes 77 / 130 / 216 / 272 / 451 -> 60 / 105 / 175 / 250 / 451, 3B 114 / 178 /
+// 302 / 405 / 706 -> 84 / 149 / 273 / 388 / 694, 8B 180 / 348 / 563 / 781 / 1,324 -> 134 / 285 / 506 / 762 / 1,310.
+// * the joined ones up to where rows x outputs x K make 3.3 million times 65,536: two passes over the sums are gone.  Of 170 of them with rows just
+//   written and weights from memory five are slower than the library by 2 % and more: 421 to 512 and 766 rows of 28,672 x 4,096, 3 to 11 % (a turn of 224
+//   workgroups); any line through the two estimates loses more elsewhere;
 // * from 155 tiles of 256 x 256 on (2,048 rows x 5,120 outputs) the library's tiles of that size fill the units and run at 1.3 to 1.6
 //   PFLOP/s against 1.2 to 1.4: 8,190 x 4,096 x 14,336 608 / 707 us; except where the outputs are no multiple of 256, 0.86 to 0.96 there;
 // * below, where the expected time is at most 1.1 of the library's; up to 64 tiles 1.3 of it, because the library's
-//   middle hides its slow choices: 0.53 to 0.98 in 111 of 129 cases.  In a layer, the output and down projections of 1B sizes at 517 / 1,203 / 2,048 rows
-//   0.6 + 13 / 7 + 18 / 3 + 8 us less, 8B 7 + 45 / 9 + 36 / 6 + 17.  Not where 64 x 64 tiles leave units idle over a long K (65 to 256 rows of 2,048 x
+//   middle hides its slow choices: 0.53 to 0.98 in 111 of 129 cases.  Not where 64 x 64 tiles leave units idle over a long K (65 to 256 rows of 2,048 x
 //   8,192 20-27 us by the library, 27-36 here) and not for a few outputs (16 of 2,048 rows and inputs: 5.1 / 6.9 us);
 // * in ranges only where 1.15 of it is: 3,072 rows of 2,048 x 8,192 are 5 us slower in two ranges of 192 x 256 in a layer.
 static int gt_plan(int M, int N, int K, int form) {

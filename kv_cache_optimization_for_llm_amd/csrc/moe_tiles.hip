@@ -7,8 +7,9 @@
 //
 // What bounds it: up to 2,000 tokens one or two turns of the units, a stage of 256 x 256 x 64 some 1.3 us of matrix products and loads,
 // and around them the first operands' way from memory and the results' to it.  Before (moe.hip's 128 x 256, two workgroups a unit) and
-// now, in the model, us: 2,048 tokens, 4 of 16 experts of 1,536 x 2,048 68 / 62 (830 TFLOP/s), of 2,048 x 768 58 / 48; all of 4
-// of 1,024 x 2,048 with erf-gelu 49.5 / 46; 2,494 tokens, all of 4 of 1,536 x 2,048 65 / 62.
+// now, in the model, us: 2,048 tokens, 4 of 16 experts of 1,536 x 2,048 68 / 64 (805 TFLOP/s), of 2,048 x 768 58 / 48; 2,494 tokens, all of
+// 4 of 1,536 x 2,048 66 / 64.  An activation that costs as much as the sums (erf-gelu, tanh) is better off in moe.hip's, where the other workgroup of
+// the unit multiplies meanwhile, unless its turns divide badly (mt_first).
 #include "tile_activations.h"
 #include "tile_product.h"
 #include <math.h>
@@ -185,32 +186,44 @@ moe_tiles_kernel(MtArgs a) {
 }
 
 // The shapes: rows and outputs a workgroup, with what one turn of the units (one workgroup each) costs beside its stages (us), a stage of
-// 64 elements of K, and a megabyte of operands, for the first product and, with a megabyte of results, for the second.  Fitted to the
-// timings of nine shapes over 45 sizes of either product: 100 to 6,000 tokens, 4 to 64 experts, 512 to 4,096 wide; the shape they
-// choose is 2 % (first) and 4 % (second) behind the best of the nine on average.
+// 64 elements of K, a megabyte of operands and one of results.  For the first product fitted, with moe_expert_rows' costs below, to the
+// timings of all nine over 7,408 layers' experts, matrices from memory: 60 to 8,190 tokens, 1 to 6 of 4 to 64 experts chosen evenly, 1,024
+// to 4,096 wide, 384 to 2,816 inside, six activations.  For the second to the nine over 45 sizes: 100 to 6,000 tokens, 4 to 64 experts, 512 to 4,096
+// wide; the shape they choose there is 4 % behind the best of the nine on average.
 struct MtShape {
-    int rows, outs;
+    int rows, outs, threads;
     struct {
         float turn, stage, megabyte, results;
     } of[2];
 };
-#define MT_SHAPES(V)                                                                          \
-    V(0, 8, 4, 2, 4, 1, 2, 2, 3.04f, 1.283f, 0.074f, 0.f, 3.13f, 1.411f, 0.029f, 0.205f)      \
-    V(1, 4, 8, 2, 2, 1, 2, 3, 1.56f, 0.852f, 0.066f, 0.f, 2.58f, 0.842f, 0.063f, 0.208f)      \
-    V(2, 4, 4, 2, 2, 2, 1, 4, 3.37f, 0.502f, 0.061f, 0.f, 0.45f, 0.556f, 0.079f, 0.402f)      \
-    V(3, 5, 4, 2, 4, 1, 2, 3, 4.81f, 0.899f, 0.018f, 0.f, 0.98f, 1.025f, 0.031f, 0.251f)      \
-    V(4, 5, 4, 2, 2, 2, 1, 4, 6.02f, 0.532f, 0.031f, 0.f, 2.72f, 0.481f, 0.043f, 0.405f)      \
-    V(5, 3, 4, 2, 2, 2, 1, 4, 0.00f, 0.552f, 0.053f, 0.f, 0.00f, 0.606f, 0.031f, 0.410f)      \
-    V(6, 6, 4, 2, 4, 1, 2, 2, 10.56f, 0.864f, 0.052f, 0.f, 5.87f, 0.900f, 0.043f, 0.219f)     \
-    V(7, 2, 2, 2, 2, 2, 1, 8, 3.05f, 0.291f, 0.000f, 0.f, 0.00f, 0.262f, 0.115f, 1.008f)      \
-    V(8, 4, 2, 2, 2, 2, 1, 6, 4.27f, 0.354f, 0.011f, 0.f, 1.04f, 0.350f, 0.080f, 0.577f)
+#define MT_SHAPES(V)                                                                             \
+    V(0, 8, 4, 2, 4, 1, 2, 2, 4.95f, 1.175f, 0.075f, 0.563f, 3.13f, 1.411f, 0.029f, 0.205f)      \
+    V(1, 4, 8, 2, 2, 1, 2, 3, 5.08f, 0.643f, 0.080f, 0.470f, 2.58f, 0.842f, 0.063f, 0.208f)      \
+    V(2, 4, 4, 2, 2, 2, 1, 4, 4.91f, 0.341f, 0.100f, 0.572f, 0.45f, 0.556f, 0.079f, 0.402f)      \
+    V(3, 5, 4, 2, 4, 1, 2, 3, 5.94f, 0.735f, 0.072f, 0.632f, 0.98f, 1.025f, 0.031f, 0.251f)      \
+    V(4, 5, 4, 2, 2, 2, 1, 4, 5.09f, 0.420f, 0.088f, 0.650f, 2.72f, 0.481f, 0.043f, 0.405f)      \
+    V(5, 3, 4, 2, 2, 2, 1, 4, 4.22f, 0.314f, 0.097f, 0.671f, 0.00f, 0.606f, 0.031f, 0.410f)      \
+    V(6, 6, 4, 2, 4, 1, 2, 2, 4.88f, 0.982f, 0.080f, 0.522f, 5.87f, 0.900f, 0.043f, 0.219f)      \
+    V(7, 2, 2, 2, 2, 2, 1, 8, 5.02f, 0.191f, 0.065f, 0.188f, 0.00f, 0.262f, 0.115f, 1.008f)      \
+    V(8, 4, 2, 2, 2, 2, 1, 6, 4.92f, 0.236f, 0.081f, 0.769f, 1.04f, 0.350f, 0.080f, 0.577f)
 #define MT_COUNT 9
 #define MT_BOTH(a, b, c, d, e, f, g, h) {a, b, c, d}, {e, f, g, h}
 static const MtShape mt_shapes[MT_COUNT] = {
-#define MT_ROW(ID, RT, NT, WR, WN, WK, KSUB, ST, ...) {16 * RT * WR, 16 * NT * WN, {MT_BOTH(__VA_ARGS__)}},
+#define MT_ROW(ID, RT, NT, WR, WN, WK, KSUB, ST, ...) {16 * RT * WR, 16 * NT * WN, 64 * WR * WN, {MT_BOTH(__VA_ARGS__)}},
     MT_SHAPES(MT_ROW)
 #undef MT_ROW
 };
+// an activation of each lane (MT_ACT_SILU ..), here a turn's and in moe_expert_rows
+static const float mt_act_here[] = {0.0223f, 0.f, 0.0807f, 0.0591f, 0.0636f, 0.f}, mt_act_rows[] = {0.0483f, 0.f, 0.0853f, 0.0760f, 0.0581f, 0.f};
+// moe_expert_rows' first product, two workgroups a unit: groups of 8 tiles against 256 outputs, against 128, groups of 4 against 128.  A stage of K in
+// turns of 512 workgroups, a workgroup and a stage where turns even out, a workgroup and a stage in turns of 256, a megabyte of operands and of results.
+struct MtRows {
+    int rows, outs;
+    float stage, even, even_stage, single, single_stage, megabyte, results;
+};
+static const MtRows mt_rows[] = {{128, 256, 0.2765f, 1.66f, 0.2623f, 0.72f, 0.4822f, 0.087f, 0.233f},
+                                 {128, 128, 0.0765f, 3.37f, 0.f, 0.48f, 0.3150f, 0.112f, 0.403f},
+                                 {64, 128, 0.0358f, 2.78f, 0.0492f, 0.f, 0.2069f, 0.134f, 0.f}};
 #define MT_UNITS 256
 #define MT_STAGE 64
 
@@ -219,36 +232,90 @@ static bool mt_sizes(long long tiles, int experts, int N, int K) {
            (long long)N * K * 2 <= 0x7fffffffll && tiles * MT_TILE * K * 2 <= 0x7fffffffll;
 }
 
-// (experts that all tokens take have as many rows each; else every expert's last block is half full on average)
+// (the second product: experts that all tokens take have as many rows each; else every expert's last block is half full on average)
 static double mt_blocks(double slots, int experts, int top, int rows, int N, int outs) {
     return ceil(top == experts ? experts * ceil(slots / experts / rows) : slots / rows + 0.5 * experts) * ((N + outs - 1) / outs);
 }
 
+// Blocks of `rows` rows of one expert over all experts, on average, and their spread: an expert's rows are as many as all tokens', or spread as an even
+// choice of `top` of `experts` spreads them.  Its blocks are those that surely fill and, of those around the mean, each by its likelihood.
+struct MtSpread {
+    double mean, spread;
+};
+static double mt_above(double z) { return 0.5 * erfc(z * 0.70710678118654752); }
+static MtSpread mt_spread(double slots, int experts, int top, int rows) {
+    const double n = slots / experts, sd = top < experts ? sqrt(n * (1.0 - (double)top / experts)) : 0.0;
+    if (sd < 0.5) return {experts * ceil(n / rows), 0.0};
+    const int sure = (int)fmax(0.0, (n - 4.0 * sd) / rows);
+    double sum = 0.0, square = 0.0;
+    for (int i = 0;; ++i) {
+        const double p = mt_above(((double)rows * (sure + i) + 0.5 - n) / sd);
+        if (p < 1e-4) break;
+        sum += p, square += (2 * i + 1) * p;
+    }
+    return {experts * (sure + sum), sqrt(experts * fmax(0.0, square - sum * sum))};
+}
+
+// turns of `at_once` workgroups that these blocks against `columns` workgroups each take on average
+static double mt_turns(MtSpread b, double columns, double at_once) {
+    if (b.spread <= 0.05) return ceil(rint(b.mean) * columns / at_once);
+    const int sure = (int)fmax(0.0, (b.mean - 4.0 * b.spread) * columns / at_once);
+    double turns = sure;
+    for (int i = sure;; ++i) {
+        const double p = i == 0 ? 1.0 : mt_above((floor(at_once * i / columns) + 0.5 - b.mean) / b.spread);
+        if (p < 1e-3) return turns;
+        turns += p;
+    }
+}
+
+// The first product: of the 7,408 (half of them not fitted to) the choice is 1.2 % behind the best on average, taken in 0.78 of them, 0.873 of
+// moe_expert_rows' time over all, and slower by more than 3 % in 3 % (with a line at 1 instead of 0.97 4 %).  Without the activation, with turns from the
+// mean number of workgroups and no estimate for moe_expert_rows: 4.7 %, 0.87, 0.903 and 14 %.  us, moe_expert_rows / here: 8,192 slots of
+// 16 experts of 1,536 x 2,048, gated silu, 64.7 / 62.3, of 1,024 x 2,048, erf-gelu, 68.5 / 49.6, 1,024 slots of 4 16.8 / 12.2; but 8,192 slots of 4
+// experts of 1,024 x 2,048 with erf-gelu 43.4 / 44.6 and with the tanh form 43.1 / 48.5, 4,812 of 32 of 1,024 x 1,024 27.3 / 33.3.
+static int mt_first(int slots, int experts, int top, int N, int K, int act, int gated, int group, long long list) {
+    const double halves = gated ? 2.0 : 1.0, operands = 2e-6 * K * ((double)N * experts + slots), results = 2e-6 * slots * N / halves, stages = K / MT_STAGE;
+    int best = -1;
+    double least = 0.0;
+    for (int i = 0; i < MT_COUNT; ++i) {
+        const MtShape &s = mt_shapes[i];
+        const double turns = mt_turns(mt_spread(slots, experts, top, s.rows), (N + s.outs - 1) / s.outs, MT_UNITS);
+        const double t = turns * (s.of[0].turn + stages * s.of[0].stage + mt_act_here[act] * s.rows * s.outs / halves / s.threads) +
+                         operands * s.of[0].megabyte + results * s.of[0].results;
+        if (best < 0 || t < least) best = i, least = t;
+    }
+    // (its kind: as ops/kernels.py:moe_wide has it, by the groups of the list)
+    const MtRows &r = mt_rows[group != 8 ? 2 : ((N + 255) / 256) * (2 * (list / 8) - experts) > 576 ? 0 : 1];
+    const MtSpread blocks = mt_spread(slots, experts, top, r.rows);
+    const double columns = (N + r.outs - 1) / r.outs, even = fmax(1.0, blocks.mean * columns / (2 * MT_UNITS));
+    const double rows = mt_turns(blocks, columns, 2 * MT_UNITS) * stages * r.stage +
+                        even * (r.even + stages * r.even_stage + mt_act_rows[act] * r.rows * r.outs / halves / 256) +
+                        mt_turns(blocks, columns, MT_UNITS) * (r.single + stages * r.single_stage) + operands * r.megabyte + results * r.results;
+    return least <= 0.97 * rows ? best : -1;
+}
+
 // Which shape is expected to be fastest for `slots` of `experts`, of which a token takes `top`; -1: sizes the kernel does not take, or
-// moe_expert_rows is expected to be faster, two workgroups a unit, of which one writes while the other multiplies.
-// First product (us, moe_expert_rows / here, matrices from memory): 8,192 slots of 16 experts of 1,536 x 2,048 68.6 / 60.6, of 4
-// experts of 1,024 x 2,048 43.6 / 40.7, 1,024 slots of 4 24.1 / 15.8, 4,000 of 16 50.5 / 36.7; 0.84 on average.  Not where many turns even out
-// what a turn costs: 12,288 slots of 64 experts of 2,816 x 2,048 212 / 241, 16,384 of 4 of 1,536 x 2,048 94 / 103 (but 8,000 of 8 of 7,168 x
-// 4,096 726 / 482).
-// Second: results in 32 bits are as long to write as a short K to multiply, and with one workgroup a unit nothing multiplies
+// moe_expert_rows in groups of `group` tiles, two workgroups a unit, of which one writes or activates while the other multiplies, is expected to be faster.
+// Second product: results in 32 bits are as long to write as a short K to multiply, and with one workgroup a unit nothing multiplies
 // meanwhile.  8,192 slots of 4 experts of 2,048 x 1,024 38 / 40, 12,000 54 / 61; of 16 of 2,048 x 768 56 / 46, where moe_expert_rows' workgroups
 // are just more than the units hold at once.  So only where a tenth less than there is expected, from the same sizes.
-extern "C" int kva_moe_tiles_plan(int slots, int experts, int top, int N, int K, int second) {
+extern "C" int kva_moe_tiles_plan(int slots, int experts, int top, int N, int K, int second, int act, int gated, int group) {
     // (tiles: of a list in groups of eight, which the other product may need)
-    if (slots <= 0 || experts <= 0 || top <= 0 || !mt_sizes((slots + 127ll * experts + 127) / 128 * 8, experts, N, K)) return -1;
+    const long long list = (slots + 127ll * experts + 127) / 128 * 8;
+    if (slots <= 0 || experts <= 0 || top <= 0 || act < MT_ACT_SILU || act > MT_ACT_RELU2 || !mt_sizes(list, experts, N, K)) return -1;
+    if (!second) return mt_first(slots, experts, top, N, K, act, gated, group, list);
     const double operands = 2e-6 * K * ((double)N * experts + slots), results = 4e-6 * slots * N, stages = K / MT_STAGE;
     int best = -1;
     double least = 0.0;
     for (int i = 0; i < MT_COUNT; ++i) {
-        const auto &s = mt_shapes[i].of[second ? 1 : 0];
+        const auto &s = mt_shapes[i].of[1];
         const double turns = ceil(mt_blocks(slots, experts, top, mt_shapes[i].rows, N, mt_shapes[i].outs) / MT_UNITS);
         const double t = turns * (s.turn + stages * s.stage) + operands * s.megabyte + results * s.results;
         if (best < 0 || t < least) best = i, least = t;
     }
-    const double wide = mt_blocks(slots, experts, top, 128, N, 256);        // moe_expert_rows' workgroups, the larger kind
-    if (!second) return wide > 700 && K < 3072 ? -1 : best;
     if (slots < 160ll * experts) return K < 1280 ? -1 : best;
-    // (past 288 of them they are taken, and below half as many outputs a workgroup)
+    // (moe_expert_rows' workgroups of the larger kind: past 288 of them they are taken, and below half as many outputs a workgroup)
+    const double wide = mt_blocks(slots, experts, top, 128, N, 256);
     const double rows = wide > 288 ? ceil(wide / 512) * stages * 1.161 + operands * 0.175 + results * 0.193
                                    : ceil(mt_blocks(slots, experts, top, 128, N, 128) / 512) * (6.41 + stages * 0.207) + operands * 0.078 + results * 0.348;
     return least <= 0.9 * rows ? best : -1;

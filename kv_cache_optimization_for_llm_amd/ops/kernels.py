@@ -2506,11 +2506,13 @@ def moe_expert_rows(x: torch.Tensor, w: torch.Tensor, out: torch.Tensor, sorted_
     return out
 
 
-def moe_tiles_plan(slots: int, experts: int, top: int, n: int, k: int, second: bool) -> int:
+def moe_tiles_plan(slots: int, experts: int, top: int, n: int, k: int, second: bool, activation: str = "silu", gated: bool = True) -> int:
     """How :func:`moe_expert_tiles` takes ``slots`` (token, choice) pairs of ``experts``, ``top`` of them a token, against matrices ``[n, k]`` in
-    the first or the second product (a number for its ``plan``), or -1: it does not take the sizes, or :func:`moe_expert_rows` in groups
-    is expected to be faster."""
-    return hip_lib().kva_moe_tiles_plan(int(slots), int(experts), int(top), int(n), int(k), 1 if second else 0)
+    the first (with its ``activation``; ``n`` both halves where it is ``gated``) or the second product (a number for its ``plan``), or -1: it does
+    not take the sizes, or :func:`moe_expert_rows` in groups is expected to be faster."""
+    group = next((g for least, g in MOE_GROUPS if slots >= least * experts), MOE_GROUPS[-1][1])
+    return hip_lib().kva_moe_tiles_plan(int(slots), int(experts), int(top), int(n), int(k), 1 if second else 0, EXPERT_ACTIVATIONS[activation],
+                                        1 if gated else 0, group)
 
 
 def moe_expert_tiles(x: torch.Tensor, w: torch.Tensor, out: torch.Tensor, sorted_slot: torch.Tensor, tile_expert: torch.Tensor, top: int,

@@ -119,7 +119,7 @@ _HIP_SIGNATURES = {
     "kva_moe_group_supported": [I, I],
     "kva_moe_table_align": [P, P, P, P, P, I, P, P, I, I, F, I, I, I, I, P],
     "kva_moe_expert_rows": [P, I, P, P, I, P, P, P, I, I, I, I, I, I, I, F, I, I, I, P],
-    "kva_moe_tiles_plan": [I, I, I, I, I, I],
+    "kva_moe_tiles_plan": [I, I, I, I, I, I, I, I, I],
     "kva_moe_tiles": [P, P, P, P, P, P, I, I, I, I, I, I, I, I, F, I, P],
     "kva_moe_few_max_tokens": [],
     "kva_moe_few_rows": [P, P, P, P, P, I, I, P, P, F, P, P, I, I, I, I, I, I, I, I, F, P, P, P, P, I, I, I, F,

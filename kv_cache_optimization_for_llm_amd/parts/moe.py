@@ -195,7 +195,7 @@ class RoutedExperts(FeedForward):
         """For both products the plan where a workgroup takes what rows of an expert there are (ops.kernels.moe_expert_tiles), or -1."""
         if not self.tiled or x.data_ptr() % 16:
             return -1, -1
-        return tuple(K.moe_tiles_plan(slots, self.experts, self.top, w.shape[1], w.shape[2], second)
+        return tuple(K.moe_tiles_plan(slots, self.experts, self.top, w.shape[1], w.shape[2], second, self.activation, self.gated)
                      for w, second in ((self.w_up, False), (self.w_down, True)))
 
     def _few(self, x) -> bool:

@@ -332,6 +332,25 @@ def test_experts_products_take_256_outputs_a_workgroup_where_128_would_not_fit_t
     assert not moe_wide(4096, moe_tiles(20000, 16, 4), 4, 16)
 
 
+def test_the_experts_first_product_goes_to_tiles_where_they_are_faster():
+    """By sizes and activation, measured (us, groups of 8 or 4 tiles / blocks of as many rows as an expert has)."""
+    from kv_cache_optimization_for_llm_amd.ops.kernels import moe_tiles_plan
+    for slots, experts, top, n, k, act, gated, tiles in (
+            (8192, 16, 4, 1536, 2048, "silu", True, True),          # 64.7/62.3
+            (8192, 16, 4, 1024, 2048, "gelu", False, True),         # 68.5/49.6
+            (2048, 4, 4, 1024, 2048, "gelu", False, True),          # 24.8/18.9
+            (8192, 4, 4, 1024, 2048, "gelu", False, False),         # 43.4/44.6
+            (8192, 4, 4, 1024, 2048, "gelu_tanh", False, False),    # 43.1/48.5
+            (8192, 16, 4, 1024, 2048, "gelu_tanh", False, True),    # 67.7/48.9
+            (4812, 32, 4, 1024, 1024, "gelu", False, False),        # 27.3/33.3
+            (4767, 8, 1, 2816, 2048, "gelu", True, False),          # 71/107
+            (17436, 32, 4, 768, 1536, "gelu_tanh", False, False),   # 66/98
+            (12000, 4, 4, 2048, 1024, "gelu", False, False),        # 74/89
+            (24000, 4, 4, 1024, 2048, "gelu", False, False),        # 103/127
+            (16384, 4, 4, 1536, 2048, "silu", True, False)):        # 98/104
+        assert (moe_tiles_plan(slots, experts, top, n, k, False, act, gated) >= 0) == tiles, (slots, experts, n, k, act)
+
+
 def test_the_choice_of_experts_is_made_inside_the_first_product_where_workgroups_and_tokens_are_few():
     """By workgroups of the launch and tokens, measured (us, in a launch of its own / inside)."""
     from kv_cache_optimization_for_llm_amd.ops.kernels import moe_choice_inside
