@@ -169,13 +169,14 @@ __global__ void rope_kv_write_vec_kernel(T *__restrict__ qkv, T *__restrict__ k_
     }
 }
 
-// Many tokens in bf16: a workgroup takes 16 neighbouring tokens and some of the heads, q's, k's or v's (blockIdx.y).  With a
-// workgroup a token the cache bounds it: neighbouring tokens' keys and values share cache lines, an element of V goes a page's row
-// further than the one before it, and eight dies write 16 and 2 bytes of a line each.  Here a line is one workgroup's, and eight
+// Many tokens in bf16 with a cache: a workgroup takes 16 neighbouring tokens and some of the heads, q's, k's or v's (blockIdx.y).
+// With a workgroup a token the cache bounds it: neighbouring tokens' keys and values share cache lines, an element of V goes a page's
+// row further than the one before it, and eight dies write 16 and 2 bytes of a line each.  Here a line is one workgroup's, and eight
 // keys that fill eight aligned places of a page go out as 16 bytes of V at a time, turned round in LDS.  A thread keeps its token's
-// cosines and sines over all of its heads.  us, before and now: 1,203 tokens (portions that begin anywhere) / 2,048 of 32 + 2 x 8
-// heads of 64 8.5 / 12.1 -> 7.6 / 8.1 (3 TB/s), 8,190 of 128 75 -> 41 (4.9 TB/s).  (Runs of four and two keys as one store, too: 9.2 at
-// 1,203 tokens, the search for them takes longer than the stores.)
+// cosines and sines over all of its heads.  us, a workgroup a token and this: 1,203 tokens (portions that begin anywhere) / 2,048 of
+// 32 + 2 x 8 heads of 64 8.5 / 12.1 and 7.6 / 8.1 (3 TB/s), 8,190 of 128 75 and 41 (4.9 TB/s).  (Runs of four and two keys as one store,
+// too: 9.2 at 1,203 tokens, the search for them takes longer than the stores.)  Few tokens are too few workgroups with a long chain
+// each: rope_tokens_wide.
 #define ROPE_TOKENS 16
 #define ROPE_HEADS 2                    // of q or k a thread takes at once
 #define ROPE_V_COLS 256
@@ -183,7 +184,7 @@ __global__ void rope_kv_write_vec_kernel(T *__restrict__ qkv, T *__restrict__ k_
 struct RopeWide {
     bf16_t *qkv, *k_cache, *v_cache;
     const float *cos_table, *sin_table;
-    const int *positions, *slot_mapping;        // slot_mapping absent: no cache
+    const int *positions, *slot_mapping;
     int tokens, num_q_heads, num_kv_heads, head_dim, page_size;
     int lanes, q_blocks, k_blocks;              // threads that share a token's chunk; workgroups of 16 tokens' q and k heads
 };
@@ -284,6 +285,22 @@ rope_kv_write_wide_kernel(RopeWide a) {
     }
 }
 
+// From where on a step in bf16 goes to rope_kv_write_wide_kernel: 2^19 elements of V, or 1,536 tokens.  Below, a workgroup of 16 tokens
+// does what 16 would at the same time: 65 / 256 tokens of a prompt of 32 + 2 x 8 heads of 64 3.5 / 4.0 us with a workgroup a token and
+// 4.9 / 4.4, decoded tokens with a page each (single stores of V) 3.4 / 4.3 and 5.4 / 6.0.  Timed over steps of 65 to 7,168 tokens, 0 to
+// 1,024 of them decoded, beside portions of 2 to 1,024, six geometries: the lines cross at 750 tokens with 512 elements of V a token,
+// 380 with 1,024, 900 with 256, 1,050 with 128 (whole prompts alone earlier, 350, 150, 550, 550), and where the step's entries begin
+// and how long they are moves them little.  All 1,842 steps: 0.86 of a workgroup a token, 0.91 with this kernel from 65 tokens on, 0.85
+// with the faster one every time; what stays slower are steps of 500 and more decoded tokens without long portions (up to 1.16).  Without a cache nothing is
+// turned round and this kernel has nothing to give: 1.39 at 65 tokens, 1.08 at 2,048, 0.94 to 1.10 at 4,096.
+static bool rope_tokens_wide(int tokens, int num_kv_heads, int head_dim, int write_cache) {
+    return write_cache && tokens > 64 && (tokens >= 1536 || (size_t)tokens * num_kv_heads * head_dim >= (size_t)1 << 19);
+}
+
+extern "C" int kva_rope_tokens_wide(int tokens, int num_kv_heads, int head_dim, int write_cache) {
+    return rope_tokens_wide(tokens, num_kv_heads, head_dim, write_cache);
+}
+
 extern "C" int kva_rope_kv_write(void *qkv, void *k_cache, void *v_cache, const float *cos_table,
                                  const float *sin_table, const int *positions,
                                  const int *slot_mapping, int tokens, int num_q_heads,
@@ -300,11 +317,11 @@ extern "C" int kva_rope_kv_write(void *qkv, void *k_cache, void *v_cache, const 
     dim3 grid(tokens), block(256);
     const uintptr_t all = (uintptr_t)qkv | (uintptr_t)k_cache | (uintptr_t)cos_table | (uintptr_t)sin_table;
     if (cos_table && rot_dim == head_dim && head_dim % 16 == 0 && (dtype == KVA_BF16 || (dtype == KVA_F32 && all % 16 == 0))) {
-        // (up to 64 tokens are too few workgroups of 16)
-        if (dtype == KVA_BF16 && tokens > 64 && head_dim <= 256 && ((all | (uintptr_t)v_cache) & 15) == 0 && (!write_cache || page_size % 8 == 0)) {
+        if (dtype == KVA_BF16 && rope_tokens_wide(tokens, num_kv_heads, head_dim, write_cache) && head_dim <= 256 &&
+            ((all | (uintptr_t)v_cache) & 15) == 0 && page_size % 8 == 0) {
             const int lanes = 256 / (ROPE_TOKENS * (head_dim / 16)), heads = lanes * ROPE_HEADS;
-            const int q_blocks = (num_q_heads + heads - 1) / heads, k_blocks = write_cache ? (num_kv_heads + heads - 1) / heads : 0;
-            const int v_blocks = write_cache ? (num_kv_heads * head_dim + ROPE_V_COLS - 1) / ROPE_V_COLS : 0;
+            const int q_blocks = (num_q_heads + heads - 1) / heads, k_blocks = (num_kv_heads + heads - 1) / heads;
+            const int v_blocks = (num_kv_heads * head_dim + ROPE_V_COLS - 1) / ROPE_V_COLS;
             if (q_blocks + k_blocks + v_blocks <= 65535) {
                 const RopeWide a{(bf16_t *)qkv, (bf16_t *)k_cache, (bf16_t *)v_cache, cos_table, sin_table, positions, slot_mapping, tokens, num_q_heads,
                                  num_kv_heads, head_dim, page_size, lanes, q_blocks, k_blocks};

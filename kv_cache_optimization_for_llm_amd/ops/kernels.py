@@ -317,6 +317,11 @@ def cast(src: torch.Tensor, out: torch.Tensor) -> torch.Tensor:
     return out
 
 
+def rope_tokens_wide(tokens: int, num_kv_heads: int, head_dim: int, cached: bool) -> bool:
+    """Whether :func:`rope_kv_write` takes so many bf16 tokens sixteen to a workgroup (aligned rows, pages of a multiple of 8)."""
+    return bool(hip_lib().kva_rope_tokens_wide(tokens, num_kv_heads, head_dim, 1 if cached else 0))
+
+
 def rope_kv_write(qkv: torch.Tensor, positions: torch.Tensor, num_q_heads: int, num_kv_heads: int,
                   head_dim: int, cos: Optional[torch.Tensor], sin: Optional[torch.Tensor],
                   k_cache: Optional[torch.Tensor], v_cache: Optional[torch.Tensor],

@@ -42,6 +42,7 @@ _HIP_SIGNATURES = {
     "kva_stream_mixed": [P, LL, P, LL, I, P, P],
     "kva_silu_mul": [P, P, I, I, I, P],
     "kva_cast": [P, P, LL, I, I, P],
+    "kva_rope_tokens_wide": [I, I, I, I],
     "kva_rope_kv_write": [P, P, P, P, P, P, P, I, I, I, I, I, I, I, I, P],
     "kva_attention_rowwise": [P, P, I, P, P, P, I, P, P, I, I, I, I, I, I, F, I, I, I, P, I, I, P],
     "kva_attention_few_reads": [I, I, I, I, I, P, P],

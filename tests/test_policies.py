@@ -351,6 +351,23 @@ def test_the_experts_first_product_goes_to_tiles_where_they_are_faster():
         assert (moe_tiles_plan(slots, experts, top, n, k, False, act, gated) >= 0) == tiles, (slots, experts, n, k, act)
 
 
+def test_rotated_tokens_share_a_workgroup_where_that_is_faster():
+    """By tokens and the elements of V of one, measured (us, a workgroup a token / sixteen tokens a workgroup)."""
+    from kv_cache_optimization_for_llm_amd.ops.kernels import rope_tokens_wide
+    for tokens, heads, dim, cached, wide in (
+            (65, 8, 64, True, False),           # 3.5/4.9; decoded tokens 3.4/5.4
+            (256, 8, 64, True, False),          # 4.0/4.4; decoded 4.3/6.0
+            (512, 2, 64, True, False),          # decoded 4.2/5.4
+            (256, 8, 128, True, False),         # decoded 5.6/7.0
+            (512, 16, 64, True, True),          # 6.5/4.9
+            (1024, 8, 64, True, True),          # 6.9/5.7
+            (2048, 1, 128, True, True),         # 6.3/5.0
+            (2048, 8, 32, True, True),          # 7.9/5.8
+            (2048, 8, 64, False, False),        # no cache: 4.8/5.2
+            (64, 64, 256, True, False)):
+        assert rope_tokens_wide(tokens, heads, dim, cached) == wide, (tokens, heads, dim, cached)
+
+
 def test_the_choice_of_experts_is_made_inside_the_first_product_where_workgroups_and_tokens_are_few():
     """By workgroups of the launch and tokens, measured (us, in a launch of its own / inside)."""
     from kv_cache_optimization_for_llm_amd.ops.kernels import moe_choice_inside

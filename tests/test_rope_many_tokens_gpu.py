@@ -8,10 +8,11 @@ pytestmark = pytest.mark.gpu
 
 
 def _slots(page, pages):
-    """Decoded tokens, tokens without a slot, and portions that begin and end anywhere in a page and go to the next one."""
+    """Decoded tokens, tokens without a slot, and portions that begin and end anywhere in a page and go to the next one; as often as
+    takes 1,536 tokens, from which the kernel for many takes any geometry."""
     g = torch.Generator().manual_seed(page)
     order, slots = torch.randperm(pages, generator=g).tolist(), []
-    for first, count in ((3, 1), (0, 1), (page - 1, 1), (5, 2 * page), (0, 3 * page), (0, 37), (7, 9), (8 % page, 41), (1, 3 * page + 2)):
+    for first, count in 10 * ((3, 1), (0, 1), (page - 1, 1), (5, 2 * page), (0, 3 * page), (0, 37), (7, 9), (8 % page, 41), (1, 3 * page + 2)):
         mine = [order.pop() for _ in range((first + count - 1) // page + 1)]
         slots += [mine[p // page] * page + p % page for p in range(first, first + count)]
     slots[11] = slots[60] = slots[-1] = -1
@@ -21,10 +22,10 @@ def _slots(page, pages):
 @pytest.mark.parametrize("cached", [True, False])
 @pytest.mark.parametrize("nq, nkv, d, page", [(32, 8, 64, 16), (5, 3, 128, 16), (3, 1, 16, 8), (7, 2, 96, 32), (2, 2, 256, 16), (40, 17, 48, 16)])
 def test_many_tokens_are_rotated_and_cached_as_few(nq, nkv, d, page, cached, gpu):
-    pages = 40
+    pages = 400
     slots = torch.tensor(_slots(page, pages), dtype=torch.int32, device=gpu)
     T = slots.numel()
-    assert T > 64 and T % 16
+    assert K.rope_tokens_wide(T, nkv, d, True) and not K.rope_tokens_wide(64, nkv, d, True) and T % 16
     g = torch.Generator().manual_seed(d)
     qkv = torch.randn((T, (nq + 2 * nkv) * d), generator=g).bfloat16().to(gpu)
     pos = torch.randint(0, 300, (T,), generator=g).to(torch.int32).to(gpu)
