@@ -9,7 +9,7 @@ pytestmark = pytest.mark.gpu
 
 
 @pytest.mark.parametrize("tokens", [1, 5, 16])
-@pytest.mark.parametrize("width", [32, 96, 544, 1024, 2048, 2080, 4096, 4608])
+@pytest.mark.parametrize("width", [32, 96, 512, 544, 1024, 1056, 1536, 2048, 2080, 4096, 4608])
 def test_the_routers_product_at_any_inner_size(width, tokens, gpu):
     g = torch.Generator().manual_seed(width + tokens)
     outputs, extra, top, ff = 6, 2, 6, 32
